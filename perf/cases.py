@@ -377,7 +377,7 @@ def tolerance(case):
     if case["dtype"] == "float32":
         return {"rel": 1e-5, "max": 1e-3}  # measured against exact(): 1.4e-6
     # bfloat16 operands, rounded in every product; measured against exact(): 0.0033 and 0.0095 (rows whose routing turns on a near tie may differ by more than the rest)
-    return {"rel": 0.013, "max": 0.5} if case["family"] == "Ranutar" else {"rel": 0.03, "max": 1.0}
+    return {"rel": 0.013, "max": 0.5} if case["family"] == "Ranutar" else {"rel": 0.03, "max": 0.99}
 
 
 # ---------------------------------------------------------------------------------------------------------------------------- the same in 64 bits, plainly
