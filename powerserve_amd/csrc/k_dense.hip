@@ -1,13 +1,15 @@
 // Dense (unquantized) matrices of the layer-list models: bfloat16 operands with fp32 accumulation on v_mfma_f32_16x16x32_bf16, or
 // fp32 throughout on v_mfma_f32_16x16x4_f32 (one rounding per product, fp32 adds: a true fp32 product, no reduced-precision mode).
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
-//   dense_mm_fast_kernel  bf16, K % 64 == 0, more than 8 tokens: 128 x 128 tiles over an operand packed to bf16 by dense_pack_kernel
-//   dense_mm_narrow_kernel bf16, K % 128 == 0, more than 8 tokens, products too small to fill the chip with 128 x 128 tiles: 32 x 32 tiles, the waves share K
+//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
+//                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
+//   dense_mm_narrow_kernel bf16, K 128 or 256, more than 8 tokens: 32 x 32 tiles, the waves share K
 //   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns): the activation rows live in LDS, a wave streams RW weight rows at a time
 // All take the same operand description (ps_seq.h psk_dense_args): ring rows, the token-shift mix and the epilogue
 // (bias, activation, scale, a factor from a second table) are part of the launch, so no mixer needs a kernel of its own around its projections.
 #include "ps_seq.h"
 
+#include <algorithm>
 #include <cmath>
 
 typedef float dn_f4 __attribute__((ext_vector_type(4)));
@@ -414,99 +416,376 @@ static void dn_launch_mv_grouped(hipStream_t st, const dn_args &g, int rows, siz
     hipLaunchKernelGGL((dense_mv_grouped_kernel<WT, RW>), dim3((unsigned)blocks, (unsigned)rows), dim3(256), lds, st, g);
 }
 
-// ---------------------------------------------------------------------------------------------------- wide mat-mul (bf16, K % 64 == 0)
-// The A operand is first packed to bfloat16 [Tp][K] (Tp = T rounded up to 128, rows beyond T zero; the ring rows and the token-shift mix
-// are resolved there), then 128 tokens x 128 outputs per work-group: four waves of 64 x 64 (4 x 4 tiles of v_mfma_f32_16x16x32_bf16), K in
-// steps of 64 through LDS (rows padded to 144 B), the next step's 16-byte global loads in flight while the matrix cores run the current one.
-__global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, unsigned short *out, int Tp) {
+// ---------------------------------------------------------------------------------------------------- wide mat-mul (bf16: K % 64 == 0, fp32: K % 32 == 0)
+// BM x BN (128 x 128, 64 x 128 or 64 x 64) tokens x outputs per work-group: four waves multiply, four load.  Both operands in blocks of 128 bytes of K per row (64 bf16 or 32 fp32)
+// through a ring of four LDS stages that the memory system fills by itself (global_load_lds_dwordx4: no registers, three blocks in flight).  What bounded the form before this one --
+// 128 x 128 tiles, one block in flight through registers, two barriers per block -- was the latency of a block: 512 x 2048 x 2048 has 64 such tiles, one wave per SIMD on a quarter
+// of the chip.  Hence the ring, smaller tiles or SPLITS of K where the tiles are fewer than the CUs (dn_ring_plan): a split product's partial tiles go to a scratch in register
+// order and a second launch adds them in a fixed order and applies the epilogue.  The loading waves are apart because a request holds its wave's issue for 60 - 185 cycles:
+// with the same four waves loading and multiplying a block of a 128 x 128 tile took 1650 cycles, 1000 of them requests, where its matrix instructions take 512.
+//   * A stage is BM token rows, then BN weight rows, 128 bytes each, unpadded.  A piece = one wave-instruction = 8 rows; the instruction fixes where a lane's 16 bytes land but
+//     not which 16 it fetches: slot s of row r holds piece s ^ (r / 2 % 8), so that the sixteen lanes a ds_read_b128 is served in meet every bank once.
+//   * One barrier per block: in front of it the loaders' shares of block k have landed (counted: the later blocks' requests stay in flight) and the reads of block k - 1 are done;
+//     behind it block k may be read and the stage of block k - 1 refilled.
+//   * Operand fragments: 16 bytes per lane.  bf16: the eight k of v_mfma_f32_32x32x16_bf16.  fp32: four k, one per v_mfma_f32_32x32x2_f32 (lanes 0-31 and 32-63 hold different k;
+//     both operands use the same assignment, so every k meets itself).
+//   * Work-group order: the token tiles of one weight piece sit 8 apart -- same XCD, same time -- so a weight is fetched into one L2 once.
+// Rows beyond T and outputs beyond N repeat the last one and are not stored.
+// Measured (kernel trace, before -> now, bf16, 512 tokens): 2048 x 2048 45 -> 14 us, 8192 x 2048 72 -> 32 us (7 of them the xIELU of its epilogue), 2048 x 8192 190 -> 25 + 13 us (the
+// sum); fp32, 300 tokens: 2048 x 2048 180 -> 30 + 11 us, 2048 x 8192 700 -> 103 + 11 us.  Loading alone takes 1030 cycles a block of 32 KiB, multiplying alone 530.  Tried and not
+// faster: five to eight stages, a wave that prefetches the weights into L2, every tile starting at another block of K.
+#define DN_STAGES 4
+size_t psk_dense_split_bytes() { return (size_t)32 << 20; } // (the parts of at most 512 tiles of 64 KiB)
+typedef float dn_f16 __attribute__((ext_vector_type(16)));
+
+struct dn_ring {
+    const char *A;      // packed operand rows (bf16 or fp32), or NULL: the rows of g.a themselves (fp32)
+    long long lda;      // bytes
+    int n_tm, tn, S;    // token tiles (grouped: at most, over all matrices), output tiles, splits of K
+    float *part;        // S > 1: [tile][S][register order]
+};
+
+// The A operand's rows with everything resolved that is not a plain row -- ring rows, token-shift mix, the slots' order and scale -- and, for bf16, rounded.
+template <typename WT>
+__global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) {
     long long row0 = g.a_row0;
     int T = g.T;
     if (!g.g_list) dn_rows(g, row0, T); // (grouped: all T slots in the order of the sorted list, whatever their matrix)
     else row0 = 0;
-    const long long per_row = g.K / 8, total = (long long)Tp * per_row;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
-        const int t = (int)((unsigned)i / (unsigned)per_row); // (the packed operand has fewer than 2^31 pieces of eight)
-        const long long k = (long long)((unsigned)i % (unsigned)per_row) * 8;
-        dn_us8 v;
+    const bool vec = g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0; // (weights of the mix are [K] vectors of their own: read one by one)
+    const unsigned per_row = (unsigned)(g.K / 8), total = (unsigned)T * per_row; // (the packed operand has fewer than 2^31 pieces of eight)
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        const int t = (int)(i / per_row);
+        const long long k = (long long)(i % per_row) * 8;
+        const float *x = dn_arow(g, row0, t) + k;
+        float v[8];
+        if (vec) {
+            *(dn_f4 *)v = *(const dn_f4 *)x;
+            *(dn_f4 *)(v + 4) = *(const dn_f4 *)(x + 4);
+        } else {
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = t < T ? dn_f2bf(dn_aval(g, row0, t, k + e)) : (unsigned short)0;
-        *(dn_us8 *)(out + (long long)t * g.K + k) = v;
+            for (int e = 0; e < 8; e++) v[e] = x[e];
+        }
+        if (g.g_list) {
+            if (g.g_scale) {
+                const float sc = g.g_scale[g.g_list[row0 + t]];
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] *= sc;
+            }
+        } else if (g.mu) {
+            const float *p = (t ? dn_arow(g, row0, t - 1) : g.shift0) + k;
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] += (p[e] - v[e]) * g.mu[k + e];
+        }
+        WT *o = out + (long long)t * g.K + k;
+        if constexpr (sizeof(WT) == 2) {
+            dn_us8 r;
+#pragma unroll
+            for (int e = 0; e < 8; e++) r[e] = dn_f2bf(v[e]);
+            *(dn_us8 *)o = r;
+        } else {
+            *(dn_f4 *)o = *(const dn_f4 *)v;
+            *(dn_f4 *)(o + 4) = *(const dn_f4 *)(v + 4);
+        }
     }
 }
 
-#define DN_FLD 72 // LDS row stride in bf16: 64 + 8
-__global__ __launch_bounds__(256) void dense_mm_fast_kernel(dn_args g, const unsigned short *A) {
-    __shared__ __attribute__((aligned(16))) unsigned short As[128 * DN_FLD];
-    __shared__ __attribute__((aligned(16))) unsigned short Bs[128 * DN_FLD];
-    long long row0;
-    int T;
+// Sixteen results of one output column n: local rows tb + 8 (r / 4) + r % 4 (the D registers of a 32 x 32 tile).  Every lane of the wave calls this.
+static __device__ __forceinline__ void dn_put16(const dn_args &g, long long row0, int T, int tb, long long n, const dn_f16 &acc) {
+    const bool nin = n < g.N;
+    const bool pair = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR;
+    float old[16];
+    if (g.accum && !pair) { // every old value is requested before the first is used
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int t = tb + 8 * (r >> 2) + (r & 3);
+            old[r] = t < T && nin ? g.out[dn_orow(g, row0, t, T) * g.ldo + n] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int t = tb + 8 * (r >> 2) + (r & 3);
+        const bool in = t < T && nin;
+        if (pair || g.em_table) { // (row n ^ 1 is the neighbouring lane's)
+            dn_put(g, dn_orow(g, row0, t, T), n, acc[r], pair ? __shfl_xor(acc[r], 1, 64) : 0.f, in);
+            continue;
+        }
+        if (!in) continue;
+        const long long o = dn_orow(g, row0, t, T);
+        const float v = dn_epi(g, acc[r], n) * (g.out_scale ? g.out_scale[o] : 1.f);
+        g.out[o * g.ldo + n] = g.accum ? old[r] + v : v;
+    }
+}
+
+// Four neighbouring results of output row t, columns n .. n + 3 (n a multiple of four).
+static __device__ __forceinline__ void dn_put4(const dn_args &g, long long t, long long n, dn_f4 acc) {
+    if (n >= g.N) return;
+    if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR || g.em_table || n + 4 > g.N || g.ldo % 4 || ((uintptr_t)g.out & 15)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) dn_put(g, t, n + e, acc[e], acc[e ^ 1], n + e < g.N);
+        return;
+    }
+    float *p = g.out + t * g.ldo + n;
+    dn_f4 v = dn_f4{0.f, 0.f, 0.f, 0.f};
+    if (g.accum) v = *(const dn_f4 *)p;
+    const float rs = g.out_scale ? g.out_scale[t] : 1.f;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float y = dn_epi(g, acc[e], n + e) * rs;
+        v[e] = g.accum ? v[e] + y : y;
+    }
+    *(dn_f4 *)p = v;
+}
+
+static __device__ __forceinline__ void dn_dma(const char *src, unsigned lds_dst) { // one wave-instruction: lane l's 16 bytes at src go to lds_dst + 16 l
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds_dst) : "memory");
+}
+
+// which tokens a tile holds: matrix e (grouped), its rows row0 .. row0 + T - 1, first local row t0; false: nothing
+template <int BM>
+static __device__ __forceinline__ bool dn_ring_rows(const dn_args &g, int tm, int &e, long long &row0, int &T, int &t0) {
+    e = 0;
+    if (g.g_seg) {
+        for (; e < g.groups; e++) { // (tiles are counted matrix by matrix)
+            row0 = g.g_seg[e];
+            T = g.g_seg[e + 1] - (int)row0;
+            const int c = (T + BM - 1) / BM;
+            if (tm < c) break;
+            tm -= c;
+        }
+        t0 = tm * BM;
+        return e < g.groups;
+    }
     dn_rows(g, row0, T);
-    const int t0 = blockIdx.y * 128;
-    if (t0 >= T) return;
-    const long long n0 = (long long)blockIdx.x * 128;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, lr = lane & 15, lq = lane >> 4;
-    const unsigned short *W = (const unsigned short *)g.w + (g.g_seg ? (long long)blockIdx.z * g.wstride : 0);
-    if (g.g_seg) A += row0 * g.K; // (the packed operand is in list order: this matrix's slots start at row0; a tile's rows beyond them are another matrix's or zero, and are not stored)
-    const long long K = g.K;
-    // staging: 128 rows x 64 k = 1024 pieces of 16 bytes per operand, four per thread: row = (tid >> 3) + 32 i, k piece = tid & 7
-    const int sr = tid >> 3, sk = (tid & 7) * 8;
-    const unsigned short *ap[4], *bp[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        ap[i] = A + (long long)(t0 + sr + 32 * i) * K + sk; // (the packed operand has Tp rows: always there)
-        long long n = n0 + sr + 32 * i;
-        if (n >= g.N) n = g.N - 1;
-        bp[i] = W + n * K + sk;
-    }
-    dn_f4 ra[4], rb[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) { ra[i] = *(const dn_f4 *)ap[i]; rb[i] = *(const dn_f4 *)bp[i]; }
-    dn_f4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = dn_f4{0.f, 0.f, 0.f, 0.f};
-    for (long long k0 = 0; k0 < K; k0 += 64) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            *(dn_f4 *)&As[(sr + 32 * i) * DN_FLD + sk] = ra[i];
-            *(dn_f4 *)&Bs[(sr + 32 * i) * DN_FLD + sk] = rb[i];
-        }
-        __syncthreads();
-        if (k0 + 64 < K) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) { ra[i] = *(const dn_f4 *)(ap[i] + k0 + 64); rb[i] = *(const dn_f4 *)(bp[i] + k0 + 64); }
-        }
-#pragma unroll
-        for (int kk = 0; kk < 64; kk += 32) {
-            dn_bf8 fa[4], fb[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const dn_f4 xa = *(const dn_f4 *)&As[(wm * 64 + i * 16 + lr) * DN_FLD + kk + lq * 8];
-                const dn_f4 xb = *(const dn_f4 *)&Bs[(wn * 64 + i * 16 + lr) * DN_FLD + kk + lq * 8];
-                __builtin_memcpy(&fa[i], &xa, 16);
-                __builtin_memcpy(&fb[i], &xb, 16);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int t = t0 + wm * 64 + i * 16 + lq * 4 + e;
-                const long long n = n0 + wn * 64 + j * 16 + lr;
-                dn_put(g, dn_orow(g, row0, t, T), n, acc[i][j][e], __shfl_xor(acc[i][j][e], 1, 64), t < T && n < g.N);
-            }
+    t0 = tm * BM;
+    return t0 < T;
 }
 
-// Products that 128 x 128 tiles cannot spread over the chip (few outputs, or an inner size of a few steps): 32 tokens x 32 outputs per work-group.  Each of the NW waves takes
+template <typename WT, int BM, int BN>
+__global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p) {
+    extern __shared__ __attribute__((aligned(16))) char dn_lds[];
+    constexpr int MI = BM / 64, NJ = BN / 64, NI = (BM + BN) / 32, STAGE = (BM + BN) * 128, NS = DN_STAGES; // instruction tiles per wave, pieces a loading wave requests per block
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = (wave >> 1) & 1, wn = wave & 1;
+    const bool loads = wave >= 4;
+    const int per = 8 * p.n_tm, b_in = (int)blockIdx.x % per, wp = ((int)blockIdx.x / per) * 8 + (b_in & 7), tm = b_in >> 3;
+    if (wp >= p.tn * p.S) return;
+    const int s = wp % p.S, tn = wp / p.S;
+    int e, T, t0;
+    long long row0;
+    if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return; // (uniform per work-group)
+    const long long n0 = (long long)tn * BN, ldw = g.K * (long long)sizeof(WT);
+    const int blocks = (int)(ldw >> 7), kb0 = (int)((long long)blocks * s / p.S), nk = (int)((long long)blocks * (s + 1) / p.S) - kb0;
+    const int fr = lane & 31, fh = lane >> 5;
+    dn_f16 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    if (loads) {
+        const int lw = wave - 4, lr = lane >> 3, ls = lane & 7;
+        const char *W = (const char *)g.w + (g.g_seg ? e * g.wstride * (long long)sizeof(WT) : 0), *src[NI];
+#pragma unroll
+        for (int j = 0; j < NI; j++) {
+            const int row = 8 * (NI * lw + j) + lr, kq = ls ^ ((row >> 1) & 7);
+            const char *q;
+            if (row < BM) {
+                const int t = min(t0 + row, T - 1);
+                q = p.A ? p.A + (g.g_seg ? row0 + t : t) * p.lda : (const char *)dn_arow(g, row0, t);
+            } else {
+                const long long n = n0 + row - BM;
+                q = W + (n < g.N ? n : g.N - 1) * ldw;
+            }
+            src[j] = q + (long long)kb0 * 128 + kq * 16;
+        }
+        const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)dn_lds + (unsigned)(NI * lw * 1024);
+        auto request = [&](const int kb) {
+            if (kb >= nk) return;
+#pragma unroll
+            for (int j = 0; j < NI; j++) dn_dma(src[j] + (long long)kb * 128, lds0 + (unsigned)((kb % NS) * STAGE + j * 1024));
+        };
+        request(0);
+        request(1);
+        request(2);
+        for (int kb = 0; kb < nk; kb++) {
+            const int later = nk - 1 - kb; // blocks requested behind this one: at most NS - 2
+            if (later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * NI) : "memory");
+            else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NI) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            request(kb + NS - 1);
+        }
+    } else {
+        const int fx = (fr >> 1) & 7;
+        const char *fa0 = dn_lds + (wm * MI * 32 + fr) * 128, *fb0 = dn_lds + (BM + wn * NJ * 32 + fr) * 128;
+        dn_f4 xa[2][2][MI], xb[2][2][NJ]; // the fragments of half a block, two sets: the next half is read while this one is multiplied
+        auto read = [&](const int kb, const int half) {
+            const char *fa = fa0 + (kb % NS) * STAGE, *fb = fb0 + (kb % NS) * STAGE;
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int po = ((4 * half + 2 * u + fh) ^ fx) << 4; // (the row bases are multiples of 32: (row / 2) % 8 = (fr / 2) % 8)
+#pragma unroll
+                for (int i = 0; i < MI; i++) xa[half][u][i] = *(const dn_f4 *)(fa + i * 32 * 128 + po);
+#pragma unroll
+                for (int j = 0; j < NJ; j++) xb[half][u][j] = *(const dn_f4 *)(fb + j * 32 * 128 + po);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto block = [&]() { // the reads of the block before are done; the next block is there
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        auto multiply = [&](const int half) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                if constexpr (sizeof(WT) == 2) {
+#pragma unroll
+                    for (int i = 0; i < MI; i++)
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) {
+                            dn_bf8 za, zb;
+                            __builtin_memcpy(&za, &xa[half][u][i], 16);
+                            __builtin_memcpy(&zb, &xb[half][u][j], 16);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(za, zb, acc[i][j], 0, 0, 0);
+                        }
+                } else {
+#pragma unroll
+                    for (int x = 0; x < 4; x++)
+#pragma unroll
+                        for (int i = 0; i < MI; i++)
+#pragma unroll
+                            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[half][u][i][x], xb[half][u][j][x], acc[i][j], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        block();
+        read(0, 0);
+        for (int kb = 0; kb < nk; kb++) {
+            read(kb, 1);
+            multiply(0);
+            if (kb + 1 < nk) {
+                block();
+                read(kb + 1, 0);
+            }
+            multiply(1);
+        }
+        if (p.S > 1) {
+            float *o = p.part + ((long long)(tm * p.tn + tn) * p.S + s) * (MI * NJ * 4096);
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        *(dn_f4 *)(o + (((i * NJ + j) * 4 + q) * 256 + tid) * 4) = dn_f4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        }
+    }
+    if (p.S > 1) return;
+    // the tile through LDS (the stages are done with), so that a thread has four neighbouring outputs of a row
+    constexpr int LD = BN + 4;
+    float *tile = (float *)dn_lds;
+    __syncthreads();
+    if (!loads) {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) tile[(wm * MI * 32 + i * 32 + 8 * (r >> 2) + 4 * fh + (r & 3)) * LD + wn * NJ * 32 + j * 32 + fr] = acc[i][j][r];
+    }
+    __syncthreads();
+    const int c = (tid % (BN / 4)) * 4;
+    for (int r = tid / (BN / 4); r < BM; r += 512 / (BN / 4)) {
+        if (t0 + r >= T) break;
+        dn_put4(g, dn_orow(g, row0, t0 + r, T), n0 + c, *(const dn_f4 *)&tile[r * LD + c]);
+    }
+}
+
+// the splits of a tile, added in order: one work-group per 32 x 32 instruction tile of every wave
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p) {
+    constexpr int MI = BM / 64, NJ = BN / 64, IJ = MI * NJ;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, ij = (int)blockIdx.x % IJ, tile = (int)blockIdx.x / IJ, tm = tile / p.tn, tn = tile % p.tn;
+    int e, T, t0;
+    long long row0;
+    if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return;
+    const float *src = p.part + (long long)tile * p.S * (IJ * 4096) + ij * 4096 + tid * 4;
+    dn_f16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.f;
+    for (int s = 0; s < p.S; s += 4) { // (sixteen loads in flight)
+        dn_f4 v[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[u][q] = *(const dn_f4 *)(src + (long long)min(s + u, p.S - 1) * (IJ * 4096) + q * 1024);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (s + u < p.S)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) acc[4 * q + x] += v[u][q][x];
+    }
+    dn_put16(g, row0, T, t0 + wm * MI * 32 + (ij / NJ) * 32 + 4 * (lane >> 5), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + (lane & 31), acc);
+}
+
+// Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
+// of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more; rounds of 256 work-groups (one per CU);
+// a split product pays a second launch and its parts' way through memory.
+struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
+static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int groups, bool bf, bool may_split) {
+    static const int shapes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
+    const int64_t blocks = kbytes / 128;
+    dn_ring_shape best{};
+    double least = 0;
+    for (auto &q : shapes) {
+        const int BM = q[0], BN = q[1], full = (rows + BM - 1) / BM, n_tm = rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0), tn = (int)((N + BN - 1) / BN);
+        const int64_t tiles = (int64_t)(groups > 0 ? std::max(full, std::min(groups, rows)) + (rows > groups * BM ? groups / 2 : 0) : n_tm) * tn; // (grouped: about half of the last tiles start a new one)
+        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = std::max(lds, mfma) + 100;
+        for (int64_t S = 1; S <= (may_split ? 16 : 1); S++) {
+            if (S > 1 && (blocks / S < 4 || tiles * S > 512 || (size_t)n_tm * tn * S * BM * BN * 4 > psk_dense_split_bytes())) break;
+            const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
+            if (!best.BM || t < least) { least = t; best = dn_ring_shape{BM, BN, n_tm, tn, (int)S}; }
+        }
+    }
+    return best;
+}
+
+template <typename WT, int BM, int BN>
+static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
+    constexpr int LDS = DN_STAGES * (BM + BN) * 128;
+    static unsigned long long mask = 0;
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    const unsigned grid = (unsigned)((p.tn * p.S + 7) / 8 * 8) * p.n_tm;
+    hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN>), dim3(grid), dim3(512), LDS, st, g, p);
+    if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64))), dim3(256), 0, st, g, p);
+}
+
+// the wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed
+template <typename WT>
+static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
+    const int64_t kbytes = g.K * (int64_t)sizeof(WT);
+    if (a.force_tiled || kbytes % 128 || !a.pack) return false;
+    const bool plain = sizeof(WT) == 4 && !g.mu && !g.g_scale && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0;
+    if (!plain && (size_t)a.T * kbytes > a.pack_bytes) return false;
+    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes());
+    dn_ring p{plain ? nullptr : (const char *)a.pack, kbytes, r.n_tm, r.tn, r.S, a.split};
+    if (!plain) {
+        const int64_t pb = ((int64_t)a.T * (g.K / 8) + 255) / 256;
+        hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192)), dim3(256), 0, st, g, (WT *)a.pack);
+    }
+    if (r.BM == 128) dn_launch_ring<WT, 128, 128>(st, g, p);
+    else if (r.BN == 128) dn_launch_ring<WT, 64, 128>(st, g, p);
+    else dn_launch_ring<WT, 64, 64>(st, g, p);
+    return true;
+}
+
+// Products with an inner size of a few steps (K <= 256: the ring would be all prologue): 32 tokens x 32 outputs per work-group.  Each of the NW waves takes
 // its share of K, its operand fragments straight from memory (the activations are rounded to bfloat16 in registers: nothing is packed beforehand), four steps of 32 in flight; the
 // partial tiles meet in LDS.  Plain rows only (no ring, no token shift, no groups).
 template <int NW>
@@ -616,15 +895,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
             return 0;
         }
         g.g_seg = a.g_seg; g.g_list = a.g_list;
-        const int Tp = (a.T + 127) / 128 * 128 + 128; // (a tile may start anywhere in the list and runs 127 rows on)
-        if (bf && !a.force_tiled && g.K % 64 == 0 && a.pack && (size_t)Tp * g.K * 2 <= a.pack_bytes) {
-            long long pb = ((long long)Tp * (g.K / 8) + 255) / 256;
-            if (pb > 8192) pb = 8192;
-            hipLaunchKernelGGL(dense_pack_kernel, dim3((unsigned)pb), dim3(256), 0, st, g, (unsigned short *)a.pack, Tp);
-            hipLaunchKernelGGL(dense_mm_fast_kernel, dim3((unsigned)((g.N + 127) / 128), (unsigned)((a.T + 127) / 128), (unsigned)a.groups), dim3(256), 0, st, g,
-                               (const unsigned short *)a.pack);
-            return 0;
-        }
+        if (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g)) return 0;
         const dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((a.T + 63) / 64), (unsigned)a.groups);
         if (bf) hipLaunchKernelGGL(dense_mm_kernel<unsigned short>, grid, dim3(256), 0, st, g);
         else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
@@ -649,21 +920,12 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
             return 0;
         }
     }
-    const int Tp = (a.T + 127) / 128 * 128;
-    if (bf && !a.force_tiled && a.T > 8 && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 &&
-        (g.K <= 256 || (g.N + 127) / 128 * (Tp / 128) < 32)) {
+    if (bf && !a.force_tiled && a.T > 8 && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 && g.K <= 256) {
         const dim3 grid((unsigned)((a.T + 31) / 32), (unsigned)((g.N + 31) / 32));
-        if (g.K % 256 == 0 && g.K >= 1024) hipLaunchKernelGGL(dense_mm_narrow_kernel<8>, grid, dim3(512), 0, st, g);
-        else hipLaunchKernelGGL(dense_mm_narrow_kernel<4>, grid, dim3(256), 0, st, g);
+        hipLaunchKernelGGL(dense_mm_narrow_kernel<4>, grid, dim3(256), 0, st, g);
         return 0;
     }
-    if (bf && !a.force_tiled && a.T > 8 && g.K % 64 == 0 && a.pack && (size_t)Tp * g.K * 2 <= a.pack_bytes) {
-        long long pb = ((long long)Tp * (g.K / 8) + 255) / 256;
-        if (pb > 8192) pb = 8192;
-        hipLaunchKernelGGL(dense_pack_kernel, dim3((unsigned)pb), dim3(256), 0, st, g, (unsigned short *)a.pack, Tp);
-        hipLaunchKernelGGL(dense_mm_fast_kernel, dim3((unsigned)((g.N + 127) / 128), (unsigned)(Tp / 128)), dim3(256), 0, st, g, (const unsigned short *)a.pack);
-        return 0;
-    }
+    if (a.T > 8 && (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g))) return 0;
     dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((a.T + 63) / 64));
     if (bf) hipLaunchKernelGGL(dense_mm_kernel<unsigned short>, grid, dim3(256), 0, st, g);
     else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
@@ -766,6 +1028,17 @@ int ps_hip_dense_matmul(ps_hip_ctx *c, const ps_dense *w, const float *x, int T,
     if (!w || T <= 0) PS_FAIL(c, "dense_matmul: bad argument");
     psk_dense_args a;
     a.w = w; a.a = x; a.lda = w->K; a.T = T; a.out = out; a.ldo = w->N; a.alpha = alpha;
+    if (T > 8) { // the wide mat-mul's scratch: the context's own, grown as needed
+        const size_t pack = ((size_t)T * w->K * (w->dtype == PS_BF16 ? 2 : 4) + 255) / 256 * 256, need = pack + psk_dense_split_bytes();
+        if (c->act_cap < need) {
+            PS_CHECK(c, hipStreamSynchronize(c->stream));
+            if (c->act_buf) (void)ps_dev_free(c->act_buf);
+            c->act_buf = nullptr; c->act_cap = 0;
+            PS_CHECK(c, ps_dev_malloc(&c->act_buf, need));
+            c->act_cap = need;
+        }
+        a.pack = c->act_buf; a.pack_bytes = pack; a.split = (float *)((char *)c->act_buf + pack); a.split_bytes = psk_dense_split_bytes();
+    }
     psk_dense(c->stream, a);
     PS_CHECK(c, hipGetLastError());
     return 0;

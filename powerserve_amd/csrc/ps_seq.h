@@ -47,8 +47,10 @@ struct psk_dense_args {
     int accum = 0; // 1: out += the result (the residual stream takes a sublayer's output projection directly)
     const float *mu = nullptr, *shift0 = nullptr;
     int force_tiled = 0; // 1: the plain tiled mat-mul whatever the shape (A/B against the mat-vec and the wide mat-mul)
-    void *pack = nullptr; // scratch for the wide mat-mul's bfloat16 copy of A (T rounded up to 128 rows of K); without it the plain tiled kernel runs
+    void *pack = nullptr; // scratch for the wide mat-mul's copy of A (T rows of K in the matrix's number format); without it the plain tiled kernel runs
     size_t pack_bytes = 0;
+    float *split = nullptr; // scratch for its splits of K (psk_dense_split_bytes); too small: K is not split
+    size_t split_bytes = 0;
     const float *out_scale = nullptr; // [T] device: row t of the result is multiplied by out_scale[t] (beside alpha)
     // ---- grouped products: w holds `groups` matrices of N / groups rows one after the other, and every row of the product belongs to one of them.
     // T counts SLOTS; slot s reads A row s / g_adiv times g_scale[s] (NULL: 1), uses matrix g_sel[s] and lands in output row s / g_odiv.
@@ -70,6 +72,7 @@ struct psk_dense_args {
     const ps_seq_step *em_step = nullptr;
 };
 int psk_dense(hipStream_t st, const psk_dense_args &a);
+size_t psk_dense_split_bytes(); // what any product's splits need at most
 void psk_dense_widen(hipStream_t st, const uint16_t *bf16, int64_t n, float *out);
 // out[t][:] = table[token(t)][:] * scale; tokens device int32 (step != NULL and T == 1: the token is step->token0)
 //   bigram given: + bigram[(prev * mul_prev + token * mul_cur) mod buckets][:], or its row `buckets` for position 0; prev = tokens[t - 1], in front of the step step->prev

@@ -73,8 +73,10 @@ struct ps_hip_seq {
     float *lstm_aux = nullptr;    // matrix memory: [max_batch][heads] products with n, then as many running maxima
     int64_t lstm_aux_n = 0;
     float *abs_scratch = nullptr; // the absorbed single-token attention's folded queries, attended latents and per-tile partials
-    void *pack = nullptr; // the wide mat-mul's bfloat16 operand copy
+    void *pack = nullptr; // the wide mat-mul's operand copy
     size_t pack_bytes = 0;
+    float *split = nullptr; // its partial tiles where K is split
+    size_t split_bytes = 0;
     int ids_cap = 0;
     int64_t n_t2q = 0; // t2: [max_batch][q_rank max] then the queries
     float *dbg_layers = nullptr;
@@ -480,16 +482,16 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         if (sb) ok = ok && alloc((void **)&m->ssd_scratch, sb);
         if (m->lstm_aux_n) ok = ok && alloc((void **)&m->lstm_aux, (size_t)m->lstm_aux_n * 2 * 4);
     }
-    if (desc->compute == 0) { // the wide mat-mul's operand copy: the widest input of any matrix x a portion's rows, or the window's rows x the latent
+    if (B > 8) { // the wide mat-mul's operand copy: the widest input of any matrix x a portion's rows (mixture of experts: slots), or the window's rows x the latent
         int64_t kmax = std::max<int64_t>(W, desc->side_dim), kvrows = 0, kvk = 0;
         mixers([&](LayerPlan &P) {
             kmax = std::max<int64_t>({kmax, P.d.ff, P.d.shared_ff, P.d.heads * (int64_t)std::max(P.d.dim, P.d.vdim), P.d.q_rank, P.d.decay_rank});
             if (P.d.kind == PS_MIX_LATENT) { kvrows = std::max<int64_t>(kvrows, P.d.window - 1 + B); kvk = std::max<int64_t>(kvk, P.d.kv_rank); }
         });
-        // (a grouped product packs its slots in list order and a tile may start anywhere in the list: one tile of rows more)
-        const int64_t r128 = std::max((B + 127) / 128 * 128, moe_slots ? (moe_slots + 127) / 128 * 128 + 128 : 0), kv128 = (kvrows + 127) / 128 * 128;
-        m->pack_bytes = (size_t)std::max(r128 * kmax, kv128 * kvk) * 2;
-        ok = ok && alloc(&m->pack, m->pack_bytes);
+        // (fp32: only the token-shift mixes and scaled slots are packed, the window's rows are read in place)
+        m->pack_bytes = desc->compute == 0 ? (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * 2 : (size_t)(std::max(B, moe_slots) * W) * 4;
+        m->split_bytes = psk_dense_split_bytes();
+        ok = ok && alloc(&m->pack, m->pack_bytes) && alloc((void **)&m->split, m->split_bytes);
     }
     m->slot_state.assign(desc->n_slots, nullptr);
     m->slot_pos.assign(desc->n_slots, -1);
@@ -550,7 +552,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
               D.bigram_mul_cur);
     auto mm = [&](const ps_dense *w, const float *a, int64_t lda, float *out, int64_t ldo) {
         psk_dense_args g;
-        g.w = w; g.a = a; g.lda = lda; g.T = T; g.out = out; g.ldo = ldo; g.force_tiled = tiled; g.pack = m->pack; g.pack_bytes = m->pack_bytes;
+        g.w = w; g.a = a; g.lda = lda; g.T = T; g.out = out; g.ldo = ldo; g.force_tiled = tiled; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
         return g;
     };
     // a sublayer boundary: x += norm_b(y) (after a sublayer), then hn = norm(x), h = conv(hn) (in front of the next one); one launch for a single token
@@ -889,7 +891,7 @@ static void seq_head(ps_hip_seq *m, const int32_t *idx, int rows) {
         psk_rmsnorm(st, m->x, D.width, idx, D.final_norm, D.norm_offset, D.norm_eps, D.width, rows, m->xn, D.width, m->groups);
     }
     psk_dense_args g;
-    g.w = D.head; g.a = m->xn; g.lda = D.width; g.T = rows; g.out = m->logits; g.ldo = D.vocab; g.alpha = D.logit_scale; g.force_tiled = (m->mode & 2) != 0; g.pack = m->pack; g.pack_bytes = m->pack_bytes;
+    g.w = D.head; g.a = m->xn; g.lda = D.width; g.T = rows; g.out = m->logits; g.ldo = D.vocab; g.alpha = D.logit_scale; g.force_tiled = (m->mode & 2) != 0; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
     if (D.logit_softcap > 0.f) { g.act = PSD_ACT_SOFTCAP; g.act_p = D.logit_softcap; }
     psk_dense(st, g);
     psk_argmax_rows(st, m->logits, D.vocab, rows, m->amax);
@@ -1003,7 +1005,7 @@ int ps_hip_seq_bench_kernel(ps_hip_seq *m, int which, int T, int reps, double *u
         const bool is_moe = P.d.ff_kind == PS_FF_MOE_SWIGLU || P.d.ff_kind == PS_FF_MOE_RELU2;
         if (P.d.ff_kind == PS_FF_NONE || is_moe != moe) continue;
         psk_dense_args g;
-        g.T = T; g.pack = m->pack; g.pack_bytes = m->pack_bytes;
+        g.T = T; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
         if (moe) {
             // the routing of this layer (all layers' launches below then reuse the LAST layer's routing: the same shapes and spread)
             const int top = P.d.top, S = T * top;

@@ -98,6 +98,32 @@ def test_dense_matmul_any_shape(ctx, dtype, T, N, K):
     dx.free(); do.free()
 
 
+# the wide mat-mul (k_dense.hip dense_mm_ring_kernel): one row more and less than its tiles of 64 and 128 tokens and outputs, one block of K and fewer blocks than stages,
+# products split along K (few tiles, long K: also uneven shares), more tiles than the chip has CUs
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,N,K", [(9, 1, 64), (63, 127, 128), (64, 128, 192), (65, 129, 256), (127, 63, 320), (128, 65, 576), (129, 200, 64), (300, 130, 1088), (16, 8, 4096), (40, 100, 4160),
+                                   (200, 256, 2240), (520, 2100, 128)])
+def test_dense_matmul_wide(ctx, dtype, T, N, K):
+    import ctypes as C
+    rng = np.random.default_rng(T * 1000 + N)
+    bits = f32_to_bf16_bits(rng.standard_normal((N, K), dtype=np.float32))
+    rnd = lambda a: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(a.shape)
+    x = rng.standard_normal((T, K), dtype=np.float32)
+    w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K)
+    h = C.c_void_p()
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, int(dtype == "float32"), C.byref(h)))
+    dx, do = ctx.to_device(x), ctx.to_device(np.full((T + 1, N), np.float32(7.0)))
+    ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, h, dx.ptr, T, do.ptr, 1.0))
+    got = do.numpy()
+    a = (x if dtype == "float32" else rnd(x)).astype(np.float64)
+    # fp32 sums of K products, in any order: at most K roundings of 2^-24, each relative to a partial sum of at most sum |a w|
+    bound = K * 2.0 ** -24 * (np.abs(a) @ np.abs(w.astype(np.float64)).T)
+    assert np.all(np.abs(got[:T] - a @ w.astype(np.float64).T) <= bound)
+    assert np.all(got[T] == 7.0)  # nothing behind the last row
+    ctx.L.ps_hip_dense_free(ctx.h, h)
+    dx.free(); do.free()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["wkv", "delta", "latent", "ff", "mixed", "aligned", "wide_heads"])
 def test_whole_prompt_against_the_plain_statement(made, name, dtype):
