@@ -137,30 +137,32 @@ void psk_latent_attn(hipStream_t st, const ps_seq_step *step, int64_t ring_off, 
 // One wave attends 16 rows to tiles of 16 keys, fp32 throughout on v_mfma_f32_16x16x4_f32:
 //   scores   S[16 x 16] = Q[16 x DK] K^T: the keys come straight from memory as 16-byte pieces (lane (key l % 16, quarter l / 16) holds 4
 //            consecutive dimensions; the row operand is read from LDS in the same order, so the sum runs over a permutation of the dimensions)
-//   soft-max online, in the accumulator layout (lane holds rows 4 (l / 16) + i of key column l % 16; a row's 16 lanes reduce by butterfly)
+//   soft-max online, in the accumulator layout (lane holds rows 4 (l / 16) + i of key column l % 16; a row's 16 lanes reduce by rotations)
 //   output   O[16 x DV] += P V: P goes through a 16 x 17 LDS patch into the row-operand layout; V comes as 16-byte pieces of 4 consecutive
 //            columns, so accumulator tile jj of a 64-column group holds columns 4 (l % 16) + jj -- undone at the final store.
 // A "row" is a (token, head) pair.  Two drivers use it: a prompt's portion over per-head keys / values expanded from the ring (rows = 16
 // consecutive tokens of one head), and the single-token step in the ABSORBED form -- rows = heads, every head's query folded through its key
 // expansion into latent space (q~_h = W_uk,h^T q_h), keys AND values the ring's latents themselves, the value expansion applied afterwards to
 // the attended latent -- where the ring is read once for all heads and nothing is expanded per key.
-// a prompt's portion: block = 64 consecutive tokens of one head (a wave per 16), keys / values expanded per head in kv (position first + row)
-// dynamic LDS: 4 x (16 x qld + 16 x 17)
-template <int NJ>
-__global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const ps_seq_step *step, long long ring_off, int cap, const float *q, long long ldq, const float *kv,
+// A prompt's portion: block = RT x 16 consecutive tokens of one head, keys / values expanded per head in kv (position first + row).  The key tiles are dealt to the block's eight waves,
+// each with its own running soft-max, and the eight partial results are merged at the end (la_merge).  What bounded the form before (a wave per 16 tokens over all its keys: 512 waves for
+// 512 tokens of 16 heads, one per SIMD on half the chip) was the latency of a key tile -- its keys, its soft-max, its values, one behind the other: 270 us per 512 tokens behind a
+// 1024-token window where the matrix instructions need 35.  Now every SIMD has two waves and a key piece serves two row tiles: 80 us.
+// dynamic LDS: RT x 16 x qld + 8 x RT x 16 x 17 floats, then the merge's slots over them
+template <int NJ, int RT>
+__global__ __launch_bounds__(512) void latent_attn_mfma_kernel(const ps_seq_step *step, long long ring_off, int cap, const float *q, long long ldq, const float *kv,
                                                                long long ldkv, const float *freq, int H, int d, int dr, int rot_dims, int dv, int kv_rank, int window,
                                                                float scale, int T, float *o, long long ldo, float rot_mag, const float *gate, long long ldg, int pairing) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4, h = blockIdx.y;
     const int qld = d + dr + 4;
-    float *qs = lds + wave * (16 * qld + 16 * 17), *pt = qs + 16 * qld;
+    float *qs = lds, *pt = lds + RT * 16 * qld + wave * RT * 16 * 17;
     const long long pos0 = step->pos0;
-    const int t0 = blockIdx.x * 64 + wave * 16;
-    if (t0 >= T) return; // (no block-wide barrier below: waves are on their own)
+    const int t0 = blockIdx.x * 16 * RT;
     const long long first = pos0 - window + 1 > 0 ? pos0 - window + 1 : 0;
     const int half = rot_dims / 2;
-    // this wave's 16 query rows into LDS (no index division, one sincos per rotated pair and row)
-    for (int r = 0; r < 16; r++) {
+    // the block's query rows into LDS (no index division, one sincos per rotated pair and row)
+    for (int r = wave; r < 16 * RT; r += 8) {
         const int t = t0 + r;
         const bool in = t < T;
         const float *qt = q + (long long)(in ? t : 0) * ldq + (long long)h * (d + dr);
@@ -176,47 +178,53 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const ps_seq_step
             qr[d + pb] = v * cs + u * sn;
         }
     }
-    __builtin_amdgcn_wave_barrier();
-    const la_src k1 = {kv + (long long)h * d, ldkv, first, 0};
-    const la_src k2 = {step->state + ring_off + kv_rank, (long long)(kv_rank + dr), 0, cap};
-    const la_src vs = {kv + (long long)H * d + (long long)h * dv, ldkv, first, 0};
-    long long rowlo[4], rowhi[4];
-    float m[4], l[4];
-    la_f4 acc[NJ];
+    __syncthreads();
+    // keys counted from position `first`
+    const la_src k1 = {kv + (long long)h * d, ldkv, 0, 0}, vs = {kv + (long long)H * d + (long long)h * dv, ldkv, 0, 0};
+    const la_src k2 = la_ring(step->state + ring_off + kv_rank, kv_rank + dr, first, cap);
+    float m[RT][4], l[RT][4];
+    la_f4 acc[RT][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const long long rp = pos0 + t0 + 4 * lq + i;
-        const bool in = t0 + 4 * lq + i < T;
-        rowlo[i] = in && rp - window + 1 > 0 ? rp - window + 1 : 0;
-        rowhi[i] = in ? rp + 1 : 0;
-        m[i] = -INFINITY; l[i] = 0.f;
+    for (int r = 0; r < RT; r++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) { m[r][i] = -INFINITY; l[r][i] = 0.f; }
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[r][j] = la_f4{0.f, 0.f, 0.f, 0.f};
     }
+    const la_window see{(int)(pos0 - first) + t0, window, T - t0, lq, 0.f};
+    const int last = see.q0 + min(16 * RT, T - t0) - 1, lo = see.q0 - window + 1 > 0 ? see.q0 - window + 1 : 0;
+    for (int j0 = lo + 16 * wave; j0 <= last; j0 += 128) la_tiles<NJ, RT, false>(qs, qld, pt, k1, k2, vs, d, dr, dv, j0, last + 1, see, scale, m, l, acc);
+    la_merge8<NJ, RT>(lds, m, l, acc);
+    if (wave) return;
 #pragma unroll
-    for (int j = 0; j < NJ; j++) acc[j] = la_f4{0.f, 0.f, 0.f, 0.f};
-    const long long plast = pos0 + (t0 + 15 < T ? t0 + 15 : T - 1), pfirst = pos0 + t0;
-    const long long lo = pfirst - window + 1 > 0 ? pfirst - window + 1 : 0;
-    for (long long j0 = lo; j0 <= plast; j0 += 16) la_tile<NJ>(qs, qld, pt, k1, k2, vs, d, dr, dv, j0, plast + 1, rowlo, rowhi, scale, m, l, acc);
+    for (int r = 0; r < RT; r++)
 #pragma unroll
-    for (int J = 0; J < NJ / 4; J++)
+        for (int J = 0; J < NJ / 4; J++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) { // a lane's four tiles of a 64-column group are four consecutive columns: one 16-byte store
-            const int t = t0 + 4 * lq + i, c = 64 * J + 4 * lr;
-            if (t < T && c < dv) {
-                const float il = (gate ? 1.f / (1.f + expf(-gate[(long long)t * ldg + h])) : 1.f) / l[i];
-                *(la_f4 *)(o + (long long)t * ldo + (long long)h * dv + c) = la_f4{acc[4 * J][i] * il, acc[4 * J + 1][i] * il, acc[4 * J + 2][i] * il, acc[4 * J + 3][i] * il};
+            for (int i = 0; i < 4; i++) { // a lane's four tiles of a 64-column group are four consecutive columns: one 16-byte store
+                const int t = t0 + 16 * r + 4 * lq + i, c = 64 * J + 4 * lr;
+                if (t < T && c < dv) {
+                    const float il = (gate ? 1.f / (1.f + expf(-gate[(long long)t * ldg + h])) : 1.f) / l[r][i];
+                    *(la_f4 *)(o + (long long)t * ldo + (long long)h * dv + c) = la_f4{acc[r][4 * J][i] * il, acc[r][4 * J + 1][i] * il, acc[r][4 * J + 2][i] * il, acc[r][4 * J + 3][i] * il};
+                }
             }
-        }
 }
-
-bool psk_latent_attn_mfma_ok(int d, int dr, int dv) { return d % 16 == 0 && dr % 16 == 0 && dv % 4 == 0 && dv <= 128 && (size_t)4 * (16 * (d + dr + 4) + 16 * 17) * 4 <= 160 * 1024; }
+bool psk_latent_attn_mfma_ok(int d, int dr, int dv) { return d % 16 == 0 && dr % 16 == 0 && dv % 4 == 0 && dv <= 128 && la_portion_lds<8, 1>(d + dr) <= 160 * 1024; }
+template <int RT>
+static void la_launch_latent(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int64_t ldq, const float *kv, int64_t ldkv, const float *freq, int H, int d,
+                             int dr, int rot_dims, int dv, int kv_rank, int window, float scale, int T, float *o, int64_t ldo, float rot_mag, const float *gate, int64_t ldg, int pairing) {
+    static unsigned long long mask = 0;
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)latent_attn_mfma_kernel<8, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    hipLaunchKernelGGL((latent_attn_mfma_kernel<8, RT>), dim3((T + 16 * RT - 1) / (16 * RT), H), dim3(512), (la_portion_lds<8, RT>(d + dr)), st, step, (long long)ring_off, cap, q, (long long)ldq, kv,
+                       (long long)ldkv, freq, H, d, dr, rot_dims, dv, kv_rank, window, scale, T, o, (long long)ldo, rot_mag, gate, (long long)ldg, pairing);
+}
 void psk_latent_attn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int64_t ldq, const float *kv, int64_t ldkv,
                           const float *freq, int H, int d, int dr, int rot_dims, int dv, int kv_rank, int window, float scale, int T, float *o, int64_t ldo, float rot_mag,
                           const float *gate, int64_t ldg, int pairing) {
-    const size_t lds = (size_t)4 * (16 * (d + dr + 4) + 16 * 17) * 4;
-    static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)latent_attn_mfma_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    hipLaunchKernelGGL(latent_attn_mfma_kernel<8>, dim3((T + 63) / 64, H), dim3(256), lds, st, step, (long long)ring_off, cap, q, (long long)ldq, kv, (long long)ldkv, freq,
-                       H, d, dr, rot_dims, dv, kv_rank, window, scale, T, o, (long long)ldo, rot_mag, gate, (long long)ldg, pairing);
+    if (la_two_tiles(T, H, la_portion_lds<8, 2>(d + dr)))
+        la_launch_latent<2>(st, step, ring_off, cap, q, ldq, kv, ldkv, freq, H, d, dr, rot_dims, dv, kv_rank, window, scale, T, o, ldo, rot_mag, gate, ldg, pairing);
+    else
+        la_launch_latent<1>(st, step, ring_off, cap, q, ldq, kv, ldkv, freq, H, d, dr, rot_dims, dv, kv_rank, window, scale, T, o, ldo, rot_mag, gate, ldg, pairing);
 }
 
 // ---------------------------------------------------------------------------------------------------- single token, absorbed
@@ -291,26 +299,26 @@ __global__ __launch_bounds__(256) void latent_absorbed_kernel(const ps_seq_step 
     __syncthreads();
     const long long tile = (long long)blockIdx.x * 4 + wave, j0 = lo + tile * 16;
     const float *ring = step->state + ring_off;
-    const la_src k1 = {ring, (long long)(R + dr), 0, cap}, k2 = {ring + R, (long long)(R + dr), 0, cap};
-    long long rowlo[4], rowhi[4];
-    float m[4], l[4];
-    la_f4 acc[NJ];
+    const la_src k1 = la_ring(ring, R + dr, lo, cap), k2 = la_ring(ring + R, R + dr, lo, cap); // keys counted from position lo
+    struct { int rows, lq; __device__ __forceinline__ bool sees(int, int i, int) const { return 4 * lq + i < rows; } } see{H - h0, lq};
+    float m[1][4], l[1][4];
+    la_f4 acc[1][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; i++) { rowlo[i] = h0 + 4 * lq + i < H ? lo : 0; rowhi[i] = h0 + 4 * lq + i < H ? p + 1 : 0; m[i] = -INFINITY; l[i] = 0.f; }
+    for (int i = 0; i < 4; i++) { m[0][i] = -INFINITY; l[0][i] = 0.f; }
 #pragma unroll
-    for (int j = 0; j < NJ; j++) acc[j] = la_f4{0.f, 0.f, 0.f, 0.f};
-    if (j0 <= p) la_tile<NJ>(qs, qld, pt, k1, k2, k1, R, dr, R, j0, p + 1, rowlo, rowhi, scale, m, l, acc);
+    for (int j = 0; j < NJ; j++) acc[0][j] = la_f4{0.f, 0.f, 0.f, 0.f};
+    if (j0 <= p) la_tiles<NJ, 1, false>(qs, qld, pt, k1, k2, k1, R, dr, R, (int)(j0 - lo), (int)(p - lo) + 1, see, scale, m, l, acc);
     // partial of (tile, head): [o[R], m, l, -, -] (rows of R + 4 floats: 16-byte stores)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int h = h0 + 4 * lq + i;
         if (h >= H) continue;
         float *pp = part + ((long long)tile * H + h) * (R + 4);
-        if (lr == 0) { pp[R] = m[i]; pp[R + 1] = l[i]; }
+        if (lr == 0) { pp[R] = m[0][i]; pp[R + 1] = l[0][i]; }
 #pragma unroll
         for (int J = 0; J < NJ / 4; J++) {
             const int c = 64 * J + 4 * lr;
-            if (c < R) *(la_f4 *)(pp + c) = la_f4{acc[4 * J][i], acc[4 * J + 1][i], acc[4 * J + 2][i], acc[4 * J + 3][i]};
+            if (c < R) *(la_f4 *)(pp + c) = la_f4{acc[0][4 * J][i], acc[0][4 * J + 1][i], acc[0][4 * J + 2][i], acc[0][4 * J + 3][i]};
         }
     }
 }

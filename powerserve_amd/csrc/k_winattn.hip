@@ -9,7 +9,7 @@
 //   winattn_prep_kernel    norms over the whole q / k projections, rotation, ring append            (one or a few blocks per token)
 //   winattn_pool_kernel    block sums in position order, turned into means when a block is complete  (a thread per channel and block)
 //   winattn_kernel         one wave per (token, head) over [front store | window]: the plain form, any size
-//   winattn_mfma_kernel    a portion on the fp32 matrix cores, 16 tokens of a head per wave (ps_attn_dev.h)
+//   winattn_mfma_kernel    a portion on the fp32 matrix cores, 32 tokens of a head per block, the keys dealt to its waves (ps_attn_dev.h)
 //   winattn_step_kernel + winattn_merge_kernel   a single token: rows = the heads that share a key / value group, a key tile per wave
 #include "ps_attn_dev.h"
 #include "ps_seq.h"
@@ -226,91 +226,101 @@ void psk_winattn(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int 
                        gate, (long long)ldg, temp, sink, H, G, d, dv, window, scale, o, (long long)ldo, softcap, gate_elem, slope);
 }
 
-// ---------------------------------------------------------------------------------------------------- matrix-core forms (ps_attn_dev.h)
-// A portion: block = 64 consecutive tokens of one head (a wave per 16).  The visible front rows first (key index = block or position), then the window's ring rows
-// (key index = position), one online soft-max over both.  dynamic LDS: 4 x (16 x (d + 4) + 16 x 17)
-template <int NJ, bool DIST>
-__global__ __launch_bounds__(256) void winattn_mfma_kernel(const ps_seq_step *step, long long ring_off, int cap, long long store_off, int pool, int keep, const float *q, long long ldq,
+// what the rows of a portion's block (tokens pfirst + n) see of the front store: the first wa_front rows (ps_attn_dev.h)
+struct wa_fronts {
+    long long pfirst;
+    int window, pool, keep, rows, lq;
+    float slope;
+    __device__ __forceinline__ bool sees(int r, int i, int j) const {
+        const int n = 16 * r + 4 * lq + i;
+        const long long out = pfirst + n - window + 1; // positions in front of the row's window
+        return n < rows && (pool > 0 ? (long long)(j + 1) * pool <= out : j < out && j < keep);
+    }
+    __device__ __forceinline__ float minus(int r, int i, int j) const { return slope * (float)(pfirst + 16 * r + 4 * lq + i - j); }
+};
+// A portion: block = RT x 16 consecutive tokens of one head, the key tiles -- the visible front rows', then the window's -- dealt to its eight waves, the eight results merged
+// (k_latent.hip latent_attn_mfma_kernel is the same form: what bounded the wave-per-16-tokens one before it stands there; 280 -> 70 us per 512 tokens behind 1024 + 64 keys).
+// dynamic LDS: la_portion_lds
+template <int NJ, int RT, bool DIST>
+__global__ __launch_bounds__(512) void winattn_mfma_kernel(const ps_seq_step *step, long long ring_off, int cap, long long store_off, int pool, int keep, const float *q, long long ldq,
                                                            const float *gate, long long ldg, const float *temp, const float *sink, int H, int G, int d, int dv, int window,
                                                            float scale, int T, float *o, long long ldo, float softcap, int gate_elem, const float *slope) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4, h = blockIdx.y, g = h / (H / G);
     const int qld = d + 4;
-    float *qs = lds + wave * (16 * qld + 16 * 17), *pt = qs + 16 * qld;
+    float *qs = lds, *pt = lds + RT * 16 * qld + wave * RT * 16 * 17;
     const long long pos0 = step->pos0;
-    const int t0 = blockIdx.x * 64 + wave * 16;
-    if (t0 >= T) return; // (no block-wide barrier below: waves are on their own)
-    for (int r = 0; r < 16; r++) {
+    const int t0 = blockIdx.x * 16 * RT;
+    for (int r = wave; r < 16 * RT; r += 8) {
         const int t = t0 + r;
         const float *qt = q + (long long)(t < T ? t : 0) * ldq + (long long)h * d;
         for (int c = lane; c < d; c += 64) qs[r * qld + c] = t < T ? qt[c] : 0.f;
     }
-    __builtin_amdgcn_wave_barrier();
+    __syncthreads();
     const long long rs = (long long)G * (d + dv);
     const float *ring = step->state + ring_off, *means = step->state + store_off;
     const float sc = scale * (temp ? temp[h] : 1.f);
-    long long rowlo[4], rowhi[4], blo[4], bhi[4], qpos[4];
-    float m[4], l[4], sl[4];
-    la_f4 acc[NJ];
+    float m[RT][4], l[RT][4];
+    la_f4 acc[RT][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const long long rp = pos0 + t0 + 4 * lq + i;
-        const bool in = t0 + 4 * lq + i < T;
-        rowlo[i] = in && rp - window + 1 > 0 ? rp - window + 1 : 0;
-        rowhi[i] = in ? rp + 1 : 0;
-        blo[i] = 0;
-        bhi[i] = in ? wa_front(rp, window, pool, keep) : 0;
-        qpos[i] = rp;
-        sl[i] = DIST ? slope[h] : 0.f;
-        m[i] = -INFINITY; l[i] = 0.f;
+    for (int r = 0; r < RT; r++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) { m[r][i] = -INFINITY; l[r][i] = 0.f; }
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[r][j] = la_f4{0.f, 0.f, 0.f, 0.f};
     }
-#pragma unroll
-    for (int j = 0; j < NJ; j++) acc[j] = la_f4{0.f, 0.f, 0.f, 0.f};
-    const long long plast = pos0 + (t0 + 15 < T ? t0 + 15 : T - 1), pfirst = pos0 + t0;
-    const long long nbmax = wa_front(plast, window, pool, keep);
+    const int rows = min(16 * RT, T - t0);
+    const long long pfirst = pos0 + t0, lo = pfirst - window + 1 > 0 ? pfirst - window + 1 : 0;
+    const int nbmax = (int)wa_front(pfirst + rows - 1, window, pool, keep), nbt = (nbmax + 15) / 16;
+    int tile = wave;
     {
         const la_src k1 = {means + (long long)g * d, rs, 0, 0}, vs = {means + (long long)G * d + (long long)g * dv, rs, 0, 0};
-        for (long long j0 = 0; j0 < nbmax; j0 += 16) la_tile<NJ, DIST>(qs, qld, pt, k1, k1, vs, d, 0, dv, j0, nbmax, blo, bhi, sc, m, l, acc, softcap, sl, qpos);
+        const wa_fronts see{pfirst, window, pool, keep, rows, lq, DIST ? slope[h] : 0.f};
+        for (; tile < nbt; tile += 8) la_tiles<NJ, RT, DIST>(qs, qld, pt, k1, k1, vs, d, 0, dv, 16 * tile, nbmax, see, sc, m, l, acc, softcap);
     }
     {
-        const la_src k1 = {ring + (long long)g * d, rs, 0, cap}, vs = {ring + (long long)G * d + (long long)g * dv, rs, 0, cap};
-        const long long lo = pfirst - window + 1 > 0 ? pfirst - window + 1 : 0;
-        for (long long j0 = lo; j0 <= plast; j0 += 16) la_tile<NJ, DIST>(qs, qld, pt, k1, k1, vs, d, 0, dv, j0, plast + 1, rowlo, rowhi, sc, m, l, acc, softcap, sl, qpos);
+        const la_src k1 = la_ring(ring + (long long)g * d, rs, lo, cap), vs = la_ring(ring + (long long)G * d + (long long)g * dv, rs, lo, cap);
+        const la_window see{(int)(pfirst - lo), window, rows, lq, DIST ? slope[h] : 0.f};
+        for (int j0 = 16 * (tile - nbt); j0 < see.q0 + rows; j0 += 128) la_tiles<NJ, RT, DIST>(qs, qld, pt, k1, k1, vs, d, 0, dv, j0, see.q0 + rows, see, sc, m, l, acc, softcap);
     }
+    la_merge8<NJ, RT>(lds, m, l, acc);
+    if (wave) return;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int t = t0 + 4 * lq + i;
-        if (t >= T) continue;
-        const float f = wa_finish(m[i], l[i], sink, h) * (gate && !gate_elem ? wa_sigmoid(gate[(long long)t * ldg + h]) : 1.f);
+    for (int r = 0; r < RT; r++)
 #pragma unroll
-        for (int J = 0; J < NJ / 4; J++) { // a lane's four tiles of a 64-column group are four consecutive columns: one 16-byte store
-            const int c = 64 * J + 4 * lr;
-            if (c >= dv) continue;
-            la_f4 r = la_f4{acc[4 * J][i] * f, acc[4 * J + 1][i] * f, acc[4 * J + 2][i] * f, acc[4 * J + 3][i] * f};
-            if (gate && gate_elem) {
-                const float *gp = gate + (long long)t * ldg + (long long)h * dv + c;
+        for (int i = 0; i < 4; i++) {
+            const int t = t0 + 16 * r + 4 * lq + i;
+            if (t >= T) continue;
+            const float f = wa_finish(m[r][i], l[r][i], sink, h) * (gate && !gate_elem ? wa_sigmoid(gate[(long long)t * ldg + h]) : 1.f);
 #pragma unroll
-                for (int e = 0; e < 4; e++) r[e] *= wa_sigmoid(gp[e]);
+            for (int J = 0; J < NJ / 4; J++) { // a lane's four tiles of a 64-column group are four consecutive columns: one 16-byte store
+                const int c = 64 * J + 4 * lr;
+                if (c >= dv) continue;
+                la_f4 v = la_f4{acc[r][4 * J][i] * f, acc[r][4 * J + 1][i] * f, acc[r][4 * J + 2][i] * f, acc[r][4 * J + 3][i] * f};
+                if (gate && gate_elem) {
+                    const float *gp = gate + (long long)t * ldg + (long long)h * dv + c;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] *= wa_sigmoid(gp[e]);
+                }
+                *(la_f4 *)(o + (long long)t * ldo + (long long)h * dv + c) = v;
             }
-            *(la_f4 *)(o + (long long)t * ldo + (long long)h * dv + c) = r;
         }
-    }
 }
-
-static size_t wa_mfma_lds(int d) { return (size_t)4 * (16 * (d + 4) + 16 * 17) * 4; }
-// the sizes the matrix-core forms take: 16-byte pieces of keys (d a multiple of 16) and values (dv of 4, at most 128 columns per head)
-bool psk_winattn_mfma_ok(int d, int dv) { return d % 16 == 0 && dv % 4 == 0 && dv <= 128 && wa_mfma_lds(d) <= 160 * 1024; }
+bool psk_winattn_mfma_ok(int d, int dv) { return d % 16 == 0 && dv % 4 == 0 && dv <= 128 && la_portion_lds<8, 1>(d) <= 160 * 1024; }
+template <int RT, bool DIST>
+static void wa_launch_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, psk_front_store fs, const float *q, int64_t ldq, const float *gate, int64_t ldg, const float *temp,
+                           const float *sink, int H, int G, int d, int dv, int window, float scale, int T, float *o, int64_t ldo, float softcap, int gate_elem, const float *slope) {
+    static unsigned long long mask = 0;
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)winattn_mfma_kernel<8, RT, DIST>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    hipLaunchKernelGGL((winattn_mfma_kernel<8, RT, DIST>), dim3((T + 16 * RT - 1) / (16 * RT), H), dim3(512), (la_portion_lds<8, RT>(d)), st, step, (long long)ring_off, cap, (long long)fs.off, fs.pool,
+                       fs.keep, q, (long long)ldq, gate, (long long)ldg, temp, sink, H, G, d, dv, window, scale, T, o, (long long)ldo, softcap, gate_elem, slope);
+}
 void psk_winattn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, psk_front_store fs, const float *q, int64_t ldq, const float *gate,
                       int64_t ldg, const float *temp, const float *sink, int H, int G, int d, int dv, int window, float scale, int T, float *o, int64_t ldo, float softcap,
                       int gate_elem, const float *slope) {
-    static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) {
-        (void)hipFuncSetAttribute((const void *)winattn_mfma_kernel<8, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void *)winattn_mfma_kernel<8, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    }
-    const auto kernel = slope ? winattn_mfma_kernel<8, true> : winattn_mfma_kernel<8, false>;
-    hipLaunchKernelGGL(kernel, dim3((T + 63) / 64, H), dim3(256), wa_mfma_lds(d), st, step, (long long)ring_off, cap, (long long)fs.off, fs.pool, fs.keep, q,
-                       (long long)ldq, gate, (long long)ldg, temp, sink, H, G, d, dv, window, scale, T, o, (long long)ldo, softcap, gate_elem, slope);
+    const bool two = la_two_tiles(T, H, la_portion_lds<8, 2>(d));
+    const auto launch = two ? (slope ? wa_launch_mfma<2, true> : wa_launch_mfma<2, false>) : (slope ? wa_launch_mfma<1, true> : wa_launch_mfma<1, false>);
+    launch(st, step, ring_off, cap, fs, q, ldq, gate, ldg, temp, sink, H, G, d, dv, window, scale, T, o, ldo, softcap, gate_elem, slope);
 }
 
 // A single token.  Rows = the heads that share key / value group g (16 per block); the keys are cut into tiles of 16 in one index space -- tiles
@@ -337,32 +347,39 @@ __global__ __launch_bounds__(256) void winattn_step_kernel(const ps_seq_step *st
     if (tile >= ntiles) return;
     const long long rs = (long long)G * (d + dv);
     const float *base = tile < nbt ? step->state + store_off : step->state + ring_off;
-    const la_src k1 = {base + (long long)g * d, rs, 0, tile < nbt ? 0 : (long long)cap}, vs = {base + (long long)G * d + (long long)g * dv, rs, 0, tile < nbt ? 0 : (long long)cap};
-    const long long j0 = tile < nbt ? tile * 16 : lo + (tile - nbt) * 16, jend = tile < nbt ? nb : p + 1;
-    long long rowlo[4], rowhi[4], qpos[4];
-    float m[4], l[4], sl[4];
-    la_f4 acc[NJ];
+    const bool front = tile < nbt;
+    const la_src k1 = front ? la_src{base + (long long)g * d, rs, 0, 0} : la_ring(base + (long long)g * d, rs, lo, cap); // keys counted from the store's first row or the window's first position
+    la_src vs = k1;
+    vs.base = base + (long long)G * d + (long long)g * dv;
+    const int j0 = (int)(front ? tile : tile - nbt) * 16, jend = (int)(front ? nb : p + 1 - lo);
+    struct {
+        int rows, lq;
+        long long gap; // distance to key 0
+        float sl[4];
+        __device__ __forceinline__ bool sees(int, int i, int) const { return 4 * lq + i < rows; }
+        __device__ __forceinline__ float minus(int, int i, int j) const { return sl[i] * (float)(gap - j); }
+    } see{hpg - r0, lq, front ? p : p - lo, {0.f, 0.f, 0.f, 0.f}};
+    float m[1][4], l[1][4];
+    la_f4 acc[1][NJ];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const bool in = r0 + 4 * lq + i < hpg;
-        rowlo[i] = 0; rowhi[i] = in ? jend : 0; m[i] = -INFINITY; l[i] = 0.f;
-        qpos[i] = p;
-        sl[i] = DIST && in ? slope[g * hpg + r0 + 4 * lq + i] : 0.f;
+        m[0][i] = -INFINITY; l[0][i] = 0.f;
+        if (DIST && r0 + 4 * lq + i < hpg) see.sl[i] = slope[g * hpg + r0 + 4 * lq + i];
     }
 #pragma unroll
-    for (int j = 0; j < NJ; j++) acc[j] = la_f4{0.f, 0.f, 0.f, 0.f};
-    la_tile<NJ, DIST>(qs, qld, pt, k1, k1, vs, d, 0, dv, j0, jend, rowlo, rowhi, scale, m, l, acc, softcap, sl, qpos);
+    for (int j = 0; j < NJ; j++) acc[0][j] = la_f4{0.f, 0.f, 0.f, 0.f};
+    la_tiles<NJ, 1, DIST>(qs, qld, pt, k1, k1, vs, d, 0, dv, j0, jend, see, scale, m, l, acc, softcap);
     const int dvp = dv + 4;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int hh = r0 + 4 * lq + i;
         if (hh >= hpg) continue;
         float *pp = part + (tile * H + g * hpg + hh) * dvp;
-        if (lr == 0) { pp[dv] = m[i]; pp[dv + 1] = l[i]; }
+        if (lr == 0) { pp[dv] = m[0][i]; pp[dv + 1] = l[0][i]; }
 #pragma unroll
         for (int J = 0; J < NJ / 4; J++) {
             const int c = 64 * J + 4 * lr;
-            if (c < dv) *(la_f4 *)(pp + c) = la_f4{acc[4 * J][i], acc[4 * J + 1][i], acc[4 * J + 2][i], acc[4 * J + 3][i]};
+            if (c < dv) *(la_f4 *)(pp + c) = la_f4{acc[0][4 * J][i], acc[0][4 * J + 1][i], acc[0][4 * J + 2][i], acc[0][4 * J + 3][i]};
         }
     }
 }

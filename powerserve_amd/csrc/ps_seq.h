@@ -183,7 +183,7 @@ void psk_latent_prep(hipStream_t st, const ps_seq_step *step, int64_t ring_off, 
 void psk_latent_attn(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int64_t ldq, const float *kv, int64_t ldkv,
                      const float *freq, int H, int d, int dr, int rot_dims, int dv, int kv_rank, int window, float scale, int T, float *o, int64_t ldo,
                      float rot_mag = 1.f, const float *gate = nullptr, int64_t ldg = 0, int pairing = PS_ROT_HALVES); // gate [T][H] raw: head h of token t times sigmoid(gate[t][h]) (all forms)
-// The same attention on the matrix cores (fp32 MFMA), 16 tokens of a head per wave; _ok: the sizes it takes (d, dr multiples of 16, dv of 4, dv <= 128).
+// The same attention on the matrix cores (fp32 MFMA); _ok: the sizes it takes (d, dr multiples of 16, dv of 4, dv <= 128).
 bool psk_latent_attn_mfma_ok(int d, int dr, int dv);
 void psk_latent_attn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int64_t ldq, const float *kv, int64_t ldkv,
                           const float *freq, int H, int d, int dr, int rot_dims, int dv, int kv_rank, int window, float scale, int T, float *o, int64_t ldo,
@@ -220,7 +220,7 @@ void psk_winattn(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int 
                  float softcap = 0.f, // softcap > 0 (all three forms): score <- softcap tanh(score / softcap) behind scale and temperature
                  int gate_elem = 0,   // 1 (all three forms): gate [T][H dv], one sigmoid per output element instead of one per head
                  const float *slope = nullptr);
-// The same attention on the fp32 matrix cores for a portion, 16 tokens of a head per wave; _ok: the sizes it takes (d a multiple of 16, dv of 4, dv <= 128).
+// The same attention on the fp32 matrix cores for a portion; _ok: the sizes it takes (d a multiple of 16, dv of 4, dv <= 128).
 bool psk_winattn_mfma_ok(int d, int dv);
 void psk_winattn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, psk_front_store fs, const float *q, int64_t ldq, const float *gate,
                       int64_t ldg, const float *temp, const float *sink, int H, int G, int d, int dv, int window, float scale, int T, float *o, int64_t ldo,

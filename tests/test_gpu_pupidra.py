@@ -106,6 +106,17 @@ def layer_adds(m, toks, sizes):
     return np.concatenate(got)
 
 
+# ---------------------------------------------------------------------------------------------------------------- attention of a portion, two row tiles per block
+@pytest.mark.parametrize("sizes", [(17, 33), (31, 64), (32, 47), (65,), (129,)])
+def test_attention_of_a_portion_in_pairs_of_row_tiles(made, sizes):
+    """64 heads: blocks of 32 tokens (k_latent.hip, k_winattn.hip la_two_tiles), their last rows missing, their keys' last tile short, fewer key tiles than a block has
+    waves and more, front rows that end inside a tile; the window's ring wraps."""
+    cfg = UC(64, 48, [UL("attention", UA(64, 16, 16, 20, 0.3, 37, 21)), UL("latent_attention", ULA(64, 16, 16, 12, 16, 0.2, 100.0)), UL("attention", UA(64, 16, 16, 20, 0.3, 140, 0, kv_from=0))])
+    m, c, t = made("pairs", max_batch=130, cfg=cfg)
+    toks = tokens_for(c, 260)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run_pupidra(c, t, toks)) < TOL["float32"]
+
+
 # ---------------------------------------------------------------------------------------------------------------- mechanisms, one at a time
 ALONE = {
     "state_space": UL("mamba2", UM(6, 10, 9, 3, 4, 4)),
