@@ -158,6 +158,17 @@ size_t psk_mlstm_chunked_scratch(int H, int d, int dv, int T);
 void psk_mlstm_chunked(hipStream_t st, const ps_seq_step *step, int64_t state_off, int64_t m_off, const float *q, const float *k, const float *v, int64_t ld, const float *iraw,
                        const float *fraw, int64_t ldb, float cap, int H, int d, int dv, int T, float *scratch, float *o, int64_t ldo, float *nq, float *mt);
 
+// ---- k_chunk.hip
+// psk_wkv_scan, psk_gla_scan and psk_delta_scan for a portion, in chunks of 16 tokens on the fp32 matrix cores (same arguments; the same result up to rounding); _ok: the head sizes they take.
+bool psk_chunked_ok(int d);
+size_t psk_chunked_scratch(int H, int d, int T);
+void psk_wkv_chunked(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *r, const float *k, const float *v, const float *z, int64_t ld, const float *bonus, int H, int d,
+                     int T, float *scratch, float *o, int64_t ldo);
+void psk_gla_chunked(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *q, const float *k, const float *v, int64_t ld, const float *z, int64_t ldz, float tau, int H,
+                     int d, int dv, int T, float *scratch, float *o, int64_t ldo);
+void psk_delta_chunked(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *q, const float *k, const float *v, const float *braw, const float *araw, int64_t ld, int64_t ldb,
+                       const float *a_log, const float *dt_bias, int H, int KH, int d, int dv, int T, float *scratch, float *o, int64_t ldo);
+
 // ---- k_moe.hip
 // Router of a mixture of experts, fp32: scores = sigmoid(router h[t]), or (softmax) the soft-max over all `experts` rows; choice scores = scores + correction (NULL: none);
 // with n_groups > 0 only rows of the `keep` groups (equal runs of neighbours) with the largest best choice score stay in the race; the `top` largest choice scores

@@ -106,7 +106,7 @@ __global__ void seq_advance_kernel(ps_seq_step *s, const int32_t *amax, int32_t 
     s->pos0 += 1;
 }
 
-static const int SSD_CHUNKED_FROM = 32; // tokens from which a portion's state-space recurrence or matrix memory runs in chunks (fewer: the scan)
+static const int CHUNKED_FROM = 32; // tokens from which a portion's recurrences run in chunks (fewer: the scans)
 
 static int seq_fail(ps_hip_ctx *c, const std::string &msg) { c->err = msg; return 2; }
 
@@ -476,8 +476,10 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         if (wb) ok = ok && alloc((void **)&m->win_scratch, wb);
         size_t sb = 0;
         mixers([&](LayerPlan &P) {
-            if (P.d.kind == PS_MIX_MLSTM && B >= SSD_CHUNKED_FROM && psk_mlstm_chunked_ok(P.d.dim, P.d.vdim)) sb = std::max(sb, psk_mlstm_chunked_scratch(P.d.heads, P.d.dim, P.d.vdim, (int)B));
-            if (P.d.kind == PS_MIX_SSD && B >= SSD_CHUNKED_FROM && psk_ssd_chunked_ok(P.d.dim, P.d.vdim)) sb = std::max(sb, psk_ssd_chunked_scratch(P.d.heads, P.d.dim, P.d.vdim, (int)B));
+            if (P.d.kind == PS_MIX_MLSTM && B >= CHUNKED_FROM && psk_mlstm_chunked_ok(P.d.dim, P.d.vdim)) sb = std::max(sb, psk_mlstm_chunked_scratch(P.d.heads, P.d.dim, P.d.vdim, (int)B));
+            if ((P.d.kind == PS_MIX_WKV || P.d.kind == PS_MIX_DELTA || P.d.kind == PS_MIX_GLA) && B >= CHUNKED_FROM && psk_chunked_ok(P.d.dim))
+                sb = std::max(sb, psk_chunked_scratch(P.d.heads, P.d.dim, (int)B));
+            if (P.d.kind == PS_MIX_SSD && B >= CHUNKED_FROM && psk_ssd_chunked_ok(P.d.dim, P.d.vdim)) sb = std::max(sb, psk_ssd_chunked_scratch(P.d.heads, P.d.dim, P.d.vdim, (int)B));
         });
         if (sb) ok = ok && alloc((void **)&m->ssd_scratch, sb);
         if (m->lstm_aux_n) ok = ok && alloc((void **)&m->lstm_aux, (size_t)m->lstm_aux_n * 2 * 4);
@@ -546,7 +548,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     hipStream_t st = m->ctx->stream;
     const ps_seq_desc &D = m->d;
     const int64_t W = D.width;
-    const bool tiled = (m->mode & 2) != 0;
+    const bool tiled = (m->mode & 2) != 0, chunked = T >= CHUNKED_FROM && !tiled && m->ssd_scratch; // a portion's recurrences
     const int64_t BW = (int64_t)D.max_batch * W;
     psk_embed(st, D.embed, from_step ? nullptr : m->tokens, m->step, T, m->embed_scale, m->hist ? m->hist : m->x, W, D.bigram, D.bigram_buckets, D.bigram_mul_prev,
               D.bigram_mul_cur);
@@ -595,15 +597,20 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 psk_dense(st, g2);
             }
             psk_state_store(st, m->step, P.off_shift, in + (int64_t)(T - 1) * W, W);
-            psk_wkv_scan(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->t3, Hd);
+            if (chunked && psk_chunked_ok((int)d)) psk_wkv_chunked(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->ssd_scratch, m->t3, Hd);
+            else psk_wkv_scan(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->t3, Hd);
             psk_headnorm_gate(st, m->t3, Hd, m->t1 + 3 * Hd, NW, l.onorm, (int)d, D.norm_eps, (int)H, (int)d, T);
             out_proj(m->t3, Hd);
         } else if (l.kind == PS_MIX_DELTA) {
             const int64_t KHd = (int64_t)l.kv_heads * d, Hv = H * dv;
             if (!P.in_ld) psk_dense(st, mm(l.in_cat, in, W, t1, ld1));
             psk_causal_conv(st, m->step, P.off_conv, t1, ld1, l.conv, l.conv_taps, 1, P.cqkv, T, m->t2, P.cqkv);
-            psk_delta_scan(st, m->step, P.off_S, m->t2, m->t2 + KHd, m->t2 + 2 * KHd, t1 + P.cqkv + Hv, t1 + P.cqkv + Hv + H, P.cqkv, ld1, l.a_log, l.dt_bias,
-                           (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, Hv);
+            if (chunked && psk_chunked_ok((int)d))
+                psk_delta_chunked(st, m->step, P.off_S, m->t2, m->t2 + KHd, m->t2 + 2 * KHd, t1 + P.cqkv + Hv, t1 + P.cqkv + Hv + H, P.cqkv, ld1, l.a_log, l.dt_bias, (int)H, l.kv_heads, (int)d,
+                                  (int)dv, T, m->ssd_scratch, m->t3, Hv);
+            else
+                psk_delta_scan(st, m->step, P.off_S, m->t2, m->t2 + KHd, m->t2 + 2 * KHd, t1 + P.cqkv + Hv, t1 + P.cqkv + Hv + H, P.cqkv, ld1, l.a_log, l.dt_bias,
+                               (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, Hv);
             psk_headnorm_gate(st, m->t3, Hv, t1 + P.cqkv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T);
             out_proj(m->t3, Hv);
         } else if (l.kind == PS_MIX_GLA) {
@@ -613,7 +620,8 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             auto g2 = mm(l.decay2, t1 + 2 * Hd + 2 * Hv, ld1, m->t2, Hd);
             g2.bias = l.decay0;
             psk_dense(st, g2);
-            psk_gla_scan(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->t3, Hv);
+            if (chunked && psk_chunked_ok((int)d)) psk_gla_chunked(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->ssd_scratch, m->t3, Hv);
+            else psk_gla_scan(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->t3, Hv);
             psk_headnorm_gate(st, m->t3, Hv, t1 + 2 * Hd + Hv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T);
             out_proj(m->t3, Hv);
         } else if (l.kind == PS_MIX_WINATTN) {
@@ -648,7 +656,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             if (!P.in_ld) psk_dense(st, mm(l.in_cat, in, W, t1, ld1));
             psk_causal_conv(st, m->step, P.off_conv, t1 + inner, ld1, l.conv, l.conv_taps, 1, P.cqkv, T, m->t2, P.cqkv, l.conv_bias);
             const float *x = m->t2, *Bv = x + inner, *Cv = Bv + GN, *dt = t1 + inner + P.cqkv;
-            if (T >= SSD_CHUNKED_FROM && !tiled && m->ssd_scratch && psk_ssd_chunked_ok((int)d, (int)dv))
+            if (chunked && psk_ssd_chunked_ok((int)d, (int)dv))
                 psk_ssd_chunked(st, m->step, P.off_S, x, Bv, Cv, P.cqkv, dt, ld1, l.a_log, l.dt_bias, l.skip, (int)H, l.kv_heads, (int)d, (int)dv, T, m->ssd_scratch, m->t3, inner);
             else
                 psk_ssd_scan(st, m->step, P.off_S, x, Bv, Cv, P.cqkv, dt, ld1, l.a_log, l.dt_bias, l.skip, (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, inner);
@@ -664,7 +672,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             }
             const float *k = t1 + Hd, *v = k + Hd, *g = v + Hv, *iz = g + Hv, *fz = iz + H;
             float *nq = m->lstm_aux, *mt = nq + m->lstm_aux_n;
-            if (T >= SSD_CHUNKED_FROM && !tiled && m->ssd_scratch && ld1 % 4 == 0 && psk_mlstm_chunked_ok((int)d, (int)dv))
+            if (chunked && ld1 % 4 == 0 && psk_mlstm_chunked_ok((int)d, (int)dv))
                 psk_mlstm_chunked(st, m->step, P.off_S, P.off_m, t1, k, v, ld1, iz, fz, ld1, l.gate_cap, (int)H, (int)d, (int)dv, T, m->ssd_scratch, m->t3, Hv, nq, mt);
             else
                 psk_mlstm_scan(st, m->step, P.off_S, P.off_m, t1, k, v, ld1, iz, fz, ld1, l.gate_cap, (int)H, (int)d, (int)dv, T, m->t3, Hv, nq, mt);

@@ -157,6 +157,14 @@ def test_token_by_token_and_portions_give_the_whole_prompts_logits(made, name, d
         assert err(run_portions(m, toks, sizes), want) < TOL[dtype], sizes
 
 
+@pytest.mark.parametrize("sizes", [(31, 33), (32,), (47, 5, 49), (100,)])
+def test_linear_attention_in_chunks(made, sizes):
+    """gated linear attention in chunks of 16 tokens (k_chunk.hip), around their edges and beside portions of fewer than 32 tokens (the scan)"""
+    m, cfg, t = made("aligned", max_batch=100)
+    toks = tokens_for(cfg, 190)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run_parallel(cfg, t, toks)) < TOL["float32"]
+
+
 def test_first_tokens_of_a_sequence(made):
     m, cfg, t = made("aligned", "float32")
     for n in (1, 2, 3, 5):

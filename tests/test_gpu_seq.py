@@ -76,6 +76,21 @@ def run_portions(m, toks, sizes):
     return np.concatenate(out)
 
 
+# wkv and delta rule in chunks of 16 tokens (k_chunk.hip): portions that end inside, on and one behind a chunk's edge, fewer than 32 tokens between them (the scan), state row tiles that
+# do not fill the four waves and more than they are, value columns that are no multiple of 16; decays from e^-20 a token to none at all
+@pytest.mark.parametrize("sizes", [(31, 33), (32,), (47, 5, 49), (64, 17), (100,)])
+def test_recurrences_in_chunks(made, sizes):
+    cfg = synth.seq_config(64, 40, [L("wkv", None, heads=2, dim=16), L("delta", None, heads=4, kv_heads=2, dim=48, vdim=20, conv=3), L("wkv", None, heads=1, dim=80),
+                                    L("delta", None, heads=1, kv_heads=1, dim=256, vdim=33, conv=2), L("delta", None, heads=3, kv_heads=1, dim=144, vdim=16, conv=1)], taps=2)
+    t = synth.seq_tensors(cfg, 5)
+    t["l0.mix.w0"], t["l2.mix.w0"] = np.linspace(-9, 3, 32, dtype=np.float32), np.linspace(3, -9, 80, dtype=np.float32)
+    t["l1.mix.A_log"] = np.asarray([-9, -2, 1, 3], np.float32)
+    t = {n: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(np.shape(a)) for n, a in t.items()}
+    m, c, t = made("chunks", max_batch=100, cfg=cfg, tensors=t)
+    toks = tokens_for(c, 230)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(1, 37, 50), (2, 64, 96), (3, 19, 7), (8, 130, 72), (9, 70, 33), (70, 129, 200), (200, 48, 48), (1, 16, 4096)])
 def test_dense_matmul_any_shape(ctx, dtype, T, N, K):
