@@ -4,6 +4,7 @@
 //   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
 //   dense_mm_narrow_kernel bf16, K 128 or 256, more than 8 tokens: 32 x 32 tiles, the waves share K
+//   dense_mv1_kernel<WT,FORM> a single token, or a few tokens' chosen experts: every wave streams its rows, the requests run ahead of everything else
 //   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns): the activation rows live in LDS, a wave streams RW weight rows at a time
 // All take the same operand description (ps_seq.h psk_dense_args): ring rows, the token-shift mix and the epilogue
 // (bias, activation, scale, a factor from a second table) are part of the launch, so no mixer needs a kernel of its own around its projections.
@@ -11,6 +12,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 typedef float dn_f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 dn_bf8 __attribute__((ext_vector_type(8)));
@@ -225,7 +227,7 @@ __global__ __launch_bounds__(256) void dense_mm_kernel(dn_args g) {
 
 // ---------------------------------------------------------------------------------------------------- a few tokens: mat-vec
 // Dynamic LDS: C rows of K activations, as bf16-rounded fp32 values (bf16 mode: the same operand rounding as the tiled kernel) or fp32.
-template <typename WT, int C, int RW> // RW rows per wave at a time: four, or one where four would leave most of the chip without a wave (no paired activation then)
+template <typename WT, int C, int RW> // RW rows per wave at a time
 __global__ __launch_bounds__(256) void dense_mv_kernel(dn_args g) {
     extern __shared__ __attribute__((aligned(16))) float xs[]; // [C][Kp]
     long long row0;
@@ -407,8 +409,9 @@ __global__ __launch_bounds__(256) void dense_mv_grouped_kernel(dn_args g) {
         for (int q = 0; q < RW; q++) dn_put(g, r, nb + q, acc[q], acc[RW > 1 ? (q ^ 1) : q], lane == 0 && nb + q < g.N);
     }
 }
-template <typename WT, int RW>
+template <typename WT>
 static void dn_launch_mv_grouped(hipStream_t st, const dn_args &g, int rows, size_t lds) {
+    constexpr int RW = 2;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv_grouped_kernel<WT, RW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     long long blocks = (g.N + 4 * RW - 1) / (4 * RW);
@@ -854,8 +857,263 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_narrow_kernel(dn_args g) {
     }
 }
 
-template <typename WT, int C, int RW = 4>
+// ---------------------------------------------------------------------------------------------------- a single token: streaming mat-vec
+// A wave walks its rows as ONE stream of 1 KiB units (16 bytes per lane, non-temporal), DN_AHEAD of them in flight, requested before the activations are staged and across row ends, so
+// that neither the prologue nor a row's reduction leaves the memory idle.  Rows are dealt to the waves of the whole launch in turn (consecutive waves read consecutive rows; a matrix
+// of 2048 rows gives each of 2048 waves one), or in neighbouring pairs for a paired activation.  What bounded dense_mv_kernel here was the number of bytes in flight: four rows per wave,
+// two pieces each, 128 work-groups of four waves for 2048 rows.  Measured, bf16, before and now: 2048 x 4096 (16.8 MB) 14.6 and 6.6 us, 8192 x 2048 (33 MB) 15 and 9, 14336 x 4096
+// (117 MB) 29 to 38 and 22 us (5.3 TB/s).  The experts of one token (top 2 of 2048 x 2048 and a shared one), which were two launches per product, 12.4 + 10.4 and 12.0 us (first product),
+// 16.6 + 17.5 and 18.0 us (second).  Sixteen units in flight, and the activations requested ahead of the weights, were tried and are slower (the registers cost a work-group per CU).
+//   FORM 0  one matrix
+//   FORM 1  grouped, the first product of an expert: work-groups in equal runs per slot (its own matrix and output row), behind them those of the shared expert (g2)
+//   FORM 2  grouped, the second product: an output row is the sum over the token's slots (and the shared expert) of the products with their matrices: a row's stream runs through
+//           all of them; blockIdx.y = token
+// dynamic LDS: the activations as bf16-rounded fp32 (fp32 mode: as they are), every vector padded with zeros to whole units
+#define DN_AHEAD 8
+struct dn_mv1 {
+    dn_args g2; // the shared expert (w NULL: none): FORM 1 its first product, FORM 2 its second (only w, a, K, out_scale are read there)
+    int slots;  // FORM 1: slots of the launch; FORM 2: slots per token
+    int kp, kp2; // padded lengths of the vectors
+    int blocks, blocks2; // FORM 1: work-groups per slot, of the shared expert
+};
+
+// one vector into LDS, by all 512 threads
+template <typename WT>
+static __device__ __forceinline__ void dn_stage(const dn_args &g, const float *x, const float *prev, float scale, float *xs, int kp) {
+    const int K = (int)g.K;
+    if (!prev && K % 4 == 0 && ((uintptr_t)x & 15) == 0) {
+        for (int k = threadIdx.x * 4; k < kp; k += 512 * 4) {
+            dn_f4 v = k < K ? *(const dn_f4 *)(x + k) : dn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] *= scale;
+                if constexpr (sizeof(WT) == 2) v[e] = dn_bf2f(dn_f2bf(v[e]));
+            }
+            *(dn_f4 *)(xs + k) = v;
+        }
+        return;
+    }
+#pragma unroll 4
+    for (int k = threadIdx.x; k < kp; k += 512) {
+        float v = k < K ? x[k] * scale : 0.f;
+        if (prev && k < K) v += (prev[k] - v) * g.mu[k]; // (the token-shift mix of dn_aval; never with a scale)
+        if constexpr (sizeof(WT) == 2) v = dn_bf2f(dn_f2bf(v));
+        xs[k] = v;
+    }
+}
+// one unit: 16 bytes of weights against the same places of x
+template <typename WT>
+static __device__ __forceinline__ float dn_unit(float acc, const dn_f4 &raw, const float *x) {
+    if constexpr (sizeof(WT) == 2) {
+        const dn_f4 x0 = *(const dn_f4 *)x, x1 = *(const dn_f4 *)(x + 4);
+        unsigned h[4];
+        __builtin_memcpy(h, &raw, 16);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            acc = fmaf(__uint_as_float(h[e] << 16), e < 2 ? x0[2 * e] : x1[2 * e - 4], acc);
+            acc = fmaf(__uint_as_float(h[e] & 0xffff0000u), e < 2 ? x0[2 * e + 1] : x1[2 * e - 3], acc);
+        }
+    } else {
+        const dn_f4 x0 = *(const dn_f4 *)x;
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = fmaf(raw[e], x0[e], acc);
+    }
+    return acc;
+}
+static __device__ __forceinline__ float dn_wave_sum(float v) { // every lane gets it: rotations inside a row of sixteen, then the four rows' sums
+    auto ror = [](float x, auto n) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + decltype(n)::value, 0xf, 0xf, true)); };
+    v += ror(v, std::integral_constant<int, 8>());
+    v += ror(v, std::integral_constant<int, 4>());
+    v += ror(v, std::integral_constant<int, 2>());
+    v += ror(v, std::integral_constant<int, 1>());
+    auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    return (row(0) + row(16)) + (row(32) + row(48));
+}
+
+template <typename WT, int FORM>
+__global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p) {
+    extern __shared__ __attribute__((aligned(16))) float xs[];
+    constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE; // elements per lane and per unit
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int y = FORM == 1 ? min((int)blockIdx.x / p.blocks, p.slots) : (int)blockIdx.y;
+    const bool shared_seg = FORM == 1 && y == p.slots;
+    dn_args g = g0;
+    if constexpr (FORM == 1) { // (field by field: the same K, activation and addition in both)
+        g.w = shared_seg ? p.g2.w : g0.w;
+        g.N = shared_seg ? p.g2.N : g0.N;
+        g.a = shared_seg ? p.g2.a : g0.a;
+        g.out = shared_seg ? p.g2.out : g0.out;
+        g.ldo = shared_seg ? p.g2.ldo : g0.ldo;
+        g.out_scale = shared_seg ? p.g2.out_scale : g0.out_scale;
+        g.bias = shared_seg ? p.g2.bias : g0.bias;
+        g.alpha = shared_seg ? p.g2.alpha : g0.alpha;
+    }
+    // lane c: the matrix of segment c of a row's stream (FORM 2: the token's slots, then the shared expert)
+    const int n_seg = FORM == 2 ? p.slots + (p.g2.w ? 1 : 0) : 1;
+    int sel = 0;
+    if constexpr (FORM == 1) sel = shared_seg ? 0 : g.g_sel[y];
+    if constexpr (FORM == 2) {
+        if (lane < p.slots) sel = g.g_sel[(long long)y * p.slots + lane];
+    }
+    auto has = [&](int c) { return FORM == 0 || (FORM == 1 ? shared_seg || sel < g.groups : c == p.slots || (int)__builtin_amdgcn_readlane(sel, c) < g.groups); };
+    auto units_of = [&](int c) { return (FORM == 2 && c == p.slots ? p.kp2 : p.kp) / UNIT; };
+    int row_units = 0; // units of a row's stream (0: identity experts only)
+    for (int c = 0; c < n_seg; c++) row_units += has(c) ? units_of(c) : 0;
+    const int N = (int)g.N;
+    const bool pair = FORM != 2 && (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR);
+    // this wave's rows: first + k step (pairs: first + (k / 2) step + k % 2), k < rows
+    const int bx = FORM == 1 ? (int)blockIdx.x - y * p.blocks : (int)blockIdx.x, nb = FORM == 1 ? (shared_seg ? p.blocks2 : p.blocks) : (int)gridDim.x;
+    const int step = nb * 8 * (pair ? 2 : 1), first = (bx * 8 + wave) * (pair ? 2 : 1);
+    const int rows = first >= N ? 0 : pair ? ((N - first + step - 2) / step) * 2 : (N - first + step - 1) / step;
+    auto row_of = [&](int k) { return pair ? first + (k >> 1) * step + (k & 1) : first + k * step; };
+    // the load side of the stream: row lk, segment lc, unit lu of lunits
+    int lk = 0, lc = -1, lu = 0, lunits = 0;
+    const char *lp = nullptr, *lrow = nullptr;
+    bool beyond = false; // this lane's bytes of a row's last unit lie behind the row's end: it reads the row's first ones, against zeros
+    auto open = [&]() { // the next segment that has a matrix
+        do {
+            if (++lc == n_seg) { lc = 0; lk++; }
+        } while (!has(lc));
+        if (lk >= rows) return;
+        const bool sh = FORM == 2 && lc == p.slots;
+        const int K = (int)(sh ? p.g2.K : g.K);
+        const long long mat = FORM == 0 || sh || shared_seg ? 0 : (long long)(FORM == 1 ? sel : (int)__builtin_amdgcn_readlane(sel, lc)) * g.wstride;
+        lrow = (const char *)((const WT *)(sh ? p.g2.w : g.w) + mat + (long long)row_of(lk) * K);
+        lp = lrow + lane * 16;
+        lu = 0; lunits = units_of(lc);
+        beyond = (lunits - 1) * UNIT + lane * VE >= K;
+    };
+    auto request = [&](dn_f4 &v) {
+        if (lk >= rows) return; // (uniform)
+        const char *q = beyond && lu == lunits - 1 ? lrow : lp;
+        v = __builtin_nontemporal_load((const dn_f4 *)q);
+        lp += 1024;
+        if (++lu == lunits) open();
+    };
+    dn_f4 ring[DN_AHEAD];
+    if (rows && row_units) {
+        open();
+#pragma unroll
+        for (int u = 0; u < DN_AHEAD; u++) request(ring[u]);
+    }
+    // the activations
+    if constexpr (FORM == 0) {
+        long long row0;
+        int T;
+        dn_rows(g, row0, T);
+        dn_stage<WT>(g, dn_arow(g, row0, 0), g.mu ? g.shift0 : nullptr, 1.f, xs, p.kp);
+    } else if constexpr (FORM == 1) {
+        if (shared_seg) dn_stage<WT>(g, g.a, nullptr, 1.f, xs, p.kp);
+        else dn_stage<WT>(g, g.a + (long long)(y / g.g_adiv) * g.lda, nullptr, g.g_scale ? g.g_scale[y] : 1.f, xs, p.kp);
+    } else {
+        for (int c = 0; c < p.slots; c++) {
+            const int s = y * p.slots + c;
+            dn_stage<WT>(g, g.a + (long long)(s / g.g_adiv) * g.lda, nullptr, g.g_scale ? g.g_scale[s] : 1.f, xs + c * p.kp, p.kp);
+        }
+        if (p.g2.w) dn_stage<WT>(p.g2, p.g2.a + y * p.g2.lda, nullptr, 1.f, xs + p.slots * p.kp, p.kp2);
+    }
+    float ident = 0.f; // FORM 2: the summed weights of the token's slots that have no matrix
+    if constexpr (FORM == 2) {
+        if (g.g_ident)
+            for (int c = 0; c < p.slots; c++)
+                if (!has(c)) ident += g.g_ident_w[y * p.slots + c];
+    }
+    const float shared_scale = FORM == 2 && p.g2.w && p.g2.out_scale ? p.g2.out_scale[y] : 1.f;
+    __syncthreads();
+    // the other side: segment cc, cu units of it left; lane k % 64 keeps row k's result until 64 of them are there or the rows are through
+    int cc = -1, cu = 0, done = 0, kept = 0;
+    const float *xp = xs;
+    float acc = 0.f, total = 0.f, res = 0.f;
+    auto next = [&]() {
+        do {
+            if (++cc == n_seg) cc = 0;
+        } while (!has(cc));
+        cu = units_of(cc);
+        xp = xs + (FORM == 2 ? cc * p.kp : 0) + lane * VE;
+    };
+    auto last_of_row = [&]() {
+        int c = cc + 1;
+        while (c < n_seg && !has(c)) c++;
+        return c == n_seg;
+    };
+    auto eat = [&](dn_f4 &v) {
+        acc = dn_unit<WT>(acc, v, xp);
+        request(v);
+        xp += UNIT;
+        if (--cu) return;
+        total = FORM == 2 && cc == p.slots ? fmaf(acc, shared_scale, total) : total + acc;
+        acc = 0.f;
+        if (last_of_row()) {
+            const float s = dn_wave_sum(total);
+            res = lane == done - kept ? s : res;
+            total = 0.f;
+            done++;
+        }
+        next();
+    };
+    auto put = [&]() { // the results of rows kept .. done - 1
+        const int k = kept + lane, n = row_of(k);
+        float v = res;
+        const bool in = k < done;
+        if constexpr (FORM == 2) {
+            if (ident != 0.f && in) v = fmaf(ident, g.g_ident[(long long)y * g.g_ident_ld + n], v);
+        }
+        dn_put(g, FORM == 0 || shared_seg ? 0 : y, n, v, __shfl_xor(v, 1, 64), in);
+        kept = done;
+    };
+    if (row_units) {
+        int left = rows * row_units;
+        if (left) next();
+        for (; left >= DN_AHEAD; left -= DN_AHEAD) {
+#pragma unroll
+            for (int q = 0; q < DN_AHEAD; q++) eat(ring[q]);
+            if (done - kept > 64 - DN_AHEAD - 2) { // (kept stays even for pairs)
+                const int odd = (done - kept) & 1;
+                if (!pair || !odd) put();
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < DN_AHEAD; q++)
+            if (q < left) eat(ring[q]);
+        put();
+    } else {
+        for (done = min(rows, 64); kept < rows; done = min(done + 64, rows)) put();
+    }
+}
+
+// Work-groups of eight waves: enough that every wave has a row, at most two per CU (one where the activations are long: each group stages them for itself).
+template <typename WT, int FORM>
+static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, int slots, int tokens) {
+    constexpr int UNIT = 64 * 16 / (int)sizeof(WT);
+    dn_mv1 p;
+    if (g2) p.g2 = *g2;
+    else { p.g2 = g; p.g2.w = nullptr; }
+    p.slots = slots;
+    p.kp = (int)((g.K + UNIT - 1) / UNIT * UNIT);
+    p.kp2 = g2 ? (int)((g2->K + UNIT - 1) / UNIT * UNIT) : 0;
+    const size_t lds = ((size_t)p.kp * (FORM == 2 ? slots : 1) + (FORM == 2 ? p.kp2 : 0)) * 4;
+    const bool aligned = (g.K * (int64_t)sizeof(WT)) % 16 == 0 && (!g2 || (g2->K * (int64_t)sizeof(WT)) % 16 == 0);
+    if (!aligned || lds > 128 * 1024 || g.N > (1 << 28) || slots > 63 || (FORM == 1 && g2 && (g2->K != g.K || g2->act != g.act || g2->accum != g.accum || g2->N > (1 << 28)))) return false;
+    static unsigned long long mask = 0;
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv1_kernel<WT, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    const int per = FORM != 2 && (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR) ? 16 : 8; // rows that a work-group takes at once
+    const int64_t most = lds <= 72 * 1024 ? 512 : 256;
+    dim3 grid;
+    if (FORM == 1) { // the same number of rows for every work-group of every matrix
+        const int64_t all = g.N * slots + (g2 ? g2->N : 0), rounds = std::max<int64_t>((all + most * per - 1) / (most * per), 1);
+        p.blocks = (int)((g.N + rounds * per - 1) / (rounds * per));
+        p.blocks2 = g2 ? (int)((g2->N + rounds * per - 1) / (rounds * per)) : 0;
+        grid = dim3((unsigned)(p.blocks * slots + p.blocks2));
+    } else {
+        grid = dim3((unsigned)std::min<int64_t>((g.N + per - 1) / per, std::max<int64_t>(most / tokens, 64)), (unsigned)tokens);
+    }
+    hipLaunchKernelGGL((dense_mv1_kernel<WT, FORM>), grid, dim3(512), lds, st, g, p);
+    return true;
+}
+
+template <typename WT, int C>
 static void dn_launch_mv(hipStream_t st, const dn_args &g) {
+    constexpr int RW = 4;
     const size_t lds = (size_t)C * ((g.K + 7) / 8 * 8) * 4;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv_kernel<WT, C, RW>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
@@ -864,8 +1122,7 @@ static void dn_launch_mv(hipStream_t st, const dn_args &g) {
     hipLaunchKernelGGL((dense_mv_kernel<WT, C, RW>), dim3((unsigned)blocks), dim3(256), lds, st, g);
 }
 
-int psk_dense(hipStream_t st, const psk_dense_args &a) {
-    if (!a.w || a.T <= 0) return 0;
+static dn_args dn_make(const psk_dense_args &a) {
     dn_args g;
     g.w = a.w->data; g.a = a.a; g.lda = a.lda; g.a_row0 = a.a_row0; g.a_mod = a.a_mod; g.a_step = a.a_step; g.T = a.T;
     g.N = a.w->N; g.K = a.w->K; g.out = a.out; g.ldo = a.ldo; g.bias = a.bias; g.act = a.act; g.act_p = a.act_p; g.act_q = a.act_q;
@@ -874,24 +1131,33 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
     g.g_ident = a.g_ident; g.g_ident_w = a.g_ident_w; g.g_ident_ld = a.g_ident_ld;
     g.em_table = a.em_table ? a.em_table->data : nullptr; g.em_bf16 = a.em_table && a.em_table->dtype == PS_BF16; g.em_ld = a.em_table ? a.em_table->K : 0;
     g.em_col = a.em_col; g.em_tokens = a.em_tokens; g.em_step = a.em_step;
+    return g;
+}
+// a few slots' grouped product as one streaming mat-vec, the shared expert's with it where there is one and it fits: 0 not taken, 1 the slots alone, 2 both
+template <typename WT>
+static int dn_grouped_mv1(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
+    const bool second = g.act == PSD_ACT_NONE; // an output row per token, the sum over its slots; an expert's first product: one per slot
+    if (!second && (a.g_inner != 1 || a.g_ident)) return 0;
+    if (a.also && a.also->w->dtype == a.w->dtype && (second || a.also->T == 1)) {
+        const dn_args g2 = dn_make(*a.also);
+        if (second ? dn_launch_mv1<WT, 2>(st, g, &g2, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, &g2, a.T, 1)) return 2;
+    }
+    return (second ? dn_launch_mv1<WT, 2>(st, g, nullptr, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, nullptr, a.T, 1)) ? 1 : 0;
+}
+
+int psk_dense(hipStream_t st, const psk_dense_args &a) {
+    if (!a.w || a.T <= 0) return 0;
+    dn_args g = dn_make(a);
     const bool bf = a.w->dtype == PS_BF16;
     const size_t kp4 = (size_t)((g.K + 7) / 8 * 8) * 4;
     if (a.groups > 0) {
         g.groups = a.groups; g.N = a.w->N / a.groups; g.wstride = g.N * g.K;
         g.g_adiv = a.g_adiv; g.g_odiv = a.g_odiv; g.g_inner = a.g_inner; g.g_sel = a.g_sel; g.g_scale = a.g_scale;
-        if (!a.g_list) { // a mat-vec per output row (T rows of g_inner slots each); four rows per wave only where that still leaves about 1024 waves
-            const long long waves4 = (g.N + 3) / 4 * a.T;
-            const int RW = waves4 >= 1024 ? 4 : (waves4 >= 512 || g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR) ? 2 : 1; // (a gate / up pair sits in one wave)
-            const size_t lds = kp4 * a.g_inner;
-            if (bf) {
-                if (RW == 4) dn_launch_mv_grouped<unsigned short, 4>(st, g, a.T, lds);
-                else if (RW == 2) dn_launch_mv_grouped<unsigned short, 2>(st, g, a.T, lds);
-                else dn_launch_mv_grouped<unsigned short, 1>(st, g, a.T, lds);
-            } else {
-                if (RW == 4) dn_launch_mv_grouped<float, 4>(st, g, a.T, lds);
-                else if (RW == 2) dn_launch_mv_grouped<float, 2>(st, g, a.T, lds);
-                else dn_launch_mv_grouped<float, 1>(st, g, a.T, lds);
-            }
+        if (!a.g_list) { // a few slots
+            const int took = bf ? dn_grouped_mv1<unsigned short>(st, a, g) : dn_grouped_mv1<float>(st, a, g);
+            if (took) return took == 2;
+            if (bf) dn_launch_mv_grouped<unsigned short>(st, g, a.T, kp4 * a.g_inner);
+            else dn_launch_mv_grouped<float>(st, g, a.T, kp4 * a.g_inner);
             return 0;
         }
         g.g_seg = a.g_seg; g.g_list = a.g_list;
@@ -902,12 +1168,11 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         return 0;
     }
     if (!a.force_tiled && a.T <= 8) {
+        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0, 1) : dn_launch_mv1<float, 0>(st, g, nullptr, 0, 1))) return 0;
         const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
         if (kp4 * C <= 64 * 1024) {
-            const bool one_row = g.N <= 1024 && g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR; // (four rows per wave: at most 64 blocks)
             if (bf) {
-                if (C == 1 && one_row) dn_launch_mv<unsigned short, 1, 1>(st, g);
-                else if (C == 1) dn_launch_mv<unsigned short, 1>(st, g);
+                if (C == 1) dn_launch_mv<unsigned short, 1>(st, g);
                 else if (C == 2) dn_launch_mv<unsigned short, 2>(st, g);
                 else if (C == 4) dn_launch_mv<unsigned short, 4>(st, g);
                 else dn_launch_mv<unsigned short, 8>(st, g);

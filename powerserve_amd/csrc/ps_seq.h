@@ -70,6 +70,9 @@ struct psk_dense_args {
     int64_t em_col = 0;
     const int32_t *em_tokens = nullptr;
     const ps_seq_step *em_step = nullptr;
+    // grouped mat-vec only: the shared expert's product that goes with it -- beside the slots' first products (T == 1, the same activation), or added to a token's sum of second products
+    // (only its w, a, lda, K and out_scale count there).  psk_dense returns 1 where the launch has made it too, 0 where it is still to be made.
+    const psk_dense_args *also = nullptr;
 };
 int psk_dense(hipStream_t st, const psk_dense_args &a);
 size_t psk_dense_split_bytes(); // what any product's splits need at most

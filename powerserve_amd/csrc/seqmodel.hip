@@ -329,7 +329,7 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
                 moe_slots = std::max(moe_slots, B * l.top);
                 moe_experts = std::max<int64_t>(moe_experts, rows);
                 moe_top = std::max<int64_t>(moe_top, l.top);
-                n4 = std::max<int64_t>({n4, (int64_t)l.top * l.ff, (int64_t)l.shared_ff});
+                n4 = std::max<int64_t>(n4, (int64_t)l.top * l.ff + 3 + l.shared_ff); // (a single token's shared expert beside its slots)
                 m->weight_bytes += (dense_bytes(l.ff_up) + dense_bytes(l.ff_down)) / l.experts * std::min(l.top, l.experts) + (uint64_t)rows * W * 4;
             }
             const int64_t up_rows = l.ff_kind == PS_FF_DENSE_SWIGLU || l.ff_kind == PS_FF_DENSE_RELU_GLU ? 2 * (int64_t)l.ff : l.ff;
@@ -758,13 +758,20 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             g.groups = E; g.g_sel = m->moe_sel;
             if (!mv) { g.g_seg = m->moe_seg; g.g_list = m->moe_list; }
         };
+        // (a single token's shared expert rides with the slots' launches where they are mat-vecs: its activations behind theirs)
+        auto su = mm(l.shared_up, in, W, m->t4 + (mv && T == 1 ? ((int64_t)top * l.ff + 3) / 4 * 4 : 0), l.shared_ff);
+        su.act = act;
+        auto sd = mm(l.shared_down, su.out, l.shared_ff, xr, W);
+        sd.accum = 1; sd.alpha = alpha; sd.out_scale = l.shared_gate ? m->moe_sg : nullptr;
+        bool up_made = false, down_made = false;
         {
             auto g = mm(l.ff_up, in, W, m->t4, l.ff);
             g.act = act; g.T = S; g.g_adiv = top;
             if (l.moe_weight_output) g.out_scale = m->moe_wgt; // (a row of the result is a slot)
             else g.g_scale = m->moe_wgt;
             grouped(g);
-            psk_dense(st, g);
+            if (l.shared_up && mv && T == 1) g.also = &su;
+            up_made = psk_dense(st, g) == 1;
         }
         bool summed = false; // the identity slots' share has joined the stream
         {
@@ -773,6 +780,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             if (mv) {
                 g.T = T; g.g_inner = top; g.accum = !store; g.alpha = alpha;
                 if (l.moe_identity) { g.g_ident = in; g.g_ident_ld = W; g.g_ident_w = m->moe_wgt; summed = true; } // (the identity slots' share inside the same launch)
+                if (up_made) g.also = &sd;
             }
             else if (top == 1) {
                 // (an identity expert's slot has no product: a store must find a zero there)
@@ -780,7 +788,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 g.T = S; g.accum = !store || l.moe_identity; g.alpha = alpha;
             }
             else { g.T = S; g.out = m->moe_y; } // (two slots of a token sit in different tiles: per-slot results, summed below)
-            psk_dense(st, g);
+            down_made = psk_dense(st, g) == 1;
             if (!mv && top > 1) {
                 psk_moe_combine(st, xr, m->moe_y, top, alpha, W, T, l.moe_identity ? m->moe_sel : nullptr, m->moe_wgt, E, in, W, store);
                 summed = true;
@@ -788,12 +796,8 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         }
         if (l.moe_identity && !summed) psk_moe_combine(st, xr, nullptr, top, alpha, W, T, m->moe_sel, m->moe_wgt, E, in, W);
         if (l.shared_up) {
-            auto g = mm(l.shared_up, in, W, m->t4, l.shared_ff);
-            g.act = act;
-            psk_dense(st, g);
-            auto g2 = mm(l.shared_down, m->t4, l.shared_ff, xr, W);
-            g2.accum = 1; g2.alpha = alpha; g2.out_scale = l.shared_gate ? m->moe_sg : nullptr;
-            psk_dense(st, g2);
+            if (!up_made) psk_dense(st, su);
+            if (!down_made) psk_dense(st, sd);
         }
     };
     const int n_runs = (int)m->L.size();

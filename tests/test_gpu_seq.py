@@ -139,6 +139,29 @@ def test_dense_matmul_wide(ctx, dtype, T, N, K):
     dx.free(); do.free()
 
 
+# one token (k_dense.hip dense_mv1_kernel): a row of less than one unit of its stream (512 numbers, fp32: 256), of exactly one, of one and a bit; fewer and more units per wave than are in flight;
+# one row, rows that are no multiple of the waves', more rows than waves and more than 64 of them per wave; the longest row that is taken, and one more, which the general kernel does
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("N,K", [(1, 8), (7, 248), (9, 256), (65, 264), (8, 504), (63, 512), (66, 520), (1, 4096), (5, 4104), (4097, 64), (300001, 16), (12289, 520), (17, 32768), (17, 32776)])
+def test_dense_matvec_in_one_stream(ctx, dtype, N, K):
+    import ctypes as C
+    rng = np.random.default_rng(N + K)
+    bits = f32_to_bf16_bits(rng.standard_normal((N, K), dtype=np.float32))
+    x = rng.standard_normal((1, K), dtype=np.float32)
+    w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K)
+    h = C.c_void_p()
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, int(dtype == "float32"), C.byref(h)))
+    dx, do = ctx.to_device(x), ctx.to_device(np.full((2, N), np.float32(7.0)))
+    ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, h, dx.ptr, 1, do.ptr, 1.0))
+    got = do.numpy()
+    a = (x if dtype == "float32" else (f32_to_bf16_bits(x).astype(np.uint32) << 16).view(np.float32).reshape(x.shape)).astype(np.float64)
+    # fp32 sums of K products, in any order: at most K roundings of 2^-24, each relative to a partial sum of at most sum |a w|
+    assert np.all(np.abs(got[0] - (w.astype(np.float64) @ a[0])) <= K * 2.0 ** -24 * (np.abs(w).astype(np.float64) @ np.abs(a[0])))
+    assert np.all(got[1] == 7.0)  # nothing behind the last row
+    ctx.L.ps_hip_dense_free(ctx.h, h)
+    dx.free(); do.free()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["wkv", "delta", "latent", "ff", "mixed", "aligned", "wide_heads"])
 def test_whole_prompt_against_the_plain_statement(made, name, dtype):
