@@ -30,22 +30,45 @@ static __device__ __forceinline__ void la_pair(int i, int half, int pairing, int
 __global__ __launch_bounds__(256) void latent_prep_kernel(const ps_seq_step *step, long long ring_off, int cap, const float *y, long long ldy, const float *qnorm,
                                                           const float *kvnorm, float eps, int q_rank, int kv_rank, int rot_dim, int rot_dims, const float *freq, float *cq,
                                                           long long ldcq, float rot_mag, int pairing) {
+    // (a thread's numbers and weights are requested together and held: 8 + 4 of them, what is beyond 2048 and 1024 is read again)
     __shared__ float red[8];
     const int t = blockIdx.x, tid = threadIdx.x;
-    const long long pos = step->pos0 + t;
     const float *yt = y + (long long)t * ldy, *ckv = yt + q_rank, *kr = ckv + kv_rank;
+    float qv[8], qw[8], kv[4], kw[4], a = 0.f, b = 0.f;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int i = tid + 256 * u;
+        qv[u] = i < q_rank ? yt[i] : 0.f;
+        qw[u] = i < q_rank ? qnorm[i] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int i = tid + 256 * u;
+        kv[u] = i < kv_rank ? ckv[i] : 0.f;
+        kw[u] = i < kv_rank ? kvnorm[i] : 0.f;
+    }
+    const long long pos = step->pos0 + t;
     float *ring = step->state + ring_off + (pos % cap) * (long long)(kv_rank + rot_dim);
-    float a = 0.f, b = 0.f;
-    for (int i = tid; i < q_rank; i += 256) a += yt[i] * yt[i];
-    for (int i = tid; i < kv_rank; i += 256) b += ckv[i] * ckv[i];
+#pragma unroll
+    for (int u = 0; u < 8; u++) a += qv[u] * qv[u];
+#pragma unroll
+    for (int u = 0; u < 4; u++) b += kv[u] * kv[u];
+    for (int i = 2048 + tid; i < q_rank; i += 256) a += yt[i] * yt[i];
+    for (int i = 1024 + tid; i < kv_rank; i += 256) b += ckv[i] * ckv[i];
     a = la_wave_sum(a);
     b = la_wave_sum(b);
     if ((tid & 63) == 0) { red[tid >> 6] = a; red[4 + (tid >> 6)] = b; }
     __syncthreads();
     const float ia = q_rank > 0 ? 1.f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)q_rank + eps) : 0.f; // (q_rank 0: the queries do not pass a latent)
     const float ib = 1.f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)kv_rank + eps);
-    for (int i = tid; i < q_rank; i += 256) cq[(long long)t * ldcq + i] = yt[i] * ia * qnorm[i];
-    for (int i = tid; i < kv_rank; i += 256) ring[i] = ckv[i] * ib * kvnorm[i];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+        if (tid + 256 * u < q_rank) cq[(long long)t * ldcq + tid + 256 * u] = qv[u] * ia * qw[u];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (tid + 256 * u < kv_rank) ring[tid + 256 * u] = kv[u] * ib * kw[u];
+    for (int i = 2048 + tid; i < q_rank; i += 256) cq[(long long)t * ldcq + i] = yt[i] * ia * qnorm[i];
+    for (int i = 1024 + tid; i < kv_rank; i += 256) ring[i] = ckv[i] * ib * kvnorm[i];
     const int half = rot_dims / 2; // the first rot_dims of the part are rotated; the rest passes unchanged
     for (int i = tid; i < half; i += 256) {
         const float ang = (float)pos * freq[i], c = cosf(ang) * rot_mag, s = sinf(ang) * rot_mag;
@@ -228,12 +251,28 @@ void psk_latent_attn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_
 }
 
 // ---------------------------------------------------------------------------------------------------- single token, absorbed
-// qa[h][r] = sum_i q[h][i] Wuk[h * d + i][r]: a head's query folded into latent space.  One block per head, a thread per latent index.
+// qa[h][r] = sum_i q[h][i] Wuk[h * d + i][r]: a head's query folded into latent space, and behind it (the last block of a head) its rotated part: qa [H][R + dr].
 template <typename WT>
-__global__ __launch_bounds__(256) void latent_fold_q_kernel(const float *q, int qstride, const WT *wuk, int d, int R, float *qa) {
+__global__ __launch_bounds__(256) void latent_fold_q_kernel(const ps_seq_step *step, const float *q, int qstride, const WT *wuk, int d, int R, int dr, int rot_dims, const float *freq,
+                                                            float rot_mag, int pairing, float *qa) {
     __shared__ float part[4][64];
     const int h = blockIdx.x, r = blockIdx.y * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6; // block: 64 latent indices x 4 slices of the head's rows
     const float *qh = q + (long long)h * qstride;
+    qa += (long long)h * (R + dr);
+    if (blockIdx.y + 1 == gridDim.y) {
+        const int half = rot_dims / 2;
+        const float p = (float)step->pos0;
+        for (int i = threadIdx.x; i < half; i += 256) {
+            const float ang = p * freq[i], cs = cosf(ang) * rot_mag, sn = sinf(ang) * rot_mag;
+            int pa, pb;
+            la_pair(i, half, pairing, pa, pb);
+            const float u = qh[d + pa], v = qh[d + pb];
+            qa[R + pa] = u * cs - v * sn;
+            qa[R + pb] = v * cs + u * sn;
+        }
+        for (int i = 2 * half + threadIdx.x; i < dr; i += 256) qa[R + i] = qh[d + i];
+        return;
+    }
     float a = 0.f;
     if (r < R) {
 #pragma unroll 8
@@ -246,7 +285,7 @@ __global__ __launch_bounds__(256) void latent_fold_q_kernel(const float *q, int 
     }
     part[grp][threadIdx.x & 63] = a;
     __syncthreads();
-    if (grp == 0 && r < R) qa[(long long)h * R + r] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+    if (grp == 0 && r < R) qa[r] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
 }
 // o[h][x] = sum_r Wuv[h * dv + x][r] ol[h][r]: the value expansion of the attended latent.  A wave per output row.
 template <typename WT>
@@ -265,119 +304,134 @@ __global__ __launch_bounds__(256) void latent_unfold_v_kernel(const float *ol, c
     if (lane == 0) o[row] = gate ? a / (1.f + expf(-gate[row / dv])) : a; // (the head's output gate)
 }
 
-// rows = heads (16 per block), keys = ring rows; wave w of block (split s, head tile) takes key tile 4 s + w of the window.  Partials:
-// per (key tile, head) R unnormalised outputs, then m and l.  dynamic LDS: 16 x qld + 4 x 16 x 17
-template <int NJ>
-__global__ __launch_bounds__(256) void latent_absorbed_kernel(const ps_seq_step *step, long long ring_off, int cap, const float *qa, const float *q, int qstride, int d,
-                                                              int dr, int rot_dims, const float *freq, int H, int R, int window, float scale, float *part, float rot_mag, int pairing) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
+// rows = heads (16 per block), keys = the 16 ring rows of block x's tile of the window.  The block's four waves share the tile: each multiplies a quarter of the dimensions, the four
+// partial scores meet in LDS, every wave takes the soft-max of all of them (a lane: one head, four keys -- the row operand of the second product as it stands) and then a quarter of
+// the value columns (groups of 64 columns, G of them per wave).  Queries, keys and values come straight from memory, requested at the start.  What bounded the form before -- a wave per
+// tile, four tiles and a copy of the 16 queries in LDS per block -- was its length (272 matrix instructions in a row behind the staging) on 17 to 65 work-groups: 25 us for 540 keys of
+// 512 + 64 dimensions and 32 heads; now 6.7 (and 3.4 instead of 7.2 for the merge below).  Partials: per (key tile, head) R unnormalised outputs, then the maximum and the sum.
+#define LA_PIECES 9 // pieces of 16 dimensions that a wave has in flight: all of them up to 576 dimensions
+template <int G>
+__global__ __launch_bounds__(256) void latent_absorbed_kernel(const ps_seq_step *step, long long ring_off, int cap, const float *qa, int dr, int H, int R, int window, float scale,
+                                                              float *part) {
+    __shared__ __attribute__((aligned(16))) float sc[4][16 * 20];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4, h0 = blockIdx.y * 16;
-    const int qld = R + dr + 4;
-    float *qs = lds, *pt = lds + 16 * qld + wave * 16 * 17;
     const long long p = step->pos0;
     const long long lo = p - window + 1 > 0 ? p - window + 1 : 0;
-    const int half = rot_dims / 2;
-    // the 16 heads' folded queries and rotated parts into LDS: wave w takes rows w, w + 4, ...; every head turns by the same angles
-    for (int r = wave; r < 16; r += 4) {
-        const int h = h0 + r;
-        float *qr = qs + r * qld;
-        for (int c = lane; c < R; c += 64) qr[c] = h < H ? qa[(long long)h * R + c] : 0.f;
-        for (int c = 2 * half + lane; c < dr; c += 64) qr[R + c] = h < H ? q[(long long)h * qstride + d + c] : 0.f;
-    }
-    for (int i = lane; i < half; i += 64) {
-        const float ang = (float)p * freq[i], cs = cosf(ang) * rot_mag, sn = sinf(ang) * rot_mag;
-        int pa, pb;
-        la_pair(i, half, pairing, pa, pb);
-        for (int r = wave; r < 16; r += 4) {
-            const int h = h0 + r;
-            const float *qt = q + (long long)(h < H ? h : 0) * qstride + d;
-            const float u = h < H ? qt[pa] : 0.f, v = h < H ? qt[pb] : 0.f;
-            qs[r * qld + R + pa] = u * cs - v * sn;
-            qs[r * qld + R + pb] = v * cs + u * sn;
+    const int j0 = blockIdx.x * 16, n = (int)(p - lo) + 1;
+    if (j0 >= n) return;
+    const la_src ring = la_ring(step->state + ring_off, R + dr, lo, cap); // keys counted from position lo
+    const float *kr = la_row(ring, min(j0 + lr, n - 1)) + 4 * lq, *qr = qa + (long long)min(h0 + lr, H - 1) * (R + dr) + 4 * lq; // (a key or head that is not there: the last, masked below)
+    const int pieces = (R + dr) / 16;
+    la_f4 s4 = {0.f, 0.f, 0.f, 0.f}, v[G][4];
+    for (int u0 = wave; u0 < pieces; u0 += 4 * LA_PIECES) {
+        la_f4 a[LA_PIECES], b[LA_PIECES];
+#pragma unroll
+        for (int u = 0; u < LA_PIECES; u++) {
+            const bool in = u0 + 4 * u < pieces; // (uniform)
+            a[u] = in ? *(const la_f4 *)(qr + 16 * (u0 + 4 * u)) : la_f4{0.f, 0.f, 0.f, 0.f};
+            b[u] = in ? *(const la_f4 *)(kr + 16 * (u0 + 4 * u)) : la_f4{0.f, 0.f, 0.f, 0.f};
         }
+#pragma unroll
+        for (int u = 0; u < LA_PIECES; u++)
+            if (u0 + 4 * u < pieces)
+#pragma unroll
+                for (int e = 0; e < 4; e++) s4 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][e], b[u][e], s4, 0, 0, 0);
     }
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) { // the value of key 4 (l / 16) + kk: the order in which the soft-max leaves its weights
+        const float *vr = la_row(ring, min(j0 + 4 * lq + kk, n - 1)) + 4 * lr;
+#pragma unroll
+        for (int g = 0; g < G; g++) v[g][kk] = 64 * (wave + 4 * g) + 4 * lr < R ? *(const la_f4 *)(vr + 64 * (wave + 4 * g)) : la_f4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) sc[wave][(4 * lq + i) * 20 + lr] = s4[i];
     __syncthreads();
-    const long long tile = (long long)blockIdx.x * 4 + wave, j0 = lo + tile * 16;
-    const float *ring = step->state + ring_off;
-    const la_src k1 = la_ring(ring, R + dr, lo, cap), k2 = la_ring(ring + R, R + dr, lo, cap); // keys counted from position lo
-    struct { int rows, lq; __device__ __forceinline__ bool sees(int, int i, int) const { return 4 * lq + i < rows; } } see{H - h0, lq};
-    float m[1][4], l[1][4];
-    la_f4 acc[1][NJ];
+    la_f4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; i++) { m[0][i] = -INFINITY; l[0][i] = 0.f; }
+    for (int w = 0; w < 4; w++) s += *(const la_f4 *)(&sc[w][lr * 20 + 4 * lq]);
+    float m = -INFINITY, l = 0.f, pw[4];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) acc[0][j] = la_f4{0.f, 0.f, 0.f, 0.f};
-    if (j0 <= p) la_tiles<NJ, 1, false>(qs, qld, pt, k1, k2, k1, R, dr, R, (int)(j0 - lo), (int)(p - lo) + 1, see, scale, m, l, acc);
+    for (int kk = 0; kk < 4; kk++) {
+        s[kk] = j0 + 4 * lq + kk < n ? s[kk] * scale : -INFINITY;
+        m = fmaxf(m, s[kk]);
+    }
+    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
+        pw[kk] = m == -INFINITY ? 0.f : la_exp(s[kk] - m);
+        l += pw[kk];
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
     // partial of (tile, head): [o[R], m, l, -, -] (rows of R + 4 floats: 16-byte stores)
+    float *pp = part + ((long long)blockIdx.x * H + h0) * (R + 4);
+    if (wave == 0 && lq == 0 && h0 + lr < H) { pp[(long long)lr * (R + 4) + R] = m; pp[(long long)lr * (R + 4) + R + 1] = l; }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int h = h0 + 4 * lq + i;
-        if (h >= H) continue;
-        float *pp = part + ((long long)tile * H + h) * (R + 4);
-        if (lr == 0) { pp[R] = m[0][i]; pp[R + 1] = l[0][i]; }
+    for (int g = 0; g < G; g++) {
+        const int c = 64 * (wave + 4 * g) + 4 * lr;
+        if (64 * (wave + 4 * g) >= R) break; // (uniform)
+        la_f4 acc[4];
 #pragma unroll
-        for (int J = 0; J < NJ / 4; J++) {
-            const int c = 64 * J + 4 * lr;
-            if (c < R) *(la_f4 *)(pp + c) = la_f4{acc[0][4 * J][i], acc[0][4 * J + 1][i], acc[0][4 * J + 2][i], acc[0][4 * J + 3][i]};
+        for (int jj = 0; jj < 4; jj++) {
+            acc[jj] = la_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) acc[jj] = __builtin_amdgcn_mfma_f32_16x16x4f32(pw[kk], v[g][kk][jj], acc[jj], 0, 0, 0);
         }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (h0 + 4 * lq + i < H && c < R) *(la_f4 *)(pp + (long long)(4 * lq + i) * (R + 4) + c) = la_f4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
     }
 }
-// ol[h][c] = sum_tiles exp(m_t - M) o_t[c] / sum_tiles exp(m_t - M) l_t
+// ol[h][c] = sum_tiles exp(m_t - M) o_t[c] / sum_tiles exp(m_t - M) l_t: block = 64 columns of a head, each wave a quarter of the tiles
 __global__ __launch_bounds__(256) void latent_combine_kernel(const ps_seq_step *step, const float *part, int H, int R, int window, int max_tiles, float *ol) {
-    extern __shared__ float wts[]; // [max_tiles] weights exp(m_t - M), then their l-weighted sum in red
-    __shared__ float red[4];
-    const int h = blockIdx.x, tid = threadIdx.x;
+    extern __shared__ float wts[]; // [max_tiles] weights exp(m_t - M)
+    __shared__ float red[8], sum[4][64];
+    const int h = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = blockIdx.y * 64 + lane;
     const long long p = step->pos0, lo = p - window + 1 > 0 ? p - window + 1 : 0;
     int nt = (int)((p - lo) / 16 + 1);
     if (nt > max_tiles) nt = max_tiles;
+    const float *ph = part + (long long)h * (R + 4);
+    const long long ts = (long long)H * (R + 4);
     float mx = -INFINITY;
-    for (int t = tid; t < nt; t += 256) mx = fmaxf(mx, part[((long long)t * H + h) * (R + 4) + R]);
+    for (int t = tid; t < nt; t += 256) mx = fmaxf(mx, ph[t * ts + R]);
     mx = la_wave_max(mx);
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    if (lane == 0) red[wave] = mx;
     __syncthreads();
     const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    __syncthreads();
     float ls = 0.f;
     for (int t = tid; t < nt; t += 256) {
-        const float *pp = part + ((long long)t * H + h) * (R + 4) + R;
-        const float w = pp[0] == -INFINITY ? 0.f : expf(pp[0] - M);
+        const float m = ph[t * ts + R], w = m == -INFINITY ? 0.f : expf(m - M);
         wts[t] = w;
-        ls = fmaf(w, pp[1], ls);
+        ls = fmaf(w, ph[t * ts + R + 1], ls);
     }
     ls = la_wave_sum(ls);
-    if ((tid & 63) == 0) red[tid >> 6] = ls;
+    if (lane == 0) red[4 + wave] = ls;
     __syncthreads();
-    const float L = red[0] + red[1] + red[2] + red[3];
-    for (int c = tid; c < R; c += 256) {
-        float a = 0.f;
+    float a = 0.f;
+    if (c < R) {
 #pragma unroll 8
-        for (int t = 0; t < nt; t++) a = fmaf(wts[t], part[((long long)t * H + h) * (R + 4) + c], a);
-        ol[(long long)h * R + c] = a / L;
+        for (int t = wave; t < nt; t += 4) a = fmaf(wts[t], ph[t * ts + c], a);
     }
+    sum[wave][lane] = a;
+    __syncthreads();
+    if (wave == 0 && c < R) ol[(long long)h * R + c] = ((sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane])) / (red[4] + red[5] + red[6] + red[7]);
 }
 
-bool psk_latent_absorbed_ok(int d, int dr, int dv, int R) { return R % 16 == 0 && dr % 16 == 0 && R <= 512 && (size_t)(16 * (R + dr + 4) + 4 * 16 * 17) * 4 <= 160 * 1024; }
-size_t psk_latent_absorbed_scratch(int H, int R, int window) { return ((size_t)((window + 15) / 16 + 4) * H * (R + 4) + (size_t)2 * H * R) * 4; }
+bool psk_latent_absorbed_ok(int d, int dr, int dv, int R) { return R % 16 == 0 && dr % 16 == 0 && R <= 512 && R + dr <= 2480; }
+size_t psk_latent_absorbed_scratch(int H, int R, int dr, int window) { return ((size_t)((window + 15) / 16 + 1) * H * (R + 4) + (size_t)H * (2 * R + dr)) * 4; }
 // q [H][d + dr] (row stride qstride) -> o [H * dv]; ukv: rows uk | uv of the expansion matrix [H d + H dv][R]; scratch from psk_latent_absorbed_scratch
 void psk_latent_absorbed(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int qstride, const ps_dense *ukv, const float *freq,
                          int H, int d, int dr, int rot_dims, int dv, int R, int window, float scale, float *scratch, float *o, float rot_mag, const float *gate, int pairing) {
     const int max_tiles = (window + 15) / 16 + 1; // (a window that does not start on a tile's edge touches one tile more)
-    float *qa = scratch, *ol = qa + (size_t)H * R, *part = ol + (size_t)H * R;
+    float *qa = scratch, *ol = qa + (size_t)H * (R + dr), *part = ol + (size_t)H * R;
     const bool bf = ukv->dtype == PS_BF16;
-    if (bf) hipLaunchKernelGGL(latent_fold_q_kernel<unsigned short>, dim3(H, (R + 63) / 64), dim3(256), 0, st, q, qstride, (const unsigned short *)ukv->data, d, R, qa);
-    else hipLaunchKernelGGL(latent_fold_q_kernel<float>, dim3(H, (R + 63) / 64), dim3(256), 0, st, q, qstride, (const float *)ukv->data, d, R, qa);
-    const size_t lds = (size_t)(16 * (R + dr + 4) + 4 * 16 * 17) * 4;
-    const dim3 grid((max_tiles + 3) / 4, (H + 15) / 16);
-    if (R <= 128) {
-        static unsigned long long mask = 0;
-        if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)latent_absorbed_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        hipLaunchKernelGGL(latent_absorbed_kernel<8>, grid, dim3(256), lds, st, step, (long long)ring_off, cap, qa, q, qstride, d, dr, rot_dims, freq, H, R, window, scale, part, rot_mag, pairing);
-    } else {
-        static unsigned long long mask = 0;
-        if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)latent_absorbed_kernel<32>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        hipLaunchKernelGGL(latent_absorbed_kernel<32>, grid, dim3(256), lds, st, step, (long long)ring_off, cap, qa, q, qstride, d, dr, rot_dims, freq, H, R, window, scale, part, rot_mag, pairing);
-    }
-    hipLaunchKernelGGL(latent_combine_kernel, dim3(H), dim3(256), (size_t)grid.x * 4 * 4, st, step, part, H, R, window, (int)grid.x * 4, ol);
+    const dim3 fold(H, (R + 63) / 64 + 1), grid(max_tiles, (H + 15) / 16);
+    if (bf) hipLaunchKernelGGL(latent_fold_q_kernel<unsigned short>, fold, dim3(256), 0, st, step, q, qstride, (const unsigned short *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa);
+    else hipLaunchKernelGGL(latent_fold_q_kernel<float>, fold, dim3(256), 0, st, step, q, qstride, (const float *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa);
+    const auto attend = R <= 256 ? latent_absorbed_kernel<1> : latent_absorbed_kernel<2>;
+    hipLaunchKernelGGL(attend, grid, dim3(256), 0, st, step, (long long)ring_off, cap, qa, dr, H, R, window, scale, part);
+    hipLaunchKernelGGL(latent_combine_kernel, dim3(H, (R + 63) / 64), dim3(256), (size_t)max_tiles * 4, st, step, part, H, R, window, max_tiles, ol);
     const int rows = H * dv;
     if (bf) hipLaunchKernelGGL(latent_unfold_v_kernel<unsigned short>, dim3((rows + 3) / 4), dim3(256), 0, st, ol, (const unsigned short *)ukv->data + (size_t)H * d * R, dv, R, rows, o, gate);
     else hipLaunchKernelGGL(latent_unfold_v_kernel<float>, dim3((rows + 3) / 4), dim3(256), 0, st, ol, (const float *)ukv->data + (size_t)H * d * R, dv, R, rows, o, gate);

@@ -205,7 +205,7 @@ void psk_latent_attn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_
 // Single-token step in the absorbed form: nothing is expanded per key, the ring's latents are keys and values for all heads at once.
 // q [H][d + dr] (row stride qstride, rotated part not yet rotated) -> o [H * dv].  ukv: rows uk | uv.  _ok: kv_rank, dr multiples of 16, kv_rank <= 512.
 bool psk_latent_absorbed_ok(int d, int dr, int dv, int R);
-size_t psk_latent_absorbed_scratch(int H, int R, int window);
+size_t psk_latent_absorbed_scratch(int H, int R, int dr, int window);
 void psk_latent_absorbed(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int qstride, const ps_dense *ukv, const float *freq,
                          int H, int d, int dr, int rot_dims, int dv, int R, int window, float scale, float *scratch, float *o, float rot_mag = 1.f,
                          const float *gate = nullptr, int pairing = PS_ROT_HALVES);

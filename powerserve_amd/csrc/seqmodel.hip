@@ -465,7 +465,7 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         size_t ab = 0;
         mixers([&](LayerPlan &P) {
             if (P.d.kind == PS_MIX_LATENT && psk_latent_absorbed_ok(P.d.dim, P.d.rot_dim, P.d.vdim, P.d.kv_rank))
-                ab = std::max(ab, psk_latent_absorbed_scratch(P.d.heads, P.d.kv_rank, P.d.window));
+                ab = std::max(ab, psk_latent_absorbed_scratch(P.d.heads, P.d.kv_rank, P.d.rot_dim, P.d.window));
         });
         if (ab) ok = ok && alloc((void **)&m->abs_scratch, ab);
         size_t wb = 0;
