@@ -7,6 +7,7 @@
 // at a time through LDS, where their per-token scalars are reduced once for all columns.
 #include "ps_seq.h"
 
+#include <algorithm>
 #include <cmath>
 
 static __device__ __forceinline__ float sq_block_sum(float v, float *red) { // 256 threads
@@ -16,6 +17,15 @@ static __device__ __forceinline__ float sq_block_sum(float v, float *red) { // 2
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     return red[0] + red[1] + red[2] + red[3];
+}
+typedef float sq_f4 __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane gets it: rotations inside a row of sixteen, then the four rows' sums (no trip through LDS)
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));
+    auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    return (row(0) + row(16)) + (row(32) + row(48));
 }
 static __device__ __forceinline__ float sq_silu(float x) { return x / (1.f + expf(-x)); }
 static __device__ __forceinline__ float sq_softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
@@ -34,9 +44,53 @@ __global__ __launch_bounds__(256) void sq_rmsnorm_kernel(const float *x, long lo
     float *yr = y + (long long)blockIdx.x * ldy + part;
     for (long long i = threadIdx.x; i < n; i += 256) yr[i] = xr[i] * inv * (offset + w[i]);
 }
+// The same with a part's numbers held in registers, C runs of four per thread, the weights requested along with them: one trip to memory instead of three.  One row of 4096: 7.4 us
+// with the loops, 4.0 now.
+template <int C>
+__global__ __launch_bounds__(1024) void sq_rmsnorm_fast_kernel(const float *x, long long ldx, const int32_t *idx, const float *w, float offset, float eps, int n, float *y, long long ldy) {
+    __shared__ float red[16];
+    const long long r = idx ? idx[blockIdx.x] : blockIdx.x, part = (long long)blockIdx.y * n;
+    const float *xr = x + r * ldx + part;
+    const int tid = threadIdx.x, nw = blockDim.x >> 6;
+    sq_f4 v[C], g[C];
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = (tid + c * (int)blockDim.x) * 4;
+        v[c] = i < n ? *(const sq_f4 *)(xr + i) : sq_f4{0.f, 0.f, 0.f, 0.f};
+        g[c] = i < n ? *(const sq_f4 *)(w + part + i) : sq_f4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) s += v[c][e] * v[c][e];
+    s = sq_wave_sum(s);
+    if ((tid & 63) == 0) red[tid >> 6] = s;
+    __syncthreads();
+    s = 0.f;
+    for (int u = 0; u < nw; u++) s += red[u];
+    const float inv = 1.f / sqrtf(s / (float)n + eps);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = (tid + c * (int)blockDim.x) * 4;
+        sq_f4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = v[c][e] * inv * (offset + g[c][e]);
+        if (i < n) *(sq_f4 *)(y + (long long)blockIdx.x * ldy + part + i) = o;
+    }
+}
 void psk_rmsnorm(hipStream_t st, const float *x, int64_t ldx, const int32_t *idx, const float *w, float offset, float eps, int64_t n, int rows, float *y, int64_t ldy,
                  int groups) {
     if (rows <= 0) return;
+    const int64_t part = n / groups;
+    if (part % 4 == 0 && part <= 8192 && ldx % 4 == 0 && ldy % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0) {
+        // (a single row has the chip to itself: a run per thread; of many rows each takes a quarter of a CU's threads and more runs in flight)
+        const int c = rows <= 8 ? (part <= 4096 ? 1 : 2) : part <= 1024 ? 1 : part <= 2048 ? 2 : part <= 4096 ? 4 : 8;
+        const int threads = (int)((part / 4 + c - 1) / c + 63) / 64 * 64;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows, groups), dim3(threads), 0, st, x, (long long)ldx, idx, w, offset, eps, (int)part, y, (long long)ldy); };
+        c == 1 ? go(sq_rmsnorm_fast_kernel<1>) : c == 2 ? go(sq_rmsnorm_fast_kernel<2>) : c == 4 ? go(sq_rmsnorm_fast_kernel<4>) : go(sq_rmsnorm_fast_kernel<8>);
+        return;
+    }
     hipLaunchKernelGGL(sq_rmsnorm_kernel, dim3(rows, groups), dim3(256), 0, st, x, (long long)ldx, idx, w, offset, eps, (long long)(n / groups), y, (long long)ldy);
 }
 
@@ -224,6 +278,84 @@ void psk_copy(hipStream_t st, const float *src, float *dst, int64_t n) {
 
 // A single token's sublayer boundary in one launch (one block):  x += y / rms(y) * (offset + wb)   (where y is given), then, where wn is given,
 // h = conv(x / rms(x) * (offset + wn)) with the convolution's residual form and its tail brought up to date -- three launches of the kernels above.
+// What bounds it is the latency of a chain: read, sum, read, sum, read.  So a thread owns C runs of four channels and requests everything that it will need of them -- x, y, both weights,
+// the filter's taps and the tail -- before the first sum, and keeps it in registers.  TAPS: 0 where wn is not given, else the taps.  n = 4096, 4 taps: 12.6 us with a loop per sum, 6.2 now;
+// n = 2048 without the second half: 2.8 to 4.6 and 2.0 to 3.9.
+template <int TAPS, int C>
+__global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw,
+                                                                 long long tail_off, float offset, float eps, int n, float *h, float *hn) {
+    __shared__ float red[2][16];
+    const int tid = threadIdx.x, nw = blockDim.x >> 6;
+    auto block_sum = [&](float v, float *r) {
+        v = sq_wave_sum(v);
+        if ((tid & 63) == 0) r[tid >> 6] = v;
+        __syncthreads();
+        float t = 0.f;
+        for (int w = 0; w < nw; w++) t += r[w];
+        return t;
+    };
+    const sq_f4 zero = {0.f, 0.f, 0.f, 0.f};
+    sq_f4 xv[C], yv[C], b4[C], n4[C], f[C][TAPS ? TAPS : 1], tl[C][TAPS > 1 ? TAPS - 1 : 1];
+    float *tail = TAPS > 1 ? step->state + tail_off : nullptr;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = (tid + c * (int)blockDim.x) * 4;
+        const bool in = i < n;
+        yv[c] = in && y ? *(const sq_f4 *)(y + i) : zero;
+        xv[c] = in ? *(const sq_f4 *)(x + i) : zero;
+        b4[c] = in && y ? *(const sq_f4 *)(wb + i) : zero;
+        if constexpr (TAPS > 0) {
+            n4[c] = in ? *(const sq_f4 *)(wn + i) : zero;
+#pragma unroll
+            for (int j = 0; j < TAPS; j++) f[c][j] = in ? *(const sq_f4 *)(cw + (long long)i * TAPS + 4 * j) : zero;
+#pragma unroll
+            for (int j = 0; j + 1 < TAPS; j++) tl[c][j] = in ? *(const sq_f4 *)(tail + (long long)j * n + i) : zero;
+        }
+    }
+    if (y) {
+        float s1 = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s1 += yv[c][e] * yv[c][e];
+        const float inv = 1.f / sqrtf(block_sum(s1, red[0]) / (float)n + eps);
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int i = (tid + c * (int)blockDim.x) * 4;
+#pragma unroll
+            for (int e = 0; e < 4; e++) xv[c][e] = xv[c][e] + yv[c][e] * inv * (offset + b4[c][e]);
+            if (i < n) *(sq_f4 *)(x + i) = xv[c];
+        }
+    }
+    if constexpr (TAPS > 0) {
+        float s2 = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s2 += xv[c][e] * xv[c][e];
+        const float inv = 1.f / sqrtf(block_sum(s2, red[1]) / (float)n + eps);
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int i = (tid + c * (int)blockDim.x) * 4;
+            if (i >= n) continue;
+            sq_f4 v, o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = xv[c][e] * inv * (offset + n4[c][e]);
+                auto tap = [&](int j) { return f[c][(e * TAPS + j) / 4][(e * TAPS + j) % 4]; };
+                float t = tap(TAPS - 1) * v[e];
+#pragma unroll
+                for (int j = 0; j + 1 < TAPS; j++) t = fmaf(tap(j), tl[c][j][e], t);
+                o[e] = v[e] + t;
+            }
+            if (hn) *(sq_f4 *)(hn + i) = v;
+            *(sq_f4 *)(h + i) = o;
+#pragma unroll
+            for (int j = 0; j + 1 < TAPS; j++) *(sq_f4 *)(tail + (long long)j * n + i) = j + 2 < TAPS ? tl[c][j + 2 < TAPS ? j + 1 : 0] : v;
+        }
+    }
+}
+// any width, any number of taps
 __global__ __launch_bounds__(1024) void sq_boundary1_kernel(const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw,
                                                             int taps, long long tail_off, float offset, float eps, long long n, float *h, float *hn) {
     __shared__ float red[16];
@@ -266,14 +398,26 @@ __global__ __launch_bounds__(1024) void sq_boundary1_kernel(const ps_seq_step *s
 }
 void psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
                    float offset, float eps, int64_t n, float *h, float *hn) {
+    auto aligned = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
+    const int t = wn ? taps : 0;
+    if (n % 4 == 0 && n <= 8192 && tail_off % 4 == 0 && (t == 0 || t == 1 || t == 4) && aligned(x) && aligned(y) && aligned(wb) && aligned(wn) && aligned(cw) && aligned(h) && aligned(hn)) {
+        const int threads = (int)std::min<int64_t>((n / 4 + 63) / 64 * 64, 1024);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), 0, st, step, x, y, wb, wn, cw, (long long)tail_off, offset, eps, (int)n, h, hn);
+        };
+        if (n <= 4096) t == 0 ? go(sq_boundary1_fast_kernel<0, 1>) : t == 1 ? go(sq_boundary1_fast_kernel<1, 1>) : go(sq_boundary1_fast_kernel<4, 1>);
+        else t == 0 ? go(sq_boundary1_fast_kernel<0, 2>) : t == 1 ? go(sq_boundary1_fast_kernel<1, 2>) : go(sq_boundary1_fast_kernel<4, 2>);
+        return;
+    }
     hipLaunchKernelGGL(sq_boundary1_kernel, dim3(1), dim3(n >= 2048 ? 1024 : 256), 0, st, step, x, y, wb, wn, cw, taps, (long long)tail_off, offset, eps, (long long)n, h, hn);
 }
 
 // ---------------------------------------------------------------------------------------------------- recurrent scans
-typedef float sq_f4 __attribute__((ext_vector_type(4)));
 #define SQ_NR 16 // state rows per lane (lane s of a column holds rows 16 s .. 16 s + 15: its per-token vectors are four 16-byte LDS reads each)
 #define SQ_TC 8  // tokens staged per round
 #define SQ_PF 8  // staged numbers per thread and vector: SQ_TC * 16 R / 256 <= 8 for R <= 16
+// (The scans of a decoded token are compiled with TC = 1: with rounds of eight they staged, decayed and summed seven tokens that are not there.  32 heads of 128 x 128:
+// wkv 12.0 -> 5.6 us, delta 11.3 -> 7.5 us; 64 heads of 64 x 128, state space: 8.2 -> 4.8 us.)
 static inline int sq_lanes_per_col(int d) { int R = 1; while (R * SQ_NR < d) R *= 2; return R; }
 
 
@@ -300,13 +444,13 @@ static __device__ __forceinline__ float sq_col_sum(float v, int R) {
 //   GLA = 0 (wkv)  o_j = sum_i r_i (S_ij + bonus_i k_i v_j), then S_ij <- w_i S_ij + k_i v_j,  w = exp(-exp(z))
 //   GLA = 1        S_ij <- w_i S_ij + k_i v_j, then o_j = sum_i (qscale r_i) S_ij,              w = sigmoid(z)^inv_tau = exp(-softplus(-z) inv_tau)
 // LDS: rs, ks, ws [TC][dp] (dp = NR * R, rows >= d zero), sc [TC] (sum_i r_i bonus_i k_i)
-template <int GLA>
+template <int GLA, int TC>
 __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *step, long long state_off, const float *r, const float *k, const float *v, const float *z,
                                                             long long ld, long long ldz, const float *bonus, int d, int dv, float qscale, float inv_tau, int R, int T,
                                                             float *o, long long ldo) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int dp = SQ_NR * R, cpb = 256 / R;
-    float *rs = lds, *ks = rs + SQ_TC * dp, *ws = ks + SQ_TC * dp, *sc = ws + SQ_TC * dp;
+    float *rs = lds, *ks = rs + TC * dp, *ws = ks + TC * dp, *sc = ws + TC * dp;
     const int h = blockIdx.y, tid = threadIdx.x, s = tid % R, j = blockIdx.x * cpb + tid / R;
     const bool col = j < dv;
     float *S0 = step->state + state_off + (long long)h * d * dv;
@@ -318,40 +462,40 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
     }
     const long long hb = (long long)h * d, vb = (long long)h * dv;
     // the next round's inputs are requested before the current round's steps run, and land in LDS after them
-    float pa[SQ_PF], pb[SQ_PF], pc[SQ_PF], pv[SQ_TC];
+    float pa[TC], pb[TC], pc[TC], pv[TC];
     auto fetch = [&](int t0) {
-        const int nt = min(SQ_TC, T - t0);
+        const int nt = min(TC, T - t0);
 #pragma unroll
-        for (int e = 0; e < SQ_PF; e++) {
+        for (int e = 0; e < TC; e++) {
             const int x = tid + 256 * e, t = x / dp, i = x % dp;
-            const bool in = x < SQ_TC * dp && t < nt && i < d;
+            const bool in = x < TC * dp && t < nt && i < d;
             const long long at = (long long)(t0 + (in ? t : 0)) * ld + hb + (in ? i : 0);
             pa[e] = in ? r[at] : 0.f;
             pb[e] = in ? k[at] : 0.f;
             pc[e] = in ? z[(long long)(t0 + t) * ldz + hb + i] : (GLA ? INFINITY : -INFINITY); // w = 1: with k = 0 a token that is not there leaves the state alone
         }
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) pv[t] = (col && t < nt) ? v[(long long)(t0 + t) * ld + vb + j] : 0.f;
+        for (int t = 0; t < TC; t++) pv[t] = (col && t < nt) ? v[(long long)(t0 + t) * ld + vb + j] : 0.f;
     };
     fetch(0);
-    for (int t0 = 0; t0 < T; t0 += SQ_TC) {
-        const int nt = min(SQ_TC, T - t0);
+    for (int t0 = 0; t0 < T; t0 += TC) {
+        const int nt = min(TC, T - t0);
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < SQ_PF; e++) {
+        for (int e = 0; e < TC; e++) {
             const int x = tid + 256 * e;
-            if (x < SQ_TC * dp) {
+            if (x < TC * dp) {
                 rs[x] = GLA ? pa[e] * qscale : pa[e];
                 ks[x] = pb[e];
                 ws[x] = GLA ? expf(-sq_softplus(-pc[e]) * inv_tau) : expf(-expf(pc[e]));
             }
         }
-        float vj[SQ_TC];
+        float vj[TC];
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) vj[t] = pv[t];
+        for (int t = 0; t < TC; t++) vj[t] = pv[t];
         __syncthreads();
-        if (t0 + SQ_TC < T) fetch(t0 + SQ_TC);
-        for (int t = tid >> 6; !GLA && t < SQ_TC; t += 4) { // one wave per token
+        if (t0 + TC < T) fetch(t0 + TC);
+        for (int t = tid >> 6; !GLA && t < TC; t += 4) { // one wave per token
             float a = 0.f;
             for (int i = tid & 63; i < d; i += 64) a += rs[t * dp + i] * bonus[hb + i] * ks[t * dp + i];
 #pragma unroll
@@ -361,7 +505,7 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
         __syncthreads();
         // (no branch per token: the steps of a round are one block of straight-line code the compiler can interleave; padded tokens are neutral)
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) {
+        for (int t = 0; t < TC; t++) {
             {
                 const sq_f4 *rt = (const sq_f4 *)(rs + t * dp + s * SQ_NR), *kt = (const sq_f4 *)(ks + t * dp + s * SQ_NR), *wt = (const sq_f4 *)(ws + t * dp + s * SQ_NR);
                 float pp[4] = {0.f, 0.f, 0.f, 0.f}; // four short chains instead of one of sixteen
@@ -393,25 +537,30 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
 void psk_wkv_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *r, const float *k, const float *v, const float *z, int64_t ld,
                   const float *bonus, int H, int d, int T, float *o, int64_t ldo) {
     const int R = sq_lanes_per_col(d), cpb = 256 / R;
-    const size_t lds = (size_t)(3 * SQ_TC * SQ_NR * R + SQ_TC) * 4;
-    hipLaunchKernelGGL(sq_decay_scan_kernel<0>, dim3((d + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, r, k, v, z, (long long)ld, (long long)ld, bonus, d, d, 1.f, 1.f,
+    const int tc = T == 1 ? 1 : SQ_TC;
+    const size_t lds = (size_t)(3 * tc * SQ_NR * R + tc) * 4;
+    const auto kernel = T == 1 ? sq_decay_scan_kernel<0, 1> : sq_decay_scan_kernel<0, SQ_TC>;
+    hipLaunchKernelGGL(kernel, dim3((d + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, r, k, v, z, (long long)ld, (long long)ld, bonus, d, d, 1.f, 1.f,
                        R, T, o, (long long)ldo);
 }
 void psk_gla_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *q, const float *k, const float *v, int64_t ld, const float *z, int64_t ldz,
                   float tau, int H, int d, int dv, int T, float *o, int64_t ldo) {
     const int R = sq_lanes_per_col(d), cpb = 256 / R;
-    const size_t lds = (size_t)(3 * SQ_TC * SQ_NR * R + SQ_TC) * 4;
-    hipLaunchKernelGGL(sq_decay_scan_kernel<1>, dim3((dv + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, q, k, v, z, (long long)ld, (long long)ldz, nullptr, d, dv,
+    const int tc = T == 1 ? 1 : SQ_TC;
+    const size_t lds = (size_t)(3 * tc * SQ_NR * R + tc) * 4;
+    const auto kernel = T == 1 ? sq_decay_scan_kernel<1, 1> : sq_decay_scan_kernel<1, SQ_TC>;
+    hipLaunchKernelGGL(kernel, dim3((dv + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, q, k, v, z, (long long)ld, (long long)ldz, nullptr, d, dv,
                        1.f / sqrtf((float)d), 1.f / tau, R, T, o, (long long)ldo);
 }
 
 // LDS: qs, ks [TC][dp]; per token: g, beta, kq
+template <int TC>
 __global__ __launch_bounds__(256) void sq_delta_scan_kernel(const ps_seq_step *step, long long state_off, const float *q, const float *k, const float *v,
                                                             const float *braw, const float *araw, long long ld, long long ldb, const float *a_log, const float *dt_bias, int H,
                                                             int KH, int d, int dv, int R, int T, float *o, long long ldo) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int dp = SQ_NR * R, cpb = 256 / R;
-    float *qs = lds, *ks = qs + SQ_TC * dp, *gs = ks + SQ_TC * dp, *bs = gs + SQ_TC, *kq = bs + SQ_TC;
+    float *qs = lds, *ks = qs + TC * dp, *gs = ks + TC * dp, *bs = gs + TC, *kq = bs + TC;
     const int h = blockIdx.y, tid = threadIdx.x, s = tid % R, j = blockIdx.x * cpb + tid / R;
     const bool col = j < dv;
     float *S0 = step->state + state_off + (long long)h * d * dv;
@@ -423,47 +572,47 @@ __global__ __launch_bounds__(256) void sq_delta_scan_kernel(const ps_seq_step *s
     }
     const long long qb = (long long)(h / (H / KH)) * d, vb = (long long)h * dv;
     const float qscale = 1.f / sqrtf((float)d), na = -expf(a_log[h]), db = dt_bias[h];
-    float pa[SQ_PF], pb[SQ_PF], pv[SQ_TC], pg = 0.f, pbeta = 0.f;
+    float pa[TC], pb[TC], pv[TC], pg = 0.f, pbeta = 0.f;
     auto fetch = [&](int t0) {
-        const int nt = min(SQ_TC, T - t0);
+        const int nt = min(TC, T - t0);
 #pragma unroll
-        for (int e = 0; e < SQ_PF; e++) {
+        for (int e = 0; e < TC; e++) {
             const int x = tid + 256 * e, t = x / dp, i = x % dp;
-            const bool in = x < SQ_TC * dp && t < nt && i < d;
+            const bool in = x < TC * dp && t < nt && i < d;
             const long long at = (long long)(t0 + (in ? t : 0)) * ld + qb + (in ? i : 0);
             pa[e] = in ? q[at] : 0.f;
             pb[e] = in ? k[at] : 0.f;
         }
-        if (tid < SQ_TC) {
+        if (tid < TC) {
             const bool in = tid < nt;
             pg = in ? araw[(long long)(t0 + tid) * ldb + h] : 0.f;
             pbeta = in ? braw[(long long)(t0 + tid) * ldb + h] : -INFINITY; // sigmoid(-inf) = 0
         }
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) pv[t] = (col && t < nt) ? v[(long long)(t0 + t) * ld + vb + j] : 0.f;
+        for (int t = 0; t < TC; t++) pv[t] = (col && t < nt) ? v[(long long)(t0 + t) * ld + vb + j] : 0.f;
     };
     fetch(0);
-    for (int t0 = 0; t0 < T; t0 += SQ_TC) {
-        const int nt = min(SQ_TC, T - t0);
+    for (int t0 = 0; t0 < T; t0 += TC) {
+        const int nt = min(TC, T - t0);
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < SQ_PF; e++) {
+        for (int e = 0; e < TC; e++) {
             const int x = tid + 256 * e;
-            if (x < SQ_TC * dp) {
+            if (x < TC * dp) {
                 qs[x] = pa[e];
                 ks[x] = pb[e];
             }
         }
-        if (tid < SQ_TC) {
+        if (tid < TC) {
             gs[tid] = tid < nt ? expf(na * sq_softplus(pg + db)) : 1.f;
             bs[tid] = 1.f / (1.f + expf(-pbeta));
         }
-        float vj[SQ_TC];
+        float vj[TC];
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) vj[t] = pv[t];
+        for (int t = 0; t < TC; t++) vj[t] = pv[t];
         __syncthreads();
-        if (t0 + SQ_TC < T) fetch(t0 + SQ_TC);
-        for (int t = tid >> 6; t < SQ_TC; t += 4) { // one wave per token: unit vectors, then k . q
+        if (t0 + TC < T) fetch(t0 + TC);
+        for (int t = tid >> 6; t < TC; t += 4) { // one wave per token: unit vectors, then k . q
             float a = 0.f, b = 0.f;
             for (int i = tid & 63; i < d; i += 64) {
                 a += qs[t * dp + i] * qs[t * dp + i];
@@ -488,7 +637,7 @@ __global__ __launch_bounds__(256) void sq_delta_scan_kernel(const ps_seq_step *s
         }
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) {
+        for (int t = 0; t < TC; t++) {
             { // (padded tokens: g = 1, beta = 0, k = 0 -- the state stays)
                 const sq_f4 *qt = (const sq_f4 *)(qs + t * dp + s * SQ_NR), *kt = (const sq_f4 *)(ks + t * dp + s * SQ_NR);
                 const float g = gs[t];
@@ -524,8 +673,10 @@ __global__ __launch_bounds__(256) void sq_delta_scan_kernel(const ps_seq_step *s
 void psk_delta_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *q, const float *k, const float *v, const float *braw,
                     const float *araw, int64_t ld, int64_t ldb, const float *a_log, const float *dt_bias, int H, int KH, int d, int dv, int T, float *o, int64_t ldo) {
     const int R = sq_lanes_per_col(d), cpb = 256 / R;
-    const size_t lds = (size_t)(2 * SQ_TC * SQ_NR * R + 3 * SQ_TC) * 4;
-    hipLaunchKernelGGL(sq_delta_scan_kernel, dim3((dv + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, q, k, v, braw, araw, (long long)ld, (long long)ldb, a_log,
+    const int tc = T == 1 ? 1 : SQ_TC;
+    const size_t lds = (size_t)(2 * tc * SQ_NR * R + 3 * tc) * 4;
+    const auto kernel = T == 1 ? sq_delta_scan_kernel<1> : sq_delta_scan_kernel<SQ_TC>;
+    hipLaunchKernelGGL(kernel, dim3((dv + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, q, k, v, braw, araw, (long long)ld, (long long)ldb, a_log,
                        dt_bias, H, KH, d, dv, R, T, o, (long long)ldo);
 }
 
@@ -550,13 +701,13 @@ void psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, in
 // group of heads.  As above a column (one of P) evolves on its own and is spread over R lanes of 16 rows; here the state is kept column by column ([H][P][N]), so a lane's rows
 // are four 16-byte pieces and a column's lanes read one run.  A lane carries NC columns (cpb apart), so that B and C come out of LDS once for all of them.
 // LDS: cs, bs [TC][dp]; per token: g, dt
-template <int NC>
+template <int NC, int TC>
 __global__ __launch_bounds__(256) void sq_ssd_scan_kernel(const ps_seq_step *step, long long state_off, const float *x, const float *B, const float *C, long long ld,
                                                           const float *dtraw, long long ldb, const float *a_log, const float *dt_bias, const float *skip, int H, int G, int N,
                                                           int P, int R, int T, float *o, long long ldo) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int dp = SQ_NR * R, cpb = 256 / R;
-    float *cs = lds, *bs = cs + SQ_TC * dp, *gs = bs + SQ_TC * dp, *ds = gs + SQ_TC;
+    float *cs = lds, *bs = cs + TC * dp, *gs = bs + TC * dp, *ds = gs + TC;
     const int h = blockIdx.y, tid = threadIdx.x, s = tid % R, j0 = blockIdx.x * cpb * NC + tid / R;
     const bool vec = N % 16 == 0; // (a lane's 16 rows are then all there or all not, and 16-byte aligned)
     float *S0 = step->state + state_off + (long long)h * P * N;
@@ -581,49 +732,49 @@ __global__ __launch_bounds__(256) void sq_ssd_scan_kernel(const ps_seq_step *ste
     const long long nb = (long long)(h / (H / G)) * N, vb = (long long)h * P;
     const float na = -expf(a_log[h]), db = dt_bias[h], sk = skip[h];
     // the next round's inputs are requested before the current round's steps run
-    float pa[SQ_PF], pb[SQ_PF], pv[NC][SQ_TC], pd = 0.f;
+    float pa[TC], pb[TC], pv[NC][TC], pd = 0.f;
     auto fetch = [&](int t0) {
-        const int nt = min(SQ_TC, T - t0);
+        const int nt = min(TC, T - t0);
 #pragma unroll
-        for (int e = 0; e < SQ_PF; e++) {
+        for (int e = 0; e < TC; e++) {
             const int i0 = tid + 256 * e, t = i0 / dp, i = i0 % dp;
-            const bool in = i0 < SQ_TC * dp && t < nt && i < N;
+            const bool in = i0 < TC * dp && t < nt && i < N;
             const long long at = (long long)(t0 + (in ? t : 0)) * ld + nb + (in ? i : 0);
             pa[e] = in ? C[at] : 0.f;
             pb[e] = in ? B[at] : 0.f;
         }
-        if (tid < SQ_TC) pd = tid < nt ? dtraw[(long long)(t0 + tid) * ldb + h] : 0.f;
+        if (tid < TC) pd = tid < nt ? dtraw[(long long)(t0 + tid) * ldb + h] : 0.f;
 #pragma unroll
         for (int c = 0; c < NC; c++)
 #pragma unroll
-            for (int t = 0; t < SQ_TC; t++) pv[c][t] = (j0 + c * cpb < P && t < nt) ? x[(long long)(t0 + t) * ld + vb + j0 + c * cpb] : 0.f;
+            for (int t = 0; t < TC; t++) pv[c][t] = (j0 + c * cpb < P && t < nt) ? x[(long long)(t0 + t) * ld + vb + j0 + c * cpb] : 0.f;
     };
     fetch(0);
-    for (int t0 = 0; t0 < T; t0 += SQ_TC) {
-        const int nt = min(SQ_TC, T - t0);
+    for (int t0 = 0; t0 < T; t0 += TC) {
+        const int nt = min(TC, T - t0);
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < SQ_PF; e++) {
+        for (int e = 0; e < TC; e++) {
             const int i0 = tid + 256 * e;
-            if (i0 < SQ_TC * dp) {
+            if (i0 < TC * dp) {
                 cs[i0] = pa[e];
                 bs[i0] = pb[e];
             }
         }
-        if (tid < SQ_TC) { // (a token that is not there: g = 1, dt = 0 -- the state stays)
+        if (tid < TC) { // (a token that is not there: g = 1, dt = 0 -- the state stays)
             const float dt = tid < nt ? sq_softplus(pd + db) : 0.f;
             ds[tid] = dt;
             gs[tid] = expf(na * dt);
         }
-        float xv[NC][SQ_TC];
+        float xv[NC][TC];
 #pragma unroll
         for (int c = 0; c < NC; c++)
 #pragma unroll
-            for (int t = 0; t < SQ_TC; t++) xv[c][t] = pv[c][t];
+            for (int t = 0; t < TC; t++) xv[c][t] = pv[c][t];
         __syncthreads();
-        if (t0 + SQ_TC < T) fetch(t0 + SQ_TC);
+        if (t0 + TC < T) fetch(t0 + TC);
 #pragma unroll
-        for (int t = 0; t < SQ_TC; t++) {
+        for (int t = 0; t < TC; t++) {
             const sq_f4 *ct = (const sq_f4 *)(cs + t * dp + s * SQ_NR), *bt = (const sq_f4 *)(bs + t * dp + s * SQ_NR);
             const float g = gs[t], dt = ds[t];
             float u[NC], pp[NC][4];
@@ -670,9 +821,10 @@ __global__ __launch_bounds__(256) void sq_ssd_scan_kernel(const ps_seq_step *ste
 void psk_ssd_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *x, const float *B, const float *C, int64_t ld, const float *dtraw, int64_t ldb,
                   const float *a_log, const float *dt_bias, const float *skip, int H, int G, int N, int P, int T, float *o, int64_t ldo) {
     const int R = sq_lanes_per_col(N), cpb = 256 / R;
-    const size_t lds = (size_t)(2 * SQ_TC * SQ_NR * R + 2 * SQ_TC) * 4;
+    const int tc = T == 1 ? 1 : SQ_TC;
+    const size_t lds = (size_t)(2 * tc * SQ_NR * R + 2 * tc) * 4;
     const bool two = T > SQ_TC && P > cpb;
-    const auto kernel = two ? sq_ssd_scan_kernel<2> : sq_ssd_scan_kernel<1>;
+    const auto kernel = two ? sq_ssd_scan_kernel<2, SQ_TC> : T == 1 ? sq_ssd_scan_kernel<1, 1> : sq_ssd_scan_kernel<1, SQ_TC>;
     const int cols = two ? 2 * cpb : cpb;
     hipLaunchKernelGGL(kernel, dim3((P + cols - 1) / cols, H), dim3(256), lds, st, step, (long long)state_off, x, B, C, (long long)ld, dtraw, (long long)ldb, a_log, dt_bias, skip,
                        H, G, N, P, R, T, o, (long long)ldo);

@@ -113,6 +113,18 @@ def test_dense_matmul_any_shape(ctx, dtype, T, N, K):
     dx.free(); do.free()
 
 
+# a token at a time: boundaries and norms of one run per thread, a run and four numbers more, two runs, no multiple of four (the general kernels), one, two and four taps; the absorbed
+# attention with one and two groups of value columns per wave, heads in and one beyond a tile of 16, windows of one tile, one key more and of two tiles, more than nine pieces of a key per wave
+@pytest.mark.parametrize("width,taps,heads,rank,rot,window", [(64, 4, 1, 16, 16, 16), (4096, 1, 16, 64, 16, 17), (4100, 4, 17, 272, 16, 32), (4104, 1, 3, 512, 32, 5), (8192, 4, 2, 256, 336, 20),
+                                                            (66, 4, 2, 48, 16, 7), (132, 2, 2, 512, 80, 18)])
+def test_kernels_of_a_single_token(made, width, taps, heads, rank, rot, window):
+    cfg = synth.seq_config(width, 40, [L("latent_attention", 24, heads=heads, dim=16, vdim=12, q_rank=20, kv_rank=rank, mask={"size": window}, scale=0.3, rot={"base": 100.0, "dims": 12},
+                                         rot_dim=rot), L("wkv", None, heads=1, dim=20)], taps=taps)
+    m, c, t = made(f"one{width}.{rank}", max_batch=16, cfg=cfg)
+    toks = tokens_for(c, 45)
+    assert err(run_portions(m, toks, (1,)), seq_oracle.run(c, t, toks)) < TOL["float32"]
+
+
 # the wide mat-mul (k_dense.hip dense_mm_ring_kernel): one row more and less than its tiles of 64 and 128 tokens and outputs, one block of K and fewer blocks than stages,
 # products split along K (few tiles, long K: also uneven shares), more tiles than the chip has CUs
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
