@@ -4,7 +4,8 @@
 //   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
 //   dense_mm_narrow_kernel bf16, K 128 or 256, more than 8 tokens: 32 x 32 tiles, the waves share K
-//   dense_mv1_kernel<WT,FORM> a single token, or a few tokens' chosen experts: every wave streams its rows, the requests run ahead of everything else
+//   dense_mv1_kernel<WT,FORM> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
+//   dense_mv2_kernel<WT,U> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
 //   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns): the activation rows live in LDS, a wave streams RW weight rows at a time
 // All take the same operand description (ps_seq.h psk_dense_args): ring rows, the token-shift mix and the epilogue
 // (bias, activation, scale, a factor from a second table) are part of the launch, so no mixer needs a kernel of its own around its projections.
@@ -862,18 +863,16 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_narrow_kernel(dn_args g) {
 // that neither the prologue nor a row's reduction leaves the memory idle.  Rows are dealt to the waves of the whole launch in turn (consecutive waves read consecutive rows; a matrix
 // of 2048 rows gives each of 2048 waves one), or in neighbouring pairs for a paired activation.  What bounded dense_mv_kernel here was the number of bytes in flight: four rows per wave,
 // two pieces each, 128 work-groups of four waves for 2048 rows.  Measured, bf16, before and now: 2048 x 4096 (16.8 MB) 14.6 and 6.6 us, 8192 x 2048 (33 MB) 15 and 9, 14336 x 4096
-// (117 MB) 29 to 38 and 22 us (5.3 TB/s).  The experts of one token (top 2 of 2048 x 2048 and a shared one), which were two launches per product, 12.4 + 10.4 and 12.0 us (first product),
-// 16.6 + 17.5 and 18.0 us (second).  Sixteen units in flight, and the activations requested ahead of the weights, were tried and are slower (the registers cost a work-group per CU).
+// (117 MB) 29 to 38 and 22 us (5.3 TB/s).  The first product of a token's experts (top 2 of 3072 x 2048 and a shared one of twice that, 50 MB), which was two launches, 12.4 + 10.4 and 12.0 us.
+//  Sixteen units in flight, and the activations requested ahead of the weights, were tried and are slower (the registers cost a work-group per CU).
 //   FORM 0  one matrix
 //   FORM 1  grouped, the first product of an expert: work-groups in equal runs per slot (its own matrix and output row), behind them those of the shared expert (g2)
-//   FORM 2  grouped, the second product: an output row is the sum over the token's slots (and the shared expert) of the products with their matrices: a row's stream runs through
-//           all of them; blockIdx.y = token
 // dynamic LDS: the activations as bf16-rounded fp32 (fp32 mode: as they are), every vector padded with zeros to whole units
 #define DN_AHEAD 8
 struct dn_mv1 {
-    dn_args g2; // the shared expert (w NULL: none): FORM 1 its first product, FORM 2 its second (only w, a, K, out_scale are read there)
-    int slots;  // FORM 1: slots of the launch; FORM 2: slots per token
-    int kp, kp2; // padded lengths of the vectors
+    dn_args g2;  // FORM 1: the shared expert's first product (w NULL: none)
+    int slots;   // FORM 1: slots of the launch
+    int kp;      // padded length of the vector
     int blocks, blocks2; // FORM 1: work-groups per slot, of the shared expert
 };
 
@@ -935,9 +934,10 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
     extern __shared__ __attribute__((aligned(16))) float xs[];
     constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE; // elements per lane and per unit
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int y = FORM == 1 ? min((int)blockIdx.x / p.blocks, p.slots) : (int)blockIdx.y;
+    const int y = FORM == 1 ? min((int)blockIdx.x / p.blocks, p.slots) : 0;
     const bool shared_seg = FORM == 1 && y == p.slots;
     dn_args g = g0;
+    int sel = 0;
     if constexpr (FORM == 1) { // (field by field: the same K, activation and addition in both)
         g.w = shared_seg ? p.g2.w : g0.w;
         g.N = shared_seg ? p.g2.N : g0.N;
@@ -947,48 +947,33 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
         g.out_scale = shared_seg ? p.g2.out_scale : g0.out_scale;
         g.bias = shared_seg ? p.g2.bias : g0.bias;
         g.alpha = shared_seg ? p.g2.alpha : g0.alpha;
+        sel = shared_seg ? 0 : g.g_sel[y];
     }
-    // lane c: the matrix of segment c of a row's stream (FORM 2: the token's slots, then the shared expert)
-    const int n_seg = FORM == 2 ? p.slots + (p.g2.w ? 1 : 0) : 1;
-    int sel = 0;
-    if constexpr (FORM == 1) sel = shared_seg ? 0 : g.g_sel[y];
-    if constexpr (FORM == 2) {
-        if (lane < p.slots) sel = g.g_sel[(long long)y * p.slots + lane];
-    }
-    auto has = [&](int c) { return FORM == 0 || (FORM == 1 ? shared_seg || sel < g.groups : c == p.slots || (int)__builtin_amdgcn_readlane(sel, c) < g.groups); };
-    auto units_of = [&](int c) { return (FORM == 2 && c == p.slots ? p.kp2 : p.kp) / UNIT; };
-    int row_units = 0; // units of a row's stream (0: identity experts only)
-    for (int c = 0; c < n_seg; c++) row_units += has(c) ? units_of(c) : 0;
-    const int N = (int)g.N;
-    const bool pair = FORM != 2 && (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR);
+    const bool has = FORM == 0 || shared_seg || sel < g.groups; // (an identity expert has no matrix: its rows are zero)
+    const int row_units = has ? p.kp / UNIT : 0, N = (int)g.N, K = (int)g.K;
+    const bool pair = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR;
     // this wave's rows: first + k step (pairs: first + (k / 2) step + k % 2), k < rows
     const int bx = FORM == 1 ? (int)blockIdx.x - y * p.blocks : (int)blockIdx.x, nb = FORM == 1 ? (shared_seg ? p.blocks2 : p.blocks) : (int)gridDim.x;
     const int step = nb * 8 * (pair ? 2 : 1), first = (bx * 8 + wave) * (pair ? 2 : 1);
     const int rows = first >= N ? 0 : pair ? ((N - first + step - 2) / step) * 2 : (N - first + step - 1) / step;
     auto row_of = [&](int k) { return pair ? first + (k >> 1) * step + (k & 1) : first + k * step; };
-    // the load side of the stream: row lk, segment lc, unit lu of lunits
-    int lk = 0, lc = -1, lu = 0, lunits = 0;
+    // the load side of the stream: row lk, unit lu
+    int lk = -1, lu = 0;
     const char *lp = nullptr, *lrow = nullptr;
-    bool beyond = false; // this lane's bytes of a row's last unit lie behind the row's end: it reads the row's first ones, against zeros
-    auto open = [&]() { // the next segment that has a matrix
-        do {
-            if (++lc == n_seg) { lc = 0; lk++; }
-        } while (!has(lc));
-        if (lk >= rows) return;
-        const bool sh = FORM == 2 && lc == p.slots;
-        const int K = (int)(sh ? p.g2.K : g.K);
-        const long long mat = FORM == 0 || sh || shared_seg ? 0 : (long long)(FORM == 1 ? sel : (int)__builtin_amdgcn_readlane(sel, lc)) * g.wstride;
-        lrow = (const char *)((const WT *)(sh ? p.g2.w : g.w) + mat + (long long)row_of(lk) * K);
+    const bool beyond = (row_units - 1) * UNIT + lane * VE >= K; // this lane's bytes of a row's last unit lie behind the row's end: it reads the row's first ones, against zeros
+    const WT *mat = (const WT *)g.w + (FORM == 0 || shared_seg ? 0 : (long long)sel * g.wstride);
+    auto open = [&]() {
+        if (++lk >= rows) return;
+        lrow = (const char *)(mat + (long long)row_of(lk) * K);
         lp = lrow + lane * 16;
-        lu = 0; lunits = units_of(lc);
-        beyond = (lunits - 1) * UNIT + lane * VE >= K;
+        lu = 0;
     };
     auto request = [&](dn_f4 &v) {
         if (lk >= rows) return; // (uniform)
-        const char *q = beyond && lu == lunits - 1 ? lrow : lp;
+        const char *q = beyond && lu == row_units - 1 ? lrow : lp;
         v = __builtin_nontemporal_load((const dn_f4 *)q);
         lp += 1024;
-        if (++lu == lunits) open();
+        if (++lu == row_units) open();
     };
     dn_f4 ring[DN_AHEAD];
     if (rows && row_units) {
@@ -1002,68 +987,35 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
         int T;
         dn_rows(g, row0, T);
         dn_stage<WT>(g, dn_arow(g, row0, 0), g.mu ? g.shift0 : nullptr, 1.f, xs, p.kp);
-    } else if constexpr (FORM == 1) {
+    } else {
         if (shared_seg) dn_stage<WT>(g, g.a, nullptr, 1.f, xs, p.kp);
         else dn_stage<WT>(g, g.a + (long long)(y / g.g_adiv) * g.lda, nullptr, g.g_scale ? g.g_scale[y] : 1.f, xs, p.kp);
-    } else {
-        for (int c = 0; c < p.slots; c++) {
-            const int s = y * p.slots + c;
-            dn_stage<WT>(g, g.a + (long long)(s / g.g_adiv) * g.lda, nullptr, g.g_scale ? g.g_scale[s] : 1.f, xs + c * p.kp, p.kp);
-        }
-        if (p.g2.w) dn_stage<WT>(p.g2, p.g2.a + y * p.g2.lda, nullptr, 1.f, xs + p.slots * p.kp, p.kp2);
     }
-    float ident = 0.f; // FORM 2: the summed weights of the token's slots that have no matrix
-    if constexpr (FORM == 2) {
-        if (g.g_ident)
-            for (int c = 0; c < p.slots; c++)
-                if (!has(c)) ident += g.g_ident_w[y * p.slots + c];
-    }
-    const float shared_scale = FORM == 2 && p.g2.w && p.g2.out_scale ? p.g2.out_scale[y] : 1.f;
     __syncthreads();
-    // the other side: segment cc, cu units of it left; lane k % 64 keeps row k's result until 64 of them are there or the rows are through
-    int cc = -1, cu = 0, done = 0, kept = 0;
-    const float *xp = xs;
-    float acc = 0.f, total = 0.f, res = 0.f;
-    auto next = [&]() {
-        do {
-            if (++cc == n_seg) cc = 0;
-        } while (!has(cc));
-        cu = units_of(cc);
-        xp = xs + (FORM == 2 ? cc * p.kp : 0) + lane * VE;
-    };
-    auto last_of_row = [&]() {
-        int c = cc + 1;
-        while (c < n_seg && !has(c)) c++;
-        return c == n_seg;
-    };
+    // the other side: cu units of the row left; lane k % 64 keeps row k's result until 64 of them are there or the rows are through
+    int cu = row_units, done = 0, kept = 0;
+    const float *xp = xs + lane * VE;
+    float acc = 0.f, res = 0.f;
     auto eat = [&](dn_f4 &v) {
         acc = dn_unit<WT>(acc, v, xp);
         request(v);
         xp += UNIT;
         if (--cu) return;
-        total = FORM == 2 && cc == p.slots ? fmaf(acc, shared_scale, total) : total + acc;
+        const float s = dn_wave_sum(acc);
+        res = lane == done - kept ? s : res;
+        done++;
         acc = 0.f;
-        if (last_of_row()) {
-            const float s = dn_wave_sum(total);
-            res = lane == done - kept ? s : res;
-            total = 0.f;
-            done++;
-        }
-        next();
+        cu = row_units;
+        xp = xs + lane * VE;
     };
     auto put = [&]() { // the results of rows kept .. done - 1
-        const int k = kept + lane, n = row_of(k);
-        float v = res;
-        const bool in = k < done;
-        if constexpr (FORM == 2) {
-            if (ident != 0.f && in) v = fmaf(ident, g.g_ident[(long long)y * g.g_ident_ld + n], v);
-        }
-        dn_put(g, FORM == 0 || shared_seg ? 0 : y, n, v, __shfl_xor(v, 1, 64), in);
+        const int k = kept + lane;
+        const float v = res;
+        dn_put(g, FORM == 0 || shared_seg ? 0 : y, row_of(k), v, __shfl_xor(v, 1, 64), k < done);
         kept = done;
     };
     if (row_units) {
         int left = rows * row_units;
-        if (left) next();
         for (; left >= DN_AHEAD; left -= DN_AHEAD) {
 #pragma unroll
             for (int q = 0; q < DN_AHEAD; q++) eat(ring[q]);
@@ -1083,31 +1035,180 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
 
 // Work-groups of eight waves: enough that every wave has a row, at most two per CU (one where the activations are long: each group stages them for itself).
 template <typename WT, int FORM>
-static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, int slots, int tokens) {
+static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, int slots) {
     constexpr int UNIT = 64 * 16 / (int)sizeof(WT);
     dn_mv1 p;
     if (g2) p.g2 = *g2;
     else { p.g2 = g; p.g2.w = nullptr; }
     p.slots = slots;
     p.kp = (int)((g.K + UNIT - 1) / UNIT * UNIT);
-    p.kp2 = g2 ? (int)((g2->K + UNIT - 1) / UNIT * UNIT) : 0;
-    const size_t lds = ((size_t)p.kp * (FORM == 2 ? slots : 1) + (FORM == 2 ? p.kp2 : 0)) * 4;
-    const bool aligned = (g.K * (int64_t)sizeof(WT)) % 16 == 0 && (!g2 || (g2->K * (int64_t)sizeof(WT)) % 16 == 0);
-    if (!aligned || lds > 128 * 1024 || g.N > (1 << 28) || slots > 63 || (FORM == 1 && g2 && (g2->K != g.K || g2->act != g.act || g2->accum != g.accum || g2->N > (1 << 28)))) return false;
+    const size_t lds = (size_t)p.kp * 4;
+    if ((g.K * (int64_t)sizeof(WT)) % 16 != 0 || lds > 128 * 1024 || g.N > (1 << 28) || (g2 && (g2->K != g.K || g2->act != g.act || g2->accum != g.accum || g2->N > (1 << 28)))) return false;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv1_kernel<WT, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    const int per = FORM != 2 && (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR) ? 16 : 8; // rows that a work-group takes at once
+    const int per = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR ? 16 : 8; // rows that a work-group takes at once
     const int64_t most = lds <= 72 * 1024 ? 512 : 256;
-    dim3 grid;
+    int64_t grid = std::min<int64_t>((g.N + per - 1) / per, most);
     if (FORM == 1) { // the same number of rows for every work-group of every matrix
         const int64_t all = g.N * slots + (g2 ? g2->N : 0), rounds = std::max<int64_t>((all + most * per - 1) / (most * per), 1);
         p.blocks = (int)((g.N + rounds * per - 1) / (rounds * per));
         p.blocks2 = g2 ? (int)((g2->N + rounds * per - 1) / (rounds * per)) : 0;
-        grid = dim3((unsigned)(p.blocks * slots + p.blocks2));
-    } else {
-        grid = dim3((unsigned)std::min<int64_t>((g.N + per - 1) / per, std::max<int64_t>(most / tokens, 64)), (unsigned)tokens);
+        grid = (int64_t)p.blocks * slots + p.blocks2;
     }
-    hipLaunchKernelGGL((dense_mv1_kernel<WT, FORM>), grid, dim3(512), lds, st, g, p);
+    hipLaunchKernelGGL((dense_mv1_kernel<WT, FORM>), dim3((unsigned)grid), dim3(512), lds, st, g, p);
+    return true;
+}
+
+// The second product of a token's experts: an output row is the sum over the token's slots (and the shared expert) of the products with their matrices, so a row runs through all of
+// them.  `waves` waves of a work-group share a row, each with the same up to U units of it, so that a wave's part of the activations (up to top + 1 vectors of different experts) stays in
+// its registers and nothing waits for a copy of all of them in LDS; eight units and more per wave are in flight, across row ends.  The waves' sums of a row meet in LDS at the end.
+// blockIdx.y = token.  Top 2 of 2048 x 3072 and a shared one of twice that (50 MB), one token: 16.6 us and 17.5 us more for the shared expert before, 18.0 as one stream with the activations in LDS
+// (as above), 14.3 now.  The form above is the better one where there is a single vector: 2048 x 4096 6.6 us there, 9 with this kernel's arrangement.
+// dynamic LDS: [8][rows] sums
+struct dn_mv2 {
+    dn_args g2; // the shared expert's second product (w NULL: none; only w, a, lda, K, out_scale are read)
+    int slots;  // per token
+    int units, units2; // of a row of a slot's matrix, of the shared expert's
+    int waves, share;  // waves per row, units per wave
+    int rows;          // the most rows that a group of waves has
+};
+template <typename WT, int U>
+__global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g, dn_mv2 p) {
+    extern __shared__ __attribute__((aligned(16))) float sums[];
+    constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE, AHEAD = U >= 8 ? 1 : 8 / U; // elements per lane and per unit; rows in flight
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), y = blockIdx.y;
+    const int sel = lane < p.slots ? g.g_sel[(long long)y * p.slots + lane] : 0; // lane c: slot c's matrix
+    const int N = (int)g.N, K = (int)g.K, K2 = (int)p.g2.K;
+    // this wave's rows: first + k step, k < rows
+    const int groups = 8 / p.waves, part = wave % p.waves, step = (int)gridDim.x * groups;
+    auto first_of = [&](int gi) { return (int)blockIdx.x * groups + gi; };
+    auto rows_of = [&](int gi) { return first_of(gi) >= N ? 0 : (N - first_of(gi) + step - 1) / step; };
+    const int first = first_of(wave / p.waves), rows = rows_of(wave / p.waves);
+    // this wave's units: where unit u of row 0 starts, its activations (a lane beyond the row's end reads the unit's first bytes, against zeros)
+    const int all = p.slots * p.units + p.units2, u0 = part * p.share, n_units = max(min(p.share, all - u0), 0);
+    const char *base[U];
+    bool has[U], second[U]; // (a slot without a matrix -- an identity expert -- has none; second: the shared expert's)
+    int lo[U];
+    float x[U][VE];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int c = min((u0 + u) / p.units, p.slots), at = u0 + u - c * p.units; // slot, unit of a row of its matrix
+        second[u] = c == p.slots;
+        has[u] = u < n_units;
+        const float *xr = p.g2.a + (long long)y * p.g2.lda;
+        const WT *w = (const WT *)p.g2.w;
+        float f = 1.f;
+        if (!second[u]) {
+            const int s = y * p.slots + c, m = __builtin_amdgcn_readlane(sel, min(c, 63));
+            has[u] = has[u] && m < g.groups;
+            xr = g.a + (long long)(s / g.g_adiv) * g.lda;
+            w = (const WT *)g.w + (long long)m * g.wstride;
+            if (g.g_scale && has[u]) f = g.g_scale[s];
+        }
+        const int k = at * UNIT + lane * VE, Kc = second[u] ? K2 : K;
+        const bool in = has[u] && k < Kc;
+        lo[u] = k < Kc ? lane * 16 : 0;
+        base[u] = (const char *)(w + (long long)at * UNIT);
+        const float *xk = xr + k;
+        if (((uintptr_t)xr & 15) == 0) { // (uniform)
+#pragma unroll
+            for (int e = 0; e < VE; e += 4) {
+                const dn_f4 v = in ? *(const dn_f4 *)(xk + e) : dn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[u][e + i] = v[i];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < VE; e++) x[u][e] = in ? xk[e] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < VE; e++) {
+            x[u][e] *= f;
+            if constexpr (sizeof(WT) == 2) x[u][e] = dn_bf2f(dn_f2bf(x[u][e]));
+        }
+    }
+    float ident = 0.f; // the summed weights of the token's slots that have no matrix
+    if (g.g_ident)
+        for (int c = 0; c < p.slots; c++)
+            if ((int)__builtin_amdgcn_readlane(sel, c) >= g.groups) ident += g.g_ident_w[y * p.slots + c];
+    const float shared_scale = p.g2.w && p.g2.out_scale ? p.g2.out_scale[y] : 1.f;
+    dn_f4 ring[AHEAD][U];
+    auto request = [&](dn_f4 (&v)[U], int k) {
+        if (k >= rows) return; // (uniform)
+        const long long r = first + (long long)k * step;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (has[u]) v[u] = __builtin_nontemporal_load((const dn_f4 *)(base[u] + r * ((second[u] ? K2 : K) * (int)sizeof(WT)) + lo[u]));
+    };
+#pragma unroll
+    for (int d = 0; d < AHEAD; d++) request(ring[d], d);
+    for (int k0 = 0; k0 < rows; k0 += AHEAD) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; d++) {
+            const int k = k0 + d;
+            if (k >= rows) break;
+            float acc = 0.f, own = 0.f;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (!has[u]) continue;
+                float a = second[u] ? own : acc;
+                if constexpr (sizeof(WT) == 2) {
+                    unsigned h[4];
+                    __builtin_memcpy(h, &ring[d][u], 16);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        a = fmaf(__uint_as_float(h[e] << 16), x[u][2 * e], a);
+                        a = fmaf(__uint_as_float(h[e] & 0xffff0000u), x[u][2 * e + 1], a);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) a = fmaf(ring[d][u][e], x[u][e], a);
+                }
+                if (second[u]) own = a;
+                else acc = a;
+            }
+            request(ring[d], k + AHEAD);
+            acc = dn_wave_sum(fmaf(own, shared_scale, acc));
+            if (lane == 0) sums[wave * p.rows + k] = acc;
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < groups * p.rows; i += 512) {
+        const int gi = i / p.rows, k = i - gi * p.rows, n = first_of(gi) + k * step;
+        if (k >= rows_of(gi)) continue;
+        float v = 0.f;
+        for (int q = 0; q < p.waves; q++) v += sums[(gi * p.waves + q) * p.rows + k];
+        if (ident != 0.f) v = fmaf(ident, g.g_ident[(long long)y * g.g_ident_ld + n], v);
+        dn_put(g, y, n, v, 0.f, true);
+    }
+}
+
+// Work-groups of eight waves, at most two per CU.  As few waves per row as keep four units of it per wave or less (fewer sums to make, 32 registers of activations), but as many as it
+// takes for 4096 waves to have a row.
+template <typename WT>
+static bool dn_launch_mv2(hipStream_t st, const dn_args &g, const dn_args *g2, int slots, int tokens) {
+    constexpr int UNIT = 64 * 16 / (int)sizeof(WT), MOST = sizeof(WT) == 2 ? 8 : 16;
+    dn_mv2 p;
+    if (g2) p.g2 = *g2;
+    else { p.g2 = g; p.g2.w = nullptr; }
+    if ((g.K * (int64_t)sizeof(WT)) % 16 != 0 || (g2 && (g2->K * (int64_t)sizeof(WT)) % 16 != 0) || g.K > (1 << 20) || p.g2.K > (1 << 20) || g.N > (1 << 28) || slots > 63) return false;
+    p.slots = slots;
+    p.units = (int)((g.K + UNIT - 1) / UNIT);
+    p.units2 = g2 ? (int)((g2->K + UNIT - 1) / UNIT) : 0;
+    const int units = slots * p.units + p.units2;
+    p.waves = 1;
+    while (p.waves < 8 && ((units + p.waves - 1) / p.waves > 4 || (g.N * tokens * p.waves < 4096 && p.waves < units))) p.waves *= 2;
+    p.share = (units + p.waves - 1) / p.waves;
+    if (p.share > MOST) return false;
+    const int per = 8 / p.waves; // rows that a work-group takes at once
+    const int64_t once = (g.N + per - 1) / per, grid = std::max(std::min<int64_t>(once, std::max(512 / tokens, 64)), (once + 1023) / 1024); // (at most 1024 rounds: 32 KiB of sums)
+    p.rows = (int)((once + grid - 1) / grid);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid, (unsigned)tokens), dim3(512), (size_t)8 * p.rows * 4, st, g, p); };
+    if (p.share == 1) go(dense_mv2_kernel<WT, 1>);
+    else if (p.share == 2) go(dense_mv2_kernel<WT, 2>);
+    else if (p.share <= 4) go(dense_mv2_kernel<WT, 4>);
+    else if (p.share <= 8) go(dense_mv2_kernel<WT, 8>);
+    else if constexpr (sizeof(WT) == 4) go(dense_mv2_kernel<WT, 16>);
     return true;
 }
 
@@ -1140,9 +1241,9 @@ static int dn_grouped_mv1(hipStream_t st, const psk_dense_args &a, const dn_args
     if (!second && (a.g_inner != 1 || a.g_ident)) return 0;
     if (a.also && a.also->w->dtype == a.w->dtype && (second || a.also->T == 1)) {
         const dn_args g2 = dn_make(*a.also);
-        if (second ? dn_launch_mv1<WT, 2>(st, g, &g2, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, &g2, a.T, 1)) return 2;
+        if (second ? dn_launch_mv2<WT>(st, g, &g2, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, &g2, a.T)) return 2;
     }
-    return (second ? dn_launch_mv1<WT, 2>(st, g, nullptr, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, nullptr, a.T, 1)) ? 1 : 0;
+    return (second ? dn_launch_mv2<WT>(st, g, nullptr, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, nullptr, a.T)) ? 1 : 0;
 }
 
 int psk_dense(hipStream_t st, const psk_dense_args &a) {
@@ -1168,7 +1269,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         return 0;
     }
     if (!a.force_tiled && a.T <= 8) {
-        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0, 1) : dn_launch_mv1<float, 0>(st, g, nullptr, 0, 1))) return 0;
+        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0) : dn_launch_mv1<float, 0>(st, g, nullptr, 0))) return 0;
         const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
         if (kp4 * C <= 64 * 1024) {
             if (bf) {
