@@ -3,6 +3,7 @@
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
 //   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
+//   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
 //   dense_mm_narrow_kernel bf16, K 128 or 256, more than 8 tokens: 32 x 32 tiles, the waves share K
 //   dense_mv1_kernel<WT,FORM> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
 //   dense_mv2_kernel<WT,U> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
@@ -494,21 +495,18 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) {
     }
 }
 
-// Sixteen results of one output column n: local rows tb + 8 (r / 4) + r % 4 (the D registers of a 32 x 32 tile).  Every lane of the wave calls this.
-static __device__ __forceinline__ void dn_put16(const dn_args &g, long long row0, int T, int tb, long long n, const dn_f16 &acc) {
+// Four results of one output column n: local rows tb .. tb + 3.  Every lane of the wave calls this.
+static __device__ __forceinline__ void dn_put4r(const dn_args &g, long long row0, int T, int tb, long long n, const dn_f4 &acc) {
     const bool nin = n < g.N;
     const bool pair = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR;
-    float old[16];
+    float old[4];
     if (g.accum && !pair) { // every old value is requested before the first is used
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int t = tb + 8 * (r >> 2) + (r & 3);
-            old[r] = t < T && nin ? g.out[dn_orow(g, row0, t, T) * g.ldo + n] : 0.f;
-        }
+        for (int r = 0; r < 4; r++) old[r] = tb + r < T && nin ? g.out[dn_orow(g, row0, tb + r, T) * g.ldo + n] : 0.f;
     }
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int t = tb + 8 * (r >> 2) + (r & 3);
+    for (int r = 0; r < 4; r++) {
+        const int t = tb + r;
         const bool in = t < T && nin;
         if (pair || g.em_table) { // (row n ^ 1 is the neighbouring lane's)
             dn_put(g, dn_orow(g, row0, t, T), n, acc[r], pair ? __shfl_xor(acc[r], 1, 64) : 0.f, in);
@@ -709,33 +707,28 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     }
 }
 
-// the splits of a tile, added in order: one work-group per 32 x 32 instruction tile of every wave
+// the splits of a tile, added in order: one work-group per quarter of the 32 x 32 instruction tiles ij of its four waves (the D registers 4 q .. 4 q + 3 of each lane).  A work-group that
+// took whole instruction tiles had one wave per SIMD of 256 CUs at work and sixteen columns of a row to write one behind the other: 14 us for the splits of
+// 512 x 2048, 16 for those of 512 x 8; 6.9 and 5.3 now.
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p) {
     constexpr int MI = BM / 64, NJ = BN / 64, IJ = MI * NJ;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, ij = (int)blockIdx.x % IJ, tile = (int)blockIdx.x / IJ, tm = tile / p.tn, tn = tile % p.tn;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, q = (int)blockIdx.x & 3, ij = (int)(blockIdx.x >> 2) % IJ, tile = (int)(blockIdx.x >> 2) / IJ,
+              tm = tile / p.tn, tn = tile % p.tn;
     int e, T, t0;
     long long row0;
     if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return;
-    const float *src = p.part + (long long)tile * p.S * (IJ * 4096) + ij * 4096 + tid * 4;
-    dn_f16 acc;
+    const float *src = p.part + (long long)tile * p.S * (IJ * 4096) + ij * 4096 + q * 1024 + tid * 4;
+    dn_f4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < p.S; s += 8) { // (eight loads in flight)
+        dn_f4 v[8];
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.f;
-    for (int s = 0; s < p.S; s += 4) { // (sixteen loads in flight)
-        dn_f4 v[4][4];
+        for (int u = 0; u < 8; u++) v[u] = *(const dn_f4 *)(src + (long long)min(s + u, p.S - 1) * (IJ * 4096));
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) v[u][q] = *(const dn_f4 *)(src + (long long)min(s + u, p.S - 1) * (IJ * 4096) + q * 1024);
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (s + u < p.S)
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-#pragma unroll
-                    for (int x = 0; x < 4; x++) acc[4 * q + x] += v[u][q][x];
+        for (int u = 0; u < 8; u++)
+            if (s + u < p.S) acc += v[u];
     }
-    dn_put16(g, row0, T, t0 + wm * MI * 32 + (ij / NJ) * 32 + 4 * (lane >> 5), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + (lane & 31), acc);
+    dn_put4r(g, row0, T, t0 + wm * MI * 32 + (ij / NJ) * 32 + 4 * (lane >> 5) + 8 * q, (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + (lane & 31), acc);
 }
 
 // Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
@@ -767,7 +760,7 @@ static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     const unsigned grid = (unsigned)((p.tn * p.S + 7) / 8 * 8) * p.n_tm;
     hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN>), dim3(grid), dim3(512), LDS, st, g, p);
-    if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64))), dim3(256), 0, st, g, p);
+    if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
 }
 
 // the wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed
@@ -787,6 +780,38 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, const dn_args 
     else if (r.BN == 128) dn_launch_ring<WT, 64, 128>(st, g, p);
     else dn_launch_ring<WT, 64, 64>(st, g, p);
     return true;
+}
+
+// Products with an inner size of a few numbers (the second matrix of a low-rank decay): a thread has an output column, its KP weights in registers, and runs over sixteen tokens whose
+// activations lie in LDS.  Nothing but the writing of the result counts here: 512 x 2048 of K = 8 took the tiled kernel 23 us (a tile's results leave a lane one number per row), 10.9 now.
+template <typename WT, int KP>
+__global__ __launch_bounds__(256) void dense_mm_few_kernel(dn_args g) {
+    __shared__ float as[16 * KP];
+    const int tid = threadIdx.x, t0 = blockIdx.y * 16, K = (int)g.K;
+    const long long n = (long long)blockIdx.x * 256 + tid;
+    float w[KP];
+#pragma unroll
+    for (int k = 0; k < KP; k++) {
+        w[k] = 0.f;
+        if (n < g.N && k < K) {
+            if constexpr (sizeof(WT) == 2) w[k] = dn_bf2f(((const unsigned short *)g.w)[n * K + k]);
+            else w[k] = ((const float *)g.w)[n * K + k];
+        }
+    }
+    for (int i = tid; i < 16 * KP; i += 256) {
+        const int t = t0 + i / KP, k = i % KP;
+        float v = t < g.T && k < K ? g.a[t * g.lda + k] : 0.f;
+        if constexpr (sizeof(WT) == 2) v = dn_bf2f(dn_f2bf(v));
+        as[i] = v;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int t = 0; t < 16; t++) {
+        float a = 0.f;
+#pragma unroll
+        for (int k = 0; k < KP; k++) a = fmaf(as[t * KP + k], w[k], a);
+        dn_put(g, t0 + t, n, a, __shfl_xor(a, 1, 64), t0 + t < g.T && n < g.N);
+    }
 }
 
 // Products with an inner size of a few steps (K <= 256: the ring would be all prologue): 32 tokens x 32 outputs per work-group.  Each of the NW waves takes
@@ -1285,6 +1310,13 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
             }
             return 0;
         }
+    }
+    if (!a.force_tiled && a.T > 8 && g.K <= 32 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0) {
+        const dim3 grid((unsigned)((g.N + 255) / 256), (unsigned)((a.T + 15) / 16));
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g); };
+        if (g.K <= 8) bf ? go(dense_mm_few_kernel<unsigned short, 8>) : go(dense_mm_few_kernel<float, 8>);
+        else bf ? go(dense_mm_few_kernel<unsigned short, 32>) : go(dense_mm_few_kernel<float, 32>);
+        return 0;
     }
     if (bf && !a.force_tiled && a.T > 8 && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 && g.K <= 256) {
         const dim3 grid((unsigned)((a.T + 31) / 32), (unsigned)((g.N + 31) / 32));

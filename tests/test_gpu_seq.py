@@ -151,6 +151,24 @@ def test_dense_matmul_wide(ctx, dtype, T, N, K):
     dx.free(); do.free()
 
 
+# the four-tap filter (k_seqmix.hip sq_conv4_kernel) in portions of one to nine tokens (its threads take four; the tail from old and new tokens) and the norms around it with one, two and four
+# runs per thread, a run and four channels more, and in the general kernels (66: no multiple of four)
+@pytest.mark.parametrize("width", [64, 66, 1024, 1028, 2052, 8192])
+@pytest.mark.parametrize("sizes", [(2,), (3, 1), (4, 2, 1), (5, 9, 8)])
+def test_filters_and_norms_of_portions(made, width, sizes):
+    cfg = synth.seq_config(width, 40, [L("delta", 24, heads=2, kv_heads=1, dim=12, vdim=20, conv=4), L("delta", None, heads=2, kv_heads=2, dim=16, vdim=8, conv=4)], taps=4)
+    m, c, t = made(f"four{width}", max_batch=16, cfg=cfg)
+    toks = tokens_for(c, 37)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
+
+
+# K up to 32 (k_dense.hip dense_mm_few_kernel): one below, at and above its two widths (33: the tiled kernel), one token and one column more and less than a work-group's
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,N,K", [(9, 1, 1), (15, 255, 7), (16, 256, 8), (17, 257, 9), (33, 70, 31), (31, 513, 32), (40, 65, 33)])
+def test_dense_matmul_of_a_short_inner_size(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
 # one token (k_dense.hip dense_mv1_kernel): a row of less than one unit of its stream (512 numbers, fp32: 256), of exactly one, of one and a bit; fewer and more units per wave than are in flight;
 # one row, rows that are no multiple of the waves', more rows than waves and more than 64 of them per wave; the longest row that is taken, and one more, which the general kernel does
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
