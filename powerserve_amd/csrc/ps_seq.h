@@ -90,7 +90,9 @@ void psk_argmax_rows(hipStream_t st, const float *x, int64_t n, int rows, int32_
 void psk_rmsnorm(hipStream_t st, const float *x, int64_t ldx, const int32_t *idx, const float *w, float offset, float eps, int64_t n, int rows, float *y, int64_t ldy,
                  int groups = 1);
 // x[r] += y[r] / sqrt(mean(y^2) + eps) * (offset + w)
-void psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups = 1);
+// (wn given: hn = norm(x) (offset + wn) behind it)
+void psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups = 1, const float *wn = nullptr,
+                       float *hn = nullptr);
 // The front of a parallel layer that has no input filter, in one launch: x[r] = sum_j mix[j] X_j[row(r)] over the nmix streams X_j = src + j stride (mix NULL:
 // the last stream alone), row(r) = idx ? idx[r] : r, stored to xout[r] (NULL: not kept); then h[r] = norm(x) (offset + w1) and h2[r] = norm(x) (offset + w2) with
 // the norm taken over `groups` parts -- two norms of one vector share their statistics.  w1 / w2 NULL: that output is not made.

@@ -563,9 +563,9 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             psk_boundary1(st, m->step, m->x, y, wb, wn, cw, D.canon_taps, tail_off, D.norm_offset, D.norm_eps, W, m->h, m->hn);
             return;
         }
-        if (y) psk_norm_residual(st, m->x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups);
+        if (y) psk_norm_residual(st, m->x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn);
         if (wn) {
-            psk_rmsnorm(st, m->x, W, nullptr, wn, D.norm_offset, D.norm_eps, W, T, m->hn, W, m->groups);
+            if (!y) psk_rmsnorm(st, m->x, W, nullptr, wn, D.norm_offset, D.norm_eps, W, T, m->hn, W, m->groups);
             psk_causal_conv(st, m->step, tail_off, m->hn, W, cw, D.canon_taps, 0, W, T, m->h, W);
         }
     };
