@@ -19,6 +19,7 @@
 typedef float dn_f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 dn_bf8 __attribute__((ext_vector_type(8)));
 typedef unsigned short dn_us8 __attribute__((ext_vector_type(8)));
+typedef unsigned short dn_us4 __attribute__((ext_vector_type(4)));
 
 static __device__ __forceinline__ unsigned short dn_f2bf(float f) { // round to nearest even
     unsigned u = __float_as_uint(f);
@@ -36,6 +37,7 @@ struct dn_args {
     int T;
     long long N, K;
     float *out;
+    unsigned short *out16; // given: the result rounded to bf16 there instead, in out's arrangement (wide mat-mul)
     long long ldo;
     const float *bias;
     int act;
@@ -112,7 +114,8 @@ static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, lon
             float *p = g.out + t * g.ldo + (n >> 1);
             if (g.bias) { acc += g.bias[n]; other += g.bias[n + 1]; }
             const float v = (g.act == PSD_ACT_SILU_PAIR ? dn_silu(acc) : fmaxf(acc, 0.f)) * other * g.alpha * rs;
-            *p = g.accum ? *p + v : v;
+            if (g.out16) g.out16[p - g.out] = dn_f2bf(v);
+            else *p = g.accum ? *p + v : v;
         }
         return;
     }
@@ -123,7 +126,8 @@ static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, lon
         const long long at = (long long)(g.em_tokens ? g.em_tokens[t] : g.em_step->token0) * g.em_ld + g.em_col + n;
         v *= g.em_bf16 ? dn_bf2f(((const unsigned short *)g.em_table)[at]) : ((const float *)g.em_table)[at];
     }
-    *p = g.accum ? *p + v : v;
+    if (g.out16) g.out16[p - g.out] = dn_f2bf(v);
+    else *p = g.accum ? *p + v : v;
 }
 // the output row of local row t (t < T): itself, or where the sorted list sends its slot
 static __device__ __forceinline__ long long dn_orow(const dn_args &g, long long row0, int t, int T) {
@@ -515,7 +519,8 @@ static __device__ __forceinline__ void dn_put4r(const dn_args &g, long long row0
         if (!in) continue;
         const long long o = dn_orow(g, row0, t, T);
         const float v = dn_epi(g, acc[r], n) * (g.out_scale ? g.out_scale[o] : 1.f);
-        g.out[o * g.ldo + n] = g.accum ? old[r] + v : v;
+        if (g.out16) g.out16[o * g.ldo + n] = dn_f2bf(v);
+        else g.out[o * g.ldo + n] = g.accum ? old[r] + v : v;
     }
 }
 
@@ -536,7 +541,14 @@ static __device__ __forceinline__ void dn_put4(const dn_args &g, long long t, lo
         const float y = dn_epi(g, acc[e], n + e) * rs;
         v[e] = g.accum ? v[e] + y : y;
     }
-    *(dn_f4 *)p = v;
+    if (g.out16) {
+        dn_us4 r;
+#pragma unroll
+        for (int e = 0; e < 4; e++) r[e] = dn_f2bf(v[e]);
+        *(dn_us4 *)(g.out16 + (p - g.out)) = r;
+    } else {
+        *(dn_f4 *)p = v;
+    }
 }
 
 static __device__ __forceinline__ void dn_dma(const char *src, unsigned lds_dst) { // one wave-instruction: lane l's 16 bytes at src go to lds_dst + 16 l
@@ -768,10 +780,12 @@ template <typename WT>
 static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
     const int64_t kbytes = g.K * (int64_t)sizeof(WT);
     if (a.force_tiled || kbytes % 128 || !a.pack) return false;
-    const bool plain = sizeof(WT) == 4 && !g.mu && !g.g_scale && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0;
+    const bool rows = !g.mu && !g.g_list && !g.a_mod && !g.a_step && !g.a_row0;
+    const bool handed = sizeof(WT) == 2 && a.a16 && rows; // (the producer has rounded them already)
+    const bool plain = handed || (sizeof(WT) == 4 && !g.mu && !g.g_scale && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0);
     if (!plain && (size_t)a.T * kbytes > a.pack_bytes) return false;
     const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes());
-    dn_ring p{plain ? nullptr : (const char *)a.pack, kbytes, r.n_tm, r.tn, r.S, a.split};
+    dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes, r.n_tm, r.tn, r.S, a.split};
     if (!plain) {
         const int64_t pb = ((int64_t)a.T * (g.K / 8) + 255) / 256;
         hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192)), dim3(256), 0, st, g, (WT *)a.pack);
@@ -1251,7 +1265,7 @@ static void dn_launch_mv(hipStream_t st, const dn_args &g) {
 static dn_args dn_make(const psk_dense_args &a) {
     dn_args g;
     g.w = a.w->data; g.a = a.a; g.lda = a.lda; g.a_row0 = a.a_row0; g.a_mod = a.a_mod; g.a_step = a.a_step; g.T = a.T;
-    g.N = a.w->N; g.K = a.w->K; g.out = a.out; g.ldo = a.ldo; g.bias = a.bias; g.act = a.act; g.act_p = a.act_p; g.act_q = a.act_q;
+    g.N = a.w->N; g.K = a.w->K; g.out = a.out; g.out16 = (unsigned short *)a.out16; g.ldo = a.ldo; g.bias = a.bias; g.act = a.act; g.act_p = a.act_p; g.act_q = a.act_q;
     g.alpha = a.alpha; g.mu = a.mu; g.shift0 = a.shift0; g.accum = a.accum; g.out_scale = a.out_scale;
     g.groups = 0; g.g_adiv = 1; g.g_odiv = 1; g.g_inner = 1; g.g_sel = nullptr; g.g_seg = nullptr; g.g_list = nullptr; g.g_scale = nullptr; g.wstride = 0;
     g.g_ident = a.g_ident; g.g_ident_w = a.g_ident_w; g.g_ident_ld = a.g_ident_ld;
@@ -1271,6 +1285,10 @@ static int dn_grouped_mv1(hipStream_t st, const psk_dense_args &a, const dn_args
     return (second ? dn_launch_mv2<WT>(st, g, nullptr, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, nullptr, a.T)) ? 1 : 0;
 }
 
+bool psk_dense_wide16(const psk_dense_args &a) {
+    return a.w && a.w->dtype == PS_BF16 && a.T > 8 && !a.force_tiled && a.pack && a.groups == 0 && !a.mu && !a.a_mod && !a.a_step && !a.a_row0 && a.w->K > 256 && a.w->K % 64 == 0 &&
+           (size_t)a.T * a.w->K * 2 <= a.pack_bytes;
+}
 int psk_dense(hipStream_t st, const psk_dense_args &a) {
     if (!a.w || a.T <= 0) return 0;
     dn_args g = dn_make(a);

@@ -27,6 +27,13 @@ static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane get
     auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
     return (row(0) + row(16)) + (row(32) + row(48));
 }
+typedef unsigned short sq_us4 __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ unsigned short sq_bf16(float f) { // round to nearest even, as the mat-mul's own copy of its operand does
+    unsigned u = __float_as_uint(f);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
+    return (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+static __device__ __forceinline__ sq_us4 sq_bf16x4(const sq_f4 &v) { return sq_us4{sq_bf16(v[0]), sq_bf16(v[1]), sq_bf16(v[2]), sq_bf16(v[3])}; }
 static __device__ __forceinline__ float sq_silu(float x) { return x / (1.f + expf(-x)); }
 static __device__ __forceinline__ float sq_softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
@@ -165,7 +172,8 @@ __global__ __launch_bounds__(256) void sq_norm_residual_kernel(float *x, const f
 // The same and the norm in front of the next sublayer (wn NULL: without it), a block per row with C runs of four numbers per thread in registers: hn = x / rms(x) * (offset + wn).  One launch
 // and one reading of x instead of two: 512 rows of 2048, 7.7 + 5.0 us before, 5.5 now.
 template <int C>
-__global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, const float *y, const float *w, const float *wn, float offset, float eps, int n, float *hn) {
+__global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, const float *y, const float *w, const float *wn, float offset, float eps, int n, float *hn,
+                                                                     unsigned short *copy16) {
     __shared__ float red[2][16];
     const int tid = threadIdx.x, nw = blockDim.x >> 6;
     const long long at = (long long)blockIdx.x * n;
@@ -203,6 +211,7 @@ __global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, c
             s += xv[c][e] * xv[c][e];
         }
         if (i < n) *(sq_f4 *)(x + at + i) = xv[c];
+        if (i < n && copy16) *(sq_us4 *)(copy16 + at + i) = sq_bf16x4(xv[c]);
     }
     if (!wn) return;
     const float invn = 1.f / sqrtf(block_sum(s, red[1]) / (float)n + eps);
@@ -215,17 +224,18 @@ __global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, c
         if (i < n) *(sq_f4 *)(hn + at + i) = o;
     }
 }
-void psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups, const float *wn, float *hn) {
-    if (rows <= 0) return;
+bool psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups, const float *wn, float *hn, uint16_t *copy16) {
+    if (rows <= 0) return false;
     if (groups == 1 && n % 4 == 0 && n <= 8192 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w | (uintptr_t)wn | (uintptr_t)hn) & 15) == 0) {
         const int c = n <= 1024 ? 1 : n <= 2048 ? 2 : 4;
         const int threads = (int)((n / 4 + c - 1) / c + 63) / 64 * 64;
-        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, st, x, y, w, wn, offset, eps, (int)n, hn); };
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, st, x, y, w, wn, offset, eps, (int)n, hn, copy16); };
         c == 1 ? go(sq_norm_residual_fast_kernel<1>) : c == 2 ? go(sq_norm_residual_fast_kernel<2>) : go(sq_norm_residual_fast_kernel<4>);
-        return;
+        return copy16 != nullptr;
     }
     hipLaunchKernelGGL(sq_norm_residual_kernel, dim3(rows, groups), dim3(256), 0, st, x, y, w, offset, eps, (long long)(n / groups));
     if (wn) psk_rmsnorm(st, x, n, nullptr, wn, offset, eps, n, rows, hn, n, groups);
+    return false;
 }
 
 // x += norm(v) (offset + w) + bias: a post-norm sublayer's end (ps_seq.h psk_postnorm), a block per row.  v = y, or the weighted sum of two outputs each divided by its own root mean
@@ -311,7 +321,7 @@ __global__ __launch_bounds__(256) void sq_conv_tail_kernel(const ps_seq_step *st
 // the only ones that read the tail, also bring it up to date, so no second launch waits for them.  512 tokens of 2048 channels: 11.7 us and 4.4 for the tail with a channel per thread, 5.4 now.
 #define SQ_CONV4 4
 __global__ __launch_bounds__(256) void sq_conv4_kernel(const ps_seq_step *step, long long tail_off, const float *in, long long ldi, const float *w, int mode, int C, int T, float *out,
-                                                       long long ldo, const float *bias) {
+                                                       long long ldo, const float *bias, unsigned short *copy16) {
     const int c = (blockIdx.x * 256 + threadIdx.x) * 4, t0 = blockIdx.y * SQ_CONV4;
     if (c >= C) return;
     float *tail = step->state + tail_off;
@@ -335,6 +345,7 @@ __global__ __launch_bounds__(256) void sq_conv4_kernel(const ps_seq_step *step, 
             o[e] = mode == 0 ? x[i + 3][e] + s : sq_silu(s);
         }
         *(sq_f4 *)(out + (long long)(t0 + i) * ldo + c) = o;
+        if (copy16) *(sq_us4 *)(copy16 + (long long)(t0 + i) * C + c) = sq_bf16x4(o);
     }
     if (t0) return;
     sq_f4 n[3]; // the inputs of tokens T - 3 .. T - 1 (before the first: the old tail, which x holds)
@@ -343,17 +354,18 @@ __global__ __launch_bounds__(256) void sq_conv4_kernel(const ps_seq_step *step, 
 #pragma unroll
     for (int i = 0; i < 3; i++) *(sq_f4 *)(tail + (long long)i * C + c) = n[i];
 }
-void psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, const float *in, int64_t ldi, const float *w, int taps, int mode, int64_t C, int T,
-                     float *out, int64_t ldo, const float *bias) {
+bool psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, const float *in, int64_t ldi, const float *w, int taps, int mode, int64_t C, int T,
+                     float *out, int64_t ldo, const float *bias, uint16_t *copy16) {
     if (taps == 4 && C % 4 == 0 && C < (1ll << 28) && ldi % 4 == 0 && ldo % 4 == 0 && tail_off % 4 == 0 && in != out &&
         (((uintptr_t)in | (uintptr_t)w | (uintptr_t)out | (uintptr_t)bias) & 15) == 0) {
         hipLaunchKernelGGL(sq_conv4_kernel, dim3((unsigned)((C / 4 + 255) / 256), (unsigned)((T + SQ_CONV4 - 1) / SQ_CONV4)), dim3(256), 0, st, step, (long long)tail_off, in, (long long)ldi,
-                           w, mode, (int)C, T, out, (long long)ldo, bias);
-        return;
+                           w, mode, (int)C, T, out, (long long)ldo, bias, copy16);
+        return copy16 != nullptr;
     }
     const unsigned gx = (unsigned)((C + 255) / 256), gy = (unsigned)((T + SQ_CONV_CHUNK - 1) / SQ_CONV_CHUNK);
     hipLaunchKernelGGL(sq_conv_kernel, dim3(gx, gy), dim3(256), 0, st, step, (long long)tail_off, in, (long long)ldi, w, taps, mode, (long long)C, T, out, (long long)ldo, bias);
     if (gy > 1 && taps > 1) hipLaunchKernelGGL(sq_conv_tail_kernel, dim3(gx), dim3(256), 0, st, step, (long long)tail_off, in, (long long)ldi, taps, (long long)C, T);
+    return false;
 }
 
 __global__ void sq_state_store_kernel(const ps_seq_step *step, long long off, const float *src, long long n) {
@@ -783,7 +795,8 @@ void psk_delta_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, 
                        dt_bias, H, KH, d, dv, R, T, o, (long long)ldo);
 }
 
-__global__ __launch_bounds__(64) void sq_headnorm_gate_kernel(float *o, long long ldo, const float *g, long long ldg, const float *w, int w_stride, float eps, int dv) {
+__global__ __launch_bounds__(64) void sq_headnorm_gate_kernel(float *o, long long ldo, const float *g, long long ldg, const float *w, int w_stride, float eps, int dv,
+                                                              unsigned short *copy16) {
     const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
     float *oh = o + (long long)t * ldo + (long long)h * dv;
     const float *gh = g + (long long)t * ldg + (long long)h * dv, *wh = w + (long long)h * w_stride;
@@ -792,10 +805,15 @@ __global__ __launch_bounds__(64) void sq_headnorm_gate_kernel(float *o, long lon
 #pragma unroll
     for (int x = 32; x > 0; x >>= 1) s += __shfl_xor(s, x, 64);
     const float inv = 1.f / sqrtf(s / (float)dv + eps);
-    for (int j = lane; j < dv; j += 64) oh[j] = oh[j] * inv * wh[j] * sq_silu(gh[j]);
+    for (int j = lane; j < dv; j += 64) {
+        const float v = oh[j] * inv * wh[j] * sq_silu(gh[j]);
+        oh[j] = v;
+        if (copy16) copy16[((long long)t * gridDim.y + h) * dv + j] = sq_bf16(v);
+    }
 }
-void psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, int64_t ldg, const float *w, int w_stride, float eps, int H, int dv, int T) {
-    hipLaunchKernelGGL(sq_headnorm_gate_kernel, dim3(T, H), dim3(64), 0, st, o, (long long)ldo, g, (long long)ldg, w, w_stride, eps, dv);
+bool psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, int64_t ldg, const float *w, int w_stride, float eps, int H, int dv, int T, uint16_t *copy16) {
+    hipLaunchKernelGGL(sq_headnorm_gate_kernel, dim3(T, H), dim3(64), 0, st, o, (long long)ldo, g, (long long)ldg, w, w_stride, eps, dv, copy16);
+    return copy16 != nullptr;
 }
 
 
@@ -1107,7 +1125,8 @@ void psk_mlstm_finish(hipStream_t st, const ps_seq_step *step, int64_t m_off, fl
 }
 
 // o <- o silu(z), then each of gridDim.y equal parts (n numbers) divided by its own root mean square, times w: block (token, part); a thread re-reads only what it wrote
-__global__ __launch_bounds__(1024) void sq_gate_partnorm_kernel(float *o, long long ldo, const float *z, long long ldz, const float *w, float eps, int n) {
+__global__ __launch_bounds__(1024) void sq_gate_partnorm_kernel(float *o, long long ldo, const float *z, long long ldz, const float *w, float eps, int n,
+                                                                unsigned short *copy16) {
     __shared__ float red[16];
     const int tid = threadIdx.x, nt = blockDim.x;
     float *op = o + (long long)blockIdx.x * ldo + (long long)blockIdx.y * n;
@@ -1126,11 +1145,16 @@ __global__ __launch_bounds__(1024) void sq_gate_partnorm_kernel(float *o, long l
     float total = 0.f;
     for (int k = 0; k < (nt >> 6); k++) total += red[k];
     const float inv = 1.f / sqrtf(total / (float)n + eps);
-    for (int i = tid; i < n; i += nt) op[i] = op[i] * inv * w[i];
+    for (int i = tid; i < n; i += nt) {
+        const float v = op[i] * inv * w[i];
+        op[i] = v;
+        if (copy16) copy16[((long long)blockIdx.x * gridDim.y + blockIdx.y) * n + i] = sq_bf16(v);
+    }
 }
-void psk_gate_partnorm(hipStream_t st, float *o, int64_t ldo, const float *z, int64_t ldz, const float *w, int parts, float eps, int64_t n, int T) {
+bool psk_gate_partnorm(hipStream_t st, float *o, int64_t ldo, const float *z, int64_t ldz, const float *w, int parts, float eps, int64_t n, int T, uint16_t *copy16) {
     const int pn = (int)(n / parts);
-    hipLaunchKernelGGL(sq_gate_partnorm_kernel, dim3(T, parts), dim3(T <= 8 && pn >= 1024 ? 1024 : 256), 0, st, o, (long long)ldo, z, (long long)ldz, w, eps, pn);
+    hipLaunchKernelGGL(sq_gate_partnorm_kernel, dim3(T, parts), dim3(T <= 8 && pn >= 1024 ? 1024 : 256), 0, st, o, (long long)ldo, z, (long long)ldz, w, eps, pn, copy16);
+    return copy16 != nullptr;
 }
 
 // ---------------------------------------------------------------------------------------------------- element-wise gated recurrence (minGRU)

@@ -73,7 +73,13 @@ struct psk_dense_args {
     // grouped mat-vec only: the shared expert's product that goes with it -- beside the slots' first products (T == 1, the same activation), or added to a token's sum of second products
     // (only its w, a, lda, K and out_scale count there).  psk_dense returns 1 where the launch has made it too, 0 where it is still to be made.
     const psk_dense_args *also = nullptr;
+    // bf16 hand-over between products and from the kernels in front of them (bit for bit what the wide mat-mul's own copy of A would hold): a16 = the A operand's rows, K apart and
+    // already rounded (used by the wide mat-mul over plain rows, a is read otherwise); out16 = the result goes there, rounded, and not to out (only where psk_dense_wide16, never
+    // with accum)
+    const void *a16 = nullptr;
+    void *out16 = nullptr;
 };
+bool psk_dense_wide16(const psk_dense_args &a); // psk_dense will run this as the wide bf16 mat-mul over plain rows
 int psk_dense(hipStream_t st, const psk_dense_args &a);
 size_t psk_dense_split_bytes(); // what any product's splits need at most
 void psk_dense_widen(hipStream_t st, const uint16_t *bf16, int64_t n, float *out);
@@ -91,8 +97,9 @@ void psk_rmsnorm(hipStream_t st, const float *x, int64_t ldx, const int32_t *idx
                  int groups = 1);
 // x[r] += y[r] / sqrt(mean(y^2) + eps) * (offset + w)
 // (wn given: hn = norm(x) (offset + wn) behind it)
-void psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups = 1, const float *wn = nullptr,
-                       float *hn = nullptr);
+// (copy16 of these and of psk_causal_conv, psk_headnorm_gate, psk_gate_partnorm: also the result -- x here -- rounded to bf16, rows side by side; returns whether that was done)
+bool psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups = 1, const float *wn = nullptr,
+                       float *hn = nullptr, uint16_t *copy16 = nullptr);
 // The front of a parallel layer that has no input filter, in one launch: x[r] = sum_j mix[j] X_j[row(r)] over the nmix streams X_j = src + j stride (mix NULL:
 // the last stream alone), row(r) = idx ? idx[r] : r, stored to xout[r] (NULL: not kept); then h[r] = norm(x) (offset + w1) and h2[r] = norm(x) (offset + w2) with
 // the norm taken over `groups` parts -- two norms of one vector share their statistics.  w1 / w2 NULL: that output is not made.
@@ -110,8 +117,8 @@ void psk_mingru_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off,
 // Causal convolution over time on each channel, taps taken from the step's rows and, before them, from the sequence's tail (the last taps - 1
 // inputs of earlier steps, [taps - 1][C] at step->state + tail_off): out[t][c] = f(sum_j w[c][j] in(t - taps + 1 + j)[c]); mode 0: f = in(t) + sum
 // (a residual around the convolution), mode 1: f = silu(sum + bias[c]) (bias NULL: none).  The tail is brought up to date behind it.
-void psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, const float *in, int64_t ldi, const float *w, int taps, int mode,
-                     int64_t C, int T, float *out, int64_t ldo, const float *bias = nullptr);
+bool psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, const float *in, int64_t ldi, const float *w, int taps, int mode,
+                     int64_t C, int T, float *out, int64_t ldo, const float *bias = nullptr, uint16_t *copy16 = nullptr);
 // One token's sublayer boundary fused: x += norm_b(y) (y may be NULL), then h = conv(norm(x)) in the residual form with the tail update (wn may be NULL: stop after x);
 // hn (may be NULL) also receives norm(x) itself, for a sublayer that reads the unfiltered input
 void psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
@@ -138,9 +145,9 @@ void psk_delta_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, 
 void psk_ssd_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *x, const float *B, const float *C, int64_t ld, const float *dtraw, int64_t ldb,
                   const float *a_log, const float *dt_bias, const float *skip, int H, int G, int N, int P, int T, float *o, int64_t ldo);
 // o[t] = part_norm(o[t] * silu(z[t])) * w: the gate first, then each of `parts` equal stretches of n / parts divided by its own root mean square
-void psk_gate_partnorm(hipStream_t st, float *o, int64_t ldo, const float *z, int64_t ldz, const float *w, int parts, float eps, int64_t n, int T);
+bool psk_gate_partnorm(hipStream_t st, float *o, int64_t ldo, const float *z, int64_t ldz, const float *w, int parts, float eps, int64_t n, int T, uint16_t *copy16 = nullptr);
 // o[t][h][:] = o / sqrt(mean_j o^2 + eps) * w(h, :) * silu(g[t][h][:]);  w_stride = dv (a weight per head) or 0 (one shared by the heads)
-void psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, int64_t ldg, const float *w, int w_stride, float eps, int H, int dv, int T);
+bool psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, int64_t ldg, const float *w, int w_stride, float eps, int H, int dv, int T, uint16_t *copy16 = nullptr);
 // Matrix memory with exponential gates.  q, k [T][H*d], v [T][H*dv] (row stride ld), iraw / fraw [T][H] (row stride ldb) the gates' pre-activations; state per head [dv + 1][d] fp32 at
 // step->state + state_off (a column's d numbers together; the last column is n, the memory of k alone), the running maximum [H] at step->state + m_off.
 //   i = c(iraw), f = ln sigmoid(c(fraw)), c(z) = cap tanh(z / cap);  m' = max(f + m, i);  S <- exp(f + m - m') S + exp(i - m') k v^T, n alike

@@ -72,6 +72,7 @@ struct ps_hip_seq {
     float *ssd_scratch = nullptr; // the chunked recurrences: a state per chunk (and the matrix memory's gates)
     float *lstm_aux = nullptr;    // matrix memory: [max_batch][heads] products with n, then as many running maxima
     int64_t lstm_aux_n = 0;
+    uint16_t *a16 = nullptr; // bf16 models: a portion's rows as the kernel in front of a product has rounded them
     float *abs_scratch = nullptr; // the absorbed single-token attention's folded queries, attended latents and per-tile partials
     void *pack = nullptr; // the wide mat-mul's operand copy
     size_t pack_bytes = 0;
@@ -494,6 +495,11 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         m->pack_bytes = desc->compute == 0 ? (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * 2 : (size_t)(std::max(B, moe_slots) * W) * 4;
         m->split_bytes = psk_dense_split_bytes();
         ok = ok && alloc(&m->pack, m->pack_bytes) && alloc((void **)&m->split, m->split_bytes);
+        if (desc->compute == 0) {
+            int64_t wide = W;
+            mixers([&](LayerPlan &P) { wide = std::max<int64_t>(wide, (int64_t)P.d.heads * std::max(P.d.dim, P.d.vdim)); });
+            ok = ok && alloc((void **)&m->a16, (size_t)B * wide * 2);
+        }
     }
     m->slot_state.assign(desc->n_slots, nullptr);
     m->slot_pos.assign(desc->n_slots, -1);
@@ -552,8 +558,13 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     const int64_t BW = (int64_t)D.max_batch * W;
     psk_embed(st, D.embed, from_step ? nullptr : m->tokens, m->step, T, m->embed_scale, m->hist ? m->hist : m->x, W, D.bigram, D.bigram_buckets, D.bigram_mul_prev,
               D.bigram_mul_cur);
+    // The kernels in front of a portion's products leave a bf16 copy of what they wrote in m->a16 as well: `rounded` says of which buffer, and is forgotten with its contents.
+    uint16_t *copy16 = T > 8 && !tiled ? m->a16 : nullptr;
+    const float *rounded = nullptr;
     auto mm = [&](const ps_dense *w, const float *a, int64_t lda, float *out, int64_t ldo) {
         psk_dense_args g;
+        if (copy16 && a == rounded && w && lda == w->K) g.a16 = copy16;
+        if (out == rounded) rounded = nullptr;
         g.w = w; g.a = a; g.lda = lda; g.T = T; g.out = out; g.ldo = ldo; g.force_tiled = tiled; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
         return g;
     };
@@ -563,10 +574,10 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             psk_boundary1(st, m->step, m->x, y, wb, wn, cw, D.canon_taps, tail_off, D.norm_offset, D.norm_eps, W, m->h, m->hn);
             return;
         }
-        if (y) psk_norm_residual(st, m->x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn);
+        if (y) rounded = psk_norm_residual(st, m->x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn, wn ? nullptr : copy16) ? m->x : nullptr;
         if (wn) {
             if (!y) psk_rmsnorm(st, m->x, W, nullptr, wn, D.norm_offset, D.norm_eps, W, T, m->hn, W, m->groups);
-            psk_causal_conv(st, m->step, tail_off, m->hn, W, cw, D.canon_taps, 0, W, T, m->h, W);
+            rounded = psk_causal_conv(st, m->step, tail_off, m->hn, W, cw, D.canon_taps, 0, W, T, m->h, W, nullptr, copy16) ? m->h : nullptr;
         }
     };
     // One mixer on the input `in`.  Its output projection writes out_scale times its result to `store` (NULL: m->y), or (into given) adds it there.
@@ -579,6 +590,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             auto g = mm(l.out, a, lda, into ? into : store ? store : m->y, W);
             g.alpha = out_scale; g.accum = into ? 1 : 0; g.bias = l.out_bias;
             psk_dense(st, g);
+            if (rounded == a) rounded = nullptr; // (the next mixer overwrites it)
         };
         if (l.kind == PS_MIX_WKV) {
             const int64_t Hd = H * d, NW = 5 * Hd;
@@ -599,7 +611,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             psk_state_store(st, m->step, P.off_shift, in + (int64_t)(T - 1) * W, W);
             if (chunked && psk_chunked_ok((int)d)) psk_wkv_chunked(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->ssd_scratch, m->t3, Hd);
             else psk_wkv_scan(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->t3, Hd);
-            psk_headnorm_gate(st, m->t3, Hd, m->t1 + 3 * Hd, NW, l.onorm, (int)d, D.norm_eps, (int)H, (int)d, T);
+            rounded = psk_headnorm_gate(st, m->t3, Hd, m->t1 + 3 * Hd, NW, l.onorm, (int)d, D.norm_eps, (int)H, (int)d, T, copy16) ? m->t3 : nullptr;
             out_proj(m->t3, Hd);
         } else if (l.kind == PS_MIX_DELTA) {
             const int64_t KHd = (int64_t)l.kv_heads * d, Hv = H * dv;
@@ -611,7 +623,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             else
                 psk_delta_scan(st, m->step, P.off_S, m->t2, m->t2 + KHd, m->t2 + 2 * KHd, t1 + P.cqkv + Hv, t1 + P.cqkv + Hv + H, P.cqkv, ld1, l.a_log, l.dt_bias,
                                (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, Hv);
-            psk_headnorm_gate(st, m->t3, Hv, t1 + P.cqkv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T);
+            rounded = psk_headnorm_gate(st, m->t3, Hv, t1 + P.cqkv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T, copy16) ? m->t3 : nullptr;
             out_proj(m->t3, Hv);
         } else if (l.kind == PS_MIX_GLA) {
             // t1 = [ q | k | v | g | a1 ]; the decay's second matrix (with its bias) -> t2; scan -> t3; per-head norm and gate; out
@@ -622,7 +634,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             psk_dense(st, g2);
             if (chunked && psk_chunked_ok((int)d)) psk_gla_chunked(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->ssd_scratch, m->t3, Hv);
             else psk_gla_scan(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->t3, Hv);
-            psk_headnorm_gate(st, m->t3, Hv, t1 + 2 * Hd + Hv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T);
+            rounded = psk_headnorm_gate(st, m->t3, Hv, t1 + 2 * Hd + Hv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T, copy16) ? m->t3 : nullptr;
             out_proj(m->t3, Hv);
         } else if (l.kind == PS_MIX_WINATTN) {
             // t1 = [ q | k | v | gate ] (+ bias); norms, rotation, ring append and block means; attention -> t3; out
@@ -660,7 +672,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 psk_ssd_chunked(st, m->step, P.off_S, x, Bv, Cv, P.cqkv, dt, ld1, l.a_log, l.dt_bias, l.skip, (int)H, l.kv_heads, (int)d, (int)dv, T, m->ssd_scratch, m->t3, inner);
             else
                 psk_ssd_scan(st, m->step, P.off_S, x, Bv, Cv, P.cqkv, dt, ld1, l.a_log, l.dt_bias, l.skip, (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, inner);
-            psk_gate_partnorm(st, m->t3, inner, t1, ld1, l.onorm, l.norm_parts, D.norm_eps, inner, T);
+            rounded = psk_gate_partnorm(st, m->t3, inner, t1, ld1, l.onorm, l.norm_parts, D.norm_eps, inner, T, copy16) ? m->t3 : nullptr;
             out_proj(m->t3, inner);
         } else if (l.kind == PS_MIX_MLSTM) {
             // t1 = [ q | k | v | g | i | f ] (+ bias); the memory -> t3, its products with n and running maxima -> lstm_aux; denominator, head norm and gate; out
@@ -724,14 +736,17 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         g.bias = P.joint_bias;
         psk_dense(st, g);
     };
-    auto ff_up = [&](const LayerPlan &P, const float *in) {
+    // the first product of a dense feed-forward; returns the bf16 rows that the second one is to read (NULL: m->t4 as it is).  512 tokens of 8192: 33 MB less through memory.
+    auto ff_up = [&](const LayerPlan &P, const float *in) -> const void * {
         const ps_seq_layer &l = P.d;
         auto g = mm(l.ff_up, in, W, m->t4, l.ff);
         if (l.ff_kind == PS_FF_DENSE_SWIGLU) g.act = PSD_ACT_SILU_PAIR;
         else if (l.ff_kind == PS_FF_DENSE_RELU_GLU) g.act = PSD_ACT_RELU_PAIR;
         else { g.act = PSD_ACT_XIELU; g.act_p = P.act_p; g.act_q = P.act_q; }
         if (l.ff_kind != PS_FF_DENSE_XIELU) g.bias = l.ff_up_bias;
+        if (psk_dense_wide16(g) && psk_dense_wide16(mm(l.ff_down, m->t4, l.ff, m->y, W))) g.out16 = m->t4;
         psk_dense(st, g);
+        return g.out16;
     };
     // The feed-forward of a layer on `in`, added to xr times alpha (store: written there instead).  Mixture of experts: slot s = t top + i is token t's i-th choice; the router's
     // score scales what the expert READS (the A operand of its first product) or, moe_weight_output, what it puts out (the rows of its inner activation: the second
@@ -741,8 +756,9 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         const ps_seq_layer &l = P.d;
         const bool moe = l.ff_kind == PS_FF_MOE_SWIGLU || l.ff_kind == PS_FF_MOE_RELU2;
         if (!moe) {
-            ff_up(P, in);
+            const void *a16 = ff_up(P, in);
             auto g = mm(l.ff_down, m->t4, l.ff, xr, W);
+            g.a16 = a16;
             g.accum = !store; g.alpha = alpha;
             if (l.ff_kind != PS_FF_DENSE_XIELU) g.bias = l.ff_down_bias;
             psk_dense(st, g);
@@ -796,6 +812,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         }
         if (l.moe_identity && !summed) psk_moe_combine(st, xr, nullptr, top, alpha, W, T, m->moe_sel, m->moe_wgt, E, in, W);
         if (l.shared_up) {
+            if (!up_made && psk_dense_wide16(su) && psk_dense_wide16(sd)) sd.a16 = su.out16 = su.out; // (as in ff_up)
             if (!up_made) psk_dense(st, su);
             if (!down_made) psk_dense(st, sd);
         }
@@ -807,6 +824,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         const ps_seq_layer &l = P.d;
         const LayerPlan *next = li + 1 < n_runs ? &m->L[li + 1] : nullptr;
         const float res = l.res_scale != 0.f ? l.res_scale : 1.f;
+        if (l.form == PS_LAYER_PRENORM || (l.form == PS_LAYER_PARALLEL && !l.canon1)) rounded = nullptr; // (their fronts write h and x themselves)
         if (l.form == PS_LAYER_PRENORM) {
             // x += mixer(norm1(x)), then x += ff(norm2(x)): each sublayer's front is one launch, its output projection adds straight into the residual stream
             psk_front(st, m->x, 0, 1, nullptr, nullptr, nullptr, l.norm1, m->h, nullptr, nullptr, m->groups, D.norm_offset, D.norm_eps, W, T, D.norm_center);
@@ -820,6 +838,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         } else if (l.form == PS_LAYER_POSTNORM) {
             // x += norm_b(mixer(x)), then x += norm_b(ff(x)): a sublayer's first product reads the residual stream, its last one writes y
             auto post = [&](const float *w, const float *b) {
+                rounded = nullptr;
                 if (D.norm_center || b) psk_postnorm(st, m->x, m->y, nullptr, 0.f, nullptr, nullptr, 0.f, w, b, D.norm_offset, D.norm_center, D.norm_eps, W, T);
                 else boundary(m->y, w, nullptr, nullptr, 0);
             };
@@ -827,6 +846,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             if (l.mix_onorm) { // the mixers' outputs side by side (y and h), normed one by one, summed, normed and added in one launch
                 mixer(P, m->x, nullptr, 1.f);
                 if (P.side) mixer(*P.side, m->x, nullptr, 1.f, m->h);
+                rounded = nullptr;
                 psk_postnorm(st, m->x, m->y, l.mix_onorm, l.mix_scale, P.side ? m->h : nullptr, P.side ? P.side->d.mix_onorm : nullptr, P.side ? P.side->d.mix_scale : 0.f, l.norm1b,
                              l.norm1b_bias, D.norm_offset, D.norm_center, D.norm_eps, W, T);
             } else {
@@ -844,6 +864,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 g.em_table = D.side_embed; g.em_col = (int64_t)P.layer * D.side_dim; g.em_tokens = from_step ? nullptr : m->tokens; g.em_step = m->step;
                 psk_dense(st, g);
                 psk_dense(st, mm(l.side_proj, m->t4, D.side_dim, m->y, W));
+                rounded = nullptr;
                 if (T == 1 && !tiled) psk_boundary1(st, m->step, m->x, m->y, l.side_norm, nullptr, nullptr, 1, 0, 0.f, D.norm_eps, W, nullptr, nullptr);
                 else psk_norm_residual(st, m->x, m->y, l.side_norm, 0.f, D.norm_eps, W, T);
             }
@@ -878,8 +899,10 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             const int64_t no = nseq ? next->off_canon1 : 0;
             if (l.ff_kind != PS_FF_NONE) {
                 boundary(m->y, l.norm1b, l.norm2, l.canon2, P.off_canon2);
-                ff_up(P, m->h);
-                psk_dense(st, mm(l.ff_down, m->t4, l.ff, m->y, W));
+                const void *a16 = ff_up(P, m->h);
+                auto g = mm(l.ff_down, m->t4, l.ff, m->y, W);
+                g.a16 = a16;
+                psk_dense(st, g);
                 boundary(m->y, l.norm2b, nn, nc, no);
             } else {
                 boundary(m->y, l.norm1b, nn, nc, no);

@@ -356,3 +356,17 @@ def test_a_sequence_longer_than_the_context_is_refused(ctx, tmp_path):
     m.forward(s, [1, 2])
     m.release(s)
     m.close()
+
+
+# bf16 rows handed from the filter and from the recurrence's head norm to the wide mat-muls behind them, with two mixers side by side that share the first and the buffer of the second
+@pytest.mark.parametrize("sizes", [(9, 40), (64,)])
+def test_bf16_rows_handed_on_side_by_side(made, sizes):
+    cfg = PC(320, 40, [PL(576, att(5, 1, 64, 64, 33, 5, 16), gla(5, 32, 64, 8.0), 1.0, 0.7), PL(320, att(4, 2, 16, 80, 20, 4, 16), gla(2, 16, 160, 4.0), 0.8, 1.0)], taps=4)
+    m, c, t = made("handed", "bfloat16", max_batch=64, cfg=cfg)
+    toks = tokens_for(c, 130)
+    want, got = seq_oracle.run_parallel(c, t, toks), run_portions(m, toks, sizes)
+    m.set_mode(2)  # the tiled mat-mul, which reads and rounds every operand itself
+    plain = run_portions(m, toks, sizes)
+    m.set_mode(0)
+    # both round the same numbers; their fp32 sums differ in order, so a rounding behind them may go the other way: an error of the same origin and size.  A row that is not its own: ~1
+    assert err(got, want) < 1.5 * err(plain, want) < 0.3

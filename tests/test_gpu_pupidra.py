@@ -573,3 +573,14 @@ def test_a_sequence_fills_its_context_and_no_more(ctx, tmp_path):
     m.release(s)
     assert err(np.concatenate(got), seq_oracle.run_pupidra(cfg, t, toks)) < TOL["float32"]
     m.close()
+
+
+# bf16 rows handed from a sublayer's end, from the gated norm of the recurrence and from the shared expert's first product to the wide mat-muls behind them (float32 beside it: nothing is)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_bf16_rows_handed_on(made, dtype):
+    cfg = UC(320, 40, [UL("mamba2", UM(10, 64, 32, 2, 4, 2), (3, 2, 64, 1.0), 448), UL("attention", UA(5, 1, 64, 64, 0.3, 30, 4), (2, 1, 320, 2.0), 320), UL("mamba2", UM(5, 64, 16, 1, 2, 5))])
+    m, c, t = made("handed", dtype, max_batch=64, cfg=cfg)
+    toks = tokens_for(c, 130)
+    want = seq_oracle.run_pupidra(c, t, toks)
+    for sizes in ((9, 40), (64,)):
+        assert close(run_portions(m, toks, sizes), want, dtype), sizes

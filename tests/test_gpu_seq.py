@@ -162,6 +162,23 @@ def test_filters_and_norms_of_portions(made, width, sizes):
     assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
+# bf16 rows handed from one kernel to the wide mat-mul behind it (inputs of more than 256 numbers, whole blocks of 64): filter -> projection, head norm -> projection, first -> second product;
+# beside them a projection that does not take them (260 is no multiple of 64), portions below and above the sizes that hand on, and what an earlier layer or portion left behind
+@pytest.mark.parametrize("sizes", [(9, 8, 64), (33, 1), (64,)])
+def test_bf16_rows_handed_on(made, sizes):
+    cfg = synth.seq_config(320, 50, [L("wkv", 576, heads=5, dim=64), L("delta", 260, heads=6, kv_heads=3, dim=32, vdim=64, conv=4),
+                                     L("latent_attention", 320, heads=5, dim=64, vdim=64, q_rank=64, kv_rank=64, mask={"size": 30}, scale=0.1, rot={"base": 500.0, "dims": 16}, rot_dim=16),
+                                     L("delta", None, heads=2, kv_heads=2, dim=16, vdim=130, conv=4)], taps=4)
+    m, c, t = made("handed", "bfloat16", max_batch=64, cfg=cfg)
+    toks = tokens_for(c, 150)
+    want, got = seq_oracle.run(c, t, toks), run_portions(m, toks, sizes)
+    m.set_mode(2)  # the tiled mat-mul, which reads and rounds every operand itself
+    plain = run_portions(m, toks, sizes)
+    m.set_mode(0)
+    # both round the same numbers; their fp32 sums differ in order, so a rounding behind them may go the other way: an error of the same origin and size.  A row that is not its own: ~1
+    assert err(got, want) < 1.5 * err(plain, want) < 0.3
+
+
 # K up to 32 (k_dense.hip dense_mm_few_kernel): one below, at and above its two widths (33: the tiled kernel), one token and one column more and less than a work-group's
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(9, 1, 1), (15, 255, 7), (16, 256, 8), (17, 257, 9), (33, 70, 31), (31, 513, 32), (40, 65, 33)])
