@@ -452,11 +452,15 @@ struct dn_ring {
     long long lda;      // bytes
     int n_tm, tn, S;    // token tiles (grouped: at most, over all matrices), output tiles, splits of K
     float *part;        // S > 1: [tile][S][register order]
+    long long each;     // > 0: the columns are those of several matrices with `each` of them (a multiple of BN), matrix i = w[i] over the operand copy i
+    const void *w[1 + psk_dense_args::MORE];
+    long long copy;     // bytes between their operand copies
 };
 
 // The A operand's rows with everything resolved that is not a plain row -- ring rows, token-shift mix, the slots' order and scale -- and, for bf16, rounded.
 template <typename WT>
-__global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) {
+__global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) { // (blockIdx.y: the copy for the i-th of several mixes)
+    if (blockIdx.y) { g.mu += (long long)blockIdx.y * g.K; out += (long long)blockIdx.y * g.T * g.K; }
     long long row0 = g.a_row0;
     int T = g.T;
     if (!g.g_list) dn_rows(g, row0, T); // (grouped: all T slots in the order of the sorted list, whatever their matrix)
@@ -600,17 +604,25 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
     if (loads) {
         const int lw = wave - 4, lr = lane >> 3, ls = lane & 7;
-        const char *W = (const char *)g.w + (g.g_seg ? e * g.wstride * (long long)sizeof(WT) : 0), *src[NI];
+        const char *W = (const char *)g.w + (g.g_seg ? e * g.wstride * (long long)sizeof(WT) : 0), *A = p.A, *src[NI];
+        long long nw = n0, n_rows = g.N; // first row of W, rows of W
+        if (p.each) { // (uniform)
+            const int i = (int)(n0 / p.each);
+            W = (const char *)(i == 0 ? p.w[0] : i == 1 ? p.w[1] : i == 2 ? p.w[2] : p.w[3]);
+            A += i * p.copy;
+            nw = n0 - i * p.each;
+            n_rows = p.each;
+        }
 #pragma unroll
         for (int j = 0; j < NI; j++) {
             const int row = 8 * (NI * lw + j) + lr, kq = ls ^ ((row >> 1) & 7);
             const char *q;
             if (row < BM) {
                 const int t = min(t0 + row, T - 1);
-                q = p.A ? p.A + (g.g_seg ? row0 + t : t) * p.lda : (const char *)dn_arow(g, row0, t);
+                q = A ? A + (g.g_seg ? row0 + t : t) * p.lda : (const char *)dn_arow(g, row0, t);
             } else {
-                const long long n = n0 + row - BM;
-                q = W + (n < g.N ? n : g.N - 1) * ldw;
+                const long long n = nw + row - BM;
+                q = W + (n < n_rows ? n : n_rows - 1) * ldw;
             }
             src[j] = q + (long long)kb0 * 128 + kq * 16;
         }
@@ -777,18 +789,25 @@ static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
 
 // the wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed
 template <typename WT>
-static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
+static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     const int64_t kbytes = g.K * (int64_t)sizeof(WT);
+    const int copies = 1 + a.n_more;
+    if (copies > 1 && (g.N % 128 || !g.mu)) return false;
     if (a.force_tiled || kbytes % 128 || !a.pack) return false;
     const bool rows = !g.mu && !g.g_list && !g.a_mod && !g.a_step && !g.a_row0;
     const bool handed = sizeof(WT) == 2 && a.a16 && rows; // (the producer has rounded them already)
     const bool plain = handed || (sizeof(WT) == 4 && !g.mu && !g.g_scale && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0);
-    if (!plain && (size_t)a.T * kbytes > a.pack_bytes) return false;
+    if (!plain && (size_t)a.T * kbytes * copies > a.pack_bytes) return false;
+    const int64_t each = g.N;
+    g.N *= copies;
     const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes());
     dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes, r.n_tm, r.tn, r.S, a.split};
+    p.each = copies > 1 ? each : 0;
+    p.copy = a.T * kbytes;
+    for (int i = 0; i < copies; i++) p.w[i] = i ? a.more[i - 1]->data : g.w;
     if (!plain) {
         const int64_t pb = ((int64_t)a.T * (g.K / 8) + 255) / 256;
-        hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192)), dim3(256), 0, st, g, (WT *)a.pack);
+        hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192), (unsigned)copies), dim3(256), 0, st, g, (WT *)a.pack);
     }
     if (r.BM == 128) dn_launch_ring<WT, 128, 128>(st, g, p);
     else if (r.BN == 128) dn_launch_ring<WT, 64, 128>(st, g, p);
@@ -906,22 +925,30 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_narrow_kernel(dn_args g) {
 //  Sixteen units in flight, and the activations requested ahead of the weights, were tried and are slower (the registers cost a work-group per CU).
 //   FORM 0  one matrix
 //   FORM 1  grouped, the first product of an expert: work-groups in equal runs per slot (its own matrix and output row), behind them those of the shared expert (g2)
+//   FORM 2  several matrices of one shape, each over its own mix of the token and the one before it (psk_dense_args::more): work-groups in equal runs per matrix.  Four of 4096 x 4096,
+//           33 MB each: 10.7 us one by one, 23.7 together (5.7 TB/s)
 // dynamic LDS: the activations as bf16-rounded fp32 (fp32 mode: as they are), every vector padded with zeros to whole units
 #define DN_AHEAD 8
 struct dn_mv1 {
     dn_args g2;  // FORM 1: the shared expert's first product (w NULL: none)
     int slots;   // FORM 1: slots of the launch
     int kp;      // padded length of the vector
-    int blocks, blocks2; // FORM 1: work-groups per slot, of the shared expert
+    int blocks, blocks2; // FORM 1: work-groups per slot, of the shared expert; FORM 2: per matrix
+    const void *w[1 + psk_dense_args::MORE]; // FORM 2: the matrices
 };
 
 // one vector into LDS, by all 512 threads
 template <typename WT>
 static __device__ __forceinline__ void dn_stage(const dn_args &g, const float *x, const float *prev, float scale, float *xs, int kp) {
     const int K = (int)g.K;
-    if (!prev && K % 4 == 0 && ((uintptr_t)x & 15) == 0) {
+    if (K % 4 == 0 && ((uintptr_t)x & 15) == 0 && (!prev || (((uintptr_t)prev | (uintptr_t)g.mu) & 15) == 0)) {
         for (int k = threadIdx.x * 4; k < kp; k += 512 * 4) {
             dn_f4 v = k < K ? *(const dn_f4 *)(x + k) : dn_f4{0.f, 0.f, 0.f, 0.f};
+            if (prev && k < K) { // (the token-shift mix of dn_aval; never with a scale)
+                const dn_f4 b = *(const dn_f4 *)(prev + k), m = *(const dn_f4 *)(g.mu + k);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] += (b[e] - v[e]) * m[e];
+            }
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 v[e] *= scale;
@@ -934,7 +961,7 @@ static __device__ __forceinline__ void dn_stage(const dn_args &g, const float *x
 #pragma unroll 4
     for (int k = threadIdx.x; k < kp; k += 512) {
         float v = k < K ? x[k] * scale : 0.f;
-        if (prev && k < K) v += (prev[k] - v) * g.mu[k]; // (the token-shift mix of dn_aval; never with a scale)
+        if (prev && k < K) v += (prev[k] - v) * g.mu[k];
         if constexpr (sizeof(WT) == 2) v = dn_bf2f(dn_f2bf(v));
         xs[k] = v;
     }
@@ -973,7 +1000,7 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
     extern __shared__ __attribute__((aligned(16))) float xs[];
     constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE; // elements per lane and per unit
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int y = FORM == 1 ? min((int)blockIdx.x / p.blocks, p.slots) : 0;
+    const int y = FORM == 1 ? min((int)blockIdx.x / p.blocks, p.slots) : FORM == 2 ? (int)blockIdx.x / p.blocks : 0;
     const bool shared_seg = FORM == 1 && y == p.slots;
     dn_args g = g0;
     int sel = 0;
@@ -988,11 +1015,16 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
         g.alpha = shared_seg ? p.g2.alpha : g0.alpha;
         sel = shared_seg ? 0 : g.g_sel[y];
     }
-    const bool has = FORM == 0 || shared_seg || sel < g.groups; // (an identity expert has no matrix: its rows are zero)
+    if constexpr (FORM == 2) {
+        g.w = y == 0 ? p.w[0] : y == 1 ? p.w[1] : y == 2 ? p.w[2] : p.w[3];
+        g.mu += (long long)y * g.K;
+        g.out += (long long)y * g.N;
+    }
+    const bool has = FORM != 1 || shared_seg || sel < g.groups; // (an identity expert has no matrix: its rows are zero)
     const int row_units = has ? p.kp / UNIT : 0, N = (int)g.N, K = (int)g.K;
     const bool pair = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR;
     // this wave's rows: first + k step (pairs: first + (k / 2) step + k % 2), k < rows
-    const int bx = FORM == 1 ? (int)blockIdx.x - y * p.blocks : (int)blockIdx.x, nb = FORM == 1 ? (shared_seg ? p.blocks2 : p.blocks) : (int)gridDim.x;
+    const int bx = FORM ? (int)blockIdx.x - y * p.blocks : (int)blockIdx.x, nb = FORM ? (shared_seg ? p.blocks2 : p.blocks) : (int)gridDim.x;
     const int step = nb * 8 * (pair ? 2 : 1), first = (bx * 8 + wave) * (pair ? 2 : 1);
     const int rows = first >= N ? 0 : pair ? ((N - first + step - 2) / step) * 2 : (N - first + step - 1) / step;
     auto row_of = [&](int k) { return pair ? first + (k >> 1) * step + (k & 1) : first + k * step; };
@@ -1000,7 +1032,7 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
     int lk = -1, lu = 0;
     const char *lp = nullptr, *lrow = nullptr;
     const bool beyond = (row_units - 1) * UNIT + lane * VE >= K; // this lane's bytes of a row's last unit lie behind the row's end: it reads the row's first ones, against zeros
-    const WT *mat = (const WT *)g.w + (FORM == 0 || shared_seg ? 0 : (long long)sel * g.wstride);
+    const WT *mat = (const WT *)g.w + (FORM != 1 || shared_seg ? 0 : (long long)sel * g.wstride);
     auto open = [&]() {
         if (++lk >= rows) return;
         lrow = (const char *)(mat + (long long)row_of(lk) * K);
@@ -1021,7 +1053,7 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
         for (int u = 0; u < DN_AHEAD; u++) request(ring[u]);
     }
     // the activations
-    if constexpr (FORM == 0) {
+    if constexpr (FORM != 1) {
         long long row0;
         int T;
         dn_rows(g, row0, T);
@@ -1050,7 +1082,7 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
     auto put = [&]() { // the results of rows kept .. done - 1
         const int k = kept + lane;
         const float v = res;
-        dn_put(g, FORM == 0 || shared_seg ? 0 : y, row_of(k), v, __shfl_xor(v, 1, 64), k < done);
+        dn_put(g, FORM != 1 || shared_seg ? 0 : y, row_of(k), v, __shfl_xor(v, 1, 64), k < done);
         kept = done;
     };
     if (row_units) {
@@ -1074,7 +1106,7 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
 
 // Work-groups of eight waves: enough that every wave has a row, at most two per CU (one where the activations are long: each group stages them for itself).
 template <typename WT, int FORM>
-static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, int slots) {
+static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, int slots, const psk_dense_args *a = nullptr) {
     constexpr int UNIT = 64 * 16 / (int)sizeof(WT);
     dn_mv1 p;
     if (g2) p.g2 = *g2;
@@ -1093,6 +1125,12 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
         p.blocks = (int)((g.N + rounds * per - 1) / (rounds * per));
         p.blocks2 = g2 ? (int)((g2->N + rounds * per - 1) / (rounds * per)) : 0;
         grid = (int64_t)p.blocks * slots + p.blocks2;
+    }
+    if (FORM == 2) {
+        const int n = 1 + a->n_more;
+        p.blocks = (int)std::max<int64_t>(std::min<int64_t>((g.N + per - 1) / per, most / n), 1);
+        grid = (int64_t)p.blocks * n;
+        for (int i = 0; i < n; i++) p.w[i] = i ? a->more[i - 1]->data : g.w;
     }
     hipLaunchKernelGGL((dense_mv1_kernel<WT, FORM>), dim3((unsigned)grid), dim3(512), lds, st, g, p);
     return true;
@@ -1293,6 +1331,21 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
     if (!a.w || a.T <= 0) return 0;
     dn_args g = dn_make(a);
     const bool bf = a.w->dtype == PS_BF16;
+    if (a.n_more) { // together where the streaming mat-vec or the wide mat-mul takes them, else one by one.  512 tokens, four of 2048 x 2048: 5.5 + 13.5 us each one by one, 6.0 + 30.0 together
+        bool alike = true;
+        for (int i = 0; i < a.n_more; i++) alike = alike && a.more[i]->dtype == a.w->dtype && a.more[i]->N == a.w->N && a.more[i]->K == a.w->K;
+        if (alike && !a.force_tiled && a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 2>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 2>(st, g, nullptr, 0, &a))) return 0;
+        if (alike && a.T > 8 && (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g))) return 0;
+        for (int i = 0; i <= a.n_more; i++) {
+            psk_dense_args one = a;
+            one.n_more = 0;
+            if (i) one.w = a.more[i - 1];
+            one.mu = a.mu + i * a.w->K;
+            one.out = a.out + i * a.w->N;
+            psk_dense(st, one);
+        }
+        return 0;
+    }
     const size_t kp4 = (size_t)((g.K + 7) / 8 * 8) * 4;
     if (a.groups > 0) {
         g.groups = a.groups; g.N = a.w->N / a.groups; g.wstride = g.N * g.K;

@@ -78,6 +78,11 @@ struct psk_dense_args {
     // with accum)
     const void *a16 = nullptr;
     void *out16 = nullptr;
+    // further matrices of w's shape and format over the same rows, each with a token-shift mix of its own: matrix i (w is 0) mixes with mu + i K and writes the columns out + i N ..
+    // (no bias, activation, addition or groups; mu given)
+    static constexpr int MORE = 3;
+    int n_more = 0;
+    const ps_dense *more[MORE] = {};
 };
 bool psk_dense_wide16(const psk_dense_args &a); // psk_dense will run this as the wide bf16 mat-mul over plain rows
 int psk_dense(hipStream_t st, const psk_dense_args &a);

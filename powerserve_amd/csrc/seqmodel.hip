@@ -488,11 +488,12 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
     if (B > 8) { // the wide mat-mul's operand copy: the widest input of any matrix x a portion's rows (mixture of experts: slots), or the window's rows x the latent
         int64_t kmax = std::max<int64_t>(W, desc->side_dim), kvrows = 0, kvk = 0;
         mixers([&](LayerPlan &P) {
+            if (P.d.kind == PS_MIX_WKV) kmax = std::max<int64_t>(kmax, 4 * W); // (four mixes side by side)
             kmax = std::max<int64_t>({kmax, P.d.ff, P.d.shared_ff, P.d.heads * (int64_t)std::max(P.d.dim, P.d.vdim), P.d.q_rank, P.d.decay_rank});
             if (P.d.kind == PS_MIX_LATENT) { kvrows = std::max<int64_t>(kvrows, P.d.window - 1 + B); kvk = std::max<int64_t>(kvk, P.d.kv_rank); }
         });
         // (fp32: only the token-shift mixes and scaled slots are packed, the window's rows are read in place)
-        m->pack_bytes = desc->compute == 0 ? (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * 2 : (size_t)(std::max(B, moe_slots) * W) * 4;
+        m->pack_bytes = desc->compute == 0 ? (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * 2 : (size_t)(std::max(4 * B, moe_slots) * W) * 4;
         m->split_bytes = psk_dense_split_bytes();
         ok = ok && alloc(&m->pack, m->pack_bytes) && alloc((void **)&m->split, m->split_bytes);
         if (desc->compute == 0) {
@@ -594,10 +595,11 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         };
         if (l.kind == PS_MIX_WKV) {
             const int64_t Hd = H * d, NW = 5 * Hd;
-            const ps_dense *ws[4] = {l.in_r, l.in_k, l.in_v, l.in_g};
-            for (int s = 0; s < 4; s++) {
-                auto g = mm(ws[s], in, W, m->t1 + s * Hd, NW);
-                g.mu = l.mu + s * W; g.shift0 = state + P.off_shift;
+            { // r | k | v | g, each over its own mix of the tokens and those before them
+                auto g = mm(l.in_r, in, W, m->t1, NW);
+                g.mu = l.mu; g.shift0 = state + P.off_shift;
+                g.n_more = 3;
+                g.more[0] = l.in_k; g.more[1] = l.in_v; g.more[2] = l.in_g;
                 psk_dense(st, g);
             }
             {

@@ -162,6 +162,23 @@ def test_filters_and_norms_of_portions(made, width, sizes):
     assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
+# the four token-shift products of a layer in one launch: columns that are whole tiles of 128 (the wide mat-mul; a tile's matrix changes with it) and that are not (one by one), a single token
+# (its state vector 16-byte aligned and not: 20 channels of another layer in front), two to eight tokens (one by one), a portion split along K
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,heads,dim", [(64, 2, 64), (64, 3, 32), (72, 1, 128), (576, 2, 192), (1024, 4, 32), (66, 2, 20)])
+def test_four_mixes_together(made, width, heads, dim, dtype):
+    wkv = L("wkv", None, heads=heads, dim=dim)
+    # (bfloat16: one layer, whose own roundings the tolerance is for; a recurrence over a recurrence carries them on)
+    cfg = synth.seq_config(width, 40, [wkv] if dtype == "bfloat16" else [wkv, L("latent_attention", 24, heads=1, dim=8, vdim=12, q_rank=9, kv_rank=11, mask={"size": 3}, scale=1.0,
+                                                                                rot={"base": 100.0, "dims": 2}, rot_dim=6), wkv], taps=2)
+    m, c, t = made(f"mixes{width}.{heads}", dtype, max_batch=64, cfg=cfg)
+    toks = tokens_for(c, 60)
+    want = seq_oracle.run(c, t, toks)
+    for sizes in ((1,), (5, 9, 2, 44)):
+        e = err(run_portions(m, toks, sizes), want)
+        assert e < TOL[dtype], (sizes, e)
+
+
 # bf16 rows handed from one kernel to the wide mat-mul behind it (inputs of more than 256 numbers, whole blocks of 64): filter -> projection, head norm -> projection, first -> second product;
 # beside them a projection that does not take them (260 is no multiple of 64), portions below and above the sizes that hand on, and what an earlier layer or portion left behind
 @pytest.mark.parametrize("sizes", [(9, 8, 64), (33, 1), (64,)])
