@@ -92,6 +92,21 @@ def first_layer_adds(m, toks, x0):
     return got
 
 
+# the router of a few tokens with sixteen waves (k_moe.hip moe_route_kernel): as many rows as waves with the shared gate's, one less and one more; rows of one round of pieces, of a round and four
+# numbers more, and of no multiple of four; eight tokens and nine (four waves)
+@pytest.mark.parametrize("width,experts,shared", [(64, 15, 8), (2052, 16, 8), (66, 16, None), (2048, 17, None), (64, 33, 8)])
+def test_router_of_a_few_tokens(made, width, experts, shared):
+    cfg = ZC(width, 40, [ZL("mingru", {"width": 24}, moe=(experts, 2, 8), shared=shared), ZL("mingru", {"width": 24}, moe=(experts, 3, 8), shared=shared)])
+    m, c, t = made(f"router{width}.{experts}", cfg=cfg)
+    toks = tokens_for(c, 19)
+    want = seq_oracle.run_zusolix(c, t, toks)
+    s, got = m.acquire(), []
+    for at, n in ((0, 1), (1, 8), (9, 9), (18, 1)):
+        got.append(m.forward(s, toks[at:at + n], np.arange(n)))
+    m.release(s)
+    assert err(np.concatenate(got), want) < TOL["float32"]
+
+
 # the experts' second product for a few tokens (k_dense.hip dense_mv2_kernel): rows of one unit or a bit of one (512 numbers, fp32: 256), units of several slots and of the shared expert with one
 # wave, one to eight waves per row, up to 8 (fp32: 16) units per wave and one more (the general kernel), more rows than groups of waves
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
