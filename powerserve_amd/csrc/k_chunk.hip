@@ -1,7 +1,7 @@
 // The recurrences whose state is a matrix S [d keys][dv values] per head -- wkv and gated linear attention (a decay per key channel), the gated delta rule (one decay per head) -- for a
 // portion of tokens, in CHUNKS of 16 on the fp32 matrix cores.  What bounded the token-by-token scans (k_seqmix.hip) was a token's chain of LDS reads, sums over a column's lanes and
-// the update, 0.6 - 0.8 us a token whatever the number of heads.  With c_t the running sum of a chunk's log decays (kept in double: a difference is as good as its own size asks
-// for; exponents are never positive), S the state in front of the chunk and tokens t, s of it:
+// the update, 0.6 - 0.8 us a token whatever the number of heads.  With c_t the running sum of a chunk's log decays (each held above CK_LEAST, kept in double: |c| <= 2048, so a
+// difference of two is good to 5e-13; exponents are never positive), S the state in front of the chunk and tokens t, s of it:
 //   decay per channel   o_t = (r_t exp(c_(t-1))) S + sum_(s < t) A_ts v_s + (r_t . bonus k_t) v_t,  A_ts = sum_i r_ti k_si exp(c_(t-1)i - c_si)      (wkv)
 //                       o_t = (q_t exp(c_t)) S + sum_(s <= t) A_ts v_s,  A_ts = sum_i q_ti k_si exp(c_ti - c_si)                                      (gated linear attention)
 //                       S   <- diag(exp(c_end)) S + sum_s (k_s exp(c_end - c_s)) v_s^T
@@ -18,6 +18,10 @@
 typedef float ck_f4 __attribute__((ext_vector_type(4)));
 #define CK_Q 16
 
+// A token's log decay, from below: e^-128 is zero in fp32 as every decay below it is (the scans' exp(-1e30) or exp(-inf)), but beside a -1e13 in the running sum the decays behind it would
+// be lost, and -inf - -inf is no number.  (A NaN stays one.)
+#define CK_LEAST -128.f
+static __device__ __forceinline__ float ck_log_decay(float x) { return x < CK_LEAST ? CK_LEAST : x; }
 static __device__ __forceinline__ float ck_softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 // What a chunk of a head leaves for the scan (floats; d a multiple of 16, so every part is 16-byte aligned)
@@ -50,7 +54,7 @@ __global__ __launch_bounds__(256) void chunk_decay_prep_kernel(const float *r, c
         double c = 0.0;
 #pragma unroll
         for (int t = 0; t < CK_Q; t++) {
-            if (t < nt) c += (double)(GLA ? -ck_softplus(-zv[t]) * inv_tau : -expf(zv[t]));
+            if (t < nt) c += (double)ck_log_decay(GLA ? -ck_softplus(-zv[t]) * inv_tau : -expf(zv[t]));
             cs[t * ldr + i] = c;
         }
         out[at.decay() + i] = expf((float)c);
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(256) void chunk_delta_prep_kernel(const float *q, c
     if (tid < CK_Q) { // running log decays and write strengths (tokens that are not there: no decay, nothing written)
         const bool in = tid < nt;
         const long long rr = t0 + min(tid, nt - 1);
-        double c = in ? (double)(-expf(a_log[h]) * ck_softplus(araw[rr * ldb + h] + dt_bias[h])) : 0.0;
+        double c = in ? (double)ck_log_decay(-expf(a_log[h]) * ck_softplus(araw[rr * ldb + h] + dt_bias[h])) : 0.0;
 #pragma unroll
         for (int o = 1; o < CK_Q; o <<= 1) {
             const double u = __shfl_up(c, o, 64);

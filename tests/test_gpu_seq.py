@@ -91,6 +91,25 @@ def test_recurrences_in_chunks(made, sizes):
     assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
+# channels and heads that forget everything at once at some tokens and next to nothing at others: a token's log decay runs from nothing over e^30 .. e^45, where a running sum of them would
+# swallow the ordinary decays behind it, to an overflow of fp32; the state that the next portion starts from is right too.  (32 tokens and more: chunks; 31 and fewer: the scan)
+@pytest.mark.parametrize("sizes", [(32,), (47, 5, 49), (31, 33)])
+def test_recurrences_in_chunks_that_forget_everything(made, sizes):
+    cfg = synth.seq_config(64, 40, [L("wkv", None, heads=2, dim=32), L("delta", None, heads=4, kv_heads=2, dim=32, vdim=20, conv=2)], taps=2)
+    t = synth.seq_tensors(cfg, 6)
+    gain = np.tile(np.float32([1, 15, 30, 45, 60, 95, 0, 1]), 8)[:, None]  # z = w0 + gain times a number of about 0.6
+    t["l0.mix.w2"] = t["l0.mix.w2"] * gain
+    t["l0.mix.w0"] = np.tile(np.float32([0, 0, 0, 0, 0, 0, 92, 37]), 8)
+    t["l1.mix.a"] = t["l1.mix.a"] * np.float32([[1], [30], [30], [1]])
+    t["l1.mix.A_log"] = np.float32([1, 30, 37, 92])
+    t = {n: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(np.shape(a)) for n, a in t.items()}
+    m, c, t = made("forget", max_batch=64, cfg=cfg, tensors=t)
+    toks = tokens_for(c, 150)
+    with np.errstate(over="ignore"):
+        want = seq_oracle.run(c, t, toks)
+    assert err(run_portions(m, toks, sizes), want) < TOL["float32"]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(1, 37, 50), (2, 64, 96), (3, 19, 7), (8, 130, 72), (9, 70, 33), (70, 129, 200), (200, 48, 48), (1, 16, 4096)])
 def test_dense_matmul_any_shape(ctx, dtype, T, N, K):
