@@ -3,8 +3,8 @@
 //   U     = sum_s exp(c_end - c_s) dt_s x_s B_s^T               what a chunk adds to the state                  ssd_state_kernel, all chunks at once
 //   S_in  <- exp(c_end) S_in + U                                the state in front of every chunk               ssd_pass_kernel, an element per lane, chunk after chunk
 //   y_t   = exp(c_t) S_in C_t + sum_(s <= t) exp(c_t - c_s) dt_s (C_t . B_s) x_s + skip x_t                     ssd_out_kernel, all chunks at once
-// Everything is fp32 (v_mfma_f32_16x16x4_f32); the running sums are kept in double, so that a difference of two of them is as good as its own size asks for.  Exponents are
-// never positive.  x [T][H P], B and C [T][G N] share a row stride; the state is [H][P][N].
+// Everything is fp32 (v_mfma_f32_16x16x4_f32); the running sums are kept in double, and a state-space token's share of them above -128 (sd_decays): |c| <= 8192, so a difference of two is
+// good to 2e-12.  Exponents are never positive.  x [T][H P], B and C [T][G N] share a row stride; the state is [H][P][N].
 //
 // The matrix memory with exponential gates (PS_MIX_MLSTM) is the same recurrence with q, k, v for C, B, x, a log decay f_t and a log input weight i_t of its own, everything relative
 // to a running maximum m_t = max(f_t + m_(t-1), i_t), and one value column more that is 1 for every token (n; the state is [H][P + 1][N]).  With c_t the running sum of f over a
@@ -30,7 +30,9 @@ static __device__ __forceinline__ void sd_decays(const float *dtraw, long long l
     if (threadIdx.x < SD_Q) {
         const int lane = threadIdx.x, t = t0 + lane;
         const float dt = t < T ? sd_softplus(dtraw[(long long)t * ldb + h] + dt_bias[h]) : 0.f;
-        double v = (double)(-expf(a_log[h]) * dt);
+        // (from below: e^-128 is zero in fp32, as the scan's decay is; beside a -1e13 in the sum the decays behind it would be lost, and -inf - -inf is no number.  A NaN stays one.)
+        const float decay = t < T ? -expf(a_log[h]) * dt : 0.f;
+        double v = (double)(decay < -128.f ? -128.f : decay);
 #pragma unroll
         for (int o = 1; o < SD_Q; o <<= 1) {
             const double u = __shfl_up(v, o, 64);

@@ -472,6 +472,22 @@ def test_fast_and_slow_decays_side_by_side(made):
         assert err(run_portions(m, toks, sizes), want) < TOL["float32"], sizes
 
 
+def test_heads_that_forget_everything(made):
+    """a log decay that runs within a chunk from nothing over e^30 .. e^45, where a running sum of them would swallow the ordinary decays behind it, to an overflow of fp32"""
+    mc = UM(8, 32, 32, 2, 4, 1)
+    cfg = UC(64, 24, [UL("mamba2", mc)], eps=1e-5)
+    t = synth.seq_tensors(cfg, 7)
+    t["l0.mix.A_log"] = np.float32([0, 5, 30, 33, 37, 40, 92, -4])
+    t["l0.mix.in"] = np.concatenate([t["l0.mix.in"][:-8], t["l0.mix.in"][-8:] * np.float32(30)])  # (the last rows: a step size per head)
+    t = bf16(t)
+    m, _, _ = made("forget", "float32", max_batch=128, cfg=cfg, tensors=t)
+    toks = tokens_for(cfg, 256, seed=11)
+    with np.errstate(over="ignore"):
+        want = seq_oracle.run_pupidra(cfg, t, toks)
+    for sizes in ([128], [1], [70, 3, 64]):
+        assert err(run_portions(m, toks, sizes), want) < TOL["float32"], sizes
+
+
 def test_the_previous_token_crosses_portions(made):
     """a model in which the bigram row decides: portions of every size, single tokens, and the captured greedy step all see the token before"""
     cfg = UC(40, 30, [UL("attention", UA(2, 1, 8, 8, 0.3, 6, 1))], bigram=(101, 13, 7), eps=1e-5)
