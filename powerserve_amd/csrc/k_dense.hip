@@ -5,8 +5,8 @@
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
 //   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
 //   dense_mm_narrow_kernel bf16, K 128 or 256, more than 8 tokens: 32 x 32 tiles, the waves share K
-//   dense_mv1_kernel<WT,FORM> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
-//   dense_mv2_kernel<WT,U> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
+//   dense_mv1_kernel<WT,FORM,RAGGED> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
+//   dense_mv2_kernel<WT,U,RAGGED> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
 //   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns): the activation rows live in LDS, a wave streams RW weight rows at a time
 // All take the same operand description (ps_seq.h psk_dense_args): ring rows, the token-shift mix and the epilogue
 // (bias, activation, scale, a factor from a second table) are part of the launch, so no mixer needs a kernel of its own around its projections.
@@ -995,7 +995,7 @@ static __device__ __forceinline__ float dn_wave_sum(float v) { // every lane get
     return (row(0) + row(16)) + (row(32) + row(48));
 }
 
-template <typename WT, int FORM>
+template <typename WT, int FORM, bool RAGGED> // RAGGED: a row ends inside a unit
 __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
     constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE; // elements per lane and per unit
@@ -1031,7 +1031,8 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
     // the load side of the stream: row lk, unit lu
     int lk = -1, lu = 0;
     const char *lp = nullptr, *lrow = nullptr;
-    const bool beyond = (row_units - 1) * UNIT + lane * VE >= K; // this lane's bytes of a row's last unit lie behind the row's end: it reads the row's first ones, against zeros
+    // this lane's bytes of a row's last unit lie behind the row's end: it reads the row's first ones and puts them aside (an infinite weight times a zero activation is no number)
+    const bool beyond = RAGGED && (row_units - 1) * UNIT + lane * VE >= K;
     const WT *mat = (const WT *)g.w + (FORM != 1 || shared_seg ? 0 : (long long)sel * g.wstride);
     auto open = [&]() {
         if (++lk >= rows) return;
@@ -1068,6 +1069,7 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
     const float *xp = xs + lane * VE;
     float acc = 0.f, res = 0.f;
     auto eat = [&](dn_f4 &v) {
+        if (RAGGED && cu == 1) v = beyond ? dn_f4{0.f, 0.f, 0.f, 0.f} : v;
         acc = dn_unit<WT>(acc, v, xp);
         request(v);
         xp += UNIT;
@@ -1116,7 +1118,10 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
     const size_t lds = (size_t)p.kp * 4;
     if ((g.K * (int64_t)sizeof(WT)) % 16 != 0 || lds > 128 * 1024 || g.N > (1 << 28) || (g2 && (g2->K != g.K || g2->act != g.act || g2->accum != g.accum || g2->N > (1 << 28)))) return false;
     static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv1_kernel<WT, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (ps_first_on_device(&mask)) {
+        (void)hipFuncSetAttribute((const void *)dense_mv1_kernel<WT, FORM, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void *)dense_mv1_kernel<WT, FORM, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    }
     const int per = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR ? 16 : 8; // rows that a work-group takes at once
     const int64_t most = lds <= 72 * 1024 ? 512 : 256;
     int64_t grid = std::min<int64_t>((g.N + per - 1) / per, most);
@@ -1132,7 +1137,8 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
         grid = (int64_t)p.blocks * n;
         for (int i = 0; i < n; i++) p.w[i] = i ? a->more[i - 1]->data : g.w;
     }
-    hipLaunchKernelGGL((dense_mv1_kernel<WT, FORM>), dim3((unsigned)grid), dim3(512), lds, st, g, p);
+    const auto kernel = p.kp == g.K ? dense_mv1_kernel<WT, FORM, false> : dense_mv1_kernel<WT, FORM, true>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), lds, st, g, p);
     return true;
 }
 
@@ -1149,7 +1155,7 @@ struct dn_mv2 {
     int waves, share;  // waves per row, units per wave
     int rows;          // the most rows that a group of waves has
 };
-template <typename WT, int U>
+template <typename WT, int U, bool RAGGED> // RAGGED: a row ends inside a unit
 __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g, dn_mv2 p) {
     extern __shared__ __attribute__((aligned(16))) float sums[];
     constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE, AHEAD = U >= 8 ? 1 : 8 / U; // elements per lane and per unit; rows in flight
@@ -1161,7 +1167,8 @@ __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g
     auto first_of = [&](int gi) { return (int)blockIdx.x * groups + gi; };
     auto rows_of = [&](int gi) { return first_of(gi) >= N ? 0 : (N - first_of(gi) + step - 1) / step; };
     const int first = first_of(wave / p.waves), rows = rows_of(wave / p.waves);
-    // this wave's units: where unit u of row 0 starts, its activations (a lane beyond the row's end reads the unit's first bytes, against zeros)
+    // this wave's units: where unit u of row 0 starts, its activations (a lane beyond the row's end reads the unit's first bytes and puts
+    // them aside: an infinite weight times a zero activation is no number)
     const int all = p.slots * p.units + p.units2, u0 = part * p.share, n_units = max(min(p.share, all - u0), 0);
     const char *base[U];
     bool has[U], second[U]; // (a slot without a matrix -- an identity expert -- has none; second: the shared expert's)
@@ -1184,7 +1191,7 @@ __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g
         }
         const int k = at * UNIT + lane * VE, Kc = second[u] ? K2 : K;
         const bool in = has[u] && k < Kc;
-        lo[u] = k < Kc ? lane * 16 : 0;
+        lo[u] = !RAGGED || k < Kc ? lane * 16 : 0;
         base[u] = (const char *)(w + (long long)at * UNIT);
         const float *xk = xr + k;
         if (((uintptr_t)xr & 15) == 0) { // (uniform)
@@ -1228,6 +1235,7 @@ __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (!has[u]) continue;
+                if (RAGGED && lo[u] != lane * 16) ring[d][u] = dn_f4{0.f, 0.f, 0.f, 0.f};
                 float a = second[u] ? own : acc;
                 if constexpr (sizeof(WT) == 2) {
                     unsigned h[4];
@@ -1281,11 +1289,16 @@ static bool dn_launch_mv2(hipStream_t st, const dn_args &g, const dn_args *g2, i
     const int64_t once = (g.N + per - 1) / per, grid = std::max(std::min<int64_t>(once, std::max(512 / tokens, 64)), (once + 1023) / 1024); // (at most 1024 rounds: 32 KiB of sums)
     p.rows = (int)((once + grid - 1) / grid);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid, (unsigned)tokens), dim3(512), (size_t)8 * p.rows * 4, st, g, p); };
-    if (p.share == 1) go(dense_mv2_kernel<WT, 1>);
-    else if (p.share == 2) go(dense_mv2_kernel<WT, 2>);
-    else if (p.share <= 4) go(dense_mv2_kernel<WT, 4>);
-    else if (p.share <= 8) go(dense_mv2_kernel<WT, 8>);
-    else if constexpr (sizeof(WT) == 4) go(dense_mv2_kernel<WT, 16>);
+    auto pick = [&](auto ragged) {
+        constexpr bool R = decltype(ragged)::value;
+        if (p.share == 1) go(dense_mv2_kernel<WT, 1, R>);
+        else if (p.share == 2) go(dense_mv2_kernel<WT, 2, R>);
+        else if (p.share <= 4) go(dense_mv2_kernel<WT, 4, R>);
+        else if (p.share <= 8) go(dense_mv2_kernel<WT, 8, R>);
+        else if constexpr (sizeof(WT) == 4) go(dense_mv2_kernel<WT, 16, R>);
+    };
+    if (g.K % UNIT || (g2 && g2->K % UNIT)) pick(std::true_type());
+    else pick(std::false_type());
     return true;
 }
 

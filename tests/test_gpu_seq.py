@@ -245,6 +245,30 @@ def test_dense_matvec_in_one_stream(ctx, dtype, N, K):
     dx.free(); do.free()
 
 
+# a weight that is infinite stays infinite in its row's result, and in no other, wherever the row ends in the stream's last unit (one token) and with more tokens
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [1, 2])
+@pytest.mark.parametrize("N,K", [(5, 8), (9, 264), (12, 520), (33, 4104), (9, 512)])
+def test_dense_matvec_with_an_infinite_weight(ctx, dtype, N, K, T):
+    import ctypes as C
+    rng = np.random.default_rng(N + K)
+    bits = f32_to_bf16_bits(rng.standard_normal((N, K), dtype=np.float32))
+    bits[3, 0], bits[1, K - 1] = 0x7F80, 0xFF80  # the first number of a row (what a lane beyond the row's end may be tempted to read), and the last
+    x = rng.uniform(0.5, 1.0, (T, K)).astype(np.float32)
+    w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K)
+    h = C.c_void_p()
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, int(dtype == "float32"), C.byref(h)))
+    dx, do = ctx.to_device(x), ctx.to_device(np.zeros((T, N), np.float32))
+    ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, h, dx.ptr, T, do.ptr, 1.0))
+    got = do.numpy()
+    assert np.all(got[:, 3] == np.inf) and np.all(got[:, 1] == -np.inf)
+    finite = [n for n in range(N) if n not in (1, 3)]
+    want = (x if dtype == "float32" else (f32_to_bf16_bits(x).astype(np.uint32) << 16).view(np.float32).reshape(x.shape)).astype(np.float64) @ w[finite].astype(np.float64).T
+    assert np.all(np.abs(got[:, finite] - want) <= K * 2.0 ** -24 * np.abs(w[finite]).astype(np.float64).sum(1))  # (fp32 sums in any order; |x| <= 1)
+    ctx.L.ps_hip_dense_free(ctx.h, h)
+    dx.free(); do.free()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["wkv", "delta", "latent", "ff", "mixed", "aligned", "wide_heads"])
 def test_whole_prompt_against_the_plain_statement(made, name, dtype):
