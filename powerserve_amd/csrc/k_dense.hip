@@ -1517,20 +1517,27 @@ void ps_hip_dense_free(ps_hip_ctx *c, ps_dense *w) {
 }
 int ps_hip_dense_matmul(ps_hip_ctx *c, const ps_dense *w, const float *x, int T, float *out, float alpha) {
     if (!w || T <= 0) PS_FAIL(c, "dense_matmul: bad argument");
-    psk_dense_args a;
-    a.w = w; a.a = x; a.lda = w->K; a.T = T; a.out = out; a.ldo = w->N; a.alpha = alpha;
-    if (T > 8) { // the wide mat-mul's scratch: the context's own, grown as needed
-        const size_t pack = ((size_t)T * w->K * (w->dtype == PS_BF16 ? 2 : 4) + 255) / 256 * 256, need = pack + psk_dense_split_bytes();
-        if (c->act_cap < need) {
-            PS_CHECK(c, hipStreamSynchronize(c->stream));
-            if (c->act_buf) (void)ps_dev_free(c->act_buf);
-            c->act_buf = nullptr; c->act_cap = 0;
-            PS_CHECK(c, ps_dev_malloc(&c->act_buf, need));
-            c->act_cap = need;
-        }
-        a.pack = c->act_buf; a.pack_bytes = pack; a.split = (float *)((char *)c->act_buf + pack); a.split_bytes = psk_dense_split_bytes();
+    // The wide mat-mul's scratch is the context's and stays with it: 64 MiB of packed rows (128 rows, where those are more) and the parts of split products.  More rows go through it piece
+    // by piece, and where the device has no room for it the product does without.  Products that the wide mat-mul does not take need none.
+    const int64_t row = w->K * (w->dtype == PS_BF16 ? 2 : 4);
+    const bool wide = T > 8 && row % 128 == 0, packs = w->dtype == PS_BF16 || ((uintptr_t)x & 15) != 0;
+    const int64_t piece = wide && packs ? std::min<int64_t>(T, std::max<int64_t>(((int64_t)64 << 20) / row / 128 * 128, 128)) : T;
+    const size_t pack = packs ? (size_t)(piece * row + 255) / 256 * 256 : 0, need = pack + psk_dense_split_bytes();
+    if (wide && c->act_cap < need) {
+        PS_CHECK(c, hipStreamSynchronize(c->stream));
+        if (c->act_buf) (void)ps_dev_free(c->act_buf);
+        c->act_buf = nullptr; c->act_cap = 0;
+        if (ps_dev_malloc(&c->act_buf, need) == hipSuccess) c->act_cap = need;
+        else { c->act_buf = nullptr; (void)hipGetLastError(); }
     }
-    psk_dense(c->stream, a);
+    for (int64_t t = 0; t < T; t += piece) {
+        psk_dense_args a;
+        a.w = w; a.a = x + t * w->K; a.lda = w->K; a.T = (int)std::min<int64_t>(piece, T - t); a.out = out + t * w->N; a.ldo = w->N; a.alpha = alpha;
+        if (wide && c->act_buf) {
+            a.pack = c->act_buf; a.pack_bytes = pack; a.split = (float *)((char *)c->act_buf + pack); a.split_bytes = psk_dense_split_bytes();
+        }
+        psk_dense(c->stream, a);
+    }
     PS_CHECK(c, hipGetLastError());
     return 0;
 }

@@ -37,6 +37,20 @@ def ctx():
     c.close()
 
 
+@pytest.fixture(scope="session")
+def free_bytes(ctx):
+    """what the device has left, as the HIP runtime that the library is linked with says it"""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so.7")
+
+    def get():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    return get
+
+
 def load_tensors(path):
     """{name: (ggml_type, raw bytes, ne0, ne1)} of a GGUF file, as oracle.binding.OracleModel takes them"""
     from powerserve_amd import gguf

@@ -269,6 +269,30 @@ def test_dense_matvec_with_an_infinite_weight(ctx, dtype, N, K, T):
     dx.free(); do.free()
 
 
+# the scratch that a product of many rows takes belongs to the context and stays: it has a bound, and the product goes through it piece by piece
+@pytest.mark.parametrize("dtype,T,N,K", [("bfloat16", 40000, 24, 2048), ("float32", 20001, 24, 2048), ("bfloat16", 1100000, 8, 16)])
+def test_dense_matmul_scratch_is_bounded(free_bytes, dtype, T, N, K):
+    import ctypes as C
+    own = hip.Ctx(0)
+    rng = np.random.default_rng(3)
+    bits = f32_to_bf16_bits(rng.standard_normal((N, K), dtype=np.float32))
+    x = rng.standard_normal((64, K), dtype=np.float32)[np.arange(T) % 61]  # (61 different rows)
+    h = C.c_void_p()
+    own.check(own.L.ps_hip_dense_upload(own.h, bits.ctypes.data_as(C.c_void_p), N, K, int(dtype == "float32"), C.byref(h)))
+    dx, do = own.to_device(x), own.to_device(np.zeros((T, N), np.float32))
+    before = free_bytes()
+    own.check(own.L.ps_hip_dense_matmul(own.h, h, dx.ptr, T, do.ptr, 1.0))
+    got = do.numpy()
+    assert before - free_bytes() <= 100 << 20  # 64 MiB of rows, 32 MiB of parts of split products
+    w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K).astype(np.float64)
+    a = (x[:61] if dtype == "float32" else (f32_to_bf16_bits(x[:61]).astype(np.uint32) << 16).view(np.float32).reshape(61, K)).astype(np.float64)
+    bound = K * 2.0 ** -24 * (np.abs(a) @ np.abs(w).T)
+    assert np.all(np.abs(got - (a @ w.T)[np.arange(T) % 61]) <= bound[np.arange(T) % 61])
+    own.L.ps_hip_dense_free(own.h, h)
+    dx.free(); do.free()
+    own.close()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["wkv", "delta", "latent", "ff", "mixed", "aligned", "wide_heads"])
 def test_whole_prompt_against_the_plain_statement(made, name, dtype):
