@@ -485,7 +485,7 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         if (sb) ok = ok && alloc((void **)&m->ssd_scratch, sb);
         if (m->lstm_aux_n) ok = ok && alloc((void **)&m->lstm_aux, (size_t)m->lstm_aux_n * 2 * 4);
     }
-    if (B > 8) { // the wide mat-mul's operand copy: the widest input of any matrix x a portion's rows (mixture of experts: slots), or the window's rows x the latent
+    { // the wide mat-mul's operand copy: the widest input of any matrix x a portion's rows (mixture of experts: slots), or the window's rows x the latent, which are many however few the tokens
         int64_t kmax = std::max<int64_t>(W, desc->side_dim), kvrows = 0, kvk = 0;
         mixers([&](LayerPlan &P) {
             if (P.d.kind == PS_MIX_WKV) kmax = std::max<int64_t>(kmax, 4 * W); // (four mixes side by side)
@@ -494,9 +494,12 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         });
         // (fp32: only the token-shift mixes and scaled slots are packed, the window's rows are read in place)
         m->pack_bytes = desc->compute == 0 ? (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * 2 : (size_t)(std::max(4 * B, moe_slots) * W) * 4;
-        m->split_bytes = psk_dense_split_bytes();
-        ok = ok && alloc(&m->pack, m->pack_bytes) && alloc((void **)&m->split, m->split_bytes);
-        if (desc->compute == 0) {
+        ok = ok && alloc(&m->pack, m->pack_bytes);
+        if (std::max({B, moe_slots, kvrows}) > 8) {
+            m->split_bytes = psk_dense_split_bytes();
+            ok = ok && alloc((void **)&m->split, m->split_bytes);
+        }
+        if (desc->compute == 0 && B > 8) {
             int64_t wide = W;
             mixers([&](LayerPlan &P) { wide = std::max<int64_t>(wide, (int64_t)P.d.heads * std::max(P.d.dim, P.d.vdim)); });
             ok = ok && alloc((void **)&m->a16, (size_t)B * wide * 2);

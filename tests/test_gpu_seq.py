@@ -293,6 +293,19 @@ def test_dense_matmul_scratch_is_bounded(free_bytes, dtype, T, N, K):
     own.close()
 
 
+# a latent layer's window is expanded with the same kernel, however few tokens the model takes at a time: the same portions give the same bits
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_model_of_few_tokens_takes_the_same_kernels(made, dtype):
+    cfg = synth.seq_config(64, 40, [L("latent_attention", None, heads=4, dim=32, vdim=48, q_rank=20, kv_rank=1088, mask={"size": 70}, scale=0.2, rot={"base": 100.0, "dims": 8}, rot_dim=16)], taps=2)
+    toks = tokens_for(cfg, 120)
+    few, c, t = made("few", dtype, max_batch=8, cfg=cfg)
+    many, _, _ = made("few", dtype, max_batch=32, cfg=cfg, tensors=t)
+    for sizes in ((8,), (2, 5, 8)):
+        got = run_portions(few, toks, sizes)
+        assert np.array_equal(got, run_portions(many, toks, sizes)), sizes
+        assert err(got, seq_oracle.run(c, t, toks)) < TOL[dtype]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["wkv", "delta", "latent", "ff", "mixed", "aligned", "wide_heads"])
 def test_whole_prompt_against_the_plain_statement(made, name, dtype):
