@@ -126,7 +126,7 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
     m->ctx = c;
     m->d = *desc;
     const int64_t W = desc->width, B = desc->max_batch;
-    int64_t off = 0, n1 = 0, n2 = 0, n3 = 0, n4 = 0, nkv = 0, nq = 0;
+    int64_t off = 0, n1 = 0, n2 = 0, n3 = 0, n4 = 0, n4_one = 0, nkv = 0, nq = 0;
     auto fail = [&](const std::string &msg) { ps_hip_seq_destroy(m); return seq_fail(c, "seq_create: " + msg); };
     auto shape = [](const ps_dense *w, int64_t N, int64_t K) { return w && w->N == N && w->K == K; };
     m->max_context = desc->max_context > 0 ? desc->max_context : 65536;
@@ -330,7 +330,8 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
                 moe_slots = std::max(moe_slots, B * l.top);
                 moe_experts = std::max<int64_t>(moe_experts, rows);
                 moe_top = std::max<int64_t>(moe_top, l.top);
-                n4 = std::max<int64_t>(n4, (int64_t)l.top * l.ff + 3 + l.shared_ff); // (a single token's shared expert beside its slots)
+                n4 = std::max<int64_t>({n4, (int64_t)l.top * l.ff, (int64_t)l.shared_ff});
+                n4_one = std::max<int64_t>(n4_one, (int64_t)l.top * l.ff + 3 + l.shared_ff); // (a single token's shared expert beside its slots)
                 m->weight_bytes += (dense_bytes(l.ff_up) + dense_bytes(l.ff_down)) / l.experts * std::min(l.top, l.experts) + (uint64_t)rows * W * 4;
             }
             const int64_t up_rows = l.ff_kind == PS_FF_DENSE_SWIGLU || l.ff_kind == PS_FF_DENSE_RELU_GLU ? 2 * (int64_t)l.ff : l.ff;
@@ -455,7 +456,7 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
     }
     ok = ok && alloc((void **)&m->step, sizeof(ps_seq_step)) && alloc((void **)&m->x, B * W * 4) && alloc((void **)&m->hn, B * W * 4) && alloc((void **)&m->h, B * W * 4) &&
          alloc((void **)&m->y, B * W * 4) && alloc((void **)&m->t1, B * std::max<int64_t>(n1, 1) * 4) && alloc((void **)&m->t2, B * std::max<int64_t>(n2, 1) * 4) &&
-         alloc((void **)&m->t3, B * std::max<int64_t>(n3, 1) * 4) && alloc((void **)&m->t4, B * std::max<int64_t>(n4, 1) * 4) &&
+         alloc((void **)&m->t3, B * std::max<int64_t>(n3, 1) * 4) && alloc((void **)&m->t4, std::max<int64_t>({B * n4, n4_one, 1}) * 4) &&
          alloc((void **)&m->kvx, std::max<int64_t>(nkv, 1) * 4) && alloc((void **)&m->xn, B * W * 4) && alloc((void **)&m->logits, B * (int64_t)desc->vocab * 4) &&
          alloc((void **)&m->tokens, B * 4) && alloc((void **)&m->want, B * 4) && alloc((void **)&m->amax, B * 4);
     if (depth) ok = ok && alloc((void **)&m->hist, (size_t)(order.size() + 1) * B * W * 4);

@@ -126,6 +126,19 @@ def test_experts_of_a_few_tokens(made, width, experts, top, ff, shared, dtype):
     assert max(rows) < TOL["float32"] if dtype == "float32" else float(np.quantile(rows, 0.9)) < TOL[dtype] and max(rows) < 1.0
 
 
+def test_memory_of_a_wide_shared_expert(ctx, free_bytes, tmp_path):
+    """the rows of a portion hold the slots' inner activations or the shared expert's, whichever are more; only a single token has them side by side"""
+    used = []
+    for i, (ff, shared) in enumerate(((8192, 8), (8192, 16384))):
+        d = str(tmp_path / str(i))
+        synth.write_seq_model_dir(d, ZC(8, 24, [ZL("mingru", {"width": 8}, moe=(2, 2, ff), shared=shared)]), 0)
+        before = free_bytes()
+        m = seqmodel.load_model(ctx, d, dtype="float32", max_batch=2048, n_slots=1, max_context=64)
+        used.append(before - free_bytes())
+        m.close()
+    assert used[1] - used[0] < 32 << 20, used  # (1.5 MB more weights; a second set of inner rows would be 134 MB)
+
+
 # ---------------------------------------------------------------------------------------------------------------- mechanisms, one at a time
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("which", ["attention", "attention_mfma", "recurrence", "dense", "mixture", "mixture_aligned"])
