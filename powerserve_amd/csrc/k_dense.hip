@@ -415,9 +415,8 @@ __global__ __launch_bounds__(256) void dense_mv_grouped_kernel(dn_args g) {
         for (int q = 0; q < RW; q++) dn_put(g, r, nb + q, acc[q], acc[RW > 1 ? (q ^ 1) : q], lane == 0 && nb + q < g.N);
     }
 }
-template <typename WT>
+template <typename WT, int RW>
 static void dn_launch_mv_grouped(hipStream_t st, const dn_args &g, int rows, size_t lds) {
-    constexpr int RW = 2;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv_grouped_kernel<WT, RW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     long long blocks = (g.N + 4 * RW - 1) / (4 * RW);
@@ -1333,6 +1332,11 @@ static int dn_grouped_mv1(hipStream_t st, const psk_dense_args &a, const dn_args
         const dn_args g2 = dn_make(*a.also);
         if (second ? dn_launch_mv2<WT>(st, g, &g2, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, &g2, a.T)) return 2;
     }
+    // Alone, the second product is the grouped kernel's where that walks a row in a few trips (two pieces of each slot's matrix at a time) and a token's matrices are not large: measured for one
+    // token and eight, us here and there: 2048 x 1024 of two slots 8.0 / 20.0 and 6.8 / 12.9 (two trips), 2048 x 2048 11.9 / 29.1 and 9.7 / 24.7 (four), 2048 x 3072 12.1 / 29.7 and
+    // 12.2 / 32.0 (six), 4096 x 2048 14.3 / 45.9 and 13.2 / 50.3 (four, 33 MB), 1024 x 512 of six slots 8.0 / 13.1 and 10.2 / 12.9 (six).
+    constexpr int64_t TRIP = 128 * 16 / (int64_t)sizeof(WT);
+    if (second && a.g_inner * ((g.K + TRIP - 1) / TRIP) < 6 && g.N * g.K * a.g_inner * (int64_t)sizeof(WT) < ((int64_t)32 << 20)) return 0;
     return (second ? dn_launch_mv2<WT>(st, g, nullptr, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, nullptr, a.T)) ? 1 : 0;
 }
 
@@ -1366,8 +1370,11 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         if (!a.g_list) { // a few slots
             const int took = bf ? dn_grouped_mv1<unsigned short>(st, a, g) : dn_grouped_mv1<float>(st, a, g);
             if (took) return took == 2;
-            if (bf) dn_launch_mv_grouped<unsigned short>(st, g, a.T, kp4 * a.g_inner);
-            else dn_launch_mv_grouped<float>(st, g, a.T, kp4 * a.g_inner);
+            const int64_t waves4 = (g.N + 3) / 4 * a.T; // four rows per wave only where that still leaves about 1024 waves (a gate / up pair sits in one wave)
+            const int RW = waves4 >= 1024 ? 4 : waves4 >= 512 || g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR ? 2 : 1;
+            const auto launch = bf ? (RW == 4 ? dn_launch_mv_grouped<unsigned short, 4> : RW == 2 ? dn_launch_mv_grouped<unsigned short, 2> : dn_launch_mv_grouped<unsigned short, 1>)
+                                   : (RW == 4 ? dn_launch_mv_grouped<float, 4> : RW == 2 ? dn_launch_mv_grouped<float, 2> : dn_launch_mv_grouped<float, 1>);
+            launch(st, g, a.T, kp4 * a.g_inner);
             return 0;
         }
         g.g_seg = a.g_seg; g.g_list = a.g_list;

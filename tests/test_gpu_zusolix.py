@@ -126,6 +126,22 @@ def test_experts_of_a_few_tokens(made, width, experts, top, ff, shared, dtype):
     assert max(rows) < TOL["float32"] if dtype == "float32" else float(np.quantile(rows, 0.9)) < TOL[dtype] and max(rows) < 1.0
 
 
+# the experts' second product without a shared expert: one, two and four rows per wave of the grouped kernel, one trip of a slot to one short of the six from which the rows in registers take
+# over, six and more.  (Every expert is chosen: no choice can go the other way, so every row is held to the tolerance in bfloat16 too)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,experts,ff", [(64, 2, 264), (2052, 1, 24), (4104, 1, 8), (64, 5, 1024), (64, 6, 520), (72, 3, 1032), (64, 2, 1016)])
+def test_second_products_on_their_own(made, width, experts, ff, dtype):
+    cfg = ZC(width, 40, [ZL("mingru", {"width": 24}, moe=(experts, experts, ff)), ZL("mingru", {"width": 24}, moe=(experts, experts, ff))])
+    m, c, t = made(f"second{width}.{ff}", dtype, cfg=cfg)
+    toks = tokens_for(c, 14)
+    want = seq_oracle.run_zusolix(c, t, toks)
+    s, got = m.acquire(), []
+    for at, n in ((0, 1), (1, 1), (2, 3), (5, 8), (13, 1)):
+        got.append(m.forward(s, toks[at:at + n], np.arange(n)))
+    m.release(s)
+    assert err(np.concatenate(got), want) < TOL[dtype]
+
+
 def test_memory_of_a_wide_shared_expert(ctx, free_bytes, tmp_path):
     """the rows of a portion hold the slots' inner activations or the shared expert's, whichever are more; only a single token has them side by side"""
     used = []
