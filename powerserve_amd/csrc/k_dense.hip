@@ -4,7 +4,7 @@
 //   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
 //   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
-//   dense_mm_narrow_kernel bf16, K 128 or 256, more than 8 tokens: 32 x 32 tiles, the waves share K
+//   dense_mm_narrow_kernel bf16, K a multiple of 128 up to 1024, more than 8 tokens, few tiles: 32 x 32 tiles, the waves share K
 //   dense_mv1_kernel<WT,FORM,RAGGED> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
 //   dense_mv2_kernel<WT,U,RAGGED> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
 //   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns): the activation rows live in LDS, a wave streams RW weight rows at a time
@@ -846,14 +846,14 @@ __global__ __launch_bounds__(256) void dense_mm_few_kernel(dn_args g) {
     }
 }
 
-// Products with an inner size of a few steps (K <= 256: the ring would be all prologue): 32 tokens x 32 outputs per work-group.  Each of the NW waves takes
-// its share of K, its operand fragments straight from memory (the activations are rounded to bfloat16 in registers: nothing is packed beforehand), four steps of 32 in flight; the
+// Products with a short inner size and few tiles (the ring would be all packing and prologue): 32 tokens x 32 outputs per work-group.  Each of the NW waves takes
+// its share of K, its operand fragments straight from memory (the activations are rounded to bfloat16 in registers: nothing is packed beforehand), all its STEPS of 32 in flight; the
 // partial tiles meet in LDS.  Plain rows only (no ring, no token shift, no groups).
-template <int NW>
+template <int NW, int STEPS> // K = NW STEPS 32
 __global__ __launch_bounds__(64 * NW) void dense_mm_narrow_kernel(dn_args g) {
     __shared__ float part[NW][32][33];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lq = lane >> 4, t0 = blockIdx.x * 32; // (rows fastest: the blocks that read the same rows of A sit on one XCD where the row tiles are a multiple of 8)
-    const long long n0 = (long long)blockIdx.y * 32, kw = g.K / NW;
+    const long long n0 = (long long)blockIdx.y * 32, kw = STEPS * 32;
     const float *ap[2];
     const unsigned short *bp[2];
 #pragma unroll
@@ -868,35 +868,30 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_narrow_kernel(dn_args g) {
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[i][j] = dn_f4{0.f, 0.f, 0.f, 0.f};
-    for (long long k0 = 0; k0 < kw; k0 += 128) {
-        dn_f4 xa[4][2][2], xb[4][2];
+    dn_f4 xa[STEPS][2][2], xb[STEPS][2];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const long long k = k0 + 32 * u < kw ? k0 + 32 * u : k0; // (a step beyond the wave's share is loaded from where there is one and not used)
+    for (int u = 0; u < STEPS; u++)
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                xa[u][i][0] = *(const dn_f4 *)(ap[i] + k);
-                xa[u][i][1] = *(const dn_f4 *)(ap[i] + k + 4);
-                xb[u][i] = *(const dn_f4 *)(bp[i] + k);
-            }
+        for (int i = 0; i < 2; i++) {
+            xa[u][i][0] = *(const dn_f4 *)(ap[i] + 32 * u);
+            xa[u][i][1] = *(const dn_f4 *)(ap[i] + 32 * u + 4);
+            xb[u][i] = *(const dn_f4 *)(bp[i] + 32 * u);
         }
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (k0 + 32 * u >= kw) continue; // (uniform)
-            dn_bf8 fa[2], fb[2];
+    for (int u = 0; u < STEPS; u++) {
+        dn_bf8 fa[2], fb[2];
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                dn_us8 r;
+        for (int i = 0; i < 2; i++) {
+            dn_us8 r;
 #pragma unroll
-                for (int e = 0; e < 8; e++) r[e] = dn_f2bf(xa[u][i][e >> 2][e & 3]);
-                __builtin_memcpy(&fa[i], &r, 16);
-                __builtin_memcpy(&fb[i], &xb[u][i], 16);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+            for (int e = 0; e < 8; e++) r[e] = dn_f2bf(xa[u][i][e >> 2][e & 3]);
+            __builtin_memcpy(&fa[i], &r, 16);
+            __builtin_memcpy(&fb[i], &xb[u][i], 16);
         }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -1409,9 +1404,23 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         else bf ? go(dense_mm_few_kernel<unsigned short, 32>) : go(dense_mm_few_kernel<float, 32>);
         return 0;
     }
-    if (bf && !a.force_tiled && a.T > 8 && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 && g.K <= 256) {
+    // K up to 256, and up to 1024 where the small tiles are not more than one per CU and nobody hands rounded rows on (the ring packs its operand first): us here and there, weights from memory,
+    // 2048 x 512: 9 tokens 5.4 and 8.0, 128 tokens 6.7 and 9.0; 1024 x 1024: 9 tokens 7.0 and 9.8, 256 tokens 9.1 and 11.2; 3072 x 1024: 64 tokens (192 tiles) 9.3 and 12.0, 128 tokens
+    // (384) 17.1 and 12.0; 2048 x 2048: 16 tokens 13.4 and 13.1, 64 tokens 15.8 and 13.4.
+    if (bf && !a.force_tiled && a.T > 8 && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 &&
+        (g.K <= 256 || (g.K <= 1024 && (int64_t)((a.T + 31) / 32) * ((g.N + 31) / 32) <= 256 && !a.a16 && !a.out16))) {
         const dim3 grid((unsigned)((a.T + 31) / 32), (unsigned)((g.N + 31) / 32));
-        hipLaunchKernelGGL(dense_mm_narrow_kernel<4>, grid, dim3(256), 0, st, g);
+        auto go = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, st, g); };
+        switch (g.K / 128) {
+        case 1: go(dense_mm_narrow_kernel<4, 1>, 4); break;
+        case 2: go(dense_mm_narrow_kernel<4, 2>, 4); break;
+        case 3: go(dense_mm_narrow_kernel<4, 3>, 4); break;
+        case 4: go(dense_mm_narrow_kernel<4, 4>, 4); break;
+        case 5: go(dense_mm_narrow_kernel<4, 5>, 4); break;
+        case 6: go(dense_mm_narrow_kernel<4, 6>, 4); break;
+        case 7: go(dense_mm_narrow_kernel<4, 7>, 4); break;
+        default: go(dense_mm_narrow_kernel<8, 4>, 8);
+        }
         return 0;
     }
     if (a.T > 8 && (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g))) return 0;

@@ -222,6 +222,14 @@ def test_dense_matmul_of_a_short_inner_size(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
 
 
+# K a multiple of 128 up to 1024 and few tiles (k_dense.hip dense_mm_narrow_kernel): every number of steps per wave, a row and a column more and less than a tile, as many tiles as CUs and more
+# (the ring), one step more of K (the ring)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,N,K", [(9, 1, 128), (33, 31, 256), (31, 33, 384), (32, 64, 512), (65, 40, 640), (12, 100, 768), (40, 65, 896), (64, 129, 1024), (256, 1024, 512), (257, 1024, 512), (9, 70, 1152)])
+def test_dense_matmul_of_few_tiles(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
 # one token (k_dense.hip dense_mv1_kernel): a row of less than one unit of its stream (512 numbers, fp32: 256), of exactly one, of one and a bit; fewer and more units per wave than are in flight;
 # one row, rows that are no multiple of the waves', more rows than waves and more than 64 of them per wave; the longest row that is taken, and one more, which the general kernel does
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
