@@ -106,7 +106,9 @@ static __device__ __forceinline__ float dn_epi(const dn_args &g, float acc, long
 }
 static __device__ __forceinline__ float dn_silu(float x) { return x / (1.f + expf(-x)); }
 // Result acc of (token t, weight row n) goes to its place.  other: the result of row n ^ 1 (the paired activation needs both; every lane of the wave calls
-// this with both values, only the even row stores).
+// this with both values, only the even row stores).  O16: the wide mat-mul's, whose result may go to g.out16 (the test of it for each of a few tokens' results, beside its arguments, cost the
+// mat-vec of eight tokens 3 to 6 %)
+template <bool O16 = false>
 static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, long long n, float acc, float other, bool in) {
     const float rs = in && g.out_scale ? g.out_scale[t] : 1.f;
     if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR) {
@@ -114,7 +116,7 @@ static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, lon
             float *p = g.out + t * g.ldo + (n >> 1);
             if (g.bias) { acc += g.bias[n]; other += g.bias[n + 1]; }
             const float v = (g.act == PSD_ACT_SILU_PAIR ? dn_silu(acc) : fmaxf(acc, 0.f)) * other * g.alpha * rs;
-            if (g.out16) g.out16[p - g.out] = dn_f2bf(v);
+            if (O16 && g.out16) g.out16[p - g.out] = dn_f2bf(v);
             else *p = g.accum ? *p + v : v;
         }
         return;
@@ -126,7 +128,7 @@ static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, lon
         const long long at = (long long)(g.em_tokens ? g.em_tokens[t] : g.em_step->token0) * g.em_ld + g.em_col + n;
         v *= g.em_bf16 ? dn_bf2f(((const unsigned short *)g.em_table)[at]) : ((const float *)g.em_table)[at];
     }
-    if (g.out16) g.out16[p - g.out] = dn_f2bf(v);
+    if (O16 && g.out16) g.out16[p - g.out] = dn_f2bf(v);
     else *p = g.accum ? *p + v : v;
 }
 // the output row of local row t (t < T): itself, or where the sorted list sends its slot
@@ -516,7 +518,7 @@ static __device__ __forceinline__ void dn_put4r(const dn_args &g, long long row0
         const int t = tb + r;
         const bool in = t < T && nin;
         if (pair || g.em_table) { // (row n ^ 1 is the neighbouring lane's)
-            dn_put(g, dn_orow(g, row0, t, T), n, acc[r], pair ? __shfl_xor(acc[r], 1, 64) : 0.f, in);
+            dn_put<true>(g, dn_orow(g, row0, t, T), n, acc[r], pair ? __shfl_xor(acc[r], 1, 64) : 0.f, in);
             continue;
         }
         if (!in) continue;
@@ -532,7 +534,7 @@ static __device__ __forceinline__ void dn_put4(const dn_args &g, long long t, lo
     if (n >= g.N) return;
     if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR || g.em_table || n + 4 > g.N || g.ldo % 4 || ((uintptr_t)g.out & 15)) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) dn_put(g, t, n + e, acc[e], acc[e ^ 1], n + e < g.N);
+        for (int e = 0; e < 4; e++) dn_put<true>(g, t, n + e, acc[e], acc[e ^ 1], n + e < g.N);
         return;
     }
     float *p = g.out + t * g.ldo + n;
@@ -1296,9 +1298,8 @@ static bool dn_launch_mv2(hipStream_t st, const dn_args &g, const dn_args *g2, i
     return true;
 }
 
-template <typename WT, int C>
+template <typename WT, int C, int RW = 4>
 static void dn_launch_mv(hipStream_t st, const dn_args &g) {
-    constexpr int RW = 4;
     const size_t lds = (size_t)C * ((g.K + 7) / 8 * 8) * 4;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mv_kernel<WT, C, RW>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
@@ -1383,7 +1384,12 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0) : dn_launch_mv1<float, 0>(st, g, nullptr, 0))) return 0;
         const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
         if (kp4 * C <= 64 * 1024) {
-            if (bf) {
+            // (a token's rows that the stream does not take: four per wave would leave at most 64 blocks.  1004 x 4102 14.2 us, with one per wave 11.9; 512 x 1026 6.7 and 5.3)
+            const bool one_row = C == 1 && g.N <= 1024 && g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR;
+            if (one_row) {
+                if (bf) dn_launch_mv<unsigned short, 1, 1>(st, g);
+                else dn_launch_mv<float, 1, 1>(st, g);
+            } else if (bf) {
                 if (C == 1) dn_launch_mv<unsigned short, 1>(st, g);
                 else if (C == 2) dn_launch_mv<unsigned short, 2>(st, g);
                 else if (C == 4) dn_launch_mv<unsigned short, 4>(st, g);
