@@ -1122,10 +1122,14 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
     const int64_t most = lds <= 72 * 1024 ? 512 : 256;
     int64_t grid = std::min<int64_t>((g.N + per - 1) / per, most);
     if (FORM == 1) { // the same number of rows for every work-group of every matrix
-        const int64_t all = g.N * slots + (g2 ? g2->N : 0), rounds = std::max<int64_t>((all + most * per - 1) / (most * per), 1);
-        p.blocks = (int)((g.N + rounds * per - 1) / (rounds * per));
-        p.blocks2 = g2 ? (int)((g2->N + rounds * per - 1) / (rounds * per)) : 0;
-        grid = (int64_t)p.blocks * slots + p.blocks2;
+        const int64_t all = g.N * slots + (g2 ? g2->N : 0);
+        int64_t rounds = std::max<int64_t>((all + most * per - 1) / (most * per), 1);
+        do { // (a round more where the matrices' last ones would add up to a work-group too many)
+            p.blocks = (int)((g.N + rounds * per - 1) / (rounds * per));
+            p.blocks2 = g2 ? (int)((g2->N + rounds * per - 1) / (rounds * per)) : 0;
+            grid = (int64_t)p.blocks * slots + p.blocks2;
+            rounds++;
+        } while (grid > most && (p.blocks > 1 || p.blocks2 > 1));
     }
     if (FORM == 2) {
         const int n = 1 + a->n_more;

@@ -132,7 +132,7 @@ def test_experts_of_a_few_tokens(made, width, experts, top, ff, shared, dtype):
 @pytest.mark.parametrize("width,experts,ff", [(64, 2, 264), (2052, 1, 24), (4104, 1, 8), (64, 5, 1024), (64, 6, 520), (72, 3, 1032), (64, 2, 1016)])
 def test_second_products_on_their_own(made, width, experts, ff, dtype):
     cfg = ZC(width, 40, [ZL("mingru", {"width": 24}, moe=(experts, experts, ff)), ZL("mingru", {"width": 24}, moe=(experts, experts, ff))])
-    m, c, t = made(f"second{width}.{ff}", dtype, cfg=cfg)
+    m, c, t = made(f"second{width}.{experts}.{ff}", dtype, cfg=cfg)
     toks = tokens_for(c, 14)
     want = seq_oracle.run_zusolix(c, t, toks)
     s, got = m.acquire(), []
@@ -140,6 +140,14 @@ def test_second_products_on_their_own(made, width, experts, ff, dtype):
         got.append(m.forward(s, toks[at:at + n], np.arange(n)))
     m.release(s)
     assert err(np.concatenate(got), want) < TOL[dtype]
+
+
+# the experts' first product (k_dense.hip dense_mv1_kernel, FORM 1) where its slots' work-groups, rounded up, would be more than two per CU (48 slots of 1024 rows: 528), so that each takes a
+# round of rows more; and one slot, and as many as it takes to fill the chip once
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,experts,ff", [(64, 6, 512), (64, 1, 520), (40, 8, 256)])
+def test_first_products_of_many_slots(made, width, experts, ff, dtype):
+    test_second_products_on_their_own(made, width, experts, ff, dtype)
 
 
 def test_memory_of_a_wide_shared_expert(ctx, free_bytes, tmp_path):
