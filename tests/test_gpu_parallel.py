@@ -157,6 +157,16 @@ def test_token_by_token_and_portions_give_the_whole_prompts_logits(made, name, d
         assert err(run_portions(m, toks, sizes), want) < TOL[dtype], sizes
 
 
+@pytest.mark.parametrize("sizes", [(17, 33), (31, 64), (65,), (129,)])
+def test_attention_of_a_portion_in_pairs_of_row_tiles(made, sizes):
+    """64 heads: blocks of 32 tokens (k_winattn.hip la_two_tiles) without a distance slope: sink, scaled rotation, pooled rows that end inside a tile (six positions per row) and fill whole
+    ones (one position per row), a window's last keys in the next tile, rings that wrap; 17 and 31 tokens beside them stay with one row tile."""
+    cfg = PC(64, 48, [PL(None, att(64, 16, 16, 20, 37, 6, 8, factor=3.0), gla(1, 8, 8, 2.0)), PL(None, att(64, 32, 32, 16, 50, 1, 32), gla(1, 8, 8, 2.0))], taps=2)
+    m, c, t = made("pairs", max_batch=130, cfg=cfg)
+    toks = tokens_for(c, 260)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run_parallel(c, t, toks)) < TOL["float32"]
+
+
 @pytest.mark.parametrize("sizes", [(31, 33), (32,), (47, 5, 49), (100,)])
 def test_linear_attention_in_chunks(made, sizes):
     """gated linear attention in chunks of 16 tokens (k_chunk.hip), around their edges and beside portions of fewer than 32 tokens (the scan)"""

@@ -103,6 +103,15 @@ def first_layer_adds(m, toks, x0):
     return got
 
 
+@pytest.mark.parametrize("sizes", [(17, 33), (31, 64), (65,), (129,)])
+def test_attention_of_a_portion_in_pairs_of_row_tiles(made, sizes):
+    """64 heads: blocks of 32 tokens (k_winattn.hip la_two_tiles) with a sink and a gate per output element, over all keys before them"""
+    cfg = PC(64, 48, [PL("attention", PA(64, 16, 16, 20, 0.3)), PL("attention", PA(64, 64, 32, 8, 0.2))])
+    m, c, t = made("pairs", max_batch=130, cfg=cfg)
+    toks = tokens_for(c, 260)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run_pokatar(c, t, toks)) < TOL["float32"]
+
+
 # ---------------------------------------------------------------------------------------------------------------- mechanisms, one at a time
 MIXTURES = {"mixture": (6, 2, 14, 2, 4, 2), "mixture_aligned": (6, 3, 64, 2, 2, 1), "mixture_top1": (5, 1, 12, 1, 0, 0)}
 
