@@ -92,6 +92,15 @@ def first_layer_adds(m, toks, x0):
     return got
 
 
+@pytest.mark.parametrize("sizes", [(17, 33), (31, 64), (65,), (129,)])
+def test_attention_of_a_portion_in_pairs_of_row_tiles(made, sizes):
+    """64 heads: blocks of 32 tokens (k_winattn.hip la_two_tiles) with a soft cap and a query temperature that steps inside a tile, over all keys before them"""
+    cfg = ZC(64, 48, [ZL("attention", ZA(64, 16, 16, 20, 0.3, 5.0, (0.4, 7))), ZL("attention", ZA(64, 64, 16, 8, 0.3, 3.0))], residual_mult=0.7)
+    m, c, t = made("pairs", max_batch=130, cfg=cfg)
+    toks = tokens_for(c, 260)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run_zusolix(c, t, toks)) < TOL["float32"]
+
+
 # the router of a few tokens with sixteen waves (k_moe.hip moe_route_kernel): as many rows as waves with the shared gate's, one less and one more; rows of one round of pieces, of a round and four
 # numbers more, and of no multiple of four; eight tokens and nine (four waves)
 @pytest.mark.parametrize("width,experts,shared", [(64, 15, 8), (2052, 16, 8), (66, 16, None), (2048, 17, None), (64, 33, 8)])
@@ -107,23 +116,35 @@ def test_router_of_a_few_tokens(made, width, experts, shared):
     assert err(np.concatenate(got), want) < TOL["float32"]
 
 
-# the experts' second product for a few tokens (k_dense.hip dense_mv2_kernel): rows of one unit or a bit of one (512 numbers, fp32: 256), units of several slots and of the shared expert with one
-# wave, one to eight waves per row, up to 8 (fp32: 16) units per wave and one more (the general kernel), more rows than groups of waves
+def steady_tokens(cfg, t, n):
+    """n tokens on which no choice of a router is a near tie -- the statement's rows stay put when every weight moves by up to 2^-8, twice what rounded activations do to a product -- and the
+    statement's logits for them"""
+    def moved(seed):
+        rng = np.random.default_rng(seed)
+        return {k: v * (1 + rng.uniform(-2.0 ** -8, 2.0 ** -8, np.shape(v))) for k, v in t.items()}
+
+    others = [moved(0), moved(1)]
+    for seed in range(100):
+        toks = tokens_for(cfg, n, seed)
+        want = seq_oracle.run_zusolix(cfg, t, toks)
+        if all(err(seq_oracle.run_zusolix(cfg, o, toks), want) < TOL["bfloat16"] / 4 for o in others):
+            return toks, want
+    raise AssertionError("no steady tokens")
+
+
+# the experts' second product for a few tokens (k_dense.hip dense_mv2_kernel, dense_mv_grouped_kernel): rows of one unit or a bit of one (512 numbers, fp32: 256), units of several slots and of the
+# shared expert with one wave, one to eight waves per row, up to 8 (fp32: 16) units per wave and one more (the general kernel), more rows than groups of waves; every row is held to the tolerance
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,experts,top,ff,shared", [(64, 3, 1, 8, 0), (72, 5, 2, 264, 40), (64, 4, 3, 256, 512), (64, 6, 5, 520, 1032), (80, 8, 8, 2056, 264), (64, 8, 8, 4088, 8), (4104, 3, 2, 16, 8)])
 def test_experts_of_a_few_tokens(made, width, experts, top, ff, shared, dtype):
     cfg = ZC(width, 40, [ZL("attention", ZA(2, 1, 16, 8, 0.3), moe=(experts, top, ff), shared=shared or None), ZL("mingru", {"width": 24}, moe=(experts, top, ff), shared=shared or None)])
     m, c, t = made(f"few{width}.{ff}", dtype, cfg=cfg)
-    toks = tokens_for(c, 14)
-    want = seq_oracle.run_zusolix(c, t, toks)
+    toks, want = steady_tokens(c, t, 14)
     s, got = m.acquire(), []
     for at, n in ((0, 1), (1, 1), (2, 3), (5, 8), (13, 1)):
         got.append(m.forward(s, toks[at:at + n], np.arange(n)))
     m.release(s)
-    # float32: every row.  bfloat16: where two of a router's scores are closer than 8-bit mantissas resolve, a choice may go the other way and that row moves: nine rows in ten, and none
-    # beyond the logits' own spread
-    rows = [err(g[None], w[None]) * np.std(w) / np.std(want) for g, w in zip(np.concatenate(got), want)]
-    assert max(rows) < TOL["float32"] if dtype == "float32" else float(np.quantile(rows, 0.9)) < TOL[dtype] and max(rows) < 1.0
+    assert err(np.concatenate(got), want) < TOL[dtype]
 
 
 # the experts' second product without a shared expert: one, two and four rows per wave of the grouped kernel, one trip of a slot to one short of the six from which the rows in registers take
