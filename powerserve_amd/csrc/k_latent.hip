@@ -383,9 +383,11 @@ __global__ __launch_bounds__(256) void latent_absorbed_kernel(const ps_seq_step 
             if (h0 + 4 * lq + i < H && c < R) *(la_f4 *)(pp + (long long)(4 * lq + i) * (R + 4) + c) = la_f4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
     }
 }
-// ol[h][c] = sum_tiles exp(m_t - M) o_t[c] / sum_tiles exp(m_t - M) l_t: block = 64 columns of a head, each wave a quarter of the tiles
+// ol[h][c] = sum_tiles exp(m_t - M) o_t[c] / sum_tiles exp(m_t - M) l_t: block = 64 columns of a head, each wave a quarter of the tiles.  The weights are kept in LDS for as many tiles as
+// LA_HELD; of a longer window's every wave makes them again where it needs them (LDS for them all ended at a window of 651 000, where the launch aborted).
+#define LA_HELD 16384
 __global__ __launch_bounds__(256) void latent_combine_kernel(const ps_seq_step *step, const float *part, int H, int R, int window, int max_tiles, float *ol) {
-    extern __shared__ float wts[]; // [max_tiles] weights exp(m_t - M)
+    extern __shared__ float wts[]; // [max_tiles] weights exp(m_t - M), where max_tiles <= LA_HELD
     __shared__ float red[8], sum[4][64];
     const int h = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = blockIdx.y * 64 + lane;
     const long long p = step->pos0, lo = p - window + 1 > 0 ? p - window + 1 : 0;
@@ -399,19 +401,26 @@ __global__ __launch_bounds__(256) void latent_combine_kernel(const ps_seq_step *
     if (lane == 0) red[wave] = mx;
     __syncthreads();
     const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const bool held = max_tiles <= LA_HELD;
+    auto weight = [&](int t) {
+        const float m = ph[t * ts + R];
+        return m == -INFINITY ? 0.f : expf(m - M);
+    };
     float ls = 0.f;
     for (int t = tid; t < nt; t += 256) {
-        const float m = ph[t * ts + R], w = m == -INFINITY ? 0.f : expf(m - M);
-        wts[t] = w;
+        const float w = weight(t);
+        if (held) wts[t] = w;
         ls = fmaf(w, ph[t * ts + R + 1], ls);
     }
     ls = la_wave_sum(ls);
     if (lane == 0) red[4 + wave] = ls;
     __syncthreads();
     float a = 0.f;
-    if (c < R) {
+    if (c < R && held) {
 #pragma unroll 8
         for (int t = wave; t < nt; t += 4) a = fmaf(wts[t], ph[t * ts + c], a);
+    } else if (c < R) {
+        for (int t = wave; t < nt; t += 4) a = fmaf(weight(t), ph[t * ts + c], a);
     }
     sum[wave][lane] = a;
     __syncthreads();
@@ -431,7 +440,7 @@ void psk_latent_absorbed(hipStream_t st, const ps_seq_step *step, int64_t ring_o
     else hipLaunchKernelGGL(latent_fold_q_kernel<float>, fold, dim3(256), 0, st, step, q, qstride, (const float *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa);
     const auto attend = R <= 256 ? latent_absorbed_kernel<1> : latent_absorbed_kernel<2>;
     hipLaunchKernelGGL(attend, grid, dim3(256), 0, st, step, (long long)ring_off, cap, qa, dr, H, R, window, scale, part);
-    hipLaunchKernelGGL(latent_combine_kernel, dim3(H, (R + 63) / 64), dim3(256), (size_t)max_tiles * 4, st, step, part, H, R, window, max_tiles, ol);
+    hipLaunchKernelGGL(latent_combine_kernel, dim3(H, (R + 63) / 64), dim3(256), max_tiles <= LA_HELD ? (size_t)max_tiles * 4 : 0, st, step, part, H, R, window, max_tiles, ol);
     const int rows = H * dv;
     if (bf) hipLaunchKernelGGL(latent_unfold_v_kernel<unsigned short>, dim3((rows + 3) / 4), dim3(256), 0, st, ol, (const unsigned short *)ukv->data + (size_t)H * d * R, dv, R, rows, o, gate);
     else hipLaunchKernelGGL(latent_unfold_v_kernel<float>, dim3((rows + 3) / 4), dim3(256), 0, st, ol, (const float *)ukv->data + (size_t)H * d * R, dv, R, rows, o, gate);

@@ -144,6 +144,19 @@ def test_kernels_of_a_single_token(made, width, taps, heads, rank, rot, window):
     assert err(run_portions(m, toks, (1,)), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
+# a single token behind a window of very many keys (k_latent.hip latent_combine_kernel): as many tiles as it keeps the weights of, one more, and more than LDS has room for
+@pytest.mark.parametrize("window", [262_128, 262_129, 652_000])
+def test_latent_attention_of_a_very_long_window(ctx, tmp_path, window):
+    cfg = synth.seq_config(64, 40, [L("latent_attention", None, heads=2, dim=16, vdim=16, q_rank=20, kv_rank=16, mask={"size": window}, scale=0.3, rot={"base": 100.0, "dims": 16}, rot_dim=16)],
+                           taps=2)
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=4, n_slots=1, max_context=700_000)
+    toks = tokens_for(cfg, 100)
+    got = run_portions(m, toks, (1,))
+    m.close()
+    assert err(got, seq_oracle.run(cfg, t, toks)) < TOL["float32"]
+
+
 # the wide mat-mul (k_dense.hip dense_mm_ring_kernel): one row more and less than its tiles of 64 and 128 tokens and outputs, one block of K and fewer blocks than stages,
 # products split along K (few tiles, long K: also uneven shares), more tiles than the chip has CUs
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
