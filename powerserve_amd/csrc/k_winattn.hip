@@ -383,10 +383,12 @@ __global__ __launch_bounds__(256) void winattn_step_kernel(const ps_seq_step *st
         }
     }
 }
-// o[h][c] = gate_h * sum_tiles exp(m_t - M) o_t[c] / (sum_tiles exp(m_t - M) l_t + exp(sink_h - M)),  M = max(max_t m_t, sink_h)
+// o[h][c] = gate_h * sum_tiles exp(m_t - M) o_t[c] / (sum_tiles exp(m_t - M) l_t + exp(sink_h - M)),  M = max(max_t m_t, sink_h).  The weights are kept in LDS
+// for as many tiles as WA_HELD; of more (a context of 655 000 and longer had no room for them, and the launch aborted) they are made again for every column.
+#define WA_HELD 16384
 __global__ __launch_bounds__(256) void winattn_merge_kernel(const ps_seq_step *step, const float *part, const float *gate, const float *sink, int pool, int keep, int H,
                                                             int dv, int window, int max_tiles, float *o, int gate_elem) {
-    extern __shared__ float wts[]; // [max_tiles] weights exp(m_t - M)
+    extern __shared__ float wts[]; // [max_tiles] weights exp(m_t - M), where max_tiles <= WA_HELD
     __shared__ float red[4];
     const int h = blockIdx.x, tid = threadIdx.x, dvp = dv + 4;
     const long long p = step->pos0, lo = p - window + 1 > 0 ? p - window + 1 : 0, nb = wa_front(p, window, pool, keep);
@@ -399,12 +401,16 @@ __global__ __launch_bounds__(256) void winattn_merge_kernel(const ps_seq_step *s
     __syncthreads();
     const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     __syncthreads();
+    const bool held = max_tiles <= WA_HELD;
+    auto weight = [&](int t) {
+        const float m = part[((long long)t * H + h) * dvp + dv];
+        return m == -INFINITY ? 0.f : expf(m - M);
+    };
     float ls = 0.f;
     for (int t = tid; t < nt; t += 256) {
-        const float *pp = part + ((long long)t * H + h) * dvp + dv;
-        const float w = pp[0] == -INFINITY ? 0.f : expf(pp[0] - M);
-        wts[t] = w;
-        ls = fmaf(w, pp[1], ls);
+        const float w = weight(t);
+        if (held) wts[t] = w;
+        ls = fmaf(w, part[((long long)t * H + h) * dvp + dv + 1], ls);
     }
     ls = wa_wave_sum(ls);
     if ((tid & 63) == 0) red[tid >> 6] = ls;
@@ -413,8 +419,12 @@ __global__ __launch_bounds__(256) void winattn_merge_kernel(const ps_seq_step *s
     const float f = (gate && !gate_elem ? wa_sigmoid(gate[h]) : 1.f) / L;
     for (int c = tid; c < dv; c += 256) {
         float a = 0.f;
+        if (held) {
 #pragma unroll 8
-        for (int t = 0; t < nt; t++) a = fmaf(wts[t], part[((long long)t * H + h) * dvp + c], a);
+            for (int t = 0; t < nt; t++) a = fmaf(wts[t], part[((long long)t * H + h) * dvp + c], a);
+        } else {
+            for (int t = 0; t < nt; t++) a = fmaf(weight(t), part[((long long)t * H + h) * dvp + c], a);
+        }
         o[(long long)h * dv + c] = a * f * (gate && gate_elem ? wa_sigmoid(gate[(long long)h * dv + c]) : 1.f);
     }
 }
@@ -441,6 +451,6 @@ void psk_winattn_step(hipStream_t st, const ps_seq_step *step, int64_t ring_off,
     const auto kernel = slope ? winattn_step_kernel<8, true> : winattn_step_kernel<8, false>;
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, step, (long long)ring_off, cap, (long long)fs.off, fs.pool, fs.keep, q, temp, H, G, d, dv, window, scale, scratch,
                        softcap, slope);
-    hipLaunchKernelGGL(winattn_merge_kernel, dim3(H), dim3(256), (size_t)grid.x * 4 * 4, st, step, scratch, gate, sink, fs.pool, fs.keep, H, dv, window, (int)grid.x * 4, o,
+    hipLaunchKernelGGL(winattn_merge_kernel, dim3(H), dim3(256), grid.x * 4 <= WA_HELD ? (size_t)grid.x * 4 * 4 : 0, st, step, scratch, gate, sink, fs.pool, fs.keep, H, dv, window, (int)grid.x * 4, o,
                        gate_elem);
 }

@@ -116,6 +116,18 @@ def test_attention_of_a_portion_in_pairs_of_row_tiles(made, sizes):
 MIXTURES = {"mixture": (6, 2, 14, 2, 4, 2), "mixture_aligned": (6, 3, 64, 2, 2, 1), "mixture_top1": (5, 1, 12, 1, 0, 0)}
 
 
+# a single token in a context of very many (k_winattn.hip winattn_merge_kernel): as many tiles as it keeps the weights of, some more, and more than LDS has room for
+@pytest.mark.parametrize("context", [262_096, 262_144, 700_000])
+def test_attention_in_a_very_long_context(ctx, tmp_path, context):
+    cfg = PC(64, 40, [PL("attention", PA(2, 1, 16, 16, 0.3), ff=32)])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=4, n_slots=1, max_context=context)
+    toks = tokens_for(cfg, 100)
+    got = run_portions(m, toks, (1,))
+    m.close()
+    assert err(got, seq_oracle.run_pokatar(cfg, t, toks)) < TOL["float32"]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("which", ["attention", "attention_mfma", "latent", "latent_mfma", "dense", "mixture", "mixture_aligned", "mixture_top1"])
 def test_each_mechanism_alone(made, which, dtype):
