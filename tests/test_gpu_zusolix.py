@@ -163,6 +163,33 @@ def test_second_products_on_their_own(made, width, experts, ff, dtype):
     assert err(np.concatenate(got), want) < TOL[dtype]
 
 
+# an infinite weight where a row's last unit begins, which the lanes behind the row's end may be tempted to read: it stays infinite in its own output and touches no other, with the shared
+# expert in the same launch and without one
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("experts,ff,shared", [(2, 264, 40), (2, 24, 1032), (6, 520, 0)])
+def test_experts_with_an_infinite_weight(made, experts, ff, shared, dtype):
+    cfg = ZC(64, 40, [ZL("mingru", {"width": 24}, moe=(experts, experts, ff), shared=shared or None)])
+    t = bf16(synth.seq_tensors(cfg, 3))
+    unit = 512 if dtype == "bfloat16" else 256
+    places = [("l0.mlp.e1.down", 3, (ff - 1) // unit * unit)] + ([("l0.mlp.shared.down", 5, (shared - 1) // unit * unit)] if shared else [])
+    for name, n, k in places:
+        t[name][n, k] = 0.0
+    toks, per = tokens_for(cfg, 1), []
+    seq_oracle.run_zusolix(cfg, t, toks, per_layer=per)
+    for name, n, k in places:
+        t[name][n, k] = np.inf
+    m, _, _ = made(f"infinite{ff}", dtype, cfg=cfg, tensors=t)
+    m.capture_layers(True)
+    s = m.acquire()
+    m.forward(s, toks)
+    got = m.layers(1)[0][0]
+    m.release(s)
+    m.capture_layers(False)
+    hit = [n for _, n, _ in places]
+    assert np.all(np.isinf(got[hit]))
+    assert np.abs(np.delete(got, hit) - np.delete(per[0][0], hit)).max() < TOL[dtype] * np.abs(per[0]).max()
+
+
 # the experts' first product (k_dense.hip dense_mv1_kernel, FORM 1) where its slots' work-groups, rounded up, would be more than two per CU (48 slots of 1024 rows: 528), so that each takes a
 # round of rows more; and one slot, and as many as it takes to fill the chip once
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
