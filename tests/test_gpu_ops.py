@@ -103,6 +103,30 @@ def test_mul_mat_batched(ctx, oracle, hip, wt, K, N, bs):
     W.free()
 
 
+@pytest.mark.parametrize("wt", [8, 2])
+@pytest.mark.parametrize("K,N,bs", [(128, 8, 2), (128, 24, 17), (256, 4100, 16), (896, 1000, 33), (256, 9000, 64), (128, 16392, 61), (128, 16392, 90), (640, 8200, 97), (384, 4104, 512)])
+def test_mul_mat_batched_blocks(ctx, oracle, hip, wt, K, N, bs):
+    """The four forms of the Q8_0 / Q4_0 batched mat-mul (one or two column tiles per wave, two to eight waves), each with a ragged last row tile (an odd number of
+    Q8_0 row groups among them), ragged columns and odd numbers of stages; block scales of every kind (negative, zero, fp16 denormals: their products round once)."""
+    from powerserve_amd import synth
+    rng = np.random.default_rng(K + N + bs + wt)
+    w = synth.random_blocks(rng, wt, N, K)
+    raw = np.ascontiguousarray(w).reshape(-1, {8: 34, 2: 18}[wt])
+    for k, h in enumerate((0x0001, 0x83FF, 0x8000, 0x0000, 0xB555, 0x0200)):
+        raw[k::29, 0], raw[k::29, 1] = h & 0xFF, h >> 8
+    w = raw.reshape(np.asarray(w).shape)
+    x = rng.standard_normal((bs, K)).astype(np.float32)
+    x[0] *= 1e-38
+    x[1, :32] = 0.0
+    want = oracle.mul_mat(wt, w, K, N, x)
+    W = ctx.upload_weight(wt, w, K, N)
+    dx, dy = ctx.to_device(x), ctx.empty((bs, N))
+    ctx.check(ctx.L.ps_hip_mul_mat(ctx.h, C.byref(dy.tensor()), C.byref(W.tensor()), C.byref(dx.tensor())))
+    got = dy.numpy()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rel_err(got, want), np.flatnonzero(got != want)[:8])
+    W.free()
+
+
 @pytest.mark.parametrize("K,N,bs", [(4096, 512, 128), (1024, 96, 120), (14336, 64, 113), (2048, 288, 128), (1024, 64, 160), (2048, 96, 200), (1024, 8224, 70), (1024, 32, 12), (4096, 160, 2), (2048, 8224, 16), (1024, 64, 5)])
 def test_mul_mat_q4k_chunk_on_matrix_cores(ctx, oracle, hip, K, N, bs):
     """Batches of a Q4_K weight from 2 columns (N % 32 == 0, K % 1024 == 0) take k_gemm4k.hip (17 and more: the wide kernel, fewer: the narrow one): fp16 MFMA contractions of
