@@ -1,4 +1,5 @@
-// Q4_K batched mat-mul (prefill chunks, tree verify) on v_mfma_f32_16x16x32_f16 -- bit-exact with ggml_vec_dot_q4_K_q8_K.
+// Q4_K batched mat-mul (tree verify, and prefill chunks whose row and column tiles are too few for k_gemm4f.hip: psk_gemm4f's rule) on v_mfma_f32_16x16x32_f16 --
+// bit-exact with ggml_vec_dot_q4_K_q8_K.
 //
 // The AVX2 kernel (libs/ggml/src/ggml-quants.c:7809-7873) keeps, per super-block of 256 weights, ONE int32 per accumulator
 // lane u:  sumi[u] = sum over the 8 sub-blocks g of  scale[g] * dot4(q[g][4u..4u+3], y[g][4u..4u+3]),  accumulated in

@@ -879,7 +879,8 @@ int psk_gemm8(hipStream_t st, int n_cu, const psk_gemv_args &a, ps_act act, int6
     if (a.pro != 0 || a.n_w < 1) return -1;
     if (a.rope && !(a.w[0]->dtype == PS_Q4_K && bs >= 2)) return -1;
     if (a.w[0]->dtype == PS_Q4_K) { // prefill chunks: fp16 matrix cores on exact integers, producer / consumer waves (k_gemm4k.hip)
-        const int rc = psk_gemm4k(st, n_cu, a, act, K, bs);
+        int rc = psk_gemm4f(st, n_cu, a, act, K, bs);
+        if (rc == -1) rc = psk_gemm4k(st, n_cu, a, act, K, bs);
         if (rc != -1) return rc;
     }
     if (a.rope) return 3; // (a batch with the RoPE epilogue requested that the chunk mat-mul did not take: psk_gemm4k_rope_ok and psk_gemm4k disagree)

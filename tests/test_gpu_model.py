@@ -251,6 +251,28 @@ def test_real_layer_shapes_match_oracle(ctx, oracle, tmp_path, preset, wt, P):
     om.close()
 
 
+@pytest.mark.parametrize("n", [20, 45, 100])
+def test_short_prompts_at_real_layer_shapes(ctx, oracle, tmp_path, n):
+    """One forward of a few tokens at Llama-3.1-8B's layer dimensions (Q4_K): the gate / up pair, Q / K / V side by side and the residual epilogues of gemm4f_kernel with two and
+    with three column tiles per wave; every token's logits and the cache rows bit for bit the oracle's."""
+    from oracle import binding as B
+    from powerserve_amd import hip, synth
+    d = str(tmp_path / "m")
+    mj = synth.write_model_dir(d, "llama-8b-dims-4l", 12, n_ctx=256, seed=5)
+    cfg = B.make_config(mj["llm_config"])
+    om = oracle.model(cfg, mj["model_arch"], load_tensors(os.path.join(d, "ggml/weights.gguf")), n_threads=min(32, os.cpu_count() or 8))
+    gm = hip.Model(ctx, d, max_batch=128, n_ctx=256)
+    toks = np.random.default_rng(n).integers(0, cfg.vocab_size, n)
+    want = om.forward(toks, np.arange(n), True)
+    got, _ = gm.forward(toks, np.arange(n), lm_head=True)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), rel_err(got, want)
+    for L in range(cfg.n_layers):
+        assert np.array_equal(gm.k_cache(L)[:n].view(np.uint32), om.k_cache(L)[:n].view(np.uint32)), L
+        assert np.array_equal(gm.v_cache(L)[:, :n].view(np.uint32), om.v_cache(L)[:, :n].view(np.uint32)), L
+    gm.close()
+    om.close()
+
+
 def test_tree_mask_plumbing(ctx, tmp_path):
     """The batch forward takes an optional [bs][bs] tree mask (speculative verify; the reference's CPU
     executor ignores mask objects, executor.cpp:210-224, so there is no CPU golden for a real tree).  A tree mask that

@@ -146,6 +146,28 @@ def test_mul_mat_q4k_chunk_on_matrix_cores(ctx, oracle, hip, K, N, bs):
     W.free()
 
 
+@pytest.mark.parametrize("K,N,bs,kernel", [(1024, 16400, 32, "gemm4f_kernel<0, 2>"), (1024, 16416, 33, "gemm4f_kernel<0, 3>"), (2048, 8224, 97, "gemm4f_kernel<0, 3>"),
+                                           (3072, 4128, 190, "gemm4f_kernel<0, 2>"), (1024, 4112, 512, "gemm4f_kernel<0, 3>"), (1024, 12288, 250, "gemm4f_kernel<0, 2>"), (4096, 8208, 81, "gemm4f_kernel<0, 2>")])
+def test_mul_mat_q4k_columns_shared_by_eight_tiles(ctx, oracle, hip, K, N, bs, kernel):
+    """gemm4f_kernel: two and three column tiles per wave, one and several items per work-group, row blocks with one to eight live tiles, ragged columns; scales and mins at
+    their ends, subnormal block scales and activations (products that round once, in fp32's subnormal range)."""
+    from powerserve_amd import synth
+    rng = np.random.default_rng(K + N + bs)
+    w = q4k_extreme_blocks(rng, N, K) if K == 4096 else synth.random_blocks(rng, 12, N, K)
+    x = (rng.standard_normal((bs, K)) * rng.uniform(0.1, 30.0, (bs, 1))).astype(np.float32)
+    x[0] *= 1e-35 / np.abs(x[0]).max()
+    x[bs - 1, 256:512] = 0.0
+    want = oracle.mul_mat(12, w, K, N, x)
+    W = ctx.upload_weight(12, w, K, N)
+    dx, dy = ctx.to_device(x), ctx.empty((bs, N))
+    for _ in range(2):
+        ctx.check(ctx.L.ps_hip_mul_mat(ctx.h, C.byref(dy.tensor()), C.byref(W.tensor()), C.byref(dx.tensor())))
+        assert ctx.L.ps_hip_last_matmul_kernel().decode() == kernel
+        got = dy.numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rel_err(got, want), np.argwhere(got != want)[:8])
+    W.free()
+
+
 @pytest.mark.parametrize("cfg,kernel", [(8, "gemm4k_par_kernel<8>"), (4, "gemm4k_par_kernel<4>"), (0, None)])
 @pytest.mark.parametrize("K,N,bs", [(14336, 64, 12), (4096, 96, 16), (2048, 32, 3), (1024, 64, 5), (3072, 32, 9), (11264, 32, 2)])
 def test_mul_mat_q4k_narrow_batch_few_tiles(ctx, oracle, hip, K, N, bs, cfg, kernel):
