@@ -1,6 +1,7 @@
 // C-ABI (include/ps_hip.h): context, device memory, stream and events -- the part of the library every model family sits on.
 #include "ps_internal.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -56,7 +57,71 @@ hipError_t ps_dev_free(void *p) {
     return hipSuccess;
 }
 
-
+// ------------------------------------------------------------------ small data in, results out (ps_internal.h)
+namespace {
+template <int W> struct PutArgs { unsigned char *dst[4]; unsigned bytes[4]; uint32_t v[W]; }; // the pieces' words one behind the other
+template <int W>
+__global__ void put_kernel(const PutArgs<W> a) {
+    for (unsigned i = threadIdx.x; i < W; i += blockDim.x) {
+        unsigned w = i;
+        int s = 0;
+        while (s < 4 && w >= (a.bytes[s] + 3) / 4) w -= (a.bytes[s++] + 3) / 4;
+        if (s == 4) return;
+        if (w * 4 + 4 <= a.bytes[s]) ((uint32_t *)a.dst[s])[w] = a.v[i];
+        else for (unsigned b = w * 4; b < a.bytes[s]; b++) a.dst[s][b] = (unsigned char)(a.v[i] >> (b % 4 * 8));
+    }
+}
+template <int W>
+void put_launch(hipStream_t st, const ps_piece *p, int n) { // n <= 4 pieces of at most W words in all
+    PutArgs<W> a{};
+    size_t at = 0;
+    for (int i = 0; i < n; i++) {
+        a.dst[i] = (unsigned char *)p[i].dst;
+        a.bytes[i] = (unsigned)p[i].bytes;
+        memcpy(a.v + at, p[i].src, p[i].bytes);
+        at += (p[i].bytes + 3) / 4;
+    }
+    hipLaunchKernelGGL(put_kernel<W>, dim3(1), dim3(W < 256 ? 64 : 256), 0, st, a);
+}
+__global__ __launch_bounds__(256) void pin_copy_kernel(const char *src, char *dst, size_t bytes) {
+    const bool wide = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
+    const size_t n16 = wide ? bytes / 16 : 0, step = (size_t)gridDim.x * blockDim.x, t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (size_t i = t; i < n16; i += step) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
+    for (size_t i = n16 * 4 + t; i < bytes / 4; i += step) ((uint32_t *)dst)[i] = ((const uint32_t *)src)[i];
+}
+} // namespace
+void ps_put(hipStream_t st, const ps_piece *p, int n) {
+    constexpr size_t CAP = 896;
+    ps_piece q[4];
+    int k = 0;
+    size_t words = 0;
+    auto flush = [&]() {
+        if (k && words <= 32) put_launch<32>(st, q, k);
+        else if (k) put_launch<CAP>(st, q, k);
+        k = 0; words = 0;
+    };
+    for (int i = 0; i < n; i++) {
+        for (size_t done = 0; done < p[i].bytes;) {
+            const size_t b = std::min(p[i].bytes - done, (CAP - words) * 4);
+            q[k++] = ps_piece{(char *)p[i].dst + done, (const char *)p[i].src + done, b};
+            words += (b + 3) / 4;
+            done += b;
+            if (k == 4 || words == CAP) flush();
+        }
+    }
+    flush();
+}
+bool ps_pin_ready(ps_hip_ctx *c) {
+    if (c->pin) return true;
+    for (auto &e : c->pin_ev)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return false; }
+    if (hipHostMalloc((void **)&c->pin, 2 * PS_PIN_HALF, hipHostMallocDefault) != hipSuccess) { c->pin = nullptr; (void)hipGetLastError(); return false; }
+    return true;
+}
+void ps_pin_copy(ps_hip_ctx *c, int half, size_t at, const void *dev, size_t bytes) {
+    const unsigned blocks = (unsigned)std::min<size_t>((bytes + 4095) / 4096, 256);
+    hipLaunchKernelGGL(pin_copy_kernel, dim3(blocks), dim3(256), 0, c->stream, (const char *)dev, c->pin + half * PS_PIN_HALF + at, bytes);
+}
 
 extern "C" {
 
@@ -91,6 +156,8 @@ void ps_hip_destroy(ps_hip_ctx *c) {
     if (c->i32_buf) (void)ps_dev_free(c->i32_buf);
     if (c->u8_buf) (void)ps_dev_free(c->u8_buf);
     if (c->rope_buf) (void)ps_dev_free(c->rope_buf);
+    if (c->pin) (void)hipHostFree(c->pin);
+    for (auto e : c->pin_ev) if (e) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -120,6 +187,12 @@ int ps_hip_memcpy_h2d(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {
     return 0;
 }
 int ps_hip_memcpy_d2h(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {
+    if (bytes && bytes % 4 == 0 && bytes <= 2 * PS_PIN_HALF && ((uintptr_t)src & 3) == 0 && ps_pin_ready(c)) { // (halves are neighbours)
+        ps_pin_copy(c, 0, 0, src, bytes);
+        PS_CHECK(c, hipStreamSynchronize(c->stream));
+        memcpy(dst, c->pin, bytes);
+        return 0;
+    }
     PS_CHECK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
     PS_CHECK(c, hipStreamSynchronize(c->stream));
     return 0;

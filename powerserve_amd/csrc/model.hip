@@ -669,11 +669,9 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
         hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, pos[0], n, 0);
         m->pin_busy = true;
     } else {
-        PS_CHECK(c, hipMemcpyAsync(m->tokens_dev, tokens, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
-        if (tree) PS_CHECK(c, hipMemcpyAsync(m->tree_dev, tree, (size_t)n * n, hipMemcpyHostToDevice, c->stream));
+        const ps_piece in[2] = {{m->tokens_dev, tokens, (size_t)n * 4}, {m->tree_dev, tree, (size_t)n * n}};
+        ps_put(c->stream, in, tree ? 2 : 1);
         hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, pos[0], n, 0);
-        PS_CHECK(c, hipStreamSynchronize(c->stream)); // tokens/tree may be host temporaries
-        m->pin_busy = false; m->pin_argmax_pending = false;
     }
     // A single token through this entry (ModelTokenIterator::decode over the op API, HIPBackend::plan's lowered graph) replays
     // a captured launch plan like ps_hip_model_decode_greedy does: the first call at a position range runs eagerly and captures.
@@ -741,7 +739,8 @@ int ps_hip_model_prefill(ps_hip_model *m, const int32_t *tokens, int n, int chun
     bool retried = false;
     for (int done = 0; done < n;) {
         const int ns = n - done < per * chunk ? n - done : per * chunk;
-        PS_CHECK(c, hipMemcpyAsync(m->tokens_dev, tokens + done, (size_t)ns * 4, hipMemcpyHostToDevice, c->stream));
+        const ps_piece in = {m->tokens_dev, tokens + done, (size_t)ns * 4};
+        ps_put(c->stream, &in, 1);
         hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, ns, 0);
         hipLaunchKernelGGL(set_sub_states_kernel, dim3(1), dim3(64), 0, c->stream, m->state_sub, (int)m->position, chunk, ns);
         m->n_kv_host = (int)m->position + ns;
@@ -750,7 +749,7 @@ int ps_hip_model_prefill(ps_hip_model *m, const int32_t *tokens, int n, int chun
         m->attn_chunk = 0; m->n_kv_host = 0;
         if (rc) return rc;
         if (ns == 1) note_single_token(m);
-        PS_CHECK(c, hipStreamSynchronize(c->stream));
+        if (ns == 1 || done + ns == n) PS_CHECK(c, hipStreamSynchronize(c->stream)); // (the host has nothing to look at in between)
         if (const int rc = check_attn_timeout(m, "model_prefill")) { // a one-token tail: once more, with the two launches
             if (rc != PS_HIP_ATTN_TIMEOUT || retried) return rc;
             retried = true; c->err.clear(); continue;
@@ -780,18 +779,19 @@ static int forward_tree_impl(ps_hip_model *m, const int32_t *tokens, int n, cons
     }
     PS_CHECK(c, hipSetDevice(c->device));
     m->pin_argmax_n = 0;
-    PS_CHECK(c, hipMemcpyAsync(m->tokens_dev, tokens, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
-    PS_CHECK(c, hipMemcpyAsync(m->rope_pos_dev, rope_pos, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
-    if (tree) PS_CHECK(c, hipMemcpyAsync(m->tree_dev, tree, (size_t)n * n, hipMemcpyHostToDevice, c->stream));
+    const ps_piece in[3] = {{m->tokens_dev, tokens, (size_t)n * 4}, {m->rope_pos_dev, rope_pos, (size_t)n * 4}, {m->tree_dev, tree, (size_t)n * n}};
+    ps_put(c->stream, in, tree ? 3 : 2);
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, n, 0);
-    PS_CHECK(c, hipStreamSynchronize(c->stream));
     m->n_kv_host = (int)m->position + n;
     const int rc_fw = enqueue_forward(m, n, lm_head != 0, tree != nullptr, false, true);
     m->n_kv_host = 0;
     if (rc_fw) return rc_fw;
     if (n == 1 && !tree) note_single_token(m);
-    if (lm_head && argmax_host) PS_CHECK(c, hipMemcpyAsync(argmax_host, m->argmax_dev, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
+    const bool pinned = lm_head && argmax_host && (size_t)n * 4 <= PS_PIN_HALF && ps_pin_ready(c);
+    if (pinned) ps_pin_copy(c, 0, 0, m->argmax_dev, (size_t)n * 4);
+    else if (lm_head && argmax_host) PS_CHECK(c, hipMemcpyAsync(argmax_host, m->argmax_dev, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
     PS_CHECK(c, hipStreamSynchronize(c->stream));
+    if (pinned) memcpy(argmax_host, c->pin, (size_t)n * 4);
     if (const int rc = check_attn_timeout(m, "model_forward_tree")) {
         if (rc != PS_HIP_ATTN_TIMEOUT || retried) return rc;
         c->err.clear();
@@ -824,9 +824,9 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     if (token < 0 || (uint32_t)token >= m->cfg.vocab_size) PS_FAIL(c, "decode_greedy: token id out of range");
     PS_CHECK(c, hipSetDevice(c->device));
     m->pin_argmax_n = 0;
-    PS_CHECK(c, hipMemcpyAsync(m->tokens_dev, &token, 4, hipMemcpyHostToDevice, c->stream));
+    const ps_piece in = {m->tokens_dev, &token, 4};
+    ps_put(c->stream, &in, 1);
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, 1, 0);
-    PS_CHECK(c, hipStreamSynchronize(c->stream));
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
     // is not far behind (a stale hint costs time, never results)

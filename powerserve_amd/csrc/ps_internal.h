@@ -28,7 +28,20 @@ struct ps_hip_ctx {
     size_t u8_cap = 0;
     float *rope_buf = nullptr;
     size_t rope_cap = 0;
+    // results on their way to pageable memory: two halves of pinned memory, an event behind what was last put into each
+    char *pin = nullptr;
+    hipEvent_t pin_ev[2] = {nullptr, nullptr};
 };
+// Host bytes into device memory in stream order, as kernel arguments (pieces of at most 3.5 KB a launch): the host's buffers are free on return and nobody waits for the stream.
+// Destinations are multiples of four bytes.  (A copy from pageable memory is staged by the runtime and wants a synchronize behind it where the source is a temporary: 10 - 25 us
+// in front of a request, measured, against 3.)
+struct ps_piece { void *dst; const void *src; size_t bytes; };
+void ps_put(hipStream_t st, const ps_piece *p, int n);
+// Device results through pinned memory: ps_pin_copy enqueues a kernel that writes `bytes` (a multiple of four, from a multiple of four) to c->pin + half * PS_PIN_HALF + at; who
+// reads them waits for the stream, or for an event of c->pin_ev recorded behind it, and is done with them before its call returns.  ps_pin_ready: whether there is pinned memory.
+constexpr size_t PS_PIN_HALF = (size_t)2 << 20;
+bool ps_pin_ready(ps_hip_ctx *c);
+void ps_pin_copy(ps_hip_ctx *c, int half, size_t at, const void *dev, size_t bytes);
 
 // Device layout of a quantized weight matrix [K, N]: a LANE-MAJOR repack of the GGUF blocks, private to the
 // backend (every GGUF byte appears exactly once; zero padding only in a partial last row group / unit).

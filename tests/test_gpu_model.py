@@ -273,6 +273,34 @@ def test_short_prompts_at_real_layer_shapes(ctx, oracle, tmp_path, n):
     om.close()
 
 
+@pytest.mark.parametrize("words", [1, 3, 4097, (2 << 18) + 1, 1 << 20, (1 << 20) + 1])
+def test_results_through_pinned_memory(ctx, words):
+    """Copies to the host of one word, of odd lengths and on both sides of what the pinned memory holds, from an aligned and from a shifted address."""
+    a = np.random.default_rng(words).integers(0, 2 ** 31, words + 1).astype(np.int32)
+    d = ctx.to_device(a)
+    for shift in (0, 1):
+        out = np.zeros(words, dtype=np.int32)
+        ctx.check(ctx.L.ps_hip_memcpy_d2h(ctx.h, out.ctypes.data, d.ptr + 4 * shift, out.nbytes))
+        assert np.array_equal(out, a[shift:shift + words])
+
+
+@pytest.mark.parametrize("n", [32, 33, 895, 896, 897, 1024])
+def test_token_ids_as_kernel_arguments(ctx, tmp_path, n):
+    """Portions whose ids fit the small launch, fill the large one and need a second: the same cache as 8 ids at a time."""
+    from powerserve_amd import hip, synth
+    d = str(tmp_path / "m")
+    synth.write_model_dir(d, "tiny-llama", 8, n_ctx=1024, seed=2)
+    toks = np.random.default_rng(n).integers(0, 512, n)
+    caches = []
+    for mb in (1024, 8):
+        gm = hip.Model(ctx, d, max_batch=mb, n_ctx=1024)
+        gm.prefill(toks, 8)
+        caches.append([(gm.k_cache(L)[:n].copy(), gm.v_cache(L)[:, :n].copy()) for L in range(2)])
+        gm.close()
+    for (k0, v0), (k1, v1) in zip(*caches):
+        assert np.array_equal(k0.view(np.uint32), k1.view(np.uint32)) and np.array_equal(v0.view(np.uint32), v1.view(np.uint32))
+
+
 def test_tree_mask_plumbing(ctx, tmp_path):
     """The batch forward takes an optional [bs][bs] tree mask (speculative verify; the reference's CPU
     executor ignores mask objects, executor.cpp:210-224, so there is no CPU golden for a real tree).  A tree mask that
