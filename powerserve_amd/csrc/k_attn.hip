@@ -1027,71 +1027,56 @@ __global__ __launch_bounds__(512, 1) void attn_pv_mfma_kernel(psl_attn_args a) {
 
 // The same contraction with its operands staged through LDS (head sizes 128 and 64).  The kernel above has every lane
 // fetch its own 128-B run of V and of p as eight 16-B loads: a wave instruction touches 64 cache lines for 1 KiB, and the
-// CU's address unit, not the matrix core, sets the time (86 us at n_kv = 2048).  Here a wave fetches the 16 x 128 block of
-// its V rows with eight row-coalesced instructions (two 512-B rows each), the workgroup fetches the 16 x 128 block of
-// probabilities once for all its waves, both are parked in LDS (rows of 128 floats whose 16-byte column index is XOR-ed with row & 7:
-// one pass for the operand reads' real lane groups, see attn_scores_mfma_kernel; rows padded to 132 floats took two) one 128-position
-// step ahead, and positions past the last full block of 32 are parked as zeros.
+// CU's address unit, not the matrix core, sets the time (86 us at n_kv = 2048).  Here a wave asks for the 16 x 128 block of
+// its V rows with eight row-coalesced instructions (two 512-B rows each) and for its share of the workgroup's 16 x 128 block of
+// probabilities, one 128-position step ahead, straight into LDS (global_load_lds_dwordx4; rows of 128 floats whose 16-byte column index is XOR-ed with row & 7:
+// one pass for the operand reads' real lane groups, see attn_scores_mfma_kernel; rows padded to 132 floats took two).  A step of 128 positions takes 1.5 us, 0.85 of them matrix
+// instructions; through registers and with the kv heads' values in all eight L2s it took 1.7 (22.4 -> 19.3 us on average over a prompt of 2048 in chunks of 128).  Operands read a half
+// step ahead, or requested two steps ahead with a second barrier: the same.
 constexpr int PVM_RS = 128;
 __device__ __forceinline__ size_t pvm_at(const int row, const int seg) { return (size_t)row * PVM_RS + ((seg ^ (row & 7)) << 2); } // float index of 16-byte column seg
+__device__ __forceinline__ void pvm_dma(const char *src, const unsigned lds_dst) { // one wave-instruction: lane l's 16 bytes at src go to lds_dst + 16 l
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds_dst) : "memory");
+}
 template <int NW> // waves per workgroup = head_size / 16
 __global__ __launch_bounds__(NW * 64, 1) void attn_pv_mfma_lds_kernel(psl_attn_args a) {
     extern __shared__ __attribute__((aligned(16))) float pvs[]; // [2][(NW + 1) * 16][PVM_RS]: the waves' V rows, then the 16 probability rows
-    constexpr int hs = NW * 16, NT = NW * 64, ROWS = (NW + 1) * 16, NPS = 512 / NT; // NPS: probability segments per thread
+    constexpr int hs = NW * 16, ROWS = (NW + 1) * 16, NPW = 8 / NW; // NPW: pairs of probability rows per wave
     const int dim = a.n_heads * hs, r2 = a.n_heads / a.n_kv_heads;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kvh = blockIdx.y, bs = att_bs(a), n_kv = att_pos0(a) + bs, np = n_kv & ~31, nblk = np >> 5, n_it = (nblk + 3) >> 2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // work-groups are dealt to the eight XCDs in turn (x fastest): numbered so that an XCD has neighbouring ones, a kv head's values are read through one L2, not through all
+    const unsigned gx = gridDim.x, n_wg = gx * gridDim.y, L = blockIdx.x + gx * blockIdx.y, xcd = L & 7, wg = xcd * (n_wg >> 3) + min(xcd, n_wg & 7) + (L >> 3);
+    const int bx = (int)(wg % gx), kvh = (int)(wg / gx), bs = att_bs(a), n_kv = att_pos0(a) + bs, np = n_kv & ~31, nblk = np >> 5, n_it = (nblk + 3) >> 2;
     const int rl = lane & 15, m = lane >> 4;
-    const int N = bs * r2, n = min((int)blockIdx.x * 16 + rl, N - 1), i = n / r2, g = n - i * r2;
+    const int N = bs * r2, n = min(bx * 16 + rl, N - 1), i = n / r2, g = n - i * r2;
     const int d0 = wave * 16;
-    // staging roles.  V: instruction k covers rows 2k, 2k + 1 of the wave's 16, 32 lanes x 16 B per row
+    // what a wave asks for per step, one instruction each: rows 2k, 2k + 1 of its 16 V rows (32 lanes x 16 B per row), and its share of the probability rows.  Lane seg of row r lands in
+    // 16-byte slot seg, so it fetches the piece that the swizzle puts there.  A piece past np re-reads the ROW's first 16 bytes: with its own column index it would leave the row -- and, in the
+    // last row of a context window of fewer than 128 slots, the allocation -- and its block of 32 is not multiplied.
     const int vrow = lane >> 5, seg = lane & 31;
-    const float *vg = a.v_cache + ((int64_t)kvh * hs + d0 + vrow) * a.n_ctx; // (the row; the lane's 16-byte segment is added where it is known to exist)
-    const float *pg[NPS];
-    int prow[NPS];
+    const char *vg = (const char *)(a.v_cache + (int64_t)kvh * hs * a.n_ctx), *pg[NPW];
 #pragma unroll
-    for (int k = 0; k < NPS; k++) {
-        const int sidx = (int)threadIdx.x + k * NT; // segment sidx: row sidx >> 5, 16-B segment sidx & 31
-        prow[k] = sidx >> 5;
-        const int nn = min((int)blockIdx.x * 16 + prow[k], N - 1), ii = nn / r2, gg = nn - ii * r2;
-        pg[k] = a.scores + ((int64_t)ii * a.n_heads + (int64_t)kvh * r2 + gg) * a.n_ctx;
+    for (int k = 0; k < NPW; k++) {
+        const int nn = min(bx * 16 + 2 * (wave * NPW + k) + vrow, N - 1), ii = nn / r2, gg = nn - ii * r2;
+        pg[k] = (const char *)(a.scores + ((int64_t)ii * a.n_heads + (int64_t)kvh * r2 + gg) * a.n_ctx);
     }
-    float4 sv[8], sp[NPS];
-    auto fetch = [&](int it) { // (clamped, never branched over: positions past np are zeroed when they are parked.  A segment past np re-reads the ROW's
-        // first 16 bytes: with its own column index it left the row -- and, in the last row of a context window of fewer than 128 slots, the allocation)
-        const int p0 = it * 128, off = p0 + seg * 4 < np ? p0 + seg * 4 : 0;
-#pragma unroll
-        for (int k = 0; k < 8; k++) sv[k] = *(const float4 *)(vg + (int64_t)(2 * k) * a.n_ctx + off);
-#pragma unroll
-        for (int k = 0; k < NPS; k++) {
-            const int sg = ((int)threadIdx.x + k * NT) & 31;
-            sp[k] = *(const float4 *)(pg[k] + (p0 + sg * 4 < np ? p0 + sg * 4 : 0));
-        }
-    };
-    auto park = [&](int it, float *buf) {
-        const int p0 = it * 128;
-        const bool vin = p0 + seg * 4 < np;
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-            *(float4 *)(buf + pvm_at(d0 + 2 * k + vrow, seg)) = vin ? sv[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int k = 0; k < NPS; k++) {
-            const int sg = ((int)threadIdx.x + k * NT) & 31;
-            *(float4 *)(buf + pvm_at(NW * 16 + prow[k], sg)) = p0 + sg * 4 < np ? sp[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+    const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)pvs;
+    auto request = [&](const int it, const int k) { // piece k of step it
+        const int row = k < 8 ? d0 + 2 * k : NW * 16 + 2 * (wave * NPW + k - 8), off = it * 512 + ((seg ^ ((row + vrow) & 7)) << 4), in = off < np * 4 ? off : 0;
+        pvm_dma(k < 8 ? vg + (int64_t)(row + vrow) * a.n_ctx * 4 + in : pg[k - 8] + in, lds0 + (unsigned)((it & 1) * (ROWS * PVM_RS * 4) + row * 512));
     };
     ps_f32x4 acc[32];
 #pragma unroll
     for (int c = 0; c < 32; c++) acc[c] = ps_f32x4{0.f, 0.f, 0.f, 0.f};
-    float *b0p = pvs, *b1p = pvs + (size_t)ROWS * PVM_RS;
-    // step `it` computes from buffer it & 1 while the block of step it + 1 (fetched a whole step ago) is parked in the other
-    // buffer and the block of step it + 2 is on its way: a fetch has one step of matrix work to hide behind
-    if (n_it > 0) { fetch(0); park(0, b0p); fetch(min(1, n_it - 1)); }
-    __syncthreads();
+    if (n_it > 0)
+#pragma unroll
+        for (int k = 0; k < 8 + NPW; k++) request(0, k);
     for (int it = 0; it < n_it; it++) {
-        float *cur = (it & 1) ? b1p : b0p, *nxt = (it & 1) ? b0p : b1p;
-        park(it + 1, nxt); // (past the last step: zeros nobody reads)
-        fetch(min(it + 2, n_it - 1));
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); // this wave's share of step `it` has landed, its operands of step it - 1 are in registers;
+        __builtin_amdgcn_s_barrier();                                // everyone's: the place of step it - 1 is free
+        asm volatile("" ::: "memory");
+        const float *cur = pvs + (it & 1) * (ROWS * PVM_RS);
         float av[32], bv[32];
 #pragma unroll
         for (int q4 = 0; q4 < 8; q4++) {
@@ -1099,9 +1084,17 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_pv_mfma_lds_kernel(psl_attn_a
             av[4 * q4] = t.x; av[4 * q4 + 1] = t.y; av[4 * q4 + 2] = t.z; av[4 * q4 + 3] = t.w;
             bv[4 * q4] = w.x; bv[4 * q4 + 1] = w.y; bv[4 * q4 + 2] = w.z; bv[4 * q4 + 3] = w.w;
         }
+        if (it * 4 + 4 > nblk) { // (the last step of a row whose blocks of 32 are no multiple of four)
+            const bool in = it * 4 + m < nblk;
 #pragma unroll
-        for (int c = 0; c < 32; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[c], bv[c], acc[c], 0, 0, 0); // sum = x*y + sum, x = V row
-        __syncthreads();
+            for (int c = 0; c < 32; c++) { av[c] = in ? av[c] : 0.f; bv[c] = in ? bv[c] : 0.f; }
+        }
+        const bool more = it + 1 < n_it;
+#pragma unroll
+        for (int c = 0; c < 32; c++) {
+            acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[c], bv[c], acc[c], 0, 0, 0); // sum = x*y + sum, x = V row
+            if (c % 3 == 1 && c / 3 < 8 + NPW && more) request(it + 1, c / 3); // (one at a time: a request holds its wave's issue, and the matrix core has the other wave's)
+        }
     }
     ps_f32x4 t3[4];
 #pragma unroll
@@ -1128,21 +1121,22 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_pv_mfma_lds_kernel(psl_attn_a
                 for (int r = 0; r < 4; r++) res[r] = ps_dot_left(res[r], vv[k][r], pj[k], j0 + k - np, n_kv - np);
             }
     }
-    if ((int)blockIdx.x * 16 + rl < N)
+    if (bx * 16 + rl < N)
         *(float4 *)(a.att + (int64_t)i * dim + ((int64_t)kvh * r2 + g) * hs + d0 + 4 * m) = make_float4(res[0], res[1], res[2], res[3]);
     // ---- optional: leave the rows quantized for the O projection (saves the quantizer launch between the two).  The workgroup
     // holds 16 (column, head) pairs x hs channels = whole Q8_K tiles of 256 consecutive `att` elements (two heads of one column
     // when hs = 128; psl_attn_pv_quantizes checks the shape): staged through LDS, one wave per tile, ps_quantize_tile as the
     // quantizer kernels run it.
     if (a.qact.qs) {
-        float *tl = pvs; // (the last step's barrier is behind every wave)
+        float *tl = pvs;
+        __syncthreads(); // (the last step's operands are in registers)
         *(float4 *)(tl + rl * hs + d0 + 4 * m) = make_float4(res[0], res[1], res[2], res[3]);
         __syncthreads();
         constexpr int TPW = hs * 16 / 256 / NW; // tiles per wave (1 for hs = 128)
 #pragma unroll
         for (int tt = 0; tt < TPW; tt++) {
             const int tile = wave * TPW + tt, p0 = tile * (256 / hs); // first pair of the tile
-            const int n0 = (int)blockIdx.x * 16 + p0;
+            const int n0 = bx * 16 + p0;
             const int nn = min(n0, N - 1), ci = nn / r2, g0 = nn - ci * r2;
             const float4 xv = *(const float4 *)(tl + tile * 256 + lane * 4);
             const float v4[4] = {xv.x, xv.y, xv.z, xv.w};
