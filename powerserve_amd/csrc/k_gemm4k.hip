@@ -1375,6 +1375,142 @@ __global__ __launch_bounds__(NWV * 64) void gemm4k_par_kernel(const G4KParams p)
 }
 constexpr int g4k_par_lds(const int nwv) { return nwv * ((8 + 4 + 2) * 64 * 16 + 16 * 36 * 4); }
 
+// ---- Q6_K, narrow batches, few tiles: gemm4k_par_kernel's arrangement.  gemm6k_kernel walks a tile pair's super-blocks one behind the other, 0.85 us each whatever the columns, with half of the
+// chip for 4096 rows; here the eight waves of a work-group take the super-blocks of a round side by side (one row tile), park the sums, and run the reference's chains behind a barrier, wave = accumulator
+// lane.  What bounds it is then the issue of a wave's super-block (building 128 + 128 operand registers is ~350 instructions) and two barriers a round.  The weights come straight into LDS two rounds
+// ahead (global_load_lds_dwordx4: their planes hold a row's 128 + 64 bytes together, the operand wants 8 + 4 of them for every accumulator lane; slots swizzled by the row, two passes at most).
+// Measured, 12 columns, with the activations' quantizer: 4096 rows of 14336 62 -> 27 us, 4096 x 4096 20.7 -> 11.8, 1024 x 4096 20.0 -> 11.1; a tree of 12 behind 700 with the Q4_K_M mix 693 -> 570 us.
+constexpr int G6P_NW = 8, G6P_RING = 3, G6P_ST = 2048 + 1024 + 64; // waves; rounds of weights; bytes of a wave's super-block: ql, qh, d of the 16 rows as fp32
+constexpr int G6P_D = G6P_NW * 8 * 1024, G6P_W = G6P_D + G6P_NW * 1024, G6P_LDS = G6P_W + G6P_RING * G6P_NW * G6P_ST;
+__device__ __forceinline__ void g6p_dma(const uint8_t *src, const unsigned lds_dst) { // one wave-instruction: lane l's 16 bytes at src go to lds_dst + 16 l
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds_dst) : "memory");
+}
+__global__ __launch_bounds__(G6P_NW * 64) void gemm6k_par_kernel(const G6KParams p) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int m = lane & 15, kb = lane >> 4, nsb = p.nsb;
+    float4 *const S = (float4 *)lds, *const D = (float4 *)(lds + G6P_D); // [wave][u][lane]: (float)sumi[u] of rows 4 kb + r;  [wave][lane]: d * yd
+    const int64_t row0 = (int64_t)blockIdx.x * 16;
+    const int col = m, colc = col < p.bs ? col : p.bs - 1;
+    const uint8_t *const qlp = p.ql + ((row0 + (lane >> 3)) * nsb) * 128, *const qhp = p.qh + ((row0 + (lane >> 2)) * nsb) * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+    const uint8_t *const scp = (const uint8_t *)p.sc + (row0 + m) * nsb * 16 + kb * 4;
+    const uint16_t *const dp = p.d + (row0 + m) * nsb;
+    const char *const qfp = (const char *)p.qf + lane * 16;
+    const uint8_t *const ydp = p.mf + colc * 4;
+    const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)lds + (unsigned)G6P_W;
+    auto clampsb = [&](const int sb) { return sb < nsb ? sb : nsb - 1; };
+    const int ql_at = ((lane & 7) ^ ((lane >> 3) & 7)) << 4; // (rows 8 j + lane / 8: the row modulo 8 is lane / 8)
+    auto request = [&](const int rd) { // this wave's super-block of round rd (past the end: the last one again, never used)
+        const int sb = clampsb(rd * G6P_NW + wave);
+        const unsigned dst = lds0 + (unsigned)((rd % G6P_RING * G6P_NW + wave) * G6P_ST);
+        g6p_dma(qlp + (int64_t)sb * 128 + ql_at, dst);
+        g6p_dma(qlp + ((int64_t)8 * nsb + sb) * 128 + ql_at, dst + 1024u);
+        g6p_dma(qhp + (int64_t)sb * 64, dst + 2048u);
+    };
+    ps_u32x4 rb[8];
+    uint32_t rsc[2];
+    float rd_[2], ryd[2];
+    auto load_meta = [&](const int s, const int rd) {
+        const int sb = clampsb(rd * G6P_NW + wave);
+        rsc[s] = *(const uint32_t *)(scp + (int64_t)sb * 16);
+        rd_[s] = ps_h2f(dp[sb]);
+        ryd[s] = *(const float *)(ydp + (int64_t)sb * 576);
+    };
+    const int n_rounds = (nsb + G6P_NW - 1) / G6P_NW;
+    request(0);
+    request(1);
+    load_meta(0, 0);
+#pragma unroll
+    for (int u = 0; u < 8; u++) rb[u] = *(const ps_u32x4 *)(qfp + ((size_t)clampsb(wave) << 13) + u * 1024);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    const g4k_f4 zf = {0.f, 0.f, 0.f, 0.f};
+    const g4k_h2 k1056 = {(_Float16)1056.f, (_Float16)1056.f};
+    const int pp = kb >> 1, sh = (kb & 1) * 4, m7 = m & 7, m4 = (m >> 2) & 3;
+#pragma unroll 1
+    for (int rd0 = 0; rd0 < n_rounds; rd0 += 2) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const int rd = rd0 + s;
+            if (rd >= n_rounds) break; // (uniform)
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); // all but the eight operands asked for last: this round's weights, requested two rounds ago, are there
+            load_meta(s ^ 1, rd + 1);
+            request(rd + 2);
+            char *const st = lds + G6P_W + (rd % G6P_RING * G6P_NW + wave) * G6P_ST; // (the wave's own: no barrier)
+            if (kb == 0) *(float *)(st + 3072 + m * 4) = rd_[s];
+            const uint32_t sw = rsc[s];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint2 q = *(const uint2 *)(st + m * 128 + ((u ^ m7) << 4) + pp * 8);
+                const uint32_t h = *(const uint32_t *)(st + 2048 + m * 64 + (((u >> 1) ^ m4) << 4) + (u & 1) * 8 + pp * 4) >> sh, w0 = q.x >> sh, w1 = q.y >> sh;
+                const int s0i = (int)(int8_t)(sw >> (8 * (u >> 2))), s1i = (int)(int8_t)(sw >> (16 + 8 * (u >> 2)));
+                const _Float16 e0 = (_Float16)(float)(s0i & ~1), e1 = (_Float16)(float)(s1i & ~1);
+                const g4k_h2 ev0 = {e0, e0}, ev1 = {e1, e1};
+                const uint32_t om0 = (s0i & 1) ? 0xffffffffu : 0u, om1 = (s1i & 1) ? 0xffffffffu : 0u;
+                const uint32_t t[4] = {(w0 & 0x000F000Fu) | ((h & 0x00030003u) << 4) | 0x64006400u, ((w0 >> 8) & 0x000F000Fu) | (((h >> 8) & 0x00030003u) << 4) | 0x64006400u,
+                                       (w1 & 0x000F000Fu) | (((h >> 2) & 0x00030003u) << 4) | 0x64006400u, ((w1 >> 8) & 0x000F000Fu) | (((h >> 10) & 0x00030003u) << 4) | 0x64006400u};
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) { // as g6k_produce
+                    g4k_h2 v;
+                    __builtin_memcpy(&v, &t[k], 4);
+                    v = v - k1056;
+                    uint32_t vb;
+                    __builtin_memcpy(&vb, &v, 4);
+                    lo[k] = vb & (k < 2 ? om0 : om1);
+                    v = v * (k < 2 ? ev0 : ev1);
+                    __builtin_memcpy(&hi[k], &v, 4);
+                }
+                g4k_h8 avh, avl, bv;
+                __builtin_memcpy(&avh, hi, 16); __builtin_memcpy(&avl, lo, 16); __builtin_memcpy(&bv, &rb[u], 16);
+                g4k_f4 si = __builtin_amdgcn_mfma_f32_16x16x32_f16(avh, bv, zf, 0, 0, 0);
+                si = __builtin_amdgcn_mfma_f32_16x16x32_f16(avl, bv, si, 0, 0, 0);
+                S[(wave * 8 + u) * 64 + lane] = make_float4(si[0], si[1], si[2], si[3]);
+            }
+            const float4 dd = *(const float4 *)(st + 3072 + kb * 16);
+            const float yd = ryd[s];
+            D[wave * 64 + lane] = make_float4(__fmul_rn(yd, dd.x), __fmul_rn(yd, dd.y), __fmul_rn(yd, dd.z), __fmul_rn(yd, dd.w));
+            const int nb = clampsb((rd + 1) * G6P_NW + wave);
+#pragma unroll
+            for (int u = 0; u < 8; u++) rb[u] = *(const ps_u32x4 *)(qfp + ((size_t)nb << 13) + u * 1024);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int cnt = min(nsb - rd * G6P_NW, G6P_NW);
+#pragma unroll
+            for (int q = 0; q < G6P_NW; q++) { // the chains of accumulator lane u = wave, over the round's super-blocks in order
+                if (q < cnt) {
+                    const float4 d4 = D[q * 64 + lane], s4 = S[(q * 8 + wave) * 64 + lane];
+                    acc[0] = __fmaf_rn(d4.x, s4.x, acc[0]); acc[1] = __fmaf_rn(d4.y, s4.y, acc[1]);
+                    acc[2] = __fmaf_rn(d4.z, s4.z, acc[2]); acc[3] = __fmaf_rn(d4.w, s4.w, acc[3]);
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (nothing may land in LDS that is no longer this work-group's)
+    // ---- the lanes meet: waves 0 and 1 finish rows 4 kb + 2 wave, + 1 in hsum_float_8's order
+    S[wave * 64 + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    __syncthreads();
+    if (wave < 2 && col < p.bs) {
+        const int64_t row = row0 + kb * 4 + 2 * wave;
+        float v[2];
+#pragma unroll
+        for (int rr = 0; rr < 2; rr++) {
+            float au[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) au[u] = ((const float *)&S[u * 64 + lane])[2 * wave + rr];
+            const float s0 = __fadd_rn(au[0], au[4]), s1 = __fadd_rn(au[1], au[5]), s2 = __fadd_rn(au[2], au[6]), s3 = __fadd_rn(au[3], au[7]);
+            v[rr] = __fadd_rn(__fadd_rn(s0, s2), __fadd_rn(s1, s3));
+            if (p.bias) v[rr] = __fadd_rn(v[rr], p.bias[row + rr]);
+            if (p.residual) v[rr] = __fadd_rn(p.residual[(int64_t)col * p.ldo + row + rr], v[rr]);
+        }
+        *(float2 *)(p.out + (int64_t)col * p.ldo + row) = make_float2(v[0], v[1]);
+    }
+}
+
 template <int EPI, int RA, int MB>
 static void g4k_launch_wav(hipStream_t st, const G4KParams &p) {
     const unsigned grid = (unsigned)(EPI == 1 ? p.n_tasks : 2 * p.n_tasks);
@@ -1498,14 +1634,23 @@ int psk_gemm5k(hipStream_t st, int n_cu, const psk_gemv6_args &a, ps_act act, in
 int psk_gemm6k(hipStream_t st, int n_cu, const psk_gemv6_args &a, ps_act act, int64_t K, int64_t bs) {
     static const bool off = getenv("PS_NO_GEMM6K") != nullptr; // (A/B switch for measurements)
     const ps_weight *w = a.w;
-    static const int64_t min_cols = [] { const char *e = getenv("PS_GEMM6K_MIN_COLS"); return e ? (int64_t)atoll(e) : (int64_t)9; }(); // (8B Q4_K_M tree forward, ms, threshold 17 / 9 / 2: 8 wide 5.9 / 6.0 / 6.2, 12: 6.9 / 6.3 / 6.3, 16: 7.6 / 6.4 / 6.3)
-    if (off || !w || w->dtype != PS_Q6_K || w->K != K || K % 1024 || w->N % 32 || a.ldo % 2 || !act.qf || bs < min_cols || bs < ps_gemm4k_min_cols()) return -1;
+    if (off || !w || w->dtype != PS_Q6_K || w->K != K || K % 1024 || w->N % 32 || a.ldo % 2 || !act.qf || bs < ps_gemm4k_min_cols()) return -1;
+    // below: k_gemv6.hip's groups of eight columns.  us, those / gemm6k_par_kernel: 14336 x 4096 2 columns 21 / 27, 3 and 4 33 / 27, 5 and more 69 / 26; 4096 x 4096 10.5 / 11.8, 13.7 / 11.5, 24 / 11.6;
+    // 128256 x 4096 119 / 254, 211 / 251, 543 / 252
+    if (bs < 3 || (bs < 5 && w->N / 16 > 2 * (int64_t)n_cu)) return -1;
     G6KParams p{};
     p.ql = w->qs; p.qh = w->qh; p.sc = (const int8_t *)w->sc; p.d = (const uint16_t *)w->aux;
     p.out = a.out; p.bias = a.bias; p.residual = a.residual; p.N = w->N; p.ldo = a.ldo;
     p.nsb = (int)(K / 256); p.bs = (int)bs; p.n_tasks = (int)(w->N / 32);
     p.qf = act.qf; p.mf = act.mf;
     const int n_ct = (int)((bs + 15) / 16);
+    if (n_ct == 1) { // (whatever the rows: 12 columns of 128256 x 4096 328 -> 257 us)
+        static unsigned long long attrp = 0;
+        if (ps_first_on_device(&attrp)) (void)hipFuncSetAttribute((const void *)gemm6k_par_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G6P_LDS);
+        psk_note_kernel("gemm6k_par_kernel");
+        hipLaunchKernelGGL(gemm6k_par_kernel, dim3((unsigned)(w->N / 16)), dim3(G6P_NW * 64), G6P_LDS, st, p);
+        return 0;
+    }
     p.n_cb = (n_ct + 3) / 4;
     p.n_items = (p.n_tasks + 7) / 8 * 8 * p.n_cb;
     int n_wg = p.n_items;

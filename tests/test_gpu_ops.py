@@ -284,6 +284,33 @@ def test_mul_mat_q5k_batch_on_matrix_cores(ctx, oracle, hip, K, N, bs):
     W.free()
 
 
+@pytest.mark.parametrize("K,N,bs", [(1024, 32, 16), (2048, 96, 3), (3072, 64, 9), (11264, 32, 5), (14336, 64, 12), (4096, 8224, 5), (4096, 4128, 4)])
+def test_mul_mat_q6k_narrow_batch(ctx, oracle, hip, K, N, bs):
+    """At most 16 columns of a Q6_K weight: gemm6k_par_kernel takes the super-blocks of a round side by side -- fewer than a round (K / 256 = 4), whole and ragged ones, even and odd
+    numbers of them -- with every scale at its ends (-128, 127, 0, odd and even), every 6-bit value at 0 and 63, d = 0, -0, subnormal and negative."""
+    from powerserve_amd import synth
+    rng = np.random.default_rng(K + N + bs)
+    w = np.ascontiguousarray(synth.random_blocks(rng, 14, N, K)).reshape(N, K // 256, 210)
+    for r in range(N):
+        for k, sc in enumerate(([0x80] * 16, [0x7F] * 16, [0x00] * 16, [0x81, 0x01, 0xFF, 0x02] * 4)):
+            if rng.random() < 0.5:
+                w[r, (r + k) % (K // 256), 192:208] = sc
+        w[r, (r + 1) % (K // 256), :192] = (0x00, 0xFF)[r & 1]
+        w[r, (r + 2) % (K // 256), 208:210] = ((0, 0), (0, 0x80), (1, 0), (0, 0xC2))[r % 4]
+    x = (rng.standard_normal((bs, K)) * rng.uniform(0.1, 30.0, (bs, 1))).astype(np.float32)
+    x[bs - 1, 256:512] = 0.0
+    x[0] *= 1e-35 / np.abs(x[0]).max()
+    want = oracle.mul_mat(14, w.reshape(-1), K, N, x)
+    W = ctx.upload_weight(14, w.reshape(-1), K, N)
+    dx, dy = ctx.to_device(x), ctx.empty((bs, N))
+    for _ in range(2):
+        ctx.check(ctx.L.ps_hip_mul_mat(ctx.h, C.byref(dy.tensor()), C.byref(W.tensor()), C.byref(dx.tensor())))
+        assert ctx.L.ps_hip_last_matmul_kernel().decode() == "gemm6k_par_kernel"
+        got = dy.numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rel_err(got, want), np.argwhere(got != want)[:8])
+    W.free()
+
+
 @pytest.mark.parametrize("wt", [12, 13, 14])
 def test_mul_mat_kquant_random_shapes(ctx, oracle, hip, wt):
     """Seeded sweep over shapes the parametrized cases do not name: column counts 2 .. 200 (narrow kernel, wide kernel with 1 .. 4
