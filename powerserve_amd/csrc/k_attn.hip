@@ -28,6 +28,14 @@ __device__ __forceinline__ void coh_store_f(float *p, float v) { __hip_atomic_st
 
 // (pos0, bs) of the forward: from the launch arguments when the host knew them at enqueue time (eager batches), else from the device-resident state
 __device__ __forceinline__ int att_pos0(const psl_attn_args &a) { return a.bs_host > 0 ? a.n_kv_host - a.bs_host : a.state->pos0; }
+// a launch over several reference chunks: from here on `a` is chunk k's
+__device__ __forceinline__ void att_chunk(psl_attn_args &a, const int k) {
+    if (a.sub <= 0) return;
+    const int first = k * a.sub, pos0 = a.n_kv_host - a.bs_host + first, bs = min(a.sub, a.bs_host - first), dim = a.n_heads * a.head_size;
+    a.bs_host = bs; a.n_kv_host = pos0 + bs;
+    a.q += (int64_t)first * dim; a.att += (int64_t)first * dim; a.scores += (int64_t)first * a.n_heads * a.n_ctx;
+}
+static int att_chunks(const psl_attn_args &a) { return a.sub > 0 ? (a.bs_host + a.sub - 1) / a.sub : 1; }
 __device__ __forceinline__ int att_bs(const psl_attn_args &a) { return a.bs_host > 0 ? a.bs_host : a.state->bs; }
 
 // ---------------------------------------------------------------- rope + KV append
@@ -141,6 +149,8 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
     auto swz = [](int row, int seg) { return row * RS + ((seg ^ (row & 7)) << 2); }; // float index of 16-byte column `seg` of row `row`
     const int dim = a.n_heads * hs, kvd = a.n_kv_heads * hs, r2 = a.n_heads / a.n_kv_heads;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int z = (int)blockIdx.z % SCM_Z;
+    att_chunk(a, (int)(gridDim.z - 1 - blockIdx.z) / SCM_Z); // (the chunks that see most first)
     const int kvh = blockIdx.y, bs = att_bs(a), n_kv = att_pos0(a) + bs;
     if ((int)blockIdx.x * 64 >= n_kv) return; // (the whole workgroup)
     const int j0 = ((int)blockIdx.x * 4 + wave) * 16;
@@ -170,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
             const int sidx = lane + k * 64, row = sidx / SEGS, sg = sidx - row * SEGS;
             sk[k] = *(const float4 *)(a.k_cache + (int64_t)min(j0 + row, n_kv - 1) * kvd + kvh * hs + sg * 4);
         }
-        q_fetch((int)blockIdx.z < n_tiles ? (int)blockIdx.z : 0);
+        q_fetch(z < n_tiles ? z : 0);
 #pragma unroll
         for (int k = 0; k < NSK; k++) {
             const int sidx = lane + k * 64, row = sidx / SEGS, sg = sidx - row * SEGS;
@@ -188,7 +198,7 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
     }
     const ps_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     int cur = 0;
-    for (int tile = blockIdx.z; tile < n_tiles; tile += SCM_Z, cur ^= 1) {
+    for (int tile = z; tile < n_tiles; tile += SCM_Z, cur ^= 1) {
         const bool more = tile + SCM_Z < n_tiles;
         q_fetch(more ? tile + SCM_Z : tile); // (the next block: one column tile of matrix work to hide behind)
         if (live) {
@@ -893,7 +903,9 @@ __global__ __launch_bounds__(PV_NT) void attn_softmax_pv_cols_kernel(psl_attn_ar
 //      grid (ceil(bs * r2 / 16), n_kv_heads), one wave per 16 head channels.
 __global__ __launch_bounds__(PV_NT) void attn_softmax_probs_kernel(psl_attn_args a) {
     extern __shared__ __attribute__((aligned(16))) float pl[]; // [r2][n_kv4]
+    att_chunk(a, (int)(gridDim.z - 1 - blockIdx.z));
     const int r2 = a.n_heads / a.n_kv_heads, kvh = blockIdx.x, i = blockIdx.y, bs = att_bs(a), pos0 = att_pos0(a);
+    if (i >= bs) return; // (the last chunk may be shorter)
     const int n_kv = pos0 + bs, n_kv4 = (n_kv + 3) & ~3;
     __shared__ float redf[R2MAX][PV_NW];
     __shared__ double redd[R2MAX][PV_NW];
@@ -913,6 +925,7 @@ __global__ __launch_bounds__(PV_NT) void attn_softmax_probs_kernel(psl_attn_args
 constexpr int SMW_MAXQ = 16; // float4 per lane: n_kv <= 64 * 4 * 16
 __global__ __launch_bounds__(256) void attn_softmax_probs_wave_kernel(psl_attn_args a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    att_chunk(a, (int)(gridDim.y - 1 - blockIdx.y));
     const int bs = att_bs(a), pos0 = att_pos0(a), n_kv = pos0 + bs, n8 = n_kv & ~7;
     const int row = (int)blockIdx.x * 4 + wave;
     if (row >= bs * a.n_heads) return;
@@ -984,6 +997,7 @@ __global__ __launch_bounds__(256) void attn_softmax_probs_wave_kernel(psl_attn_a
 }
 
 __global__ __launch_bounds__(512, 1) void attn_pv_mfma_kernel(psl_attn_args a) {
+    att_chunk(a, (int)(gridDim.z - 1 - blockIdx.z));
     const int hs = a.head_size, dim = a.n_heads * hs, r2 = a.n_heads / a.n_kv_heads;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int kvh = blockIdx.y, bs = att_bs(a), n_kv = att_pos0(a) + bs, np = n_kv & ~31, nblk = np >> 5;
@@ -1043,6 +1057,7 @@ template <int NW> // waves per workgroup = head_size / 16
 __global__ __launch_bounds__(NW * 64, 1) void attn_pv_mfma_lds_kernel(psl_attn_args a) {
     extern __shared__ __attribute__((aligned(16))) float pvs[]; // [2][(NW + 1) * 16][PVM_RS]: the waves' V rows, then the 16 probability rows
     constexpr int hs = NW * 16, ROWS = (NW + 1) * 16, NPW = 8 / NW; // NPW: pairs of probability rows per wave
+    att_chunk(a, (int)(gridDim.z - 1 - blockIdx.z));
     const int dim = a.n_heads * hs, r2 = a.n_heads / a.n_kv_heads;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // work-groups are dealt to the eight XCDs in turn (x fastest): numbered so that an XCD has neighbouring ones, a kv head's values are read through one L2, not through all
@@ -1326,7 +1341,7 @@ void psl_attn_scores(hipStream_t st, const psl_attn_args &a, int bs) {
     // batch kernel: 36 us per call whatever n_kv is) — so eager forwards size the grid with the host's copy of the position
     const int nk = a.n_kv_host > 0 && a.n_kv_host < a.n_ctx ? a.n_kv_host : a.n_ctx;
     if (bs >= 8) { // batches: matrix cores (exact f32 chains), one wave per 16 positions
-        dim3 gm((unsigned)((nk + 63) / 64), (unsigned)a.n_kv_heads, (unsigned)SCM_Z);
+        dim3 gm((unsigned)((nk + 63) / 64), (unsigned)a.n_kv_heads, (unsigned)(SCM_Z * att_chunks(a)));
         if (a.head_size == 128) hipLaunchKernelGGL(attn_scores_mfma_kernel<4>, gm, dim3(256), 0, st, a);
         else if (a.head_size == 64) hipLaunchKernelGGL(attn_scores_mfma_kernel<2>, gm, dim3(256), 0, st, a);
         else if (a.head_size == 32) hipLaunchKernelGGL(attn_scores_mfma_kernel<1>, gm, dim3(256), 0, st, a);
@@ -1353,10 +1368,11 @@ void psl_attn_softmax_pv(hipStream_t st, const psl_attn_args &a, int bs) {
         static unsigned long long attrp = 0; // devices that have the attribute
         if (ps_first_on_device(&attrp)) { (void)hipFuncSetAttribute((const void *)attn_softmax_probs_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024); }
         const int r2p = a.n_heads / a.n_kv_heads;
+        const unsigned n_sub = (unsigned)att_chunks(a);
         const size_t ldsp = (size_t)r2p * (((size_t)a.n_ctx + 3) & ~(size_t)3) * 4;
-        if (a.n_ctx <= 64 * 4 * SMW_MAXQ) hipLaunchKernelGGL(attn_softmax_probs_wave_kernel, dim3((unsigned)((bs * a.n_heads + 3) / 4)), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(attn_softmax_probs_kernel, dim3((unsigned)a.n_kv_heads, (unsigned)bs), dim3(PV_NT), ldsp, st, a);
-        const dim3 gpv((unsigned)((bs * r2p + 15) / 16), (unsigned)a.n_kv_heads);
+        if (a.n_ctx <= 64 * 4 * SMW_MAXQ) hipLaunchKernelGGL(attn_softmax_probs_wave_kernel, dim3((unsigned)((bs * a.n_heads + 3) / 4), n_sub), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL(attn_softmax_probs_kernel, dim3((unsigned)a.n_kv_heads, (unsigned)bs, n_sub), dim3(PV_NT), ldsp, st, a);
+        const dim3 gpv((unsigned)((bs * r2p + 15) / 16), (unsigned)a.n_kv_heads, n_sub);
         if (a.head_size == 128 || a.head_size == 64) {
             static unsigned long long attrl = 0;
             if (ps_first_on_device(&attrl)) {

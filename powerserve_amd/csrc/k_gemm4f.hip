@@ -8,9 +8,9 @@
 //   * a wave owns 16 rows and CT column tiles WHOLE -- all eight accumulator lanes and the four mins lanes, 48 CT chains per lane.  Its weights become operands in its own
 //     registers (nine instructions per accumulator lane) and meet CT column tiles; no wave waits for another's, and the sums over the lanes at the end are in-lane;
 //   * eight waves share the columns: 128 rows x 16 CT columns per work-group, one work-group per CU, persistent.  Activations, weights, headers and column metadata come by
-//     global_load_lds_dwordx4 into a ring of three stages of one super-block.  One barrier in the middle of a stage says both that the next stage is there and that the one
+//     global_load_lds_dwordx4 into a ring of three stages of one super-block.  One barrier a quarter into a stage says both that the next stage is there and that the one
 //     before has been left, so that its place is asked for at once -- piece by piece: asked for in one go, the wave stands still while the memory pipe takes them (a stage of
-//     CT = 3: 1.60 us, 1.44 spread);
+//     CT = 3: 1.60 us, 1.44 with a piece every other step; the barrier in the middle of the stage leaves the last pieces too little time: 3 % more);
 //   * the operands of the activations are read NY steps ahead, across the stages; the next stage's scales and metadata at the end of this one (1.60 us against 2.0 read when
 //     needed).  CT = 4 would need 30 registers more than two waves per SIMD have.
 // Measured (with the activations' quantizer in front, k_gemm4k.hip's wide kernel -> this): 4096 x 28672, 512 columns 382 -> 278 us, 203 columns 200 -> 141, 32 columns 59 -> 29;
@@ -129,7 +129,8 @@ __global__ __launch_bounds__(G4F_NRW * 64, G4F_NRW / 4) void gemm4f_kernel(const
         r_hm = lane < 16 ? W.aux + ((size_t)(2 * t + (m >> 3)) * nsb) * 128 + (m & 7) * 16
                          : p.mf + (size_t)min(I.cb * CT + min(wave, CT - 1), last) * nsb * 576 + (lane - 16) * 16;
     };
-    constexpr int NP = NB + 3, SP = 4 * CT / NP; // pieces of a stage per wave, steps from one to the next
+    constexpr int NP = NB + 3; // pieces of a stage per wave
+    static_assert(2 * CT + 2 * NP <= 8 * CT, "asked for within the stage");
     auto request_piece = [&](const unsigned st, const int i) {
         if (i < 2) g4f_dma64(r_w + 64 * i, st + (unsigned)(W0 + wave * 2048 + i * 1024));
         else if (i == 2) { if (lane < n_hm) g4f_dma64(r_hm, st + (unsigned)wave_hm); }
@@ -265,13 +266,13 @@ __global__ __launch_bounds__(G4F_NRW * 64, G4F_NRW / 4) void gemm4f_kernel(const
                 }
                 D = P;
                 __builtin_amdgcn_sched_barrier(0);
-                if (s == 4 * CT - 1) { // the next stage is there for all; every wave has left the one before the present one behind, whose place the stage after next takes
+                if (s == 2 * CT - 1) { // the next stage is there for all; every wave has left the one before the present one behind, whose place the stage after next takes
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                 }
                 if (EPI != 1 || sb + 1 < nsb) { // ... which it is asked for piece by piece (all at once, the wave stands still while the memory pipe takes them: 0.28 us of a stage)
-                    if (s >= 4 * CT && (s - 4 * CT) % SP == 0 && (s - 4 * CT) / SP < NP) request_piece(r_st, (s - 4 * CT) / SP);
+                    if (s >= 2 * CT && (s - 2 * CT) % 2 == 0 && (s - 2 * CT) / 2 < NP) request_piece(r_st, (s - 2 * CT) / 2);
                     if (s == 8 * CT - 1) advance();
                 }
                 if (s == 5 * CT) read_head(ns);

@@ -343,7 +343,20 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
             // a super-chunk of several reference-sized chunks (ps_hip_model_prefill): the mat-muls above and below take all bs columns
             // at once (they are column-wise: chunking cannot change their bits), the attention runs chunk by chunk with the n_kv the
             // reference's chunk would have seen -- its soft-max and V.p sums depend on where a chunk ends
-            for (int c0 = 0, k = 0; c0 < bs; c0 += m->attn_chunk, k++) {
+            // (all chunks of at least 8 tokens in one launch each of scores, soft-max and V.p, where the host knows the positions: with three launches per chunk of 128 the boundaries were
+            //  a tenth of a prompt's attention, and the first chunks' grids an eighth of the chip)
+            const int rest = bs % m->attn_chunk, together = rest && rest < 8 ? bs - rest : bs;
+            int c0 = 0, k = 0;
+            if (m->n_kv_host > 0 && m->attn_chunk >= 8 && together > m->attn_chunk && dim % 16 == 0 && f.head_size % 16 == 0) {
+                psl_attn_args as = aa;
+                as.n_kv_host = m->n_kv_host - (bs - together);
+                as.bs_host = together; as.sub = m->attn_chunk;
+                as.qact = ps_act{}; as.dbg = nullptr;
+                psl_attn_scores(st, as, m->attn_chunk);
+                psl_attn_softmax_pv(st, as, m->attn_chunk);
+                c0 = together; k = (together + m->attn_chunk - 1) / m->attn_chunk;
+            }
+            for (; c0 < bs; c0 += m->attn_chunk, k++) {
                 const int nb = bs - c0 < m->attn_chunk ? bs - c0 : m->attn_chunk;
                 psl_attn_args as = aa;
                 as.state = m->state_sub + k;
