@@ -131,9 +131,8 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(psl_attn_args a) {
 // with k = the 32-element block index gives the 16 x 16 tile of chain-c partials (16 positions x 16 (column, head)
 // pairs), and GGML_F32x8_REDUCE becomes 31 element-wise adds of tiles in its own association.  No cross-lane reduction
 // at all; a K row is fetched once per 16 positions and meets every column of the batch.
-// grid (ceil(n_ctx / 64), n_kv_heads, SCM_Z): one wave per 16 positions, the column tiles split over blockIdx.z.
+// grid (ceil(n_ctx / 64), n_kv_heads, chunks x psl_attn_args::zs): one wave per 16 positions, the column tiles split over zs work-groups.
 typedef float ps_f32x4 __attribute__((ext_vector_type(4)));
-constexpr int SCM_Z = 8;
 // Operands go through LDS: a lane's operand run is 128 B of one row, and fetched directly a wave instruction touches 64
 // cache lines for 1 KiB (the CU's address unit, not the matrix core, set the time).  So a wave fetches its 16 K rows with
 // row-coalesced instructions into its own LDS block once, the workgroup fetches each 16-column block of q once for its
@@ -147,10 +146,10 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
     // the swizzle is (tools/lds_bank_check.py: one pass, reads and parks, head sizes 64 and 128)
     constexpr int hs = NV * 32, RS = hs, SEGS = hs / 4, NSK = 16 * SEGS / 64, NSQ = (16 * SEGS + 255) / 256; // float4 segments per lane: K block / q block
     auto swz = [](int row, int seg) { return row * RS + ((seg ^ (row & 7)) << 2); }; // float index of 16-byte column `seg` of row `row`
-    const int dim = a.n_heads * hs, kvd = a.n_kv_heads * hs, r2 = a.n_heads / a.n_kv_heads;
+    const int kvd = a.n_kv_heads * hs, r2 = a.n_heads / a.n_kv_heads;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int z = (int)blockIdx.z % SCM_Z;
-    att_chunk(a, (int)(gridDim.z - 1 - blockIdx.z) / SCM_Z); // (the chunks that see most first)
+    const int Z = a.zs, z = (int)blockIdx.z % Z;
+    att_chunk(a, (int)(gridDim.z - 1 - blockIdx.z) / Z); // (the chunks that see most first)
     const int kvh = blockIdx.y, bs = att_bs(a), n_kv = att_pos0(a) + bs;
     if ((int)blockIdx.x * 64 >= n_kv) return; // (the whole workgroup)
     const int j0 = ((int)blockIdx.x * 4 + wave) * 16;
@@ -159,11 +158,15 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
     __shared__ __attribute__((aligned(16))) float ql[2][16 * RS];
     const int rl = lane & 15, m = lane >> 4; // A: row rl (position), k = m;  B: k = m, column rl
     const int N = bs * r2, n_tiles = (N + 15) / 16;
+    // columns are pairs (i, g): n / r2 by its reciprocal (n (r2 - 1) < 2^32: exact)
+    const unsigned inv_r2 = r2 > 1 ? 0xffffffffu / (unsigned)r2 + 1 : 0;
+    auto by_r2 = [&](const int n) { return r2 > 1 ? (int)__umulhi((unsigned)n, inv_r2) : n; };
+    const float *const qh = a.q + kvh * r2 * hs;
     float4 sq0, sq1; // (named, not an array: the array went to scratch)
     auto q_fetch1 = [&](int tile, int k) -> float4 { // (segment indices past the block are clamped here and not parked)
         const int sidx = min((int)threadIdx.x + k * 256, 16 * SEGS - 1), row = sidx / SEGS, sg = sidx - row * SEGS;
-        const int n = min(tile * 16 + row, N - 1), i = n / r2, g = n - i * r2;
-        return *(const float4 *)(a.q + (int64_t)i * dim + (int64_t)(kvh * r2 + g) * hs + sg * 4);
+        const int n = min(tile * 16 + row, N - 1), i = by_r2(n), g = n - i * r2;
+        return *(const float4 *)(qh + (unsigned)((i * a.n_heads + g) * hs + sg * 4));
     };
     auto q_fetch = [&](int tile) { sq0 = q_fetch1(tile, 0); if (NSQ > 1) sq1 = q_fetch1(tile, 1); };
     auto q_park1 = [&](float *buf, int k, const float4 v) {
@@ -198,11 +201,11 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
     }
     const ps_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     int cur = 0;
-    for (int tile = z; tile < n_tiles; tile += SCM_Z, cur ^= 1) {
-        const bool more = tile + SCM_Z < n_tiles;
-        q_fetch(more ? tile + SCM_Z : tile); // (the next block: one column tile of matrix work to hide behind)
+    for (int tile = z; tile < n_tiles; tile += Z, cur ^= 1) {
+        const bool more = tile + Z < n_tiles;
+        q_fetch(more ? tile + Z : tile); // (the next block: one column tile of matrix work to hide behind)
         if (live) {
-            const int n = min(tile * 16 + rl, N - 1), i = n / r2, g = n - i * r2;
+            const int n = min(tile * 16 + rl, N - 1), i = by_r2(n), g = n - i * r2;
             float qb[32]; // B operand of chain c: q[i][kvh * r2 + g][32 m + c]
 #pragma unroll
             for (int q4 = 0; q4 < 8; q4++) {
@@ -243,7 +246,7 @@ __global__ __launch_bounds__(256, 2) void attn_scores_mfma_kernel(psl_attn_args 
             const ps_f32x4 res = (t3[0] + t3[1]) + (t3[2] + t3[3]);
             // D: column = lane & 15 (the (i, g) pair), rows 4 * (lane >> 4) + r (positions)
             if (tile * 16 + rl < N) {
-                float *sb = a.scores + ((int64_t)i * a.n_heads + (int64_t)kvh * r2 + g) * a.n_ctx;
+                float *sb = a.scores + (int64_t)(i * a.n_heads + kvh * r2 + g) * a.n_ctx;
                 const int jb = j0 + 4 * m;
                 if (jb + 3 < n_kv) *(float4 *)(sb + jb) = make_float4(res[0], res[1], res[2], res[3]);
                 else
@@ -1341,11 +1344,18 @@ void psl_attn_scores(hipStream_t st, const psl_attn_args &a, int bs) {
     // batch kernel: 36 us per call whatever n_kv is) — so eager forwards size the grid with the host's copy of the position
     const int nk = a.n_kv_host > 0 && a.n_kv_host < a.n_ctx ? a.n_kv_host : a.n_ctx;
     if (bs >= 8) { // batches: matrix cores (exact f32 chains), one wave per 16 positions
-        dim3 gm((unsigned)((nk + 63) / 64), (unsigned)a.n_kv_heads, (unsigned)(SCM_Z * att_chunks(a)));
-        if (a.head_size == 128) hipLaunchKernelGGL(attn_scores_mfma_kernel<4>, gm, dim3(256), 0, st, a);
-        else if (a.head_size == 64) hipLaunchKernelGGL(attn_scores_mfma_kernel<2>, gm, dim3(256), 0, st, a);
-        else if (a.head_size == 32) hipLaunchKernelGGL(attn_scores_mfma_kernel<1>, gm, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(attn_scores_mfma_kernel<3>, gm, dim3(256), 0, st, a);
+        // work-groups that share a block of 64 positions: as many as eight where the blocks are few, two where they alone fill the chip -- each fetches its K rows and its first q block before it can
+        // multiply, four tiles' time (four chunks of 128 at 2048 positions, 32 heads of 128: 95 / 87 / 83 / 89 us a launch with 8 / 4 / 2 / 1) -- and no more than there are column tiles
+        const int64_t base = (int64_t)((nk + 63) / 64) * a.n_kv_heads * att_chunks(a), tiles = (bs * (a.n_heads / a.n_kv_heads) + 15) / 16;
+        psl_attn_args b = a;
+        b.zs = 8;
+        while (b.zs > 2 && base * b.zs > 1024) b.zs /= 2;
+        if (b.zs > tiles) b.zs = (int)tiles;
+        dim3 gm((unsigned)((nk + 63) / 64), (unsigned)a.n_kv_heads, (unsigned)(b.zs * att_chunks(a)));
+        if (a.head_size == 128) hipLaunchKernelGGL(attn_scores_mfma_kernel<4>, gm, dim3(256), 0, st, b);
+        else if (a.head_size == 64) hipLaunchKernelGGL(attn_scores_mfma_kernel<2>, gm, dim3(256), 0, st, b);
+        else if (a.head_size == 32) hipLaunchKernelGGL(attn_scores_mfma_kernel<1>, gm, dim3(256), 0, st, b);
+        else hipLaunchKernelGGL(attn_scores_mfma_kernel<3>, gm, dim3(256), 0, st, b);
         return;
     }
     dim3 g((unsigned)((nk + 31) / 32), (unsigned)a.n_kv_heads, (unsigned)bs);

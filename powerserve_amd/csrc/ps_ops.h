@@ -41,6 +41,7 @@ struct psl_attn_args {
     int n_kv_host;           // pos0 + bs when the host knows it at enqueue time (eager forwards), 0 inside a captured graph: sizes the score grids
     int bs_host;             // with n_kv_host: the batch size, so that the batch kernels need not wait for the device-resident state (an L2 miss at the head of every launch)
     int sub;                 // > 0 (with n_kv_host and bs_host; batches of at least 8, no tree): the bs_host columns are reference chunks of `sub`, each attended with n_kv = its own end, in one launch
+    int zs;                  // the batch score kernel's work-groups per 64 positions and kv head, which share the columns (set by psl_attn_scores)
     _Float16 *k16, *v16;     // optional fp16 mirrors of the caches, both [n_ctx][kv_dim] (fp16-KV decode mode: ps_hip_model_set_mode bit 3)
     float *part;             // [n_heads][FL_SPLITS][head_size + 2] partial (o, m, l) of the split-KV decode attention
     unsigned long long *dbg; // timeline buffer of the single-token kernels (ps_hip_debug_timeline keys 40 / 41), or null
