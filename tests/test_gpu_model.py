@@ -379,6 +379,26 @@ def test_prefill_in_super_chunks_keeps_the_reference_chunking(ctx, oracle, tmp_p
     om.close()
 
 
+@pytest.mark.parametrize("preset,wt,chunk,P,n_ctx", [("odd-llama-hs96", 8, 8, 67, 256), ("odd-llama-hs32", 2, 24, 147, 256), ("odd-qwen2-r3", 8, 40, 256, 512), ("odd-llama-r5", 8, 16, 103, 256),
+                                                     ("odd-llama-r6", 8, 64, 202, 256), ("odd-llama-r8", 2, 128, 391, 512), ("tiny-llama", 8, 64, 200, 4352), ("small-llama-hs128", 12, 128, 519, 4352)])
+def test_chunks_attended_in_one_launch(ctx, tmp_path, preset, wt, chunk, P, n_ctx):
+    """The attention of a launch sequence's chunks in one launch each of scores, soft-max and V.p: head sizes 32, 64, 96 and 128, groups of 1 .. 8 heads, chunks of 8, a shorter last chunk of
+    at least 8 tokens (in the launch) and of fewer (behind it), a context window beyond the wave form of the soft-max; the same cache rows as one chunk at a time, on bits."""
+    from powerserve_amd import hip, synth
+    d = str(tmp_path / "m")
+    mj = synth.write_model_dir(d, preset, wt, n_ctx=n_ctx, seed=3)
+    toks = np.random.default_rng(P).integers(0, mj["llm_config"]["vocab_size"], P)
+    caches = []
+    for mb in (chunk, 512):
+        gm = hip.Model(ctx, d, max_batch=mb, n_ctx=n_ctx)
+        gm.prefill(toks[:11], chunk)
+        gm.prefill(toks[11:], chunk)
+        caches.append([(gm.k_cache(L)[:P].copy(), gm.v_cache(L)[:, :P].copy()) for L in range(gm.cfg.n_layers)])
+        gm.close()
+    for (k0, v0), (k1, v1) in zip(*caches):
+        assert np.array_equal(k0.view(np.uint32), k1.view(np.uint32)) and np.array_equal(v0.view(np.uint32), v1.view(np.uint32))
+
+
 @pytest.mark.parametrize("preset,wt,chunk", [("small-llama-hs128", 12, 256), ("small-llama-hs128", 12, 512), ("small-llama-hs128", 1015, 384), ("tiny-llama", 8, 256), ("tiny-qwen2", 2, 320)])
 def test_wide_prefill_chunks_match_oracle(ctx, oracle, tmp_path, preset, wt, chunk):
     """hparams batch_size above the reference's default of 128 (bench.py reports a 512-token-chunk prefill next to the headline):
