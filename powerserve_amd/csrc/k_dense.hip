@@ -504,46 +504,32 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) { /
     }
 }
 
-// Four results of one output column n: local rows tb .. tb + 3.  Every lane of the wave calls this.
-static __device__ __forceinline__ void dn_put4r(const dn_args &g, long long row0, int T, int tb, long long n, const dn_f4 &acc) {
-    const bool nin = n < g.N;
-    const bool pair = g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR;
-    float old[4];
-    if (g.accum && !pair) { // every old value is requested before the first is used
-#pragma unroll
-        for (int r = 0; r < 4; r++) old[r] = tb + r < T && nin ? g.out[dn_orow(g, row0, tb + r, T) * g.ldo + n] : 0.f;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int t = tb + r;
-        const bool in = t < T && nin;
-        if (pair || g.em_table) { // (row n ^ 1 is the neighbouring lane's)
-            dn_put<true>(g, dn_orow(g, row0, t, T), n, acc[r], pair ? __shfl_xor(acc[r], 1, 64) : 0.f, in);
-            continue;
-        }
-        if (!in) continue;
-        const long long o = dn_orow(g, row0, t, T);
-        const float v = dn_epi(g, acc[r], n) * (g.out_scale ? g.out_scale[o] : 1.f);
-        if (g.out16) g.out16[o * g.ldo + n] = dn_f2bf(v);
-        else g.out[o * g.ldo + n] = g.accum ? old[r] + v : v;
-    }
-}
-
-// Four neighbouring results of output row t, columns n .. n + 3 (n a multiple of four).
+// Four neighbouring results of output row t, columns n .. n + 3 (n a multiple of four).  The four go through ONE copy of the epilogue's code, the registers turning by one
+// each time: code that runs a few times per launch has to be fetched first.  Four copies took 7.0 us in the sums of 512 x 2048, one 6.3; the activations of a wide product the same.
 static __device__ __forceinline__ void dn_put4(const dn_args &g, long long t, long long n, dn_f4 acc) {
     if (n >= g.N) return;
     if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR || g.em_table || n + 4 > g.N || g.ldo % 4 || ((uintptr_t)g.out & 15)) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) dn_put<true>(g, t, n + e, acc[e], acc[e ^ 1], n + e < g.N);
+#pragma unroll 1
+        for (int e = 0; e < 4; e++) {
+            dn_put<true>(g, t, n + e, acc[0], acc[1], n + e < g.N); // (a pair is stored by its even row)
+            acc = dn_f4{acc[1], acc[2], acc[3], acc[0]};
+        }
         return;
     }
     float *p = g.out + t * g.ldo + n;
     dn_f4 v = dn_f4{0.f, 0.f, 0.f, 0.f};
     if (g.accum) v = *(const dn_f4 *)p;
     const float rs = g.out_scale ? g.out_scale[t] : 1.f;
+    if (g.act != PSD_ACT_NONE || g.bias) { // (uniform)
+#pragma unroll 1
+        for (int e = 0; e < 4; e++) acc = dn_f4{acc[1], acc[2], acc[3], dn_epi(g, acc[0], n + e)};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] *= g.alpha;
+    }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const float y = dn_epi(g, acc[e], n + e) * rs;
+        const float y = acc[e] * rs;
         v[e] = g.accum ? v[e] + y : y;
     }
     if (g.out16) {
@@ -676,7 +662,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
                             dn_bf8 za, zb;
                             __builtin_memcpy(&za, &xa[half][u][i], 16);
                             __builtin_memcpy(&zb, &xb[half][u][j], 16);
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(za, zb, acc[i][j], 0, 0, 0);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(zb, za, acc[i][j], 0, 0, 0);
                         }
                 } else {
 #pragma unroll
@@ -684,7 +670,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
 #pragma unroll
                         for (int i = 0; i < MI; i++)
 #pragma unroll
-                            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[half][u][i][x], xb[half][u][j][x], acc[i][j], 0, 0, 0);
+                            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xb[half][u][j][x], xa[half][u][i][x], acc[i][j], 0, 0, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -712,7 +698,37 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
         }
     }
     if (p.S > 1) return;
-    // the tile through LDS (the stages are done with), so that a thread has four neighbouring outputs of a row
+    // The weights are the matrix instructions' first operand, so a lane has four neighbouring outputs of a token in four registers: results that need no epilogue go straight to their
+    // places.  Through LDS (two barriers, a loop of eight trips) 512 x 8192 of K = 2048 took 35.0 us with its packing, 31.2 this way, 512 x 2048 18.3 and 17.3.
+    // An activation of each of the 64 results of a lane, written out, is code that every CU has to fetch once: 40.6 us against 32.6 for a loop; it goes through LDS.
+    if (g.act == PSD_ACT_NONE && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
+        if (loads) return;
+#pragma unroll
+        for (int i = 0; i < MI; i++) {
+            const int t = t0 + wm * MI * 32 + i * 32 + fr;
+            if (t >= T) continue;
+            const long long at = dn_orow(g, row0, t, T) * g.ldo + n0 + wn * NJ * 32 + 4 * fh;
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (n0 + wn * NJ * 32 + j * 32 + 8 * q + 4 * fh >= g.N) continue;
+                    dn_f4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * q + e] * g.alpha;
+                    if (g.out16) {
+                        dn_us4 r;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) r[e] = dn_f2bf(v[e]);
+                        *(dn_us4 *)(g.out16 + at + j * 32 + 8 * q) = r;
+                    } else {
+                        *(dn_f4 *)(g.out + at + j * 32 + 8 * q) = v;
+                    }
+                }
+        }
+        return;
+    }
+    // the tile through LDS (the stages are done with), so that the loading waves have their part in the epilogue
     constexpr int LD = BN + 4;
     float *tile = (float *)dn_lds;
     __syncthreads();
@@ -722,7 +738,8 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
 #pragma unroll
             for (int j = 0; j < NJ; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) tile[(wm * MI * 32 + i * 32 + 8 * (r >> 2) + 4 * fh + (r & 3)) * LD + wn * NJ * 32 + j * 32 + fr] = acc[i][j][r];
+                for (int q = 0; q < 4; q++)
+                    *(dn_f4 *)&tile[(wm * MI * 32 + i * 32 + fr) * LD + wn * NJ * 32 + j * 32 + 8 * q + 4 * fh] = dn_f4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
     }
     __syncthreads();
     const int c = (tid % (BN / 4)) * 4;
@@ -732,18 +749,21 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     }
 }
 
-// the splits of a tile, added in order: one work-group per quarter of the 32 x 32 instruction tiles ij of its four waves (the D registers 4 q .. 4 q + 3 of each lane).  A work-group that
-// took whole instruction tiles had one wave per SIMD of 256 CUs at work and sixteen columns of a row to write one behind the other: 14 us for the splits of
-// 512 x 2048, 16 for those of 512 x 8; 6.9 and 5.3 now.
+// the splits of a tile, added in order: one work-group per 32 x 32 instruction tile ij of a wave, read as it was written (a kilobyte per wave-instruction) and turned in LDS, so that
+// eight lanes have 128 bytes of a row of the result: 7.5 us, the mean of a mixture-of-experts prompt's launches.  Eight lanes per row in the reading as well took 10.3 (128-byte pieces),
+// a lane's registers straight to the result 10.3 too (32-byte pieces).
+// A work-group that took the tiles of all four waves had one wave per SIMD of 256 CUs at work and sixteen columns of a row to write one behind the other: 14 us for
+// the splits of 512 x 2048, 16 for those of 512 x 8; 5.7 and 4.8 now.
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p) {
     constexpr int MI = BM / 64, NJ = BN / 64, IJ = MI * NJ;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, q = (int)blockIdx.x & 3, ij = (int)(blockIdx.x >> 2) % IJ, tile = (int)(blockIdx.x >> 2) / IJ,
-              tm = tile / p.tn, tn = tile % p.tn;
+    __shared__ __attribute__((aligned(16))) float turn[32 * 36];
+    const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6, wave = (int)blockIdx.x & 3, wm = wave >> 1, wn = wave & 1; // (read: D registers 4 q .. 4 q + 3 of `lane`)
+    const int ij = (int)(blockIdx.x >> 2) % IJ, tile = (int)(blockIdx.x >> 2) / IJ, tm = tile / p.tn, tn = tile % p.tn;
     int e, T, t0;
     long long row0;
     if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return;
-    const float *src = p.part + (long long)tile * p.S * (IJ * 4096) + ij * 4096 + q * 1024 + tid * 4;
+    const float *src = p.part + (long long)tile * p.S * (IJ * 4096) + ij * 4096 + (q * 256 + wave * 64 + lane) * 4;
     dn_f4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < p.S; s += 8) { // (eight loads in flight)
         dn_f4 v[8];
@@ -753,7 +773,10 @@ __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p)
         for (int u = 0; u < 8; u++)
             if (s + u < p.S) acc += v[u];
     }
-    dn_put4r(g, row0, T, t0 + wm * MI * 32 + (ij / NJ) * 32 + 4 * (lane >> 5) + 8 * q, (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + (lane & 31), acc);
+    *(dn_f4 *)&turn[(lane & 31) * 36 + 8 * q + 4 * (lane >> 5)] = acc;
+    __syncthreads();
+    const int r = tid >> 3, c = (tid & 7) * 4, t = t0 + wm * MI * 32 + (ij / NJ) * 32 + r;
+    if (t < T) dn_put4(g, dn_orow(g, row0, t, T), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + c, *(const dn_f4 *)&turn[r * 36 + c]);
 }
 
 // Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block

@@ -228,6 +228,14 @@ def test_bf16_rows_handed_on(made, sizes):
     assert err(got, want) < 1.5 * err(plain, want) < 0.3
 
 
+# results without an epilogue (k_dense.hip dense_mm_ring_kernel): columns in fours, stored from the registers, the last four of a tile, one four and three fours into the next one; no fours
+# (through LDS); split along K, where the sums are stored in fours or one by one
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,N,K", [(9, 4, 64), (65, 60, 128), (130, 132, 192), (513, 2060, 128), (130, 134, 192), (33, 36, 4160), (31, 68, 4096), (40, 102, 4160)])
+def test_dense_matmul_stored_in_fours(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
 # K up to 32 (k_dense.hip dense_mm_few_kernel): one below, at and above its two widths (33: the tiled kernel), one token and one column more and less than a work-group's
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(9, 1, 1), (15, 255, 7), (16, 256, 8), (17, 257, 9), (33, 70, 31), (31, 513, 32), (40, 65, 33)])
