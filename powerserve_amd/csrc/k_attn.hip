@@ -8,6 +8,7 @@
 //   attn_scores      s = K·q       (ggml_vec_dot_f32, libs/ggml/src/ggml.c:2092-2133)
 //   attn_softmax_pv  scale + mask + softmax (ggml.c:14889-14925, ggml_vec_soft_max_f32 :2814-2863) held in LDS,
 //                    then out = V·p (ggml_vec_dot_f32 again, rows of the transposed V cache)
+// (a single token: all three in one launch, attn_decode1_kernel, or the last two, attn_decode2_kernel)
 // KV layout is the reference's: K [n_ctx][kv_dim], V [kv_dim][n_ctx] FP32 (backend/ggml/ggml_kv_cache.cpp:48-57).
 //
 // Exact order: ggml_vec_dot_f32's AVX build keeps 4 accumulators x 8 lanes = 32 fp32 chains over elements
@@ -824,6 +825,229 @@ __global__ __launch_bounds__(NT) void attn_decode2_kernel(psl_attn_args a) {
     if (dbg) { dbg[10] = __builtin_amdgcn_s_memtime(); dbg[30] = __builtin_amdgcn_s_memrealtime(); }
 }
 
+// ---------------------------------------------------------------- single token: RoPE + KV append + scores + soft-max + V.p in ONE launch, nothing exchanged
+// attn_decode1_kernel: work-group (head h, block of `ch` channels) makes ALL scores of its head, its soft-max and the V.p of its channels.  The scores of a head are made hs / ch times -- from
+// the L2s, where a kv head's K rows are after the first reading -- which up to a few thousand positions costs less than what it replaces: the boundary of a launch (about 4 us of a captured step each
+// for rotation, scores and soft-max.V.p) or attn_decode2_kernel's exchange, and it needs neither residency nor groups of at most four heads.
+//   t = 0    position, q, k, v of the step and the cached rows the host knows of (psl_attn_args::n_kv_lo: a hint) in one go
+//   rotate   q and (every work-group for itself: the new position's score needs it) k into LDS, ps_rope_pair as in rope_append_kernel; the first head of a kv head stores the K row and its V channels
+//   scores   eight lanes per position, four of ggml_vec_dot_f32's chains each (as in attn_decode2_kernel); straight to LDS, scaled and masked
+//   soft-max ggml_v_expf on groups of 8 with the in-group sum tree, libm's expf on the n % 8 tail, a lane each; double sums (attn_softmax_rows)
+//   V.p      a lane per (chain, channel): 32 chains over columns 32 i + c, GGML_F32x8_REDUCE, the n % 32 leftovers in order (attn_softmax_pv_kernel)
+// grid: hs / ch x n_heads; 512 threads.  dynamic LDS: n_ctx floats rounded up to 32, and 32 more (masked reads of a full window's last group)
+constexpr int D1_NT = 512, D1_PASSES = 4, D1_VPRE = 16; // a pass of the scores: 64 positions; V blocks of 32 positions requested up front
+template <int NV>
+__global__ __launch_bounds__(D1_NT) void attn_decode1_kernel(psl_attn_args a, int ch, int rope) {
+    extern __shared__ __attribute__((aligned(16))) float pl[]; // [n_ctx] logits, then e_j
+    constexpr int hs = NV * 32, NW = D1_NT / 64, SP = NW * 8; // SP: positions per pass
+    __shared__ __attribute__((aligned(16))) float qs[hs], ks[hs], vl[16 * 36];
+    __shared__ float redf[NW];
+    __shared__ double redd[NW];
+    __shared__ uint64_t etab[PS_EXP2F_N];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), p8 = lane >> 3, tq = lane & 7;
+    const int nb = hs / ch, h = (int)blockIdx.x / nb, bx = (int)blockIdx.x % nb, r2 = a.n_heads / a.n_kv_heads, kvh = h / r2, kvd = a.n_kv_heads * hs;
+    const bool owner = rope && h % r2 == 0; // stores the new position's V channels, and (first block of channels) its K row
+    const float *const sq = a.q + (int64_t)h * hs, *const sk = a.k + (int64_t)kvh * hs, *const sv = a.v + (int64_t)kvh * hs + bx * ch;
+
+    // ---- t = 0: the position, what the step's mat-vec left, and the cached rows in front of the hint (clamped: a row behind the cache length is fetched and not used)
+    const int pos0 = att_pos0(a), rp = a.rope_pos ? a.rope_pos[0] : pos0;
+    const int nlo = a.n_kv_lo, half = a.n_dims / 2;
+    const bool rot_k = tid >= 64; // threads 0 .. hs / 2 - 1: pairs of q, 64 .. 64 + hs / 2 - 1: pairs of k
+    const int pi = tid & 63, i0 = 2 * pi;
+    const bool pair = tid < 128 && pi < hs / 2, turns = rope && i0 < a.n_dims;
+    const int ia = turns && a.neox ? pi : i0, ib = turns && a.neox ? pi + half : i0 + 1;
+    const float *src = rot_k ? sk : sq;
+    const float x0 = src[pair ? ia : 0], x1 = src[pair ? ib : 0];
+    const uint64_t et_w = ps_exp2f_tab[tid & (PS_EXP2F_N - 1)];
+    const int c = tid & 31, slot = tid >> 5; // V.p: chain and channel (16 channels at a time)
+    const float *const vbase = a.v_cache + ((int64_t)kvh * hs + bx * ch) * a.n_ctx;
+    const float *const vr0 = vbase + (int64_t)(slot < ch ? slot : 0) * a.n_ctx;
+    const float *const kb = a.k_cache + kvh * hs + 4 * tq;
+    float4 kf[D1_PASSES][NV];
+    auto k_pass = [&](const int ps, const int j0) { // this wave's eight positions j0 .. j0 + 7
+        const float *kr = kb + (int64_t)min(j0 + p8, a.n_ctx - 1) * kvd;
+#pragma unroll
+        for (int m = 0; m < NV; m++) kf[ps][m] = *(const float4 *)(kr + m * 32);
+    };
+    float vf[D1_VPRE];
+    auto v_block = [&](const float *vr, const int k) { return vr[min(32 * k + c, a.n_ctx - 1)]; };
+    const bool k_early = nlo > SP * (D1_PASSES - 2), v_early = nlo > 32; // (uniform)
+    if (k_early)
+#pragma unroll
+        for (int ps = 0; ps < D1_PASSES; ps++) k_pass(ps, ps * SP + wave * 8);
+    if (v_early) {
+#pragma unroll
+        for (int k = 0; k < D1_VPRE; k++) vf[k] = 32 * k <= nlo + 32 ? v_block(vr0, k) : 0.f; // (uniform)
+    }
+    // ---- everything below depends on the position
+    const int n_kv = pos0 + 1, n8 = n_kv & ~7, np = n_kv & ~31, ntail = n_kv - n8, nleft = n_kv - np;
+    if (!k_early)
+#pragma unroll
+        for (int ps = 0; ps < D1_PASSES; ps++)
+            if (ps * SP + wave * 8 < n_kv) k_pass(ps, ps * SP + wave * 8); // (uniform)
+#pragma unroll
+    for (int k = 0; k < D1_VPRE; k++)
+        if (!(v_early && 32 * k <= nlo + 32)) vf[k] = 32 * k < n_kv ? v_block(vr0, k) : 0.f; // (uniform)
+    if (pair) {
+        float ra = x0, rb = x1;
+        if (turns) ps_rope_pair(x0, x1, a.rope_table[(int64_t)rp * hs + i0], a.rope_table[(int64_t)rp * hs + i0 + 1], ra, rb);
+        float *const to = rot_k ? ks : qs;
+        to[ia] = ra;
+        to[ib] = rb;
+        if (rot_k && owner && bx == 0) {
+            float *const row = a.k_cache + (int64_t)pos0 * kvd + kvh * hs;
+            row[ia] = ra;
+            row[ib] = rb;
+        }
+    }
+    if (owner && tid < ch) a.v_cache[((int64_t)kvh * hs + bx * ch + tid) * a.n_ctx + pos0] = sv[tid];
+    if (tid < PS_EXP2F_N) etab[tid] = et_w;
+    __syncthreads();
+
+    // ---- scores (ggml_vec_dot_f32, ggml.c:2092-2133, GGML_F32x8_REDUCE :1354-1371), scaled and masked (softmax_ext :14889-14914), and the row's maximum
+    float4 qv[NV];
+#pragma unroll
+    for (int m = 0; m < NV; m++) qv[m] = *(const float4 *)(qs + m * 32 + 4 * tq);
+    float lmax = -INFINITY;
+    auto score = [&](const int ps, const int j) {
+        float x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NV; m++) {
+            const float4 kv = kf[ps][m];
+            x[0] = __fmaf_rn(kv.x, qv[m].x, x[0]); // sum = x*y + sum, x = K row (src0)
+            x[1] = __fmaf_rn(kv.y, qv[m].y, x[1]);
+            x[2] = __fmaf_rn(kv.z, qv[m].z, x[2]);
+            x[3] = __fmaf_rn(kv.w, qv[m].w, x[3]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = __fadd_rn(x[e], dpp_f<0x104>(x[e])); // tq < 4: + lane tq + 4
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = __fadd_rn(x[e], dpp_f<0x102>(x[e])); // tq < 2: + lane tq + 2
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = __fadd_rn(x[e], dpp_f<0x101>(x[e])); // tq = 0: + lane 1
+        const float s = __fmul_rn(__fadd_rn(__fadd_rn(x[0], x[1]), __fadd_rn(x[2], x[3])), a.scale);
+        if (tq == 0 && j < n_kv) {
+            pl[j] = s;
+            lmax = fmaxf(lmax, s);
+        }
+    };
+    int base = 0;
+    for (; base + SP * D1_PASSES < n_kv; base += SP * D1_PASSES) { // (no branch around a request: the waits stay counts, and a chunk of 256 positions is in flight)
+#pragma unroll
+        for (int ps = 0; ps < D1_PASSES; ps++) {
+            const int j0 = base + ps * SP + wave * 8;
+            score(ps, j0 + p8);
+            k_pass(ps, j0 + SP * D1_PASSES);
+        }
+    }
+#pragma unroll
+    for (int ps = 0; ps < D1_PASSES; ps++) {
+        const int j0 = base + ps * SP + wave * 8;
+        if (rope && j0 <= pos0 && pos0 < j0 + 8 && p8 == pos0 - j0) // the new position's row may not be in the cache yet
+#pragma unroll
+            for (int m = 0; m < NV; m++) kf[ps][m] = *(const float4 *)(ks + m * 32 + 4 * tq);
+        if (j0 < n_kv) score(ps, j0 + p8); // (uniform)
+    }
+    if (a.kv_vis) { // (uniform) hidden cache slots (KVCacheInterface::mask): -inf before the maximum
+        __syncthreads();
+        lmax = -INFINITY;
+        for (int j = tid; j < n_kv; j += D1_NT) {
+            const float s = __fadd_rn(pl[j], j < pos0 && a.kv_vis[j] == 0 ? -INFINITY : 0.f);
+            pl[j] = s;
+            lmax = fmaxf(lmax, s);
+        }
+    }
+    {
+        const float wm = wave_max_dpp(lmax);
+        if (lane == 0) redf[wave] = wm;
+    }
+    const float v_new = rope ? sv[slot < ch ? slot : 0] : 0.f;
+    { // the V columns behind the last whole block: first 16 channels
+        float v = c < nleft ? vr0[np + c] : 0.f;
+        if (rope && c == nleft - 1) v = v_new;
+        vl[slot * 36 + c] = v;
+    }
+    __syncthreads();
+    // ---- e_j = exp(x_j - max), double sums (ggml_vec_soft_max_f32, ggml.c:2831-2866)
+    float mx = redf[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) mx = fmaxf(mx, redf[w]);
+    double rs = 0.0;
+    for (int j = tid * 8; j < n8; j += D1_NT * 8) {
+        const float4 lo = *(const float4 *)(pl + j), hi = *(const float4 *)(pl + j + 4);
+        float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        ps_v_expf_n<8>(v, mx);
+        *(float4 *)(pl + j)     = make_float4(v[0], v[1], v[2], v[3]);
+        *(float4 *)(pl + j + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        const float a0 = __fadd_rn(v[4], v[0]), a1 = __fadd_rn(v[5], v[1]), a2 = __fadd_rn(v[6], v[2]), a3 = __fadd_rn(v[7], v[3]);
+        rs += (double)__fadd_rn(__fadd_rn(a0, a2), __fadd_rn(a1, a3));
+    }
+    if (D1_NT - 1 - tid < ntail) {
+        const int j = n8 + D1_NT - 1 - tid;
+        const float e = ps_expf_glibc(__fsub_rn(pl[j], mx), etab);
+        pl[j] = e;
+        rs += (double)e;
+    }
+    {
+        const double sw = wave_sum_d_dpp(rs);
+        if (lane == 0) redd[wave] = sw;
+    }
+    __syncthreads();
+    double tot = redd[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) tot += redd[w];
+    const float inv = (float)(1.0 / tot);
+
+    // ---- V.p: out = ggml_vec_dot_f32(V[channel], p), p_j = e_j * (float)(1/sum) formed where it is used
+    for (int cb = 0; cb < ch; cb += 16) { // (uniform)
+        const float *const vr = cb == 0 ? vr0 : vbase + (int64_t)(cb + slot < ch ? cb + slot : 0) * a.n_ctx;
+        const float vn = cb == 0 ? v_new : rope ? sv[cb + slot < ch ? cb + slot : 0] : 0.f;
+        if (cb > 0) {
+#pragma unroll
+            for (int k = 0; k < D1_VPRE; k++)
+                if (32 * k < np) vf[k] = v_block(vr, k); // (uniform)
+            float v = c < nleft ? vr[np + c] : 0.f;
+            if (rope && c == nleft - 1) v = vn;
+            __syncthreads(); // (the leftovers of the channels before are read)
+            vl[slot * 36 + c] = v;
+            __syncthreads();
+        }
+        float acc = 0.f;
+        int k0 = 0;
+        for (; 32 * (k0 + D1_VPRE) < np; k0 += D1_VPRE) { // sixteen blocks in flight
+            float e[D1_VPRE];
+#pragma unroll
+            for (int k = 0; k < D1_VPRE; k++) e[k] = pl[32 * (k0 + k) + c];
+#pragma unroll
+            for (int k = 0; k < D1_VPRE; k++) {
+                acc = __fmaf_rn(vf[k], __fmul_rn(e[k], inv), acc); // x = V row (src0), y = p
+                vf[k] = v_block(vr, k0 + k + D1_VPRE);
+            }
+        }
+        float e[D1_VPRE];
+#pragma unroll
+        for (int k = 0; k < D1_VPRE; k++) e[k] = pl[min(32 * (k0 + k), np) + c]; // (np + 31: inside the row's length in LDS)
+#pragma unroll
+        for (int k = 0; k < D1_VPRE; k++) {
+            const int j = 32 * (k0 + k);
+            if (j < np) acc = __fmaf_rn(rope && j + c == pos0 ? vn : vf[k], __fmul_rn(e[k], inv), acc); // (uniform)
+        }
+        float res = reduce_f32x8x4(acc);
+        if (nleft > 0) { // (uniform) leftovers, in order
+            float lv[32], lp[32];
+#pragma unroll
+            for (int jj = 0; jj < 32; jj += 4) {
+                *(float4 *)(lv + jj) = *(const float4 *)(vl + slot * 36 + jj);
+                *(float4 *)(lp + jj) = *(const float4 *)(pl + np + jj); // (np + 32 <= the row's length in LDS; entries past the cache length are never added)
+            }
+#pragma unroll
+            for (int jj = 0; jj < 32; jj++)
+                if (jj < nleft) res = ps_dot_left(res, lv[jj], __fmul_rn(lp[jj], inv), jj, nleft); // (uniform)
+        }
+        if (c == 0 && cb + slot < ch) a.att[(int64_t)h * hs + bx * ch + cb + slot] = res;
+    }
+}
+
 // Batches (prefill chunks, tree verify): one workgroup per (kv head, CI batch columns).  The softmax of a row is computed
 // once (not once per channel tile as in the single-token kernel, whose grid has to fill the chip from one column), and a
 // V element fetched from L2 serves r2 heads x CI columns.  thread: chain c = tid & 31, channels (tid >> 5) + 32k.
@@ -1431,10 +1655,14 @@ bool psl_attn_decode_f16(hipStream_t st, const psl_attn_args &a) {
 
 // single token, one launch (attn_decode2_kernel); false: not covered, the caller launches scores + softmax / V.p
 size_t psl_attn_decode2_xchg_bytes(int n_kv_heads, int n_ctx) { return (size_t)n_kv_heads * 4 * (((size_t)n_ctx + 31) & ~(size_t)31) * 4; }
-bool psl_attn_decode2(hipStream_t st, int n_cu, const psl_attn_args &a) {
+bool psl_attn_decode2_covers(int n_cu, const psl_attn_args &a) {
     const int r2 = a.n_heads / a.n_kv_heads, gx = a.head_size / 4;
     if (!a.xchg || !a.tick || !a.sync || a.tree || r2 > 4 || a.n_kv_heads > 32 || a.n_ctx > D2_MAXCTX || (a.head_size != 128 && a.head_size != 64)) return false;
-    if (gx * a.n_kv_heads > n_cu) return false; // every workgroup resident (one per CU at n_ctx = 4096)
+    return gx * a.n_kv_heads <= n_cu; // every workgroup resident (one per CU at n_ctx = 4096)
+}
+bool psl_attn_decode2(hipStream_t st, int n_cu, const psl_attn_args &a) {
+    if (!psl_attn_decode2_covers(n_cu, a)) return false;
+    const int gx = a.head_size / 4;
     const int RS = ((a.n_ctx + 127) & ~127) + 36;
     const size_t lds = ((size_t)8 * RS + 512 + 128 + 16 + 32 + 4 * a.head_size + (16 * 32 / (a.head_size / 32)) * 4 + 32 + 64) * 4;
     static unsigned long long attr = 0; // devices that have the attribute
@@ -1464,6 +1692,32 @@ bool psl_attn_decode2(hipStream_t st, int n_cu, const psl_attn_args &a) {
     if (a.head_size == 128) { if (a.kv_stream) hipLaunchKernelGGL((attn_decode2_kernel<4, 1024, 1>), g, dim3(1024), lds, st, a); else hipLaunchKernelGGL((attn_decode2_kernel<4, 1024, 0>), g, dim3(1024), lds, st, a); }
     else { if (a.kv_stream) hipLaunchKernelGGL((attn_decode2_kernel<2, 1024, 1>), g, dim3(1024), lds, st, a); else hipLaunchKernelGGL((attn_decode2_kernel<2, 1024, 0>), g, dim3(1024), lds, st, a); }
     return true;
+}
+
+// Single token, one launch (attn_decode1_kernel), as long as a work-group's reading of its head's K rows costs less than the two launches it saves: up to 160 K floats of them.  Us per token of
+// two layers, rotation + scores + soft-max.V.p | one launch, at 100, 1000, 2000 and 4000 positions: 14 heads of 64 over 2 kv heads 87.8 93.7 98.2 109.3 | 71.9 79.0 87.7 106.0;
+// 12 of 128 over 2: 92.1 98.6 102.7 115.9 | 76.9 89.0 102.7 124.4; 28 of 128 over 4: 113.9 121.8 128.5 142.4 | 98.3 112.7 123.6 146.8; 32 of 96 over 32: 125.4 140.3 145.0 166.9 | 106.0 127.9 149.2 198.8
+bool psl_attn_decode1_covers(const psl_attn_args &a) {
+    return !a.tree && !a.k16 && a.head_size % 32 == 0 && a.head_size <= 128 && a.n_dims <= a.head_size && a.n_ctx <= 32768 && (int64_t)a.n_kv_hi * a.head_size <= 160 * 1024;
+}
+void psl_attn_decode1(hipStream_t st, int n_cu, const psl_attn_args &a, bool rope) {
+    // channels per work-group: four (the shortest V.p) where the heads' work-groups then fit on the chip side by side, else as many more as it takes
+    int nb = a.head_size / 4;
+    while (nb % 2 == 0 && nb * a.n_heads > n_cu) nb /= 2;
+    const int ch = a.head_size / nb;
+    const dim3 g((unsigned)(nb * a.n_heads)), b(D1_NT);
+    const size_t lds = ((((size_t)a.n_ctx + 31) & ~(size_t)31) + 32) * 4;
+    static unsigned long long attr = 0; // devices that have the attribute
+    if (ps_first_on_device(&attr)) {
+        (void)hipFuncSetAttribute((const void *)attn_decode1_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 132 * 1024);
+        (void)hipFuncSetAttribute((const void *)attn_decode1_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 132 * 1024);
+        (void)hipFuncSetAttribute((const void *)attn_decode1_kernel<3>, hipFuncAttributeMaxDynamicSharedMemorySize, 132 * 1024);
+        (void)hipFuncSetAttribute((const void *)attn_decode1_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, 132 * 1024);
+    }
+    if (a.head_size == 128) hipLaunchKernelGGL(attn_decode1_kernel<4>, g, b, lds, st, a, ch, (int)rope);
+    else if (a.head_size == 96) hipLaunchKernelGGL(attn_decode1_kernel<3>, g, b, lds, st, a, ch, (int)rope);
+    else if (a.head_size == 64) hipLaunchKernelGGL(attn_decode1_kernel<2>, g, b, lds, st, a, ch, (int)rope);
+    else hipLaunchKernelGGL(attn_decode1_kernel<1>, g, b, lds, st, a, ch, (int)rope);
 }
 
 void psl_argmax2(hipStream_t st, const float *src, int64_t n, int64_t rows, int32_t *out, float *part_v, int *part_i,

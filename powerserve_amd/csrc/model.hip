@@ -3,7 +3,7 @@
 // src/model/module/norm_attention.cpp:26-160; FFN::build, src/model/module/ffn.cpp:22-42).
 //
 // Launch plan per layer (single token, Q4_K, the headline's shape):
-//   [matvec[Wq|Wk|Wv] + RMSNorm + quantizer + RoPE + KV append + attention]  (k_qkvattn.hip; elsewhere the mat-vec, then attn_decode2 or scores + soft-max.V.p)
+//   [matvec[Wq|Wk|Wv] + RMSNorm + quantizer + RoPE + KV append + attention]  (k_qkvattn.hip; elsewhere the mat-vec, then attn_decode2, attn_decode1 or scores + soft-max.V.p)
 //   -> matvec[Wo] + quantizer + residual -> matvec[Wgate|Wup] + RMSNorm + quantizer + SiLU*up -> matvec[Wdown] + quantizer + residual
 // Batches: quantize_act(rmsnorm) -> mat-mul[Wq|Wk|Wv] -> rope_append -> attn_scores -> soft-max -> V.p (+ quantize) -> mat-mul[Wo] + residual
 //   -> quantize_act(rmsnorm) -> mat-mul[Wgate|Wup] SiLU*up -> quantize_act -> mat-mul[Wdown] + residual
@@ -60,6 +60,8 @@ struct ps_hip_model {
     float *attn_xchg = nullptr;    // attn_decode2: scores in flight between workgroups (k_attn.hip)
     unsigned *attn_tick = nullptr; // attn_decode2: [64 * kv head] arrival counters
     size_t graph_hint = 0;                   // KV position the captured step was given as its prefetch hint (n_kv_lo)
+    size_t graph_hi = 0;           // ... and the cache length it may be replayed to (which attention launch a long cache gets depends on it)
+    int n_kv_bound = 0;            // cache length the step being enqueued may be replayed to (0: n_ctx)
     int n_kv_hint = 0;             // capture of a single-token forward: the lower bound of n_kv its prefetch hint is baked with
     int n_kv_host = 0;             // pos0 + bs of the forward being enqueued eagerly (0 while a graph is captured / replayed)
     float *scores = nullptr, *logits = nullptr, *rope_table = nullptr;
@@ -290,6 +292,8 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
     aa.kv_stream = kvs_own;
     aa.n_kv_lo = m->n_kv_host > 0 ? m->n_kv_host : (m->n_kv_hint > 0 ? m->n_kv_hint : (int)m->position); // (a hint: rows below it are requested before the device-side position has arrived)
 
+    aa.n_kv_hi = m->n_kv_host > 0 ? m->n_kv_host : m->n_kv_bound > 0 ? m->n_kv_bound : (int)f.seq_len;
+
     for (uint32_t L = 0; L < f.n_layers; L++) {
         ps_act a1 = act_for(dim);
         psk_gemv_args g{};
@@ -332,9 +336,14 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         } else if (mm(m, g, a1, dim, bs)) return 2;
 
         aa.kv_stream = kvs_own; aa.dbg = nullptr; // (also when the fused launch declined the shape)
-        if (f16 || (!fuse_rope && !fuse_rope_b)) psl_rope_append(st, aa, bs);
+        // a single token's attention where attn_decode2 does not take it: rotation, append and attention in one launch
+        const bool rotate = f16 || (!fuse_rope && !fuse_rope_b);
+        const bool one = bs == 1 && !use_tree && one_launch && !fused_qa && !kv16 && !psl_attn_decode2_covers(c->n_cu, aa) && psl_attn_decode1_covers(aa);
+        if (rotate && !one) psl_rope_append(st, aa, bs);
         bool att_quantized = false;
         if (fused_qa) {
+        } else if (one) {
+            psl_attn_decode1(st, c->n_cu, aa, rotate);
         } else if (bs == 1 && !use_tree && kv16 && psl_attn_decode_f16(st, aa)) {
             // fp16-KV decode mode (not bit-exact): split-KV online soft-max over the fp16 mirrors
         } else if (bs == 1 && !use_tree && one_launch && (aa.dbg = psk_gemv_dbg_buf(10, 2), psl_attn_decode2(st, c->n_cu, aa))) { // timeline key 42
@@ -702,11 +711,11 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
         if (graphable) { // capture the same launches (nothing executes); the hint stays a lower bound of n_kv for 1024 positions
             hipGraph_t g = nullptr;
             PS_CHECK(c, hipStreamSynchronize(c->stream));
-            m->n_kv_host = 0; m->n_kv_hint = pos[0]; // (no host-side n_kv inside a graph: the score grids cover n_ctx)
+            m->n_kv_host = 0; m->n_kv_hint = pos[0]; m->n_kv_bound = std::min(pos[0] + 1024, (int)m->cfg.seq_len); // (no host-side n_kv inside a graph: the score grids cover n_ctx)
             PS_CHECK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             const int rc = enqueue_forward(m, 1, lm_head != 0, false);
             const hipError_t e = hipStreamEndCapture(c->stream, &g);
-            m->n_kv_hint = 0;
+            m->n_kv_hint = 0; m->n_kv_bound = 0;
             if (!rc && e == hipSuccess && hipGraphInstantiate(&m->fwd1_graph[gk], g, nullptr, nullptr, 0) == hipSuccess) m->fwd1_hint[gk] = (size_t)pos[0];
             else m->fwd1_graph[gk] = nullptr; // (stay eager)
             if (g) (void)hipGraphDestroy(g);
@@ -843,7 +852,11 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
     // is not far behind (a stale hint costs time, never results)
-    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024)) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
+    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024 || m->position + (size_t)steps > m->graph_hi)) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
+    const size_t hi_now = std::min<size_t>(m->position + std::max<size_t>(1024 + 64, (size_t)steps), m->cfg.seq_len); // (64: a call of a few tokens late in the 1024)
+    if (!m->step_graph) m->graph_hi = hi_now;
+    m->n_kv_bound = (int)m->graph_hi;
+    const struct bound_guard { ps_hip_model *m; ~bound_guard() { m->n_kv_bound = 0; } } bound{m};
     if ((m->mode & 1) == 0 && !m->step_graph) {
         // first step runs eagerly (also performs every one-time hipFuncSetAttribute), then the identical
         // launch sequence is captured; capture itself executes nothing

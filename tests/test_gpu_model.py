@@ -399,6 +399,52 @@ def test_chunks_attended_in_one_launch(ctx, tmp_path, preset, wt, chunk, P, n_ct
         assert np.array_equal(k0.view(np.uint32), k1.view(np.uint32)) and np.array_equal(v0.view(np.uint32), v1.view(np.uint32))
 
 
+@pytest.mark.parametrize("preset,wt,n_ctx", [("odd-llama-hs96", 8, 200), ("odd-llama-hs32", 2, 352), ("odd-llama-r5", 8, 100), ("odd-llama-r6", 8, 1280), ("odd-llama-r8", 2, 544),
+                                             ("qwen2-0.5b-dims-2l", 8, 1100)])
+def test_single_token_attention_without_exchange(ctx, tmp_path, preset, wt, n_ctx):
+    """k_attn.hip attn_decode1_kernel (rotation, append, scores, soft-max and V.p of a token in one launch) against the separate launches, on bits: logits, the new K row and V column; an empty
+    cache, one position around the groups of 8, blocks of 32, a pass of 64, the 256 positions and the 512 columns requested up front, a full window (multiples of 32 and not), both rotations,
+    four to 32 channels per work-group, head sizes 32 to 128, groups of 1 to 8 heads; eager, captured and behind hidden positions."""
+    from powerserve_amd import hip, synth
+    d = str(tmp_path / "m")
+    mj = synth.write_model_dir(d, preset, wt, n_ctx=n_ctx, seed=5)
+    toks = np.random.default_rng(n_ctx).integers(0, mj["llm_config"]["vocab_size"], n_ctx)
+    gm = hip.Model(ctx, d, max_batch=64, n_ctx=n_ctx)
+
+    def step(mode, P, hide):
+        gm.set_mode(mode)
+        for i in hide:
+            gm.kv_mask(i, False)
+        got, _ = gm.forward([int(toks[P])], [P], True)
+        out = [got.copy()] + [x for L in range(gm.cfg.n_layers) for x in (gm.k_cache(L)[:P + 1].copy(), gm.v_cache(L)[:, :P + 1].copy())]
+        gm.kv_rollback(1)
+        for i in hide:
+            gm.kv_mask(i, True)
+        return out
+
+    at = 0
+    for P in sorted({p for e in (8, 32, 64, 256, 512) for p in (e - 1, e, e + 1)} | {0, 1, n_ctx - 1}):
+        if P >= n_ctx:
+            continue
+        if P > at:
+            gm.set_mode(0)
+            gm.prefill(toks[at:P], 64)
+            at = P
+        for hide in ((), (0, P // 2)) if P > 1 else ((),):
+            want = step(16, P, hide)
+            for mode in (0, 0, 1):  # (the second call of a mode is a replay)
+                for w, g in zip(want, step(mode, P, hide)):
+                    assert np.array_equal(w.view(np.uint32), g.view(np.uint32)), (P, mode, hide)
+        if P + 5 <= n_ctx:
+            ids = []
+            for mode in (0, 16):
+                gm.set_mode(mode)
+                ids.append(gm.decode_greedy(int(toks[P]), 5).tolist())
+                gm.kv_rollback(5)
+            assert ids[0] == ids[1], P
+    gm.close()
+
+
 @pytest.mark.parametrize("preset,wt,chunk", [("small-llama-hs128", 12, 256), ("small-llama-hs128", 12, 512), ("small-llama-hs128", 1015, 384), ("tiny-llama", 8, 256), ("tiny-qwen2", 2, 320)])
 def test_wide_prefill_chunks_match_oracle(ctx, oracle, tmp_path, preset, wt, chunk):
     """hparams batch_size above the reference's default of 128 (bench.py reports a 512-token-chunk prefill next to the headline):
