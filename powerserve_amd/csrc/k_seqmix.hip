@@ -19,14 +19,6 @@ static __device__ __forceinline__ float sq_block_sum(float v, float *red) { // 2
     return red[0] + red[1] + red[2] + red[3];
 }
 typedef float sq_f4 __attribute__((ext_vector_type(4)));
-static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane gets it: rotations inside a row of sixteen, then the four rows' sums (no trip through LDS)
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));
-    auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
-    return (row(0) + row(16)) + (row(32) + row(48));
-}
 typedef unsigned short sq_us4 __attribute__((ext_vector_type(4)));
 static __device__ __forceinline__ unsigned short sq_bf16(float f) { // round to nearest even, as the mat-mul's own copy of its operand does
     unsigned u = __float_as_uint(f);

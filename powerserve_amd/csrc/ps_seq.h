@@ -124,6 +124,14 @@ void psk_mingru_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off,
 // (a residual around the convolution), mode 1: f = silu(sum + bias[c]) (bias NULL: none).  The tail is brought up to date behind it.
 bool psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, const float *in, int64_t ldi, const float *w, int taps, int mode,
                      int64_t C, int T, float *out, int64_t ldo, const float *bias = nullptr, uint16_t *copy16 = nullptr);
+static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane gets it: rotations inside a row of sixteen, then the four rows' sums (no trip through LDS)
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));
+    auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    return (row(0) + row(16)) + (row(32) + row(48));
+}
 // One token's sublayer boundary fused: x += norm_b(y) (y may be NULL), then h = conv(norm(x)) in the residual form with the tail update (wn may be NULL: stop after x);
 // hn (may be NULL) also receives norm(x) itself, for a sublayer that reads the unfiltered input
 void psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
@@ -191,9 +199,12 @@ void psk_delta_chunked(hipStream_t st, const ps_seq_step *step, int64_t state_of
 // with n_groups > 0 only rows of the `keep` groups (equal runs of neighbours) with the largest best choice score stay in the race; the `top` largest choice scores
 // (ties: the lower index) -> sel[t top + i], wgt[t top + i] (their SCORES, divided by their sum where norm_top, times scale); sgate[t] = sigmoid(shared_gate . h[t]) where given.
 // bias (NULL: none) joins the logits.  softmax 2: the logits themselves are the scores of the choice, and the weights are the soft-max over the chosen logits alone, times scale.
+// front (one token): first x += y / rms(y) * (offset + w), in the same launch; h is that x.  psk_moe_front_ok: whether it can be taken along.
+struct psk_moe_front { float *x; const float *y, *w; float offset, eps; };
+bool psk_moe_front_ok(const psk_moe_front &f, const float *router, const float *shared_gate, int experts, int64_t K);
 void psk_moe_route(hipStream_t st, const float *h, int64_t ldh, const float *router, const float *shared_gate, int experts, int top, int norm_top, int64_t K, int T,
                    int32_t *sel, float *wgt, float *sgate, int softmax = 0, const float *correction = nullptr, int n_groups = 0, int keep = 0, float scale = 1.f,
-                   const float *bias = nullptr);
+                   const float *bias = nullptr, const psk_moe_front *front = nullptr);
 // The S slots sorted by expert: seg [experts + 1] (slots of expert e are list[seg[e] .. seg[e + 1])), list [S]
 void psk_moe_plan(hipStream_t st, const int32_t *sel, int S, int experts, int32_t *seg, int32_t *list);
 // x[t] += alpha * sum_i (y[t top + i], or, for a slot whose sel >= n_real (an identity expert), wgt[slot] * h[t]);  y NULL: only the identity slots; sel NULL: only y; store: x[t] = instead of +=

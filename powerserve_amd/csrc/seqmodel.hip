@@ -758,7 +758,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     // score scales what the expert READS (the A operand of its first product) or, moe_weight_output, what it puts out (the rows of its inner activation: the second
     // product is linear); a few tokens run grouped mat-vecs, a portion tiles over the slots sorted by expert.  A choice beyond the experts that have matrices is an
     // identity expert: no product touches its slot, and its weight times the input joins the sum.
-    auto feed_forward = [&](const LayerPlan &P, const float *in, float *xr, float alpha, bool store = false) {
+    auto feed_forward = [&](const LayerPlan &P, const float *in, float *xr, float alpha, bool store = false, const psk_moe_front *front = nullptr) {
         const ps_seq_layer &l = P.d;
         const bool moe = l.ff_kind == PS_FF_MOE_SWIGLU || l.ff_kind == PS_FF_MOE_RELU2;
         if (!moe) {
@@ -773,7 +773,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         const int E = l.experts, rows = E + l.moe_identity, top = l.top, S = T * top;
         const int act = l.ff_kind == PS_FF_MOE_RELU2 ? PSD_ACT_RELU2 : PSD_ACT_SILU_PAIR;
         psk_moe_route(st, in, W, l.router, l.shared_gate, rows, top, l.moe_norm_top, W, T, m->moe_sel, m->moe_wgt, m->moe_sg, l.moe_softmax, l.moe_correction, l.moe_groups,
-                      l.moe_keep, l.moe_scale != 0.f ? l.moe_scale : 1.f, l.router_bias);
+                      l.moe_keep, l.moe_scale != 0.f ? l.moe_scale : 1.f, l.router_bias, front);
         const bool mv = !tiled && T <= 8 && (size_t)std::max<int64_t>(W, (int64_t)top * l.ff) * 4 + 64 <= 128 * 1024;
         if (!mv) psk_moe_plan(st, m->moe_sel, S, rows, m->moe_seg, m->moe_list);
         auto grouped = [&](psk_dense_args &g) {
@@ -848,6 +848,10 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 if (D.norm_center || b) psk_postnorm(st, m->x, m->y, nullptr, 0.f, nullptr, nullptr, 0.f, w, b, D.norm_offset, D.norm_center, D.norm_eps, W, T);
                 else boundary(m->y, w, nullptr, nullptr, 0);
             };
+            // a token's boundary in front of a mixture of experts goes along with the routing
+            const psk_moe_front front = {m->x, m->y, l.norm1b, D.norm_offset, D.norm_eps};
+            const bool along = T == 1 && !tiled && m->groups == 1 && !l.mix_onorm && !D.norm_center && !l.norm1b_bias && (l.ff_kind == PS_FF_MOE_SWIGLU || l.ff_kind == PS_FF_MOE_RELU2) &&
+                               psk_moe_front_ok(front, l.router, l.shared_gate, l.experts + (int)l.moe_identity, W);
             joint_in(P, m->x);
             if (l.mix_onorm) { // the mixers' outputs side by side (y and h), normed one by one, summed, normed and added in one launch
                 mixer(P, m->x, nullptr, 1.f);
@@ -858,10 +862,10 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             } else {
                 mixer(P, m->x, nullptr, l.mix_scale);
                 if (P.side) mixer(*P.side, m->x, m->y, P.side->d.mix_scale);
-                post(l.norm1b, l.norm1b_bias);
+                if (!along) post(l.norm1b, l.norm1b_bias);
             }
             if (l.ff_kind != PS_FF_NONE) {
-                feed_forward(P, m->x, m->y, 1.f, true);
+                feed_forward(P, m->x, m->y, 1.f, true, along ? &front : nullptr);
                 post(l.norm2b, l.norm2b_bias);
             }
             if (l.side_gate) { // the token's own input to this layer: (gelu(gate x) * its stretch of the table row) in one product, the projection, norm and add

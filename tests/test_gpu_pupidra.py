@@ -193,6 +193,16 @@ def test_whole_prompt_against_the_plain_statement(made, name, dtype):
     assert close(got, want, dtype)
 
 
+# a token's boundary and routing in one launch (k_moe.hip moe_boundary_route_kernel): widths that fill no wave, one run beyond a chunk of 2048 and beyond a thread's first run of channels, the
+# widest; rows for one wave, one more than there are waves (with the gate's), the most; a width that is no multiple of four and one row too many (two launches)
+@pytest.mark.parametrize("width,experts,top,shared", [(68, 1, 1, None), (2052, 16, 3, 8), (4100, 17, 4, None), (8192, 5, 2, 12), (66, 6, 2, 8), (132, 64, 7, 4), (132, 65, 7, 4)])
+def test_boundary_and_routing_of_a_token(made, width, experts, top, shared):
+    cfg = UC(width, 40, [UL("attention", UA(2, 1, 16, 8, 0.3, 9, 2), (experts, top, 12, 1.7), shared), UL("attention", UA(2, 2, 8, 8, 0.3, 9, 0), (experts, top, 8, 0.9), shared)])
+    m, cfg, t = made(f"front{width}.{experts}", cfg=cfg)
+    toks = tokens_for(cfg, 25)
+    assert err(run_portions(m, toks, (1,)), seq_oracle.run_pupidra(cfg, t, toks)) < TOL["float32"]
+
+
 @pytest.mark.parametrize("name", ["odd", "aligned", "wide"])
 def test_the_residual_stream_after_every_layer(made, name):
     m, cfg, t = made(name, "float32", max_batch=64)
