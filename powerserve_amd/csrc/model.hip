@@ -336,9 +336,11 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         } else if (mm(m, g, a1, dim, bs)) return 2;
 
         aa.kv_stream = kvs_own; aa.dbg = nullptr; // (also when the fused launch declined the shape)
-        // a single token's attention where attn_decode2 does not take it: rotation, append and attention in one launch
+        // a single token's attention without an exchange, rotation and append with it: where attn_decode2 does not take the shape, and where it would need the rotation's launch in front (16 heads of 64
+        // over 4 kv heads, two layers, us per token behind 100, 500 and 1000 positions: 74.8 75.6 77.9 -> 66.8 71.3 75.5).  Rotated in the mat-vec's epilogue, attn_decode2 is the faster one from a few
+        // hundred positions on (32 heads over 8: 91.4 91.5 92.6 against 87.0 94.8 99.4)
         const bool rotate = f16 || (!fuse_rope && !fuse_rope_b);
-        const bool one = bs == 1 && !use_tree && one_launch && !fused_qa && !kv16 && !psl_attn_decode2_covers(c->n_cu, aa) && psl_attn_decode1_covers(aa);
+        const bool one = bs == 1 && !use_tree && one_launch && !fused_qa && !kv16 && (rotate || !psl_attn_decode2_covers(c->n_cu, aa)) && psl_attn_decode1_covers(aa);
         if (rotate && !one) psl_rope_append(st, aa, bs);
         bool att_quantized = false;
         if (fused_qa) {

@@ -400,7 +400,7 @@ def test_chunks_attended_in_one_launch(ctx, tmp_path, preset, wt, chunk, P, n_ct
 
 
 @pytest.mark.parametrize("preset,wt,n_ctx", [("odd-llama-hs96", 8, 200), ("odd-llama-hs32", 2, 352), ("odd-llama-r5", 8, 100), ("odd-llama-r6", 8, 1280), ("odd-llama-r8", 2, 544),
-                                             ("qwen2-0.5b-dims-2l", 8, 1100)])
+                                             ("qwen2-0.5b-dims-2l", 8, 1100), ("odd-qwen2-r3", 8, 256)])
 def test_single_token_attention_without_exchange(ctx, tmp_path, preset, wt, n_ctx):
     """k_attn.hip attn_decode1_kernel (rotation, append, scores, soft-max and V.p of a token in one launch) against the separate launches, on bits: logits, the new K row and V column; an empty
     cache, one position around the groups of 8, blocks of 32, a pass of 64, the 256 positions and the 512 columns requested up front, a full window (multiples of 32 and not), both rotations,
