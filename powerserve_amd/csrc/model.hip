@@ -60,7 +60,8 @@ struct ps_hip_model {
     float *attn_xchg = nullptr;    // attn_decode2: scores in flight between workgroups (k_attn.hip)
     unsigned *attn_tick = nullptr; // attn_decode2: [64 * kv head] arrival counters
     size_t graph_hint = 0;                   // KV position the captured step was given as its prefetch hint (n_kv_lo)
-    size_t graph_hi = 0;           // ... and the cache length it may be replayed to (which attention launch a long cache gets depends on it)
+    size_t graph_hi = 0;           // ... the cache length it may be replayed to (which attention launch a long cache gets depends on it)
+    bool step_one = false, graph_one = false; // whether attn_decode1 is in the forward enqueued last, and in the captured step
     int n_kv_bound = 0;            // cache length the step being enqueued may be replayed to (0: n_ctx)
     int n_kv_hint = 0;             // capture of a single-token forward: the lower bound of n_kv its prefetch hint is baked with
     int n_kv_host = 0;             // pos0 + bs of the forward being enqueued eagerly (0 while a graph is captured / replayed)
@@ -346,6 +347,7 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         if (fused_qa) {
         } else if (one) {
             psl_attn_decode1(st, c->n_cu, aa, rotate);
+            m->step_one = true;
         } else if (bs == 1 && !use_tree && kv16 && psl_attn_decode_f16(st, aa)) {
             // fp16-KV decode mode (not bit-exact): split-KV online soft-max over the fp16 mirrors
         } else if (bs == 1 && !use_tree && one_launch && (aa.dbg = psk_gemv_dbg_buf(10, 2), psl_attn_decode2(st, c->n_cu, aa))) { // timeline key 42
@@ -854,9 +856,9 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
     // is not far behind (a stale hint costs time, never results)
-    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024 || m->position + (size_t)steps > m->graph_hi)) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
+    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024 || (m->graph_one && m->position + (size_t)steps > m->graph_hi))) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
     const size_t hi_now = std::min<size_t>(m->position + std::max<size_t>(1024 + 64, (size_t)steps), m->cfg.seq_len); // (64: a call of a few tokens late in the 1024)
-    if (!m->step_graph) m->graph_hi = hi_now;
+    if (!m->step_graph) { m->graph_hi = hi_now; m->step_one = false; }
     m->n_kv_bound = (int)m->graph_hi;
     const struct bound_guard { ps_hip_model *m; ~bound_guard() { m->n_kv_bound = 0; } } bound{m};
     if ((m->mode & 1) == 0 && !m->step_graph) {
@@ -872,6 +874,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         if (rc || e != hipSuccess) { c->err = "decode_greedy: graph capture failed: " + c->err; if (g) (void)hipGraphDestroy(g); return 2; }
         PS_CHECK(c, hipGraphInstantiate(&m->step_graph, g, nullptr, nullptr, 0));
+        m->graph_one = m->step_one;
         (void)hipGraphDestroy(g);
     }
     for (; s < steps; s++) {
