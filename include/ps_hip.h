@@ -489,8 +489,9 @@ int ps_hip_seq_release(ps_hip_seq *m, int slot);
 int64_t ps_hip_seq_position(const ps_hip_seq *m, int slot);
 size_t ps_hip_seq_slot_bytes(const ps_hip_seq *m);
 /* The step function: the next n tokens of the sequence in `slot` (HOST ids), from the state earlier steps left.
- * want: n_want indices into these tokens (HOST, may be NULL) whose logits are written to logits_host [n_want][vocab]
- * and whose arg-max ids to argmax_host (either may be NULL). */
+ * want: n_want ascending indices into these tokens (HOST, may be NULL; an index may repeat, max_batch of them at most
+ * point into one portion of max_batch tokens) whose logits are written to logits_host [n_want][vocab] and whose arg-max
+ * ids to argmax_host (either may be NULL). */
 int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, const int32_t *want, int n_want,
                        float *logits_host, int32_t *argmax_host);
 /* Greedy single-token steps: feeds `token`, then its own arg-max, `steps` times (captured launch sequence, no host round trip

@@ -953,11 +953,15 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
         if (tokens[i] < 0 || tokens[i] >= m->d.vocab) return seq_fail(c, "seq_forward: token id outside the vocabulary");
     for (int i = 0; i < n_want; i++)
         if (want[i] < 0 || want[i] >= n || (i && want[i] < want[i - 1])) return seq_fail(c, "seq_forward: want must be ascending indices into the step's tokens");
+    const int B = m->d.max_batch;
+    for (int i = 0, in = 0; i < n_want; i++) { // (an index may repeat; m->want, the logits and their ids hold max_batch rows)
+        in = i && want[i] / B == want[i - 1] / B ? in + 1 : 1;
+        if (in > B) return seq_fail(c, "seq_forward: more wanted rows in a portion of max_batch tokens than max_batch");
+    }
     PS_CHECK(c, hipSetDevice(c->device));
     // Portions follow each other on the stream without the host in between: tokens and indices travel as kernel arguments, results through two halves of pinned memory -- those of one
     // portion are handed on while the next one computes.  (With a synchronize behind every portion and copies into pageable memory the GPU stood still for 90 - 110 us of a
     // portion's 1450.)  Results that do not fit a half are copied the plain way.
-    const int B = m->d.max_batch;
     const size_t row = (logits_host ? (size_t)m->d.vocab * 4 : 0) + (argmax_host ? 4 : 0);
     struct Held { int first = 0, rows = 0; } held[2];
     auto take = [&](const int half) {

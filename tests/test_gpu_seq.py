@@ -382,6 +382,32 @@ def test_first_tokens_of_a_sequence(made):
         assert err(run_portions(m, toks, [1]), seq_oracle.run(cfg, t, toks)) < TOL["float32"]
 
 
+def test_results_of_a_call_of_several_portions(made):
+    """wanted rows that repeat, up to max_batch of them; rows of a portion too many for a half of the pinned memory between portions whose rows fit, portions without any"""
+    cfg = synth.seq_config(40, 40000, [L("wkv", 24, heads=1, dim=8)], taps=2)
+    m, cfg, t = made("40000", "float32", max_batch=16, cfg=cfg)
+    toks = tokens_for(cfg, 75, seed=3)
+    rows = seq_oracle.run(cfg, t, toks)
+    s = m.acquire()
+    for want in (np.array([0, 0, 3] + list(range(16, 32)) + [48, 63, 63] + [70]), np.full(16, 5), np.array([2] * 16 + [74] * 11)):
+        for argmax in (False, True):
+            m.release(s)
+            s = m.acquire()
+            got = m.forward(s, toks, want=want, argmax=argmax)
+            assert m.position(s) == 75
+            if argmax:
+                assert np.array_equal(got, ids)
+            else:
+                assert err(got, rows[want]) < TOL["float32"]
+                ids = got.argmax(-1)
+    m.release(s)
+    s = m.acquire()
+    with pytest.raises(hip.PSHipError, match="wanted rows"):
+        m.forward(s, toks, want=np.full(17, 40))
+    assert m.position(s) == 0
+    m.release(s)
+
+
 def test_interleaved_requests_and_reused_slots(made):
     m, cfg, t = made("mixed", "float32", max_batch=16)
     seqs = [tokens_for(cfg, n, seed=20 + n) for n in (37, 9, 58)]

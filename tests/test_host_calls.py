@@ -1,0 +1,64 @@
+"""What the C entries do on the host before, between and behind their launches, without a GPU: a child process loads tests/fake_hip.cpp in front of the library, so that every call of the HIP runtime
+lands there -- which memory a copy would touch, on which device a thing is made, and errors where a test wants one."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from powerserve_amd import hip
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes as C, sys
+import numpy as np
+fake = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
+fake.fake_stray.restype = C.c_size_t
+from powerserve_amd import hip, seqmodel, synth
+def fail(name, n=1): fake.fake_fail(name.encode(), n)
+def count(name): return fake.fake_count(name.encode())
+def refused(f):
+    try: f()
+    except hip.PSHipError as e: return str(e)
+    raise AssertionError("accepted")
+L = synth.seq_layer
+def seq(ctx, max_batch=8, vocab=30):
+    cfg = synth.seq_config(24, vocab, [L("delta", 20, heads=4, kv_heads=2, dim=6, vdim=10, conv=4), L("wkv", None, heads=3, dim=8)], taps=3)
+    synth.write_seq_model_dir({tmp!r} + "/seq", cfg, 1)
+    return seqmodel.SeqModel(ctx, {tmp!r} + "/seq", max_batch=max_batch)
+"""
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-o", so, os.path.join(HERE, "fake_hip.cpp")], check=True)
+    return so
+
+
+@pytest.fixture()
+def child(fake, tmp_path):
+    if not os.path.exists(hip.LIB_PATH):
+        pytest.skip("lib/libps_hip.so not built")
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRELUDE.format(fake=fake, tmp=str(tmp_path)) + code + "\nprint('done', flush=True)\nimport os; os._exit(0)"], cwd=os.path.dirname(HERE),
+                           capture_output=True, text=True, timeout=120)
+        assert p.returncode == 0 and p.stdout.endswith("done\n"), (p.stdout[-1000:], p.stderr[-3000:])
+
+    return run
+
+
+def test_more_wanted_rows_than_a_portion_holds_are_refused(child):
+    """ps_hip_seq_forward: an index may repeat, but a portion's logits have max_batch rows; a longer list is refused before anything is launched."""
+    child("""
+ctx = hip.Ctx(0)
+m = seq(ctx)
+s = m.acquire()
+fake.fake_reset()
+for tokens, want in (([1], [0] * 9), ([1] * 20, [0, 1] + [9] * 9), ([1] * 20, [16] * 600)):
+    refused(lambda: m.forward(s, tokens, want=want))
+    assert count("hipLaunchKernel") == count("put_kernel") == count("hipMemcpyAsync") == 0 and m.position(s) == 0
+m.forward(s, [1] * 20, want=[0] * 8 + [8] * 8 + [19] * 8)
+assert m.position(s) == 20 and fake.fake_stray() == 0
+""")
