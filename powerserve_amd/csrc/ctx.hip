@@ -123,6 +123,22 @@ void ps_pin_copy(ps_hip_ctx *c, int half, size_t at, const void *dev, size_t byt
     hipLaunchKernelGGL(pin_copy_kernel, dim3(blocks), dim3(256), 0, c->stream, (const char *)dev, c->pin + half * PS_PIN_HALF + at, bytes);
 }
 
+// Whether a caller's copy to the host may be a kernel that reads src: src lies whole in an allocation of the context's device and dst is host memory.  A copy checks its operands and comes back
+// with an error, a kernel faults; what is not known to be in order is left to the copy.
+static bool kernel_may_copy(const ps_hip_ctx *c, const void *dst, const void *src, size_t bytes) {
+    hipPointerAttribute_t s{}, d{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (!dst || !src) return false;
+    if (hipPointerGetAttributes(&s, src) != hipSuccess || s.type != hipMemoryTypeDevice || s.device != c->device || hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)src) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if ((size_t)((const char *)src - (const char *)base) + bytes > size) return false;
+    if (hipPointerGetAttributes(&d, dst) != hipSuccess) { (void)hipGetLastError(); return true; } // (pageable memory, to runtimes that do not say so)
+    return d.type == hipMemoryTypeUnregistered || d.type == hipMemoryTypeHost;
+}
+
 extern "C" {
 
 int ps_hip_abi_version(void) { return PS_HIP_ABI_VERSION; }
@@ -187,7 +203,7 @@ int ps_hip_memcpy_h2d(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {
     return 0;
 }
 int ps_hip_memcpy_d2h(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {
-    if (bytes && bytes % 4 == 0 && bytes <= 2 * PS_PIN_HALF && ((uintptr_t)src & 3) == 0 && ps_pin_ready(c)) { // (halves are neighbours)
+    if (bytes && bytes % 4 == 0 && bytes <= 2 * PS_PIN_HALF && ((uintptr_t)src & 3) == 0 && kernel_may_copy(c, dst, src, bytes) && ps_pin_ready(c)) { // (halves are neighbours)
         ps_pin_copy(c, 0, 0, src, bytes);
         PS_CHECK(c, hipStreamSynchronize(c->stream));
         memcpy(dst, c->pin, bytes);

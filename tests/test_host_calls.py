@@ -62,3 +62,24 @@ for tokens, want in (([1], [0] * 9), ([1] * 20, [0, 1] + [9] * 9), ([1] * 20, [1
 m.forward(s, [1] * 20, want=[0] * 8 + [8] * 8 + [19] * 8)
 assert m.position(s) == 20 and fake.fake_stray() == 0
 """)
+
+
+def test_copies_to_the_host_keep_their_error_cases(child):
+    """ps_hip_memcpy_d2h: what a kernel could not read without a fault is left to the runtime's copy, whatever that says"""
+    child("""
+ctx, other = hip.Ctx(0), hip.Ctx(1)
+out = np.zeros(256, np.float32)
+def d2h(dst, src, n): ctx.check(ctx.L.ps_hip_memcpy_d2h(ctx.h, dst, src, n))
+p, q, far = ctx.malloc(1024), ctx.malloc(1024), other.malloc(1024)
+fake.fake_reset()
+for dst, src, n in ((out.ctypes.data, None, 64), (out.ctypes.data, p, 1028), (out.ctypes.data, p + 512, 1024), (None, p, 64), (out.ctypes.data, 4096, 64)):
+    refused(lambda: d2h(dst, src, n))
+d2h(out.ctypes.data, far, 1024)
+d2h(q, p, 1024)
+assert count("pin_copy_kernel") == 0 and count("hipMemcpyAsync") == 7 and fake.fake_stray() == 0
+d2h(out.ctypes.data, p + 512, 512)
+assert count("pin_copy_kernel") == 1 and count("hipMemcpyAsync") == 7 and fake.fake_stray() == 0
+d2h(out.ctypes.data, p + 2, 64)
+d2h(out.ctypes.data, p, 1023)
+d2h(out.ctypes.data, p, 0)
+""")
