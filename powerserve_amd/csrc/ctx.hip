@@ -203,7 +203,7 @@ int ps_hip_memcpy_h2d(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {
     return 0;
 }
 int ps_hip_memcpy_d2h(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {
-    if (bytes && bytes % 4 == 0 && bytes <= 2 * PS_PIN_HALF && ((uintptr_t)src & 3) == 0 && kernel_may_copy(c, dst, src, bytes) && ps_pin_ready(c)) { // (halves are neighbours)
+    if (bytes && bytes % 4 == 0 && bytes <= PS_PIN_WAITED && ((uintptr_t)src & 3) == 0 && kernel_may_copy(c, dst, src, bytes) && ps_pin_ready(c)) {
         ps_pin_copy(c, 0, 0, src, bytes);
         PS_CHECK(c, hipStreamSynchronize(c->stream));
         memcpy(dst, c->pin, bytes);

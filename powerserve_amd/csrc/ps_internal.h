@@ -40,6 +40,9 @@ void ps_put(hipStream_t st, const ps_piece *p, int n);
 // Device results through pinned memory: ps_pin_copy enqueues a kernel that writes `bytes` (a multiple of four, from a multiple of four) to c->pin + half * PS_PIN_HALF + at; who
 // reads them waits for the stream, or for an event of c->pin_ev recorded behind it, and is done with them before its call returns.  ps_pin_ready: whether there is pinned memory.
 constexpr size_t PS_PIN_HALF = (size_t)2 << 20;
+// What is waited for at once goes this way up to here.  us a call, the runtime's copy into pageable memory and a kernel into pinned with the host's copy behind it: 1 KB 20 and 14, 16 KB 26 and 15,
+// 24 KB 18 and 14; 32 KB 10.5 and 14, 64 KB 12 and 15, 256 KB 19 and 22, 4 MB 222 and 228.
+constexpr size_t PS_PIN_WAITED = 24 * 1024;
 bool ps_pin_ready(ps_hip_ctx *c);
 void ps_pin_copy(ps_hip_ctx *c, int half, size_t at, const void *dev, size_t bytes);
 
