@@ -113,6 +113,7 @@ void ps_put(hipStream_t st, const ps_piece *p, int n) {
 }
 bool ps_pin_ready(ps_hip_ctx *c) {
     if (c->pin) return true;
+    if (hipSetDevice(c->device) != hipSuccess) { (void)hipGetLastError(); return false; } // (an event belongs to the device that is current)
     for (auto &e : c->pin_ev)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return false; }
     if (hipHostMalloc((void **)&c->pin, 2 * PS_PIN_HALF, hipHostMallocDefault) != hipSuccess) { c->pin = nullptr; (void)hipGetLastError(); return false; }
@@ -129,7 +130,8 @@ static bool kernel_may_copy(const ps_hip_ctx *c, const void *dst, const void *sr
     hipPointerAttribute_t s{}, d{};
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
-    if (!dst || !src) return false;
+    int dev = -1;
+    if (!dst || !src || hipGetDevice(&dev) != hipSuccess || dev != c->device) return false; // (a copy may be enqueued whichever device is current, a kernel not)
     if (hipPointerGetAttributes(&s, src) != hipSuccess || s.type != hipMemoryTypeDevice || s.device != c->device || hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)src) != hipSuccess) {
         (void)hipGetLastError();
         return false;

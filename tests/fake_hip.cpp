@@ -55,7 +55,8 @@ void __hipRegisterFunction(void **, const void *host, char *, const char *name, 
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
 static dim3 no_dim;
 hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *s, hipStream_t *st) { *g = *b = no_dim; *s = 0; *st = nullptr; return hipSuccess; }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t s) {
+    if (s && ((Thing *)s)->device != current) return call("hipLaunchKernel", hipErrorInvalidHandle);
     const std::string &n = kernels[f];
     if (n.find("pin_copy_kernel") != std::string::npos) {
         if (call("pin_copy_kernel")) return hipErrorUnknown;

@@ -101,3 +101,19 @@ for tokens, want, kernels, copies in ((8, 2, 1, 0), (8, 3, 0, 1), (16, 16, 2, 0)
     m.forward(s, [1] * tokens, want=np.arange(want))
     assert (count("pin_copy_kernel"), count("hipMemcpyAsync")) == (kernels, copies), (tokens, want)
 """)
+
+
+def test_pinned_memory_and_its_events_are_made_on_the_contexts_device(child):
+    """two contexts: copies on the first while the second's device is current (before and after there is pinned memory), then portions on the first, whose events have to be the first's"""
+    child("""
+ctx = hip.Ctx(0)
+m = seq(ctx, 8, 3000)
+s, p, out = m.acquire(), ctx.malloc(64), np.zeros(16, np.float32)
+other = hip.Ctx(1)
+fake.fake_reset()
+for _ in range(2):
+    fake.hipSetDevice(1)
+    ctx.check(ctx.L.ps_hip_memcpy_d2h(ctx.h, out.ctypes.data, p, 64))
+    m.forward(s, [1] * 16, want=np.arange(16))
+assert count("hipEventRecord") == 4 and count("hipMemcpyAsync") == 2
+""")
