@@ -71,6 +71,7 @@ ctx, other = hip.Ctx(0), hip.Ctx(1)
 out = np.zeros(256, np.float32)
 def d2h(dst, src, n): ctx.check(ctx.L.ps_hip_memcpy_d2h(ctx.h, dst, src, n))
 p, q, far = ctx.malloc(1024), ctx.malloc(1024), other.malloc(1024)
+fake.hipSetDevice(0)
 fake.fake_reset()
 for dst, src, n in ((out.ctypes.data, None, 64), (out.ctypes.data, p, 1028), (out.ctypes.data, p + 512, 1024), (None, p, 64), (out.ctypes.data, 4096, 64)):
     refused(lambda: d2h(dst, src, n))
