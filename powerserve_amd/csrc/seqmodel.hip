@@ -977,18 +977,21 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
         return hipSuccess;
     };
     int wi = 0, half = 0;
-    int64_t pos0 = m->slot_pos[slot];
     std::vector<int32_t> idx;
-    for (int t0 = 0; t0 < n; t0 += B) {
-        const int T = std::min(B, n - t0), w0 = wi;
-        idx.clear();
-        while (wi < n_want && want[wi] < t0 + T) idx.push_back(want[wi++] - t0);
-        const ps_piece in[2] = {{m->tokens, tokens + t0, (size_t)T * 4}, {m->want, idx.data(), idx.size() * 4}};
-        ps_put(c->stream, in, 2);
-        hipLaunchKernelGGL(seq_set_step_kernel, dim3(1), dim3(1), 0, c->stream, m->step, (long long)pos0, T, slot, m->slot_state[slot], (int)tokens[t0], (int)tokens[t0 + T - 1],
-                           m->prev_of(slot));
-        seq_layers(m, m->slot_state[slot], T, pos0, false, false);
-        if (!idx.empty()) {
+    auto portions = [&]() -> int {
+        for (int t0 = 0; t0 < n; t0 += B) {
+            const int T = std::min(B, n - t0), w0 = wi;
+            const int64_t pos0 = m->slot_pos[slot];
+            idx.clear();
+            while (wi < n_want && want[wi] < t0 + T) idx.push_back(want[wi++] - t0);
+            const ps_piece in[2] = {{m->tokens, tokens + t0, (size_t)T * 4}, {m->want, idx.data(), idx.size() * 4}};
+            ps_put(c->stream, in, 2);
+            hipLaunchKernelGGL(seq_set_step_kernel, dim3(1), dim3(1), 0, c->stream, m->step, (long long)pos0, T, slot, m->slot_state[slot], (int)tokens[t0], (int)tokens[t0 + T - 1],
+                               m->prev_of(slot));
+            seq_layers(m, m->slot_state[slot], T, pos0, false, false);
+            PS_CHECK(c, hipGetLastError());
+            m->slot_pos[slot] = pos0 + T; // (the slot's recurrent states move with these launches, whatever becomes of the results)
+            if (idx.empty()) continue;
             const int rows = (int)idx.size();
             seq_head(m, m->want, rows);
             if (row && rows * row <= (n > B ? PS_PIN_HALF : PS_PIN_WAITED) && ps_pin_ready(c)) { // (a call of one portion has nothing to hand on meanwhile)
@@ -1004,15 +1007,19 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
                 if (logits_host) PS_CHECK(c, hipMemcpyAsync(logits_host + (size_t)w0 * m->d.vocab, m->logits, (size_t)rows * m->d.vocab * 4, hipMemcpyDeviceToHost, c->stream));
                 if (argmax_host) PS_CHECK(c, hipMemcpyAsync(argmax_host + w0, m->amax, (size_t)rows * 4, hipMemcpyDeviceToHost, c->stream));
             }
+            PS_CHECK(c, hipGetLastError());
         }
+        PS_CHECK(c, hipStreamSynchronize(c->stream));
         PS_CHECK(c, hipGetLastError());
-        pos0 += T;
+        for (int h = 0; h < 2; h++) PS_CHECK(c, take(h));
+        return 0;
+    };
+    const int rc = portions();
+    if (rc) { // copies into the caller's memory may be under way; and the error is this call's, not the next one's
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipGetLastError();
     }
-    PS_CHECK(c, hipStreamSynchronize(c->stream));
-    PS_CHECK(c, hipGetLastError());
-    for (int h = 0; h < 2; h++) PS_CHECK(c, take(h));
-    m->slot_pos[slot] = pos0;
-    return 0;
+    return rc;
 }
 
 int ps_hip_seq_decode_greedy(ps_hip_seq *m, int slot, int32_t token, int steps, int32_t *out_ids) {

@@ -1,6 +1,6 @@
 // A HIP runtime for host-side tests: device memory is host memory with a list of what is allocated, streams run at once, kernels are counted and not run -- but for the two that carry bytes between
 // host and device (csrc/ctx.hip: put_kernel, pin_copy_kernel), which copy.  Loaded in front of the library under test (RTLD_GLOBAL), whose calls it then takes.
-// fake_fail(name, n): the n-th call of that name from now on fails; fake_count(name): calls since the last fake_reset(); fake_stray(): bytes that a kernel would have touched outside an allocation.
+// fake_fail(name, n): the n-th call of that name from now on fails; fake_count(name): calls since the last fake_reset(), launches of a kernel also by its name; fake_stray(): bytes that a kernel would have touched outside an allocation.
 #include <hip/hip_runtime_api.h>
 #include <cstdlib>
 #include <cstring>
@@ -46,7 +46,12 @@ hipError_t alloc(void **p, size_t bytes, hipMemoryType type) {
 extern "C" {
 void fake_reset() { count.clear(); fail.clear(); stray = 0; }
 void fake_fail(const char *name, int n) { fail[name] = n; }
-int fake_count(const char *name) { return count[name]; }
+int fake_count(const char *name) { // (of every name with this in it: a kernel's is mangled)
+    int n = 0;
+    for (auto &c : count)
+        if (c.first.find(name) != std::string::npos) n += c.second;
+    return n;
+}
 size_t fake_stray() { return stray; }
 
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
@@ -72,6 +77,7 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
             if (bytes[i]) move(((void **)a)[i], v, bytes[i], true, false);
         return hipSuccess;
     }
+    count[n]++;
     return call("hipLaunchKernel");
 }
 

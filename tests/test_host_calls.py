@@ -118,3 +118,27 @@ for _ in range(2):
     m.forward(s, [1] * 16, want=np.arange(16))
 assert count("hipEventRecord") == 4 and count("hipMemcpyAsync") == 2
 """)
+
+
+def test_a_slots_position_follows_its_state_when_a_later_portion_fails(child):
+    """the recurrent states move with every portion that was launched, whatever becomes of its results: so does the position, and nothing is still on its way to the caller's memory"""
+    child("""
+ctx = hip.Ctx(0)
+m = seq(ctx, 8, 3000)
+for name, nth in (("hipEventSynchronize", 1), ("hipEventSynchronize", 2), ("hipEventRecord", 1), ("hipEventRecord", 3), ("hipStreamSynchronize", 1)):
+    s = m.acquire()
+    fake.fake_reset()
+    fail(name, nth)
+    refused(lambda: m.forward(s, [1] * 32, want=np.arange(32)))
+    ran = count("seq_set_step_kernel")
+    assert ran and m.position(s) == 8 * ran and count("hipStreamSynchronize"), (name, nth, ran, m.position(s))
+    at = m.position(s)
+    m.forward(s, [1] * 9, want=[8])
+    assert m.position(s) == at + 9
+    m.release(s)
+s = m.acquire()
+fake.fake_reset()
+fail("hipGetLastError", 2)
+refused(lambda: m.forward(s, [1] * 32))
+assert m.position(s) == 8 * (count("seq_set_step_kernel") - 1) == 8  # (a portion whose launches failed has not been taken)
+""")
