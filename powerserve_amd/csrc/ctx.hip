@@ -72,7 +72,7 @@ __global__ void put_kernel(const PutArgs<W> a) {
     }
 }
 template <int W>
-void put_launch(hipStream_t st, const ps_piece *p, int n) { // n <= 4 pieces of at most W words in all
+hipError_t put_launch(hipStream_t st, const ps_piece *p, int n) { // n <= 4 pieces of at most W words in all
     PutArgs<W> a{};
     size_t at = 0;
     for (int i = 0; i < n; i++) {
@@ -81,7 +81,8 @@ void put_launch(hipStream_t st, const ps_piece *p, int n) { // n <= 4 pieces of 
         memcpy(a.v + at, p[i].src, p[i].bytes);
         at += (p[i].bytes + 3) / 4;
     }
-    hipLaunchKernelGGL(put_kernel<W>, dim3(1), dim3(W < 256 ? 64 : 256), 0, st, a);
+    void *args[] = {&a};
+    return hipLaunchKernel((const void *)put_kernel<W>, dim3(1), dim3(W < 256 ? 64 : 256), args, 0, st); // (its own result: hipGetLastError may hold somebody else's)
 }
 __global__ __launch_bounds__(256) void pin_copy_kernel(const char *src, char *dst, size_t bytes) {
     const bool wide = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
@@ -90,15 +91,24 @@ __global__ __launch_bounds__(256) void pin_copy_kernel(const char *src, char *ds
     for (size_t i = n16 * 4 + t; i < bytes / 4; i += step) ((uint32_t *)dst)[i] = ((const uint32_t *)src)[i];
 }
 } // namespace
-void ps_put(hipStream_t st, const ps_piece *p, int n) {
+hipError_t ps_put(hipStream_t st, const ps_piece *p, int n) {
     constexpr size_t CAP = 896;
+    size_t total = 0;
+    for (int i = 0; i < n; i++) total += p[i].bytes;
+    if (total > PS_PUT_MAX) {
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < n && e == hipSuccess; i++)
+            if (p[i].bytes) e = hipMemcpyAsync(p[i].dst, p[i].src, p[i].bytes, hipMemcpyHostToDevice, st);
+        const hipError_t w = hipStreamSynchronize(st); // (the sources may be temporaries)
+        return e != hipSuccess ? e : w;
+    }
     ps_piece q[4];
     int k = 0;
     size_t words = 0;
     auto flush = [&]() {
-        if (k && words <= 32) put_launch<32>(st, q, k);
-        else if (k) put_launch<CAP>(st, q, k);
+        const hipError_t e = !k ? hipSuccess : words <= 32 ? put_launch<32>(st, q, k) : put_launch<CAP>(st, q, k);
         k = 0; words = 0;
+        return e;
     };
     for (int i = 0; i < n; i++) {
         for (size_t done = 0; done < p[i].bytes;) {
@@ -106,10 +116,11 @@ void ps_put(hipStream_t st, const ps_piece *p, int n) {
             q[k++] = ps_piece{(char *)p[i].dst + done, (const char *)p[i].src + done, b};
             words += (b + 3) / 4;
             done += b;
-            if (k == 4 || words == CAP) flush();
+            if (k == 4 || words == CAP)
+                if (const hipError_t e = flush()) return e;
         }
     }
-    flush();
+    return flush();
 }
 bool ps_pin_ready(ps_hip_ctx *c) {
     if (c->pin) return true;

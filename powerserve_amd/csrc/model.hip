@@ -696,7 +696,7 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
         m->pin_busy = true;
     } else {
         const ps_piece in[2] = {{m->tokens_dev, tokens, (size_t)n * 4}, {m->tree_dev, tree, (size_t)n * n}};
-        ps_put(c->stream, in, tree ? 2 : 1);
+        PS_CHECK(c, ps_put(c->stream, in, tree ? 2 : 1));
         hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, pos[0], n, 0);
     }
     // A single token through this entry (ModelTokenIterator::decode over the op API, HIPBackend::plan's lowered graph) replays
@@ -766,7 +766,7 @@ int ps_hip_model_prefill(ps_hip_model *m, const int32_t *tokens, int n, int chun
     for (int done = 0; done < n;) {
         const int ns = n - done < per * chunk ? n - done : per * chunk;
         const ps_piece in = {m->tokens_dev, tokens + done, (size_t)ns * 4};
-        ps_put(c->stream, &in, 1);
+        PS_CHECK(c, ps_put(c->stream, &in, 1));
         hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, ns, 0);
         hipLaunchKernelGGL(set_sub_states_kernel, dim3(1), dim3(64), 0, c->stream, m->state_sub, (int)m->position, chunk, ns);
         m->n_kv_host = (int)m->position + ns;
@@ -806,7 +806,7 @@ static int forward_tree_impl(ps_hip_model *m, const int32_t *tokens, int n, cons
     PS_CHECK(c, hipSetDevice(c->device));
     m->pin_argmax_n = 0;
     const ps_piece in[3] = {{m->tokens_dev, tokens, (size_t)n * 4}, {m->rope_pos_dev, rope_pos, (size_t)n * 4}, {m->tree_dev, tree, (size_t)n * n}};
-    ps_put(c->stream, in, tree ? 3 : 2);
+    PS_CHECK(c, ps_put(c->stream, in, tree ? 3 : 2));
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, n, 0);
     m->n_kv_host = (int)m->position + n;
     const int rc_fw = enqueue_forward(m, n, lm_head != 0, tree != nullptr, false, true);
@@ -851,7 +851,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     PS_CHECK(c, hipSetDevice(c->device));
     m->pin_argmax_n = 0;
     const ps_piece in = {m->tokens_dev, &token, 4};
-    ps_put(c->stream, &in, 1);
+    PS_CHECK(c, ps_put(c->stream, &in, 1));
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, 1, 0);
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that

@@ -33,10 +33,12 @@ struct ps_hip_ctx {
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
 };
 // Host bytes into device memory in stream order, as kernel arguments (pieces of at most 3.5 KB a launch): the host's buffers are free on return and nobody waits for the stream.
-// Destinations are multiples of four bytes.  (A copy from pageable memory is staged by the runtime and wants a synchronize behind it where the source is a temporary: 10 - 25 us
-// in front of a request, measured, against 3.)
+// Destinations are multiples of four bytes.  (A copy from pageable memory is staged by the runtime and wants a synchronize behind it where the source is a temporary.)  More than PS_PUT_MAX
+// bytes are copied that way all the same: us of a tree forward of a tiny model, ids and n x n mask copied | as arguments, n = 12 160 | 148, 64 171 | 155, 128 (17 KB) 181 | 178, 160 187 | 189,
+// 192 (38 KB) 190 | 196, 256 209 | 228, 350 212 | 300.
 struct ps_piece { void *dst; const void *src; size_t bytes; };
-void ps_put(hipStream_t st, const ps_piece *p, int n);
+constexpr size_t PS_PUT_MAX = 20 * 1024;
+hipError_t ps_put(hipStream_t st, const ps_piece *p, int n);
 // Device results through pinned memory: ps_pin_copy enqueues a kernel that writes `bytes` (a multiple of four, from a multiple of four) to c->pin + half * PS_PIN_HALF + at; who
 // reads them waits for the stream, or for an event of c->pin_ev recorded behind it, and is done with them before its call returns.  ps_pin_ready: whether there is pinned memory.
 constexpr size_t PS_PIN_HALF = (size_t)2 << 20;

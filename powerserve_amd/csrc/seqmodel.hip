@@ -985,7 +985,7 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
             idx.clear();
             while (wi < n_want && want[wi] < t0 + T) idx.push_back(want[wi++] - t0);
             const ps_piece in[2] = {{m->tokens, tokens + t0, (size_t)T * 4}, {m->want, idx.data(), idx.size() * 4}};
-            ps_put(c->stream, in, 2);
+            PS_CHECK(c, ps_put(c->stream, in, 2));
             hipLaunchKernelGGL(seq_set_step_kernel, dim3(1), dim3(1), 0, c->stream, m->step, (long long)pos0, T, slot, m->slot_state[slot], (int)tokens[t0], (int)tokens[t0 + T - 1],
                                m->prev_of(slot));
             seq_layers(m, m->slot_state[slot], T, pos0, false, false);

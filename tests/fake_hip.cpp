@@ -44,7 +44,7 @@ hipError_t alloc(void **p, size_t bytes, hipMemoryType type) {
 } // namespace
 
 extern "C" {
-void fake_reset() { count.clear(); fail.clear(); stray = 0; }
+void fake_reset() { count.clear(); fail.clear(); stray = 0; last = hipSuccess; }
 void fake_fail(const char *name, int n) { fail[name] = n; }
 int fake_count(const char *name) { // (of every name with this in it: a kernel's is mangled)
     int n = 0;

@@ -22,6 +22,9 @@ def refused(f):
     except hip.PSHipError as e: return str(e)
     raise AssertionError("accepted")
 L = synth.seq_layer
+def quant(ctx, max_batch):
+    synth.write_model_dir({tmp!r} + "/quant", "tiny-llama", 8, n_ctx=1024, seed=1)
+    return hip.Model(ctx, {tmp!r} + "/quant", max_batch=max_batch, n_ctx=1024)
 def seq(ctx, max_batch=8, vocab=30):
     cfg = synth.seq_config(24, vocab, [L("delta", 20, heads=4, kv_heads=2, dim=6, vdim=10, conv=4), L("wkv", None, heads=3, dim=8)], taps=3)
     synth.write_seq_model_dir({tmp!r} + "/seq", cfg, 1)
@@ -141,4 +144,36 @@ fake.fake_reset()
 fail("hipGetLastError", 2)
 refused(lambda: m.forward(s, [1] * 32))
 assert m.position(s) == 8 * (count("seq_set_step_kernel") - 1) == 8  # (a portion whose launches failed has not been taken)
+""")
+
+
+def test_inputs_travel_as_arguments_up_to_a_size_and_their_errors_come_back(child):
+    """csrc/ctx.hip ps_put: a large tree's mask is one copy, not 75 launches; a launch that fails ends the call"""
+    child("""
+ctx = hip.Ctx(0)
+m = quant(ctx, 512)
+for n, launches in ((12, 1), (139, 6), (140, 0), (512, 0)):
+    t = np.arange(n) % 500
+    see = np.tril(np.ones((n, n), np.uint8))
+    fake.fake_reset()
+    m.forward_tree(t, np.arange(n), see)
+    assert (count("put_kernel"), count("hipMemcpyAsync")) == (launches, 0 if launches else 3), (n, count("put_kernel"), count("hipMemcpyAsync"))
+    assert fake.fake_stray() == 0
+m.set_mode(1)
+q = seq(ctx)
+s = q.acquire()
+for f in (lambda: m.forward_tree([1, 2], [0, 1], np.tril(np.ones((2, 2), np.uint8))), lambda: m.forward_tree(np.arange(500), np.arange(500), np.ones((500, 500), np.uint8)),
+          lambda: m.forward([1, 2], [0, 1]), lambda: m.prefill(np.arange(20), 10), lambda: m.decode_greedy(1, 3), lambda: q.forward(s, [1, 2])):
+    fake.fake_reset()
+    f()
+    m.kv_rollback(m.position)
+    at = q.position(s)
+    for name in ("put_kernel", "hipMemcpyAsync"):
+        fake.fake_reset()
+        fail(name)
+        try: f()
+        except hip.PSHipError: assert m.position == 0 and q.position(s) == at
+        else: assert name == "hipMemcpyAsync" or not count(name), name
+        m.kv_rollback(m.position)
+        at = q.position(s)
 """)
