@@ -491,11 +491,12 @@ __device__ __forceinline__ void gemm8_stage(const int8_t *aq, const float *ad, c
     // LDS image: one record per (unit, column), records of a unit adjacent, so that every per-column read of the inner
     // loop is  base(unit, lane) + compile-time offset:
     //   Q4_K  REC 304: [256 B quants, dwords transposed (g, u) -> [u][g]] [8 int sums of 32] [float d] [pad]
-    //   Q8_0  REC 144: [128 B quants, transposed] [4 float d]
+    //   Q8_0 / Q4_0  REC 144: [128 B quants, transposed] [4 float d]
     constexpr int REC = (WT == PS_Q4_K) ? 304 : 144, UDW = TR::UNIT / 4; // dwords of quants per unit and column
     auto tpos = [](int i) { // dword i of a unit -> its place in the transposed record
         if (WT == PS_Q4_K) return (i & 7) * 8 + (i >> 3);                 // (g, u) -> [u][g]
-        return (i & 7) * 4 + (i >> 3);                                    // Q8_0: (block b, d) -> [d][b]
+        if (WT == PS_Q8_0) return (i & 7) * 4 + (i >> 3);                 // (block b, d) -> [d][b]
+        return (i & 3) * 8 + (i >> 3) * 2 + ((i >> 2) & 1);               // Q4_0: (b, half*4 + u') -> [u'][b][half]
     };
     {   // 16-byte global loads, SB of them in flight per thread, then the transposed dword stores
         constexpr int SB = 8;
@@ -707,28 +708,32 @@ __global__ __launch_bounds__(NWV * 64) void gemm8m_kernel(const GemvParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Q8_0 batched mat-mul of few columns and rows (psk_gemm8 says which) with the quad dots on the matrix cores (same idea as gemm8m_kernel; here every quad dot
+// Q8_0 / Q4_0 batched mat-mul of up to 8 columns (psk_gemm8 says which) with the quad dots on the matrix cores (same idea as gemm8m_kernel; here every quad dot
 // meets its own fp32 block scale, so the MFMAs do not accumulate: D = dot4(weight quad, activation quad), then
-// acc[u] = fma(d_w * d_y, (float)D, acc[u]) block after block as in ggml_vec_dot_q8_0_q8_0).  Bound by the latency of one wave's chain: 8 rows x 8 columns per wave.
-//   (row groups of 8)  qs = lane >> 4 owns u = qs, qs + 4;  A row (lane >> 3 & 1) * 4 + s;  column (lane >> 2 & 1) * 4 + s
-template <int EPI>
-__global__ __launch_bounds__(256) void gemm8b_kernel(const GemvParams p) {
-    using TR = WTraits<PS_Q8_0>;
-    constexpr int NWV = 4, NT = NWV * 64, C = 8, REC = 144;
+// acc[u] = fma(d_w * d_y, (float)D, acc[u]) block after block as in ggml_vec_dot_q8_0_q8_0 / q4_0_q8_0).  Bound by the latency of one wave's chain where the rows are few, by its
+// issue where they are many: a wave has only 8 columns' fmas, NWV of them share the activations' image (128256 x 4096, 2 columns: Q4_0 104 us in eights, 133 in fours, 106 in sixteens).
+//   Q8_0 (row groups of 8):  qs = lane >> 4 owns u = qs, qs + 4;  A row (lane >> 3 & 1) * 4 + s;  column (lane >> 2 & 1) * 4 + s
+//   Q4_0 (row groups of 16): qs = lane >> 4: the low nibbles of piece (row, qs) are u = qs, the high ones u = qs + 4;
+//                            A row (lane >> 2 & 3) * 4 + s;  columns s and s + 4 (two sets)
+template <int WT, int EPI, int NWV>
+__global__ __launch_bounds__(NWV * 64) void gemm8b_kernel(const GemvParams p) {
+    using TR = WTraits<WT>;
+    constexpr int NT = NWV * 64, C = 8, REC = 144, NCS = (WT == PS_Q4_0) ? 2 : 1;
+    constexpr uint32_t M = 0x0F0F0F0Fu;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int K = (int)p.K, n_units = K / 128, c0 = blockIdx.y * C, nc = min(C, (int)p.bs - c0);
-    gemm8_stage<PS_Q8_0, NT, C>(p.aq, p.ad, p.abs16, K, smem, c0, nc);
+    gemm8_stage<WT, NT, C>(p.aq, p.ad, p.abs16, K, smem, c0, nc);
     __syncthreads();
 
     const int qs = lane >> 4, s4 = lane & 3;
-    const int rqi  = (lane >> 3) & 1; // row quad of the row group
+    const int rqi  = (WT == PS_Q4_0) ? (lane >> 2) & 3 : (lane >> 3) & 1; // row quad of the row group
     const int arow = rqi * 4 + s4;
-    const int col  = ((lane >> 2) & 1) * 4 + s4;
+    const int col0 = (WT == PS_Q4_0) ? s4 : ((lane >> 2) & 1) * 4 + s4;   // column of set cs: col0 + 4 cs (Q4_0 only has cs = 1)
     const int64_t n_tasks = (EPI == 1) ? p.w[0].n_groups : p.groups_total;
     const int64_t task = (int64_t)blockIdx.x * NWV + wave;
     if (task >= n_tasks) return;
-    float yg[4];
+    float yg[NCS][4];
 #pragma unroll
     for (int pass = 0; pass < (EPI == 1 ? 2 : 1); pass++) {
         int wi = 0;
@@ -742,45 +747,69 @@ __global__ __launch_bounds__(256) void gemm8b_kernel(const GemvParams p) {
         const uint8_t *qsb = p.w[0].qs, *ax = p.w[0].aux;
         if (wi == 1) { qsb = p.w[1].qs; ax = p.w[1].aux; }
         if (wi == 2) { qsb = p.w[2].qs; ax = p.w[2].aux; }
-        const uint8_t *qg = qsb + grp * n_units * 1024 + (arow * 8 + qs) * 16; // pieces (row, qs) and (row, qs + 4), 64 bytes apart
+        // Q8_0: pieces (row, qs) and (row, qs + 4), 64 bytes apart;  Q4_0: the one piece (row, qs)
+        const uint8_t *qg = qsb + grp * n_units * 1024 + ((WT == PS_Q4_0) ? (arow * 4 + qs) : (arow * 8 + qs)) * 16;
         const uint8_t *ag = ax + grp * n_units * (TR::RG * 8) + arow * 8;
-        float acc[2][4];
+        float acc[NCS][2][4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) { acc[0][r] = 0.f; acc[1][r] = 0.f; }
+        for (int cs = 0; cs < NCS; cs++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) { acc[cs][0][r] = 0.f; acc[cs][1][r] = 0.f; }
 
         auto unit = [&](const int un, const uint4 qa, const uint4 qb, const uint2 h) {
+            // A operands: [u half][block]
+            int wa[2][4];
             const uint32_t w0[4] = {qa.x, qa.y, qa.z, qa.w}, w1[4] = {qb.x, qb.y, qb.z, qb.w};
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                if (WT == PS_Q8_0) { wa[0][b] = (int)w0[b]; wa[1][b] = (int)w1[b]; }
+                else { // nibble - 8 as signed bytes
+                    wa[0][b] = (int)((((w0[b] & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+                    wa[1][b] = (int)(((((w0[b] >> 4) & M) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+                }
+            }
             // this lane's row: the four fp16 block scales as floats
             const float dwo[4] = {ps_h2f((uint16_t)(h.x & 0xffff)), ps_h2f((uint16_t)(h.x >> 16)), ps_h2f((uint16_t)(h.y & 0xffff)), ps_h2f((uint16_t)(h.y >> 16))};
-            const char *rec = smem + (un * C + col) * REC;
-            const int4 t0 = *(const int4 *)(rec + qs * 16), t1 = *(const int4 *)(rec + (qs + 4) * 16);
-            const int y0[4] = {t0.x, t0.y, t0.z, t0.w}, y1[4] = {t1.x, t1.y, t1.z, t1.w};
-            const float4 yd = *(const float4 *)(rec + 128);
-            const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
-#define PS_G8B_ROW(r, CTRL)                                                                          \
-            {                                                                                        \
-                const float d = __fmul_rn(dpp_f<CTRL>(dwo[b]), ydv[b]);                               \
-                acc[0][r] = __fmaf_rn(d, (float)D0[r], acc[0][r]);                                    \
-                acc[1][r] = __fmaf_rn(d, (float)D1[r], acc[1][r]);                                    \
-            }
 #pragma unroll
-            for (int b = 0; b < 4; b++) { // block after block: the products of a block are consumed before the next ones exist
-                const ps_i32x4 D0 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)w0[b], y0[b], ps_i32x4{0, 0, 0, 0}, 0, 0, 0);
-                const ps_i32x4 D1 = __builtin_amdgcn_mfma_i32_4x4x4i8((int)w1[b], y1[b], ps_i32x4{0, 0, 0, 0}, 0, 0, 0);
-                PS_G8B_ROW(0, 0x00) PS_G8B_ROW(1, 0x55) PS_G8B_ROW(2, 0xAA) PS_G8B_ROW(3, 0xFF)
-            }
+            for (int cs = 0; cs < NCS; cs++) {
+                const char *rec = smem + (un * C + col0 + 4 * cs) * REC;
+                int y[2][4]; // [u half][block]
+                if (WT == PS_Q8_0) {
+                    const int4 t0 = *(const int4 *)(rec + qs * 16), t1 = *(const int4 *)(rec + (qs + 4) * 16);
+                    y[0][0] = t0.x; y[0][1] = t0.y; y[0][2] = t0.z; y[0][3] = t0.w;
+                    y[1][0] = t1.x; y[1][1] = t1.y; y[1][2] = t1.z; y[1][3] = t1.w;
+                } else { // record of u' = qs: dword 2 b + half
+                    const int4 t0 = *(const int4 *)(rec + qs * 32), t1 = *(const int4 *)(rec + qs * 32 + 16);
+                    y[0][0] = t0.x; y[1][0] = t0.y; y[0][1] = t0.z; y[1][1] = t0.w;
+                    y[0][2] = t1.x; y[1][2] = t1.y; y[0][3] = t1.z; y[1][3] = t1.w;
+                }
+                const float4 yd = *(const float4 *)(rec + 128);
+                const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
+#define PS_G8B_ROW(r, CTRL)                                                                                  \
+                    {                                                                                        \
+                        const float d = __fmul_rn(dpp_f<CTRL>(dwo[b]), ydv[b]);                               \
+                        acc[cs][0][r] = __fmaf_rn(d, (float)D0[r], acc[cs][0][r]);                            \
+                        acc[cs][1][r] = __fmaf_rn(d, (float)D1[r], acc[cs][1][r]);                            \
+                    }
+#pragma unroll
+                for (int b = 0; b < 4; b++) { // block after block: the products of a block are consumed before the next ones exist
+                    const ps_i32x4 D0 = __builtin_amdgcn_mfma_i32_4x4x4i8(wa[0][b], y[0][b], ps_i32x4{0, 0, 0, 0}, 0, 0, 0);
+                    const ps_i32x4 D1 = __builtin_amdgcn_mfma_i32_4x4x4i8(wa[1][b], y[1][b], ps_i32x4{0, 0, 0, 0}, 0, 0, 0);
+                    PS_G8B_ROW(0, 0x00) PS_G8B_ROW(1, 0x55) PS_G8B_ROW(2, 0xAA) PS_G8B_ROW(3, 0xFF)
+                }
 #undef PS_G8B_ROW
+            }
         };
         auto load_h = [&](int un) { return *(const uint2 *)(ag + (int64_t)un * (TR::RG * 8)); };
         {   // PF units in flight per wave (register ring); loads unconditional (index clamped to the last unit)
-            constexpr int PF = 4;
+            constexpr int PF = (NWV == 4) ? 4 : 2;
             uint4 qar[PF], qbr[PF];
             uint2 hr[PF];
 #pragma unroll
             for (int s = 0; s < PF; s++) {
                 const int uc = min(s, n_units - 1);
                 qar[s] = ld_stream16(qg + (int64_t)uc * 1024);
-                qbr[s] = ld_stream16(qg + (int64_t)uc * 1024 + 64);
+                qbr[s] = (WT == PS_Q8_0) ? ld_stream16(qg + (int64_t)uc * 1024 + 64) : make_uint4(0, 0, 0, 0);
                 hr[s] = load_h(uc);
             }
             for (int un0 = 0; un0 < n_units; un0 += PF) {
@@ -792,7 +821,7 @@ __global__ __launch_bounds__(256) void gemm8b_kernel(const GemvParams p) {
                     const uint2 h = hr[s];
                     const int nx = min(un + PF, n_units - 1);
                     qar[s] = ld_stream16(qg + (int64_t)nx * 1024);
-                    qbr[s] = ld_stream16(qg + (int64_t)nx * 1024 + 64);
+                    if (WT == PS_Q8_0) qbr[s] = ld_stream16(qg + (int64_t)nx * 1024 + 64);
                     hr[s] = load_h(nx);
                     unit(un, qa, qb, h);
                 }
@@ -805,15 +834,18 @@ __global__ __launch_bounds__(256) void gemm8b_kernel(const GemvParams p) {
         if (wi == 1) { Nw = p.w[1].N; ldo = p.w[1].ldo; o = p.w[1].out; b = p.w[1].bias; }
         if (wi == 2) { Nw = p.w[2].N; ldo = p.w[2].ldo; o = p.w[2].out; b = p.w[2].bias; }
 #pragma unroll
+        for (int cs = 0; cs < NCS; cs++)
+#pragma unroll
         for (int r = 0; r < 4; r++) {
-            float v = __fadd_rn(acc[1][r], acc[0][r]); // a[k + 4] + a[k]
+            float v = __fadd_rn(acc[cs][1][r], acc[cs][0][r]); // a[k + 4] + a[k]
             v = __fadd_rn(v, __shfl_xor(v, 32, 64));
             v = __fadd_rn(v, __shfl_xor(v, 16, 64));
-            if (EPI == 1 && pass == 0) { yg[r] = v; continue; }
+            if (EPI == 1 && pass == 0) { yg[cs][r] = v; continue; }
             const int64_t row = grp * TR::RG + rqi * 4 + r;
+            const int col = col0 + 4 * cs;
             if (qs == 0 && row < Nw && col < nc) {
                 if (EPI == 1) {
-                    p.w[0].out[(int64_t)(c0 + col) * p.w[0].ldo + row] = ps_silu_mul(yg[r], v);
+                    p.w[0].out[(int64_t)(c0 + col) * p.w[0].ldo + row] = ps_silu_mul(yg[cs][r], v);
                 } else {
                     float val = v;
                     if (b) val = __fadd_rn(val, b[row]);
@@ -868,12 +900,17 @@ static void launch_gemm8m_k(hipStream_t st, const GemvParams &p, const dim3 grid
     psk_note_kernel("gemm8m_kernel<%d, %d, %d>", EPI, NWV, C);
     hipLaunchKernelGGL((gemm8m_kernel<EPI, NWV, C>), grid, dim3(NWV * 64), smem, st, p);
 }
-template <int EPI>
-static void launch_gemm8b(hipStream_t st, const GemvParams &p, const dim3 grid, size_t smem) {
+template <int WT, int EPI, int NWV>
+static void launch_gemm8b_k(hipStream_t st, const GemvParams &p, int64_t n_tasks, int64_t ncg, size_t smem) {
     static unsigned long long attr = 0; // devices that have the attribute
-    if (ps_first_on_device(&attr)) { (void)hipFuncSetAttribute((const void *)gemm8b_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024); }
-    psk_note_kernel("gemm8b_kernel<%d>", EPI);
-    hipLaunchKernelGGL((gemm8b_kernel<EPI>), grid, dim3(256), smem, st, p);
+    if (ps_first_on_device(&attr)) { (void)hipFuncSetAttribute((const void *)gemm8b_kernel<WT, EPI, NWV>, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024); }
+    psk_note_kernel("gemm8b_kernel<%d, %d, %d>", WT, EPI, NWV);
+    hipLaunchKernelGGL((gemm8b_kernel<WT, EPI, NWV>), dim3((unsigned)((n_tasks + NWV - 1) / NWV), (unsigned)ncg), dim3(NWV * 64), smem, st, p);
+}
+template <int WT>
+static void launch_gemm8b(hipStream_t st, const GemvParams &p, int epi, int nwv, int64_t n_tasks, int64_t ncg, size_t smem) {
+    if (nwv == 4) { if (epi) launch_gemm8b_k<WT, 1, 4>(st, p, n_tasks, ncg, smem); else launch_gemm8b_k<WT, 0, 4>(st, p, n_tasks, ncg, smem); }
+    else { if (epi) launch_gemm8b_k<WT, 1, 8>(st, p, n_tasks, ncg, smem); else launch_gemm8b_k<WT, 0, 8>(st, p, n_tasks, ncg, smem); }
 }
 int psk_gemm8(hipStream_t st, int n_cu, const psk_gemv_args &a, ps_act act, int64_t K, int64_t bs) {
     if (a.pro != 0 || a.n_w < 1) return -1;
@@ -902,16 +939,23 @@ int psk_gemm8(hipStream_t st, int n_cu, const psk_gemv_args &a, ps_act act, int6
     const size_t smem = (size_t)(K / unit) * 8 * (wt == PS_Q4_K ? 304 : 144); // [unit][column] records (gemm8_stage)
     const int64_t n_tasks = epi == 1 ? p.w[0].n_groups : p.groups_total;
     int64_t ncg = (bs + 7) / 8;
-    // Q8_0 / Q4_0: k_gemm8.hip, but for Q8_0 products so small that work-groups of four waves, 8 rows x 8 columns each, find a CU each (up to 8 columns, where a wave there
-    // works on 16: half a CU): such a launch lasts as long as ONE wave's chain, and gemm8b's is the shorter one (14336 x 4096, 16 columns: 59.6 us against 76.8; where they
-    // take turns: 24 columns 109 against 77, 511 columns 976 against 336)
-    if (wt != PS_Q4_K && (wt == PS_Q4_0 || (n_tasks + 3) / 4 * ncg > (ncg == 1 ? 2 : 1) * n_cu || smem > 158 * 1024)) return psk_gemm8f(st, n_cu, a, act, K, bs);
-    if (smem > 158 * 1024) return -1;
-    if (wt == PS_Q8_0) {
-        const dim3 grid((unsigned)((n_tasks + 3) / 4), (unsigned)ncg);
-        if (epi) launch_gemm8b<1>(st, p, grid, smem); else launch_gemm8b<0>(st, p, grid, smem);
+    // Q8_0 / Q4_0: k_gemm8.hip, whose waves work on 16 rows x 16 columns, or gemm8b_kernel with 8 columns and a quarter (Q8_0: 8 rows) or half of that per wave, nwv waves to a work-group.
+    // Up to 8 columns the wider wave works on as many that are not there.  By row groups per CU (us, 4096 long rows, 2 and 8 columns, weights out of memory, k_gemm8.hip | gemm8b in fours |
+    // in eights):  Q8_0 (groups of 8)  2: 26 27 | 19 20 | 23 24;  4: 28 28 | 20 21 | 23 24;  8: 32 32 | 28 28 | 26 25;  10: 40 38 | 38 37 | 43 43;  12: 41 39 | 41 38 | 45 43;
+    // 14: 59 56 | 52 48 | 45 44;  32: 115 112 | 106 94 | 92 84;  Q4_0 (groups of 16)  1: 26 25 | 26 27 | 32 33;  3.5: 28 29 | 27 29 | 32 33;  5: 38 37 | 39 41 | 33 34;
+    // 7: 57 54 | 41 42 | 34 34;  16: 111 104 | 76 70 | 59 57;  128256 rows 221 199 | 133 124 | 104 98.  Rows of up to 2048: the same, but that fours are nowhere the better for Q4_0.
+    // More columns: Q8_0 in fours as long as those find a CU each (14336 x 4096, 16 columns: 59.6 us against 76.8; where they take turns: 24 columns 109 against 77, 511 columns 976 against 336)
+    if (wt != PS_Q4_K) {
+        int nwv = 0;
+        if (ncg > 1) nwv = wt == PS_Q8_0 && (n_tasks + 3) / 4 * ncg <= n_cu ? 4 : 0;
+        else if (wt == PS_Q8_0) nwv = n_tasks <= 4 * (int64_t)n_cu ? 4 : n_tasks <= 8 * (int64_t)n_cu || n_tasks > 12 * (int64_t)n_cu ? 8 : 0;
+        else nwv = n_tasks > 4 * (int64_t)n_cu ? 8 : n_tasks > 2 * (int64_t)n_cu && K > 2048 ? 4 : 0;
+        if (!nwv || smem > 158 * 1024) return psk_gemm8f(st, n_cu, a, act, K, bs);
+        if (wt == PS_Q8_0) launch_gemm8b<PS_Q8_0>(st, p, epi, nwv, n_tasks, ncg, smem);
+        else launch_gemm8b<PS_Q4_0>(st, p, epi, nwv, n_tasks, ncg, smem);
         return 0;
     }
+    if (smem > 158 * 1024) return -1;
     // one wave per row group; 16-wave workgroups amortise the LDS staging of the 8 columns, 4-wave workgroups spread a
     // small launch (tree verify, short prefill tails) over all CUs
     int nwv = ((n_tasks + 15) / 16) * ncg < (int64_t)n_cu ? 4 : 16;

@@ -2,6 +2,7 @@
 
 north_star bar: bit-exact greedy token ids, logits within 1e-3 relative.
 """
+import ctypes as C
 import os
 
 import numpy as np
@@ -443,6 +444,33 @@ def test_single_token_attention_without_exchange(ctx, tmp_path, preset, wt, n_ct
                 gm.kv_rollback(5)
             assert ids[0] == ids[1], P
     gm.close()
+
+
+@pytest.mark.parametrize("wt,hidden,kernel", [(2, 12288, "gemm8b_kernel<2, 1, 4>"), (2, 16512, "gemm8b_kernel<2, 1, 8>"), (8, 8064, "gemm8b_kernel<8, 1, 4>"), (8, 8320, "gemm8b_kernel<8, 1, 8>")])
+def test_gate_and_up_of_many_rows_and_few_columns(ctx, oracle, tmp_path, monkeypatch, wt, hidden, kernel):
+    """Gate and up in one launch with SiLU behind them, up to 8 tokens, as many rows as take gemm8b_kernel in fours and eights: logits against the oracle, on bits."""
+    from oracle import binding as B
+    from powerserve_amd import hip, synth
+    heads = 18 if (wt, hidden) == (2, 12288) else 2  # (2304 wide: fours take Q4_0 rows of more than 2048)
+    monkeypatch.setitem(synth.PRESETS, "wide-ff", ("llama", 128 * heads, hidden, 1, heads, heads // 2 if heads == 2 else 6, 128, 512, 1e4, 0, True, 1e-5))
+    d = str(tmp_path / "m")
+    mj = synth.write_model_dir(d, "wide-ff", wt, n_ctx=64, seed=4)
+    cfg = B.make_config(mj["llm_config"])
+    om = oracle.model(cfg, mj["model_arch"], load_tensors(os.path.join(d, "ggml/weights.gguf")), n_threads=16)
+    gm = hip.Model(ctx, d, max_batch=16, n_ctx=64)
+    toks = np.random.default_rng(hidden).integers(0, cfg.vocab_size, 18)
+    at = 0
+    for n in (2, 8, 3, 5):
+        want = om.forward(toks[at:at + n], np.arange(at, at + n), True)
+        got = gm.forward(toks[at:at + n], np.arange(at, at + n), True)[0]
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (n, rel_err(got, want))
+        at += n
+    if "256 CUs" in ctx.name():
+        a, b, c = C.c_double(), C.c_double(), C.c_int()
+        ctx.check(ctx.L.ps_hip_model_bench_matmul(gm.h, 1, 1, 8, C.byref(a), C.byref(b), C.byref(c)))
+        assert ctx.L.ps_hip_last_matmul_kernel().decode() == kernel
+    gm.close()
+    om.close()
 
 
 @pytest.mark.parametrize("preset,wt,chunk", [("small-llama-hs128", 12, 256), ("small-llama-hs128", 12, 512), ("small-llama-hs128", 1015, 384), ("tiny-llama", 8, 256), ("tiny-qwen2", 2, 320)])

@@ -106,7 +106,7 @@ def test_mul_mat_batched(ctx, oracle, hip, wt, K, N, bs):
 @pytest.mark.parametrize("wt", [8, 2])
 @pytest.mark.parametrize("K,N,bs", [(128, 8, 2), (128, 24, 17), (256, 4100, 16), (896, 1000, 33), (256, 9000, 64), (128, 16392, 61), (128, 16392, 90), (640, 8200, 97), (384, 4104, 512)])
 def test_mul_mat_batched_blocks(ctx, oracle, hip, wt, K, N, bs):
-    """The four forms of the Q8_0 / Q4_0 batched mat-mul (one or two column tiles per wave, two to eight waves), each with a ragged last row tile (an odd number of
+    """The Q8_0 / Q4_0 batched mat-mul (which of its forms: test_mul_mat_forms_of_the_block_types) with ragged last row tiles (an odd number of
     Q8_0 row groups among them), ragged columns and odd numbers of stages; block scales of every kind (negative, zero, fp16 denormals: their products round once)."""
     from powerserve_amd import synth
     rng = np.random.default_rng(K + N + bs + wt)
@@ -122,6 +122,33 @@ def test_mul_mat_batched_blocks(ctx, oracle, hip, wt, K, N, bs):
     W = ctx.upload_weight(wt, w, K, N)
     dx, dy = ctx.to_device(x), ctx.empty((bs, N))
     ctx.check(ctx.L.ps_hip_mul_mat(ctx.h, C.byref(dy.tensor()), C.byref(W.tensor()), C.byref(dx.tensor())))
+    got = dy.numpy()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rel_err(got, want), np.flatnonzero(got != want)[:8])
+    W.free()
+
+
+@pytest.mark.parametrize("wt,K,N,bs,kernel", [
+    # k_gemm8.hip: 16 columns a wave in twos and fours, 32 in fours and eights; ragged rows, tiles that do not fill the waves, ragged columns, odd numbers of stages
+    (2, 384, 4099, 13, "gemm8f_kernel<2, 0, 1, 2>"), (8, 128, 4100, 50, "gemm8f_kernel<8, 0, 1, 4>"), (2, 128, 9000, 33, "gemm8f_kernel<2, 0, 1, 4>"), (8, 640, 16392, 61, "gemm8f_kernel<8, 0, 2, 4>"),
+    (2, 384, 15001, 61, "gemm8f_kernel<2, 0, 2, 8>"), (8, 384, 15001, 61, "gemm8f_kernel<8, 0, 2, 8>"), (2, 128, 30007, 50, "gemm8f_kernel<2, 0, 2, 8>"), (8, 896, 30007, 55, "gemm8f_kernel<8, 0, 2, 8>"),
+    # up to 8 columns, by row groups per CU: gemm8b_kernel in fours and eights, and on both sides of every line of psk_gemm8's rule
+    (2, 2176, 8192, 5, "gemm8f_kernel<2, 0, 1, 2>"), (2, 2176, 8193, 5, "gemm8b_kernel<2, 0, 4>"), (2, 2176, 16384, 2, "gemm8b_kernel<2, 0, 4>"), (2, 2048, 16384, 7, "gemm8f_kernel<2, 0, 1, 4>"),
+    (2, 128, 16385, 8, "gemm8b_kernel<2, 0, 8>"), (2, 640, 17003, 3, "gemm8b_kernel<2, 0, 8>"), (8, 128, 8185, 8, "gemm8b_kernel<8, 0, 4>"), (8, 384, 8193, 7, "gemm8b_kernel<8, 0, 8>"),
+    (8, 128, 16384, 2, "gemm8b_kernel<8, 0, 8>"), (8, 256, 16385, 6, "gemm8f_kernel<8, 0, 1, 4>"), (8, 256, 24576, 4, "gemm8f_kernel<8, 0, 1, 4>"), (8, 640, 24583, 5, "gemm8b_kernel<8, 0, 8>"),
+    # the activations' image too large for LDS
+    (2, 18048, 24, 4, "gemm8f_kernel<2, 0, 1, 2>"), (8, 18048, 24, 4, "gemm8f_kernel<8, 0, 1, 2>"), (8, 17920, 24, 4, "gemm8b_kernel<8, 0, 4>")])
+def test_mul_mat_forms_of_the_block_types(ctx, oracle, hip, wt, K, N, bs, kernel):
+    """Which kernel a Q8_0 / Q4_0 product takes on 256 CUs, and its bits."""
+    from powerserve_amd import synth
+    rng = np.random.default_rng(K + N + bs + wt)
+    w = synth.random_blocks(rng, wt, N, K)
+    x = rng.standard_normal((bs, K)).astype(np.float32)
+    want = oracle.mul_mat(wt, w, K, N, x)
+    W = ctx.upload_weight(wt, w, K, N)
+    dx, dy = ctx.to_device(x), ctx.empty((bs, N))
+    ctx.check(ctx.L.ps_hip_mul_mat(ctx.h, C.byref(dy.tensor()), C.byref(W.tensor()), C.byref(dx.tensor())))
+    if "256 CUs" in ctx.name():
+        assert ctx.L.ps_hip_last_matmul_kernel().decode() == kernel
     got = dy.numpy()
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rel_err(got, want), np.flatnonzero(got != want)[:8])
     W.free()
