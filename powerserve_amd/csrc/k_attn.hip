@@ -1694,11 +1694,28 @@ bool psl_attn_decode2(hipStream_t st, int n_cu, const psl_attn_args &a) {
     return true;
 }
 
-// Single token, one launch (attn_decode1_kernel), as long as a work-group's reading of its head's K rows costs less than the two launches it saves: up to 160 K floats of them.  Us per token of
-// two layers, rotation + scores + soft-max.V.p | one launch, at 100, 1000, 2000 and 4000 positions: 14 heads of 64 over 2 kv heads 87.8 93.7 98.2 109.3 | 71.9 79.0 87.7 106.0;
-// 12 of 128 over 2: 92.1 98.6 102.7 115.9 | 76.9 89.0 102.7 124.4; 28 of 128 over 4: 113.9 121.8 128.5 142.4 | 98.3 112.7 123.6 146.8; 32 of 96 over 32: 125.4 140.3 145.0 166.9 | 106.0 127.9 149.2 198.8
-bool psl_attn_decode1_covers(const psl_attn_args &a) {
-    return !a.tree && !a.k16 && a.head_size % 32 == 0 && a.head_size <= 128 && a.n_dims <= a.head_size && a.n_ctx <= 32768 && (int64_t)a.n_kv_hi * a.head_size <= 160 * 1024;
+// Single token, one launch (attn_decode1_kernel): the cache length up to which it is the faster one; 0: not covered.  It saves one or two launches, or attn_decode2_kernel's exchange, and reads a
+// head's K rows once per work-group, through eight L2s for every kv head: 5 to 8 us per layer and 1000 positions for a few kv heads, 17 for 32 of 128.  rope: the rotation's launch is saved as well;
+// else2: attn_decode2_kernel is what it replaces.  Measured over 102 shapes of heads, two layers, us per token with this launch | without, in front of and behind a line (heads x kv heads x size):
+//   attn_decode2, by the cache's size   16x4x64 1000 72 | 74, 1400 79 | 76;  32x8x64 500 79.1 | 80.5, 1000 85 | 82;  16x16x64 100 66 | 73, 500 79 | 73;  8x2x64 1400 70 | 74, 2000 75 | 73;
+//                                       8x2x128 500 72 | 75, 1000 77 | 75;  16x4x128 100 73 | 81, 500 82.1 | 81.7;  32x8x128 500 100 | 101, 1000 106 | 103
+//   groups of six to eight              14x2x64 rope 2500 85 | 94, 3900 98 | 103;  32x4x64 2000 93 | 95, 2500 98 | 97;  28x4x128 rope 2000 113 | 116, 2500 118.3 | 118.1;
+//                                       16x2x128 rope 1600 96 | 97, 2000 100 | 98.5;  48x8x128 600 | 1000 -0.8 | +0.2;  16x2x96 rope 1500 17 % the faster
+//   of five                             40x8x128 500 120.3 | 120.2, 1000 128 | 126;  the same, rope 1280 | 1400 132.6 | 132.7, 2000 140 | 137;  20x4x64 1750 | 2000 -0.2 | +1
+//   one head per kv head                32x32x128 1000 142 | 151, 1280 158 | 153;  rope 1280 157.5 | 157.6, 1600 168 | 160;  40x40x128 2000 182 | 194, 3300 225 | 216;
+//                                       32x32x64 1000 100 | 103, 1400 109 | 105;  8x8x32 1400 76.5 | 78, 2000 84 | 79;  32x32x96 1400 125 | 131, 2000 137 | 134
+//   two to four elsewhere               24x8x96 100 77 | 84, 500 88 | 87;  16x4x96 600 | 1000 -5 | +1;  32x8x32 1400 78 | 82, 2000 86 | 83;  32x16x128 800 | 1150 -4.5 % | +0.1 %
+// The line of a class is its earliest crossing.
+int psl_attn_decode1_until(const psl_attn_args &a, bool rope, bool else2) {
+    if (a.tree || a.k16 || a.head_size % 32 || a.head_size > 128 || a.n_dims > a.head_size || a.n_ctx > 32768) return 0;
+    const int kv = a.n_kv_heads, g = a.n_heads / kv;
+    if (else2) return min(1600, 200 * 1024 / (kv * a.head_size));
+    switch (a.head_size) {
+    case 32: return g >= 6 ? 3500 : kv >= 40 ? 3000 : rope ? 2300 : kv <= 8 ? 1500 : 700;
+    case 64: return g >= 6 ? (rope ? 3400 : 2400) : kv >= 40 || (g == 5 && (rope || kv <= 2)) ? 2400 : g == 5 && kv <= 4 ? 1800 : rope ? 1400 : 1150;
+    case 96: return kv >= 24 || (g >= 6 && (rope || kv <= 2)) ? 1600 : rope ? (kv <= 4 ? 1100 : 850) : kv <= 4 ? 800 : 280;
+    default: return rope ? (g >= 6 ? 1700 : 1280) : kv >= 40 ? 2300 : g == 1 ? 1150 : kv <= 2 ? 1280 : g == 5 ? 500 : 930;
+    }
 }
 void psl_attn_decode1(hipStream_t st, int n_cu, const psl_attn_args &a, bool rope) {
     // channels per work-group: four (the shortest V.p) where the heads' work-groups then fit on the chip side by side, else as many more as it takes

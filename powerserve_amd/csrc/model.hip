@@ -60,9 +60,9 @@ struct ps_hip_model {
     float *attn_xchg = nullptr;    // attn_decode2: scores in flight between workgroups (k_attn.hip)
     unsigned *attn_tick = nullptr; // attn_decode2: [64 * kv head] arrival counters
     size_t graph_hint = 0;                   // KV position the captured step was given as its prefetch hint (n_kv_lo)
-    size_t graph_hi = 0;           // ... the cache length it may be replayed to (which attention launch a long cache gets depends on it)
-    bool step_one = false, graph_one = false; // whether attn_decode1 is in the forward enqueued last, and in the captured step
-    int n_kv_bound = 0;            // cache length the step being enqueued may be replayed to (0: n_ctx)
+    size_t graph_until = 0;        // ... and the cache length up to which its attention launches are the right ones
+    size_t step_until = 0;         // the same of the forward enqueued last (SIZE_MAX: any)
+    int n_kv_bound = 0;            // cache length that the call whose step is being captured comes to (0: n_ctx)
     int n_kv_hint = 0;             // capture of a single-token forward: the lower bound of n_kv its prefetch hint is baked with
     int n_kv_host = 0;             // pos0 + bs of the forward being enqueued eagerly (0 while a graph is captured / replayed)
     float *scores = nullptr, *logits = nullptr, *rope_table = nullptr;
@@ -88,7 +88,7 @@ struct ps_hip_model {
     int attn_chunk = 0;                 // > 0 while such a forward is enqueued: the attention runs chunk by chunk
     hipGraphExec_t step_graph = nullptr;
     hipGraphExec_t fwd1_graph[2] = {nullptr, nullptr}; // single-token forward without / with lm_head (the lowered op-API path)
-    size_t fwd1_hint[2] = {0, 0};
+    size_t fwd1_hint[2] = {0, 0}, fwd1_until[2] = {0, 0};
     uint64_t weight_bytes = 0;
     std::vector<void *> owned;
 };
@@ -293,6 +293,7 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
     aa.kv_stream = kvs_own;
     aa.n_kv_lo = m->n_kv_host > 0 ? m->n_kv_host : (m->n_kv_hint > 0 ? m->n_kv_hint : (int)m->position); // (a hint: rows below it are requested before the device-side position has arrived)
 
+    m->step_until = SIZE_MAX;
     aa.n_kv_hi = m->n_kv_host > 0 ? m->n_kv_host : m->n_kv_bound > 0 ? m->n_kv_bound : (int)f.seq_len;
 
     for (uint32_t L = 0; L < f.n_layers; L++) {
@@ -337,17 +338,18 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         } else if (mm(m, g, a1, dim, bs)) return 2;
 
         aa.kv_stream = kvs_own; aa.dbg = nullptr; // (also when the fused launch declined the shape)
-        // a single token's attention without an exchange, rotation and append with it: where attn_decode2 does not take the shape, and where it would need the rotation's launch in front (16 heads of 64
-        // over 4 kv heads, two layers, us per token behind 100, 500 and 1000 positions: 74.8 75.6 77.9 -> 66.8 71.3 75.5).  Rotated in the mat-vec's epilogue, attn_decode2 is the faster one from a few
-        // hundred positions on (32 heads over 8: 91.4 91.5 92.6 against 87.0 94.8 99.4)
-        const bool rotate = f16 || (!fuse_rope && !fuse_rope_b);
-        const bool one = bs == 1 && !use_tree && one_launch && !fused_qa && !kv16 && (rotate || !psl_attn_decode2_covers(c->n_cu, aa)) && psl_attn_decode1_covers(aa);
+        // a single token's attention without an exchange, rotation and append with it: where attn_decode2 does not take the shape or would need the rotation's launch in front, up to the length that
+        // psl_attn_decode1_until gives.  Rotated in the mat-vec's epilogue, attn_decode2 is the faster one from a few hundred positions on (32 heads over 8, two layers, us per token behind
+        // 100, 500 and 1000 positions: 91.4 91.5 92.6 against 87.0 94.8 99.4)
+        const bool rotate = f16 || (!fuse_rope && !fuse_rope_b), two = psl_attn_decode2_covers(c->n_cu, aa);
+        const int until = bs == 1 && !use_tree && one_launch && !fused_qa && !kv16 && (rotate || !two) ? psl_attn_decode1_until(aa, rotate, two) : 0;
+        const bool one = aa.n_kv_hi <= until;
         if (rotate && !one) psl_rope_append(st, aa, bs);
         bool att_quantized = false;
         if (fused_qa) {
         } else if (one) {
             psl_attn_decode1(st, c->n_cu, aa, rotate);
-            m->step_one = true;
+            m->step_until = std::min(m->step_until, (size_t)until);
         } else if (bs == 1 && !use_tree && kv16 && psl_attn_decode_f16(st, aa)) {
             // fp16-KV decode mode (not bit-exact): split-KV online soft-max over the fp16 mirrors
         } else if (bs == 1 && !use_tree && one_launch && (aa.dbg = psk_gemv_dbg_buf(10, 2), psl_attn_decode2(st, c->n_cu, aa))) { // timeline key 42
@@ -703,7 +705,7 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
     // a captured launch plan like ps_hip_model_decode_greedy does: the first call at a position range runs eagerly and captures.
     const int gk = lm_head ? 1 : 0;
     const bool graphable = n == 1 && !tree && (m->mode & 1) == 0 && m->n_hidden == 0;
-    if (graphable && m->fwd1_graph[gk] && ((size_t)pos[0] < m->fwd1_hint[gk] || (size_t)pos[0] >= m->fwd1_hint[gk] + 1024)) {
+    if (graphable && m->fwd1_graph[gk] && ((size_t)pos[0] < m->fwd1_hint[gk] || (size_t)pos[0] >= m->fwd1_hint[gk] + 1024 || (size_t)pos[0] >= m->fwd1_until[gk])) {
         (void)hipGraphExecDestroy(m->fwd1_graph[gk]); m->fwd1_graph[gk] = nullptr;
     }
     if (graphable && m->fwd1_graph[gk]) {
@@ -715,12 +717,12 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
         if (graphable) { // capture the same launches (nothing executes); the hint stays a lower bound of n_kv for 1024 positions
             hipGraph_t g = nullptr;
             PS_CHECK(c, hipStreamSynchronize(c->stream));
-            m->n_kv_host = 0; m->n_kv_hint = pos[0]; m->n_kv_bound = std::min(pos[0] + 1024, (int)m->cfg.seq_len); // (no host-side n_kv inside a graph: the score grids cover n_ctx)
+            m->n_kv_host = 0; m->n_kv_hint = pos[0]; m->n_kv_bound = pos[0] + 1; // (no host-side n_kv inside a graph: the score grids cover n_ctx)
             PS_CHECK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             const int rc = enqueue_forward(m, 1, lm_head != 0, false);
             const hipError_t e = hipStreamEndCapture(c->stream, &g);
             m->n_kv_hint = 0; m->n_kv_bound = 0;
-            if (!rc && e == hipSuccess && hipGraphInstantiate(&m->fwd1_graph[gk], g, nullptr, nullptr, 0) == hipSuccess) m->fwd1_hint[gk] = (size_t)pos[0];
+            if (!rc && e == hipSuccess && hipGraphInstantiate(&m->fwd1_graph[gk], g, nullptr, nullptr, 0) == hipSuccess) { m->fwd1_hint[gk] = (size_t)pos[0]; m->fwd1_until[gk] = m->step_until; }
             else m->fwd1_graph[gk] = nullptr; // (stay eager)
             if (g) (void)hipGraphDestroy(g);
         }
@@ -856,10 +858,8 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
     // is not far behind (a stale hint costs time, never results)
-    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024 || (m->graph_one && m->position + (size_t)steps > m->graph_hi))) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
-    const size_t hi_now = std::min<size_t>(m->position + std::max<size_t>(1024 + 64, (size_t)steps), m->cfg.seq_len); // (64: a call of a few tokens late in the 1024)
-    if (!m->step_graph) { m->graph_hi = hi_now; m->step_one = false; }
-    m->n_kv_bound = (int)m->graph_hi;
+    m->n_kv_bound = (int)std::min<size_t>(m->position + (size_t)steps, m->cfg.seq_len);
+    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024 || (size_t)m->n_kv_bound > m->graph_until)) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
     const struct bound_guard { ps_hip_model *m; ~bound_guard() { m->n_kv_bound = 0; } } bound{m};
     if ((m->mode & 1) == 0 && !m->step_graph) {
         // first step runs eagerly (also performs every one-time hipFuncSetAttribute), then the identical
@@ -874,7 +874,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         if (rc || e != hipSuccess) { c->err = "decode_greedy: graph capture failed: " + c->err; if (g) (void)hipGraphDestroy(g); return 2; }
         PS_CHECK(c, hipGraphInstantiate(&m->step_graph, g, nullptr, nullptr, 0));
-        m->graph_one = m->step_one;
+        m->graph_until = m->step_until;
         (void)hipGraphDestroy(g);
     }
     for (; s < steps; s++) {

@@ -49,7 +49,7 @@ struct psl_attn_args {
     float *xchg;             // attn_decode2: raw scores in flight between the workgroups of a kv head, [n_kv_heads][4][n_ctx rounded up to 32]; null: not used
     unsigned *tick;          // attn_decode2: [64 * kv head] arrival counters, zeroed once (epoch = ticket / workgroups per head)
     int n_kv_lo;             // attn_decode2: a lower bound of pos0 + 1 known to the host at enqueue time (a prefetch HINT only)
-    int n_kv_hi;             // single token: the cache length up to which this launch may be replayed (chooses between kernels, which hold for any length)
+    int n_kv_hi;             // single token: the longest cache that the call at hand comes to (chooses between kernels, which hold for any length)
     int kv_stream;           // single-token kernels: 1 = the cached K rows / V channels are read with non-temporal loads (the model's whole cache does not fit the memory-side
                              // cache, so nothing of it survives from token to token and it should not displace what does); 0 = plain loads (a small cache is served from there)
 };
@@ -62,7 +62,7 @@ bool psl_attn_decode2(hipStream_t st, int n_cu, const psl_attn_args &a); // sing
 bool psl_attn_decode2_covers(int n_cu, const psl_attn_args &a); // whether it would launch
 size_t psl_attn_decode2_xchg_bytes(int n_kv_heads, int n_ctx);
 // single token: (rope: rotation and KV append,) scores, soft-max and V.p in one launch without an exchange: every work-group makes its head's scores; any group of heads
-bool psl_attn_decode1_covers(const psl_attn_args &a);
+int psl_attn_decode1_until(const psl_attn_args &a, bool rope, bool else2); // the cache length up to which it is the faster one (else2: than psl_attn_decode2); 0: not covered
 void psl_attn_decode1(hipStream_t st, int n_cu, const psl_attn_args &a, bool rope);
 // Q / K / V mat-vec (RMSNorm + quantizer prologue, RoPE + KV append: g.rope set) AND the single-token attention in one launch (k_qkvattn.hip): four launches per decode
 // layer instead of five; false: not covered, the caller issues psk_gemv4 + psl_attn_decode2

@@ -1,4 +1,4 @@
-// A HIP runtime for host-side tests: device memory is host memory with a list of what is allocated, streams run at once, kernels are counted and not run -- but for the two that carry bytes between
+// A HIP runtime for host-side tests: device memory is host memory with a list of what is allocated, streams run at once, kernels are counted and not run (a captured one when its graph is launched) -- but for the two that carry bytes between
 // host and device (csrc/ctx.hip: put_kernel, pin_copy_kernel), which copy.  Loaded in front of the library under test (RTLD_GLOBAL), whose calls it then takes.
 // fake_fail(name, n): the n-th call of that name from now on fails; fake_count(name): calls since the last fake_reset(), launches of a kernel also by its name; fake_stray(): bytes that a kernel would have touched outside an allocation.
 #include <hip/hip_runtime_api.h>
@@ -6,16 +6,19 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <vector>
 
 namespace {
 struct Alloc { size_t bytes; int device; hipMemoryType type; };
 std::map<char *, Alloc> mem;
-std::map<std::string, int> count, fail;
+std::map<std::string, int> count, fail, blocks;
 std::map<const void *, std::string> kernels;
 int current = 0;
 size_t stray = 0;
 hipError_t last = hipSuccess;
 struct Thing { int device; }; // a stream or an event
+using Graph = std::vector<std::string>; // the kernels' names
+Graph *capturing = nullptr;
 hipError_t call(const char *name, hipError_t e = hipSuccess) {
     count[name]++;
     auto f = fail.find(name);
@@ -44,7 +47,7 @@ hipError_t alloc(void **p, size_t bytes, hipMemoryType type) {
 } // namespace
 
 extern "C" {
-void fake_reset() { count.clear(); fail.clear(); stray = 0; last = hipSuccess; }
+void fake_reset() { blocks.clear(); count.clear(); fail.clear(); stray = 0; last = hipSuccess; }
 void fake_fail(const char *name, int n) { fail[name] = n; }
 int fake_count(const char *name) { // (of every name with this in it: a kernel's is mangled)
     int n = 0;
@@ -53,14 +56,19 @@ int fake_count(const char *name) { // (of every name with this in it: a kernel's
     return n;
 }
 size_t fake_stray() { return stray; }
+int fake_blocks(const char *name) { // work-groups of the last launch of such a kernel
+    for (auto &b : blocks)
+        if (b.first.find(name) != std::string::npos) return b.second;
+    return 0;
+}
 
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *, void *, int *) { kernels[host] = name; }
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
-static dim3 no_dim;
-hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *s, hipStream_t *st) { *g = *b = no_dim; *s = 0; *st = nullptr; return hipSuccess; }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t s) {
+static struct { dim3 grid, block; size_t lds; hipStream_t st; } config;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t s, hipStream_t st) { config = {g, b, s, st}; return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *s, hipStream_t *st) { *g = config.grid; *b = config.block; *s = config.lds; *st = config.st; return hipSuccess; }
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t s) {
     if (s && ((Thing *)s)->device != current) return call("hipLaunchKernel", hipErrorInvalidHandle);
     const std::string &n = kernels[f];
     if (n.find("pin_copy_kernel") != std::string::npos) {
@@ -77,9 +85,20 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
             if (bytes[i]) move(((void **)a)[i], v, bytes[i], true, false);
         return hipSuccess;
     }
+    blocks[n] = (int)(grid.x * grid.y * grid.z);
+    if (capturing) { capturing->push_back(n); return hipSuccess; }
     count[n]++;
     return call("hipLaunchKernel");
 }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { capturing = new Graph; return call("hipStreamBeginCapture"); }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { *g = (hipGraph_t)capturing; capturing = nullptr; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *, char *, size_t) { *e = (hipGraphExec_t) new Graph(*(Graph *)g); return call("hipGraphInstantiate"); }
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+    for (auto &n : *(Graph *)e) count[n]++;
+    return call("hipGraphLaunch");
+}
+hipError_t hipGraphDestroy(hipGraph_t g) { delete (Graph *)g; return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete (Graph *)e; return hipSuccess; }
 
 hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
 hipError_t hipSetDevice(int d) { current = d; return call("hipSetDevice"); }

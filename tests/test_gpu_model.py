@@ -405,7 +405,7 @@ def test_chunks_attended_in_one_launch(ctx, tmp_path, preset, wt, chunk, P, n_ct
 def test_single_token_attention_without_exchange(ctx, tmp_path, preset, wt, n_ctx):
     """k_attn.hip attn_decode1_kernel (rotation, append, scores, soft-max and V.p of a token in one launch) against the separate launches, on bits: logits, the new K row and V column; an empty
     cache, one position around the groups of 8, blocks of 32, a pass of 64, the 256 positions and the 512 columns requested up front, a full window (multiples of 32 and not), both rotations,
-    four to 32 channels per work-group, head sizes 32 to 128, groups of 1 to 8 heads; eager, captured and behind hidden positions."""
+    four channels per work-group, head sizes 32 to 128, groups of 1 to 8 heads; eager, captured and behind hidden positions."""
     from powerserve_amd import hip, synth
     d = str(tmp_path / "m")
     mj = synth.write_model_dir(d, preset, wt, n_ctx=n_ctx, seed=5)
@@ -443,6 +443,43 @@ def test_single_token_attention_without_exchange(ctx, tmp_path, preset, wt, n_ct
                 ids.append(gm.decode_greedy(int(toks[P]), 5).tolist())
                 gm.kv_rollback(5)
             assert ids[0] == ids[1], P
+    gm.close()
+
+
+@pytest.mark.parametrize("name,n_ctx", [("wide-8", 1060), ("wide-16", 580), ("wide-32-of-96", 140), ("wide-32-of-32", 580), ("wide-64", 140)])
+def test_single_token_attention_of_many_heads(ctx, tmp_path, monkeypatch, name, n_ctx):
+    """The same with 8, 16, 32 and 64 channels per work-group (tests/test_host_calls.py holds the widths): several passes over 16 channels, every one with its own leftovers and new value; heads of
+    96 in three blocks, heads in one."""
+    from powerserve_amd import synth
+    from test_host_calls import WIDE
+    heads, kv, size, _ = WIDE[name]
+    monkeypatch.setitem(synth.PRESETS, name, ("llama", heads * size, 128, 1, heads, kv, size, 128, 1e4, 0, True, 1e-5))
+    test_single_token_attention_without_exchange(ctx, tmp_path, name, 8, n_ctx)
+
+
+@pytest.mark.parametrize("arch,heads,kv,size,line", [("qwen2", 8, 8, 128, 200), ("llama", 24, 8, 96, 280)])
+def test_single_token_attention_across_its_line(ctx, tmp_path, monkeypatch, arch, heads, kv, size, line):
+    """Greedy calls in front of, up to and across the cache length from which another launch takes the attention, and single tokens on both sides: captured steps that are replayed, dropped and
+    captured anew give what the separate launches give."""
+    from powerserve_amd import hip, synth
+    monkeypatch.setitem(synth.PRESETS, "line", (arch, heads * size, 256, 2, heads, kv, size, 512, 1e4, 2 if arch == "qwen2" else 0, True, 1e-5))
+    d = str(tmp_path / "m")
+    synth.write_model_dir(d, "line", 8, n_ctx=512, seed=6)
+    gm = hip.Model(ctx, d, max_batch=64, n_ctx=512)
+    toks = np.random.default_rng(line).integers(0, 512, line - 50)
+    out = []
+    for mode in (16, 0):
+        gm.set_mode(mode)
+        gm.kv_rollback(gm.position)
+        gm.prefill(toks, 64)
+        got = [gm.decode_greedy(int(toks[0]), n) for n in (8, 42, 9, 30)]  # (the second ends at the line)
+        gm.kv_rollback(60)
+        got += [gm.decode_greedy(3, 60), gm.decode_greedy(4, 5)]           # across the line in one call
+        gm.kv_rollback(gm.position - line + 3)
+        for t in range(6):
+            got.append(gm.forward([t], [gm.position], True)[0].view(np.int32).ravel())
+        out.append(np.concatenate(got))
+    assert np.array_equal(out[0], out[1])
     gm.close()
 
 

@@ -22,9 +22,9 @@ def refused(f):
     except hip.PSHipError as e: return str(e)
     raise AssertionError("accepted")
 L = synth.seq_layer
-def quant(ctx, max_batch):
-    synth.write_model_dir({tmp!r} + "/quant", "tiny-llama", 8, n_ctx=1024, seed=1)
-    return hip.Model(ctx, {tmp!r} + "/quant", max_batch=max_batch, n_ctx=1024)
+def quant(ctx, max_batch, preset="tiny-llama", n_ctx=1024):
+    synth.write_model_dir({tmp!r} + "/quant", preset, 8, n_ctx=n_ctx, seed=1)
+    return hip.Model(ctx, {tmp!r} + "/quant", max_batch=max_batch, n_ctx=n_ctx)
 def seq(ctx, max_batch=8, vocab=30):
     cfg = synth.seq_config(24, vocab, [L("delta", 20, heads=4, kv_heads=2, dim=6, vdim=10, conv=4), L("wkv", None, heads=3, dim=8)], taps=3)
     synth.write_seq_model_dir({tmp!r} + "/seq", cfg, 1)
@@ -159,7 +159,6 @@ for n, launches in ((12, 1), (139, 6), (140, 0), (512, 0)):
     m.forward_tree(t, np.arange(n), see)
     assert (count("put_kernel"), count("hipMemcpyAsync")) == (launches, 0 if launches else 3), (n, count("put_kernel"), count("hipMemcpyAsync"))
     assert fake.fake_stray() == 0
-m.set_mode(1)
 q = seq(ctx)
 s = q.acquire()
 for f in (lambda: m.forward_tree([1, 2], [0, 1], np.tril(np.ones((2, 2), np.uint8))), lambda: m.forward_tree(np.arange(500), np.arange(500), np.ones((500, 500), np.uint8)),
@@ -177,3 +176,57 @@ for f in (lambda: m.forward_tree([1, 2], [0, 1], np.tril(np.ones((2, 2), np.uint
         m.kv_rollback(m.position)
         at = q.position(s)
 """)
+
+
+@pytest.mark.parametrize("arch,heads,kv,size,line", [("qwen2", 16, 4, 64, 800), ("qwen2", 14, 2, 64, 3400), ("qwen2", 8, 8, 128, 200), ("qwen2", 40, 8, 128, 1280), ("llama", 24, 8, 96, 280),
+                                                     ("llama", 32, 32, 128, 1150), ("llama", 40, 8, 128, 500), ("llama", 16, 4, 64, 0)])
+def test_single_token_attention_by_the_length_a_call_comes_to(child, arch, heads, kv, size, line):
+    """attn_decode1_kernel up to a cache length (k_attn.hip psl_attn_decode1_until): eager and captured single tokens and greedy calls on both sides of it.  A captured step that holds the kernel is
+    dropped by the first call that would outgrow the line, a step without it stays; every layer of every token takes the one or the other."""
+    child("""
+arch, heads, kv, size, line = %r
+synth.PRESETS["one"] = (arch, heads * size, 256, 2, heads, kv, size, 512, 1e4, 2 if arch == "qwen2" else 0, True, 1e-5)
+ctx = hip.Ctx(0)
+m = quant(ctx, 64, "one", 3600)
+def took(f, at):
+    if m.position > at: m.kv_rollback(m.position - at)
+    if m.position < at: m.prefill(np.ones(at - m.position, int), 64)
+    fake.fake_reset()
+    f()
+    n, all_ = count("attn_decode1_kernel"), count("attn_decode1_kernel") + count("attn_decode2_kernel") + count("attn_softmax_pv_kernel")
+    return n, all_, count("hipStreamBeginCapture")
+def same(got, want): assert got[:len(want)] == want, (mode, got, want)
+greedy = lambda n: lambda: m.decode_greedy(1, n)
+token = lambda: m.forward([1], [m.position])
+for mode in (0, 1):
+    m.set_mode(mode)
+    if line:
+        at = line - 40
+        same(took(greedy(8), at), (16, 16))
+        same(took(greedy(32), at + 8), (64, 64, 0))     # to the line: replayed
+        same(took(greedy(33), at + 8), (0, 66, 1 - mode))
+        same(took(greedy(4), at + 8), (8 * mode, 8, 0))    # (a step without it is kept)
+        same(took(token, line - 1), (2, 2))
+        same(took(token, line - 1), (2, 2, 0))
+    at = max(line, 8)
+    same(took(token, at), (0, 2))
+    same(took(token, at), (0, 2, 0))
+    same(took(greedy(4), at), (0, 8))
+    m.kv_rollback(m.position)
+""" % ((arch, heads, kv, size, line),))
+
+
+WIDE = {"wide-8": (64, 8, 32, 8), "wide-16": (32, 32, 96, 16), "wide-32-of-96": (48, 48, 96, 32), "wide-32-of-32": (136, 17, 32, 32), "wide-64": (136, 17, 64, 64)}  # heads, kv heads, size, channels
+
+
+@pytest.mark.parametrize("heads,kv,size,channels", WIDE.values(), ids=WIDE.keys())
+def test_channels_per_work_group_of_the_single_token_attention(child, heads, kv, size, channels):
+    """four channels of a head per work-group where all of them then fit on 256 CUs, else as many more as it takes: the shapes that tests/test_gpu_model.py runs have the widths it says"""
+    child("""
+heads, kv, size, channels = %r
+synth.PRESETS["one"] = ("llama", heads * size, 128, 1, heads, kv, size, 128, 1e4, 0, True, 1e-5)
+ctx = hip.Ctx(0)
+m = quant(ctx, 8, "one", 64)
+m.forward([1], [0])
+assert fake.fake_blocks(b"attn_decode1_kernel") == heads * size // channels
+""" % ((heads, kv, size, channels),))
