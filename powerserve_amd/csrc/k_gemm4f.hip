@@ -10,12 +10,12 @@
 //   * eight waves share the columns: 128 rows x 16 CT columns per work-group, one work-group per CU, persistent.  Activations, weights, headers and column metadata come by
 //     global_load_lds_dwordx4 into a ring of three stages of one super-block.  One barrier a quarter into a stage says both that the next stage is there and that the one
 //     before has been left, so that its place is asked for at once -- piece by piece: asked for in one go, the wave stands still while the memory pipe takes them (a stage of
-//     CT = 3: 1.60 us, 1.44 with a piece every other step; the barrier in the middle of the stage leaves the last pieces too little time: 3 % more);
-//   * the operands of the activations are read NY steps ahead, across the stages; the next stage's scales and metadata at the end of this one (1.60 us against 2.0 read when
+//     CT = 3 on an eighth of the chip: 1.60 us, 1.44 with a piece every other step; the barrier in the middle of the stage leaves the last pieces too little time: 3 % more);
+//   * the operands of the activations are read NY steps ahead, across the stages; the next stage's scales and metadata at the end of this one (there 1.60 us against 2.0 read when
 //     needed).  CT = 4 would need 30 registers more than two waves per SIMD have.
-// Measured (with the activations' quantizer in front, k_gemm4k.hip's wide kernel -> this): 4096 x 28672, 512 columns 382 -> 278 us, 203 columns 200 -> 141, 32 columns 59 -> 29;
-// 14336 x 4096, 512 columns 201 -> 169; 4096 x 6144 98 -> 76; 4096 x 4096 69 -> 55.  A stage takes 1.30 us with two column tiles and 1.63 with three on a full chip (1.1 and
-// 1.44 on an eighth of it, where the clock stays up).
+// Measured (with the activations' quantizer in front, k_gemm4k.hip's wide kernel -> this): 4096 x 28672, 512 columns 360 -> 247 us, 203 columns 180 -> 125, 32 columns 57 -> 27;
+// 14336 x 4096, 512 columns 190 -> 150; 4096 x 6144 95 -> 70; 4096 x 4096 68 -> 51.  A stage on a full chip takes 1.26 us with two column tiles and 1.63 with three in a single
+// round of work-groups, 1.17 and 1.37 over several.
 #include "ps_gemv_dev.h"
 
 namespace {
@@ -388,7 +388,8 @@ int psk_gemm4f(hipStream_t st, int n_cu, const psk_gemv_args &a, ps_act act, int
     p.n_tiles = (int)tiles;
     p.n_rb = (int)(a.silu_pair ? (pairs + G4F_NRW / 2 - 1) / (G4F_NRW / 2) : (tiles + G4F_NRW - 1) / G4F_NRW);
     // By the time of a super-block step times the rounds of work-groups: 1.30 us with two column tiles per wave, 1.63 with three (8 row tiles per work-group in both), 0.92 of
-    // k_gemm4k.hip's wide kernel, whose work-groups hold two row tiles and 64 columns and therefore fill the chip first (measured at K = 4096 and 14336, N 4096 .. 28672)
+    // k_gemm4k.hip's wide kernel, whose work-groups hold two row tiles and 64 columns and therefore fill the chip first.  What this picks is within 6 % of the best of the three over
+    // K 1024, 4096 and 14336, N 1024 .. 28672 and 17 .. 512 columns (fourteen of each); the three themselves are up to 2.2 x apart
     const int64_t r2 = g4f_rounds(n_cu, p.n_rb, bs, 32), r3 = g4f_rounds(n_cu, p.n_rb, bs, 48), old = g4f_rounds(n_cu, (tiles / 2 + 7) / 8 * 8, bs, 64);
     if (min(r2 * 130, r3 * 163) >= old * 92) return -1;
     const bool two = r2 * 130 <= r3 * 163;

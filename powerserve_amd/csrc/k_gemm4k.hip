@@ -1379,7 +1379,7 @@ constexpr int g4k_par_lds(const int nwv) { return nwv * ((8 + 4 + 2) * 64 * 16 +
 // chip for 4096 rows; here the eight waves of a work-group take the super-blocks of a round side by side (one row tile), park the sums, and run the reference's chains behind a barrier, wave = accumulator
 // lane.  What bounds it is then the issue of a wave's super-block (building 128 + 128 operand registers is ~350 instructions) and two barriers a round.  The weights come straight into LDS two rounds
 // ahead (global_load_lds_dwordx4: their planes hold a row's 128 + 64 bytes together, the operand wants 8 + 4 of them for every accumulator lane; slots swizzled by the row, two passes at most).
-// Measured, 12 columns, with the activations' quantizer: 4096 rows of 14336 62 -> 27 us, 4096 x 4096 20.7 -> 11.8, 1024 x 4096 20.0 -> 11.1; a tree of 12 behind 700 with the Q4_K_M mix 693 -> 570 us.
+// Measured, 12 columns, with the activations' quantizer: 4096 rows of 14336 62 -> 27 us, 4096 x 4096 20.7 -> 11.8, 1024 x 4096 20.0 -> 11.1; a tree of 12 behind 700 with the Q4_K_M mix (8B's shape, four layers) 659 -> 552 us.
 constexpr int G6P_NW = 8, G6P_RING = 3, G6P_ST = 2048 + 1024 + 64; // waves; rounds of weights; bytes of a wave's super-block: ql, qh, d of the 16 rows as fp32
 constexpr int G6P_D = G6P_NW * 8 * 1024, G6P_W = G6P_D + G6P_NW * 1024, G6P_LDS = G6P_W + G6P_RING * G6P_NW * G6P_ST;
 __device__ __forceinline__ void g6p_dma(const uint8_t *src, const unsigned lds_dst) { // one wave-instruction: lane l's 16 bytes at src go to lds_dst + 16 l
