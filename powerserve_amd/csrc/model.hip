@@ -815,7 +815,7 @@ static int forward_tree_impl(ps_hip_model *m, const int32_t *tokens, int n, cons
     m->n_kv_host = 0;
     if (rc_fw) return rc_fw;
     if (n == 1 && !tree) note_single_token(m);
-    const bool pinned = lm_head && argmax_host && (size_t)n * 4 <= PS_PIN_WAITED && ps_pin_ready(c);
+    const bool pinned = lm_head && argmax_host && (size_t)n * 4 <= PS_PIN_HALF && ps_pin_ready(c);
     if (pinned) ps_pin_copy(c, 0, 0, m->argmax_dev, (size_t)n * 4);
     else if (lm_head && argmax_host) PS_CHECK(c, hipMemcpyAsync(argmax_host, m->argmax_dev, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
     PS_CHECK(c, hipStreamSynchronize(c->stream));

@@ -42,9 +42,10 @@ hipError_t ps_put(hipStream_t st, const ps_piece *p, int n);
 // Device results through pinned memory: ps_pin_copy enqueues a kernel that writes `bytes` (a multiple of four, from a multiple of four) to c->pin + half * PS_PIN_HALF + at; who
 // reads them waits for the stream, or for an event of c->pin_ev recorded behind it, and is done with them before its call returns.  ps_pin_ready: whether there is pinned memory.
 constexpr size_t PS_PIN_HALF = (size_t)2 << 20;
-// What is waited for at once goes this way up to here.  us a call, the runtime's copy into pageable memory and a kernel into pinned with the host's copy behind it: 1 KB 20 and 14, 16 KB 26 and 15,
-// 24 KB 18 and 14; 32 KB 10.5 and 14, 64 KB 12 and 15, 256 KB 19 and 22, 4 MB 222 and 228.
-constexpr size_t PS_PIN_WAITED = 24 * 1024;
+// A copy that the caller waits for (ps_hip_memcpy_d2h: most often a finished forward's logits) goes this way up to here.  us a call, the runtime's copy into pageable memory and a kernel into
+// pinned with the host's copy behind it: 1 KB 21 and 13, 16 KB 25 and 14, 20 KB 17 and 14; 24 KB 11 - 18 and 15, 32 KB 11 and 15, 64 KB 13 and 16, 256 KB 23 and 27, 600 KB 38 and 43.  (Behind
+// work that still runs the kernel stays the faster one by 8 us; asking the stream costs as much.)
+constexpr size_t PS_PIN_WAITED = 20 * 1024;
 bool ps_pin_ready(ps_hip_ctx *c);
 void ps_pin_copy(ps_hip_ctx *c, int half, size_t at, const void *dev, size_t bytes);
 

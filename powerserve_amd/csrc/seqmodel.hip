@@ -994,7 +994,7 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
             if (idx.empty()) continue;
             const int rows = (int)idx.size();
             seq_head(m, m->want, rows);
-            if (row && rows * row <= (n > B ? PS_PIN_HALF : PS_PIN_WAITED) && ps_pin_ready(c)) { // (a call of one portion has nothing to hand on meanwhile)
+            if (row && rows * row <= PS_PIN_HALF && ps_pin_ready(c)) {
                 PS_CHECK(c, take(half)); // (the portion before the last one's: long there)
                 const size_t lb = logits_host ? (size_t)rows * m->d.vocab * 4 : 0;
                 if (logits_host) ps_pin_copy(c, half, 0, m->logits, lb);

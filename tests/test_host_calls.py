@@ -89,18 +89,18 @@ d2h(out.ctypes.data, p, 0)
 """)
 
 
-def test_only_short_results_that_are_waited_for_go_through_pinned_memory(child):
-    """up to 24 KB, where the runtime's copy is the slower one; a portion's rows also above that, up to a half of the pinned memory, where another portion computes meanwhile"""
+def test_results_through_pinned_memory_by_size(child):
+    """a copy that is waited for up to 20 KB, where the runtime's is the slower one; a portion's rows, which come behind its launches, up to a half of the pinned memory"""
     child("""
 ctx = hip.Ctx(0)
 p, out = ctx.malloc(1 << 20), np.zeros(1 << 18, np.float32)
-for n, kernel in ((4, 1), (24576, 1), (24580, 0), (65536, 0), (1 << 20, 0)):
+for n, kernel in ((4, 1), (20480, 1), (20484, 0), (65536, 0), (1 << 20, 0)):
     fake.fake_reset()
     ctx.check(ctx.L.ps_hip_memcpy_d2h(ctx.h, out.ctypes.data, p, n))
     assert (count("pin_copy_kernel"), count("hipMemcpyAsync")) == (kernel, 1 - kernel), n
-m = seq(ctx, 8, 3000)
+m = seq(ctx, 8, 100000)
 s = m.acquire()
-for tokens, want, kernels, copies in ((8, 2, 1, 0), (8, 3, 0, 1), (16, 16, 2, 0)):
+for tokens, want, kernels, copies in ((8, 5, 1, 0), (8, 6, 0, 1), (16, 13, 1, 1)):
     fake.fake_reset()
     m.forward(s, [1] * tokens, want=np.arange(want))
     assert (count("pin_copy_kernel"), count("hipMemcpyAsync")) == (kernels, copies), (tokens, want)
