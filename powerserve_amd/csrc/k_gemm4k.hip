@@ -1635,16 +1635,20 @@ int psk_gemm6k(hipStream_t st, int n_cu, const psk_gemv6_args &a, ps_act act, in
     static const bool off = getenv("PS_NO_GEMM6K") != nullptr; // (A/B switch for measurements)
     const ps_weight *w = a.w;
     if (off || !w || w->dtype != PS_Q6_K || w->K != K || K % 1024 || w->N % 32 || a.ldo % 2 || !act.qf || bs < ps_gemm4k_min_cols()) return -1;
-    // below: k_gemv6.hip's groups of eight columns.  us, those / gemm6k_par_kernel: 14336 x 4096 2 columns 21 / 27, 3 and 4 33 / 27, 5 and more 69 / 26; 4096 x 4096 10.5 / 11.8, 13.7 / 11.5, 24 / 11.6;
-    // 128256 x 4096 119 / 254, 211 / 251, 543 / 252
-    if (bs < 3 || (bs < 5 && w->N / 16 > 2 * (int64_t)n_cu)) return -1;
+    // below: k_gemv6.hip's groups of eight columns, whose time follows the rows, where gemm6k_par_kernel's follows its rounds of one row tile per CU.  us, those / gemm6k_par_kernel, 3 and 4 columns:
+    // K = 14336, N = 1024 16 / 24, 2048 21.5 / 24.4, 4096 33 / 27, 6144 44.5 / 46, 8192 57 / 48; K = 4096 10.5 / 11, 10.4 / 11.1, 13.7 / 11.7, 17.5 / 17.6, 20.4 / 18.8, 12288 26.6 / 28; K = 8192,
+    // N = 1024 12 / 16; K of 1024 and 2048 the same for one round.  2 columns: 14336 x 4096 21 / 27; 5 and more: 69 / 26, and nowhere the slower (4096 x 256 17 / 11, 32768 x 2048 76 / 40)
+    const int64_t tiles = w->N / 16, rounds = (tiles + n_cu - 1) / n_cu;
+    if (bs < 3 || (bs < 5 && (K <= 2048 ? rounds > 1 : rounds > 2 || tiles * 5 < rounds * n_cu * 4))) return -1;
     G6KParams p{};
     p.ql = w->qs; p.qh = w->qh; p.sc = (const int8_t *)w->sc; p.d = (const uint16_t *)w->aux;
     p.out = a.out; p.bias = a.bias; p.residual = a.residual; p.N = w->N; p.ldo = a.ldo;
     p.nsb = (int)(K / 256); p.bs = (int)bs; p.n_tasks = (int)(w->N / 32);
     p.qf = act.qf; p.mf = act.mf;
     const int n_ct = (int)((bs + 15) / 16);
-    if (n_ct == 1) { // (whatever the rows: 12 columns of 128256 x 4096 328 -> 257 us)
+    // (whatever the rows: 12 columns of 128256 x 4096 328 -> 257 us; but of the waves of a round four have no super-block in rows of 1024: 9 to 16 columns, gemm6k_kernel / this, N = 4096 10.9 / 10.2,
+    // 8192 11 / 12.4, 16384 15 / 20, 32768 23.5 / 35)
+    if (n_ct == 1 && (K > 1024 || rounds <= 1)) {
         static unsigned long long attrp = 0;
         if (ps_first_on_device(&attrp)) (void)hipFuncSetAttribute((const void *)gemm6k_par_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G6P_LDS);
         psk_note_kernel("gemm6k_par_kernel");
