@@ -506,9 +506,24 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) { /
 
 // Four neighbouring results of output row t, columns n .. n + 3 (n a multiple of four).  The four go through ONE copy of the epilogue's code, the registers turning by one
 // each time: code that runs a few times per launch has to be fetched first.  Four copies took 7.0 us in the sums of 512 x 2048, one 6.3; the activations of a wide product the same.
+// ODD (dn_odd): rows that no 16-byte store fits, number by number.  A form of the kernels of its own: through the loop 282 x 10173 of K = 2304 took 41.5 us (36.4 in four copies, 33.5 so), and a
+// branch for it in the other form costs a prompt of experts 1 %.
+template <bool ODD>
 static __device__ __forceinline__ void dn_put4(const dn_args &g, long long t, long long n, dn_f4 acc) {
     if (n >= g.N) return;
-    if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR || g.em_table || n + 4 > g.N || g.ldo % 4 || ((uintptr_t)g.out & 15)) {
+    if constexpr (ODD) {
+        if (g.act == PSD_ACT_NONE && !g.bias && !g.accum && !g.out_scale && !g.out16) { // (uniform)
+            float *p = g.out + t * g.ldo + n;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + e < g.N) p[e] = acc[e] * g.alpha;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) dn_put<true>(g, t, n + e, acc[e], 0.f, n + e < g.N);
+        }
+        return;
+    }
+    if (__builtin_expect(g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR || g.em_table != nullptr, 0)) { // (uniform; out of the others' way: a prompt of experts 6 255 -> 6 206 us)
 #pragma unroll 1
         for (int e = 0; e < 4; e++) {
             dn_put<true>(g, t, n + e, acc[0], acc[1], n + e < g.N); // (a pair is stored by its even row)
@@ -567,7 +582,7 @@ static __device__ __forceinline__ bool dn_ring_rows(const dn_args &g, int tm, in
     return t0 < T;
 }
 
-template <typename WT, int BM, int BN>
+template <typename WT, int BM, int BN, bool ODD>
 __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p) {
     extern __shared__ __attribute__((aligned(16))) char dn_lds[];
     constexpr int MI = BM / 64, NJ = BN / 64, NI = (BM + BN) / 32, STAGE = (BM + BN) * 128, NS = DN_STAGES; // instruction tiles per wave, pieces a loading wave requests per block
@@ -745,7 +760,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     const int c = (tid % (BN / 4)) * 4;
     for (int r = tid / (BN / 4); r < BM; r += 512 / (BN / 4)) {
         if (t0 + r >= T) break;
-        dn_put4(g, dn_orow(g, row0, t0 + r, T), n0 + c, *(const dn_f4 *)&tile[r * LD + c]);
+        dn_put4<ODD>(g, dn_orow(g, row0, t0 + r, T), n0 + c, *(const dn_f4 *)&tile[r * LD + c]);
     }
 }
 
@@ -754,7 +769,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
 // a lane's registers straight to the result 10.3 too (32-byte pieces).
 // A work-group that took the tiles of all four waves had one wave per SIMD of 256 CUs at work and sixteen columns of a row to write one behind the other: 14 us for
 // the splits of 512 x 2048, 16 for those of 512 x 8; 5.7 and 4.8 now.
-template <int BM, int BN>
+template <int BM, int BN, bool ODD>
 __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p) {
     constexpr int MI = BM / 64, NJ = BN / 64, IJ = MI * NJ;
     __shared__ __attribute__((aligned(16))) float turn[32 * 36];
@@ -776,7 +791,7 @@ __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p)
     *(dn_f4 *)&turn[(lane & 31) * 36 + 8 * q + 4 * (lane >> 5)] = acc;
     __syncthreads();
     const int r = tid >> 3, c = (tid & 7) * 4, t = t0 + wm * MI * 32 + (ij / NJ) * 32 + r;
-    if (t < T) dn_put4(g, dn_orow(g, row0, t, T), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + c, *(const dn_f4 *)&turn[r * 36 + c]);
+    if (t < T) dn_put4<ODD>(g, dn_orow(g, row0, t, T), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + c, *(const dn_f4 *)&turn[r * 36 + c]);
 }
 
 // Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
@@ -801,14 +816,17 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int group
     return best;
 }
 
-template <typename WT, int BM, int BN>
+static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR && !g.em_table && (g.N % 4 || g.ldo % 4 || ((uintptr_t)g.out & 15)); }
+template <typename WT, int BM, int BN, bool ODD>
 static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
+    if constexpr (!ODD)
+        if (dn_odd(g)) return dn_launch_ring<WT, BM, BN, true>(st, g, p);
     constexpr int LDS = DN_STAGES * (BM + BN) * 128;
     static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN, ODD>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     const unsigned grid = (unsigned)((p.tn * p.S + 7) / 8 * 8) * p.n_tm;
-    hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN>), dim3(grid), dim3(512), LDS, st, g, p);
-    if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
+    hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN, ODD>), dim3(grid), dim3(512), LDS, st, g, p);
+    if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN, ODD>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
 }
 
 // the wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed
@@ -833,9 +851,9 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
         const int64_t pb = ((int64_t)a.T * (g.K / 8) + 255) / 256;
         hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192), (unsigned)copies), dim3(256), 0, st, g, (WT *)a.pack);
     }
-    if (r.BM == 128) dn_launch_ring<WT, 128, 128>(st, g, p);
-    else if (r.BN == 128) dn_launch_ring<WT, 64, 128>(st, g, p);
-    else dn_launch_ring<WT, 64, 64>(st, g, p);
+    if (r.BM == 128) dn_launch_ring<WT, 128, 128, false>(st, g, p);
+    else if (r.BN == 128) dn_launch_ring<WT, 64, 128, false>(st, g, p);
+    else dn_launch_ring<WT, 64, 64, false>(st, g, p);
     return true;
 }
 

@@ -236,6 +236,16 @@ def test_dense_matmul_stored_in_fours(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
 
 
+# the same with an activation, a bias or a sum behind rows that no 16-byte store fits (k_dense.hip dn_put4<true>), in the product and in the sums of its splits
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,ff", [(64, 130), (128, 258), (4160, 67)])
+def test_odd_rows_behind_an_epilogue(made, dtype, width, ff):
+    cfg = synth.seq_config(width, 50, [L("wkv", ff, heads=2, dim=16)], taps=2)
+    m, cfg, t = made("odd-%d" % width, dtype, max_batch=64, cfg=cfg)
+    toks = tokens_for(cfg, 75, seed=ff)
+    assert err(run_portions(m, toks, [64, 11]), seq_oracle.run(cfg, t, toks)) < TOL[dtype]
+
+
 # K up to 32 (k_dense.hip dense_mm_few_kernel): one below, at and above its two widths (33: the tiled kernel), one token and one column more and less than a work-group's
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(9, 1, 1), (15, 255, 7), (16, 256, 8), (17, 257, 9), (33, 70, 31), (31, 513, 32), (40, 65, 33)])
