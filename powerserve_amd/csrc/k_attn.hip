@@ -1696,25 +1696,39 @@ bool psl_attn_decode2(hipStream_t st, int n_cu, const psl_attn_args &a) {
 
 // Single token, one launch (attn_decode1_kernel): the cache length up to which it is the faster one; 0: not covered.  It saves one or two launches, or attn_decode2_kernel's exchange, and reads a
 // head's K rows once per work-group, through eight L2s for every kv head: 5 to 8 us per layer and 1000 positions for a few kv heads, 17 for 32 of 128.  rope: the rotation's launch is saved as well;
-// else2: attn_decode2_kernel is what it replaces.  Measured over 102 shapes of heads, two layers, us per token with this launch | without, in front of and behind a line (heads x kv heads x size):
+// else2: attn_decode2_kernel is what it replaces.  Measured over 540 shapes (groups of 1 to 8 heads, 1 to 40 kv heads, 100 to 3300 positions in windows of 2048, 3428 and 4096), two layers; us per
+// token with this launch | without, in front of a line and behind it (heads x kv heads x size):
 //   attn_decode2, by the cache's size   16x4x64 1000 72 | 74, 1400 79 | 76;  32x8x64 500 79.1 | 80.5, 1000 85 | 82;  16x16x64 100 66 | 73, 500 79 | 73;  8x2x64 1400 70 | 74, 2000 75 | 73;
 //                                       8x2x128 500 72 | 75, 1000 77 | 75;  16x4x128 100 73 | 81, 500 82.1 | 81.7;  32x8x128 500 100 | 101, 1000 106 | 103
 //   groups of six to eight              14x2x64 rope 2500 85 | 94, 3900 98 | 103;  32x4x64 2000 93 | 95, 2500 98 | 97;  28x4x128 rope 2000 113 | 116, 2500 118.3 | 118.1;
-//                                       16x2x128 rope 1600 96 | 97, 2000 100 | 98.5;  48x8x128 600 | 1000 -0.8 | +0.2;  16x2x96 rope 1500 17 % the faster
-//   of five                             40x8x128 500 120.3 | 120.2, 1000 128 | 126;  the same, rope 1280 | 1400 132.6 | 132.7, 2000 140 | 137;  20x4x64 1750 | 2000 -0.2 | +1
-//   one head per kv head                32x32x128 1000 142 | 151, 1280 158 | 153;  rope 1280 157.5 | 157.6, 1600 168 | 160;  40x40x128 2000 182 | 194, 3300 225 | 216;
-//                                       32x32x64 1000 100 | 103, 1400 109 | 105;  8x8x32 1400 76.5 | 78, 2000 84 | 79;  32x32x96 1400 125 | 131, 2000 137 | 134
-//   two to four elsewhere               24x8x96 100 77 | 84, 500 88 | 87;  16x4x96 600 | 1000 -5 | +1;  32x8x32 1400 78 | 82, 2000 86 | 83;  32x16x128 800 | 1150 -4.5 % | +0.1 %
-// The line of a class is its earliest crossing.
+//                                       16x2x128 rope 1600 96 | 97, 2000 100 | 98.5;  12x2x128 1000 -7 %, 1600 +1;  16x2x96 rope 1500 -17 %
+//   of five                             40x8x128 100 109 | 115, 500 120.3 | 120.2;  the same, rope 1280 132.5 | 133, 2000 140 | 137;  20x4x64 1750 -0.4 us, 2000 +2
+//   of one to four                      32x32x128 1000 142 | 151, 1280 158 | 153;  rope 1280 157.5 | 157.6, 1600 168 | 160;  40x40x128 2000 182 | 194, 3300 225 | 216;
+//                                       32x32x64 1000 100 | 103, 1400 109 | 105;  8x8x32 1400 76.5 | 78, 2000 84 | 79;  32x32x96 1400 125 | 131, 2000 137 | 134;  24x8x96 100 77 | 84, 750 91 | 88.5
+// The line of a class is its earliest crossing: no token of any of them is slower by more than 1.2 %, and of the 7.4 % that the better of the two would save on average 7.0 are left.
 int psl_attn_decode1_until(const psl_attn_args &a, bool rope, bool else2) {
     if (a.tree || a.k16 || a.head_size % 32 || a.head_size > 128 || a.n_dims > a.head_size || a.n_ctx > 32768) return 0;
     const int kv = a.n_kv_heads, g = a.n_heads / kv;
-    if (else2) return min(1600, 200 * 1024 / (kv * a.head_size));
+    if (else2) return min(a.head_size == 64 ? 1700 : 880, 220 * 1024 / (kv * a.head_size));
     switch (a.head_size) {
-    case 32: return g >= 6 ? 3500 : kv >= 40 ? 3000 : rope ? 2300 : kv <= 8 ? 1500 : 700;
-    case 64: return g >= 6 ? (rope ? 3400 : 2400) : kv >= 40 || (g == 5 && (rope || kv <= 2)) ? 2400 : g == 5 && kv <= 4 ? 1800 : rope ? 1400 : 1150;
-    case 96: return kv >= 24 || (g >= 6 && (rope || kv <= 2)) ? 1600 : rope ? (kv <= 4 ? 1100 : 850) : kv <= 4 ? 800 : 280;
-    default: return rope ? (g >= 6 ? 1700 : 1280) : kv >= 40 ? 2300 : g == 1 ? 1150 : kv <= 2 ? 1280 : g == 5 ? 500 : 930;
+    case 32:
+        if (g >= 5 || kv >= 40) return 3300;
+        if (rope) return g == 4 ? 2150 : g == 3 ? 3000 : g == 2 ? 1650 : kv <= 24 ? 1150 : 700;
+        return g == 4 ? 1400 : g == 3 ? 1700 : kv <= 12 ? 1100 : 340;
+    case 64:
+        if (kv >= 40) return 2300;
+        if (g >= 6) return rope ? (kv <= 8 ? 3300 : 2400) : kv <= 8 ? 2250 : 1100;
+        if (g == 5) return rope ? 2000 : kv <= 3 ? 3000 : kv <= 6 ? 2000 : 230;
+        return rope ? 1600 : 1200;
+    case 96:
+        if (kv >= 12) return rope ? 1750 : 1450;
+        if (rope) return g >= 5 ? 1700 : g == 4 ? 1400 : g == 3 ? 1250 : g == 2 ? 1050 : 800;
+        return kv <= 2 ? 1450 : kv == 3 ? 1200 : g >= 7 ? 1000 : kv <= 6 && g >= 5 ? 880 : kv == 4 ? 850 : 390;
+    default:
+        if (kv >= 40) return 2300;
+        if (rope) return g >= 7 ? 1850 : 1350;
+        if (g <= 4) return 1160;
+        return kv == 1 ? 2000 : kv == 2 ? 1340 : g >= 7 || kv == 3 ? 1000 : kv == 4 ? 730 : 250;
     }
 }
 void psl_attn_decode1(hipStream_t st, int n_cu, const psl_attn_args &a, bool rope) {

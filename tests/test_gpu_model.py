@@ -457,7 +457,7 @@ def test_single_token_attention_of_many_heads(ctx, tmp_path, monkeypatch, name, 
     test_single_token_attention_without_exchange(ctx, tmp_path, name, 8, n_ctx)
 
 
-@pytest.mark.parametrize("arch,heads,kv,size,line", [("qwen2", 8, 8, 128, 200), ("llama", 24, 8, 96, 280)])
+@pytest.mark.parametrize("arch,heads,kv,size,line", [("qwen2", 8, 8, 128, 220), ("llama", 24, 8, 96, 390)])
 def test_single_token_attention_across_its_line(ctx, tmp_path, monkeypatch, arch, heads, kv, size, line):
     """Greedy calls in front of, up to and across the cache length from which another launch takes the attention, and single tokens on both sides: captured steps that are replayed, dropped and
     captured anew give what the separate launches give."""
