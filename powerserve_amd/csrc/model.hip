@@ -89,6 +89,7 @@ struct ps_hip_model {
     hipGraphExec_t step_graph = nullptr;
     hipGraphExec_t fwd1_graph[2] = {nullptr, nullptr}; // single-token forward without / with lm_head (the lowered op-API path)
     size_t fwd1_hint[2] = {0, 0}, fwd1_until[2] = {0, 0};
+    int graph_late = 0, fwd1_late[2] = {0, 0}; // tokens of each plan since its hint fell behind (plan_outlived)
     uint64_t weight_bytes = 0;
     std::vector<void *> owned;
 };
@@ -622,6 +623,15 @@ int ps_hip_model_kv_append_tokens(ps_hip_model *m, size_t n, size_t *old_positio
 
 static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, const int32_t *pos, const uint8_t *tree, int lm_head,
                               int32_t *argmax_host, bool advance, bool retried = false);
+// The position that a captured plan was made at is its prefetch hint, a LOWER bound: never above the position, not a thousand behind it.  attn_decode1_kernel (until: plans with it have one)
+// requests up to 512 positions early and waits for the position before it requests what lies behind the hint: 8 kv heads of 96, two layers, 89 us per token behind 549 positions with a hint of 100,
+// 84 with one of 549 (and 86.6 without the kernel).  A new plan costs 75 us a layer for a few layers and 40 for many, what 20 to 40 tokens save: made once as many as `late` counts were late.
+static bool plan_outlived(size_t hint, size_t until, size_t pos, int steps, int &late) {
+    if (pos < hint || pos >= hint + 1024) return true;
+    if (until == SIZE_MAX || hint >= 480 || pos < hint + hint / 2 + 96) return false;
+    late += std::min(steps, 32);
+    return late >= 32;
+}
 // The one-launch attentions wait for each other's workgroups inside the launch (bounded); a wait that gave up raises
 // attn_sync[31].  Read it behind every synchronised single-token forward, clear it, and fall back to the two launches
 // from here on (mode bit 4): the forward that timed out has no valid result.  Expects the stream to be idle.
@@ -705,7 +715,7 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
     // a captured launch plan like ps_hip_model_decode_greedy does: the first call at a position range runs eagerly and captures.
     const int gk = lm_head ? 1 : 0;
     const bool graphable = n == 1 && !tree && (m->mode & 1) == 0 && m->n_hidden == 0;
-    if (graphable && m->fwd1_graph[gk] && ((size_t)pos[0] < m->fwd1_hint[gk] || (size_t)pos[0] >= m->fwd1_hint[gk] + 1024 || (size_t)pos[0] >= m->fwd1_until[gk])) {
+    if (graphable && m->fwd1_graph[gk] && ((size_t)pos[0] >= m->fwd1_until[gk] || plan_outlived(m->fwd1_hint[gk], m->fwd1_until[gk], (size_t)pos[0], 1, m->fwd1_late[gk]))) {
         (void)hipGraphExecDestroy(m->fwd1_graph[gk]); m->fwd1_graph[gk] = nullptr;
     }
     if (graphable && m->fwd1_graph[gk]) {
@@ -722,7 +732,7 @@ static int model_forward_impl(ps_hip_model *m, const int32_t *tokens, int n, con
             const int rc = enqueue_forward(m, 1, lm_head != 0, false);
             const hipError_t e = hipStreamEndCapture(c->stream, &g);
             m->n_kv_hint = 0; m->n_kv_bound = 0;
-            if (!rc && e == hipSuccess && hipGraphInstantiate(&m->fwd1_graph[gk], g, nullptr, nullptr, 0) == hipSuccess) { m->fwd1_hint[gk] = (size_t)pos[0]; m->fwd1_until[gk] = m->step_until; }
+            if (!rc && e == hipSuccess && hipGraphInstantiate(&m->fwd1_graph[gk], g, nullptr, nullptr, 0) == hipSuccess) { m->fwd1_hint[gk] = (size_t)pos[0]; m->fwd1_until[gk] = m->step_until; m->fwd1_late[gk] = 0; }
             else m->fwd1_graph[gk] = nullptr; // (stay eager)
             if (g) (void)hipGraphDestroy(g);
         }
@@ -859,7 +869,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
     // is not far behind (a stale hint costs time, never results)
     m->n_kv_bound = (int)std::min<size_t>(m->position + (size_t)steps, m->cfg.seq_len);
-    if (m->step_graph && (m->position < m->graph_hint || m->position >= m->graph_hint + 1024 || (size_t)m->n_kv_bound > m->graph_until)) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
+    if (m->step_graph && ((size_t)m->n_kv_bound > m->graph_until || plan_outlived(m->graph_hint, m->graph_until, m->position, steps, m->graph_late))) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
     const struct bound_guard { ps_hip_model *m; ~bound_guard() { m->n_kv_bound = 0; } } bound{m};
     if ((m->mode & 1) == 0 && !m->step_graph) {
         // first step runs eagerly (also performs every one-time hipFuncSetAttribute), then the identical
@@ -875,6 +885,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
         if (rc || e != hipSuccess) { c->err = "decode_greedy: graph capture failed: " + c->err; if (g) (void)hipGraphDestroy(g); return 2; }
         PS_CHECK(c, hipGraphInstantiate(&m->step_graph, g, nullptr, nullptr, 0));
         m->graph_until = m->step_until;
+        m->graph_late = 0;
         (void)hipGraphDestroy(g);
     }
     for (; s < steps; s++) {

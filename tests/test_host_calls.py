@@ -216,6 +216,32 @@ for mode in (0, 1):
 """ % ((arch, heads, kv, size, line),))
 
 
+
+def test_a_captured_step_is_made_again_when_its_hint_is_far_behind(child):
+    """csrc/model.hip plan_outlived: a plan with attn_decode1_kernel made behind 100 positions outlives 246 by 31 tokens, greedy or one by one; one made behind 480, and one without the kernel, by 1024"""
+    child("""
+def go(preset, lines):
+    m = quant(ctx, 64, preset, 3600)
+    def made(f, at):
+        if m.position > at: m.kv_rollback(m.position - at)
+        if m.position < at: m.prefill(np.ones(at - m.position, int), 64)
+        fake.fake_reset()
+        f()
+        return count("hipStreamBeginCapture")
+    greedy = lambda n: lambda: m.decode_greedy(1, n)
+    token = lambda: m.forward([1], [m.position])
+    for at, n, want in lines: assert made(greedy(n), at) == want, (preset, at, n)
+    m.kv_rollback(m.position)
+    for at, n, want in lines: assert sum(made(token, at) for _ in range(n)) == want, (preset, at, n)
+    m.close()
+synth.PRESETS["with"] = ("qwen2", 14 * 64, 256, 1, 14, 2, 64, 512, 1e4, 2, True, 1e-5)
+synth.PRESETS["without"] = ("llama", 16 * 64, 256, 1, 16, 4, 64, 512, 1e4, 0, True, 1e-5)
+ctx = hip.Ctx(0)
+go("with", [(100, 1, 1), (200, 40, 0), (245, 1, 0), (246, 16, 0), (300, 15, 0), (300, 1, 1), (300, 40, 0), (545, 40, 0), (546, 40, 1), (1569, 40, 0), (1570, 1, 1), (0, 1, 1), (95, 1, 0), (96, 32, 1)])
+go("without", [(100, 1, 1), (300, 40, 0), (1123, 1, 0), (1124, 1, 1), (480, 1, 1), (1503, 1, 0), (1504, 1, 1)])
+""")
+
+
 WIDE = {"wide-8": (64, 8, 32, 8), "wide-16": (32, 32, 96, 16), "wide-32-of-96": (48, 48, 96, 32), "wide-32-of-32": (136, 17, 32, 32), "wide-64": (136, 17, 64, 64)}  # heads, kv heads, size, channels
 
 
