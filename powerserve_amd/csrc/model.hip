@@ -867,7 +867,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, 1, 0);
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
-    // is not far behind (a stale hint costs time, never results)
+    // is not far behind (plan_outlived: a stale hint costs time, never results)
     m->n_kv_bound = (int)std::min<size_t>(m->position + (size_t)steps, m->cfg.seq_len);
     if (m->step_graph && ((size_t)m->n_kv_bound > m->graph_until || plan_outlived(m->graph_hint, m->graph_until, m->position, steps, m->graph_late))) { (void)hipGraphExecDestroy(m->step_graph); m->step_graph = nullptr; }
     const struct bound_guard { ps_hip_model *m; ~bound_guard() { m->n_kv_bound = 0; } } bound{m};
