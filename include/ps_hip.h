@@ -455,7 +455,8 @@ typedef struct ps_seq_layer_s {
 
 typedef struct {
     int32_t n_layers, width, vocab, canon_taps;
-    int32_t max_batch;   /* most tokens one launch sequence takes; longer inputs are cut into portions of this size */
+    int32_t max_batch;   /* tokens the step function is asked for at a time, and most rows of logits it makes at a time.  A longer input is cut into launch sequences of this size, or (from 64 on)
+                          * of up to four times as many tokens, no more than 2048 or max_context, where the memory for that is there */
     int32_t n_slots;     /* sequence states held at once */
     int32_t compute;     /* 0: bfloat16 matrix products, 1: fp32 */
     float norm_eps, norm_offset /* weight applied as (offset + w) */, logit_scale;

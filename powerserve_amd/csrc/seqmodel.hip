@@ -54,6 +54,7 @@ struct ps_hip_seq {
     ps_hip_ctx *ctx = nullptr;
     ps_seq_desc d;
     std::vector<LayerPlan> L; // layer runs in execution order
+    int64_t rows = 0;         // most tokens of a launch sequence: max_batch, or more of them where a long input is cut (seq_rows)
     int64_t max_context = 0;
     bool needs_context = false; // some mixer's memory grows with the sequence: a sequence may hold at most max_context tokens
     float embed_scale = 1.f;
@@ -64,13 +65,13 @@ struct ps_hip_seq {
     float *x = nullptr, *hn = nullptr, *h = nullptr, *y = nullptr, *t1 = nullptr, *t2 = nullptr, *t3 = nullptr, *t4 = nullptr, *kvx = nullptr, *xn = nullptr,
           *logits = nullptr;
     int32_t *tokens = nullptr, *want = nullptr, *amax = nullptr, *ids = nullptr;
-    float *hist = nullptr;        // depth_mix: [runs + 1][max_batch][width], X_0 = the embedding, run i writes X_(i+1)
+    float *hist = nullptr;        // depth_mix: [runs + 1][rows][width], X_0 = the embedding, run i writes X_(i+1)
     int groups = 1;               // parts of every RMS norm over the width
     int32_t *moe_sel = nullptr, *moe_seg = nullptr, *moe_list = nullptr; // mixture of experts: expert per slot, the slots sorted by expert
     float *moe_wgt = nullptr, *moe_sg = nullptr, *moe_y = nullptr;       // weight per slot, the shared expert's gate per token, per-slot results (top > 1)
     float *win_scratch = nullptr; // the windowed attention's single-token partials
     float *ssd_scratch = nullptr; // the chunked recurrences: a state per chunk (and the matrix memory's gates)
-    float *lstm_aux = nullptr;    // matrix memory: [max_batch][heads] products with n, then as many running maxima
+    float *lstm_aux = nullptr;    // matrix memory: [rows][heads] products with n, then as many running maxima
     int64_t lstm_aux_n = 0;
     uint16_t *a16 = nullptr; // bf16 models: a portion's rows as the kernel in front of a product has rounded them
     float *abs_scratch = nullptr; // the absorbed single-token attention's folded queries, attended latents and per-tile partials
@@ -79,7 +80,7 @@ struct ps_hip_seq {
     float *split = nullptr; // its partial tiles where K is split
     size_t split_bytes = 0;
     int ids_cap = 0;
-    int64_t n_t2q = 0; // t2: [max_batch][q_rank max] then the queries
+    int64_t n_t2q = 0; // t2: [rows][q_rank max] then the queries
     float *dbg_layers = nullptr;
     int mode = 0;
     std::map<int, hipGraphExec_t> graphs; // single-token greedy step, per slot
@@ -113,19 +114,26 @@ static int seq_fail(ps_hip_ctx *c, const std::string &msg) { c->err = msg; retur
 
 static uint64_t dense_bytes(const ps_dense *w) { return w ? (uint64_t)w->N * w->K * (w->dtype == PS_BF16 ? 2 : 4) : 0; }
 
+// Tokens of a launch sequence for an input longer than max_batch.  The wider it is, the fewer launches (5 us of a small one is its start), the larger the tiles that still fill the chip,
+// the fewer partly empty ones of an expert, and the fewer expansions of one window's keys: Ranutar 2048 x 6, 2047 tokens behind max_batch 512 in portions of 512, 1024, 2048: 5552, 4527,
+// 3947 us; Pupidra 2048 x 6, 1500 tokens: 6118, 5060, 4280.  Not below 64, where the caller has asked for little memory; no more than four times what was asked for, and no more than
+// 2048, behind which the tiles fill the chip anyway.
+static int64_t seq_rows(const ps_seq_desc *d) {
+    const int64_t B = d->max_batch, most = d->max_context > 0 ? d->max_context : 65536;
+    return B < 64 ? B : std::max(B, std::min<int64_t>({4 * B, 2048, most}));
+}
+
+// out of memory: the one failure that a narrower launch sequence may mend
+static const int SEQ_NO_MEMORY = -1;
+
 extern "C" {
 
-int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) {
-    *out = nullptr;
-    if (!desc || desc->n_layers <= 0 || desc->width <= 0 || desc->vocab <= 0 || desc->max_batch <= 0 || desc->n_slots <= 0 || desc->canon_taps < 1)
-        return seq_fail(c, "seq_create: bad descriptor");
-    if (!desc->embed || !desc->head || !desc->final_norm) return seq_fail(c, "seq_create: embed / head / final_norm missing");
-    if (desc->embed->K != desc->width || desc->head->K != desc->width || desc->head->N != desc->vocab) return seq_fail(c, "seq_create: embed / head shape");
-    PS_CHECK(c, hipSetDevice(c->device));
+static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, ps_hip_seq **out) {
     auto m = new ps_hip_seq();
     m->ctx = c;
     m->d = *desc;
-    const int64_t W = desc->width, B = desc->max_batch;
+    m->rows = B;
+    const int64_t W = desc->width;
     int64_t off = 0, n1 = 0, n2 = 0, n3 = 0, n4 = 0, n4_one = 0, nkv = 0, nq = 0;
     auto fail = [&](const std::string &msg) { ps_hip_seq_destroy(m); return seq_fail(c, "seq_create: " + msg); };
     auto shape = [](const ps_dense *w, int64_t N, int64_t K) { return w && w->N == N && w->K == K; };
@@ -457,8 +465,8 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
     ok = ok && alloc((void **)&m->step, sizeof(ps_seq_step)) && alloc((void **)&m->x, B * W * 4) && alloc((void **)&m->hn, B * W * 4) && alloc((void **)&m->h, B * W * 4) &&
          alloc((void **)&m->y, B * W * 4) && alloc((void **)&m->t1, B * std::max<int64_t>(n1, 1) * 4) && alloc((void **)&m->t2, B * std::max<int64_t>(n2, 1) * 4) &&
          alloc((void **)&m->t3, B * std::max<int64_t>(n3, 1) * 4) && alloc((void **)&m->t4, std::max<int64_t>({B * n4, n4_one, 1}) * 4) &&
-         alloc((void **)&m->kvx, std::max<int64_t>(nkv, 1) * 4) && alloc((void **)&m->xn, B * W * 4) && alloc((void **)&m->logits, B * (int64_t)desc->vocab * 4) &&
-         alloc((void **)&m->tokens, B * 4) && alloc((void **)&m->want, B * 4) && alloc((void **)&m->amax, B * 4);
+         alloc((void **)&m->kvx, std::max<int64_t>(nkv, 1) * 4) && alloc((void **)&m->xn, desc->max_batch * W * 4) && alloc((void **)&m->logits, desc->max_batch * (int64_t)desc->vocab * 4) &&
+         alloc((void **)&m->tokens, B * 4) && alloc((void **)&m->want, desc->max_batch * 4) && alloc((void **)&m->amax, desc->max_batch * 4);
     if (depth) ok = ok && alloc((void **)&m->hist, (size_t)(order.size() + 1) * B * W * 4);
     if (moe_slots)
         ok = ok && alloc((void **)&m->moe_sel, moe_slots * 4) && alloc((void **)&m->moe_list, moe_slots * 4) && alloc((void **)&m->moe_seg, (moe_experts + 1) * 4) &&
@@ -509,9 +517,28 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
     m->slot_state.assign(desc->n_slots, nullptr);
     m->slot_pos.assign(desc->n_slots, -1);
     for (int s = 0; ok && s < desc->n_slots; s++) ok = alloc((void **)&m->slot_state[s], (size_t)m->state_floats * 4);
-    if (!ok) return fail("out of device memory");
+    if (!ok) {
+        fail("out of device memory");
+        return SEQ_NO_MEMORY;
+    }
     *out = m;
     return 0;
+}
+
+int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) {
+    *out = nullptr;
+    if (!desc || desc->n_layers <= 0 || desc->width <= 0 || desc->vocab <= 0 || desc->max_batch <= 0 || desc->n_slots <= 0 || desc->canon_taps < 1)
+        return seq_fail(c, "seq_create: bad descriptor");
+    if (!desc->embed || !desc->head || !desc->final_norm) return seq_fail(c, "seq_create: embed / head / final_norm missing");
+    if (desc->embed->K != desc->width || desc->head->K != desc->width || desc->head->N != desc->vocab) return seq_fail(c, "seq_create: embed / head shape");
+    PS_CHECK(c, hipSetDevice(c->device));
+    const int64_t rows = seq_rows(desc);
+    int rc = seq_create(c, desc, rows, out);
+    if (rc == SEQ_NO_MEMORY && rows > desc->max_batch) {
+        (void)hipGetLastError();
+        rc = seq_create(c, desc, desc->max_batch, out);
+    }
+    return rc == SEQ_NO_MEMORY ? 2 : rc;
 }
 
 void ps_hip_seq_destroy(ps_hip_seq *m) {
@@ -552,7 +579,7 @@ int ps_hip_seq_set_mode(ps_hip_seq *m, int mode) { m->mode = mode; return 0; }
 
 } // extern "C"
 
-// The launches of one portion: T <= max_batch tokens (device ids in m->tokens, or the step's own token0 when from_step) of the slot whose state
+// The launches of one portion: T <= m->rows tokens (device ids in m->tokens, or the step's own token0 when from_step) of the slot whose state
 // pointer is `state`.  any_pos: a captured sequence that must hold for any position -- whatever depends on the position (the rows of a window's
 // expansion, the visible blocks) is launched for its most and cut on the device; otherwise the step's position is known on the host (pos0).
 static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool any_pos, bool from_step) {
@@ -560,7 +587,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     const ps_seq_desc &D = m->d;
     const int64_t W = D.width;
     const bool tiled = (m->mode & 2) != 0, chunked = T >= CHUNKED_FROM && !tiled && m->ssd_scratch; // a portion's recurrences
-    const int64_t BW = (int64_t)D.max_batch * W;
+    const int64_t BW = m->rows * W, DW = (int64_t)D.max_batch * W; // (results of a run: in `hist`, in the debugging buffer)
     psk_embed(st, D.embed, from_step ? nullptr : m->tokens, m->step, T, m->embed_scale, m->hist ? m->hist : m->x, W, D.bigram, D.bigram_buckets, D.bigram_mul_prev,
               D.bigram_mul_cur);
     // The kernels in front of a portion's products leave a bf16 copy of what they wrote in m->a16 as well: `rounded` says of which buffer, and is forgotten with its contents.
@@ -709,7 +736,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             // t1 = [ dq | dkv ], or with direct queries [ q | dkv | gate ]; the latents' norms, rotation of the shared key part and ring append; attention -> t3; out
             const int64_t dr = l.rot_dim, rs = l.kv_rank + dr, Hv = H * dv, nq = H * (d + dr);
             const bool direct = l.q_rank == 0;
-            float *cq = m->t2, *q = direct ? m->t1 : m->t2 + (int64_t)D.max_batch * m->n_t2q;
+            float *cq = m->t2, *q = direct ? m->t1 : m->t2 + m->rows * m->n_t2q;
             const int64_t ldq = direct ? P.ncat : nq;
             const float *gate = l.gated ? m->t1 + P.ncat - H : nullptr;
             psk_dense(st, mm(l.in_cat, in, W, m->t1, P.ncat));
@@ -890,7 +917,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             if (P.side) mixer(*P.side, m->h, xr, res * P.side->d.mix_scale);
             if (l.ff_kind != PS_FF_NONE) feed_forward(P, h2 ? h2 : m->h, xr, res);
             if (m->dbg_layers && !any_pos && m->hist)
-                psk_front(st, m->hist, BW, li + 2, l.depth_mix, nullptr, m->dbg_layers + (int64_t)li * BW, nullptr, nullptr, nullptr, nullptr, 1, 0.f, D.norm_eps, W, T);
+                psk_front(st, m->hist, BW, li + 2, l.depth_mix, nullptr, m->dbg_layers + (int64_t)li * DW, nullptr, nullptr, nullptr, nullptr, 1, 0.f, D.norm_eps, W, T);
         } else if (l.form == PS_LAYER_PARALLEL) {
             // hn = norm(x), h = conv(hn); both mixers and the feed-forward add their output projections straight into the residual stream
             boundary(nullptr, nullptr, l.norm1, l.canon1, P.off_canon1);
@@ -918,7 +945,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 boundary(m->y, l.norm1b, nn, nc, no);
             }
         }
-        if (m->dbg_layers && !any_pos && !m->hist) psk_copy(st, m->x, m->dbg_layers + (int64_t)li * BW, (int64_t)T * W);
+        if (m->dbg_layers && !any_pos && !m->hist) psk_copy(st, m->x, m->dbg_layers + (int64_t)li * DW, (int64_t)T * W);
     }
 }
 
@@ -928,7 +955,7 @@ static void seq_head(ps_hip_seq *m, const int32_t *idx, int rows) {
     const ps_seq_desc &D = m->d;
     if (m->hist) { // what the last layer hands on (its depth average, or its own result) and the final norm in one launch
         const int runs = (int)m->L.size();
-        psk_front(st, m->hist, (int64_t)D.max_batch * D.width, runs + 1, m->L[runs - 1].d.depth_mix, idx, nullptr, D.final_norm, m->xn, nullptr, nullptr, m->groups,
+        psk_front(st, m->hist, m->rows * D.width, runs + 1, m->L[runs - 1].d.depth_mix, idx, nullptr, D.final_norm, m->xn, nullptr, nullptr, m->groups,
                   D.norm_offset, D.norm_eps, D.width, rows, 0, D.final_norm_bias);
     } else if (D.norm_center || D.final_norm_bias) {
         psk_front(st, m->x, 0, 1, nullptr, idx, nullptr, D.final_norm, m->xn, nullptr, nullptr, m->groups, D.norm_offset, D.norm_eps, D.width, rows, D.norm_center, D.final_norm_bias);
@@ -978,12 +1005,38 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
     };
     int wi = 0, half = 0;
     std::vector<int32_t> idx;
+    // the logits of the wanted rows idx (at most max_batch of them, the caller's w0 and on): they are in m->want
+    auto results = [&](const int w0) -> int {
+        const int rows = (int)idx.size();
+        seq_head(m, m->want, rows);
+        if (row && rows * row <= PS_PIN_HALF && ps_pin_ready(c)) {
+            PS_CHECK(c, take(half)); // (those before the last ones: long there)
+            const size_t lb = logits_host ? (size_t)rows * m->d.vocab * 4 : 0;
+            if (logits_host) ps_pin_copy(c, half, 0, m->logits, lb);
+            if (argmax_host) ps_pin_copy(c, half, lb, m->amax, (size_t)rows * 4);
+            PS_CHECK(c, hipEventRecord(c->pin_ev[half], c->stream));
+            held[half] = Held{w0, rows};
+            half ^= 1;
+            PS_CHECK(c, take(half));
+        } else {
+            if (logits_host) PS_CHECK(c, hipMemcpyAsync(logits_host + (size_t)w0 * m->d.vocab, m->logits, (size_t)rows * m->d.vocab * 4, hipMemcpyDeviceToHost, c->stream));
+            if (argmax_host) PS_CHECK(c, hipMemcpyAsync(argmax_host + w0, m->amax, (size_t)rows * 4, hipMemcpyDeviceToHost, c->stream));
+        }
+        PS_CHECK(c, hipGetLastError());
+        return 0;
+    };
+    const int step = m->dbg_layers ? B : (int)m->rows; // (the debugging buffer holds max_batch rows of a run)
     auto portions = [&]() -> int {
-        for (int t0 = 0; t0 < n; t0 += B) {
-            const int T = std::min(B, n - t0), w0 = wi;
+        for (int t0 = 0; t0 < n; t0 += step) {
+            const int T = std::min(step, n - t0);
             const int64_t pos0 = m->slot_pos[slot];
-            idx.clear();
-            while (wi < n_want && want[wi] < t0 + T) idx.push_back(want[wi++] - t0);
+            auto wanted = [&]() { // the next of the portion's wanted rows, as many as the head takes at a time; where they begin
+                const int w0 = wi;
+                idx.clear();
+                while (wi < n_want && want[wi] < t0 + T && (int)idx.size() < B) idx.push_back(want[wi++] - t0);
+                return w0;
+            };
+            int w0 = wanted();
             const ps_piece in[2] = {{m->tokens, tokens + t0, (size_t)T * 4}, {m->want, idx.data(), idx.size() * 4}};
             PS_CHECK(c, ps_put(c->stream, in, 2));
             hipLaunchKernelGGL(seq_set_step_kernel, dim3(1), dim3(1), 0, c->stream, m->step, (long long)pos0, T, slot, m->slot_state[slot], (int)tokens[t0], (int)tokens[t0 + T - 1],
@@ -991,23 +1044,13 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
             seq_layers(m, m->slot_state[slot], T, pos0, false, false);
             PS_CHECK(c, hipGetLastError());
             m->slot_pos[slot] = pos0 + T; // (the slot's recurrent states move with these launches, whatever becomes of the results)
-            if (idx.empty()) continue;
-            const int rows = (int)idx.size();
-            seq_head(m, m->want, rows);
-            if (row && rows * row <= PS_PIN_HALF && ps_pin_ready(c)) {
-                PS_CHECK(c, take(half)); // (the portion before the last one's: long there)
-                const size_t lb = logits_host ? (size_t)rows * m->d.vocab * 4 : 0;
-                if (logits_host) ps_pin_copy(c, half, 0, m->logits, lb);
-                if (argmax_host) ps_pin_copy(c, half, lb, m->amax, (size_t)rows * 4);
-                PS_CHECK(c, hipEventRecord(c->pin_ev[half], c->stream));
-                held[half] = Held{w0, rows};
-                half ^= 1;
-                PS_CHECK(c, take(half));
-            } else {
-                if (logits_host) PS_CHECK(c, hipMemcpyAsync(logits_host + (size_t)w0 * m->d.vocab, m->logits, (size_t)rows * m->d.vocab * 4, hipMemcpyDeviceToHost, c->stream));
-                if (argmax_host) PS_CHECK(c, hipMemcpyAsync(argmax_host + w0, m->amax, (size_t)rows * 4, hipMemcpyDeviceToHost, c->stream));
+            while (!idx.empty()) {
+                if (const int rc = results(w0)) return rc;
+                w0 = wanted();
+                if (idx.empty()) break;
+                const ps_piece more = {m->want, idx.data(), idx.size() * 4};
+                PS_CHECK(c, ps_put(c->stream, &more, 1));
             }
-            PS_CHECK(c, hipGetLastError());
         }
         PS_CHECK(c, hipStreamSynchronize(c->stream));
         PS_CHECK(c, hipGetLastError());

@@ -109,7 +109,10 @@ hipError_t hipGetLastError() { hipError_t e = last; last = hipSuccess; return ca
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) { *n = 1; return hipSuccess; }
 
-hipError_t hipMalloc(void **p, size_t bytes) { return alloc(p, bytes, hipMemoryTypeDevice); }
+hipError_t hipMalloc(void **p, size_t bytes) {
+    const hipError_t e = call("hipMalloc");
+    return e != hipSuccess ? e : alloc(p, bytes, hipMemoryTypeDevice);
+}
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return call("hipHostMalloc") ? hipErrorUnknown : alloc(p, bytes, hipMemoryTypeHost); }
 hipError_t hipFree(void *p) { mem.erase((char *)p); free(p); return hipSuccess; }
 hipError_t hipHostFree(void *p) { return hipFree(p); }

@@ -418,6 +418,26 @@ def test_results_of_a_call_of_several_portions(made):
     m.release(s)
 
 
+# inputs longer than max_batch, whose launch sequences take up to four times as many tokens (seq_rows): every row wanted, more than the head takes at a time; a last one of a single token; a width of four
+# times max_batch that the context cuts; rows of a second group that repeat
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("max_batch,n,max_context", [(64, 300, 1024), (64, 257, 1024), (150, 420, 500), (63, 200, 1024)])
+def test_a_long_input_in_launch_sequences_wider_than_max_batch(ctx, tmp_path, dtype, max_batch, n, max_context):
+    cfg = CONFIGS["mixed"]
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype, max_batch=max_batch, n_slots=1, max_context=max_context)
+    toks = tokens_for(cfg, n, seed=6)
+    # (bfloat16: against calls of max_batch tokens.  Rounding alone moves row 151 by 0.1175, in portions of any size and token by token; another cut may round it the other way: a tenth of that)
+    rows, tol = (seq_oracle.run(cfg, t, toks), TOL[dtype]) if dtype == "float32" else (run_portions(m, toks, (max_batch,)), 0.012)
+    for want in (np.arange(n), np.array([0] * max_batch + [max_batch] * max_batch + [n - 1] * 3)):
+        s = m.acquire()
+        assert err(m.forward(s, toks, want), rows[want]) < tol
+        assert m.position(s) == n
+        m.release(s)
+    assert err(run_portions(m, toks, (n - 1, 1)), rows) < tol
+    m.close()
+
+
 def test_interleaved_requests_and_reused_slots(made):
     m, cfg, t = made("mixed", "float32", max_batch=16)
     seqs = [tokens_for(cfg, n, seed=20 + n) for n in (37, 9, 58)]

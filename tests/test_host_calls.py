@@ -67,6 +67,28 @@ assert m.position(s) == 20 and fake.fake_stray() == 0
 """)
 
 
+def test_a_model_without_room_for_wide_launch_sequences(child):
+    """ps_hip_seq_create: launch sequences of four times max_batch where the memory is there, of max_batch where it is not; more wanted rows than the head takes at a time go in groups"""
+    child("""
+ctx = hip.Ctx(0)
+toks, want = [1] * 300, list(range(300))
+fake.fake_reset()
+m = seq(ctx, 64)
+allocations = count("hipMalloc")
+s = m.acquire()
+fake.fake_reset()
+m.forward(s, toks, want=want)
+assert count("seq_set_step_kernel") == 2 and count("dense_argmax_kernel") == 5 and m.position(s) == 300 and fake.fake_stray() == 0
+for n in (0, 1, 7): # (the last ones are the model's own)
+    fail("hipMalloc", allocations - n)
+    m = seq(ctx, 64)
+    s = m.acquire()
+    fake.fake_reset()
+    m.forward(s, toks, want=want)
+    assert count("seq_set_step_kernel") == 5 and count("dense_argmax_kernel") == 5 and m.position(s) == 300 and fake.fake_stray() == 0
+""")
+
+
 def test_copies_to_the_host_keep_their_error_cases(child):
     """ps_hip_memcpy_d2h: what a kernel could not read without a fault is left to the runtime's copy, whatever that says"""
     child("""
