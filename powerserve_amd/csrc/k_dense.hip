@@ -3,6 +3,7 @@
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
 //   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
+//   dense_mm_big_kernel   the same operands, bf16, 256 x 256 tiles where they fill the chip in fewer rounds
 //   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
 //   dense_mm_narrow_kernel bf16, K a multiple of 128 up to 1024, more than 8 tokens, few tiles: 32 x 32 tiles, the waves share K
 //   dense_mv1_kernel<WT,FORM,RAGGED> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
@@ -794,20 +795,206 @@ __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p)
     if (t < T) dn_put4<ODD>(g, dn_orow(g, row0, t, T), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + c, *(const dn_f4 *)&turn[r * 36 + c]);
 }
 
+// 256 x 256 tiles, for products that fill the chip with them (bf16).  Eight waves, a wave 64 x 32 of each quarter of the tile; K in blocks of 64, two LDS stages in four pieces of 128 rows (half
+// of the tokens' rows or of the weights').  A block is four phases, one per quarter, a phase two slots: in one a wave reads fragments and requests a piece, in the other it multiplies (sixteen
+// instructions), and the waves 4 - 7 are one slot behind the waves 0 - 3 of the same SIMDs, so that the matrix cores have one wave of a SIMD in every slot while the other's requests and reads hold
+// only that one.  A piece is requested over the one that all waves have just read (both groups' reads are back at the barrier in front), six phases before it is read itself; a wait per
+// phase is for all but the six youngest pieces.
+// What bounded the 128 x 128 tiles here were the bytes from L2 (64 a clock and CU for the matrix instructions' rate, half of that comes) and the reads in front of them; these take half of both per
+// product.  Without requests and reads a block takes 1.03 us, the matrix instructions at the 2 GHz they hold; 1.15 as it is.  2047 tokens, bf16, in the 128 x 128 form and here: 8192 x 2048
+// 122 -> 59 us (16 of them the 67 MB of results, behind the last product of a CU's only tile), 6208 x 2048 96 -> 57; 1000 tokens 14336 x 4096 177 -> 117.
+#define DN_BIG 256
+#define DN_BIG_LDS ((DN_BIG / 2) * (DN_BIG + 4) * 4)
+static __device__ __forceinline__ void dn_dma_at(const char *base, unsigned off, unsigned lds_dst) { // (as dn_dma, from a uniform base)
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst) : "memory");
+}
+template <bool ODD>
+__global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p) {
+    extern __shared__ __attribute__((aligned(16))) char dn_lds[];
+    constexpr int BM = DN_BIG, BN = DN_BIG, HALF = 128 * 128;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3;
+    const int per = 8 * p.n_tm, b_in = (int)blockIdx.x % per, tn = ((int)blockIdx.x / per) * 8 + (b_in & 7), tm = b_in >> 3;
+    if (tn >= p.tn) return;
+    int e, T, t0;
+    long long row0;
+    if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return; // (uniform per work-group)
+    const long long n0 = (long long)tn * BN, ldw = g.K * 2;
+    const int nk = (int)(ldw >> 7);
+    // this wave's two requests of a piece: rows 16 wave + 8 j + lane / 8, sixteen bytes each
+    const char *W = (const char *)g.w + (g.g_seg ? e * g.wstride * 2 : 0), *A = p.A;
+    long long nw = n0, n_rows = g.N;
+    if (p.each) { // (uniform)
+        const int i = (int)(n0 / p.each);
+        W = (const char *)(i == 0 ? p.w[0] : i == 1 ? p.w[1] : i == 2 ? p.w[2] : p.w[3]);
+        A += i * p.copy;
+        nw = n0 - i * p.each;
+        n_rows = p.each;
+    }
+    A += (g.g_seg ? row0 + t0 : t0) * p.lda;
+    W += nw * ldw;
+    unsigned oa[2][2], ob[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int r = 16 * wave + 8 * j + (lane >> 3), kq = (lane & 7) ^ ((r >> 1) & 7);
+            oa[h][j] = (unsigned)min(h * 128 + r, T - 1 - t0) * (unsigned)p.lda + kq * 16;
+            ob[h][j] = (unsigned)min((long long)(h * 128 + r), n_rows - 1 - nw) * (unsigned)ldw + kq * 16;
+        }
+    const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)dn_lds + (unsigned)(wave * 2048);
+    auto request_a = [&](const int kb, const int h) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) dn_dma_at(A + (long long)kb * 128, oa[h][j], lds0 + (unsigned)((2 * (kb & 1) + h) * HALF + j * 1024));
+    };
+    auto request_w = [&](const int kb, const int h) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) dn_dma_at(W + (long long)kb * 128, ob[h][j], lds0 + (unsigned)((4 + 2 * (kb & 1) + h) * HALF + j * 1024));
+    };
+    dn_f4 acc[2][2][4][2], xa[2][4], xb[2][2][2]; // (tokens' half, weights' half)
+#pragma unroll
+    for (int mh = 0; mh < 2; mh++)
+#pragma unroll
+        for (int nh = 0; nh < 2; nh++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[mh][nh][i][j] = dn_f4{0.f, 0.f, 0.f, 0.f};
+    const int fr = lane & 15, po = (((lane >> 4) ^ (fr >> 1)) << 4); // (row bases are multiples of sixteen; the second half of a block: the piece's number with its third bit turned)
+    const char *fa[2] = {dn_lds + (wm * 64 + fr) * 128 + po, dn_lds + (wm * 64 + fr) * 128 + (po ^ 64)};
+    const char *fb[2] = {dn_lds + 4 * HALF + (wn * 32 + fr) * 128 + po, dn_lds + 4 * HALF + (wn * 32 + fr) * 128 + (po ^ 64)};
+    auto read_a = [&](const int kb, const int h) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) xa[u][i] = *(const dn_f4 *)(fa[u] + (2 * (kb & 1) + h) * HALF + i * 2048);
+    };
+    auto read_w = [&](const int kb, const int h) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) xb[h][u][j] = *(const dn_f4 *)(fb[u] + (2 * (kb & 1) + h) * HALF + j * 2048);
+    };
+    auto multiply = [&](const int mh, const int nh) { // between two barriers: the other group's slot of reads and requests
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    dn_bf8 za, zb;
+                    __builtin_memcpy(&za, &xa[u][i], 16);
+                    __builtin_memcpy(&zb, &xb[nh][u][j], 16);
+                    acc[mh][nh][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(zb, za, acc[mh][nh][i][j], 0, 0, 0);
+                }
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    for (int kb = 0; kb < min(nk, 2); kb++) { request_w(kb, 0); request_a(kb, 0); request_w(kb, 1); request_a(kb, 1); }
+    if (nk > 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read_w(0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (wm) __builtin_amdgcn_s_barrier();
+    for (int kb = 0; kb < nk; kb++) {
+        const bool more = kb + 2 < nk;
+#define DN_BIG_LANDED                                                     \
+    if (more) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");           \
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        read_a(kb, 0);
+        if (more) request_w(kb + 2, 0);
+        DN_BIG_LANDED
+        multiply(0, 0);
+        read_w(kb, 1);
+        if (more) request_a(kb + 2, 0);
+        DN_BIG_LANDED
+        multiply(0, 1);
+        read_a(kb, 1);
+        if (more) request_w(kb + 2, 1);
+        DN_BIG_LANDED
+        multiply(1, 0);
+        if (kb + 1 < nk) read_w(kb + 1, 0);
+        if (more) request_a(kb + 2, 1);
+        DN_BIG_LANDED
+        multiply(1, 1);
+#undef DN_BIG_LANDED
+    }
+    if (!wm) __builtin_amdgcn_s_barrier();
+    if (g.act == PSD_ACT_NONE && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
+#pragma unroll
+        for (int mh = 0; mh < 2; mh++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int t = t0 + mh * 128 + wm * 64 + i * 16 + fr;
+                if (t >= T) continue;
+                const long long at = dn_orow(g, row0, t, T) * g.ldo + n0;
+#pragma unroll
+                for (int nh = 0; nh < 2; nh++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const int c = nh * 128 + wn * 32 + j * 16 + 4 * (lane >> 4);
+                        if (n0 + c >= g.N) continue;
+                        dn_f4 v;
+#pragma unroll
+                        for (int x = 0; x < 4; x++) v[x] = acc[mh][nh][i][j][x] * g.alpha;
+                        if (g.out16) {
+                            dn_us4 r;
+#pragma unroll
+                            for (int x = 0; x < 4; x++) r[x] = dn_f2bf(v[x]);
+                            *(dn_us4 *)(g.out16 + at + c) = r;
+                        } else {
+                            *(dn_f4 *)(g.out + at + c) = v;
+                        }
+                    }
+            }
+        return;
+    }
+    // half of the tile at a time through LDS (the stages are done with)
+    constexpr int LD = BN + 4;
+    float *tile = (float *)dn_lds;
+#pragma unroll
+    for (int mh = 0; mh < 2; mh++) {
+        __syncthreads();
+#pragma unroll
+        for (int nh = 0; nh < 2; nh++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) *(dn_f4 *)&tile[(wm * 64 + i * 16 + fr) * LD + nh * 128 + wn * 32 + j * 16 + 4 * (lane >> 4)] = acc[mh][nh][i][j];
+        __syncthreads();
+        for (int r = wave; r < 128; r += 8) {
+            const int t = t0 + mh * 128 + r;
+            if (t >= T) break;
+            dn_put4<ODD>(g, dn_orow(g, row0, t, T), n0 + 4 * lane, *(const dn_f4 *)&tile[r * LD + 4 * lane]);
+        }
+    }
+}
 // Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
 // of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more; rounds of 256 work-groups (one per CU);
-// a split product pays a second launch and its parts' way through memory.
+// a split product pays a second launch and its parts' way through memory.  The 256 x 256 tiles' block is what they measured beside the 128 x 128 ones: 1.7 times their time where both fill the chip
+// once (512 tokens x 8192 x 2048: 28 us there, 48 here), half of it where the smaller ones need four rounds; they are not split (2047 x 2048 x 8192 in two: 98 us, 84 as 128 x 128 tiles).
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
-static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int groups, bool bf, bool may_split) {
-    static const int shapes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
+static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int groups, bool bf, bool may_split, bool big) {
+    static const int shapes[4][2] = {{128, 128}, {64, 128}, {64, 64}, {DN_BIG, DN_BIG}};
     const int64_t blocks = kbytes / 128;
     dn_ring_shape best{};
     double least = 0;
     for (auto &q : shapes) {
+        if (q[0] == DN_BIG && !(bf && big)) continue;
         const int BM = q[0], BN = q[1], full = (rows + BM - 1) / BM, n_tm = rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0), tn = (int)((N + BN - 1) / BN);
         const int64_t tiles = (int64_t)(groups > 0 ? std::max(full, std::min(groups, rows)) + (rows > groups * BM ? groups / 2 : 0) : n_tm) * tn; // (grouped: about half of the last tiles start a new one)
-        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = std::max(lds, mfma) + 100;
-        for (int64_t S = 1; S <= (may_split ? 16 : 1); S++) {
+        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = BM == DN_BIG ? 1700 : std::max(lds, mfma) + 100;
+        for (int64_t S = 1; S <= (may_split && BM != DN_BIG ? 16 : 1); S++) {
             if (S > 1 && (blocks / S < 4 || tiles * S > 512 || (size_t)n_tm * tn * S * BM * BN * 4 > psk_dense_split_bytes())) break;
             const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
             if (!best.BM || t < least) { least = t; best = dn_ring_shape{BM, BN, n_tm, tn, (int)S}; }
@@ -829,6 +1016,15 @@ static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN, ODD>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
 }
 
+template <bool ODD>
+static void dn_launch_big(hipStream_t st, const dn_args &g, const dn_ring &p) {
+    if constexpr (!ODD)
+        if (dn_odd(g)) return dn_launch_big<true>(st, g, p);
+    static unsigned long long mask = 0;
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_big_kernel<ODD>, hipFuncAttributeMaxDynamicSharedMemorySize, DN_BIG_LDS);
+    hipLaunchKernelGGL(dense_mm_big_kernel<ODD>, dim3((unsigned)((p.tn + 7) / 8 * 8) * p.n_tm), dim3(512), DN_BIG_LDS, st, g, p);
+}
+
 // the wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed
 template <typename WT>
 static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
@@ -842,7 +1038,7 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     if (!plain && (size_t)a.T * kbytes * copies > a.pack_bytes) return false;
     const int64_t each = g.N;
     g.N *= copies;
-    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes());
+    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes(), (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 23)); // (rows of a tile by 32-bit offsets)
     dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes, r.n_tm, r.tn, r.S, a.split};
     p.each = copies > 1 ? each : 0;
     p.copy = a.T * kbytes;
@@ -851,7 +1047,8 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
         const int64_t pb = ((int64_t)a.T * (g.K / 8) + 255) / 256;
         hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192), (unsigned)copies), dim3(256), 0, st, g, (WT *)a.pack);
     }
-    if (r.BM == 128) dn_launch_ring<WT, 128, 128, false>(st, g, p);
+    if (r.BM == DN_BIG) dn_launch_big<false>(st, g, p);
+    else if (r.BM == 128) dn_launch_ring<WT, 128, 128, false>(st, g, p);
     else if (r.BN == 128) dn_launch_ring<WT, 64, 128, false>(st, g, p);
     else dn_launch_ring<WT, 64, 64, false>(st, g, p);
     return true;

@@ -161,7 +161,9 @@ def test_latent_attention_of_a_very_long_window(ctx, tmp_path, window):
 # products split along K (few tiles, long K: also uneven shares), more tiles than the chip has CUs
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(9, 1, 64), (63, 127, 128), (64, 128, 192), (65, 129, 256), (127, 63, 320), (128, 65, 576), (129, 200, 64), (300, 130, 1088), (16, 8, 4096), (40, 100, 4160),
-                                   (200, 256, 2240), (520, 2100, 128)])
+                                   (200, 256, 2240), (520, 2100, 128),
+                                   # dense_mm_big_kernel (bf16): one block of K, two, three and more than its stages; a row, a column and four columns more than a tile; no fours
+                                   (2047, 2100, 64), (2049, 2305, 64), (1999, 3001, 192), (1030, 4100, 320), (1793, 2304, 128), (300, 20004, 64)])
 def test_dense_matmul_wide(ctx, dtype, T, N, K):
     import ctypes as C
     rng = np.random.default_rng(T * 1000 + N)
@@ -226,6 +228,30 @@ def test_bf16_rows_handed_on(made, sizes):
     m.set_mode(0)
     # both round the same numbers; their fp32 sums differ in order, so a rounding behind them may go the other way: an error of the same origin and size.  A row that is not its own: ~1
     assert err(got, want) < 1.5 * err(plain, want) < 0.3
+
+
+# 256 x 256 tiles behind an epilogue (k_dense.hip dense_mm_big_kernel): an activation whose rounded rows the second product reads, pairs, the four mixes of a token shift, the slots of experts (tiles
+# that end inside an expert, an expert without slots) with a factor per row
+@pytest.mark.parametrize("which", ["xielu", "pairs", "experts", "mixes"])
+def test_large_tiles_behind_an_epilogue(ctx, tmp_path, which):
+    V = 30
+    if which == "experts":
+        cfg = synth.pupidra_config(64, V, [synth.pupidra_layer("attention", synth.pupidra_attention(2, 1, 16, 16, 0.3, 9, 2), moe=(5, 2, 6144, 1.7), shared=8)])
+    elif which == "mixes":
+        cfg = synth.seq_config(64, V, [L("wkv", None, heads=16, dim=128)], taps=2)
+    elif which == "pairs":
+        cfg = synth.pokatar_config(64, V, [synth.pokatar_layer("attention", synth.pokatar_attention(2, 1, 16, 16, 0.3), 4096)])
+    else:
+        cfg = synth.seq_config(64, V, [L("delta", 8192, heads=2, kv_heads=1, dim=16, vdim=16, conv=2)], taps=2)
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="bfloat16", max_batch=640, n_slots=1, max_context=700)
+    toks = tokens_for(cfg, 600)
+    got = run_portions(m, toks, (600,))
+    m.set_mode(2)  # the tiled mat-mul
+    plain = run_portions(m, toks, (600,))
+    m.close()
+    # both round the same numbers; their fp32 sums differ in order, so a rounding behind them may go the other way (2^-9 of a number, a few numbers of a row).  A row that is not its own: ~1
+    assert err(got, plain) < 0.03
 
 
 # results without an epilogue (k_dense.hip dense_mm_ring_kernel): columns in fours, stored from the registers, the last four of a tile, one four and three fours into the next one; no fours
