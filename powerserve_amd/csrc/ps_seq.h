@@ -235,6 +235,32 @@ void psk_latent_absorbed(hipStream_t st, const ps_seq_step *step, int64_t ring_o
                          int H, int d, int dr, int rot_dims, int dv, int R, int window, float scale, float *scratch, float *o, float rot_mag = 1.f,
                          const float *gate = nullptr, int pairing = PS_ROT_HALVES);
 
+// ---- k_splitattn.hip: the attention of a portion of many rows (position pos0 and on, H heads over G key / value groups) whose window is known on the host
+struct psk_split_attn_args {
+    int H = 0, G = 0, own = 0, n_shared = 0; // numbers of a key: a group's own, then those all groups share; values have 128
+    int64_t pos0 = 0, first = 0;             // first = max(0, pos0 - window + 1): the position of window row 0
+    int T = 0, window = 0, pool = 0, keep = 0, n_front = 0, n_window = 0; // front rows that some row sees; n_window = pos0 + T - first
+    // window row j: row (j + off), wrapped once at mod (0: not), of k / v (stride ldk; group g: own, 128 numbers on); the shared part alike; front rows
+    const float *k = nullptr, *v = nullptr, *shared = nullptr, *front_k = nullptr, *front_v = nullptr;
+    int64_t ldk = 0, ld_shared = 0;
+    int mod = 0, off = 0, shared_mod = 0, shared_off = 0;
+    const float *q = nullptr; // head h of row t: q + t ldq + h (own + n_shared); its part behind `own` is rotated here where rot_dims > 0
+    int64_t ldq = 0;
+    const float *freq = nullptr;
+    int rot_dims = 0, pairing = 0;
+    float rot_mag = 1.f, scale = 1.f, softcap = 0.f;
+    const float *temp = nullptr, *slope = nullptr, *sink = nullptr, *gate = nullptr;
+    int64_t ldg = 0;
+    int gate_elem = 0;
+    float *o = nullptr; // [T][ldo], head h at 128 h
+    int64_t ldo = 0;
+    void *scratch = nullptr; // psk_split_attn_scratch bytes
+};
+bool psk_split_attn_ok(int own, int shared, int dv);
+bool psk_split_attn_takes(int T, int H); // enough rows to fill the chip
+size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window);
+void psk_split_attn(hipStream_t st, const psk_split_attn_args &a);
+
 // ---- k_winattn.hip
 // What a token sees in front of its window comes from a second store with the ring's row layout at step->state + off: one row per POOLED BLOCK (pool > 0), or the rows of the
 // sequence's FIRST tokens (keep > 0: row = position; visible are those not in the window themselves), never both.  slope [H] (NULL: none): slope[h] * (query position - key

@@ -74,6 +74,7 @@ struct ps_hip_seq {
     float *lstm_aux = nullptr;    // matrix memory: [rows][heads] products with n, then as many running maxima
     int64_t lstm_aux_n = 0;
     uint16_t *a16 = nullptr; // bf16 models: a portion's rows as the kernel in front of a product has rounded them
+    void *sa_scratch = nullptr; // the split keys and values of a portion's attention
     float *abs_scratch = nullptr; // the absorbed single-token attention's folded queries, attended latents and per-tile partials
     void *pack = nullptr; // the wide mat-mul's operand copy
     size_t pack_bytes = 0;
@@ -517,6 +518,15 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
     m->slot_state.assign(desc->n_slots, nullptr);
     m->slot_pos.assign(desc->n_slots, -1);
     for (int s = 0; ok && s < desc->n_slots; s++) ok = alloc((void **)&m->slot_state[s], (size_t)m->state_floats * 4);
+    if (ok) { // (where there is no room for it, the attention goes without)
+        size_t sa = 0;
+        mixers([&](LayerPlan &P) {
+            const bool lat = P.d.kind == PS_MIX_LATENT, win = P.d.kind == PS_MIX_WINATTN;
+            if ((lat || win) && psk_split_attn_ok(P.d.dim, lat ? P.d.rot_dim : 0, P.d.vdim) && psk_split_attn_takes((int)B, P.d.heads))
+                sa = std::max(sa, psk_split_attn_scratch(lat ? P.d.heads : P.d.kv_heads, P.d.dim, lat ? P.d.rot_dim : 0, P.d.vdim, win ? P.pool_rows : 0, P.d.window - 1 + B));
+        });
+        if (sa && !alloc(&m->sa_scratch, sa)) (void)hipGetLastError();
+    }
     if (!ok) {
         fail("out of device memory");
         return SEQ_NO_MEMORY;
@@ -612,6 +622,14 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             rounded = psk_causal_conv(st, m->step, tail_off, m->hn, W, cw, D.canon_taps, 0, W, T, m->h, W, nullptr, copy16) ? m->h : nullptr;
         }
     };
+    // a portion's attention with its keys and values split beforehand (l: own numbers of a key, then `shared` ones that all heads have): whether it is taken, and what all mixers tell it
+    auto split_attn = [&](const ps_seq_layer &l, const int64_t shared) {
+        return m->sa_scratch && !any_pos && !tiled && pos0 + T < (1 << 30) && psk_split_attn_ok(l.dim, (int)shared, l.vdim) && psk_split_attn_takes(T, l.heads);
+    };
+    auto split_attn_run = [&](const ps_seq_layer &l, psk_split_attn_args &g) {
+        g.H = l.heads; g.own = l.dim; g.pos0 = pos0; g.T = T; g.window = l.window; g.scale = l.scale; g.o = m->t3; g.ldo = (int64_t)l.heads * l.vdim; g.scratch = m->sa_scratch;
+        psk_split_attn(st, g);
+    };
     // One mixer on the input `in`.  Its output projection writes out_scale times its result to `store` (NULL: m->y), or (into given) adds it there.
     auto mixer = [&](const LayerPlan &P, const float *in, float *into, float out_scale, float *store = nullptr) {
         const ps_seq_layer &l = P.d;
@@ -685,7 +703,17 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             const float *gate = l.gated ? t1 + Hd + (reads ? 0 : G * d + G * dv) : nullptr;
             const int ge = l.gated == 2; // a gate per output element
             const bool mfma = (m->mode & 2) == 0 && (G * (d + dv)) % 4 == 0 && psk_winattn_mfma_ok((int)d, (int)dv);
-            if (mfma && T == 1 && m->win_scratch)
+            if (mfma && split_attn(l, 0)) {
+                const int64_t past = std::min<int64_t>(pos0, l.window - 1), out = pos0 + T - l.window; // (positions in front of the last token's window)
+                psk_split_attn_args g;
+                g.G = (int)G; g.first = pos0 - past;
+                g.pool = fs.pool; g.keep = fs.keep; g.n_front = (int)(out <= 0 ? 0 : fs.pool > 0 ? out / fs.pool : std::min<int64_t>(out, fs.keep)); g.n_window = (int)(past + T);
+                g.k = state + P.off_ring; g.v = g.k + G * d; g.front_k = state + P.off_pool; g.front_v = g.front_k + G * d; g.ldk = G * (d + dv);
+                g.mod = P.cap; g.off = (int)(g.first % P.cap);
+                g.q = m->t2; g.ldq = Hd;
+                g.softcap = l.softcap; g.temp = l.temp; g.slope = l.dist_slope; g.sink = l.sink; g.gate = gate; g.ldg = ld1; g.gate_elem = ge;
+                split_attn_run(l, g);
+            } else if (mfma && T == 1 && m->win_scratch)
                 psk_winattn_step(st, m->step, P.off_ring, P.cap, fs, m->t2, gate, l.temp, l.sink, (int)H, (int)G, (int)d, (int)dv, l.window, l.scale,
                                  m->max_context, m->win_scratch, m->t3, l.softcap, ge, l.dist_slope);
             else if (mfma)
@@ -753,7 +781,16 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 g.a_step = m->step; g.a_row0 = -(int64_t)(l.window - 1); g.a_mod = P.cap;
                 g.T = any_pos ? l.window - 1 + T : (int)(std::min<int64_t>(pos0, l.window - 1) + T);
                 psk_dense(st, g);
-                if (!plain && rows4 && psk_latent_attn_mfma_ok((int)d, (int)dr, (int)dv))
+                if (!plain && rows4 && split_attn(l, dr)) {
+                    const int64_t past = std::min<int64_t>(pos0, l.window - 1);
+                    psk_split_attn_args g;
+                    g.G = (int)H; g.n_shared = (int)dr; g.first = pos0 - past; g.n_window = (int)(past + T);
+                    g.k = m->kvx; g.v = g.k + H * d; g.ldk = H * d + Hv;
+                    g.shared = state + P.off_ring + l.kv_rank; g.ld_shared = rs; g.shared_mod = P.cap; g.shared_off = (int)(g.first % P.cap);
+                    g.q = q; g.ldq = ldq; g.freq = P.freq; g.rot_dims = l.rot_dims; g.pairing = l.rot_pairing; g.rot_mag = P.rot_mag;
+                    g.gate = gate; g.ldg = P.ncat;
+                    split_attn_run(l, g);
+                } else if (!plain && rows4 && psk_latent_attn_mfma_ok((int)d, (int)dr, (int)dv))
                     psk_latent_attn_mfma(st, m->step, P.off_ring, P.cap, q, ldq, m->kvx, H * d + Hv, P.freq, (int)H, (int)d, (int)dr, l.rot_dims, (int)dv, l.kv_rank, l.window,
                                          l.scale, T, m->t3, Hv, P.rot_mag, gate, P.ncat, l.rot_pairing);
                 else

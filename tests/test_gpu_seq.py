@@ -254,6 +254,35 @@ def test_large_tiles_behind_an_epilogue(ctx, tmp_path, which):
     assert err(got, plain) < 0.03
 
 
+# attention of many rows with its operands split into three bf16 numbers (k_splitattn.hip: two blocks of 128 rows of 64 heads and more): keys of 192 and 128 numbers, windows that end inside blocks of
+# 32 keys and inside a portion, with and without kept first tokens (fewer and more than a block), means of blocks, distance slopes, a reader of another layer's keys, gates, temperatures and sinks,
+# a soft cap, rotated queries of both pairings, key / value groups; a ring that has wrapped; portions of fewer rows (the fp32 instruction) in between; one row of the last block of 128
+@pytest.mark.parametrize("which", ["latent", "latent direct", "keep", "pool", "softcap"])
+def test_attention_of_many_rows(ctx, tmp_path, which):
+    V, sizes = 40, (200, 1, 129, 140)
+    if which == "latent":
+        run, cfg = seq_oracle.run, synth.seq_config(64, V, [L("latent_attention", None, heads=64, dim=128, vdim=128, q_rank=40, kv_rank=64, mask={"size": 77}, scale=0.09,
+                                                              rot={"base": 500.0, "dims": 48}, rot_dim=64)], taps=2)
+    elif which == "latent direct":
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("latent_attention", synth.pupidra_latent(64, 96, 32, 128, 32, 0.1, 1e4))])
+    elif which == "keep":
+        at = lambda size, keep, own=None: synth.pupidra_attention(64, 2, 128, 128, 1.0, size, keep, own)
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("attention", at(150, 40)), synth.pupidra_layer("attention", at(31, 5, 0))])
+    elif which == "pool":
+        at = {"heads": 64, "kv_heads": 4, "dim": 128, "vdim": 128, "mask": {"size": 33, "pool": 3}, "rot": {"base": 100.0, "dims": 64}, "scale": 0.1}
+        run, cfg = seq_oracle.run_parallel, synth.parallel_config(64, V, [synth.parallel_layer(None, at, {"heads": 1, "dim": 16, "vdim": 16, "tau": 4.0}, 1.0, 0.5)], taps=2)
+    else:
+        run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(64, 8, 128, 128, 0.1, 5.0, (0.4, 7)), ff=64)])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=200, n_slots=1, max_context=500)
+    toks = tokens_for(cfg, sum(sizes))
+    want, got = run(cfg, t, toks), run_portions(m, toks, sizes)
+    m.set_mode(2)  # the plain kernels
+    plain = run_portions(m, toks, sizes)
+    m.close()
+    assert err(got, want) < min(TOL["float32"], 2 * err(plain, want) + 2e-6)
+
+
 # results without an epilogue (k_dense.hip dense_mm_ring_kernel): columns in fours, stored from the registers, the last four of a tile, one four and three fours into the next one; no fours
 # (through LDS); split along K, where the sums are stored in fours or one by one
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
