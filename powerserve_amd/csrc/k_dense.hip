@@ -1,5 +1,6 @@
 // Dense (unquantized) matrices of the layer-list models: bfloat16 operands with fp32 accumulation on v_mfma_f32_16x16x32_bf16, or
-// fp32 throughout on v_mfma_f32_16x16x4_f32 (one rounding per product, fp32 adds: a true fp32 product, no reduced-precision mode).
+// fp32 throughout on v_mfma_f32_16x16x4_f32 (one rounding per product, fp32 adds: a true fp32 product, no reduced-precision mode), or on the bf16 instruction with the operand as three bf16 lines
+// and the weights as they came (dn_ring_take, PL 3: no product is rounded at all).
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
 //   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
@@ -460,9 +461,10 @@ struct dn_ring {
 };
 
 // The A operand's rows with everything resolved that is not a plain row -- ring rows, token-shift mix, the slots' order and scale -- and, for bf16, rounded.
-template <typename WT>
+// PL 3: fp32 numbers as three of bf16, a row's three lines of K one behind the other -- rounded, the rounded rest, the rest of that: 24 bits, nothing lost.
+template <typename WT, int PL>
 __global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) { // (blockIdx.y: the copy for the i-th of several mixes)
-    if (blockIdx.y) { g.mu += (long long)blockIdx.y * g.K; out += (long long)blockIdx.y * g.T * g.K; }
+    if (blockIdx.y) { g.mu += (long long)blockIdx.y * g.K; out += (long long)blockIdx.y * g.T * g.K * PL; }
     long long row0 = g.a_row0;
     int T = g.T;
     if (!g.g_list) dn_rows(g, row0, T); // (grouped: all T slots in the order of the sorted list, whatever their matrix)
@@ -492,8 +494,21 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(dn_args g, WT *out) { /
 #pragma unroll
             for (int e = 0; e < 8; e++) v[e] += (p[e] - v[e]) * g.mu[k + e];
         }
-        WT *o = out + (long long)t * g.K + k;
-        if constexpr (sizeof(WT) == 2) {
+        WT *o = out + (long long)t * g.K * PL + k;
+        if constexpr (PL == 3) {
+            dn_us8 r[3];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                // (a finite number that rounds to infinity is cut off instead; infinity has no rest)
+                unsigned short b = dn_f2bf(v[e]);
+                if ((b & 0x7fff) == 0x7f80) b = (unsigned short)(__float_as_uint(v[e]) >> 16);
+                const float rest = (b & 0x7fff) == 0x7f80 ? 0.f : v[e] - dn_bf2f(b);
+                const unsigned short b2 = dn_f2bf(rest);
+                r[0][e] = b; r[1][e] = b2; r[2][e] = dn_f2bf(rest - dn_bf2f(b2));
+            }
+#pragma unroll
+            for (int x = 0; x < 3; x++) *(dn_us8 *)(o + x * g.K) = r[x];
+        } else if constexpr (sizeof(WT) == 2) {
             dn_us8 r;
 #pragma unroll
             for (int e = 0; e < 8; e++) r[e] = dn_f2bf(v[e]);
@@ -583,10 +598,11 @@ static __device__ __forceinline__ bool dn_ring_rows(const dn_args &g, int tm, in
     return t0 < T;
 }
 
-template <typename WT, int BM, int BN, bool ODD>
+template <typename WT, int BM, int BN, bool ODD, int PL>
 __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p) {
     extern __shared__ __attribute__((aligned(16))) char dn_lds[];
     constexpr int MI = BM / 64, NJ = BN / 64, NI = (BM + BN) / 32, STAGE = (BM + BN) * 128, NS = DN_STAGES; // instruction tiles per wave, pieces a loading wave requests per block
+    constexpr int NA = BM / 32, NW = BN / 32, WL = NS * BM * 128; // PL 3: of them of the operand and of the weights; where the weights' two stages begin
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = (wave >> 1) & 1, wn = wave & 1;
     const bool loads = wave >= 4;
     const int per = 8 * p.n_tm, b_in = (int)blockIdx.x % per, wp = ((int)blockIdx.x / per) * 8 + (b_in & 7), tm = b_in >> 3;
@@ -596,7 +612,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     long long row0;
     if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return; // (uniform per work-group)
     const long long n0 = (long long)tn * BN, ldw = g.K * (long long)sizeof(WT);
-    const int blocks = (int)(ldw >> 7), kb0 = (int)((long long)blocks * s / p.S), nk = (int)((long long)blocks * (s + 1) / p.S) - kb0;
+    const int blocks = (int)(ldw >> 7), kb0 = (int)((long long)blocks * s / p.S), nk = ((int)((long long)blocks * (s + 1) / p.S) - kb0) * PL; // (PL 3: block kb is line kb % 3 of K's block kb / 3)
     const int fr = lane & 31, fh = lane >> 5;
     dn_f16 acc[MI][NJ];
 #pragma unroll
@@ -618,7 +634,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
         }
 #pragma unroll
         for (int j = 0; j < NI; j++) {
-            const int row = 8 * (NI * lw + j) + lr, kq = ls ^ ((row >> 1) & 7);
+            const int row = PL == 3 ? (j < NW ? BM + 8 * (NW * lw + j) : 8 * (NA * lw + j - NW)) + lr : 8 * (NI * lw + j) + lr, kq = ls ^ ((row >> 1) & 7); // (PL 3: the weights' pieces first)
             const char *q;
             if (row < BM) {
                 const int t = min(t0 + row, T - 1);
@@ -632,6 +648,17 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
         const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)dn_lds + (unsigned)(NI * lw * 1024);
         auto request = [&](const int kb) {
             if (kb >= nk) return;
+            if constexpr (PL == 3) { // a block of the weights serves its three lines of the operand: two stages of it, requested with the first line
+                const int kq = kb / 3, line = kb - 3 * kq;
+                const unsigned at = lds0 - (unsigned)(NI * lw * 1024);
+                if (line == 0) {
+#pragma unroll
+                    for (int j = 0; j < NW; j++) dn_dma(src[j] + (long long)kq * 128, at + (unsigned)(WL + (kq & 1) * BN * 128 + (NW * lw + j) * 1024));
+                }
+#pragma unroll
+                for (int j = 0; j < NA; j++) dn_dma(src[NW + j] + line * ldw + (long long)kq * 128, at + (unsigned)((kb % NS) * BM * 128 + (NA * lw + j) * 1024));
+                return;
+            }
 #pragma unroll
             for (int j = 0; j < NI; j++) dn_dma(src[j] + (long long)kb * 128, lds0 + (unsigned)((kb % NS) * STAGE + j * 1024));
         };
@@ -640,7 +667,12 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
         request(2);
         for (int kb = 0; kb < nk; kb++) {
             const int later = nk - 1 - kb; // blocks requested behind this one: at most NS - 2
-            if (later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * NI) : "memory");
+            if (PL == 3) { // (with the weights of the next block of K among them, but behind its first line; whole blocks of three lines)
+                if (later >= 3 && kb % 3) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * NA + NW) : "memory");
+                else if (later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * NA) : "memory");
+                else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NA) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else if (later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * NI) : "memory");
             else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(NI) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
@@ -648,10 +680,10 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
         }
     } else {
         const int fx = (fr >> 1) & 7;
-        const char *fa0 = dn_lds + (wm * MI * 32 + fr) * 128, *fb0 = dn_lds + (BM + wn * NJ * 32 + fr) * 128;
+        const char *fa0 = dn_lds + (wm * MI * 32 + fr) * 128, *fb0 = dn_lds + (PL == 3 ? WL : BM * 128) + (wn * NJ * 32 + fr) * 128;
         dn_f4 xa[2][2][MI], xb[2][2][NJ]; // the fragments of half a block, two sets: the next half is read while this one is multiplied
         auto read = [&](const int kb, const int half) {
-            const char *fa = fa0 + (kb % NS) * STAGE, *fb = fb0 + (kb % NS) * STAGE;
+            const char *fa = fa0 + (kb % NS) * (PL == 3 ? BM * 128 : STAGE), *fb = fb0 + (PL == 3 ? (kb / 3 & 1) * BN * 128 : (kb % NS) * STAGE);
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 const int po = ((4 * half + 2 * u + fh) ^ fx) << 4; // (the row bases are multiples of 32: (row / 2) % 8 = (fr / 2) % 8)
@@ -809,7 +841,7 @@ static __device__ __forceinline__ void dn_dma_at(const char *base, unsigned off,
     unsigned keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst) : "memory");
 }
-template <bool ODD>
+template <bool ODD, int PL>
 __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p) {
     extern __shared__ __attribute__((aligned(16))) char dn_lds[];
     constexpr int BM = DN_BIG, BN = DN_BIG, HALF = 128 * 128;
@@ -820,7 +852,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
     long long row0;
     if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return; // (uniform per work-group)
     const long long n0 = (long long)tn * BN, ldw = g.K * 2;
-    const int nk = (int)(ldw >> 7);
+    const int nk = (int)(ldw >> 7) * PL; // (PL 3: block kb is line kb % 3 of K's block kb / 3; the weights' pieces stay for three of them)
     // this wave's two requests of a piece: rows 16 wave + 8 j + lane / 8, sixteen bytes each
     const char *W = (const char *)g.w + (g.g_seg ? e * g.wstride * 2 : 0), *A = p.A;
     long long nw = n0, n_rows = g.N;
@@ -845,9 +877,9 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
     const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)dn_lds + (unsigned)(wave * 2048);
     auto request_a = [&](const int kb, const int h) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) dn_dma_at(A + (long long)kb * 128, oa[h][j], lds0 + (unsigned)((2 * (kb & 1) + h) * HALF + j * 1024));
+        for (int j = 0; j < 2; j++) dn_dma_at(A + (PL == 3 ? kb % 3 * ldw + (long long)(kb / 3) * 128 : (long long)kb * 128), oa[h][j], lds0 + (unsigned)((2 * (kb & 1) + h) * HALF + j * 1024));
     };
-    auto request_w = [&](const int kb, const int h) {
+    auto request_w = [&](const int kb, const int h) { // (PL 3: kb counts blocks of K)
 #pragma unroll
         for (int j = 0; j < 2; j++) dn_dma_at(W + (long long)kb * 128, ob[h][j], lds0 + (unsigned)((4 + 2 * (kb & 1) + h) * HALF + j * 1024));
     };
@@ -873,7 +905,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #pragma unroll
         for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) xb[h][u][j] = *(const dn_f4 *)(fb[u] + (2 * (kb & 1) + h) * HALF + j * 2048);
+            for (int j = 0; j < 2; j++) xb[h][u][j] = *(const dn_f4 *)(fb[u] + (2 * ((PL == 3 ? kb / 3 : kb) & 1) + h) * HALF + j * 2048);
     };
     auto multiply = [&](const int mh, const int nh) { // between two barriers: the other group's slot of reads and requests
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -896,8 +928,13 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    for (int kb = 0; kb < min(nk, 2); kb++) { request_w(kb, 0); request_a(kb, 0); request_w(kb, 1); request_a(kb, 1); }
-    if (nk > 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    if constexpr (PL == 3) {
+        request_w(0, 0); request_a(0, 0); request_w(0, 1); request_a(0, 1); request_a(1, 0); request_a(1, 1);
+    } else {
+        for (int kb = 0; kb < min(nk, 2); kb++) { request_w(kb, 0); request_a(kb, 0); request_w(kb, 1); request_a(kb, 1); }
+    }
+    if (PL == 3) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (nk > 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -909,10 +946,14 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
     for (int kb = 0; kb < nk; kb++) {
         const bool more = kb + 2 < nk;
 #define DN_BIG_LANDED                                                     \
-    if (more) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");           \
+    if (PL == 3 && more) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); \
+    else if (more) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");      \
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // (PL 3: the next block of K's weights with its first line; behind the piece that is waited for are three of the operand's)
+        const bool more_w = PL == 3 ? kb % 3 == 0 && kb + 3 < nk : more;
+        const int kw = PL == 3 ? kb / 3 + 1 : kb + 2;
         read_a(kb, 0);
-        if (more) request_w(kb + 2, 0);
+        if (more_w) request_w(kw, 0);
         DN_BIG_LANDED
         multiply(0, 0);
         read_w(kb, 1);
@@ -920,7 +961,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
         DN_BIG_LANDED
         multiply(0, 1);
         read_a(kb, 1);
-        if (more) request_w(kb + 2, 1);
+        if (more_w) request_w(kw, 1);
         DN_BIG_LANDED
         multiply(1, 0);
         if (kb + 1 < nk) read_w(kb + 1, 0);
@@ -984,7 +1025,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 // a split product pays a second launch and its parts' way through memory.  The 256 x 256 tiles' block is what they measured beside the 128 x 128 ones: 1.7 times their time where both fill the chip
 // once (512 tokens x 8192 x 2048: 28 us there, 48 here), half of it where the smaller ones need four rounds; they are not split (2047 x 2048 x 8192 in two: 98 us, 84 as 128 x 128 tiles).
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
-static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int groups, bool bf, bool may_split, bool big) {
+static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines, int groups, bool bf, bool may_split, bool big) {
     static const int shapes[4][2] = {{128, 128}, {64, 128}, {64, 64}, {DN_BIG, DN_BIG}};
     const int64_t blocks = kbytes / 128;
     dn_ring_shape best{};
@@ -996,7 +1037,7 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int group
         const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = BM == DN_BIG ? 1700 : std::max(lds, mfma) + 100;
         for (int64_t S = 1; S <= (may_split && BM != DN_BIG ? 16 : 1); S++) {
             if (S > 1 && (blocks / S < 4 || tiles * S > 512 || (size_t)n_tm * tn * S * BM * BN * 4 > psk_dense_split_bytes())) break;
-            const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
+            const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * lines * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
             if (!best.BM || t < least) { least = t; best = dn_ring_shape{BM, BN, n_tm, tn, (int)S}; }
         }
     }
@@ -1004,54 +1045,67 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int group
 }
 
 static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR && !g.em_table && (g.N % 4 || g.ldo % 4 || ((uintptr_t)g.out & 15)); }
-template <typename WT, int BM, int BN, bool ODD>
+template <typename WT, int BM, int BN, bool ODD, int PL>
 static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if constexpr (!ODD)
-        if (dn_odd(g)) return dn_launch_ring<WT, BM, BN, true>(st, g, p);
+        if (dn_odd(g)) return dn_launch_ring<WT, BM, BN, true, PL>(st, g, p);
     constexpr int LDS = DN_STAGES * (BM + BN) * 128;
     static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN, ODD>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN, ODD, PL>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     const unsigned grid = (unsigned)((p.tn * p.S + 7) / 8 * 8) * p.n_tm;
-    hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN, ODD>), dim3(grid), dim3(512), LDS, st, g, p);
+    hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN, ODD, PL>), dim3(grid), dim3(512), LDS, st, g, p);
     if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN, ODD>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
 }
 
-template <bool ODD>
+template <bool ODD, int PL>
 static void dn_launch_big(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if constexpr (!ODD)
-        if (dn_odd(g)) return dn_launch_big<true>(st, g, p);
+        if (dn_odd(g)) return dn_launch_big<true, PL>(st, g, p);
     static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_big_kernel<ODD>, hipFuncAttributeMaxDynamicSharedMemorySize, DN_BIG_LDS);
-    hipLaunchKernelGGL(dense_mm_big_kernel<ODD>, dim3((unsigned)((p.tn + 7) / 8 * 8) * p.n_tm), dim3(512), DN_BIG_LDS, st, g, p);
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_big_kernel<ODD, PL>, hipFuncAttributeMaxDynamicSharedMemorySize, DN_BIG_LDS);
+    hipLaunchKernelGGL((dense_mm_big_kernel<ODD, PL>), dim3((unsigned)((p.tn + 7) / 8 * 8) * p.n_tm), dim3(512), DN_BIG_LDS, st, g, p);
 }
 
-// the wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed
-template <typename WT>
+// The wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed.  PL 3 (WT: bf16): an fp32 product on the bf16 instruction -- the weights as they came, which is in
+// bf16, the operand as the sum of three bf16 lines (dense_pack_kernel): every product is exact, the sums are fp32.  A block of the weights stays in LDS for its three lines.  What bounded the
+// fp32 instruction was its rate, a sixteenth of the other's; 300 tokens, it and this: 8192 x 2048 126 -> 64 us, 2048 x 8192 148 + 5 -> 69 + 5, 2048 x 2048 62 -> 31; whole requests from 9
+// tokens on (Ranutar 2048 x 3: 9 tokens 505 -> 465 us, 64: 530 -> 475, 512: 1698 -> 1044; Pupidra 4096 x 3, 200: 3662 -> 2149).  Error against 64 bits, ranutar-f32-prompt: 1.0e-6 -> 6.2e-7.
+template <typename WT, int PL>
 static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     const int64_t kbytes = g.K * (int64_t)sizeof(WT);
     const int copies = 1 + a.n_more;
     if (copies > 1 && (g.N % 128 || !g.mu)) return false;
     if (a.force_tiled || kbytes % 128 || !a.pack) return false;
     const bool rows = !g.mu && !g.g_list && !g.a_mod && !g.a_step && !g.a_row0;
-    const bool handed = sizeof(WT) == 2 && a.a16 && rows; // (the producer has rounded them already)
+    const bool handed = sizeof(WT) == 2 && PL == 1 && a.a16 && rows; // (the producer has rounded them already)
     const bool plain = handed || (sizeof(WT) == 4 && !g.mu && !g.g_scale && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0);
-    if (!plain && (size_t)a.T * kbytes * copies > a.pack_bytes) return false;
+    if (!plain && (size_t)a.T * kbytes * PL * copies > a.pack_bytes) return false;
+    if (PL == 3) {
+        for (int i = 0; i < copies; i++)
+            if (!(i ? a.more[i - 1] : a.w)->half) return false;
+        g.w = a.w->half;
+    }
     const int64_t each = g.N;
     g.N *= copies;
-    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes(), (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 23)); // (rows of a tile by 32-bit offsets)
-    dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes, r.n_tm, r.tn, r.S, a.split};
+    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, PL, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes(), (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 22)); // (rows of a tile by 32-bit offsets)
+    dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes * PL, r.n_tm, r.tn, r.S, a.split};
     p.each = copies > 1 ? each : 0;
-    p.copy = a.T * kbytes;
-    for (int i = 0; i < copies; i++) p.w[i] = i ? a.more[i - 1]->data : g.w;
+    p.copy = a.T * kbytes * PL;
+    for (int i = 0; i < copies; i++) p.w[i] = i ? (PL == 3 ? a.more[i - 1]->half : a.more[i - 1]->data) : g.w;
     if (!plain) {
         const int64_t pb = ((int64_t)a.T * (g.K / 8) + 255) / 256;
-        hipLaunchKernelGGL(dense_pack_kernel<WT>, dim3((unsigned)std::min<int64_t>(pb, 8192), (unsigned)copies), dim3(256), 0, st, g, (WT *)a.pack);
+        hipLaunchKernelGGL((dense_pack_kernel<WT, PL>), dim3((unsigned)std::min<int64_t>(pb, 8192), (unsigned)copies), dim3(256), 0, st, g, (WT *)a.pack);
     }
-    if (r.BM == DN_BIG) dn_launch_big<false>(st, g, p);
-    else if (r.BM == 128) dn_launch_ring<WT, 128, 128, false>(st, g, p);
-    else if (r.BN == 128) dn_launch_ring<WT, 64, 128, false>(st, g, p);
-    else dn_launch_ring<WT, 64, 64, false>(st, g, p);
+    if (r.BM == DN_BIG) {
+        if constexpr (sizeof(WT) == 2) dn_launch_big<false, PL>(st, g, p);
+    } else if (r.BM == 128) dn_launch_ring<WT, 128, 128, false, PL>(st, g, p);
+    else if (r.BN == 128) dn_launch_ring<WT, 64, 128, false, PL>(st, g, p);
+    else dn_launch_ring<WT, 64, 64, false, PL>(st, g, p);
     return true;
+}
+static bool dn_wide(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
+    if (a.w->dtype == PS_BF16) return dn_ring_take<unsigned short, 1>(st, a, g);
+    return (a.w->half && dn_ring_take<unsigned short, 3>(st, a, g)) || dn_ring_take<float, 1>(st, a, g);
 }
 
 // Products with an inner size of a few numbers (the second matrix of a low-rank decay): a thread has an output column, its KP weights in registers, and runs over sixteen tokens whose
@@ -1590,7 +1644,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         bool alike = true;
         for (int i = 0; i < a.n_more; i++) alike = alike && a.more[i]->dtype == a.w->dtype && a.more[i]->N == a.w->N && a.more[i]->K == a.w->K;
         if (alike && !a.force_tiled && a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 2>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 2>(st, g, nullptr, 0, &a))) return 0;
-        if (alike && a.T > 8 && (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g))) return 0;
+        if (alike && a.T > 8 && dn_wide(st, a, g)) return 0;
         for (int i = 0; i <= a.n_more; i++) {
             psk_dense_args one = a;
             one.n_more = 0;
@@ -1616,7 +1670,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
             return 0;
         }
         g.g_seg = a.g_seg; g.g_list = a.g_list;
-        if (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g)) return 0;
+        if (dn_wide(st, a, g)) return 0;
         const dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((a.T + 63) / 64), (unsigned)a.groups);
         if (bf) hipLaunchKernelGGL(dense_mm_kernel<unsigned short>, grid, dim3(256), 0, st, g);
         else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
@@ -1671,7 +1725,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         }
         return 0;
     }
-    if (a.T > 8 && (bf ? dn_ring_take<unsigned short>(st, a, g) : dn_ring_take<float>(st, a, g))) return 0;
+    if (a.T > 8 && dn_wide(st, a, g)) return 0;
     dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((a.T + 63) / 64));
     if (bf) hipLaunchKernelGGL(dense_mm_kernel<unsigned short>, grid, dim3(256), 0, st, g);
     else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
@@ -1681,6 +1735,10 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
 // ---------------------------------------------------------------------------------------------------- upload, embedding, arg-max
 __global__ void dense_widen_kernel(const unsigned short *in, long long n, float *out) {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) out[i] = dn_bf2f(in[i]);
+}
+__global__ void dense_odd_kernel(const unsigned short *in, long long n, int32_t *odd) { // infinities and NaN
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+        if ((in[i] & 0x7f80) == 0x7f80) *odd = 1;
 }
 void psk_dense_widen(hipStream_t st, const uint16_t *bf16, int64_t n, float *out) {
     long long blocks = (n + 255) / 256;
@@ -1759,16 +1817,26 @@ int ps_hip_dense_upload(ps_hip_ctx *c, const uint16_t *host, int64_t N, int64_t 
     uint16_t *raw = nullptr;
     if (ps_dev_malloc((void **)&raw, n * 2 + 64) != hipSuccess) { delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
     if (hipMemcpyAsync(raw, host, n * 2, hipMemcpyHostToDevice, c->stream) != hipSuccess) { (void)ps_dev_free(raw); delete w; PS_FAIL(c, "dense_upload: copy"); }
+    // An fp32 matrix keeps its bf16 form for the wide mat-mul (PL 3 there) where all its numbers are finite (an infinite one meets the zeros of the operand's lower lines) and where half of the
+    // device's memory is free beside it.
+    int32_t *odd = (int32_t *)((char *)raw + (n * 2 + 15) / 16 * 16), is_odd = 0;
     if (as_f32) {
         float *f = nullptr;
         if (ps_dev_malloc((void **)&f, n * 4 + 64) != hipSuccess) { (void)ps_dev_free(raw); delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
         psk_dense_widen(c->stream, raw, (int64_t)n, f);
         w->data = f;
+        psk_fill(c->stream, (float *)odd, 0.f, 1);
+        hipLaunchKernelGGL(dense_odd_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, c->stream, raw, (long long)n, odd);
     } else {
         w->data = raw;
     }
     hipError_t e = hipStreamSynchronize(c->stream);
-    if (as_f32) (void)ps_dev_free(raw);
+    if (as_f32) {
+        size_t free = 0, all = 0;
+        const bool keep = e == hipSuccess && hipMemcpy(&is_odd, odd, 4, hipMemcpyDeviceToHost) == hipSuccess && !is_odd && hipMemGetInfo(&free, &all) == hipSuccess && free > all / 2;
+        if (keep) w->half = raw;
+        else (void)ps_dev_free(raw);
+    }
     if (e != hipSuccess) { (void)ps_dev_free(w->data); delete w; PS_FAIL(c, std::string("dense_upload: ") + hipGetErrorString(e)); }
     *out = w;
     return 0;
@@ -1777,14 +1845,16 @@ void ps_hip_dense_free(ps_hip_ctx *c, ps_dense *w) {
     if (!w) return;
     if (c) (void)hipStreamSynchronize(c->stream);
     (void)ps_dev_free(w->data);
+    if (w->half) (void)ps_dev_free(w->half);
     delete w;
 }
 int ps_hip_dense_matmul(ps_hip_ctx *c, const ps_dense *w, const float *x, int T, float *out, float alpha) {
     if (!w || T <= 0) PS_FAIL(c, "dense_matmul: bad argument");
     // The wide mat-mul's scratch is the context's and stays with it: 64 MiB of packed rows (128 rows, where those are more) and the parts of split products.  More rows go through it piece
     // by piece, and where the device has no room for it the product does without.  Products that the wide mat-mul does not take need none.
-    const int64_t row = w->K * (w->dtype == PS_BF16 ? 2 : 4);
-    const bool wide = T > 8 && row % 128 == 0, packs = w->dtype == PS_BF16 || ((uintptr_t)x & 15) != 0;
+    const bool lines = w->half && w->K % 64 == 0; // (fp32 on the bf16 instruction)
+    const int64_t row = w->K * (w->dtype == PS_BF16 ? 2 : lines ? 6 : 4);
+    const bool wide = T > 8 && row % 128 == 0, packs = w->dtype == PS_BF16 || lines || ((uintptr_t)x & 15) != 0;
     const int64_t piece = wide && packs ? std::min<int64_t>(T, std::max<int64_t>(((int64_t)64 << 20) / row / 128 * 128, 128)) : T;
     const size_t pack = packs ? (size_t)(piece * row + 255) / 256 * 256 : 0, need = pack + psk_dense_split_bytes();
     if (wide && c->act_cap < need) {

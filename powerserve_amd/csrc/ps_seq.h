@@ -8,6 +8,7 @@ struct ps_dense {
     int dtype = PS_BF16; // PS_BF16 or PS_F32
     int64_t N = 0, K = 0;
     void *data = nullptr;
+    void *half = nullptr; // PS_F32: the same numbers in bf16, as they came (NULL: not kept, or not all of them finite)
 };
 
 // What every kernel of a step reads from DEVICE memory, so that one captured launch sequence replays for any position and slot:
@@ -47,7 +48,7 @@ struct psk_dense_args {
     int accum = 0; // 1: out += the result (the residual stream takes a sublayer's output projection directly)
     const float *mu = nullptr, *shift0 = nullptr;
     int force_tiled = 0; // 1: the plain tiled mat-mul whatever the shape (A/B against the mat-vec and the wide mat-mul)
-    void *pack = nullptr; // scratch for the wide mat-mul's copy of A (T rows of K in the matrix's number format); without it the plain tiled kernel runs
+    void *pack = nullptr; // scratch for the wide mat-mul's copy of A (T rows of K in bf16, or for fp32 matrices three times that); without it the plain tiled kernel runs
     size_t pack_bytes = 0;
     float *split = nullptr; // scratch for its splits of K (psk_dense_split_bytes); too small: K is not split
     size_t split_bytes = 0;

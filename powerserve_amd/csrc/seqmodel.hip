@@ -454,6 +454,11 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
                         if (P.side->d.in_bias) ok = ok && hipMemcpyAsync(bias + a->N + skip, P.side->d.in_bias, (size_t)b->N * 4, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
                     }
                 }
+                if (ok && a->half && b->half && (ok = alloc(&j->half, (na + nz + nb) / 2))) {
+                    psk_fill(c->stream, (float *)j->half, 0.f, (int64_t)((na + nz) / 8 + 1));
+                    ok = hipMemcpyAsync(j->half, a->half, na / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess &&
+                         hipMemcpyAsync((char *)j->half + (na + nz) / 2, b->half, nb / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
+                }
                 ok = ok && hipStreamSynchronize(c->stream) == hipSuccess;
                 it = joint_of.emplace(P.layer, std::make_pair((const ps_dense *)j, (const float *)bias)).first;
             }
@@ -502,8 +507,7 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
             kmax = std::max<int64_t>({kmax, P.d.ff, P.d.shared_ff, P.d.heads * (int64_t)std::max(P.d.dim, P.d.vdim), P.d.q_rank, P.d.decay_rank});
             if (P.d.kind == PS_MIX_LATENT) { kvrows = std::max<int64_t>(kvrows, P.d.window - 1 + B); kvk = std::max<int64_t>(kvk, P.d.kv_rank); }
         });
-        // (fp32: only the token-shift mixes and scaled slots are packed, the window's rows are read in place)
-        m->pack_bytes = desc->compute == 0 ? (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * 2 : (size_t)(std::max(4 * B, moe_slots) * W) * 4;
+        m->pack_bytes = (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * (desc->compute == 0 ? 2 : 6); // (fp32: three bf16 lines)
         ok = ok && alloc(&m->pack, m->pack_bytes);
         if (std::max({B, moe_slots, kvrows}) > 8) {
             m->split_bytes = psk_dense_split_bytes();

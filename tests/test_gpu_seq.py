@@ -230,6 +230,41 @@ def test_bf16_rows_handed_on(made, sizes):
     assert err(got, want) < 1.5 * err(plain, want) < 0.3
 
 
+# fp32 products on the bf16 instruction (k_dense.hip dn_ring_take, three lines of the operand): numbers that round to infinity in bf16, infinite and NaN operands and weights, numbers of every size --
+# finite rows and columns beside them as exact as ever, the others infinite or NaN as fp32 arithmetic has them
+@pytest.mark.parametrize("T,N,K", [(16, 24, 64), (70, 130, 192), (700, 5000, 64)])
+@pytest.mark.parametrize("odd_weights", [False, True])
+def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights):
+    import ctypes as C
+    rng = np.random.default_rng(T)
+    w = rng.standard_normal((N, K), dtype=np.float32)
+    if odd_weights:
+        w[3, 5], w[7, 1] = np.inf, np.nan
+    bits = f32_to_bf16_bits(w)
+    w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K)
+    x = rng.standard_normal((T, K), dtype=np.float32)
+    x[1] *= np.float32(10.0) ** rng.integers(-30, 30, K).astype(np.float32)
+    x[2], x[2, 9] = 0, np.float32(3.4028e38)  # (the next bf16 is infinity)
+    x[4, 0], x[5, 3] = np.inf, np.nan
+    x[6] = 1  # (its lower lines are zeros)
+    h = C.c_void_p()
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, 1, C.byref(h)))
+    dx, do = ctx.to_device(x), ctx.empty((T, N))
+    ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, h, dx.ptr, T, do.ptr, 2.0 ** -8))
+    got = do.numpy()
+    with np.errstate(all="ignore"):
+        want = (x.astype(np.float64) @ w.astype(np.float64).T) * 2.0 ** -8
+        bound = (K + 2) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T) * 2.0 ** -8
+        over, beyond = (np.abs(want) * 2.0 ** 8 > v for v in (3.4e38, 3.41e38))  # (fp32's largest number is 3.4028e38: sums near it may or may not end at infinity, sums beyond it do)
+    fine = np.isfinite(want) & ~over
+    assert np.all(np.abs(got[fine] - want[fine]) <= bound[fine])
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isfinite(want) & ~np.isnan(want)], want[~np.isfinite(want) & ~np.isnan(want)].astype(np.float32))
+    assert np.all(np.isinf(got[beyond & np.isfinite(want)]))
+    ctx.L.ps_hip_dense_free(ctx.h, h)
+    dx.free(); do.free()
+
+
 # 256 x 256 tiles behind an epilogue (k_dense.hip dense_mm_big_kernel): an activation whose rounded rows the second product reads, pairs, the four mixes of a token shift, the slots of experts (tiles
 # that end inside an expert, an expert without slots) with a factor per row
 @pytest.mark.parametrize("which", ["xielu", "pairs", "experts", "mixes"])
