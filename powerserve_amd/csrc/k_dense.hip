@@ -1223,6 +1223,7 @@ struct dn_mv1 {
     int kp;      // padded length of the vector
     int blocks, blocks2; // FORM 1: work-groups per slot, of the shared expert; FORM 2: per matrix
     const void *w[1 + psk_dense_args::MORE]; // FORM 2: the matrices
+    psk_dense_pre pre;
 };
 
 // one vector into LDS, by all 512 threads
@@ -1283,7 +1284,79 @@ static __device__ __forceinline__ float dn_wave_sum(float v) { // every lane get
     return (row(0) + row(16)) + (row(32) + row(48));
 }
 
-template <typename WT, int FORM, bool RAGGED> // RAGGED: a row ends inside a unit
+// One vector into LDS through what stands in front of the product (ps_seq.h psk_dense_pre), by all 512 threads: a thread's up to four runs of four numbers, 2048 apart.  All of it is requested in
+// front of the weights (dn_pre_request), whose way from memory covers the sums.  A boundary of 2048 numbers and the first product behind it 4.6 + 10.1 us -> 10.9, 4.6 + 5.9 -> 6.8 (kernel trace).
+struct dn_pre_runs { dn_f4 x[4], z[4], w[4]; };
+template <int PRE>
+static __device__ __forceinline__ void dn_pre_request(const dn_args &g, const psk_dense_pre &r, dn_pre_runs &o) {
+    const int K = (int)g.K, tid = threadIdx.x;
+    const float *second = PRE == psk_dense_pre::BOUNDARY ? r.y : r.gate;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int k = (tid + 512 * j) * 4;
+        const bool in = k < K;
+        o.x[j] = in ? *(const dn_f4 *)(g.a + k) : dn_f4{0.f, 0.f, 0.f, 0.f};
+        o.z[j] = in ? *(const dn_f4 *)(second + k) : dn_f4{0.f, 0.f, 0.f, 0.f};
+        o.w[j] = in ? *(const dn_f4 *)(r.w + (PRE == psk_dense_pre::HEADS ? k / r.part * r.w_stride + k % r.part : k)) : dn_f4{0.f, 0.f, 0.f, 0.f};
+    }
+}
+template <typename WT, int PRE>
+static __device__ __forceinline__ void dn_stage_pre(const dn_args &g, const psk_dense_pre &r, dn_pre_runs &o, float *xs) {
+    __shared__ float red[32];
+    const int K = (int)g.K, tid = threadIdx.x, runs = (K + 2047) / 2048;
+    auto &x = o.x;
+    auto &z = o.z;
+    auto &w = o.w;
+    float s[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        s[j] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float v = PRE == psk_dense_pre::BOUNDARY ? z[j][e] : x[j][e];
+            s[j] = fmaf(v, v, s[j]);
+        }
+    }
+    if (PRE == psk_dense_pre::HEADS) { // (a head: part / 4 lanes of a wave)
+        for (int o = r.part / 8; o > 0; o >>= 1)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (j < runs) s[j] += __shfl_xor(s[j], o, 64);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (j < runs) {
+                const float t = dn_wave_sum(s[j]);
+                if ((tid & 63) == 0) red[8 * j + (tid >> 6)] = t;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j >= runs) continue;
+            s[j] = 0.f;
+            for (int q = 0; q < K / 256; q++) s[j] += red[q];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int k = (tid + 512 * j) * 4;
+        if (k >= K) continue;
+        const float inv = 1.f / sqrtf(s[j] / (float)(PRE == psk_dense_pre::BOUNDARY ? K : r.part) + r.eps);
+        dn_f4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (PRE == psk_dense_pre::HEADS) v[e] = x[j][e] * inv * w[j][e] * dn_silu(z[j][e]);
+            else v[e] = x[j][e] + z[j][e] * inv * (r.offset + w[j][e]);
+        }
+        if (PRE == psk_dense_pre::BOUNDARY && blockIdx.x == 0) *(dn_f4 *)(r.xout + k) = v;
+        if constexpr (sizeof(WT) == 2) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = dn_bf2f(dn_f2bf(v[e]));
+        }
+        *(dn_f4 *)(xs + k) = v;
+    }
+}
+template <typename WT, int FORM, bool RAGGED, int PRE = 0> // RAGGED: a row ends inside a unit; PRE: psk_dense_pre (whole units)
 __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
     constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE; // elements per lane and per unit
@@ -1336,13 +1409,20 @@ __global__ __launch_bounds__(512, 4) void dense_mv1_kernel(dn_args g0, dn_mv1 p)
         if (++lu == row_units) open();
     };
     dn_f4 ring[DN_AHEAD];
+    dn_pre_runs pre;
+    if constexpr (PRE) {
+        dn_pre_request<PRE>(g, p.pre, pre);
+        asm volatile("" ::: "memory"); // (in front of the weights)
+    }
     if (rows && row_units) {
         open();
 #pragma unroll
         for (int u = 0; u < DN_AHEAD; u++) request(ring[u]);
     }
     // the activations
-    if constexpr (FORM != 1) {
+    if constexpr (PRE) {
+        dn_stage_pre<WT, PRE>(g, p.pre, pre, xs);
+    } else if constexpr (FORM != 1) {
         long long row0;
         int T;
         dn_rows(g, row0, T);
@@ -1430,6 +1510,14 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
         for (int i = 0; i < n; i++) p.w[i] = i ? a->more[i - 1]->data : g.w;
     }
     const auto kernel = p.kp == g.K ? dense_mv1_kernel<WT, FORM, false> : dense_mv1_kernel<WT, FORM, true>;
+    if constexpr (FORM == 0) {
+        if (a && a->pre.kind) {
+            p.pre = a->pre;
+            const auto with = p.pre.kind == psk_dense_pre::HEADS ? dense_mv1_kernel<WT, 0, false, psk_dense_pre::HEADS> : dense_mv1_kernel<WT, 0, false, psk_dense_pre::BOUNDARY>;
+            hipLaunchKernelGGL(with, dim3((unsigned)grid), dim3(512), lds, st, g, p); // (at most 32 KB of activations: no attribute)
+            return true;
+        }
+    }
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), lds, st, g, p);
     return true;
 }
@@ -1438,7 +1526,7 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
 // them.  `waves` waves of a work-group share a row, each with the same up to U units of it, so that a wave's part of the activations (up to top + 1 vectors of different experts) stays in
 // its registers and nothing waits for a copy of all of them in LDS; eight units and more per wave are in flight, across row ends.  The waves' sums of a row meet in LDS at the end.
 // blockIdx.y = token.  Top 2 of 2048 x 3072 and a shared one of twice that (50 MB), one token: 16.6 us and 17.5 us more for the shared expert before, 18.0 as one stream with the activations in LDS
-// (as above), 14.3 now.  The form above is the better one where there is a single vector: 2048 x 4096 6.6 us there, 9 with this kernel's arrangement.
+// (as above), 14.3 then; 13.9 since the weights are requested in front of what is done to the activations.  The form above is the better one where there is a single vector: 2048 x 4096 6.6 us there, 9 with this kernel's arrangement.
 // dynamic LDS: [8][rows] sums
 struct dn_mv2 {
     dn_args g2; // the shared expert's second product (w NULL: none; only w, a, lda, K, out_scale are read)
@@ -1465,7 +1553,9 @@ __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g
     const char *base[U];
     bool has[U], second[U]; // (a slot without a matrix -- an identity expert -- has none; second: the shared expert's)
     int lo[U];
-    float x[U][VE];
+    float x[U][VE], f[U];
+    bool in[U];
+    // (requests only, the weights' behind them: what is done to the activations waits for them alone and runs while the weights are on their way)
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int c = min((u0 + u) / p.units, p.slots), at = u0 + u - c * p.units; // slot, unit of a row of its matrix
@@ -1473,34 +1563,29 @@ __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g
         has[u] = u < n_units;
         const float *xr = p.g2.a + (long long)y * p.g2.lda;
         const WT *w = (const WT *)p.g2.w;
-        float f = 1.f;
+        f[u] = 1.f;
         if (!second[u]) {
             const int s = y * p.slots + c, m = __builtin_amdgcn_readlane(sel, min(c, 63));
             has[u] = has[u] && m < g.groups;
             xr = g.a + (long long)(s / g.g_adiv) * g.lda;
             w = (const WT *)g.w + (long long)m * g.wstride;
-            if (g.g_scale && has[u]) f = g.g_scale[s];
+            if (g.g_scale && has[u]) f[u] = g.g_scale[s];
         }
         const int k = at * UNIT + lane * VE, Kc = second[u] ? K2 : K;
-        const bool in = has[u] && k < Kc;
+        in[u] = has[u] && k < Kc;
         lo[u] = !RAGGED || k < Kc ? lane * 16 : 0;
         base[u] = (const char *)(w + (long long)at * UNIT);
-        const float *xk = xr + k;
+        const float *xk = xr + (in[u] ? k : 0); // (the row's first numbers are there whatever is asked for)
         if (((uintptr_t)xr & 15) == 0) { // (uniform)
 #pragma unroll
             for (int e = 0; e < VE; e += 4) {
-                const dn_f4 v = in ? *(const dn_f4 *)(xk + e) : dn_f4{0.f, 0.f, 0.f, 0.f};
+                const dn_f4 v = *(const dn_f4 *)(xk + (in[u] ? e : 0));
 #pragma unroll
                 for (int i = 0; i < 4; i++) x[u][e + i] = v[i];
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < VE; e++) x[u][e] = in ? xk[e] : 0.f;
-        }
-#pragma unroll
-        for (int e = 0; e < VE; e++) {
-            x[u][e] *= f;
-            if constexpr (sizeof(WT) == 2) x[u][e] = dn_bf2f(dn_f2bf(x[u][e]));
+            for (int e = 0; e < VE; e++) x[u][e] = xk[in[u] ? e : 0];
         }
     }
     float ident = 0.f; // the summed weights of the token's slots that have no matrix
@@ -1518,6 +1603,14 @@ __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g
     };
 #pragma unroll
     for (int d = 0; d < AHEAD; d++) request(ring[d], d);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int e = 0; e < VE; e++) {
+            x[u][e] = in[u] ? x[u][e] * f[u] : 0.f;
+            if constexpr (sizeof(WT) == 2) x[u][e] = dn_bf2f(dn_f2bf(x[u][e]));
+        }
     for (int k0 = 0; k0 < rows; k0 += AHEAD) {
 #pragma unroll
         for (int d = 0; d < AHEAD; d++) {
@@ -1632,6 +1725,16 @@ static int dn_grouped_mv1(hipStream_t st, const psk_dense_args &a, const dn_args
     return (second ? dn_launch_mv2<WT>(st, g, nullptr, a.g_inner, a.T) : dn_launch_mv1<WT, 1>(st, g, nullptr, a.T)) ? 1 : 0;
 }
 
+bool psk_dense_takes_pre(const psk_dense_args &a) {
+    auto aligned = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
+    if (!a.w || a.T != 1 || a.force_tiled || a.groups || a.mu || a.a_mod || a.a_step || a.a_row0 || a.n_more || a.w->N > (1 << 28)) return false;
+    const int64_t K = a.w->K, unit = a.w->dtype == PS_BF16 ? 512 : 256; // (whole units of the stream; four runs a thread)
+    const psk_dense_pre &r = a.pre;
+    if (K % unit || K > 8192 || !aligned(a.a) || !aligned(r.w)) return false;
+    // (heads: 4096 numbers and as many of the gate read by 512 work-groups take what the launch in front did: a token of Ranutar 2048 x 6 367 -> 360 us with it, of 4096 x 3 335 -> 336)
+    if (r.kind == psk_dense_pre::HEADS) return K <= 2048 && aligned(r.gate) && r.part >= 4 && r.part <= 256 && (r.part & (r.part - 1)) == 0 && K % r.part == 0 && r.w_stride % 4 == 0;
+    return r.kind == psk_dense_pre::BOUNDARY && aligned(r.y) && aligned(r.xout) && r.xout != a.a;
+}
 bool psk_dense_wide16(const psk_dense_args &a) {
     return a.w && a.w->dtype == PS_BF16 && a.T > 8 && !a.force_tiled && a.pack && a.groups == 0 && !a.mu && !a.a_mod && !a.a_step && !a.a_row0 && a.w->K > 256 && a.w->K % 64 == 0 &&
            (size_t)a.T * a.w->K * 2 <= a.pack_bytes;
@@ -1677,7 +1780,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         return 0;
     }
     if (!a.force_tiled && a.T <= 8) {
-        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0) : dn_launch_mv1<float, 0>(st, g, nullptr, 0))) return 0;
+        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 0>(st, g, nullptr, 0, &a))) return 0;
         const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
         if (kp4 * C <= 64 * 1024) {
             // (a token's rows that the stream does not take: four per wave would leave at most 64 blocks.  1004 x 4102 14.2 us, with one per wave 11.9; 512 x 1026 6.7 and 5.3)
@@ -1770,12 +1873,9 @@ void psk_embed(hipStream_t st, const ps_dense *table, const int32_t *tokens, con
                        (long long)ldo, bigram ? bigram->data : nullptr, (long long)buckets, (long long)mul_prev, (long long)mul_cur);
 }
 
-// a row's largest logit, the lowest index among equals: a block per row, four numbers per load where the row is aligned (32000 logits: 8.5 us with 256 threads and single numbers, 3.1 now)
-__global__ __launch_bounds__(1024) void dense_argmax_kernel(const float *x, long long n, int32_t *out) {
-    __shared__ float bv[16];
-    __shared__ int bi[16];
-    const float *row = x + (long long)blockIdx.x * n;
-    const int tid = threadIdx.x, count = (int)n;
+// index of row's first maximum among `count` numbers (thread 0 has it), by 1024 threads: four numbers per load where the row is aligned (32000 logits: 8.5 us with 256 threads and single numbers, 3.1 now)
+static __device__ __forceinline__ int dn_first_max(const float *row, int count, float *bv, int *bi) {
+    const int tid = threadIdx.x;
     float best = -INFINITY;
     int at = count;
     auto take = [&](float v, int i) {
@@ -1799,8 +1899,43 @@ __global__ __launch_bounds__(1024) void dense_argmax_kernel(const float *x, long
         best = tid < 16 ? bv[tid] : -INFINITY;
         at = tid < 16 ? bi[tid] : count;
         for (int o = 8; o > 0; o >>= 1) take(__shfl_xor(best, o, 64), __shfl_xor(at, o, 64));
-        if (tid == 0) out[blockIdx.x] = at < count ? at : 0;
     }
+    return at < count ? at : 0;
+}
+// A greedy step's end and the next one's beginning in one block (ps_seq.h psk_next_token): the arg-max, the step's numbers and the embedding were three launches of 4 us each, most of it their start.
+__global__ __launch_bounds__(1024) void dense_next_kernel(const float *x, long long n, ps_seq_step *step, int32_t *ids, int32_t *prev, const void *table, int is_bf16, long long K, float scale, float *out,
+                                                          const void *bigram, long long buckets, long long mul_prev, long long mul_cur) {
+    __shared__ float bv[16];
+    __shared__ int bi[16], id;
+    const int before = step->token0, kept = step->_pad; // (thread 0 writes them behind the barrier)
+    const int at = dn_first_max(x, (int)n, bv, bi);
+    if (threadIdx.x == 0) {
+        id = at;
+        ids[kept] = at;
+        step->prev = before;
+        if (prev) *prev = before;
+        step->_pad = kept + 1;
+        step->token0 = at;
+        step->pos0 += 1;
+    }
+    __syncthreads();
+    const long long tok = id, row = bigram ? ((long long)before * mul_prev + tok * mul_cur) % buckets : 0; // (never a sequence's first token)
+    for (long long k = threadIdx.x; k < K; k += 1024) {
+        const float v = dn_table(table, is_bf16, tok * K + k) * scale;
+        out[k] = bigram ? v + dn_table(bigram, is_bf16, row * K + k) : v;
+    }
+}
+void psk_next_token(hipStream_t st, const float *logits, int64_t n, ps_seq_step *step, int32_t *ids, int32_t *prev, const ps_dense *table, float scale, float *out, const ps_dense *bigram,
+                    int64_t buckets, int64_t mul_prev, int64_t mul_cur) {
+    hipLaunchKernelGGL(dense_next_kernel, dim3(1), dim3(1024), 0, st, logits, (long long)n, step, ids, prev, table->data, table->dtype == PS_BF16 ? 1 : 0, (long long)table->K, scale, out,
+                       bigram ? bigram->data : nullptr, (long long)buckets, (long long)mul_prev, (long long)mul_cur);
+}
+// a row's largest logit, the lowest index among equals: a block per row
+__global__ __launch_bounds__(1024) void dense_argmax_kernel(const float *x, long long n, int32_t *out) {
+    __shared__ float bv[16];
+    __shared__ int bi[16];
+    const int at = dn_first_max(x + (long long)blockIdx.x * n, (int)n, bv, bi);
+    if (threadIdx.x == 0) out[blockIdx.x] = at;
 }
 void psk_argmax_rows(hipStream_t st, const float *x, int64_t n, int rows, int32_t *out) {
     hipLaunchKernelGGL(dense_argmax_kernel, dim3(rows), dim3(1024), 0, st, x, (long long)n, out);

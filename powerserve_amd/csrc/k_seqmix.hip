@@ -386,10 +386,12 @@ void psk_copy(hipStream_t st, const float *src, float *dst, int64_t n) {
 // A single token's sublayer boundary in one launch (one block):  x += y / rms(y) * (offset + wb)   (where y is given), then, where wn is given,
 // h = conv(x / rms(x) * (offset + wn)) with the convolution's residual form and its tail brought up to date -- three launches of the kernels above.
 // What bounds it is the latency of a chain: read, sum, read, sum, read.  So a thread owns C runs of four channels and requests everything that it will need of them -- x, y, both weights,
-// the filter's taps and the tail -- before the first sum, and keeps it in registers.  TAPS: 0 where wn is not given, else the taps.  n = 4096, 4 taps: 12.6 us with a loop per sum, 6.2 now;
+// the filter's taps and the tail -- before the first sum, and keeps it in registers.  TAPS: 0 where wn is not given, -1 where there is no filter (hn alone is made), else the taps.  n = 4096, 4 taps: 12.6 us with a loop per sum, 6.2 now;
 // n = 2048 without the second half: 2.8 to 4.6 and 2.0 to 3.9.
+// Several blocks (then x_out is not x): each makes both sums for itself and what follows for its share of the threads' runs, so that the filters and the tail, 112 KB of 4096 channels from memory, come
+// to several CUs: 4096, 4 taps 6.4 -> 4.9 us in four.
 template <int TAPS, int C>
-__global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw,
+__global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_step *step, const float *x, float *x_out, const float *y, const float *wb, const float *wn, const float *cw,
                                                                  long long tail_off, float offset, float eps, int n, float *h, float *hn) {
     __shared__ float red[2][16];
     const int tid = threadIdx.x, nw = blockDim.x >> 6;
@@ -402,7 +404,8 @@ __global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_st
         return t;
     };
     const sq_f4 zero = {0.f, 0.f, 0.f, 0.f};
-    sq_f4 xv[C], yv[C], b4[C], n4[C], f[C][TAPS ? TAPS : 1], tl[C][TAPS > 1 ? TAPS - 1 : 1];
+    const bool mine = tid * (int)gridDim.x / (int)blockDim.x == (int)blockIdx.x;
+    sq_f4 xv[C], yv[C], b4[C], n4[C], f[C][TAPS > 0 ? TAPS : 1], tl[C][TAPS > 1 ? TAPS - 1 : 1];
     float *tail = TAPS > 1 ? step->state + tail_off : nullptr;
 #pragma unroll
     for (int c = 0; c < C; c++) {
@@ -411,12 +414,12 @@ __global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_st
         yv[c] = in && y ? *(const sq_f4 *)(y + i) : zero;
         xv[c] = in ? *(const sq_f4 *)(x + i) : zero;
         b4[c] = in && y ? *(const sq_f4 *)(wb + i) : zero;
+        if constexpr (TAPS != 0) n4[c] = in && mine ? *(const sq_f4 *)(wn + i) : zero;
         if constexpr (TAPS > 0) {
-            n4[c] = in ? *(const sq_f4 *)(wn + i) : zero;
 #pragma unroll
-            for (int j = 0; j < TAPS; j++) f[c][j] = in ? *(const sq_f4 *)(cw + (long long)i * TAPS + 4 * j) : zero;
+            for (int j = 0; j < TAPS; j++) f[c][j] = in && mine ? *(const sq_f4 *)(cw + (long long)i * TAPS + 4 * j) : zero;
 #pragma unroll
-            for (int j = 0; j + 1 < TAPS; j++) tl[c][j] = in ? *(const sq_f4 *)(tail + (long long)j * n + i) : zero;
+            for (int j = 0; j + 1 < TAPS; j++) tl[c][j] = in && mine ? *(const sq_f4 *)(tail + (long long)j * n + i) : zero;
         }
     }
     if (y) {
@@ -431,10 +434,10 @@ __global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_st
             const int i = (tid + c * (int)blockDim.x) * 4;
 #pragma unroll
             for (int e = 0; e < 4; e++) xv[c][e] = xv[c][e] + yv[c][e] * inv * (offset + b4[c][e]);
-            if (i < n) *(sq_f4 *)(x + i) = xv[c];
+            if (i < n && mine) *(sq_f4 *)(x_out + i) = xv[c];
         }
     }
-    if constexpr (TAPS > 0) {
+    if constexpr (TAPS != 0) {
         float s2 = 0.f;
 #pragma unroll
         for (int c = 0; c < C; c++)
@@ -444,21 +447,24 @@ __global__ __launch_bounds__(1024) void sq_boundary1_fast_kernel(const ps_seq_st
 #pragma unroll
         for (int c = 0; c < C; c++) {
             const int i = (tid + c * (int)blockDim.x) * 4;
-            if (i >= n) continue;
+            if (i >= n || !mine) continue;
             sq_f4 v, o;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                v[e] = xv[c][e] * inv * (offset + n4[c][e]);
-                auto tap = [&](int j) { return f[c][(e * TAPS + j) / 4][(e * TAPS + j) % 4]; };
-                float t = tap(TAPS - 1) * v[e];
+            for (int e = 0; e < 4; e++) v[e] = xv[c][e] * inv * (offset + n4[c][e]);
+            if constexpr (TAPS > 0) {
 #pragma unroll
-                for (int j = 0; j + 1 < TAPS; j++) t = fmaf(tap(j), tl[c][j][e], t);
-                o[e] = v[e] + t;
+                for (int e = 0; e < 4; e++) {
+                    auto tap = [&](int j) { return f[c][(e * TAPS + j) / 4][(e * TAPS + j) % 4]; };
+                    float t = tap(TAPS - 1) * v[e];
+#pragma unroll
+                    for (int j = 0; j + 1 < TAPS; j++) t = fmaf(tap(j), tl[c][j][e], t);
+                    o[e] = v[e] + t;
+                }
+                *(sq_f4 *)(h + i) = o;
+#pragma unroll
+                for (int j = 0; j + 1 < TAPS; j++) *(sq_f4 *)(tail + (long long)j * n + i) = j + 2 < TAPS ? tl[c][j + 2 < TAPS ? j + 1 : 0] : v;
             }
             if (hn) *(sq_f4 *)(hn + i) = v;
-            *(sq_f4 *)(h + i) = o;
-#pragma unroll
-            for (int j = 0; j + 1 < TAPS; j++) *(sq_f4 *)(tail + (long long)j * n + i) = j + 2 < TAPS ? tl[c][j + 2 < TAPS ? j + 1 : 0] : v;
         }
     }
 }
@@ -503,20 +509,24 @@ __global__ __launch_bounds__(1024) void sq_boundary1_kernel(const ps_seq_step *s
         if (taps > 1) tail[(long long)(taps - 2) * n + c] = v;
     }
 }
-void psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
-                   float offset, float eps, int64_t n, float *h, float *hn) {
+bool psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
+                   float offset, float eps, int64_t n, float *h, float *hn, float *x_out) {
     auto aligned = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
-    const int t = wn ? taps : 0;
-    if (n % 4 == 0 && n <= 8192 && tail_off % 4 == 0 && (t == 0 || t == 1 || t == 4) && aligned(x) && aligned(y) && aligned(wb) && aligned(wn) && aligned(cw) && aligned(h) && aligned(hn)) {
+    const int t = wn ? (cw ? taps : -1) : 0;
+    if (n % 4 == 0 && n <= 8192 && tail_off % 4 == 0 && (t == 0 || t == -1 || t == 1 || t == 4) && aligned(x) && aligned(y) && aligned(wb) && aligned(wn) && aligned(cw) && aligned(h) && aligned(hn)) {
         const int threads = (int)std::min<int64_t>((n / 4 + 63) / 64 * 64, 1024);
+        const bool several = x_out && y && t == 4 && n >= 2048 && aligned(x_out) && threads % 256 == 0;
         auto go = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), 0, st, step, x, y, wb, wn, cw, (long long)tail_off, offset, eps, (int)n, h, hn);
+            hipLaunchKernelGGL(kernel, dim3(several ? 4 : 1), dim3(threads), 0, st, step, x, several ? x_out : x, y, wb, wn, cw, (long long)tail_off, offset, eps, (int)n, h, hn);
         };
-        if (n <= 4096) t == 0 ? go(sq_boundary1_fast_kernel<0, 1>) : t == 1 ? go(sq_boundary1_fast_kernel<1, 1>) : go(sq_boundary1_fast_kernel<4, 1>);
+        if (t < 0) n <= 4096 ? go(sq_boundary1_fast_kernel<-1, 1>) : go(sq_boundary1_fast_kernel<-1, 2>);
+        else if (n <= 4096) t == 0 ? go(sq_boundary1_fast_kernel<0, 1>) : t == 1 ? go(sq_boundary1_fast_kernel<1, 1>) : go(sq_boundary1_fast_kernel<4, 1>);
         else t == 0 ? go(sq_boundary1_fast_kernel<0, 2>) : t == 1 ? go(sq_boundary1_fast_kernel<1, 2>) : go(sq_boundary1_fast_kernel<4, 2>);
-        return;
+        return several;
     }
-    hipLaunchKernelGGL(sq_boundary1_kernel, dim3(1), dim3(n >= 2048 ? 1024 : 256), 0, st, step, x, y, wb, wn, cw, taps, (long long)tail_off, offset, eps, (long long)n, h, hn);
+    hipLaunchKernelGGL(sq_boundary1_kernel, dim3(1), dim3(n >= 2048 ? 1024 : 256), 0, st, step, x, y, wb, t < 0 ? nullptr : wn, cw, taps, (long long)tail_off, offset, eps, (long long)n, h, hn);
+    if (t < 0) psk_rmsnorm(st, x, n, nullptr, wn, offset, eps, n, 1, hn, n);
+    return false;
 }
 
 // ---------------------------------------------------------------------------------------------------- recurrent scans

@@ -34,6 +34,16 @@ enum { PSD_ACT_NONE = 0, PSD_ACT_XIELU = 1, PSD_ACT_TANH = 2,
 //   ring starting at the device-side a_step->pos0 + a_row0 (clamped at 0) -- see k_latent.hip;
 //   with mu: the token-shift mix a[t][k] + (prev(t)[k] - a[t][k]) * mu[k], prev(t) = t ? a[t-1] : shift0.
 // In the bf16 mode A is rounded to bfloat16 (nearest even) before the product; accumulation is fp32 in both modes.
+// What a single token's mat-vec does to its operand a on the way to LDS, every work-group for itself (psk_dense_takes_pre), in place of a launch in front of it:
+//   heads     a[k] / rms(a over its head of `part` numbers) * w[head w_stride + k % part] * silu(gate[k])
+//   boundary  v = a[k] + y[k] / rms(y) * (offset + w[k]), which is also written to xout (not a: other work-groups still read it)
+struct psk_dense_pre {
+    enum { NONE = 0, HEADS = 1, BOUNDARY = 2 };
+    int kind = NONE, w_stride = 0, part = 0;
+    const float *gate = nullptr, *w = nullptr, *y = nullptr;
+    float eps = 0.f, offset = 0.f;
+    float *xout = nullptr;
+};
 struct psk_dense_args {
     const ps_dense *w = nullptr;
     const float *a = nullptr;
@@ -84,7 +94,9 @@ struct psk_dense_args {
     static constexpr int MORE = 3;
     int n_more = 0;
     const ps_dense *more[MORE] = {};
+    psk_dense_pre pre; // (only where psk_dense_takes_pre)
 };
+bool psk_dense_takes_pre(const psk_dense_args &a);
 bool psk_dense_wide16(const psk_dense_args &a); // psk_dense will run this as the wide bf16 mat-mul over plain rows
 int psk_dense(hipStream_t st, const psk_dense_args &a);
 size_t psk_dense_split_bytes(); // what any product's splits need at most
@@ -93,6 +105,10 @@ void psk_dense_widen(hipStream_t st, const uint16_t *bf16, int64_t n, float *out
 //   bigram given: + bigram[(prev * mul_prev + token * mul_cur) mod buckets][:], or its row `buckets` for position 0; prev = tokens[t - 1], in front of the step step->prev
 void psk_embed(hipStream_t st, const ps_dense *table, const int32_t *tokens, const ps_seq_step *step, int T, float scale, float *out, int64_t ldo, const ps_dense *bigram = nullptr,
                int64_t buckets = 0, int64_t mul_prev = 0, int64_t mul_cur = 0);
+// the end of a greedy step and the beginning of the next one: id = the first maximum of logits[0..n), kept at ids[step->_pad++]; step->prev (and *prev, where given) = step->token0, which becomes id;
+// the position moves on; out = id's embedding (psk_embed)
+void psk_next_token(hipStream_t st, const float *logits, int64_t n, ps_seq_step *step, int32_t *ids, int32_t *prev, const ps_dense *table, float scale, float *out, const ps_dense *bigram,
+                    int64_t buckets, int64_t mul_prev, int64_t mul_cur);
 // out[r] = index of the first maximum of x[r][0..n)
 void psk_argmax_rows(hipStream_t st, const float *x, int64_t n, int rows, int32_t *out);
 
@@ -135,8 +151,9 @@ static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane get
 }
 // One token's sublayer boundary fused: x += norm_b(y) (y may be NULL), then h = conv(norm(x)) in the residual form with the tail update (wn may be NULL: stop after x);
 // hn (may be NULL) also receives norm(x) itself, for a sublayer that reads the unfiltered input
-void psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
-                   float offset, float eps, int64_t n, float *h, float *hn);
+// (wn without cw: no filter, hn alone); x_out given: the new x may go there instead of to x; returns whether it has
+bool psk_boundary1(hipStream_t st, const ps_seq_step *step, float *x, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off,
+                   float offset, float eps, int64_t n, float *h, float *hn, float *x_out = nullptr);
 // state row copy: (step->state + off)[0..n) = src[0..n)
 void psk_state_store(hipStream_t st, const ps_seq_step *step, int64_t off, const float *src, int64_t n);
 void psk_fill(hipStream_t st, float *p, float v, int64_t n);

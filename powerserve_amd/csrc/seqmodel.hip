@@ -62,7 +62,7 @@ struct ps_hip_seq {
     std::vector<float *> slot_state;
     std::vector<int64_t> slot_pos; // -1: free
     ps_seq_step *step = nullptr;   // device
-    float *x = nullptr, *hn = nullptr, *h = nullptr, *y = nullptr, *t1 = nullptr, *t2 = nullptr, *t3 = nullptr, *t4 = nullptr, *kvx = nullptr, *xn = nullptr,
+    float *x = nullptr, *x2 = nullptr, *hn = nullptr, *h = nullptr, *y = nullptr, *t1 = nullptr, *t2 = nullptr, *t3 = nullptr, *t4 = nullptr, *kvx = nullptr, *xn = nullptr,
           *logits = nullptr;
     int32_t *tokens = nullptr, *want = nullptr, *amax = nullptr, *ids = nullptr;
     float *hist = nullptr;        // depth_mix: [runs + 1][rows][width], X_0 = the embedding, run i writes X_(i+1)
@@ -98,17 +98,6 @@ __global__ void seq_set_step_kernel(ps_seq_step *s, long long pos0, int n, int s
     s->prev = prev ? *prev : 0; s->_pad2 = 0;
     if (prev) *prev = last;
 }
-// behind a greedy single-token step: the arg-max becomes the next token, the position moves on, the id is kept at ids[_pad++]
-__global__ void seq_advance_kernel(ps_seq_step *s, const int32_t *amax, int32_t *ids, int32_t *prev) {
-    const int32_t id = amax[0];
-    s->prev = s->token0;
-    if (prev) *prev = s->token0;
-    ids[s->_pad] = id;
-    s->_pad += 1;
-    s->token0 = id;
-    s->pos0 += 1;
-}
-
 static const int CHUNKED_FROM = 32; // tokens from which a portion's recurrences run in chunks (fewer: the scans)
 
 static int seq_fail(ps_hip_ctx *c, const std::string &msg) { c->err = msg; return 2; }
@@ -468,7 +457,7 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
             n1 = std::max(n1, P.in_ld);
         }
     }
-    ok = ok && alloc((void **)&m->step, sizeof(ps_seq_step)) && alloc((void **)&m->x, B * W * 4) && alloc((void **)&m->hn, B * W * 4) && alloc((void **)&m->h, B * W * 4) &&
+    ok = ok && alloc((void **)&m->step, sizeof(ps_seq_step)) && alloc((void **)&m->x, B * W * 4) && alloc((void **)&m->x2, W * 4) && alloc((void **)&m->hn, B * W * 4) && alloc((void **)&m->h, B * W * 4) &&
          alloc((void **)&m->y, B * W * 4) && alloc((void **)&m->t1, B * std::max<int64_t>(n1, 1) * 4) && alloc((void **)&m->t2, B * std::max<int64_t>(n2, 1) * 4) &&
          alloc((void **)&m->t3, B * std::max<int64_t>(n3, 1) * 4) && alloc((void **)&m->t4, std::max<int64_t>({B * n4, n4_one, 1}) * 4) &&
          alloc((void **)&m->kvx, std::max<int64_t>(nkv, 1) * 4) && alloc((void **)&m->xn, desc->max_batch * W * 4) && alloc((void **)&m->logits, desc->max_batch * (int64_t)desc->vocab * 4) &&
@@ -501,13 +490,15 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
         if (m->lstm_aux_n) ok = ok && alloc((void **)&m->lstm_aux, (size_t)m->lstm_aux_n * 2 * 4);
     }
     { // the wide mat-mul's operand copy: the widest input of any matrix x a portion's rows (mixture of experts: slots), or the window's rows x the latent, which are many however few the tokens
-        int64_t kmax = std::max<int64_t>(W, desc->side_dim), kvrows = 0, kvk = 0;
+        int64_t kmax = std::max<int64_t>(W, desc->side_dim), kslot = moe_slots ? W : 0, kvrows = 0, kvk = 0; // (a mixture's own products have a row per slot, its shared expert's one per token)
         mixers([&](LayerPlan &P) {
+            const bool moe = P.d.ff_kind == PS_FF_MOE_SWIGLU || P.d.ff_kind == PS_FF_MOE_RELU2;
             if (P.d.kind == PS_MIX_WKV) kmax = std::max<int64_t>(kmax, 4 * W); // (four mixes side by side)
-            kmax = std::max<int64_t>({kmax, P.d.ff, P.d.shared_ff, P.d.heads * (int64_t)std::max(P.d.dim, P.d.vdim), P.d.q_rank, P.d.decay_rank});
+            kmax = std::max<int64_t>({kmax, moe ? 0 : P.d.ff, P.d.shared_ff, P.d.heads * (int64_t)std::max(P.d.dim, P.d.vdim), P.d.q_rank, P.d.decay_rank});
+            if (moe) kslot = std::max<int64_t>(kslot, P.d.ff);
             if (P.d.kind == PS_MIX_LATENT) { kvrows = std::max<int64_t>(kvrows, P.d.window - 1 + B); kvk = std::max<int64_t>(kvk, P.d.kv_rank); }
         });
-        m->pack_bytes = (size_t)std::max(std::max(B, moe_slots) * kmax, kvrows * kvk) * (desc->compute == 0 ? 2 : 6); // (fp32: three bf16 lines)
+        m->pack_bytes = (size_t)std::max({B * kmax, moe_slots * kslot, kvrows * kvk}) * (desc->compute == 0 ? 2 : 6); // (fp32: three bf16 lines)
         ok = ok && alloc(&m->pack, m->pack_bytes);
         if (std::max({B, moe_slots, kvrows}) > 8) {
             m->split_bytes = psk_dense_split_bytes();
@@ -593,17 +584,19 @@ int ps_hip_seq_set_mode(ps_hip_seq *m, int mode) { m->mode = mode; return 0; }
 
 } // extern "C"
 
-// The launches of one portion: T <= m->rows tokens (device ids in m->tokens, or the step's own token0 when from_step) of the slot whose state
+// The launches of one portion: T <= m->rows tokens (device ids in m->tokens; from_step: the step's own token0, whose embedding is there) of the slot whose state
 // pointer is `state`.  any_pos: a captured sequence that must hold for any position -- whatever depends on the position (the rows of a window's
 // expansion, the visible blocks) is launched for its most and cut on the device; otherwise the step's position is known on the host (pos0).
-static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool any_pos, bool from_step) {
+// rows: how many the head is asked for.  Returns whether the last boundary has made the final norm as well (m->xn: a single token that is asked for once); otherwise the stream is in m->x.
+static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool any_pos, bool from_step, int rows) {
     hipStream_t st = m->ctx->stream;
+    float *x = m->x; // the residual stream (a single token's may stand in m->x2 for some layers)
     const ps_seq_desc &D = m->d;
     const int64_t W = D.width;
     const bool tiled = (m->mode & 2) != 0, chunked = T >= CHUNKED_FROM && !tiled && m->ssd_scratch; // a portion's recurrences
     const int64_t BW = m->rows * W, DW = (int64_t)D.max_batch * W; // (results of a run: in `hist`, in the debugging buffer)
-    psk_embed(st, D.embed, from_step ? nullptr : m->tokens, m->step, T, m->embed_scale, m->hist ? m->hist : m->x, W, D.bigram, D.bigram_buckets, D.bigram_mul_prev,
-              D.bigram_mul_cur);
+    if (!from_step)
+        psk_embed(st, D.embed, m->tokens, m->step, T, m->embed_scale, m->hist ? m->hist : x, W, D.bigram, D.bigram_buckets, D.bigram_mul_prev, D.bigram_mul_cur);
     // The kernels in front of a portion's products leave a bf16 copy of what they wrote in m->a16 as well: `rounded` says of which buffer, and is forgotten with its contents.
     uint16_t *copy16 = T > 8 && !tiled ? m->a16 : nullptr;
     const float *rounded = nullptr;
@@ -615,14 +608,18 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         return g;
     };
     // a sublayer boundary: x += norm_b(y) (after a sublayer), then hn = norm(x), h = conv(hn) (in front of the next one); one launch for a single token
-    auto boundary = [&](const float *y, const float *wb, const float *wn, const float *cw, int64_t tail_off) {
+    bool final_made = false;
+    const bool plain_final = T == 1 && rows == 1 && !tiled && m->groups == 1 && !m->hist && !D.norm_center && !D.final_norm_bias;
+    auto boundary = [&](const float *y, const float *wb, const float *wn, const float *cw, int64_t tail_off, const bool last = false) {
         if (T == 1 && !tiled && m->groups == 1) {
-            psk_boundary1(st, m->step, m->x, y, wb, wn, cw, D.canon_taps, tail_off, D.norm_offset, D.norm_eps, W, m->h, m->hn);
+            final_made = last && !wn && plain_final;
+            if (final_made) psk_boundary1(st, m->step, x, y, wb, D.final_norm, nullptr, 0, 0, D.norm_offset, D.norm_eps, W, nullptr, m->xn);
+            else if (psk_boundary1(st, m->step, x, y, wb, wn, cw, D.canon_taps, tail_off, D.norm_offset, D.norm_eps, W, m->h, m->hn, x == m->x ? m->x2 : m->x)) x = x == m->x ? m->x2 : m->x;
             return;
         }
-        if (y) rounded = psk_norm_residual(st, m->x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn, wn ? nullptr : copy16) ? m->x : nullptr;
+        if (y) rounded = psk_norm_residual(st, x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn, wn ? nullptr : copy16) ? x : nullptr;
         if (wn) {
-            if (!y) psk_rmsnorm(st, m->x, W, nullptr, wn, D.norm_offset, D.norm_eps, W, T, m->hn, W, m->groups);
+            if (!y) psk_rmsnorm(st, x, W, nullptr, wn, D.norm_offset, D.norm_eps, W, T, m->hn, W, m->groups);
             rounded = psk_causal_conv(st, m->step, tail_off, m->hn, W, cw, D.canon_taps, 0, W, T, m->h, W, nullptr, copy16) ? m->h : nullptr;
         }
     };
@@ -634,17 +631,40 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         g.H = l.heads; g.own = l.dim; g.pos0 = pos0; g.T = T; g.window = l.window; g.scale = l.scale; g.o = m->t3; g.ldo = (int64_t)l.heads * l.vdim; g.scratch = m->sa_scratch;
         psk_split_attn(st, g);
     };
+    // what the next layer's first product, which reads x, does to it in front of that (post-norm layers, a single token): x is then where that launch leaves it
+    psk_dense_pre pending;
+    auto first_product = [&](psk_dense_args g) {
+        if (pending.kind && g.a == x) {
+            g.pre = pending;
+            x = pending.xout;
+            pending = psk_dense_pre();
+        }
+        psk_dense(st, g);
+    };
     // One mixer on the input `in`.  Its output projection writes out_scale times its result to `store` (NULL: m->y), or (into given) adds it there.
     auto mixer = [&](const LayerPlan &P, const float *in, float *into, float out_scale, float *store = nullptr) {
         const ps_seq_layer &l = P.d;
         const int64_t H = l.heads, d = l.dim, dv = l.vdim;
         float *t1 = m->t1 + P.in_off;                       // this mixer's columns of the (possibly joint) input projection
         const int64_t ld1 = P.in_ld ? P.in_ld : P.ncat;
-        auto out_proj = [&](const float *a, int64_t lda) {
+        auto out_proj = [&](const float *a, int64_t lda, const psk_dense_pre *pre = nullptr) {
             auto g = mm(l.out, a, lda, into ? into : store ? store : m->y, W);
             g.alpha = out_scale; g.accum = into ? 1 : 0; g.bias = l.out_bias;
+            if (pre) {
+                g.pre = *pre;
+                if (!psk_dense_takes_pre(g)) return false;
+            }
             psk_dense(st, g);
             if (rounded == a) rounded = nullptr; // (the next mixer overwrites it)
+            return true;
+        };
+        // the output projection of o [H][n] behind its heads' norms and a gate: in one launch for a single token of few numbers
+        auto normed_out = [&](float *o, int64_t n, const float *gate, int64_t ldg, const float *w, int w_stride) {
+            psk_dense_pre r;
+            r.kind = psk_dense_pre::HEADS; r.gate = gate; r.w = w; r.w_stride = w_stride; r.part = (int)n; r.eps = D.norm_eps;
+            if (T == 1 && out_proj(o, H * n, &r)) return;
+            rounded = psk_headnorm_gate(st, o, H * n, gate, ldg, w, w_stride, D.norm_eps, (int)H, (int)n, T, copy16) ? o : nullptr;
+            out_proj(o, H * n);
         };
         if (l.kind == PS_MIX_WKV) {
             const int64_t Hd = H * d, NW = 5 * Hd;
@@ -666,11 +686,10 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             psk_state_store(st, m->step, P.off_shift, in + (int64_t)(T - 1) * W, W);
             if (chunked && psk_chunked_ok((int)d)) psk_wkv_chunked(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->ssd_scratch, m->t3, Hd);
             else psk_wkv_scan(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->t3, Hd);
-            rounded = psk_headnorm_gate(st, m->t3, Hd, m->t1 + 3 * Hd, NW, l.onorm, (int)d, D.norm_eps, (int)H, (int)d, T, copy16) ? m->t3 : nullptr;
-            out_proj(m->t3, Hd);
+            normed_out(m->t3, d, m->t1 + 3 * Hd, NW, l.onorm, (int)d);
         } else if (l.kind == PS_MIX_DELTA) {
             const int64_t KHd = (int64_t)l.kv_heads * d, Hv = H * dv;
-            if (!P.in_ld) psk_dense(st, mm(l.in_cat, in, W, t1, ld1));
+            if (!P.in_ld) first_product(mm(l.in_cat, in, W, t1, ld1));
             psk_causal_conv(st, m->step, P.off_conv, t1, ld1, l.conv, l.conv_taps, 1, P.cqkv, T, m->t2, P.cqkv);
             if (chunked && psk_chunked_ok((int)d))
                 psk_delta_chunked(st, m->step, P.off_S, m->t2, m->t2 + KHd, m->t2 + 2 * KHd, t1 + P.cqkv + Hv, t1 + P.cqkv + Hv + H, P.cqkv, ld1, l.a_log, l.dt_bias, (int)H, l.kv_heads, (int)d,
@@ -678,26 +697,24 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             else
                 psk_delta_scan(st, m->step, P.off_S, m->t2, m->t2 + KHd, m->t2 + 2 * KHd, t1 + P.cqkv + Hv, t1 + P.cqkv + Hv + H, P.cqkv, ld1, l.a_log, l.dt_bias,
                                (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, Hv);
-            rounded = psk_headnorm_gate(st, m->t3, Hv, t1 + P.cqkv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T, copy16) ? m->t3 : nullptr;
-            out_proj(m->t3, Hv);
+            normed_out(m->t3, dv, t1 + P.cqkv, ld1, l.onorm, 0);
         } else if (l.kind == PS_MIX_GLA) {
             // t1 = [ q | k | v | g | a1 ]; the decay's second matrix (with its bias) -> t2; scan -> t3; per-head norm and gate; out
             const int64_t Hd = H * d, Hv = H * dv;
-            if (!P.in_ld) psk_dense(st, mm(l.in_cat, in, W, t1, ld1));
+            if (!P.in_ld) first_product(mm(l.in_cat, in, W, t1, ld1));
             auto g2 = mm(l.decay2, t1 + 2 * Hd + 2 * Hv, ld1, m->t2, Hd);
             g2.bias = l.decay0;
             psk_dense(st, g2);
             if (chunked && psk_chunked_ok((int)d)) psk_gla_chunked(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->ssd_scratch, m->t3, Hv);
             else psk_gla_scan(st, m->step, P.off_S, t1, t1 + Hd, t1 + 2 * Hd, ld1, m->t2, Hd, l.tau, (int)H, (int)d, (int)dv, T, m->t3, Hv);
-            rounded = psk_headnorm_gate(st, m->t3, Hv, t1 + 2 * Hd + Hv, ld1, l.onorm, 0, D.norm_eps, (int)H, (int)dv, T, copy16) ? m->t3 : nullptr;
-            out_proj(m->t3, Hv);
+            normed_out(m->t3, dv, t1 + 2 * Hd + Hv, ld1, l.onorm, 0);
         } else if (l.kind == PS_MIX_WINATTN) {
             // t1 = [ q | k | v | gate ] (+ bias); norms, rotation, ring append and block means; attention -> t3; out
             const int64_t G = l.kv_heads, Hd = H * d, Hv = H * dv;
             if (!P.in_ld) {
                 auto g = mm(l.in_cat, in, W, t1, ld1);
                 g.bias = l.in_bias;
-                psk_dense(st, g);
+                first_product(g);
             }
             const bool reads = P.owner >= 0; // (another layer's keys and values: queries only)
             psk_winattn_prep(st, m->step, P.off_ring, P.cap, psk_front_store{P.off_pool, l.pool, reads ? 0 : P.keep_rows}, t1, ld1, l.qnorm, l.knorm, D.norm_eps, (int)H,
@@ -730,7 +747,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         } else if (l.kind == PS_MIX_SSD) {
             // t1 = [ z | x | B | C | dt ]; x, B and C through the convolution -> t2; scan -> t3; gate and norm; out
             const int64_t inner = H * dv, GN = (int64_t)l.kv_heads * d;
-            if (!P.in_ld) psk_dense(st, mm(l.in_cat, in, W, t1, ld1));
+            if (!P.in_ld) first_product(mm(l.in_cat, in, W, t1, ld1));
             psk_causal_conv(st, m->step, P.off_conv, t1 + inner, ld1, l.conv, l.conv_taps, 1, P.cqkv, T, m->t2, P.cqkv, l.conv_bias);
             const float *x = m->t2, *Bv = x + inner, *Cv = Bv + GN, *dt = t1 + inner + P.cqkv;
             if (chunked && psk_ssd_chunked_ok((int)d, (int)dv))
@@ -745,7 +762,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             if (!P.in_ld) {
                 auto g = mm(l.in_cat, in, W, t1, ld1);
                 g.bias = l.in_bias;
-                psk_dense(st, g);
+                first_product(g);
             }
             const float *k = t1 + Hd, *v = k + Hd, *g = v + Hv, *iz = g + Hv, *fz = iz + H;
             float *nq = m->lstm_aux, *mt = nq + m->lstm_aux_n;
@@ -760,7 +777,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             if (!P.in_ld) {
                 auto g = mm(l.in_cat, in, W, t1, ld1);
                 g.bias = l.in_bias;
-                psk_dense(st, g);
+                first_product(g);
             }
             psk_mingru_scan(st, m->step, P.off_S, t1, ld1, d, T, m->t3, d);
             out_proj(m->t3, d);
@@ -771,7 +788,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             float *cq = m->t2, *q = direct ? m->t1 : m->t2 + m->rows * m->n_t2q;
             const int64_t ldq = direct ? P.ncat : nq;
             const float *gate = l.gated ? m->t1 + P.ncat - H : nullptr;
-            psk_dense(st, mm(l.in_cat, in, W, m->t1, P.ncat));
+            first_product(mm(l.in_cat, in, W, m->t1, P.ncat));
             psk_latent_prep(st, m->step, P.off_ring, P.cap, direct ? m->t1 + nq : m->t1, P.ncat, l.qnorm, l.kvnorm, D.norm_eps, l.q_rank, l.kv_rank, (int)dr, l.rot_dims, P.freq, T,
                             cq, l.q_rank, P.rot_mag, l.rot_pairing);
             if (!direct) psk_dense(st, mm(l.uq, cq, l.q_rank, q, nq));
@@ -808,7 +825,7 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         if (!P.joint) return;
         auto g = mm(P.joint, in, W, m->t1, P.in_ld);
         g.bias = P.joint_bias;
-        psk_dense(st, g);
+        first_product(g);
     };
     // the first product of a dense feed-forward; returns the bf16 rows that the second one is to read (NULL: m->t4 as it is).  512 tokens of 8192: 33 MB less through memory.
     auto ff_up = [&](const LayerPlan &P, const float *in) -> const void * {
@@ -901,58 +918,65 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         if (l.form == PS_LAYER_PRENORM || (l.form == PS_LAYER_PARALLEL && !l.canon1)) rounded = nullptr; // (their fronts write h and x themselves)
         if (l.form == PS_LAYER_PRENORM) {
             // x += mixer(norm1(x)), then x += ff(norm2(x)): each sublayer's front is one launch, its output projection adds straight into the residual stream
-            psk_front(st, m->x, 0, 1, nullptr, nullptr, nullptr, l.norm1, m->h, nullptr, nullptr, m->groups, D.norm_offset, D.norm_eps, W, T, D.norm_center);
+            psk_front(st, x, 0, 1, nullptr, nullptr, nullptr, l.norm1, m->h, nullptr, nullptr, m->groups, D.norm_offset, D.norm_eps, W, T, D.norm_center);
             joint_in(P, m->h);
-            mixer(P, m->h, m->x, l.mix_scale);
-            if (P.side) mixer(*P.side, m->h, m->x, P.side->d.mix_scale);
+            mixer(P, m->h, x, l.mix_scale);
+            if (P.side) mixer(*P.side, m->h, x, P.side->d.mix_scale);
             if (l.ff_kind != PS_FF_NONE) {
-                psk_front(st, m->x, 0, 1, nullptr, nullptr, nullptr, l.norm2, m->h, nullptr, nullptr, m->groups, D.norm_offset, D.norm_eps, W, T, D.norm_center);
-                feed_forward(P, m->h, m->x, 1.f);
+                psk_front(st, x, 0, 1, nullptr, nullptr, nullptr, l.norm2, m->h, nullptr, nullptr, m->groups, D.norm_offset, D.norm_eps, W, T, D.norm_center);
+                feed_forward(P, m->h, x, 1.f);
             }
         } else if (l.form == PS_LAYER_POSTNORM) {
             // x += norm_b(mixer(x)), then x += norm_b(ff(x)): a sublayer's first product reads the residual stream, its last one writes y
-            auto post = [&](const float *w, const float *b) {
+            auto post = [&](const float *w, const float *b, const bool last = false) {
                 rounded = nullptr;
-                if (D.norm_center || b) psk_postnorm(st, m->x, m->y, nullptr, 0.f, nullptr, nullptr, 0.f, w, b, D.norm_offset, D.norm_center, D.norm_eps, W, T);
-                else boundary(m->y, w, nullptr, nullptr, 0);
+                if (D.norm_center || b) psk_postnorm(st, x, m->y, nullptr, 0.f, nullptr, nullptr, 0.f, w, b, D.norm_offset, D.norm_center, D.norm_eps, W, T);
+                else boundary(m->y, w, nullptr, nullptr, 0, last);
             };
             // a token's boundary in front of a mixture of experts goes along with the routing
-            const psk_moe_front front = {m->x, m->y, l.norm1b, D.norm_offset, D.norm_eps};
+            psk_moe_front front = {x, m->y, l.norm1b, D.norm_offset, D.norm_eps};
             const bool along = T == 1 && !tiled && m->groups == 1 && !l.mix_onorm && !D.norm_center && !l.norm1b_bias && (l.ff_kind == PS_FF_MOE_SWIGLU || l.ff_kind == PS_FF_MOE_RELU2) &&
                                psk_moe_front_ok(front, l.router, l.shared_gate, l.experts + (int)l.moe_identity, W);
-            joint_in(P, m->x);
+            joint_in(P, x);
             if (l.mix_onorm) { // the mixers' outputs side by side (y and h), normed one by one, summed, normed and added in one launch
-                mixer(P, m->x, nullptr, 1.f);
-                if (P.side) mixer(*P.side, m->x, nullptr, 1.f, m->h);
+                mixer(P, x, nullptr, 1.f);
+                if (P.side) mixer(*P.side, x, nullptr, 1.f, m->h);
                 rounded = nullptr;
-                psk_postnorm(st, m->x, m->y, l.mix_onorm, l.mix_scale, P.side ? m->h : nullptr, P.side ? P.side->d.mix_onorm : nullptr, P.side ? P.side->d.mix_scale : 0.f, l.norm1b,
+                psk_postnorm(st, x, m->y, l.mix_onorm, l.mix_scale, P.side ? m->h : nullptr, P.side ? P.side->d.mix_onorm : nullptr, P.side ? P.side->d.mix_scale : 0.f, l.norm1b,
                              l.norm1b_bias, D.norm_offset, D.norm_center, D.norm_eps, W, T);
             } else {
-                mixer(P, m->x, nullptr, l.mix_scale);
-                if (P.side) mixer(*P.side, m->x, m->y, P.side->d.mix_scale);
-                if (!along) post(l.norm1b, l.norm1b_bias);
+                mixer(P, x, nullptr, l.mix_scale);
+                if (P.side) mixer(*P.side, x, m->y, P.side->d.mix_scale);
+                front.x = x;
+                if (!along) post(l.norm1b, l.norm1b_bias, !next && l.ff_kind == PS_FF_NONE && !l.side_gate);
             }
             if (l.ff_kind != PS_FF_NONE) {
-                feed_forward(P, m->x, m->y, 1.f, true, along ? &front : nullptr);
-                post(l.norm2b, l.norm2b_bias);
+                feed_forward(P, x, m->y, 1.f, true, along ? &front : nullptr);
+                // (a token's boundary in front of a layer whose first product can take it along: in that launch)
+                psk_dense_pre r;
+                r.kind = psk_dense_pre::BOUNDARY; r.w = l.norm2b; r.y = m->y; r.eps = D.norm_eps; r.offset = D.norm_offset; r.xout = x == m->x ? m->x2 : m->x;
+                auto g = next ? mm(next->joint ? next->joint : next->d.in_cat, x, W, m->t1, 0) : psk_dense_args();
+                g.pre = r;
+                if (T == 1 && !tiled && m->groups == 1 && !D.norm_center && !l.norm2b_bias && !l.side_gate && !m->dbg_layers && next && next->d.form == PS_LAYER_POSTNORM && psk_dense_takes_pre(g)) pending = r;
+                else post(l.norm2b, l.norm2b_bias, !next && !l.side_gate);
             }
             if (l.side_gate) { // the token's own input to this layer: (gelu(gate x) * its stretch of the table row) in one product, the projection, norm and add
-                auto g = mm(l.side_gate, m->x, W, m->t4, D.side_dim);
+                auto g = mm(l.side_gate, x, W, m->t4, D.side_dim);
                 g.act = PSD_ACT_GELU_TANH;
                 g.em_table = D.side_embed; g.em_col = (int64_t)P.layer * D.side_dim; g.em_tokens = from_step ? nullptr : m->tokens; g.em_step = m->step;
                 psk_dense(st, g);
                 psk_dense(st, mm(l.side_proj, m->t4, D.side_dim, m->y, W));
                 rounded = nullptr;
-                if (T == 1 && !tiled) psk_boundary1(st, m->step, m->x, m->y, l.side_norm, nullptr, nullptr, 1, 0, 0.f, D.norm_eps, W, nullptr, nullptr);
-                else psk_norm_residual(st, m->x, m->y, l.side_norm, 0.f, D.norm_eps, W, T);
+                if (T == 1 && !tiled) psk_boundary1(st, m->step, x, m->y, l.side_norm, nullptr, nullptr, 1, 0, 0.f, D.norm_eps, W, nullptr, nullptr);
+                else psk_norm_residual(st, x, m->y, l.side_norm, 0.f, D.norm_eps, W, T);
             }
         } else if (l.form == PS_LAYER_PARALLEL && !l.canon1) {
             // No input filter: one launch makes the layer's input (with depth_mix: the previous layer's average over X_0 .. X_li, kept as this layer's X to add
             // into) and both sublayers' norms; mixers and feed-forward add their output projections, times res, straight into the layer's X
-            float *xr = m->hist ? m->hist + (int64_t)(li + 1) * BW : m->x;
+            float *xr = m->hist ? m->hist + (int64_t)(li + 1) * BW : x;
             float *h2 = l.norm2 ? m->hn : nullptr;
             if (m->hist) psk_front(st, m->hist, BW, li + 1, li ? m->L[li - 1].d.depth_mix : nullptr, nullptr, xr, l.norm1, m->h, l.norm2, h2, m->groups, D.norm_offset, D.norm_eps, W, T);
-            else psk_front(st, m->x, 0, 1, nullptr, nullptr, nullptr, l.norm1, m->h, l.norm2, h2, m->groups, D.norm_offset, D.norm_eps, W, T);
+            else psk_front(st, x, 0, 1, nullptr, nullptr, nullptr, l.norm1, m->h, l.norm2, h2, m->groups, D.norm_offset, D.norm_eps, W, T);
             joint_in(P, m->h);
             mixer(P, m->h, xr, res * l.mix_scale);
             if (P.side) mixer(*P.side, m->h, xr, res * P.side->d.mix_scale);
@@ -963,9 +987,9 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             // hn = norm(x), h = conv(hn); both mixers and the feed-forward add their output projections straight into the residual stream
             boundary(nullptr, nullptr, l.norm1, l.canon1, P.off_canon1);
             joint_in(P, m->h);
-            mixer(P, m->h, m->x, res * l.mix_scale);
-            if (P.side) mixer(*P.side, m->h, m->x, res * P.side->d.mix_scale);
-            if (l.ff_kind != PS_FF_NONE) feed_forward(P, m->hn, m->x, res);
+            mixer(P, m->h, x, res * l.mix_scale);
+            if (P.side) mixer(*P.side, m->h, x, res * P.side->d.mix_scale);
+            if (l.ff_kind != PS_FF_NONE) feed_forward(P, m->hn, x, res);
         } else {
             const bool summed = P.side != nullptr || l.mix_scale != 1.f;
             if (summed) psk_fill(st, m->y, 0.f, (int64_t)T * W);
@@ -981,20 +1005,23 @@ static void seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 auto g = mm(l.ff_down, m->t4, l.ff, m->y, W);
                 g.a16 = a16;
                 psk_dense(st, g);
-                boundary(m->y, l.norm2b, nn, nc, no);
+                boundary(m->y, l.norm2b, nn, nc, no, !next);
             } else {
-                boundary(m->y, l.norm1b, nn, nc, no);
+                boundary(m->y, l.norm1b, nn, nc, no, !next);
             }
         }
-        if (m->dbg_layers && !any_pos && !m->hist) psk_copy(st, m->x, m->dbg_layers + (int64_t)li * DW, (int64_t)T * W);
+        if (m->dbg_layers && !any_pos && !m->hist) psk_copy(st, x, m->dbg_layers + (int64_t)li * DW, (int64_t)T * W);
     }
+    if (x != m->x && !final_made && rows) psk_copy(st, x, m->x, W);
+    return final_made;
 }
 
 // final norm on `rows` rows of x (idx: device indices, or NULL for rows 0 ..), logits, arg-max
-static void seq_head(ps_hip_seq *m, const int32_t *idx, int rows) {
+static void seq_head(ps_hip_seq *m, const int32_t *idx, int rows, bool normed, bool argmax = true) { // normed: m->xn is made (one row)
     hipStream_t st = m->ctx->stream;
     const ps_seq_desc &D = m->d;
-    if (m->hist) { // what the last layer hands on (its depth average, or its own result) and the final norm in one launch
+    if (normed) {
+    } else if (m->hist) { // what the last layer hands on (its depth average, or its own result) and the final norm in one launch
         const int runs = (int)m->L.size();
         psk_front(st, m->hist, m->rows * D.width, runs + 1, m->L[runs - 1].d.depth_mix, idx, nullptr, D.final_norm, m->xn, nullptr, nullptr, m->groups,
                   D.norm_offset, D.norm_eps, D.width, rows, 0, D.final_norm_bias);
@@ -1007,7 +1034,7 @@ static void seq_head(ps_hip_seq *m, const int32_t *idx, int rows) {
     g.w = D.head; g.a = m->xn; g.lda = D.width; g.T = rows; g.out = m->logits; g.ldo = D.vocab; g.alpha = D.logit_scale; g.force_tiled = (m->mode & 2) != 0; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
     if (D.logit_softcap > 0.f) { g.act = PSD_ACT_SOFTCAP; g.act_p = D.logit_softcap; }
     psk_dense(st, g);
-    psk_argmax_rows(st, m->logits, D.vocab, rows, m->amax);
+    if (argmax) psk_argmax_rows(st, m->logits, D.vocab, rows, m->amax);
 }
 
 extern "C" {
@@ -1047,9 +1074,9 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
     int wi = 0, half = 0;
     std::vector<int32_t> idx;
     // the logits of the wanted rows idx (at most max_batch of them, the caller's w0 and on): they are in m->want
-    auto results = [&](const int w0) -> int {
+    auto results = [&](const int w0, const bool normed) -> int {
         const int rows = (int)idx.size();
-        seq_head(m, m->want, rows);
+        seq_head(m, m->want, rows, normed);
         if (row && rows * row <= PS_PIN_HALF && ps_pin_ready(c)) {
             PS_CHECK(c, take(half)); // (those before the last ones: long there)
             const size_t lb = logits_host ? (size_t)rows * m->d.vocab * 4 : 0;
@@ -1082,11 +1109,11 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
             PS_CHECK(c, ps_put(c->stream, in, 2));
             hipLaunchKernelGGL(seq_set_step_kernel, dim3(1), dim3(1), 0, c->stream, m->step, (long long)pos0, T, slot, m->slot_state[slot], (int)tokens[t0], (int)tokens[t0 + T - 1],
                                m->prev_of(slot));
-            seq_layers(m, m->slot_state[slot], T, pos0, false, false);
+            const bool normed = seq_layers(m, m->slot_state[slot], T, pos0, false, false, (int)idx.size());
             PS_CHECK(c, hipGetLastError());
             m->slot_pos[slot] = pos0 + T; // (the slot's recurrent states move with these launches, whatever becomes of the results)
             while (!idx.empty()) {
-                if (const int rc = results(w0)) return rc;
+                if (const int rc = results(w0, normed)) return rc;
                 w0 = wanted();
                 if (idx.empty()) break;
                 const ps_piece more = {m->want, idx.data(), idx.size() * 4};
@@ -1122,10 +1149,11 @@ int ps_hip_seq_decode_greedy(ps_hip_seq *m, int slot, int32_t token, int steps, 
     }
     float *state = m->slot_state[slot];
     hipLaunchKernelGGL(seq_set_step_kernel, dim3(1), dim3(1), 0, c->stream, m->step, (long long)m->slot_pos[slot], 1, slot, state, (int)token, (int)token, m->prev_of(slot));
-    auto one = [&]() {
-        seq_layers(m, state, 1, 0, true, true);
-        seq_head(m, nullptr, 1);
-        hipLaunchKernelGGL(seq_advance_kernel, dim3(1), dim3(1), 0, c->stream, m->step, m->amax, m->ids, m->prev_of(slot));
+    psk_embed(c->stream, m->d.embed, nullptr, m->step, 1, m->embed_scale, m->hist ? m->hist : m->x, m->d.width, m->d.bigram, m->d.bigram_buckets, m->d.bigram_mul_prev, m->d.bigram_mul_cur);
+    auto one = [&]() { // (the token's embedding is there: the step before has made it)
+        seq_head(m, nullptr, 1, seq_layers(m, state, 1, 0, true, true, 1), false);
+        psk_next_token(c->stream, m->logits, m->d.vocab, m->step, m->ids, m->prev_of(slot), m->d.embed, m->embed_scale, m->hist ? m->hist : m->x, m->d.bigram, m->d.bigram_buckets,
+                       m->d.bigram_mul_prev, m->d.bigram_mul_cur);
     };
     if (m->mode & 1) {
         for (int i = 0; i < steps; i++) one();

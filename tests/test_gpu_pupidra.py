@@ -203,6 +203,37 @@ def test_boundary_and_routing_of_a_token(made, width, experts, top, shared):
     assert err(run_portions(m, toks, (1,)), seq_oracle.run_pupidra(cfg, t, toks)) < TOL["float32"]
 
 
+# a token's boundary inside the next layer's first product (k_dense.hip dn_stage_pre), the stream then in one of two buffers: an even and an odd number of them, one run of a thread, several, the
+# most, widths that are no whole units (a launch of its own), a layer without experts behind it; captured steps, which begin and end in the same buffer
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,layers", [(256, 2), (512, 3), (2560, 4), (8192, 2), (520, 3)])
+def test_boundary_in_front_of_the_next_layers_product(made, width, layers, dtype):
+    kinds = [("attention", UA(2, 1, 16, 8, 0.3, 9, 2)), ("mamba2", UM(4, 16, 16, 2, 3, 2)), ("latent_attention", ULA(2, 16, 16, 16, 32, 0.2, 100.0)), ("attention", UA(2, 1, 16, 8, 0.3, 9, 0, 0))]
+    cfg = UC(width, 40, [UL(k, mc, (4, 2, 16, 1.5) if i != 1 or layers == 2 else None, 8 if i % 2 else None) for i, (k, mc) in enumerate(kinds[:layers])])
+    m, cfg, t = made(f"defer{width}", dtype, cfg=cfg)
+    toks = tokens_for(cfg, 20)
+    want = seq_oracle.run_pupidra(cfg, t, toks)
+    assert close(run_portions(m, toks, (1,)), want, dtype)
+    s = m.acquire()
+    for i in range(0, 18, 3):
+        m.forward(s, toks[i:i + 1])
+        assert np.array_equal(*m.forward(s, toks[i + 1:i + 2], [0, 0]))
+        m.forward(s, toks[i + 2:i + 3], [0])
+    m.forward(s, toks[18:19])
+    a = m.forward(s, toks[19:20], [0])
+    m.release(s)
+    assert close(a, want[19:], dtype)
+    ids = []
+    for mode in (0, 1):
+        m.set_mode(mode)
+        s = m.acquire()
+        m.forward(s, toks[:9])
+        ids.append(list(m.decode_greedy(s, int(toks[9]), 5)) + list(m.decode_greedy(s, int(toks[10]), 6)))
+        m.release(s)
+    m.set_mode(0)
+    assert ids[0] == ids[1]
+
+
 @pytest.mark.parametrize("name", ["odd", "aligned", "wide"])
 def test_the_residual_stream_after_every_layer(made, name):
     m, cfg, t = made(name, "float32", max_batch=64)

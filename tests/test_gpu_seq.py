@@ -144,6 +144,25 @@ def test_kernels_of_a_single_token(made, width, taps, heads, rank, rot, window):
     assert err(run_portions(m, toks, (1,)), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
+# heads' norms and gates inside a token's output projection (k_dense.hip dn_stage_pre): heads of four numbers, of a wave's 256, one run of 2048 and less than one; sizes it does not take (no whole
+# units, heads of 48 numbers); steps of one token that are asked for nothing, once and twice
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,dim,vdim", [(128, 4, 4), (2, 256, 256), (16, 128, 128), (1, 64, 512), (4, 16, 64), (16, 16, 48), (12, 32, 128)])
+def test_norms_in_front_of_a_tokens_output_projection(made, heads, dim, vdim, dtype):
+    layers = [L("delta", 24, heads=heads, kv_heads=1, dim=dim, vdim=vdim, conv=2)] + ([L("wkv", None, heads=heads, dim=dim)] if dim == vdim else [])
+    cfg = synth.seq_config(64, 40, layers[:1] if dtype == "bfloat16" else layers, taps=4)
+    m, c, t = made(f"pre{heads}.{dim}.{vdim}", dtype, cfg=cfg)
+    toks = tokens_for(c, 24)
+    want = seq_oracle.run(c, t, toks)
+    assert err(run_portions(m, toks, (1,)), want) < TOL[dtype]
+    s = m.acquire()
+    for i in range(0, 24, 3):
+        m.forward(s, toks[i:i + 1])
+        assert err(m.forward(s, toks[i + 1:i + 2], [0, 0]), want[[i + 1, i + 1]]) < TOL[dtype]
+        m.forward(s, toks[i + 2:i + 3], [0])
+    m.release(s)
+
+
 # a single token behind a window of very many keys (k_latent.hip latent_combine_kernel): as many tiles as it keeps the weights of, one more, and more than LDS has room for
 @pytest.mark.parametrize("window", [262_128, 262_129, 652_000])
 def test_latent_attention_of_a_very_long_window(ctx, tmp_path, window):
