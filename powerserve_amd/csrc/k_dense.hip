@@ -1210,13 +1210,15 @@ __global__ __launch_bounds__(64 * NW) void dense_mm_narrow_kernel(dn_args g) {
 // of 2048 rows gives each of 2048 waves one), or in neighbouring pairs for a paired activation.  What bounded dense_mv_kernel here was the number of bytes in flight: four rows per wave,
 // two pieces each, 128 work-groups of four waves for 2048 rows.  Measured, bf16, before and now: 2048 x 4096 (16.8 MB) 14.6 and 6.6 us, 8192 x 2048 (33 MB) 15 and 9, 14336 x 4096
 // (117 MB) 29 to 38 and 22 us (5.3 TB/s).  The first product of a token's experts (top 2 of 3072 x 2048 and a shared one of twice that, 50 MB), which was two launches, 12.4 + 10.4 and 12.0 us.
-//  Sixteen units in flight, and the activations requested ahead of the weights, were tried and are slower (the registers cost a work-group per CU).
+//  Four units in flight: a token of Ranutar 4096 x 3, 2048 x 6, Pupidra 2048 x 6, 4096 x 3 in us with two units 349 351 378 405, three 334 340 376 395, four 322 343 376 387, five 331 348 378 392,
+//  six 339 352 386 399, eight (as it was) 326 356 390 389, sixteen 326 353 390 397; 768 and 1024 work-groups instead of 512: the same or up to 5 % more; ordinary loads instead of
+//  non-temporal ones: 357 383 412 420.  (mv2's in flight: one row per wave, three units of it, 376 against 381 with two rows and 382 with its eight.)
 //   FORM 0  one matrix
 //   FORM 1  grouped, the first product of an expert: work-groups in equal runs per slot (its own matrix and output row), behind them those of the shared expert (g2)
 //   FORM 2  several matrices of one shape, each over its own mix of the token and the one before it (psk_dense_args::more): work-groups in equal runs per matrix.  Four of 4096 x 4096,
 //           33 MB each: 10.7 us one by one, 23.7 together (5.7 TB/s)
 // dynamic LDS: the activations as bf16-rounded fp32 (fp32 mode: as they are), every vector padded with zeros to whole units
-#define DN_AHEAD 8
+#define DN_AHEAD 4
 struct dn_mv1 {
     dn_args g2;  // FORM 1: the shared expert's first product (w NULL: none)
     int slots;   // FORM 1: slots of the launch
@@ -1524,7 +1526,7 @@ static bool dn_launch_mv1(hipStream_t st, const dn_args &g, const dn_args *g2, i
 
 // The second product of a token's experts: an output row is the sum over the token's slots (and the shared expert) of the products with their matrices, so a row runs through all of
 // them.  `waves` waves of a work-group share a row, each with the same up to U units of it, so that a wave's part of the activations (up to top + 1 vectors of different experts) stays in
-// its registers and nothing waits for a copy of all of them in LDS; eight units and more per wave are in flight, across row ends.  The waves' sums of a row meet in LDS at the end.
+// its registers and nothing waits for a copy of all of them in LDS; a row of each wave is in flight (two units at least), across row ends.  The waves' sums of a row meet in LDS at the end.
 // blockIdx.y = token.  Top 2 of 2048 x 3072 and a shared one of twice that (50 MB), one token: 16.6 us and 17.5 us more for the shared expert before, 18.0 as one stream with the activations in LDS
 // (as above), 14.3 then; 13.9 since the weights are requested in front of what is done to the activations.  The form above is the better one where there is a single vector: 2048 x 4096 6.6 us there, 9 with this kernel's arrangement.
 // dynamic LDS: [8][rows] sums
@@ -1538,7 +1540,7 @@ struct dn_mv2 {
 template <typename WT, int U, bool RAGGED> // RAGGED: a row ends inside a unit
 __global__ __launch_bounds__(512, U > 8 ? 2 : 4) void dense_mv2_kernel(dn_args g, dn_mv2 p) {
     extern __shared__ __attribute__((aligned(16))) float sums[];
-    constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE, AHEAD = U >= 8 ? 1 : 8 / U; // elements per lane and per unit; rows in flight
+    constexpr int VE = 16 / (int)sizeof(WT), UNIT = 64 * VE, AHEAD = U >= 3 ? 1 : 4 / U; // elements per lane and per unit; rows in flight
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), y = blockIdx.y;
     const int sel = lane < p.slots ? g.g_sel[(long long)y * p.slots + lane] : 0; // lane c: slot c's matrix
     const int N = (int)g.N, K = (int)g.K, K2 = (int)p.g2.K;
@@ -1678,6 +1680,7 @@ static bool dn_launch_mv2(hipStream_t st, const dn_args &g, const dn_args *g2, i
         constexpr bool R = decltype(ragged)::value;
         if (p.share == 1) go(dense_mv2_kernel<WT, 1, R>);
         else if (p.share == 2) go(dense_mv2_kernel<WT, 2, R>);
+        else if (p.share == 3) go(dense_mv2_kernel<WT, 3, R>);
         else if (p.share <= 4) go(dense_mv2_kernel<WT, 4, R>);
         else if (p.share <= 8) go(dense_mv2_kernel<WT, 8, R>);
         else if constexpr (sizeof(WT) == 4) go(dense_mv2_kernel<WT, 16, R>);
