@@ -2,14 +2,14 @@
 // fp32 throughout on v_mfma_f32_16x16x4_f32 (one rounding per product, fp32 adds: a true fp32 product, no reduced-precision mode), or on the bf16 instruction with the operand as three bf16 lines
 // and the weights as they came (dn_ring_take, PL 3: no product is rounded at all).
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
-//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than 8 tokens: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
+//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than one token: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
 //   dense_mm_big_kernel   the same operands, bf16, 256 x 256 tiles where they fill the chip in fewer rounds
 //   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
-//   dense_mm_narrow_kernel bf16, K a multiple of 128 up to 1024, more than 8 tokens, few tiles: 32 x 32 tiles, the waves share K
+//   dense_mm_narrow_kernel bf16, K a multiple of 128 up to 1024, more than one token, few tiles: 32 x 32 tiles, the waves share K
 //   dense_mv1_kernel<WT,FORM,RAGGED> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
 //   dense_mv2_kernel<WT,U,RAGGED> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
-//   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns): the activation rows live in LDS, a wave streams RW weight rows at a time
+//   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns) of a K the ring does not take: the activation rows live in LDS, a wave streams RW weight rows at a time
 // All take the same operand description (ps_seq.h psk_dense_args): ring rows, the token-shift mix and the epilogue
 // (bias, activation, scale, a factor from a second table) are part of the launch, so no mixer needs a kernel of its own around its projections.
 #include "ps_seq.h"
@@ -1739,7 +1739,7 @@ bool psk_dense_takes_pre(const psk_dense_args &a) {
     return r.kind == psk_dense_pre::BOUNDARY && aligned(r.y) && aligned(r.xout) && r.xout != a.a;
 }
 bool psk_dense_wide16(const psk_dense_args &a) {
-    return a.w && a.w->dtype == PS_BF16 && a.T > 8 && !a.force_tiled && a.pack && a.groups == 0 && !a.mu && !a.a_mod && !a.a_step && !a.a_row0 && a.w->K > 256 && a.w->K % 64 == 0 &&
+    return a.w && a.w->dtype == PS_BF16 && a.T > PSD_FEW && !a.force_tiled && a.pack && a.groups == 0 && !a.mu && !a.a_mod && !a.a_step && !a.a_row0 && a.w->K > 256 && a.w->K % 64 == 0 &&
            (size_t)a.T * a.w->K * 2 <= a.pack_bytes;
 }
 int psk_dense(hipStream_t st, const psk_dense_args &a) {
@@ -1750,7 +1750,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         bool alike = true;
         for (int i = 0; i < a.n_more; i++) alike = alike && a.more[i]->dtype == a.w->dtype && a.more[i]->N == a.w->N && a.more[i]->K == a.w->K;
         if (alike && !a.force_tiled && a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 2>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 2>(st, g, nullptr, 0, &a))) return 0;
-        if (alike && a.T > 8 && dn_wide(st, a, g)) return 0;
+        if (alike && a.T > PSD_FEW && dn_wide(st, a, g)) return 0;
         for (int i = 0; i <= a.n_more; i++) {
             psk_dense_args one = a;
             one.n_more = 0;
@@ -1782,6 +1782,33 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
         return 0;
     }
+    if (!a.force_tiled && a.T > 8 && g.K <= 32 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0) {
+        const dim3 grid((unsigned)((g.N + 255) / 256), (unsigned)((a.T + 15) / 16));
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g); };
+        if (g.K <= 8) bf ? go(dense_mm_few_kernel<unsigned short, 8>) : go(dense_mm_few_kernel<float, 8>);
+        else bf ? go(dense_mm_few_kernel<unsigned short, 32>) : go(dense_mm_few_kernel<float, 32>);
+        return 0;
+    }
+    // K up to 256, and up to 1024 where the small tiles are not more than one per CU and nobody hands rounded rows on (the ring packs its operand first): us here and there, weights from memory,
+    // 2048 x 512: 9 tokens 5.4 and 8.0, 128 tokens 6.7 and 9.0; 1024 x 1024: 9 tokens 7.0 and 9.8, 256 tokens 9.1 and 11.2; 3072 x 1024: 64 tokens (192 tiles) 9.3 and 12.0, 128 tokens
+    // (384) 17.1 and 12.0; 2048 x 2048: 16 tokens 13.4 and 13.1, 64 tokens 15.8 and 13.4.
+    if (bf && !a.force_tiled && a.T > PSD_FEW && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 &&
+        (g.K <= 256 || (g.K <= 1024 && (int64_t)((a.T + 31) / 32) * ((g.N + 31) / 32) <= 256 && !a.a16 && !a.out16))) {
+        const dim3 grid((unsigned)((a.T + 31) / 32), (unsigned)((g.N + 31) / 32));
+        auto go = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, st, g); };
+        switch (g.K / 128) {
+        case 1: go(dense_mm_narrow_kernel<4, 1>, 4); break;
+        case 2: go(dense_mm_narrow_kernel<4, 2>, 4); break;
+        case 3: go(dense_mm_narrow_kernel<4, 3>, 4); break;
+        case 4: go(dense_mm_narrow_kernel<4, 4>, 4); break;
+        case 5: go(dense_mm_narrow_kernel<4, 5>, 4); break;
+        case 6: go(dense_mm_narrow_kernel<4, 6>, 4); break;
+        case 7: go(dense_mm_narrow_kernel<4, 7>, 4); break;
+        default: go(dense_mm_narrow_kernel<8, 4>, 8);
+        }
+        return 0;
+    }
+    if (a.T > PSD_FEW && dn_wide(st, a, g)) return 0;
     if (!a.force_tiled && a.T <= 8) {
         if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 0>(st, g, nullptr, 0, &a))) return 0;
         const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
@@ -1805,33 +1832,6 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
             return 0;
         }
     }
-    if (!a.force_tiled && a.T > 8 && g.K <= 32 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0) {
-        const dim3 grid((unsigned)((g.N + 255) / 256), (unsigned)((a.T + 15) / 16));
-        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g); };
-        if (g.K <= 8) bf ? go(dense_mm_few_kernel<unsigned short, 8>) : go(dense_mm_few_kernel<float, 8>);
-        else bf ? go(dense_mm_few_kernel<unsigned short, 32>) : go(dense_mm_few_kernel<float, 32>);
-        return 0;
-    }
-    // K up to 256, and up to 1024 where the small tiles are not more than one per CU and nobody hands rounded rows on (the ring packs its operand first): us here and there, weights from memory,
-    // 2048 x 512: 9 tokens 5.4 and 8.0, 128 tokens 6.7 and 9.0; 1024 x 1024: 9 tokens 7.0 and 9.8, 256 tokens 9.1 and 11.2; 3072 x 1024: 64 tokens (192 tiles) 9.3 and 12.0, 128 tokens
-    // (384) 17.1 and 12.0; 2048 x 2048: 16 tokens 13.4 and 13.1, 64 tokens 15.8 and 13.4.
-    if (bf && !a.force_tiled && a.T > 8 && g.K % 128 == 0 && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0 &&
-        (g.K <= 256 || (g.K <= 1024 && (int64_t)((a.T + 31) / 32) * ((g.N + 31) / 32) <= 256 && !a.a16 && !a.out16))) {
-        const dim3 grid((unsigned)((a.T + 31) / 32), (unsigned)((g.N + 31) / 32));
-        auto go = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, st, g); };
-        switch (g.K / 128) {
-        case 1: go(dense_mm_narrow_kernel<4, 1>, 4); break;
-        case 2: go(dense_mm_narrow_kernel<4, 2>, 4); break;
-        case 3: go(dense_mm_narrow_kernel<4, 3>, 4); break;
-        case 4: go(dense_mm_narrow_kernel<4, 4>, 4); break;
-        case 5: go(dense_mm_narrow_kernel<4, 5>, 4); break;
-        case 6: go(dense_mm_narrow_kernel<4, 6>, 4); break;
-        case 7: go(dense_mm_narrow_kernel<4, 7>, 4); break;
-        default: go(dense_mm_narrow_kernel<8, 4>, 8);
-        }
-        return 0;
-    }
-    if (a.T > 8 && dn_wide(st, a, g)) return 0;
     dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((a.T + 63) / 64));
     if (bf) hipLaunchKernelGGL(dense_mm_kernel<unsigned short>, grid, dim3(256), 0, st, g);
     else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
@@ -1992,7 +1992,7 @@ int ps_hip_dense_matmul(ps_hip_ctx *c, const ps_dense *w, const float *x, int T,
     // by piece, and where the device has no room for it the product does without.  Products that the wide mat-mul does not take need none.
     const bool lines = w->half && w->K % 64 == 0; // (fp32 on the bf16 instruction)
     const int64_t row = w->K * (w->dtype == PS_BF16 ? 2 : lines ? 6 : 4);
-    const bool wide = T > 8 && row % 128 == 0, packs = w->dtype == PS_BF16 || lines || ((uintptr_t)x & 15) != 0;
+    const bool wide = T > PSD_FEW && row % 128 == 0, packs = w->dtype == PS_BF16 || lines || ((uintptr_t)x & 15) != 0;
     const int64_t piece = wide && packs ? std::min<int64_t>(T, std::max<int64_t>(((int64_t)64 << 20) / row / 128 * 128, 128)) : T;
     const size_t pack = packs ? (size_t)(piece * row + 255) / 256 * 256 : 0, need = pack + psk_dense_split_bytes();
     if (wide && c->act_cap < need) {

@@ -500,11 +500,11 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
         });
         m->pack_bytes = (size_t)std::max({B * kmax, moe_slots * kslot, kvrows * kvk}) * (desc->compute == 0 ? 2 : 6); // (fp32: three bf16 lines)
         ok = ok && alloc(&m->pack, m->pack_bytes);
-        if (std::max({B, moe_slots, kvrows}) > 8) {
+        if (std::max({B, moe_slots, kvrows}) > PSD_FEW) {
             m->split_bytes = psk_dense_split_bytes();
             ok = ok && alloc((void **)&m->split, m->split_bytes);
         }
-        if (desc->compute == 0 && B > 8) {
+        if (desc->compute == 0 && B > PSD_FEW) {
             int64_t wide = W;
             mixers([&](LayerPlan &P) { wide = std::max<int64_t>(wide, (int64_t)P.d.heads * std::max(P.d.dim, P.d.vdim)); });
             ok = ok && alloc((void **)&m->a16, (size_t)B * wide * 2);
@@ -598,7 +598,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     if (!from_step)
         psk_embed(st, D.embed, m->tokens, m->step, T, m->embed_scale, m->hist ? m->hist : x, W, D.bigram, D.bigram_buckets, D.bigram_mul_prev, D.bigram_mul_cur);
     // The kernels in front of a portion's products leave a bf16 copy of what they wrote in m->a16 as well: `rounded` says of which buffer, and is forgotten with its contents.
-    uint16_t *copy16 = T > 8 && !tiled ? m->a16 : nullptr;
+    uint16_t *copy16 = T > PSD_FEW && !tiled ? m->a16 : nullptr;
     const float *rounded = nullptr;
     auto mm = [&](const ps_dense *w, const float *a, int64_t lda, float *out, int64_t ldo) {
         psk_dense_args g;
@@ -841,7 +841,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     };
     // The feed-forward of a layer on `in`, added to xr times alpha (store: written there instead).  Mixture of experts: slot s = t top + i is token t's i-th choice; the router's
     // score scales what the expert READS (the A operand of its first product) or, moe_weight_output, what it puts out (the rows of its inner activation: the second
-    // product is linear); a few tokens run grouped mat-vecs, a portion tiles over the slots sorted by expert.  A choice beyond the experts that have matrices is an
+    // product is linear); a few tokens (psk_few_slots) run grouped mat-vecs, a portion tiles over the slots sorted by expert.  A choice beyond the experts that have matrices is an
     // identity expert: no product touches its slot, and its weight times the input joins the sum.
     auto feed_forward = [&](const LayerPlan &P, const float *in, float *xr, float alpha, bool store = false, const psk_moe_front *front = nullptr) {
         const ps_seq_layer &l = P.d;
@@ -859,7 +859,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         const int act = l.ff_kind == PS_FF_MOE_RELU2 ? PSD_ACT_RELU2 : PSD_ACT_SILU_PAIR;
         psk_moe_route(st, in, W, l.router, l.shared_gate, rows, top, l.moe_norm_top, W, T, m->moe_sel, m->moe_wgt, m->moe_sg, l.moe_softmax, l.moe_correction, l.moe_groups,
                       l.moe_keep, l.moe_scale != 0.f ? l.moe_scale : 1.f, l.router_bias, front);
-        const bool mv = !tiled && T <= 8 && (size_t)std::max<int64_t>(W, (int64_t)top * l.ff) * 4 + 64 <= 128 * 1024;
+        const bool mv = !tiled && psk_few_slots(T, top, E, W % 64 == 0 && l.ff % 64 == 0) && (size_t)std::max<int64_t>(W, (int64_t)top * l.ff) * 4 + 64 <= 128 * 1024;
         if (!mv) psk_moe_plan(st, m->moe_sel, S, rows, m->moe_seg, m->moe_list);
         auto grouped = [&](psk_dense_args &g) {
             g.groups = E; g.g_sel = m->moe_sel;
@@ -1208,7 +1208,7 @@ int ps_hip_seq_bench_kernel(ps_hip_seq *m, int which, int T, int reps, double *u
         if (moe) {
             // the routing of this layer (all layers' launches below then reuse the LAST layer's routing: the same shapes and spread)
             const int top = P.d.top, S = T * top;
-            const bool mv = T <= 8;
+            const bool mv = psk_few_slots(T, top, P.d.experts, W % 64 == 0 && P.d.ff % 64 == 0);
             const int rows = P.d.experts + P.d.moe_identity;
             std::vector<int32_t> sel((size_t)S);
             // (a few tokens: the first run of tokens none of whose choices is an identity expert, so that a mat-vec launch has its full work)

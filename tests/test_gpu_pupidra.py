@@ -203,6 +203,16 @@ def test_boundary_and_routing_of_a_token(made, width, experts, top, shared):
     assert err(run_portions(m, toks, (1,)), seq_oracle.run_pupidra(cfg, t, toks)) < TOL["float32"]
 
 
+# a mixture's products on either side of where the wide mat-mul takes them (ps_seq.h psk_few_slots: 2 of 8 experts, from 6 tokens; 2 of 3, from 3), whole blocks of K and not
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("experts,ff", [(8, 64), (8, 72), (3, 64)])
+def test_experts_of_a_few_tokens(made, dtype, experts, ff):
+    cfg = UC(128, 40, [UL("attention", UA(2, 1, 16, 8, 0.3, 9, 2), (experts, 2, ff, 1.7), 64)])
+    m, cfg, t = made(f"few-slots{experts}.{ff}", dtype, cfg=cfg)
+    toks = tokens_for(cfg, 35)
+    assert close(run_portions(m, toks, (2, 3, 4, 5, 6, 7, 8)), seq_oracle.run_pupidra(cfg, t, toks), dtype)
+
+
 # a token's boundary inside the next layer's first product (k_dense.hip dn_stage_pre), the stream then in one of two buffers: an even and an odd number of them, one run of a thread, several, the
 # most, widths that are no whole units (a launch of its own), a layer without experts behind it; captured steps, which begin and end in the same buffer
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

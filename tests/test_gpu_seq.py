@@ -370,6 +370,13 @@ def test_dense_matmul_of_few_tiles(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
 
 
+# two to eight tokens on the wide mat-mul (ps_seq.h PSD_FEW): the narrow tiles, the ring with and without a split along K, and the mat-vec where K is no whole 128 bytes (the same bound)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,N,K", [(2, 1, 64), (3, 33, 128), (4, 129, 1024), (5, 70, 4160), (8, 2100, 192), (7, 65, 2048), (2, 300, 72), (8, 40, 1056)])
+def test_dense_matmul_of_a_few_tokens(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
 # one token (k_dense.hip dense_mv1_kernel): a row of less than one unit of its stream (512 numbers, fp32: 256), of exactly one, of one and a bit; fewer and more units per wave than are in flight;
 # one row, rows that are no multiple of the waves', more rows than waves and more than 64 of them per wave; the longest row that is taken, and one more, which the general kernel does
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
