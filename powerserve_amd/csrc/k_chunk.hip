@@ -9,14 +9,16 @@
 //                       o_t = (q_t exp(c_t)) S + sum_(s <= t) B_ts u_s,  B_ts = exp(c_t - c_s) (q_t . k_s);   S <- exp(c_end) S + sum_s (k_s exp(c_end - c_s)) u_s^T
 // Everything that does not depend on the state -- the scaled q, k rows, the 16 x 16 matrices (M by forward substitution in double) -- is made for all chunks at once by the two
 // prep kernels; chunk_scan_kernel walks the chunks with the state in the matrix instructions' accumulators.  Measured, 512 tokens of 16 heads of 128 x 128: wkv 303 -> 19 + 32 us,
-// delta rule 391 -> 13 + 45 us.
+// delta rule 391 -> 13 + 45 us (token by token and in chunks, the first form of the scan); 2047 tokens, the scan alone, that form and now, under the profiler: wkv 148 -> 70 us, delta rule 222 -> 115.
 #include "ps_attn_dev.h"
 #include "ps_seq.h"
 
 #include <cmath>
+#include <type_traits>
 
 typedef float ck_f4 __attribute__((ext_vector_type(4)));
 #define CK_Q 16
+#define CK_AHEAD 2 // chunks (3 and 4 are no faster)
 
 // A token's log decay, from below: e^-128 is zero in fp32 as every decay below it is (the scans' exp(-1e30) or exp(-inf)), but beside a -1e13 in the running sum the decays behind it would
 // be lost, and -inf - -inf is no number.  (A NaN stays one.)
@@ -179,106 +181,193 @@ __global__ __launch_bounds__(256) void chunk_delta_prep_kernel(const float *q, c
     }
 }
 
-// block (16 value columns, head), wave w keeps the state's row tiles w, w + 4, ... (16 rows each, NT of them) in accumulators: lane (column l % 16, quarter l / 16) holds rows
+// block (16 value columns, head), wave w of the first four keeps the state's row tiles w, w + 4, ... (16 rows each, NT of them) in accumulators: lane (column l % 16, quarter l / 16) holds rows
 // 4 (l / 16) + i, which is also what the next product's column operand asks of it when k is taken in that order -- the state never leaves its registers.  A wave's part of the
-// products with the state meets the others' in LDS (two buffers, one barrier per chunk); a chunk's operands are requested two chunks ahead.
-template <int NT, bool DELTA>
-__global__ __launch_bounds__(256) void chunk_scan_kernel(const ps_seq_step *step, long long state_off, const float *scratch, const float *v, long long ld, int d, int dv, int T, float *o,
+// products with the state meets the others' in LDS (two buffers, one barrier per chunk); the fifth wave adds them, makes the chunk's outputs and stores them, beside the others' next chunk.
+// What bounds it is the chain of a chunk, 16 matrix instructions per state wave (NT 2; delta rule 28, those with q where the wave would wait for the others): 0.55 and 0.9 us a chunk, in proportion to
+// them, with eight state waves of half the tiles too (0.54 and 1.06: each makes u).  A chunk's operands are requested CK_AHEAD chunks ahead, at addresses that are a scalar and a constant per
+// lane; FULL (d = 64 NT, whole column blocks): no branch between the requests, so a wait counts them and none drains the queue, as each did before.
+template <int NT, bool DELTA, bool FULL>
+__global__ __launch_bounds__(320) void chunk_scan_kernel(const ps_seq_step *step, long long state_off, const float *scratch, const float *v, long long ld, int d, int dv, int T, float *o,
                                                          long long ldo) {
     __shared__ ck_f4 part[2][DELTA ? 2 : 1][4][64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lq = lane >> 4, h = blockIdx.y, H = gridDim.y, tiles = d / 16, chunks = (T + CK_Q - 1) / CK_Q;
-    const int col = blockIdx.x * 16 + lr, colc = min(col, dv - 1);
-    const ck_layout at{d};
-    float *S0 = step->state + state_off + (long long)h * d * dv;
-    const float *vh = v + (long long)h * dv + colc;
-    ck_f4 S[NT];
-#pragma unroll
-    for (int x = 0; x < NT; x++) {
-        const int tile = wave + 4 * x;
-#pragma unroll
-        for (int i = 0; i < 4; i++) S[x][i] = tile < tiles && col < dv ? S0[(long long)(16 * tile + 4 * lq + i) * dv + col] : 0.f;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lq = lane >> 4, H = gridDim.y, tiles = FULL ? 4 * NT : d / 16;
+    const int chunks = (T + CK_Q - 1) / CK_Q, last = chunks - 1;
+    int h = blockIdx.y, block = blockIdx.x;
+    if (H % 8 == 0) { // a head's column blocks, which read the same operands, on one XCD (work-groups go to the eight in turn)
+        const int id = blockIdx.x + gridDim.x * blockIdx.y;
+        h = id % 8 + 8 * (id / 8 / (int)gridDim.x);
+        block = id / 8 % (int)gridDim.x;
     }
+    const int col = block * 16 + lr, colc = FULL ? col : min(col, dv - 1);
+    const ck_layout at{d};
+    const char *ph = (const char *)(scratch + (long long)h * at.size()), *vh = (const char *)(v + (long long)h * dv);
+    const long long per = (long long)H * at.size() * 4;
     struct operands { ck_f4 q[NT], k[DELTA ? NT : 1], kt[NT], dec[DELTA ? 1 : NT], in, m; float v[4]; };
-    auto fetch = [&](int c, operands &a) {
-        const float *p = scratch + ((long long)min(c, chunks - 1) * H + h) * at.size();
+    unsigned at_v[4], at_end[4]; // bytes from a chunk's first row to the lane's four, in a whole chunk and in the last one (rows that are not there repeat the last one: nothing is made of them)
 #pragma unroll
-        for (int x = 0; x < NT; x++) {
-            const int row = 16 * min(wave + 4 * x, tiles - 1); // (a tile that is not there repeats the last one; its rows of the state are zero and not stored)
-            a.q[x] = *(const ck_f4 *)(p + at.rows1() + lr * d + row + 4 * lq);
-            if constexpr (DELTA) a.k[x] = *(const ck_f4 *)(p + at.rows2() + lr * d + row + 4 * lq);
-            a.kt[x] = *(const ck_f4 *)(p + at.keys() + (row + lr) * CK_Q + 4 * lq);
-            if constexpr (!DELTA) a.dec[x] = *(const ck_f4 *)(p + at.decay() + row + 4 * lq);
+    for (int i = 0; i < 4; i++) {
+        at_v[i] = (unsigned)(((long long)(4 * lq + i) * ld + colc) * 4);
+        at_end[i] = (unsigned)(((long long)min(4 * lq + i, T - 1 - last * CK_Q) * ld + colc) * 4);
+    }
+    auto fetch_v = [&](int c, operands &a) { // (c: at most the last)
+        const char *p = vh + (long long)c * CK_Q * ld * 4;
+#pragma unroll
+        for (int i = 0; i < 4; i++) a.v[i] = *(const float *)(p + (c < last ? at_v[i] : at_end[i]));
+    };
+    const unsigned at_m = (unsigned)(at.solve() + lr * CK_Q + 4 * lq) * 4, at_in = (unsigned)(at.intra() + lr * CK_Q + 4 * lq) * 4;
+    if (wave == 4) {
+        auto fetch = [&](int c, operands &a) {
+            c = min(c, last);
+            const char *p = ph + c * per;
+            if constexpr (DELTA) a.m = *(const ck_f4 *)(p + at_m);
+            a.in = *(const ck_f4 *)(p + at_in);
+            fetch_v(c, a);
+        };
+        ck_f4 held_in, held_u; // the delta rule's products with q are there one barrier later
+        auto finish = [&](auto whole, int c, const ck_f4 &in, const ck_f4 &u) {
+            const int buf = c & 1;
+            ck_f4 y = (part[buf][0][0][lane] + part[buf][0][1][lane]) + (part[buf][0][2][lane] + part[buf][0][3][lane]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(in[i], u[i], y, 0, 0, 0);
+            float *oh = o + (long long)(c * CK_Q + 4 * lq) * ldo + (long long)h * dv + col;
+            if constexpr (whole.value) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) oh[i * ldo] = y[i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (c * CK_Q + 4 * lq + i < T && col < dv) oh[i * ldo] = y[i];
+            }
+        };
+        auto chunk = [&](auto whole, int c, const operands &b, operands &later) {
+            fetch(c + CK_AHEAD, later);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            ck_f4 u = {b.v[0], b.v[1], b.v[2], b.v[3]};
+            if constexpr (DELTA) {
+                const int buf = c & 1;
+                const ck_f4 w = (part[buf][1][0][lane] + part[buf][1][1][lane]) + (part[buf][1][2][lane] + part[buf][1][3][lane]);
+                u = ck_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < 4; i++) u = __builtin_amdgcn_mfma_f32_16x16x4f32(b.m[i], b.v[i] - w[i], u, 0, 0, 0);
+                if (c) finish(std::integral_constant<bool, FULL>(), c - 1, held_in, held_u); // (not the last chunk: all its rows are there)
+                held_in = b.in;
+                held_u = u;
+            } else finish(whole, c, b.in, u);
+        };
+        operands a[CK_AHEAD + 1];
+#pragma unroll
+        for (int i = 0; i < CK_AHEAD; i++) fetch(i, a[i]);
+        int c = 0;
+        for (; FULL && c + CK_AHEAD < T / CK_Q; c += CK_AHEAD + 1) {
+#pragma unroll
+            for (int i = 0; i <= CK_AHEAD; i++) chunk(std::true_type(), c + i, a[i], a[(i + CK_AHEAD) % (CK_AHEAD + 1)]);
+        }
+        for (; c < chunks; c += CK_AHEAD + 1) {
+#pragma unroll
+            for (int i = 0; i <= CK_AHEAD; i++)
+                if (c + i < chunks) chunk(std::false_type(), c + i, a[i], a[(i + CK_AHEAD) % (CK_AHEAD + 1)]); // (uniform)
         }
         if constexpr (DELTA) {
-            const float g = p[at.decay()];
-            a.dec[0] = ck_f4{g, g, g, g};
-            a.m = *(const ck_f4 *)(p + at.solve() + lr * CK_Q + 4 * lq);
+            __syncthreads();
+            finish(std::false_type(), last, held_in, held_u);
         }
-        a.in = *(const ck_f4 *)(p + at.intra() + lr * CK_Q + 4 * lq);
+        return;
+    }
+    float *S0 = step->state + state_off + (long long)h * d * dv;
+    ck_f4 S[NT];
+    unsigned at_q[NT], at_kt[NT], at_dec[NT]; // (a tile that is not there repeats the last one; its rows of the state are zero and not stored)
 #pragma unroll
-        for (int i = 0; i < 4; i++) a.v[i] = vh[(long long)min(c * CK_Q + 4 * lq + i, T - 1) * ld];
+    for (int x = 0; x < NT; x++) {
+        const int tile = wave + 4 * x, row = 16 * min(tile, tiles - 1);
+        at_q[x] = (unsigned)(lr * d + row + 4 * lq) * 4;
+        at_kt[x] = (unsigned)(at.keys() + (row + lr) * CK_Q + 4 * lq) * 4;
+        at_dec[x] = (unsigned)(at.decay() + row + 4 * lq) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; i++) S[x][i] = FULL || (tile < tiles && col < dv) ? S0[(long long)(16 * tile + 4 * lq + i) * dv + col] : 0.f;
+    }
+    auto fetch = [&](int c, operands &a) {
+        c = min(c, last);
+        const char *p = ph + c * per;
+#pragma unroll
+        for (int x = 0; x < NT; x++) {
+            if constexpr (DELTA) a.k[x] = *(const ck_f4 *)(p + at.rows2() * 4 + at_q[x]);
+            a.q[x] = *(const ck_f4 *)(p + at.rows1() * 4 + at_q[x]);
+            a.kt[x] = *(const ck_f4 *)(p + at_kt[x]);
+            if constexpr (!DELTA) a.dec[x] = *(const ck_f4 *)(p + at_dec[x]);
+        }
+        if constexpr (DELTA) {
+            const float g = *(const float *)(p + at.decay() * 4);
+            a.dec[0] = ck_f4{g, g, g, g};
+            a.m = *(const ck_f4 *)(p + at_m);
+        }
+        fetch_v(c, a);
     };
-    auto chunk = [&](int c, const operands &b, operands &later) { // later: whose operands are those of chunk c + 2
-        if (c >= chunks) return; // (uniform)
-        fetch(c + 2, later);
+    auto chunk = [&](int c, const operands &b, operands &later) {
         const int buf = c & 1;
         ck_f4 oq = {0.f, 0.f, 0.f, 0.f}, ok = {0.f, 0.f, 0.f, 0.f};
+        auto with_q = [&](int from, int to) {
 #pragma unroll
-        for (int x = 0; x < NT; x++)
-            if (wave + 4 * x < tiles) { // (uniform per wave)
+            for (int x = from; x < to; x++)
+                if (FULL || wave + 4 * x < tiles) { // (uniform per wave)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    if constexpr (DELTA) ok = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[x][i], S[x][i], ok, 0, 0, 0);
-                    oq = __builtin_amdgcn_mfma_f32_16x16x4f32(b.q[x][i], S[x][i], oq, 0, 0, 0);
-                }
-            }
-        part[buf][0][wave][lane] = oq;
-        if constexpr (DELTA) part[buf][1][wave][lane] = ok;
-        ck_f4 u; // what the chunk's tokens write
-        auto update = [&]() {
-#pragma unroll
-            for (int x = 0; x < NT; x++)
-                if (wave + 4 * x < tiles) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) S[x][i] *= b.dec[DELTA ? 0 : x][i];
-#pragma unroll
-                    for (int i = 0; i < 4; i++) S[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.kt[x][i], u[i], S[x], 0, 0, 0);
+                    for (int i = 0; i < 4; i++) oq = __builtin_amdgcn_mfma_f32_16x16x4f32(b.q[x][i], S[x][i], oq, 0, 0, 0);
                 }
         };
-        if constexpr (!DELTA) {
-            u = ck_f4{b.v[0], b.v[1], b.v[2], b.v[3]};
-            update();
+        fetch(c + CK_AHEAD, later);
+        ck_f4 u = {b.v[0], b.v[1], b.v[2], b.v[3]}; // what the chunk's tokens write
+        if constexpr (DELTA) {
+#pragma unroll
+            for (int x = 0; x < NT; x++)
+                if (FULL || wave + 4 * x < tiles) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ok = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[x][i], S[x][i], ok, 0, 0, 0);
+                }
+            part[buf][1][wave][lane] = ok;
+            __builtin_amdgcn_sched_barrier(0);
+            with_q(0, NT / 2); // (the products with q where the others' parts are waited for)
             __syncthreads();
-        } else {
-            __syncthreads();
-            const ck_f4 w = (part[buf][1][0][lane] + part[buf][1][1][lane]) + (part[buf][1][2][lane] + part[buf][1][3][lane]);
+            const ck_f4 p0 = part[buf][1][0][lane], p1 = part[buf][1][1][lane], p2 = part[buf][1][2][lane], p3 = part[buf][1][3][lane];
+            __builtin_amdgcn_sched_barrier(0);
+            with_q(NT / 2, NT);
+            const ck_f4 w = (p0 + p1) + (p2 + p3);
             u = ck_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < 4; i++) u = __builtin_amdgcn_mfma_f32_16x16x4f32(b.m[i], b.v[i] - w[i], u, 0, 0, 0);
-            update();
-        }
-        if (wave == (c & 3)) { // the outputs, the waves in turn
-            ck_f4 y = (part[buf][0][0][lane] + part[buf][0][1][lane]) + (part[buf][0][2][lane] + part[buf][0][3][lane]);
+        } else with_q(0, NT);
+        part[buf][0][wave][lane] = oq;
+        __builtin_amdgcn_sched_barrier(0); // (the requests have gone out here)
 #pragma unroll
-            for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(b.in[i], u[i], y, 0, 0, 0);
+        for (int x = 0; x < NT; x++)
+            if (FULL || wave + 4 * x < tiles) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int t = c * CK_Q + 4 * lq + i;
-                if (t < T && col < dv) o[(long long)t * ldo + (long long)h * dv + col] = y[i];
+                for (int i = 0; i < 4; i++) S[x][i] *= b.dec[DELTA ? 0 : x][i];
             }
-        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int x = 0; x < NT; x++)
+                if (FULL || wave + 4 * x < tiles) S[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.kt[x][i], u[i], S[x], 0, 0, 0);
+        if constexpr (!DELTA) __syncthreads();
     };
-    operands a0, a1, a2;
-    fetch(0, a0);
-    fetch(1, a1);
-    for (int c = 0; c < chunks; c += 3) {
-        chunk(c, a0, a2);
-        chunk(c + 1, a1, a0);
-        chunk(c + 2, a2, a1);
+    operands a[CK_AHEAD + 1];
+#pragma unroll
+    for (int i = 0; i < CK_AHEAD; i++) fetch(i, a[i]);
+#pragma unroll
+    for (int x = 0; x < NT; x++) asm volatile("" : "+v"(S[x])); // (there before the loop: a wait for them inside would wait for everything, each time around)
+    int c = 0;
+    for (; c + CK_AHEAD < chunks; c += CK_AHEAD + 1) {
+#pragma unroll
+        for (int i = 0; i <= CK_AHEAD; i++) chunk(c + i, a[i], a[(i + CK_AHEAD) % (CK_AHEAD + 1)]);
     }
 #pragma unroll
+    for (int i = 0; i < CK_AHEAD; i++)
+        if (c + i < chunks) chunk(c + i, a[i], a[(i + CK_AHEAD) % (CK_AHEAD + 1)]); // (uniform)
+    if constexpr (DELTA) __syncthreads();
+#pragma unroll
     for (int x = 0; x < NT; x++)
-        if (wave + 4 * x < tiles && col < dv) {
+        if (FULL || (wave + 4 * x < tiles && col < dv)) {
 #pragma unroll
             for (int i = 0; i < 4; i++) S0[(long long)(16 * (wave + 4 * x) + 4 * lq + i) * dv + col] = S[x][i];
         }
@@ -289,8 +378,10 @@ size_t psk_chunked_scratch(int H, int d, int T) { return (size_t)((T + CK_Q - 1)
 
 template <bool DELTA>
 static void ck_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *scratch, const float *v, int64_t ld, int H, int d, int dv, int T, float *o, int64_t ldo) {
-    const auto kernel = d <= 64 ? chunk_scan_kernel<1, DELTA> : d <= 128 ? chunk_scan_kernel<2, DELTA> : d <= 192 ? chunk_scan_kernel<3, DELTA> : chunk_scan_kernel<4, DELTA>;
-    hipLaunchKernelGGL(kernel, dim3((dv + 15) / 16, H), dim3(256), 0, st, step, (long long)state_off, scratch, v, (long long)ld, d, dv, T, o, (long long)ldo);
+    const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((dv + 15) / 16, H), dim3(320), 0, st, step, (long long)state_off, scratch, v, (long long)ld, d, dv, T, o, (long long)ldo); };
+    const int nt = (d + 63) / 64;
+    if (d % 64 == 0 && dv % 16 == 0) launch(nt == 1 ? chunk_scan_kernel<1, DELTA, true> : nt == 2 ? chunk_scan_kernel<2, DELTA, true> : nt == 3 ? chunk_scan_kernel<3, DELTA, true> : chunk_scan_kernel<4, DELTA, true>);
+    else launch(nt == 1 ? chunk_scan_kernel<1, DELTA, false> : nt == 2 ? chunk_scan_kernel<2, DELTA, false> : nt == 3 ? chunk_scan_kernel<3, DELTA, false> : chunk_scan_kernel<4, DELTA, false>);
 }
 template <bool GLA>
 static void ck_decay(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *r, const float *k, const float *v, int64_t ld, const float *z, int64_t ldz, const float *bonus,

@@ -91,6 +91,22 @@ def test_recurrences_in_chunks(made, sizes):
     assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
+# the same scan without branches (k_chunk.hip chunk_scan_kernel, FULL: whole tiles for each of the four waves, one to four of them; heads in eights and not): two to nine chunks, so fewer than are
+# requested ahead, one more, every number that the loop's three leave over, a last chunk of one, of fifteen and of sixteen tokens
+@pytest.mark.parametrize("sizes", [(32, 33), (48, 63, 64), (65, 80, 81), (95, 96, 112), (127, 128, 130)])
+def test_recurrences_in_whole_tiles(made, sizes):
+    cfg = synth.seq_config(64, 40, [L("wkv", None, heads=8, dim=64), L("delta", None, heads=16, kv_heads=8, dim=64, vdim=32, conv=3), L("wkv", None, heads=1, dim=128),
+                                    L("delta", None, heads=2, kv_heads=1, dim=192, vdim=16, conv=2), L("delta", None, heads=8, kv_heads=2, dim=128, vdim=48, conv=1), L("wkv", None, heads=2, dim=256),
+                                    L("delta", None, heads=1, kv_heads=1, dim=256, vdim=64, conv=2)], taps=2)
+    t = synth.seq_tensors(cfg, 5)
+    t["l0.mix.w0"], t["l2.mix.w0"] = np.linspace(-9, 3, 512, dtype=np.float32), np.linspace(3, -9, 128, dtype=np.float32)
+    t["l1.mix.A_log"] = np.linspace(-9, 3, 16, dtype=np.float32)
+    t = {n: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(np.shape(a)) for n, a in t.items()}
+    m, c, t = made("whole-tiles", max_batch=130, cfg=cfg, tensors=t)
+    toks = tokens_for(c, sum(sizes) + 40)
+    assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
+
+
 # channels and heads that forget everything at once at some tokens and next to nothing at others: a token's log decay runs from nothing over e^30 .. e^45, where a running sum of them would
 # swallow the ordinary decays behind it, to an overflow of fp32; the state that the next portion starts from is right too.  (32 tokens and more: chunks; 31 and fewer: the scan)
 @pytest.mark.parametrize("sizes", [(32,), (47, 5, 49), (31, 33)])
