@@ -17,6 +17,8 @@
 #include <type_traits>
 
 typedef float ck_f4 __attribute__((ext_vector_type(4)));
+typedef float ck_f2 __attribute__((ext_vector_type(2)));
+typedef double ck_d2 __attribute__((ext_vector_type(2)));
 #define CK_Q 16
 #define CK_AHEAD 2 // chunks (3 and 4 are no faster)
 
@@ -38,17 +40,20 @@ struct ck_layout {
     __host__ __device__ int size() const { return solve() + CK_Q * CK_Q; }
 };
 
-// block (chunk, head).  dynamic LDS: doubles [16][d + 1], floats 2 x [16][d + 1]
+// block (chunk, head).  dynamic LDS: doubles [16][d + 2], floats 2 x [16][d + 2], 2 x [16][16] (two channels a read; the sixteen rows of a wave's reads lie in banks of their own).  What bounds it is the
+// matrix A, an exponential per channel and pair of tokens and the LDS reads for it: the 120 pairs stand in 120 threads for each half of the channels (all 256 pairs in a thread each: the half
+// above the diagonal waits; 2047 tokens, 16 heads of 128: 55 us, 40 now).
 template <bool GLA>
 __global__ __launch_bounds__(256) void chunk_decay_prep_kernel(const float *r, const float *k, const float *z, long long ld, long long ldz, const float *bonus, int d, float qscale,
                                                                float inv_tau, int T, float *scratch) {
     extern __shared__ double ck_lds[];
-    const int ldr = d + 1, tid = threadIdx.x, h = blockIdx.y, H = gridDim.y, t0 = blockIdx.x * CK_Q, nt = min(CK_Q, T - t0);
+    const int ldr = d + 2, tid = threadIdx.x, h = blockIdx.y, H = gridDim.y, t0 = blockIdx.x * CK_Q, nt = min(CK_Q, T - t0);
     double *cs = ck_lds;
-    float *rs = (float *)(cs + CK_Q * ldr), *ks = rs + CK_Q * ldr;
+    float *rs = (float *)(cs + CK_Q * ldr), *ks = rs + CK_Q * ldr, *parts = ks + CK_Q * ldr;
     const ck_layout at{d};
     float *out = scratch + ((long long)blockIdx.x * H + h) * at.size();
     const long long hb = (long long)h * d;
+    parts[tid] = parts[CK_Q * CK_Q + tid] = 0.f;
     for (int i = tid; i < d; i += 256) { // running log decays (tokens that are not there: k = r = 0 and no decay)
         float zv[CK_Q];
 #pragma unroll
@@ -88,19 +93,34 @@ __global__ __launch_bounds__(256) void chunk_decay_prep_kernel(const float *r, c
         *(ck_f4 *)(out + at.keys() + i * CK_Q + t8 + 4) = ck_f4{kv[4], kv[5], kv[6], kv[7]};
     }
     __syncthreads();
-    const int t = tid >> 4, s = tid & 15;
-    float a = 0.f;
-    if (GLA ? s <= t : s < t) {
+    const int half = tid >> 7, pair = tid & 127;
+    if (pair < 120) { // tokens s < t, t (t - 1) / 2 pairs in front of a t's first
+        int t = (int)((1.f + sqrtf(1.f + 8.f * (float)pair)) * 0.5f);
+        t -= t * (t - 1) / 2 > pair;
+        t += t * (t + 1) / 2 <= pair;
+        const int s = pair - t * (t - 1) / 2;
         const double *ct = cs + (GLA ? t : t - 1) * ldr, *cp = cs + s * ldr;
         const float *rt = rs + t * ldr, *kp = ks + s * ldr;
-#pragma unroll 8
-        for (int i = 0; i < d; i++) a = fmaf(rt[i] * kp[i], la_exp((float)(ct[i] - cp[i])), a);
-    } else if (!GLA && s == t) {
-        const float *rt = rs + t * ldr, *kp = ks + s * ldr;
+        ck_f2 a = {0.f, 0.f};
+        const int to = (half + 1) * (d / 2);
 #pragma unroll 4
-        for (int i = 0; i < d; i++) a = fmaf(rt[i] * bonus[hb + i], kp[i], a);
+        for (int i = half * (d / 2); i < to; i += 2) {
+            const ck_d2 x = *(const ck_d2 *)(ct + i), y = *(const ck_d2 *)(cp + i);
+            const ck_f2 u = *(const ck_f2 *)(rt + i), w = *(const ck_f2 *)(kp + i);
+#pragma unroll
+            for (int e = 0; e < 2; e++) a[e] = fmaf(u[e] * w[e], la_exp((float)(x[e] - y[e])), a[e]);
+        }
+        parts[half * CK_Q * CK_Q + t * CK_Q + s] = a[0] + a[1];
+    } else { // the diagonal, eight tokens for each half of the threads
+        const int t = half * 8 + pair - 120;
+        const float *rt = rs + t * ldr, *kp = ks + t * ldr;
+        float a = 0.f;
+#pragma unroll 4
+        for (int i = 0; i < d; i++) a = fmaf(GLA ? rt[i] : rt[i] * bonus[hb + i], kp[i], a);
+        parts[t * CK_Q + t] = a;
     }
-    out[at.intra() + tid] = a;
+    __syncthreads();
+    out[at.intra() + tid] = parts[tid] + parts[CK_Q * CK_Q + tid];
 }
 
 // block (chunk, head).  dynamic LDS: floats 2 x [16][d + 4], 16 x 17 doubles in front
@@ -388,7 +408,7 @@ static void ck_decay(hipStream_t st, const ps_seq_step *step, int64_t state_off,
                      float qscale, float inv_tau, int H, int d, int dv, int T, float *scratch, float *o, int64_t ldo) {
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)chunk_decay_prep_kernel<GLA>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    hipLaunchKernelGGL(chunk_decay_prep_kernel<GLA>, dim3((T + CK_Q - 1) / CK_Q, H), dim3(256), (size_t)CK_Q * (d + 1) * 16, st, r, k, z, (long long)ld, (long long)ldz, bonus, d, qscale,
+    hipLaunchKernelGGL(chunk_decay_prep_kernel<GLA>, dim3((T + CK_Q - 1) / CK_Q, H), dim3(256), (size_t)CK_Q * (d + 2) * 16 + 2 * CK_Q * CK_Q * 4, st, r, k, z, (long long)ld, (long long)ldz, bonus, d, qscale,
                        inv_tau, T, scratch);
     ck_scan<false>(st, step, state_off, scratch, v, ld, H, d, dv, T, o, ldo);
 }
