@@ -324,6 +324,20 @@ def test_large_tiles_behind_an_epilogue(ctx, tmp_path, which):
     assert err(got, plain) < 0.03
 
 
+# xIELU behind a wide product (k_dense.hip dn_xielu): arguments from 2^-20 to beyond -64, where its exponent is held; rows of the first product scaled up and the second's columns down, so
+# that every scale counts alike in the result
+def test_activation_of_any_size(made):
+    cfg = synth.seq_config(64, 40, [L("wkv", 128, heads=2, dim=16)], taps=2)
+    t = synth.seq_tensors(cfg, 11)
+    scale = np.exp2(np.linspace(-20, 9, 128, dtype=np.float32))
+    t["l0.mlp.up"] = t["l0.mlp.up"] * scale[:, None]
+    t["l0.mlp.down"] = t["l0.mlp.down"] / np.maximum(scale, scale * scale)
+    t = {n: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(np.shape(a)) for n, a in t.items()}
+    m, c, t = made("xielu", max_batch=64, cfg=cfg, tensors=t)
+    toks = tokens_for(c, 100)
+    assert err(run_portions(m, toks, (64, 36)), seq_oracle.run(c, t, toks)) < TOL["float32"]
+
+
 # attention of many rows with its operands split into three bf16 numbers (k_splitattn.hip: two blocks of 128 rows of 64 heads and more): keys of 192 and 128 numbers, windows that end inside blocks of
 # 32 keys and inside a portion, with and without kept first tokens (fewer and more than a block), means of blocks, distance slopes, a reader of another layer's keys, gates, temperatures and sinks,
 # a soft cap, rotated queries of both pairings, key / value groups; a ring that has wrapped; portions of fewer rows (the fp32 instruction) in between; one row of the last block of 128
