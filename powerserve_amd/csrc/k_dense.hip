@@ -116,6 +116,7 @@ static __device__ __forceinline__ float dn_xielu(float x, float p, float q) {
     const float below = fmaf(s, y * (r * r), fmaf(t, r, fmaf(-n, 0.693147181f, t))) + (c - x);
     return fmaf(x > 0.f ? p * x : q, x > 0.f ? x : below, 0.5f * x);
 }
+static __device__ __forceinline__ float dn_relu2(const dn_args &g, float x) { return g.act == PSD_ACT_RELU2 ? (x > 0.f ? x * x : 0.f) : x; }
 static __device__ __forceinline__ float dn_silu(float x) { return x / (1.f + expf(-x)); }
 // Result acc of (token t, weight row n) goes to its place.  other: the result of row n ^ 1 (the paired activation needs both; every lane of the wave calls
 // this with both values, only the even row stores).  O16: the wide mat-mul's, whose result may go to g.out16 (the test of it for each of a few tokens' results, beside its arguments, cost the
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     // The weights are the matrix instructions' first operand, so a lane has four neighbouring outputs of a token in four registers: results that need no epilogue go straight to their
     // places.  Through LDS (two barriers, a loop of eight trips) 512 x 8192 of K = 2048 took 35.0 us with its packing, 31.2 this way, 512 x 2048 18.3 and 17.3.
     // An activation of each of the 64 results of a lane, written out, is code that every CU has to fetch once: 40.6 us against 32.6 for a loop; it goes through LDS.
-    if (g.act == PSD_ACT_NONE && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
+    if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
         if (loads) return;
 #pragma unroll
         for (int i = 0; i < MI; i++) {
@@ -776,7 +777,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
                     if (n0 + wn * NJ * 32 + j * 32 + 8 * q + 4 * fh >= g.N) continue;
                     dn_f4 v;
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * q + e] * g.alpha;
+                    for (int e = 0; e < 4; e++) v[e] = dn_relu2(g, acc[i][j][4 * q + e]) * g.alpha;
                     if (g.out16) {
                         dn_us4 r;
 #pragma unroll
@@ -984,7 +985,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #undef DN_BIG_LANDED
     }
     if (!wm) __builtin_amdgcn_s_barrier();
-    if (g.act == PSD_ACT_NONE && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
+    if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
 #pragma unroll
         for (int mh = 0; mh < 2; mh++)
 #pragma unroll
@@ -1000,7 +1001,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
                         if (n0 + c >= g.N) continue;
                         dn_f4 v;
 #pragma unroll
-                        for (int x = 0; x < 4; x++) v[x] = acc[mh][nh][i][j][x] * g.alpha;
+                        for (int x = 0; x < 4; x++) v[x] = dn_relu2(g, acc[mh][nh][i][j][x]) * g.alpha;
                         if (g.out16) {
                             dn_us4 r;
 #pragma unroll
