@@ -121,9 +121,12 @@ static __device__ __forceinline__ float dn_silu(float x) { return x / (1.f + exp
 // Result acc of (token t, weight row n) goes to its place.  other: the result of row n ^ 1 (the paired activation needs both; every lane of the wave calls
 // this with both values, only the even row stores).  O16: the wide mat-mul's, whose result may go to g.out16 (the test of it for each of a few tokens' results, beside its arguments, cost the
 // mat-vec of eight tokens 3 to 6 %)
+static __device__ __forceinline__ float dn_row_scale(const dn_args &g, long long t) { // of output row t (wide mat-mul)
+    return g.out_scale ? g.out_scale[g.g_list && g.out16 ? g.g_list[t] / g.g_odiv : t] : 1.f;
+}
 template <bool O16 = false>
 static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, long long n, float acc, float other, bool in) {
-    const float rs = in && g.out_scale ? g.out_scale[t] : 1.f;
+    const float rs = !in ? 1.f : O16 ? dn_row_scale(g, t) : g.out_scale ? g.out_scale[t] : 1.f;
     if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR) {
         if (in && !(n & 1)) {
             float *p = g.out + t * g.ldo + (n >> 1);
@@ -147,7 +150,7 @@ static __device__ __forceinline__ void dn_put(const dn_args &g, long long t, lon
 // the output row of local row t (t < T): itself, or where the sorted list sends its slot
 static __device__ __forceinline__ long long dn_orow(const dn_args &g, long long row0, int t, int T) {
     if (!g.g_list) return t;
-    return t < T ? g.g_list[row0 + t] / g.g_odiv : 0;
+    return t < T ? g.out16 ? row0 + t : g.g_list[row0 + t] / g.g_odiv : 0; // (rounded rows of slots: in the list's order, as the next product takes them)
 }
 
 // ---------------------------------------------------------------------------------------------------- tiled mat-mul
@@ -561,7 +564,7 @@ static __device__ __forceinline__ void dn_put4(const dn_args &g, long long t, lo
     float *p = g.out + t * g.ldo + n;
     dn_f4 v = dn_f4{0.f, 0.f, 0.f, 0.f};
     if (g.accum) v = *(const dn_f4 *)p;
-    const float rs = g.out_scale ? g.out_scale[t] : 1.f;
+    const float rs = dn_row_scale(g, t);
     if (g.act == PSD_ACT_XIELU && !g.bias) { // (uniform)
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[e] = dn_xielu(acc[e], g.act_p, g.act_q) * g.alpha;
@@ -763,13 +766,14 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     // The weights are the matrix instructions' first operand, so a lane has four neighbouring outputs of a token in four registers: results that need no epilogue go straight to their
     // places.  Through LDS (two barriers, a loop of eight trips) 512 x 8192 of K = 2048 took 35.0 us with its packing, 31.2 this way, 512 x 2048 18.3 and 17.3.
     // An activation of each of the 64 results of a lane, written out, is code that every CU has to fetch once: 40.6 us against 32.6 for a loop; it goes through LDS.
-    if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
+    if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
         if (loads) return;
 #pragma unroll
         for (int i = 0; i < MI; i++) {
             const int t = t0 + wm * MI * 32 + i * 32 + fr;
             if (t >= T) continue;
-            const long long at = dn_orow(g, row0, t, T) * g.ldo + n0 + wn * NJ * 32 + 4 * fh;
+            const long long to = dn_orow(g, row0, t, T), at = to * g.ldo + n0 + wn * NJ * 32 + 4 * fh;
+            const float f = g.out_scale ? g.alpha * dn_row_scale(g, to) : g.alpha;
 #pragma unroll
             for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -777,7 +781,7 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
                     if (n0 + wn * NJ * 32 + j * 32 + 8 * q + 4 * fh >= g.N) continue;
                     dn_f4 v;
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = dn_relu2(g, acc[i][j][4 * q + e]) * g.alpha;
+                    for (int e = 0; e < 4; e++) v[e] = dn_relu2(g, acc[i][j][4 * q + e]) * f;
                     if (g.out16) {
                         dn_us4 r;
 #pragma unroll
@@ -985,14 +989,15 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #undef DN_BIG_LANDED
     }
     if (!wm) __builtin_amdgcn_s_barrier();
-    if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.out_scale && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
+    if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
 #pragma unroll
         for (int mh = 0; mh < 2; mh++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int t = t0 + mh * 128 + wm * 64 + i * 16 + fr;
                 if (t >= T) continue;
-                const long long at = dn_orow(g, row0, t, T) * g.ldo + n0;
+                const long long to = dn_orow(g, row0, t, T), at = to * g.ldo + n0;
+                const float f = g.out_scale ? g.alpha * dn_row_scale(g, to) : g.alpha;
 #pragma unroll
                 for (int nh = 0; nh < 2; nh++)
 #pragma unroll
@@ -1001,7 +1006,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
                         if (n0 + c >= g.N) continue;
                         dn_f4 v;
 #pragma unroll
-                        for (int x = 0; x < 4; x++) v[x] = dn_relu2(g, acc[mh][nh][i][j][x]) * g.alpha;
+                        for (int x = 0; x < 4; x++) v[x] = dn_relu2(g, acc[mh][nh][i][j][x]) * f;
                         if (g.out16) {
                             dn_us4 r;
 #pragma unroll
@@ -1091,7 +1096,7 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     if (copies > 1 && (g.N % 128 || !g.mu)) return false;
     if (a.force_tiled || kbytes % 128 || !a.pack) return false;
     const bool rows = !g.mu && !g.g_list && !g.a_mod && !g.a_step && !g.a_row0;
-    const bool handed = sizeof(WT) == 2 && PL == 1 && a.a16 && rows; // (the producer has rounded them already)
+    const bool handed = sizeof(WT) == 2 && PL == 1 && a.a16 && (rows || (g.g_list && !g.g_scale)); // (the producer has rounded them already; slots: in the list's order)
     const bool plain = handed || (sizeof(WT) == 4 && !g.mu && !g.g_scale && g.lda % 4 == 0 && ((uintptr_t)g.a & 15) == 0);
     if (!plain && (size_t)a.T * kbytes * PL * copies > a.pack_bytes) return false;
     if (PL == 3) {
@@ -1755,6 +1760,9 @@ bool psk_dense_takes_pre(const psk_dense_args &a) {
 bool psk_dense_wide16(const psk_dense_args &a) {
     return a.w && a.w->dtype == PS_BF16 && a.T > PSD_FEW && !a.force_tiled && a.pack && a.groups == 0 && !a.mu && !a.a_mod && !a.a_step && !a.a_row0 && a.w->K > 256 && a.w->K % 64 == 0 &&
            (size_t)a.T * a.w->K * 2 <= a.pack_bytes;
+}
+bool psk_dense_listed16(const psk_dense_args &a) { // (as dn_ring_take)
+    return a.w && a.w->dtype == PS_BF16 && a.groups > 0 && a.g_list && !a.force_tiled && a.pack && a.w->K % 64 == 0 && (size_t)a.T * a.w->K * 2 <= a.pack_bytes;
 }
 int psk_dense(hipStream_t st, const psk_dense_args &a) {
     if (!a.w || a.T <= 0) return 0;

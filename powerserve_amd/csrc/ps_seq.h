@@ -103,6 +103,7 @@ static const int PSD_FEW = 1;
 // The same for a mixture's own products, whose mat-vecs read a matrix per slot and the wide mat-mul a tile per matrix: up to two tokens, and up to a quarter more slots than there are experts.  Top 2 of
 // 8, mat-vecs | wide, Pupidra 2048 x 6: 2 tokens 696 | 874, 4 788 | 904, 5 827 | 917, 6 905 | 928; 4096 x 3: 4 772 | 840, 5 819 | 873, 6 931 | 920; float32 4 1094 | 1237, 5 1164 | 1243, 6 1316 | 1257.
 static inline bool psk_few_slots(int T, int top, int experts, bool wide) { return T <= 8 && (!wide || T <= 2 || 4 * T * top <= 5 * experts); } // (wide: the wide mat-mul takes both products)
+bool psk_dense_listed16(const psk_dense_args &a); // it will run this grouped product so: out16's and a16's rows are slots in g_list's order
 bool psk_dense_wide16(const psk_dense_args &a); // psk_dense will run this as the wide bf16 mat-mul over plain rows
 int psk_dense(hipStream_t st, const psk_dense_args &a);
 size_t psk_dense_split_bytes(); // what any product's splits need at most

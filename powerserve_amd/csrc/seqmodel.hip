@@ -863,6 +863,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         if (!mv) psk_moe_plan(st, m->moe_sel, S, rows, m->moe_seg, m->moe_list);
         auto grouped = [&](psk_dense_args &g) {
             g.groups = E; g.g_sel = m->moe_sel;
+            g.a16 = nullptr; // (rows of tokens, not of slots)
             if (!mv) { g.g_seg = m->moe_seg; g.g_list = m->moe_list; }
         };
         // (a single token's shared expert rides with the slots' launches where they are mat-vecs: its activations behind theirs)
@@ -871,6 +872,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         auto sd = mm(l.shared_down, su.out, l.shared_ff, xr, W);
         sd.accum = 1; sd.alpha = alpha; sd.out_scale = l.shared_gate ? m->moe_sg : nullptr;
         bool up_made = false, down_made = false;
+        const void *hidden16 = nullptr; // a portion's slots, rounded
         {
             auto g = mm(l.ff_up, in, W, m->t4, l.ff);
             g.act = act; g.T = S; g.g_adiv = top;
@@ -878,12 +880,17 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             else g.g_scale = m->moe_wgt;
             grouped(g);
             if (l.shared_up && mv && T == 1) g.also = &su;
+            auto down = mm(l.ff_down, m->t4, l.ff, xr, W);
+            grouped(down);
+            down.T = S;
+            if (psk_dense_listed16(g) && psk_dense_listed16(down)) hidden16 = g.out16 = m->t4;
             up_made = psk_dense(st, g) == 1;
         }
         bool summed = false; // the identity slots' share has joined the stream
         {
             auto g = mm(l.ff_down, m->t4, l.ff, xr, W);
             grouped(g);
+            g.a16 = hidden16;
             if (mv) {
                 g.T = T; g.g_inner = top; g.accum = !store; g.alpha = alpha;
                 if (l.moe_identity) { g.g_ident = in; g.g_ident_ld = W; g.g_ident_w = m->moe_wgt; summed = true; } // (the identity slots' share inside the same launch)

@@ -213,6 +213,29 @@ def test_experts_of_a_few_tokens(made, dtype, experts, ff):
     assert close(run_portions(m, toks, (2, 3, 4, 5, 6, 7, 8)), seq_oracle.run_pupidra(cfg, t, toks), dtype)
 
 
+# a mixture whose first products hand their rounded rows on in the list's order (seqmodel.hip hidden16), its scores at the result's rows: squared relu (from the registers) and gate / up pairs
+# (through LDS), one, two and three slots a token, products of ff behind them that no whole blocks fit; against the tiled mat-mul, which hands nothing on
+@pytest.mark.parametrize("top,ff", [(1, 64), (2, 128), (3, 320), (2, 72)])
+@pytest.mark.parametrize("family", ["squared relu", "pairs", "identity"])
+def test_experts_that_hand_rounded_rows_on(ctx, tmp_path, family, top, ff):
+    if family == "pairs":
+        cfg = synth.zusolix_config(64, 40, [synth.zusolix_layer("attention", synth.zusolix_attention(2, 1, 16, 16, 0.3), moe=(5, top, ff), shared=64)])
+    elif family == "identity":  # (slots without a product, behind the others in the list)
+        cfg = synth.pokatar_config(64, 40, [synth.pokatar_layer("attention", synth.pokatar_attention(2, 1, 16, 16, 0.3), moe=(5, top, ff, 3, 0, 0), shared=64)])
+    else:
+        cfg = UC(64, 40, [UL("attention", UA(2, 1, 16, 16, 0.3, 9, 2), (5, top, ff, 1.7), 64)])
+    synth.write_seq_model_dir(str(tmp_path), cfg, 3, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="bfloat16", max_batch=300, n_slots=1, max_context=700)
+    toks = tokens_for(cfg, 350)
+    sizes = (9, 300, 41)
+    got = run_portions(m, toks, sizes)
+    m.set_mode(2)  # the tiled mat-mul
+    want = run_portions(m, toks, sizes)
+    m.close()
+    # the same numbers are rounded, behind fp32 sums in another order: 2^-9 of a number now and then.  A row that is not its own, or a score: ~1
+    assert err(got, want) < 0.03
+
+
 # a token's boundary inside the next layer's first product (k_dense.hip dn_stage_pre), the stream then in one of two buffers: an even and an odd number of them, one run of a thread, several, the
 # most, widths that are no whole units (a launch of its own), a layer without experts behind it; captured steps, which begin and end in the same buffer
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
