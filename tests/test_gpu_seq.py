@@ -248,6 +248,21 @@ def test_four_mixes_together(made, width, heads, dim, dtype):
         assert e < TOL[dtype], (sizes, e)
 
 
+# all four mixes of a row by one thread (k_dense.hip dense_pack_kernel, 512 rows of 1024 and more), in a portion that begins a sequence and one that does not
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_four_mixes_of_many_rows(ctx, tmp_path, dtype):
+    cfg = synth.seq_config(1024, 40, [L("wkv", None, heads=4, dim=32)], taps=2)
+    synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype, max_batch=520, n_slots=1, max_context=1100)
+    toks = tokens_for(cfg, 1030)
+    got = run_portions(m, toks, (520, 510))
+    m.set_mode(2)  # the tiled mat-mul, which mixes where it reads
+    want = run_portions(m, toks, (520, 510))
+    m.close()
+    # fp32: a few ulps of fp32 sums; bf16: a rounding now and then goes the other way.  A mix that is not its own: ~1
+    assert err(got, want) < (TOL["float32"] if dtype == "float32" else 0.03)
+
+
 # bf16 rows handed from one kernel to the wide mat-mul behind it (inputs of more than 256 numbers, whole blocks of 64): filter -> projection, head norm -> projection, first -> second product;
 # beside them a projection that does not take them (260 is no multiple of 64), portions below and above the sizes that hand on, and what an earlier layer or portion left behind
 @pytest.mark.parametrize("sizes", [(9, 8, 64), (33, 1), (64,)])
