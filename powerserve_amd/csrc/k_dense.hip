@@ -779,7 +779,8 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     if (p.S > 1) return;
     // The weights are the matrix instructions' first operand, so a lane has four neighbouring outputs of a token in four registers: results that need no epilogue go straight to their
     // places.  Through LDS (two barriers, a loop of eight trips) 512 x 8192 of K = 2048 took 35.0 us with its packing, 31.2 this way, 512 x 2048 18.3 and 17.3.
-    // An activation of each of the 64 results of a lane, written out, is code that every CU has to fetch once: 40.6 us against 32.6 for a loop; it goes through LDS.
+    // An activation of each of the 64 results of a lane, written out, is code that every CU has to fetch once: 40.6 us against 32.6 for a loop; it goes through LDS
+    // (a squared relu is two instructions, a row's factor none: 1500 tokens of Pupidra 2048 x 6, 3514 us through LDS, 3283 so, with rounded rows handed on).
     if ((g.act == PSD_ACT_NONE || g.act == PSD_ACT_RELU2) && !g.bias && !g.accum && !g.em_table && g.N % 4 == 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out & 15) == 0 && ((uintptr_t)g.out16 & 7) == 0) { // (uniform)
         if (loads) return;
 #pragma unroll
