@@ -92,14 +92,14 @@ int ps_hip_weight_upload(ps_hip_ctx *c, int dtype, const void *host, int64_t K, 
     const size_t raw = (size_t)w->gguf_bytes;
     auto fail = [&](const char *m) { ps_hip_weight_free(c, w); c->err = m; return 1; };
     if (dtype == PS_F32) {
-        if (ps_dev_malloc((void **)&w->qs, raw) != hipSuccess) return fail("weight_upload: hipMalloc");
+        if (hipMalloc((void **)&w->qs, raw) != hipSuccess) return fail("weight_upload: hipMalloc");
         if (hipMemcpyAsync(w->qs, host, raw, hipMemcpyHostToDevice, c->stream) != hipSuccess) return fail("weight_upload: copy");
         PS_CHECK(c, hipStreamSynchronize(c->stream));
         *out = w;
         return 0;
     }
     uint8_t *tmp = nullptr;
-    if (ps_dev_malloc((void **)&tmp, raw + 64) != hipSuccess) return fail("weight_upload: ps_dev_malloc(tmp)");
+    if (hipMalloc((void **)&tmp, raw + 64) != hipSuccess) return fail("weight_upload: hipMalloc(tmp)");
     size_t qs_b = 0, aux_b = 0, qh_b = 0, sc_b = 0;
     if (dtype == PS_Q4_0 || dtype == PS_Q8_0 || dtype == PS_Q4_K) { // lane-major repack: 1 KiB units per row group
         const int64_t rg = ps_w_rg(dtype), ng = (N + rg - 1) / rg, nu = (K + ps_w_unit(dtype) - 1) / ps_w_unit(dtype);
@@ -108,13 +108,13 @@ int ps_hip_weight_upload(ps_hip_ctx *c, int dtype, const void *host, int64_t K, 
     }
     if (dtype == PS_Q6_K) { qs_b = (size_t)N * K / 2; qh_b = (size_t)N * K / 4; sc_b = (size_t)N * K / 16; aux_b = (size_t)N * (K / 256) * 2; }
     if (dtype == PS_Q5_K) { qs_b = (size_t)N * K / 2; qh_b = (size_t)N * K / 8; sc_b = (size_t)N * (K / 256) * 16; aux_b = 0; }
-    bool ok = ps_dev_malloc((void **)&w->qs, qs_b + 64) == hipSuccess && ps_dev_malloc((void **)&w->aux, aux_b + 64) == hipSuccess;
-    if (ok && qh_b) ok = ps_dev_malloc((void **)&w->qh, qh_b + 64) == hipSuccess && ps_dev_malloc((void **)&w->sc, sc_b + 64) == hipSuccess;
-    if (!ok) { (void)ps_dev_free(tmp); return fail("weight_upload: ps_dev_malloc(planes)"); }
-    if (hipMemcpyAsync(tmp, host, raw, hipMemcpyHostToDevice, c->stream) != hipSuccess) { (void)ps_dev_free(tmp); return fail("weight_upload: copy"); }
+    bool ok = hipMalloc((void **)&w->qs, qs_b + 64) == hipSuccess && hipMalloc((void **)&w->aux, aux_b + 64) == hipSuccess;
+    if (ok && qh_b) ok = hipMalloc((void **)&w->qh, qh_b + 64) == hipSuccess && hipMalloc((void **)&w->sc, sc_b + 64) == hipSuccess;
+    if (!ok) { (void)hipFree(tmp); return fail("weight_upload: hipMalloc(planes)"); }
+    if (hipMemcpyAsync(tmp, host, raw, hipMemcpyHostToDevice, c->stream) != hipSuccess) { (void)hipFree(tmp); return fail("weight_upload: copy"); }
     psk_repack_weight(c->stream, dtype, tmp, K, N, w);
     hipError_t e = hipStreamSynchronize(c->stream);
-    (void)ps_dev_free(tmp);
+    (void)hipFree(tmp);
     if (e != hipSuccess) return fail("weight_upload: repack");
     *out = w;
     return 0;
@@ -123,10 +123,10 @@ int ps_hip_weight_upload(ps_hip_ctx *c, int dtype, const void *host, int64_t K, 
 void ps_hip_weight_free(ps_hip_ctx *c, ps_weight *w) {
     if (!w) return;
     (void)c;
-    if (w->qs) (void)ps_dev_free(w->qs);
-    if (w->aux) (void)ps_dev_free(w->aux);
-    if (w->qh) (void)ps_dev_free(w->qh);
-    if (w->sc) (void)ps_dev_free(w->sc);
+    if (w->qs) (void)hipFree(w->qs);
+    if (w->aux) (void)hipFree(w->aux);
+    if (w->qh) (void)hipFree(w->qh);
+    if (w->sc) (void)hipFree(w->sc);
     delete w;
 }
 uint64_t ps_hip_weight_gguf_bytes(const ps_weight *w) { return w->gguf_bytes; }
@@ -136,10 +136,10 @@ int ps_hip_weight_dtype(const ps_weight *w) { return w->dtype; }
 static int ensure(ps_hip_ctx *c, void **buf, size_t *cap, size_t need) {
     if (*cap >= need) return 0;
     PS_CHECK(c, hipStreamSynchronize(c->stream));
-    if (*buf) PS_CHECK(c, ps_dev_free(*buf));
+    if (*buf) PS_CHECK(c, hipFree(*buf));
     *buf = nullptr;
     *cap = 0;
-    PS_CHECK(c, ps_dev_malloc(buf, need));
+    PS_CHECK(c, hipMalloc(buf, need));
     *cap = need;
     return 0;
 }

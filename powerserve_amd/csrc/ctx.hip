@@ -4,58 +4,6 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
-#include <unordered_map>
-
-// ------------------------------------------------------------------ device allocations (ps_internal.h)
-namespace {
-struct GuardRec { void *va; size_t reserved, mapped; hipMemGenericAllocationHandle_t h; };
-std::mutex g_guard_mu;
-std::unordered_map<void *, GuardRec> g_guard;
-int guard_align() { static const int a = getenv("PS_HIP_GUARD") ? atoi(getenv("PS_HIP_GUARD")) : 0; return a; } // 0: off; 1: on, hipMalloc's 256-byte alignment kept; 16 / 64 / ...: that alignment
-bool guard_on() { return guard_align() != 0; }
-} // namespace
-hipError_t ps_dev_malloc(void **p, size_t bytes) {
-    if (!guard_on()) return hipMalloc(p, bytes);
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    hipMemAllocationProp prop = {};
-    prop.type = hipMemAllocationTypePinned;
-    prop.location.type = hipMemLocationTypeDevice;
-    prop.location.id = dev;
-    size_t gran = 0;
-    if ((e = hipMemGetAllocationGranularity(&gran, &prop, hipMemAllocationGranularityMinimum)) != hipSuccess) return e;
-    const size_t al = guard_align() >= 16 ? (size_t)guard_align() : 256;
-    const size_t user = (bytes + al - 1) / al * al, mapped = (user + gran - 1) / gran * gran, reserved = mapped + gran; // (the last granule stays unmapped)
-    GuardRec r{nullptr, reserved, mapped, {}};
-    if ((e = hipMemAddressReserve(&r.va, reserved, gran, nullptr, 0)) != hipSuccess) return e;
-    if ((e = hipMemCreate(&r.h, mapped, &prop, 0)) != hipSuccess) { (void)hipMemAddressFree(r.va, reserved); return e; }
-    if ((e = hipMemMap(r.va, mapped, 0, r.h, 0)) != hipSuccess) { (void)hipMemRelease(r.h); (void)hipMemAddressFree(r.va, reserved); return e; }
-    hipMemAccessDesc acc = {};
-    acc.location = prop.location;
-    acc.flags = hipMemAccessFlagsProtReadWrite;
-    if ((e = hipMemSetAccess(r.va, mapped, &acc, 1)) != hipSuccess) { (void)hipMemUnmap(r.va, mapped); (void)hipMemRelease(r.h); (void)hipMemAddressFree(r.va, reserved); return e; }
-    *p = (char *)r.va + (mapped - user);
-    std::lock_guard<std::mutex> lk(g_guard_mu);
-    g_guard[*p] = r;
-    return hipSuccess;
-}
-hipError_t ps_dev_free(void *p) {
-    if (!p) return hipSuccess;
-    if (!guard_on()) return hipFree(p);
-    GuardRec r;
-    {
-        std::lock_guard<std::mutex> lk(g_guard_mu);
-        auto it = g_guard.find(p);
-        if (it == g_guard.end()) return hipFree(p);
-        r = it->second;
-        g_guard.erase(it);
-    }
-    // the range is never handed back: with hipMemUnmap / hipMemRelease / hipMemAddressFree behind every free, later allocations of the same process read
-    // wrong data now and then (ops tests failed at random under recycling and pass without it); a debugging run can afford the memory
-    return hipSuccess;
-}
 
 // ------------------------------------------------------------------ small data in, results out (ps_internal.h)
 namespace {
@@ -181,10 +129,10 @@ void ps_hip_destroy(ps_hip_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    if (c->act_buf) (void)ps_dev_free(c->act_buf);
-    if (c->i32_buf) (void)ps_dev_free(c->i32_buf);
-    if (c->u8_buf) (void)ps_dev_free(c->u8_buf);
-    if (c->rope_buf) (void)ps_dev_free(c->rope_buf);
+    if (c->act_buf) (void)hipFree(c->act_buf);
+    if (c->i32_buf) (void)hipFree(c->i32_buf);
+    if (c->u8_buf) (void)hipFree(c->u8_buf);
+    if (c->rope_buf) (void)hipFree(c->rope_buf);
     if (c->pin) (void)hipHostFree(c->pin);
     for (auto e : c->pin_ev) if (e) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(c->stream);
@@ -202,12 +150,12 @@ int ps_hip_device_name(const ps_hip_ctx *c, char *buf, size_t cap) {
 
 int ps_hip_malloc(ps_hip_ctx *c, size_t bytes, void **dptr) {
     PS_CHECK(c, hipSetDevice(c->device));
-    PS_CHECK(c, ps_dev_malloc(dptr, bytes ? bytes : 16));
+    PS_CHECK(c, hipMalloc(dptr, bytes ? bytes : 16));
     return 0;
 }
 int ps_hip_free(ps_hip_ctx *c, void *dptr) {
     PS_CHECK(c, hipStreamSynchronize(c->stream));
-    PS_CHECK(c, ps_dev_free(dptr));
+    PS_CHECK(c, hipFree(dptr));
     return 0;
 }
 int ps_hip_memcpy_h2d(ps_hip_ctx *c, void *dst, const void *src, size_t bytes) {

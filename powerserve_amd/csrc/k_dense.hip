@@ -1991,14 +1991,14 @@ int ps_hip_dense_upload(ps_hip_ctx *c, const uint16_t *host, int64_t N, int64_t 
     w->N = N; w->K = K; w->dtype = as_f32 ? PS_F32 : PS_BF16;
     const size_t n = (size_t)N * K;
     uint16_t *raw = nullptr;
-    if (ps_dev_malloc((void **)&raw, n * 2 + 64) != hipSuccess) { delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
-    if (hipMemcpyAsync(raw, host, n * 2, hipMemcpyHostToDevice, c->stream) != hipSuccess) { (void)ps_dev_free(raw); delete w; PS_FAIL(c, "dense_upload: copy"); }
+    if (hipMalloc((void **)&raw, n * 2 + 64) != hipSuccess) { delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
+    if (hipMemcpyAsync(raw, host, n * 2, hipMemcpyHostToDevice, c->stream) != hipSuccess) { (void)hipFree(raw); delete w; PS_FAIL(c, "dense_upload: copy"); }
     // An fp32 matrix keeps its bf16 form for the wide mat-mul (PL 3 there) where all its numbers are finite (an infinite one meets the zeros of the operand's lower lines) and where half of the
     // device's memory is free beside it.
     int32_t *odd = (int32_t *)((char *)raw + (n * 2 + 15) / 16 * 16), is_odd = 0;
     if (as_f32) {
         float *f = nullptr;
-        if (ps_dev_malloc((void **)&f, n * 4 + 64) != hipSuccess) { (void)ps_dev_free(raw); delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
+        if (hipMalloc((void **)&f, n * 4 + 64) != hipSuccess) { (void)hipFree(raw); delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
         psk_dense_widen(c->stream, raw, (int64_t)n, f);
         w->data = f;
         psk_fill(c->stream, (float *)odd, 0.f, 1);
@@ -2011,17 +2011,17 @@ int ps_hip_dense_upload(ps_hip_ctx *c, const uint16_t *host, int64_t N, int64_t 
         size_t free = 0, all = 0;
         const bool keep = e == hipSuccess && hipMemcpy(&is_odd, odd, 4, hipMemcpyDeviceToHost) == hipSuccess && !is_odd && hipMemGetInfo(&free, &all) == hipSuccess && free > all / 2;
         if (keep) w->half = raw;
-        else (void)ps_dev_free(raw);
+        else (void)hipFree(raw);
     }
-    if (e != hipSuccess) { (void)ps_dev_free(w->data); delete w; PS_FAIL(c, std::string("dense_upload: ") + hipGetErrorString(e)); }
+    if (e != hipSuccess) { (void)hipFree(w->data); delete w; PS_FAIL(c, std::string("dense_upload: ") + hipGetErrorString(e)); }
     *out = w;
     return 0;
 }
 void ps_hip_dense_free(ps_hip_ctx *c, ps_dense *w) {
     if (!w) return;
     if (c) (void)hipStreamSynchronize(c->stream);
-    (void)ps_dev_free(w->data);
-    if (w->half) (void)ps_dev_free(w->half);
+    (void)hipFree(w->data);
+    if (w->half) (void)hipFree(w->half);
     delete w;
 }
 int ps_hip_dense_matmul(ps_hip_ctx *c, const ps_dense *w, const float *x, int T, float *out, float alpha) {
@@ -2035,9 +2035,9 @@ int ps_hip_dense_matmul(ps_hip_ctx *c, const ps_dense *w, const float *x, int T,
     const size_t pack = packs ? (size_t)(piece * row + 255) / 256 * 256 : 0, need = pack + psk_dense_split_bytes();
     if (wide && c->act_cap < need) {
         PS_CHECK(c, hipStreamSynchronize(c->stream));
-        if (c->act_buf) (void)ps_dev_free(c->act_buf);
+        if (c->act_buf) (void)hipFree(c->act_buf);
         c->act_buf = nullptr; c->act_cap = 0;
-        if (ps_dev_malloc(&c->act_buf, need) == hipSuccess) c->act_cap = need;
+        if (hipMalloc(&c->act_buf, need) == hipSuccess) c->act_cap = need;
         else { c->act_buf = nullptr; (void)hipGetLastError(); }
     }
     for (int64_t t = 0; t < T; t += piece) {

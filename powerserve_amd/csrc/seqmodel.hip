@@ -387,7 +387,7 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
         if (P.owner >= 0) { const LayerPlan &O = m->L[P.owner]; P.off_ring = O.off_ring; P.off_pool = O.off_pool; P.cap = O.cap; }
     m->state_floats = off;
     auto alloc = [&](void **p, size_t bytes) {
-        if (ps_dev_malloc(p, bytes + 256) != hipSuccess) return false;
+        if (hipMalloc(p, bytes + 256) != hipSuccess) return false;
         m->owned.push_back(*p);
         return true;
     };
@@ -551,9 +551,9 @@ void ps_hip_seq_destroy(ps_hip_seq *m) {
     (void)hipSetDevice(m->ctx->device);
     (void)hipStreamSynchronize(m->ctx->stream);
     for (auto &g : m->graphs) (void)hipGraphExecDestroy(g.second);
-    for (void *p : m->owned) (void)ps_dev_free(p);
+    for (void *p : m->owned) (void)hipFree(p);
     for (ps_dense *j : m->joints) delete j; // (their data is in `owned`)
-    if (m->ids) (void)ps_dev_free(m->ids);
+    if (m->ids) (void)hipFree(m->ids);
     delete m;
 }
 
@@ -1148,8 +1148,8 @@ int ps_hip_seq_decode_greedy(ps_hip_seq *m, int slot, int32_t token, int steps, 
     if (m->needs_context && m->slot_pos[slot] + steps > m->max_context) return seq_fail(c, "seq_decode_greedy: the sequence would exceed max_context");
     PS_CHECK(c, hipSetDevice(c->device));
     if (steps > m->ids_cap) {
-        if (m->ids) { PS_CHECK(c, hipStreamSynchronize(c->stream)); (void)ps_dev_free(m->ids); m->ids = nullptr; }
-        PS_CHECK(c, ps_dev_malloc((void **)&m->ids, (size_t)steps * 4 + 256));
+        if (m->ids) { PS_CHECK(c, hipStreamSynchronize(c->stream)); (void)hipFree(m->ids); m->ids = nullptr; }
+        PS_CHECK(c, hipMalloc((void **)&m->ids, (size_t)steps * 4 + 256));
         m->ids_cap = steps;
         for (auto &g : m->graphs) (void)hipGraphExecDestroy(g.second); // (the captured sequences hold the old pointer)
         m->graphs.clear();
