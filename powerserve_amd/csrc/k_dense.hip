@@ -1944,7 +1944,7 @@ static __device__ __forceinline__ int dn_first_max(const float *row, int count, 
     return at < count ? at : 0;
 }
 // A greedy step's end and the next one's beginning in one block (ps_seq.h psk_next_token): the arg-max, the step's numbers and the embedding were three launches of 4 us each, most of it their start.
-__global__ __launch_bounds__(1024) void dense_next_kernel(const float *x, long long n, ps_seq_step *step, int32_t *ids, int32_t *prev, const void *table, int is_bf16, long long K, float scale, float *out,
+__global__ __launch_bounds__(1024) void dense_next_kernel(const float *x, long long n, ps_seq_step *step, int32_t *ids, int32_t *prev, const void *table, int is_bf16, long long rows, long long K, float scale, float *out,
                                                           const void *bigram, long long buckets, long long mul_prev, long long mul_cur) {
     __shared__ float bv[16];
     __shared__ int bi[16], id;
@@ -1962,13 +1962,13 @@ __global__ __launch_bounds__(1024) void dense_next_kernel(const float *x, long l
     __syncthreads();
     const long long tok = id, row = bigram ? ((long long)before * mul_prev + tok * mul_cur) % buckets : 0; // (never a sequence's first token)
     for (long long k = threadIdx.x; k < K; k += 1024) {
-        const float v = dn_table(table, is_bf16, tok * K + k) * scale;
+        const float v = tok < rows ? dn_table(table, is_bf16, tok * K + k) * scale : 0.f; // (the logits may be more than the table's rows)
         out[k] = bigram ? v + dn_table(bigram, is_bf16, row * K + k) : v;
     }
 }
 void psk_next_token(hipStream_t st, const float *logits, int64_t n, ps_seq_step *step, int32_t *ids, int32_t *prev, const ps_dense *table, float scale, float *out, const ps_dense *bigram,
                     int64_t buckets, int64_t mul_prev, int64_t mul_cur) {
-    hipLaunchKernelGGL(dense_next_kernel, dim3(1), dim3(1024), 0, st, logits, (long long)n, step, ids, prev, table->data, table->dtype == PS_BF16 ? 1 : 0, (long long)table->K, scale, out,
+    hipLaunchKernelGGL(dense_next_kernel, dim3(1), dim3(1024), 0, st, logits, (long long)n, step, ids, prev, table->data, table->dtype == PS_BF16 ? 1 : 0, (long long)table->N, (long long)table->K, scale, out,
                        bigram ? bigram->data : nullptr, (long long)buckets, (long long)mul_prev, (long long)mul_cur);
 }
 // a row's largest logit, the lowest index among equals: a block per row

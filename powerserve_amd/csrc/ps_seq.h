@@ -113,7 +113,7 @@ void psk_dense_widen(hipStream_t st, const uint16_t *bf16, int64_t n, float *out
 void psk_embed(hipStream_t st, const ps_dense *table, const int32_t *tokens, const ps_seq_step *step, int T, float scale, float *out, int64_t ldo, const ps_dense *bigram = nullptr,
                int64_t buckets = 0, int64_t mul_prev = 0, int64_t mul_cur = 0);
 // the end of a greedy step and the beginning of the next one: id = the first maximum of logits[0..n), kept at ids[step->_pad++]; step->prev (and *prev, where given) = step->token0, which becomes id;
-// the position moves on; out = id's embedding (psk_embed)
+// the position moves on; out = id's embedding (psk_embed; zeros for an id without a row)
 void psk_next_token(hipStream_t st, const float *logits, int64_t n, ps_seq_step *step, int32_t *ids, int32_t *prev, const ps_dense *table, float scale, float *out, const ps_dense *bigram,
                     int64_t buckets, int64_t mul_prev, int64_t mul_cur);
 // out[r] = index of the first maximum of x[r][0..n)

@@ -89,6 +89,7 @@ struct ps_hip_seq {
     std::vector<void *> owned;
     std::vector<ps_dense *> joints;
     int64_t off_prev = -1; // bigram embedding: where a slot's state keeps the last token (an int32)
+    int64_t ids_end() const { return std::min<int64_t>(d.vocab, d.embed->N); } // token ids that have a row of the embedding
     int32_t *prev_of(int slot) const { return off_prev < 0 ? nullptr : (int32_t *)(slot_state[slot] + off_prev); }
 };
 
@@ -1052,7 +1053,7 @@ int ps_hip_seq_forward(ps_hip_seq *m, int slot, const int32_t *tokens, int n, co
     if (n <= 0 || !tokens) return seq_fail(c, "seq_forward: no tokens");
     if (m->needs_context && m->slot_pos[slot] + n > m->max_context) return seq_fail(c, "seq_forward: the sequence would exceed max_context");
     for (int i = 0; i < n; i++)
-        if (tokens[i] < 0 || tokens[i] >= m->d.vocab) return seq_fail(c, "seq_forward: token id outside the vocabulary");
+        if (tokens[i] < 0 || tokens[i] >= m->ids_end()) return seq_fail(c, "seq_forward: token id outside the vocabulary");
     for (int i = 0; i < n_want; i++)
         if (want[i] < 0 || want[i] >= n || (i && want[i] < want[i - 1])) return seq_fail(c, "seq_forward: want must be ascending indices into the step's tokens");
     const int B = m->d.max_batch;
@@ -1144,7 +1145,7 @@ int ps_hip_seq_decode_greedy(ps_hip_seq *m, int slot, int32_t token, int steps, 
     ps_hip_ctx *c = m->ctx;
     if (slot < 0 || slot >= (int)m->slot_pos.size() || m->slot_pos[slot] < 0) return seq_fail(c, "seq_decode_greedy: not a live slot");
     if (steps <= 0) return 0;
-    if (token < 0 || token >= m->d.vocab) return seq_fail(c, "seq_decode_greedy: token id outside the vocabulary");
+    if (token < 0 || token >= m->ids_end()) return seq_fail(c, "seq_decode_greedy: token id outside the vocabulary");
     if (m->needs_context && m->slot_pos[slot] + steps > m->max_context) return seq_fail(c, "seq_decode_greedy: the sequence would exceed max_context");
     PS_CHECK(c, hipSetDevice(c->device));
     if (steps > m->ids_cap) {
@@ -1195,7 +1196,7 @@ int ps_hip_seq_bench_kernel(ps_hip_seq *m, int which, int T, int reps, double *u
     const int64_t W = m->d.width;
     auto embed_from = [&](int first) { // tokens first, first + 1, ... embedded as the input: a routing as spread as the router's rows make it
         std::vector<int32_t> ids((size_t)T);
-        for (int i = 0; i < T; i++) ids[i] = (first + i) % m->d.vocab;
+        for (int i = 0; i < T; i++) ids[i] = (int32_t)((first + i) % m->ids_end());
         if (hipMemcpyAsync(m->tokens, ids.data(), (size_t)T * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) return false;
         psk_embed(c->stream, m->d.embed, m->tokens, m->step, T, m->embed_scale, m->h, W);
         return hipStreamSynchronize(c->stream) == hipSuccess;

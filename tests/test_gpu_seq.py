@@ -599,6 +599,27 @@ def test_a_long_input_in_launch_sequences_wider_than_max_batch(ctx, tmp_path, dt
     m.close()
 
 
+# a head of more rows than the embedding has: a generated id beyond them embeds as zeros (k_dense.hip dense_next_kernel), the ones in front of it as their rows; eager and captured
+@pytest.mark.parametrize("mode", [0, 1])
+def test_a_generated_id_without_a_row_of_the_embedding(ctx, tmp_path, mode):
+    cfg = synth.seq_config(48, 300, [L("wkv", 40, heads=2, dim=24)], taps=2)
+    t = synth.seq_tensors(cfg, 3)
+    t["embed"], t["head"] = t["embed"][:20], t["head"].copy()
+    t["head"][:280] = 0  # (so that every generated id is one of the last twenty)
+    synth.write_seq_model_dir(str(tmp_path), cfg, 3, t)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=8, n_slots=2)
+    t = {n: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(np.shape(a)) for n, a in t.items()}
+    t["embed"] = np.concatenate([t["embed"], np.zeros((280, 48), np.float32)])
+    m.set_mode(mode)
+    s = m.acquire()
+    ids = m.decode_greedy(s, 7, 4)
+    want = seq_oracle.run(cfg, t, np.array([7, *ids[:3]]))
+    assert ids.min() >= 280 and np.array_equal(ids, want.argmax(-1))
+    with pytest.raises(hip.PSHipError):
+        m.forward(s, ids[-1:], [0])
+    m.close()
+
+
 def test_interleaved_requests_and_reused_slots(made):
     m, cfg, t = made("mixed", "float32", max_batch=16)
     seqs = [tokens_for(cfg, n, seed=20 + n) for n in (37, 9, 58)]

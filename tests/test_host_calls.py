@@ -49,6 +49,7 @@ def child(fake, tmp_path):
                            capture_output=True, text=True, timeout=120)
         assert p.returncode == 0 and p.stdout.endswith("done\n"), (p.stdout[-1000:], p.stderr[-3000:])
 
+    run.tmp = tmp_path
     return run
 
 
@@ -65,6 +66,24 @@ for tokens, want in (([1], [0] * 9), ([1] * 20, [0, 1] + [9] * 9), ([1] * 20, [1
 m.forward(s, [1] * 20, want=[0] * 8 + [8] * 8 + [19] * 8)
 assert m.position(s) == 20 and fake.fake_stray() == 0
 """)
+
+
+def test_ids_without_a_row_of_the_embedding_are_refused(child):
+    """a table shorter than the vocabulary: an id that it has no row for is refused before anything is launched, one that it has is taken"""
+    child("""
+cfg = synth.seq_config(24, 30, [L("wkv", None, heads=3, dim=8)], taps=3)
+t = synth.seq_tensors(cfg, 1)
+t["embed"] = t["embed"][:20]
+synth.write_seq_model_dir(".short", cfg, 1, t)
+m = seqmodel.SeqModel(hip.Ctx(0), ".short", max_batch=8)
+s = m.acquire()
+fake.fake_reset()
+for f in (lambda: m.forward(s, [19, 20]), lambda: m.forward(s, [29]), lambda: m.decode_greedy(s, 20, 3)):
+    assert "outside the vocabulary" in refused(f)
+assert count("hipLaunchKernel") == count("put_kernel") == 0
+m.forward(s, [19, 0])
+m.decode_greedy(s, 19, 3)
+""".replace(".short", str(child.tmp / "short")))
 
 
 def test_a_model_without_room_for_wide_launch_sequences(child):
