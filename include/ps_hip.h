@@ -334,8 +334,14 @@ enum ps_layer_form {
 enum ps_rot_pairing { PS_ROT_HALVES = 0 /* (i, i + dims/2) */, PS_ROT_NEIGHBOURS = 1 /* (2i, 2i + 1) */ };
 
 /* Dense matrix [N rows = outputs][K = inputs], row-major, applied as W x.  host_bf16: N*K bfloat16 bit patterns.
- * as_f32 != 0 widens it to fp32 on the device (the fp32 compute mode). */
+ * as_f32: PS_DENSE_BF16 keeps them; PS_DENSE_F32 (and any other number) widens them to fp32 on the device (the fp32 compute mode: 4 bytes per number, every product on the fp32 instruction);
+ * PS_DENSE_F32_LINES widens them and keeps the bfloat16 form beside it (6 bytes per number), with which products of several tokens run on the bfloat16 instruction, their operand as three
+ * bfloat16 numbers -- K a multiple of 64, every number of the matrix finite; otherwise as PS_DENSE_F32.  Both are fp32 products; their sums run in other orders. */
+enum ps_dense_form { PS_DENSE_BF16 = 0, PS_DENSE_F32 = 1, PS_DENSE_F32_LINES = 2 };
 int ps_hip_dense_upload(ps_hip_ctx *ctx, const uint16_t *host_bf16, int64_t N, int64_t K, int as_f32, ps_dense **out);
+/* which fp32 form a model of so many numbers in all is loaded in: PS_DENSE_F32_LINES where the bfloat16 forms take up to an eighth of the device's memory (whatever is free of it at the moment) */
+int ps_hip_dense_f32_form(ps_hip_ctx *ctx, uint64_t numbers);
+int ps_hip_dense_form(const ps_dense *w); /* the form a matrix is held in */
 void ps_hip_dense_free(ps_hip_ctx *ctx, ps_dense *w);
 /* out[T][N] = alpha * (x[T][K] . W^T), device fp32 in and out (tests, micro-benchmarks; the model uses the same launchers) */
 int ps_hip_dense_matmul(ps_hip_ctx *ctx, const ps_dense *w, const float *x_dev, int T, float *out_dev, float alpha);

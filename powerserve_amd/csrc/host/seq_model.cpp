@@ -79,7 +79,7 @@ const float *SeqUploader::vec(const std::vector<float> &a) {
 const ps_dense *SeqUploader::mat(const std::vector<uint16_t> &bits, int64_t rows, int64_t cols) {
     POWERSERVE_ASSERT((int64_t)bits.size() == rows * cols);
     ps_dense *w = nullptr;
-    hip_ok(ctx, ps_hip_dense_upload(ctx, bits.data(), rows, cols, as_f32 ? 1 : 0, &w), "ps_hip_dense_upload");
+    hip_ok(ctx, ps_hip_dense_upload(ctx, bits.data(), rows, cols, form, &w), "ps_hip_dense_upload");
     mats.push_back(w);
     return w;
 }
@@ -790,7 +790,9 @@ SeqModel::SeqModel(const std::string &model_dir, const std::string &dtype, int d
     arch = cfg.at("architecture").str;
     SafeTensorsFile st(model_dir + "/model.safetensors");
     if (ps_hip_create(device, &m_ctx) != 0) POWERSERVE_ABORT("no HIP device: the MI355X backend cannot run (there is no CPU fallback)");
-    m_up = SeqUploader{m_ctx, dtype == "float32", {}, {}, {}};
+    uint64_t numbers = 0;
+    for (const auto &[name, t] : st.tensors) numbers += (uint64_t)t.numel();
+    m_up = SeqUploader{m_ctx, dtype == "float32" ? ps_hip_dense_f32_form(m_ctx, numbers) : (int)PS_DENSE_BF16, {}, {}, {}};
     std::vector<ps_seq_layer> layers;
     ps_seq_desc d{};
     try {

@@ -40,7 +40,7 @@ private:
 // puts tensors on the device and keeps them until the model goes
 struct SeqUploader {
     ps_hip_ctx *ctx;
-    bool as_f32;
+    int form; // enum ps_dense_form
     std::vector<void *> vecs;
     std::vector<ps_dense *> mats;
     std::deque<ps_seq_layer> beside; // descriptors of second mixers, pointed to from the layers (addresses stay put)

@@ -1993,30 +1993,39 @@ int ps_hip_dense_upload(ps_hip_ctx *c, const uint16_t *host, int64_t N, int64_t 
     uint16_t *raw = nullptr;
     if (hipMalloc((void **)&raw, n * 2 + 64) != hipSuccess) { delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
     if (hipMemcpyAsync(raw, host, n * 2, hipMemcpyHostToDevice, c->stream) != hipSuccess) { (void)hipFree(raw); delete w; PS_FAIL(c, "dense_upload: copy"); }
-    // An fp32 matrix keeps its bf16 form for the wide mat-mul (PL 3 there) where all its numbers are finite (an infinite one meets the zeros of the operand's lower lines) and where half of the
-    // device's memory is free beside it.
-    int32_t *odd = (int32_t *)((char *)raw + (n * 2 + 15) / 16 * 16), is_odd = 0;
+    // PS_DENSE_F32_LINES keeps the bf16 form for the wide mat-mul (PL 3 there) where all its numbers are finite (an infinite one meets the zeros of the operand's lower lines).
+    const bool lines = as_f32 == PS_DENSE_F32_LINES;
+    int32_t *odd = (int32_t *)((char *)raw + (n * 2 + 15) / 16 * 16), is_odd = 1;
     if (as_f32) {
         float *f = nullptr;
         if (hipMalloc((void **)&f, n * 4 + 64) != hipSuccess) { (void)hipFree(raw); delete w; PS_FAIL(c, "dense_upload: out of device memory"); }
         psk_dense_widen(c->stream, raw, (int64_t)n, f);
         w->data = f;
-        psk_fill(c->stream, (float *)odd, 0.f, 1);
-        hipLaunchKernelGGL(dense_odd_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, c->stream, raw, (long long)n, odd);
+        if (lines) {
+            psk_fill(c->stream, (float *)odd, 0.f, 1);
+            hipLaunchKernelGGL(dense_odd_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, c->stream, raw, (long long)n, odd);
+        }
     } else {
         w->data = raw;
     }
-    hipError_t e = hipStreamSynchronize(c->stream);
+    hipError_t e = lines ? hipMemcpyAsync(&is_odd, odd, 4, hipMemcpyDeviceToHost, c->stream) : hipSuccess;
+    const hipError_t done = hipStreamSynchronize(c->stream); // (whatever came before: the copy reads and writes memory of this call)
+    if (e == hipSuccess) e = done;
     if (as_f32) {
-        size_t free = 0, all = 0;
-        const bool keep = e == hipSuccess && hipMemcpy(&is_odd, odd, 4, hipMemcpyDeviceToHost) == hipSuccess && !is_odd && hipMemGetInfo(&free, &all) == hipSuccess && free > all / 2;
-        if (keep) w->half = raw;
+        if (e == hipSuccess && !is_odd) w->half = raw;
         else (void)hipFree(raw);
     }
     if (e != hipSuccess) { (void)hipFree(w->data); delete w; PS_FAIL(c, std::string("dense_upload: ") + hipGetErrorString(e)); }
     *out = w;
     return 0;
 }
+int ps_hip_dense_f32_form(ps_hip_ctx *c, uint64_t numbers) {
+    size_t free = 0, all = 0;
+    const bool known = hipSetDevice(c->device) == hipSuccess && hipMemGetInfo(&free, &all) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    return known && numbers <= all / 16 ? PS_DENSE_F32_LINES : PS_DENSE_F32;
+}
+int ps_hip_dense_form(const ps_dense *w) { return w->dtype == PS_BF16 ? PS_DENSE_BF16 : w->half ? PS_DENSE_F32_LINES : PS_DENSE_F32; }
 void ps_hip_dense_free(ps_hip_ctx *c, ps_dense *w) {
     if (!w) return;
     if (c) (void)hipStreamSynchronize(c->stream);

@@ -8,7 +8,7 @@ struct ps_dense {
     int dtype = PS_BF16; // PS_BF16 or PS_F32
     int64_t N = 0, K = 0;
     void *data = nullptr;
-    void *half = nullptr; // PS_F32: the same numbers in bf16, as they came (NULL: not kept, or not all of them finite)
+    void *half = nullptr; // PS_F32: the same numbers in bf16, as they came (PS_DENSE_F32_LINES; NULL: not asked for, or not all of them finite)
 };
 
 // What every kernel of a step reads from DEVICE memory, so that one captured launch sequence replays for any position and slot:

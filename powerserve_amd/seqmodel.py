@@ -609,8 +609,8 @@ def read_config(model_dir: str) -> dict:
 
 
 class _Uploader:
-    def __init__(self, ctx: hip.Ctx, as_f32: bool):
-        self.ctx, self.as_f32, self.vecs, self.mats = ctx, as_f32, [], []
+    def __init__(self, ctx: hip.Ctx, form: int):
+        self.ctx, self.form, self.vecs, self.mats = ctx, form, [], []
 
     def vec(self, a: np.ndarray) -> int:
         d = self.ctx.to_device(np.ascontiguousarray(a, dtype=np.float32))
@@ -620,23 +620,26 @@ class _Uploader:
     def mat(self, bits: np.ndarray) -> int:
         bits = np.ascontiguousarray(bits, dtype=np.uint16)
         h = C.c_void_p()
-        self.ctx.check(self.ctx.L.ps_hip_dense_upload(self.ctx.h, bits.ctypes.data_as(C.c_void_p), bits.shape[0], bits.shape[1], int(self.as_f32), C.byref(h)))
+        self.ctx.check(self.ctx.L.ps_hip_dense_upload(self.ctx.h, bits.ctypes.data_as(C.c_void_p), bits.shape[0], bits.shape[1], self.form, C.byref(h)))
         self.mats.append(h.value)
         return h.value
 
 
 class SeqModel:
     """ps_hip_seq over a model directory.  dtype "bfloat16": matrix products on bfloat16 operands, fp32 accumulation; "float32": fp32
-    throughout.  Sequences live in slots (acquire / release); forward() is the step function, generate() the greedy / sampled loop."""
+    throughout.  f32_form: the form of a float32 model's matrices (hip.DENSE_F32 / DENSE_F32_LINES; None: by the model's size,
+    ps_hip_dense_f32_form).  Sequences live in slots (acquire / release); forward() is the step function, generate() the greedy / sampled loop."""
 
-    def __init__(self, ctx: hip.Ctx, model_dir: str, dtype: str = "bfloat16", max_batch: int = 256, n_slots: int = 2, max_context: int = 0):
+    def __init__(self, ctx: hip.Ctx, model_dir: str, dtype: str = "bfloat16", max_batch: int = 256, n_slots: int = 2, max_context: int = 0, f32_form: int | None = None):
         if dtype not in ("bfloat16", "float32"):
             raise ConfigError(f"dtype {dtype!r}: bfloat16 or float32")
         self.ctx, self.dtype = ctx, dtype
         self.cfg = read_config(model_dir)
         self.arch = self.cfg["architecture"]
         st = SafeTensors(os.path.join(model_dir, "model.safetensors"))
-        self._up = _Uploader(ctx, dtype == "float32")
+        if f32_form is None:
+            f32_form = int(ctx.L.ps_hip_dense_f32_form(ctx.h, sum(int(np.prod(st.shape(n))) for n in st.names())))
+        self._up = _Uploader(ctx, f32_form if dtype == "float32" else hip.DENSE_BF16)
         layers, top = ARCHITECTURES[self.arch](self.cfg, st, self._up)
         self._layers = (hip.SeqLayer * len(layers))(*layers)
         d = hip.SeqDesc()

@@ -113,6 +113,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
     const hipError_t e = call("hipMalloc");
     return e != hipSuccess ? e : alloc(p, bytes, hipMemoryTypeDevice);
 }
+hipError_t hipMemGetInfo(size_t *free, size_t *all) { *free = (size_t)1 << 30; *all = (size_t)288 << 30; return call("hipMemGetInfo"); }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return call("hipHostMalloc") ? hipErrorUnknown : alloc(p, bytes, hipMemoryTypeHost); }
 hipError_t hipFree(void *p) { mem.erase((char *)p); free(p); return hipSuccess; }
 hipError_t hipHostFree(void *p) { return hipFree(p); }

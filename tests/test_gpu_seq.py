@@ -32,6 +32,8 @@ CONFIGS = {
 # float32: a few ulps of fp32 sums.  bfloat16: the operands of every matrix product are rounded to 8 bits of mantissa, which in models this
 # narrow (48 to 128 channels) leaves 1-3 % on a typical row and up to 7 % on the worst of a hundred rows, whatever the schedule
 TOL = {"float32": 2e-4, "bfloat16": 1e-1}
+# what ps_hip_dense_upload makes of a matrix: fp32 on the fp32 instruction, fp32 on the bf16 instruction (three lines of the operand), bf16
+FORMS = {"float32": hip.DENSE_F32, "float32 lines": hip.DENSE_F32_LINES, "bfloat16": hip.DENSE_BF16}
 
 
 def err(got, want):
@@ -194,7 +196,7 @@ def test_latent_attention_of_a_very_long_window(ctx, tmp_path, window):
 
 # the wide mat-mul (k_dense.hip dense_mm_ring_kernel): one row more and less than its tiles of 64 and 128 tokens and outputs, one block of K and fewer blocks than stages,
 # products split along K (few tiles, long K: also uneven shares), more tiles than the chip has CUs
-@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dtype", list(FORMS))
 @pytest.mark.parametrize("T,N,K", [(9, 1, 64), (63, 127, 128), (64, 128, 192), (65, 129, 256), (127, 63, 320), (128, 65, 576), (129, 200, 64), (300, 130, 1088), (16, 8, 4096), (40, 100, 4160),
                                    (200, 256, 2240), (520, 2100, 128),
                                    # dense_mm_big_kernel (bf16): one block of K, two, three and more than its stages; a row, a column and four columns more than a tile; no fours
@@ -207,11 +209,12 @@ def test_dense_matmul_wide(ctx, dtype, T, N, K):
     x = rng.standard_normal((T, K), dtype=np.float32)
     w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K)
     h = C.c_void_p()
-    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, int(dtype == "float32"), C.byref(h)))
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, FORMS[dtype], C.byref(h)))
+    assert ctx.L.ps_hip_dense_form(h) == FORMS[dtype]
     dx, do = ctx.to_device(x), ctx.to_device(np.full((T + 1, N), np.float32(7.0)))
     ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, h, dx.ptr, T, do.ptr, 1.0))
     got = do.numpy()
-    a = (x if dtype == "float32" else rnd(x)).astype(np.float64)
+    a = (rnd(x) if dtype == "bfloat16" else x).astype(np.float64)
     # fp32 sums of K products, in any order: at most K roundings of 2^-24, each relative to a partial sum of at most sum |a w|
     bound = K * 2.0 ** -24 * (np.abs(a) @ np.abs(w.astype(np.float64)).T)
     assert np.all(np.abs(got[:T] - a @ w.astype(np.float64).T) <= bound)
@@ -284,7 +287,8 @@ def test_bf16_rows_handed_on(made, sizes):
 # finite rows and columns beside them as exact as ever, the others infinite or NaN as fp32 arithmetic has them
 @pytest.mark.parametrize("T,N,K", [(16, 24, 64), (70, 130, 192), (700, 5000, 64)])
 @pytest.mark.parametrize("odd_weights", [False, True])
-def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights):
+@pytest.mark.parametrize("dtype", ["float32", "float32 lines"])
+def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights, dtype):
     import ctypes as C
     rng = np.random.default_rng(T)
     w = rng.standard_normal((N, K), dtype=np.float32)
@@ -298,7 +302,8 @@ def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights):
     x[4, 0], x[5, 3] = np.inf, np.nan
     x[6] = 1  # (its lower lines are zeros)
     h = C.c_void_p()
-    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, 1, C.byref(h)))
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, FORMS[dtype], C.byref(h)))
+    assert ctx.L.ps_hip_dense_form(h) == (hip.DENSE_F32 if odd_weights else FORMS[dtype])
     dx, do = ctx.to_device(x), ctx.empty((T, N))
     ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, h, dx.ptr, T, do.ptr, 2.0 ** -8))
     got = do.numpy()
@@ -313,6 +318,27 @@ def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights):
     assert np.all(np.isinf(got[beyond & np.isfinite(want)]))
     ctx.L.ps_hip_dense_free(ctx.h, h)
     dx.free(); do.free()
+
+
+# a float32 model in either form of its matrices: four mixes, several mixers' projections, the latent's window, experts; a joint projection of two mixers; portions and single tokens
+@pytest.mark.parametrize("dtype", ["float32", "float32 lines"])
+@pytest.mark.parametrize("which", ["mixes", "experts", "joint"])
+def test_float32_models_in_either_form(ctx, tmp_path, which, dtype):
+    V = 40
+    if which == "mixes":
+        run, cfg = seq_oracle.run, synth.seq_config(128, V, [L("wkv", 192, heads=4, dim=32), L("latent_attention", 64, heads=4, dim=32, vdim=32, q_rank=64, kv_rank=64, mask={"size": 33}, scale=0.2,
+                                                                                             rot={"base": 100.0, "dims": 8}, rot_dim=16), L("delta", 64, heads=4, kv_heads=2, dim=32, vdim=32, conv=3)], taps=2)
+    elif which == "experts":
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(128, V, [synth.pupidra_layer("attention", synth.pupidra_attention(2, 1, 64, 64, 0.3, 9, 2), moe=(5, 2, 128, 1.7), shared=64)])
+    else:
+        run, cfg = seq_oracle.run_parallel, synth.parallel_config(128, V, [synth.parallel_layer(128, {"heads": 4, "kv_heads": 2, "dim": 32, "vdim": 32, "mask": {"size": 33, "pool": 3},
+                                                                  "rot": {"base": 100.0, "dims": 16}, "scale": 0.2}, {"heads": 4, "dim": 32, "vdim": 32, "tau": 4.0}, 1.0, 0.5)], taps=2)
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=300, n_slots=1, max_context=700, f32_form=FORMS[dtype])
+    assert {ctx.L.ps_hip_dense_form(w) for w in m._up.mats} == {FORMS[dtype]}
+    toks = tokens_for(cfg, 350)
+    assert err(run_portions(m, toks, (300, 1, 5, 44)), run(cfg, t, toks)) < TOL["float32"]
+    m.close()
 
 
 # 256 x 256 tiles behind an epilogue (k_dense.hip dense_mm_big_kernel): an activation whose rounded rows the second product reads, pairs, the four mixes of a token shift, the slots of experts (tiles
@@ -409,14 +435,14 @@ def test_dense_matmul_of_a_short_inner_size(ctx, dtype, T, N, K):
 
 # K a multiple of 128 up to 1024 and few tiles (k_dense.hip dense_mm_narrow_kernel): every number of steps per wave, a row and a column more and less than a tile, as many tiles as CUs and more
 # (the ring), one step more of K (the ring)
-@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dtype", list(FORMS))
 @pytest.mark.parametrize("T,N,K", [(9, 1, 128), (33, 31, 256), (31, 33, 384), (32, 64, 512), (65, 40, 640), (12, 100, 768), (40, 65, 896), (64, 129, 1024), (256, 1024, 512), (257, 1024, 512), (9, 70, 1152)])
 def test_dense_matmul_of_few_tiles(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
 
 
 # two to eight tokens on the wide mat-mul (ps_seq.h PSD_FEW): the narrow tiles, the ring with and without a split along K, and the mat-vec where K is no whole 128 bytes (the same bound)
-@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dtype", list(FORMS))
 @pytest.mark.parametrize("T,N,K", [(2, 1, 64), (3, 33, 128), (4, 129, 1024), (5, 70, 4160), (8, 2100, 192), (7, 65, 2048), (2, 300, 72), (8, 40, 1056)])
 def test_dense_matmul_of_a_few_tokens(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
@@ -470,7 +496,7 @@ def test_dense_matvec_with_an_infinite_weight(ctx, dtype, N, K, T):
 
 
 # the scratch that a product of many rows takes belongs to the context and stays: it has a bound, and the product goes through it piece by piece
-@pytest.mark.parametrize("dtype,T,N,K", [("bfloat16", 40000, 24, 2048), ("float32", 20001, 24, 2048), ("bfloat16", 1100000, 8, 16)])
+@pytest.mark.parametrize("dtype,T,N,K", [("bfloat16", 40000, 24, 2048), ("float32", 20001, 24, 2048), ("float32 lines", 20001, 24, 2048), ("bfloat16", 1100000, 8, 16)])
 def test_dense_matmul_scratch_is_bounded(free_bytes, dtype, T, N, K):
     import ctypes as C
     own = hip.Ctx(0)
@@ -478,14 +504,14 @@ def test_dense_matmul_scratch_is_bounded(free_bytes, dtype, T, N, K):
     bits = f32_to_bf16_bits(rng.standard_normal((N, K), dtype=np.float32))
     x = rng.standard_normal((64, K), dtype=np.float32)[np.arange(T) % 61]  # (61 different rows)
     h = C.c_void_p()
-    own.check(own.L.ps_hip_dense_upload(own.h, bits.ctypes.data_as(C.c_void_p), N, K, int(dtype == "float32"), C.byref(h)))
+    own.check(own.L.ps_hip_dense_upload(own.h, bits.ctypes.data_as(C.c_void_p), N, K, FORMS[dtype], C.byref(h)))
     dx, do = own.to_device(x), own.to_device(np.zeros((T, N), np.float32))
     before = free_bytes()
     own.check(own.L.ps_hip_dense_matmul(own.h, h, dx.ptr, T, do.ptr, 1.0))
     got = do.numpy()
     assert before - free_bytes() <= 100 << 20  # 64 MiB of rows, 32 MiB of parts of split products
     w = (bits.astype(np.uint32) << 16).view(np.float32).reshape(N, K).astype(np.float64)
-    a = (x[:61] if dtype == "float32" else (f32_to_bf16_bits(x[:61]).astype(np.uint32) << 16).view(np.float32).reshape(61, K)).astype(np.float64)
+    a = ((f32_to_bf16_bits(x[:61]).astype(np.uint32) << 16).view(np.float32).reshape(61, K) if dtype == "bfloat16" else x[:61]).astype(np.float64)
     bound = K * 2.0 ** -24 * (np.abs(a) @ np.abs(w).T)
     assert np.all(np.abs(got - (a @ w.T)[np.arange(T) % 61]) <= bound[np.arange(T) % 61])
     own.L.ps_hip_dense_free(own.h, h)

@@ -86,6 +86,39 @@ m.decode_greedy(s, 19, 3)
 """.replace(".short", str(child.tmp / "short")))
 
 
+def test_the_form_of_float32_matrices_does_not_depend_on_what_is_free(child):
+    """ps_hip_dense_upload makes the form that it is asked for, and ps_hip_dense_f32_form chooses one by a model's size (tests/fake_hip.cpp: 1 GiB free of 288)"""
+    child("""
+ctx = hip.Ctx(0)
+lib = ctx.L
+bits = np.full((64, 64), 0x3f80, np.uint16)
+def upload(form):
+    h = C.c_void_p()
+    ctx.check(lib.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), 64, 64, form, C.byref(h)))
+    return h
+for form, want in ((hip.DENSE_BF16, hip.DENSE_BF16), (hip.DENSE_F32, hip.DENSE_F32), (hip.DENSE_F32_LINES, hip.DENSE_F32_LINES), (7, hip.DENSE_F32), (-1, hip.DENSE_F32)):
+    fake.fake_reset()
+    h = upload(form)
+    assert lib.ps_hip_dense_form(h) == want and count("hipMemGetInfo") == 0, form
+    lib.ps_hip_dense_free(ctx.h, h)
+for name in ("hipMemcpyAsync", "hipStreamSynchronize", "hipMalloc"):
+    for nth in (1, 2):
+        fake.fake_reset()
+        fail(name, nth)
+        if (name, nth) != ("hipStreamSynchronize", 2): refused(lambda: upload(hip.DENSE_F32_LINES))
+for numbers, want in ((0, hip.DENSE_F32_LINES), (18 << 30, hip.DENSE_F32_LINES), ((18 << 30) + 1, hip.DENSE_F32), (1 << 50, hip.DENSE_F32)):
+    assert lib.ps_hip_dense_f32_form(ctx.h, numbers) == want, numbers
+fail("hipMemGetInfo")
+assert lib.ps_hip_dense_f32_form(ctx.h, 1) == hip.DENSE_F32
+cfg = synth.seq_config(64, 30, [L("wkv", None, heads=1, dim=64)], taps=3)
+synth.write_seq_model_dir(".dir", cfg, 1)
+for dtype, form, want in (("bfloat16", None, hip.DENSE_BF16), ("float32", None, hip.DENSE_F32_LINES), ("float32", hip.DENSE_F32, hip.DENSE_F32), ("bfloat16", hip.DENSE_F32, hip.DENSE_BF16)):
+    m = seqmodel.SeqModel(ctx, ".dir", dtype=dtype, max_batch=8, f32_form=form)
+    assert {lib.ps_hip_dense_form(w) for w in m._up.mats} == {want}, (dtype, form)
+    m.close()
+""".replace(".dir", str(child.tmp / "dir")))
+
+
 def test_a_model_without_room_for_wide_launch_sequences(child):
     """ps_hip_seq_create: launch sequences of four times max_batch where the memory is there, of max_batch where it is not; more wanted rows than the head takes at a time go in groups"""
     child("""
