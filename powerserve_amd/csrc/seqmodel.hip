@@ -444,10 +444,15 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
                         if (P.side->d.in_bias) ok = ok && hipMemcpyAsync(bias + a->N + skip, P.side->d.in_bias, (size_t)b->N * 4, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
                     }
                 }
-                if (ok && a->half && b->half && (ok = alloc(&j->half, (na + nz + nb) / 2))) {
-                    psk_fill(c->stream, (float *)j->half, 0.f, (int64_t)((na + nz) / 8 + 1));
-                    ok = hipMemcpyAsync(j->half, a->half, na / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess &&
-                         hipMemcpyAsync((char *)j->half + (na + nz) / 2, b->half, nb / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
+                if (ok && a->half && b->half) {
+                    if (alloc(&j->half, (na + nz + nb) / 2)) {
+                        psk_fill(c->stream, (float *)j->half, 0.f, (int64_t)((na + nz) / 8 + 1));
+                        ok = hipMemcpyAsync(j->half, a->half, na / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess &&
+                             hipMemcpyAsync((char *)j->half + (na + nz) / 2, b->half, nb / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
+                    } else { // (its products run on the fp32 instruction)
+                        j->half = nullptr;
+                        (void)hipGetLastError();
+                    }
                 }
                 ok = ok && hipStreamSynchronize(c->stream) == hipSuccess;
                 it = joint_of.emplace(P.layer, std::make_pair((const ps_dense *)j, (const float *)bias)).first;
@@ -544,6 +549,7 @@ int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) 
         (void)hipGetLastError();
         rc = seq_create(c, desc, desc->max_batch, out);
     }
+    if (rc) (void)hipGetLastError(); // (the error is this call's, not the next one's)
     return rc == SEQ_NO_MEMORY ? 2 : rc;
 }
 

@@ -119,6 +119,36 @@ for dtype, form, want in (("bfloat16", None, hip.DENSE_BF16), ("float32", None, 
 """.replace(".dir", str(child.tmp / "dir")))
 
 
+def test_a_joint_projection_without_room_for_its_second_form(child):
+    """ps_hip_seq_create: of all the memory a float32 model asks for, the bfloat16 form of two mixers' joint projection is the one piece that it can do without; its products then run as fp32 ones"""
+    child("""
+ctx = hip.Ctx(0)
+att = {"heads": 2, "kv_heads": 1, "dim": 32, "vdim": 32, "mask": {"size": 9, "pool": 3}, "rot": {"base": 100.0, "dims": 8}, "scale": 0.2}
+cfg = synth.parallel_config(64, 30, [synth.parallel_layer(None, att, {"heads": 2, "dim": 32, "vdim": 32, "tau": 4.0}, 1.0, 0.5)], taps=2)
+synth.write_seq_model_dir(".dir", cfg, 1)
+def load(): return seqmodel.SeqModel(ctx, ".dir", dtype="float32", max_batch=8)
+fake.fake_reset()
+load().close()
+took = []
+for n in range(1, count("hipMalloc") + 1):
+    fake.fake_reset()
+    fail("hipMalloc", n)
+    try: m = load()
+    except hip.PSHipError: continue
+    s = m.acquire()
+    fake.fake_reset()
+    m.forward(s, [1] * 8, want=[7])
+    took.append((count("dense_mm_ring_kernelIf"), count("hipLaunchKernel") > 0, fake.fake_stray()))
+    m.close()
+assert took == [(1, True, 0)], took
+m = load()
+s = m.acquire()
+fake.fake_reset()
+m.forward(s, [1] * 8, want=[7])
+assert count("dense_mm_ring_kernelIf") == 0 and count("dense_mm_ring_kernelIt") > 0
+""".replace(".dir", str(child.tmp / "dir")))
+
+
 def test_a_model_without_room_for_wide_launch_sequences(child):
     """ps_hip_seq_create: launch sequences of four times max_batch where the memory is there, of max_batch where it is not; more wanted rows than the head takes at a time go in groups"""
     child("""
