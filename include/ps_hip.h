@@ -462,8 +462,9 @@ typedef struct ps_seq_layer_s {
 typedef struct {
     int32_t n_layers, width, vocab, canon_taps;
     int32_t max_batch;   /* tokens the step function is asked for at a time, and most rows of logits it makes at a time.  A longer input is cut into launch sequences of this size, or (from 64 on)
-                          * of up to four times as many tokens, no more than 2048 or max_context, where the memory for that is there */
-    int32_t n_slots;     /* sequence states held at once */
+                          * of four times or twice as many tokens, no more than 2048 or max_context, where what that takes in memory is at most a 64th of the device's (ps_hip_seq_create_sized
+                          * sets the size).  Buffers grow by the token, and every slot by a row per token of every attention layer's ring */
+    int32_t n_slots;     /* sequence states held at once, each with rings of window - 1 + (tokens of a launch sequence) rows */
     int32_t compute;     /* 0: bfloat16 matrix products, 1: fp32 */
     float norm_eps, norm_offset /* weight applied as (offset + w) */, logit_scale;
     const ps_dense *embed, *head; /* [vocab, width] both */
@@ -487,6 +488,9 @@ typedef struct {
 } ps_seq_desc;
 
 int ps_hip_seq_create(ps_hip_ctx *ctx, const ps_seq_desc *desc, ps_hip_seq **out);
+/* The same with launch sequences of launch_rows tokens (max_batch or more; 0: as ps_hip_seq_create).  launch_rows = max_batch takes the least memory: nothing beyond what max_batch tokens need. */
+int ps_hip_seq_create_sized(ps_hip_ctx *ctx, const ps_seq_desc *desc, int launch_rows, ps_hip_seq **out);
+int ps_hip_seq_launch_rows(const ps_hip_seq *m); /* tokens of its launch sequences */
 void ps_hip_seq_destroy(ps_hip_seq *m);
 /* State manager: a slot holds everything a sequence carries from token to token (convolution tails, token-shift rows,
  * recurrent states, the latent ring) and its position.  acquire hands out a zeroed slot at position 0 (-1 in *slot and a

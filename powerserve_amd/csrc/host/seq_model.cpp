@@ -781,7 +781,7 @@ bool is_seq_model_dir(const std::string &dir) {
 }
 
 // ---------------------------------------------------------------- the model
-SeqModel::SeqModel(const std::string &model_dir, const std::string &dtype, int device, size_t max_batch, int n_slots, int max_context) {
+SeqModel::SeqModel(const std::string &model_dir, const std::string &dtype, int device, size_t max_batch, int n_slots, int max_context, int launch_rows) {
     if (dtype != "bfloat16" && dtype != "float32") POWERSERVE_ABORT("dtype " + dtype + ": bfloat16 or float32");
     JsonValue cfg;
     try { cfg = JsonValue::parse_file(model_dir + "/config.json"); } catch (const std::exception &e) { POWERSERVE_ABORT(std::string("config.json: ") + e.what()); }
@@ -804,7 +804,7 @@ SeqModel::SeqModel(const std::string &model_dir, const std::string &dtype, int d
     d.compute = dtype == "float32";
     d.max_context = max_context;
     d.layers = layers.data();
-    hip_ok(m_ctx, ps_hip_seq_create(m_ctx, &d, &m_h), "ps_hip_seq_create");
+    hip_ok(m_ctx, ps_hip_seq_create_sized(m_ctx, &d, launch_rows, &m_h), "ps_hip_seq_create_sized");
     vocab = (uint32_t)d.vocab; width = (uint32_t)d.width; n_layers = (uint32_t)d.n_layers;
 }
 SeqModel::~SeqModel() {
@@ -847,9 +847,9 @@ std::vector<Token> SeqModel::generate(const std::vector<Token> &prompt, int step
     release(slot);
     return out;
 }
-auto load_seq_model(const std::string &model_dir, const std::string &dtype, int device, size_t max_batch, int n_slots, int max_context) -> std::shared_ptr<SeqModel> {
+auto load_seq_model(const std::string &model_dir, const std::string &dtype, int device, size_t max_batch, int n_slots, int max_context, int launch_rows) -> std::shared_ptr<SeqModel> {
     if (!is_seq_model_dir(model_dir)) POWERSERVE_ABORT(model_dir + ": config.json + model.safetensors expected");
-    return std::make_shared<SeqModel>(model_dir, dtype, device, max_batch, n_slots, max_context);
+    return std::make_shared<SeqModel>(model_dir, dtype, device, max_batch, n_slots, max_context, launch_rows);
 }
 
 } // namespace powerserve

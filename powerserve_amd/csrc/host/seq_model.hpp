@@ -50,7 +50,7 @@ struct SeqUploader {
 };
 
 struct SeqModel {
-    SeqModel(const std::string &model_dir, const std::string &dtype, int device, size_t max_batch, int n_slots, int max_context = 0);
+    SeqModel(const std::string &model_dir, const std::string &dtype, int device, size_t max_batch, int n_slots, int max_context = 0, int launch_rows = 0); // launch_rows: ps_hip_seq_create_sized
     ~SeqModel();
     SeqModel(const SeqModel &) = delete;
     int acquire();
@@ -74,6 +74,6 @@ using SeqArchitecture = std::function<void(const JsonValue &cfg, const SafeTenso
 const std::map<std::string, SeqArchitecture> &seq_architectures();
 bool is_seq_model_dir(const std::string &model_dir);
 auto load_seq_model(const std::string &model_dir, const std::string &dtype = "bfloat16", int device = 0, size_t max_batch = 256, int n_slots = 2,
-                    int max_context = 0) -> std::shared_ptr<SeqModel>;
+                    int max_context = 0, int launch_rows = 0) -> std::shared_ptr<SeqModel>;
 
 } // namespace powerserve

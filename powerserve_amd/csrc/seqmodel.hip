@@ -109,9 +109,16 @@ static uint64_t dense_bytes(const ps_dense *w) { return w ? (uint64_t)w->N * w->
 // the fewer partly empty ones of an expert, and the fewer expansions of one window's keys: Ranutar 2048 x 6, 2047 tokens behind max_batch 512 in portions of 512, 1024, 2048: 5552, 4527,
 // 3947 us; Pupidra 2048 x 6, 1500 tokens: 6118, 5060, 4280.  Not below 64, where the caller has asked for little memory; no more than four times what was asked for, and no more than
 // 2048, behind which the tiles fill the chip anyway.
-static int64_t seq_rows(const ps_seq_desc *d) {
+static int64_t seq_rows(const ps_seq_desc *d, int times) {
     const int64_t B = d->max_batch, most = d->max_context > 0 ? d->max_context : 65536;
-    return B < 64 ? B : std::max(B, std::min<int64_t>({4 * B, 2048, most}));
+    return B < 64 ? B : std::max(B, std::min<int64_t>({times * B, 2048, most}));
+}
+// What such a width may take beyond the memory of launch sequences of max_batch tokens (buffers by the token, and every ring of every slot longer by as many rows), and what the split attention's
+// images may: a 64th of the device's memory (4.5 GB), however much of it is free -- a model runs the same way whatever is beside it.
+static size_t seq_spare() {
+    size_t free = 0, all = 0;
+    if (hipMemGetInfo(&free, &all) != hipSuccess) { (void)hipGetLastError(); return 0; }
+    return all / 64;
 }
 
 // out of memory: the one failure that a narrower launch sequence may mend
@@ -119,7 +126,8 @@ static const int SEQ_NO_MEMORY = -1;
 
 extern "C" {
 
-static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, ps_hip_seq **out) {
+// bytes given: nothing is made, only the device memory counted that it would take
+static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, const size_t spare, ps_hip_seq **out, size_t *bytes = nullptr) {
     auto m = new ps_hip_seq();
     m->ctx = c;
     m->d = *desc;
@@ -387,11 +395,17 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
     for (auto &P : m->L)
         if (P.owner >= 0) { const LayerPlan &O = m->L[P.owner]; P.off_ring = O.off_ring; P.off_pool = O.off_pool; P.cap = O.cap; }
     m->state_floats = off;
-    auto alloc = [&](void **p, size_t bytes) {
-        if (hipMalloc(p, bytes + 256) != hipSuccess) return false;
+    size_t counted = 0;
+    auto alloc = [&](void **p, size_t n) {
+        counted += n + 256;
+        if (bytes) return true;
+        if (hipMalloc(p, n + 256) != hipSuccess) return false;
         m->owned.push_back(*p);
         return true;
     };
+    auto fill = [&](void *p, int64_t n) { if (!bytes) psk_fill(c->stream, (float *)p, 0.f, n); }; // zeros
+    auto copy = [&](void *to, const void *from, size_t n, hipMemcpyKind kind = hipMemcpyDeviceToDevice) { return bytes || hipMemcpyAsync(to, from, n, kind, c->stream) == hipSuccess; };
+    auto there = [&]() { return bytes || hipStreamSynchronize(c->stream) == hipSuccess; };
     bool ok = true;
     std::map<const void *, float *> freq_of; // one table per layer (keyed by its output matrix), shared by its runs
     mixers([&](LayerPlan &P) {
@@ -414,7 +428,7 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
             }
         }
         ok = ok && alloc((void **)&P.freq, half * 4);
-        if (ok) ok = hipMemcpyAsync(P.freq, f.data(), half * 4, hipMemcpyHostToDevice, c->stream) == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess;
+        if (ok) ok = copy(P.freq, f.data(), half * 4, hipMemcpyHostToDevice) && there();
         freq_of[P.d.out] = P.freq;
     });
     {
@@ -432,29 +446,27 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
                 m->joints.push_back(j);
                 j->dtype = a->dtype; j->N = a->N + skip + b->N; j->K = a->K;
                 ok = ok && alloc(&j->data, na + nz + nb);
-                if (ok) psk_fill(c->stream, (float *)j->data, 0.f, (int64_t)((na + nz) / 4));
-                ok = ok && hipMemcpyAsync(j->data, a->data, na, hipMemcpyDeviceToDevice, c->stream) == hipSuccess &&
-                     hipMemcpyAsync((char *)j->data + na + nz, b->data, nb, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
+                if (ok) fill(j->data, (na + nz) / 4);
+                ok = ok && copy(j->data, a->data, na) && copy((char *)j->data + na + nz, b->data, nb);
                 float *bias = nullptr;
                 if (ok && (P.d.in_bias || P.side->d.in_bias)) {
                     ok = alloc((void **)&bias, (size_t)j->N * 4);
                     if (ok) {
-                        psk_fill(c->stream, bias, 0.f, j->N);
-                        if (P.d.in_bias) ok = ok && hipMemcpyAsync(bias, P.d.in_bias, (size_t)a->N * 4, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
-                        if (P.side->d.in_bias) ok = ok && hipMemcpyAsync(bias + a->N + skip, P.side->d.in_bias, (size_t)b->N * 4, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
+                        fill(bias, j->N);
+                        if (P.d.in_bias) ok = ok && copy(bias, P.d.in_bias, (size_t)a->N * 4);
+                        if (P.side->d.in_bias) ok = ok && copy(bias + a->N + skip, P.side->d.in_bias, (size_t)b->N * 4);
                     }
                 }
                 if (ok && a->half && b->half) {
                     if (alloc(&j->half, (na + nz + nb) / 2)) {
-                        psk_fill(c->stream, (float *)j->half, 0.f, (int64_t)((na + nz) / 8 + 1));
-                        ok = hipMemcpyAsync(j->half, a->half, na / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess &&
-                             hipMemcpyAsync((char *)j->half + (na + nz) / 2, b->half, nb / 2, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
+                        fill(j->half, (na + nz) / 8 + 1);
+                        ok = copy(j->half, a->half, na / 2) && copy((char *)j->half + (na + nz) / 2, b->half, nb / 2);
                     } else { // (its products run on the fp32 instruction)
                         j->half = nullptr;
                         (void)hipGetLastError();
                     }
                 }
-                ok = ok && hipStreamSynchronize(c->stream) == hipSuccess;
+                ok = ok && there();
                 it = joint_of.emplace(P.layer, std::make_pair((const ps_dense *)j, (const float *)bias)).first;
             }
             P.joint = it->second.first; P.joint_bias = it->second.second;
@@ -526,7 +538,12 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
             if ((lat || win) && psk_split_attn_ok(P.d.dim, lat ? P.d.rot_dim : 0, P.d.vdim) && psk_split_attn_takes((int)B, P.d.heads))
                 sa = std::max(sa, psk_split_attn_scratch(lat ? P.d.heads : P.d.kv_heads, P.d.dim, lat ? P.d.rot_dim : 0, P.d.vdim, win ? P.pool_rows : 0, P.d.window - 1 + B));
         });
-        if (sa && !alloc(&m->sa_scratch, sa)) (void)hipGetLastError();
+        if (sa && sa <= spare && !alloc(&m->sa_scratch, sa)) (void)hipGetLastError();
+    }
+    if (bytes) {
+        *bytes = counted;
+        ps_hip_seq_destroy(m);
+        return 0;
     }
     if (!ok) {
         fail("out of device memory");
@@ -536,18 +553,29 @@ static int seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, const int64_t B, p
     return 0;
 }
 
-int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) {
+int ps_hip_seq_create(ps_hip_ctx *c, const ps_seq_desc *desc, ps_hip_seq **out) { return ps_hip_seq_create_sized(c, desc, 0, out); }
+int ps_hip_seq_launch_rows(const ps_hip_seq *m) { return (int)m->rows; }
+
+int ps_hip_seq_create_sized(ps_hip_ctx *c, const ps_seq_desc *desc, int launch_rows, ps_hip_seq **out) {
     *out = nullptr;
     if (!desc || desc->n_layers <= 0 || desc->width <= 0 || desc->vocab <= 0 || desc->max_batch <= 0 || desc->n_slots <= 0 || desc->canon_taps < 1)
         return seq_fail(c, "seq_create: bad descriptor");
     if (!desc->embed || !desc->head || !desc->final_norm) return seq_fail(c, "seq_create: embed / head / final_norm missing");
     if (desc->embed->K != desc->width || desc->head->K != desc->width || desc->head->N != desc->vocab) return seq_fail(c, "seq_create: embed / head shape");
+    if (launch_rows != 0 && launch_rows < desc->max_batch) return seq_fail(c, "seq_create: launch_rows below max_batch");
     PS_CHECK(c, hipSetDevice(c->device));
-    const int64_t rows = seq_rows(desc);
-    int rc = seq_create(c, desc, rows, out);
-    if (rc == SEQ_NO_MEMORY && rows > desc->max_batch) {
+    const size_t spare = seq_spare();
+    int64_t rows = launch_rows ? launch_rows : desc->max_batch;
+    if (!launch_rows && seq_rows(desc, 4) > desc->max_batch) {
+        size_t narrow = 0, wide = 0;
+        if (const int rc = seq_create(c, desc, desc->max_batch, spare, nullptr, &narrow)) return rc;
+        for (int times = 4; rows == desc->max_batch && times > 1; times -= 2)
+            if (seq_create(c, desc, seq_rows(desc, times), spare, nullptr, &wide) == 0 && wide <= narrow + spare) rows = seq_rows(desc, times);
+    }
+    int rc = seq_create(c, desc, rows, spare, out);
+    if (rc == SEQ_NO_MEMORY && !launch_rows && rows > desc->max_batch) {
         (void)hipGetLastError();
-        rc = seq_create(c, desc, desc->max_batch, out);
+        rc = seq_create(c, desc, desc->max_batch, spare, out);
     }
     if (rc) (void)hipGetLastError(); // (the error is this call's, not the next one's)
     return rc == SEQ_NO_MEMORY ? 2 : rc;

@@ -35,7 +35,7 @@ EXPORTS = [
     "ps_hip_model_forward", "ps_hip_model_decode_greedy", "ps_hip_model_logits", "ps_hip_model_scratch", "ps_hip_model_k_cache",
     "ps_hip_model_v_cache", "ps_hip_model_weight_bytes_per_token", "ps_hip_model_set_mode", "ps_hip_model_bench_gemv", "ps_hip_model_bench_matmul", "ps_hip_debug_timeline", "ps_hip_last_matmul_kernel", "ps_hip_debug_set", "ps_hip_debug_f16_gemm", "ps_hip_model_forward_tree", "ps_hip_model_prefill", "ps_hip_model_forward_lowered", "ps_hip_model_sync_check", "ps_hip_model_kv_mask",
     "ps_hip_soft_max", "ps_hip_model_kv_copy", "ps_hip_model_kv_save_tokens", "ps_hip_model_kv_unmask_tokens", "ps_hip_model_kv_append_tokens", "ps_hip_model_argmax",
-    "ps_hip_dense_upload", "ps_hip_dense_free", "ps_hip_dense_matmul", "ps_hip_dense_f32_form", "ps_hip_dense_form", "ps_hip_seq_create", "ps_hip_seq_destroy", "ps_hip_seq_acquire", "ps_hip_seq_release",
+    "ps_hip_dense_upload", "ps_hip_dense_free", "ps_hip_dense_matmul", "ps_hip_dense_f32_form", "ps_hip_dense_form", "ps_hip_seq_create", "ps_hip_seq_create_sized", "ps_hip_seq_launch_rows", "ps_hip_seq_destroy", "ps_hip_seq_acquire", "ps_hip_seq_release",
     "ps_hip_seq_position", "ps_hip_seq_slot_bytes", "ps_hip_seq_layer_runs", "ps_hip_seq_forward", "ps_hip_seq_decode_greedy", "ps_hip_seq_debug_layers", "ps_hip_seq_set_mode",
     "ps_hip_seq_weight_bytes_per_token", "ps_hip_seq_bench_kernel",
 ]
@@ -173,6 +173,7 @@ def lib(seq_only_ok: bool = False) -> C.CDLL:
         "ps_hip_debug_f16_gemm": (i32, [vp, i32, C.c_int64, C.c_int64, i32, C.c_float, C.POINTER(C.c_double), C.POINTER(C.c_double)]),
         "ps_hip_dense_upload": (i32, [vp, vp, i64, i64, i32, C.POINTER(vp)]), "ps_hip_dense_free": (None, [vp, vp]),
         "ps_hip_dense_matmul": (i32, [vp, vp, vp, i32, vp, C.c_float]), "ps_hip_dense_f32_form": (i32, [vp, C.c_uint64]), "ps_hip_dense_form": (i32, [vp]),
+        "ps_hip_seq_create_sized": (i32, [vp, C.POINTER(SeqDesc), i32, C.POINTER(vp)]), "ps_hip_seq_launch_rows": (i32, [vp]),
         "ps_hip_seq_create": (i32, [vp, C.POINTER(SeqDesc), C.POINTER(vp)]), "ps_hip_seq_destroy": (None, [vp]),
         "ps_hip_seq_acquire": (i32, [vp, C.POINTER(i32)]), "ps_hip_seq_release": (i32, [vp, i32]), "ps_hip_seq_position": (i64, [vp, i32]),
         "ps_hip_seq_slot_bytes": (sz, [vp]), "ps_hip_seq_layer_runs": (i32, [vp]), "ps_hip_seq_forward": (i32, [vp, i32, vp, i32, vp, i32, vp, vp]),

@@ -628,16 +628,18 @@ class _Uploader:
 class SeqModel:
     """ps_hip_seq over a model directory.  dtype "bfloat16": matrix products on bfloat16 operands, fp32 accumulation; "float32": fp32
     throughout.  f32_form: the form of a float32 model's matrices (hip.DENSE_F32 / DENSE_F32_LINES; None: by the model's size,
-    ps_hip_dense_f32_form).  Sequences live in slots (acquire / release); forward() is the step function, generate() the greedy / sampled loop."""
+    ps_hip_dense_f32_form).  launch_rows: tokens of a launch sequence (0: max_batch to four times as many, ps_hip_seq_create; max_batch takes the
+    least memory).  Sequences live in slots (acquire / release); forward() is the step function, generate() the greedy / sampled loop."""
 
-    def __init__(self, ctx: hip.Ctx, model_dir: str, dtype: str = "bfloat16", max_batch: int = 256, n_slots: int = 2, max_context: int = 0, f32_form: int | None = None):
+    def __init__(self, ctx: hip.Ctx, model_dir: str, dtype: str = "bfloat16", max_batch: int = 256, n_slots: int = 2, max_context: int = 0, f32_form: int | None = None,
+                 launch_rows: int = 0):
         if dtype not in ("bfloat16", "float32"):
             raise ConfigError(f"dtype {dtype!r}: bfloat16 or float32")
         self.ctx, self.dtype = ctx, dtype
         self.cfg = read_config(model_dir)
         self.arch = self.cfg["architecture"]
         st = SafeTensors(os.path.join(model_dir, "model.safetensors"))
-        if f32_form is None:
+        if dtype == "float32" and f32_form is None:
             f32_form = int(ctx.L.ps_hip_dense_f32_form(ctx.h, sum(int(np.prod(st.shape(n))) for n in st.names())))
         self._up = _Uploader(ctx, f32_form if dtype == "float32" else hip.DENSE_BF16)
         layers, top = ARCHITECTURES[self.arch](self.cfg, st, self._up)
@@ -651,7 +653,7 @@ class SeqModel:
         d.layers = self._layers
         self.vocab, self.width, self.n_layers, self.max_batch = d.vocab, d.width, d.n_layers, int(max_batch)
         h = C.c_void_p()
-        ctx.check(ctx.L.ps_hip_seq_create(ctx.h, C.byref(d), C.byref(h)))
+        ctx.check(ctx.L.ps_hip_seq_create_sized(ctx.h, C.byref(d), int(launch_rows), C.byref(h)))
         self.h = h
         self.n_runs = int(ctx.L.ps_hip_seq_layer_runs(h))  # executions of a layer per forward (a looped stretch counts every time)
         self._dbg = None
@@ -678,6 +680,10 @@ class SeqModel:
 
     def position(self, slot: int) -> int:
         return int(self.ctx.L.ps_hip_seq_position(self.h, int(slot)))
+
+    @property
+    def launch_rows(self) -> int:
+        return int(self.ctx.L.ps_hip_seq_launch_rows(self.h))
 
     @property
     def slot_bytes(self) -> int:

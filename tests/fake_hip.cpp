@@ -14,7 +14,7 @@ std::map<char *, Alloc> mem;
 std::map<std::string, int> count, fail, blocks;
 std::map<const void *, std::string> kernels;
 int current = 0;
-size_t stray = 0;
+size_t stray = 0, memory = (size_t)288 << 30;
 hipError_t last = hipSuccess;
 struct Thing { int device; }; // a stream or an event
 using Graph = std::vector<std::string>; // the kernels' names
@@ -56,6 +56,12 @@ int fake_count(const char *name) { // (of every name with this in it: a kernel's
     return n;
 }
 size_t fake_stray() { return stray; }
+void fake_memory(size_t bytes) { memory = bytes; } // the device's memory in all
+size_t fake_held() { // device memory that is allocated
+    size_t n = 0;
+    for (auto &a : mem) n += a.second.type == hipMemoryTypeDevice ? a.second.bytes : 0;
+    return n;
+}
 int fake_blocks(const char *name) { // work-groups of the last launch of such a kernel
     for (auto &b : blocks)
         if (b.first.find(name) != std::string::npos) return b.second;
@@ -113,7 +119,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
     const hipError_t e = call("hipMalloc");
     return e != hipSuccess ? e : alloc(p, bytes, hipMemoryTypeDevice);
 }
-hipError_t hipMemGetInfo(size_t *free, size_t *all) { *free = (size_t)1 << 30; *all = (size_t)288 << 30; return call("hipMemGetInfo"); }
+hipError_t hipMemGetInfo(size_t *free, size_t *all) { *free = (size_t)1 << 30; *all = memory; return call("hipMemGetInfo"); }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return call("hipHostMalloc") ? hipErrorUnknown : alloc(p, bytes, hipMemoryTypeHost); }
 hipError_t hipFree(void *p) { mem.erase((char *)p); free(p); return hipSuccess; }
 hipError_t hipHostFree(void *p) { return hipFree(p); }

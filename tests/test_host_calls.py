@@ -13,7 +13,8 @@ PRELUDE = """
 import ctypes as C, sys
 import numpy as np
 fake = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
-fake.fake_stray.restype = C.c_size_t
+fake.fake_stray.restype = fake.fake_held.restype = C.c_size_t
+fake.fake_memory.argtypes = [C.c_size_t]
 from powerserve_amd import hip, seqmodel, synth
 def fail(name, n=1): fake.fake_fail(name.encode(), n)
 def count(name): return fake.fake_count(name.encode())
@@ -169,6 +170,63 @@ for n in (0, 1, 7): # (the last ones are the model's own)
     m.forward(s, toks, want=want)
     assert count("seq_set_step_kernel") == 5 and count("dense_argmax_kernel") == 5 and m.position(s) == 300 and fake.fake_stray() == 0
 """)
+
+
+def test_what_wide_launch_sequences_may_take(child):
+    """ps_hip_seq_create: four times max_batch tokens where that takes at most a 64th of the device's memory beyond what max_batch does, else twice as many, else max_batch; the rings of all slots are
+    part of it.  ps_hip_seq_create_sized makes the size that it is asked for"""
+    child("""
+ctx = hip.Ctx(0)
+cfg = synth.seq_config(24, 30, [L("latent_attention", 20, heads=2, dim=8, vdim=8, q_rank=8, kv_rank=16, rot={"base": 1e4, "dims": 8}, rot_dim=8, mask={"size": 9}, scale=0.3), L("wkv", None, heads=3, dim=8)], taps=3)
+synth.write_seq_model_dir(".dir", cfg, 1)
+def load(slots=2, rows=0, batch=64, context=0):
+    m = seqmodel.SeqModel(ctx, ".dir", max_batch=batch, n_slots=slots, launch_rows=rows, max_context=context)
+    held, r, slot = fake.fake_held(), m.launch_rows, m.slot_bytes
+    s = m.acquire()
+    fake.fake_reset()
+    m.forward(s, [1] * 300, want=[0, 299])
+    assert count("seq_set_step_kernel") == -(-300 // r) and fake.fake_stray() == 0
+    m.close()
+    return r, held, slot
+bytes_ = {(n, r): load(n, r) for n in (2, 40) for r in (64, 128, 256)}
+for (n, r), (rows, held, slot) in bytes_.items(): assert rows == r and slot - bytes_[n, 64][2] == (r - 64) * (16 + 8) * 4
+for n in (2, 40):
+    extra = {r: bytes_[n, r][1] - bytes_[n, 64][1] for r in (128, 256)}
+    for spare, want in ((extra[256], 256), (extra[256] - 1, 128), (extra[128], 128), (extra[128] - 1, 64), (0, 64)):
+        fake.fake_memory(64 * spare)
+        assert load(n)[0] == want, (n, spare)
+        for r in (64, 128, 256, 200): assert load(n, r)[0] == r
+fake.fake_memory(288 << 30)
+fake.fake_reset()
+fail("hipMemGetInfo")
+assert load()[0] == 64
+for batch, context, want in ((63, 0, 63), (64, 400, 256), (128, 400, 400), (600, 0, 2048), (3000, 0, 3000)): assert load(batch=batch, context=context)[0] == want, batch
+assert "launch_rows" in refused(lambda: load(rows=63))
+""".replace(".dir", str(child.tmp / "dir")))
+
+
+def test_images_of_the_split_attention_have_a_bound(child):
+    """a window of everything behind many heads: their images may take a 64th of the device's memory, beyond that the fp32 form attends"""
+    child("""
+ctx = hip.Ctx(0)
+cfg = synth.seq_config(64, 30, [L("latent_attention", None, heads=80, dim=128, vdim=128, q_rank=8, kv_rank=16, rot={"base": 1e4, "dims": 8}, rot_dim=64, mask={"size": 3000}, scale=0.3)], taps=1)
+synth.write_seq_model_dir(".dir", cfg, 1)
+def load():
+    m = seqmodel.SeqModel(ctx, ".dir", max_batch=128, n_slots=1, launch_rows=128, max_context=3000)
+    held, s = fake.fake_held(), m.acquire()
+    fake.fake_reset()
+    m.forward(s, [1] * 128)
+    took = count("split_attn_kernel"), count("latent_attn_mfma_kernel")
+    m.close()
+    return held, took
+with_, took = load()
+fake.fake_memory(0)
+without, plain = load()
+assert took == (1, 0) and plain == (0, 1) and with_ > without
+for spare, want in ((with_ - without, took), (with_ - without - 1 - 256, plain)):
+    fake.fake_memory(64 * spare)
+    assert load()[1] == want
+""".replace(".dir", str(child.tmp / "dir")))
 
 
 def test_copies_to_the_host_keep_their_error_cases(child):
