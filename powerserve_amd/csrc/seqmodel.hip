@@ -1267,15 +1267,18 @@ int ps_hip_seq_bench_kernel(ps_hip_seq *m, int which, int T, int reps, double *u
             if (!mv) psk_moe_plan(c->stream, m->moe_sel, S, rows, m->moe_seg, m->moe_list);
             g.groups = P.d.experts; g.g_sel = m->moe_sel;
             if (!mv) { g.g_seg = m->moe_seg; g.g_list = m->moe_list; }
-            if (which == 2) {
-                g.w = P.d.ff_up; g.a = m->h; g.lda = W; g.out = m->t4; g.ldo = P.d.ff; g.T = S; g.g_adiv = top;
-                g.act = P.d.ff_kind == PS_FF_MOE_RELU2 ? PSD_ACT_RELU2 : PSD_ACT_SILU_PAIR;
-                if (P.d.moe_weight_output) g.out_scale = m->moe_wgt;
-                else g.g_scale = m->moe_wgt;
-            } else {
-                g.w = P.d.ff_down; g.a = m->t4; g.lda = P.d.ff; g.ldo = W;
-                if (mv) { g.T = T; g.g_inner = top; g.out = m->y; }
-                else { g.T = S; g.out = top == 1 ? m->y : m->moe_y; }
+            psk_dense_args down = g; // (both products as seq_layers makes them)
+            g.w = P.d.ff_up; g.a = m->h; g.lda = W; g.out = m->t4; g.ldo = P.d.ff; g.T = S; g.g_adiv = top;
+            g.act = P.d.ff_kind == PS_FF_MOE_RELU2 ? PSD_ACT_RELU2 : PSD_ACT_SILU_PAIR;
+            if (P.d.moe_weight_output) g.out_scale = m->moe_wgt;
+            else g.g_scale = m->moe_wgt;
+            down.w = P.d.ff_down; down.a = m->t4; down.lda = P.d.ff; down.ldo = W;
+            if (mv) { down.T = T; down.g_inner = top; down.out = m->y; }
+            else { down.T = S; down.out = top == 1 ? m->y : m->moe_y; }
+            if (psk_dense_listed16(g) && psk_dense_listed16(down)) down.a16 = g.out16 = m->t4;
+            if (which == 3) {
+                psk_dense(c->stream, g); // (the rows that the second one reads)
+                g = down;
             }
             // what this routing makes a launch do: the slots that go to an expert with matrices (identity experts take none) and the matrices they touch
             std::vector<char> seen((size_t)P.d.experts, 0);

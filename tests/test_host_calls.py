@@ -229,6 +229,23 @@ for spare, want in ((with_ - without, took), (with_ - without - 1 - 256, plain))
 """.replace(".dir", str(child.tmp / "dir")))
 
 
+def test_the_measured_products_of_experts_are_the_ones_that_run(child):
+    """ps_hip_seq_bench_kernel: a portion's second product of the experts reads the rounded rows of the first one, in a step and where it is measured"""
+    child("""
+ctx = hip.Ctx(0)
+for ff in (128, 72): # (72: no whole blocks, the tiled kernel)
+    cfg = synth.pupidra_config(64, 30, [synth.pupidra_layer("attention", synth.pupidra_attention(2, 1, 16, 16, 0.3, 9, 2), moe=(5, 2, ff, 1.7), shared=None)])
+    synth.write_seq_model_dir(".dir", cfg, 1)
+    m = seqmodel.SeqModel(ctx, ".dir", max_batch=64)
+    us, by, fl = C.c_double(), C.c_double(), C.c_double()
+    def packed(which, reps):
+        fake.fake_reset()
+        ctx.check(ctx.L.ps_hip_seq_bench_kernel(m.h, which, 64, reps, C.byref(us), C.byref(by), C.byref(fl)))
+        return count("dense_pack_kernel")
+    for which, want in ((2, 1), (3, 0)): assert packed(which, 5) - packed(which, 2) == 3 * want, (ff, which)
+""".replace(".dir", str(child.tmp / "dir")))
+
+
 def test_copies_to_the_host_keep_their_error_cases(child):
     """ps_hip_memcpy_d2h: what a kernel could not read without a fault is left to the runtime's copy, whatever that says"""
     child("""
