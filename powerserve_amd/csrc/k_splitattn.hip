@@ -26,6 +26,7 @@ static __device__ __forceinline__ unsigned sa_round2(float a, float b) { // two 
     __builtin_memcpy(&u, &r, 4);
     return u;
 }
+static __device__ __forceinline__ bool sa_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
 // Two numbers as three pairs.  WIDE: any numbers -- one that rounds to infinity is cut off instead, infinity has no rest (weights of a soft-max are at most 1).
 template <bool WIDE>
 static __device__ __forceinline__ void sa_split2(float a, float b, unsigned &u1, unsigned &u2, unsigned &u3) {
@@ -50,6 +51,13 @@ static __device__ __forceinline__ void sa_split8(const float (&v)[8], sa_u4 (&p)
         unsigned a, b, c;
         sa_split2<WIDE>(v[2 * e], v[2 * e + 1], a, b, c);
         p[0][e] = a; p[1][e] = b; p[2][e] = c;
+    }
+}
+static __device__ __forceinline__ void sa_join8(const sa_u4 (&p)[3], float (&v)[8]) { // back (the sum is exact)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        auto line = [&](const int x) { return __uint_as_float(e & 1 ? p[x][e >> 1] & 0xffff0000u : p[x][e >> 1] << 16); };
+        v[e] = line(0) + (line(1) + line(2));
     }
 }
 static __device__ __forceinline__ sa_f4 sa_mfma(const sa_u4 &a, const sa_u4 &b, const sa_f4 &c) {
@@ -83,6 +91,7 @@ struct sa_keys {
     int ks_own, ks_shared, nj;      // k steps of 32 numbers of a head's own key part and of the shared one, value tiles of 16 columns
     int G;
     char *img, *img_shared;
+    int *odd; // [G + 1][nb]: does an image hold a number that is not finite (the shared ones last)
 };
 static __device__ __forceinline__ const float *sa_row(const sa_rows &r, long long step, int j) {
     int n = j + r.off;
@@ -95,6 +104,7 @@ __global__ __launch_bounds__(256) void split_keys_kernel(sa_keys a) {
     const int i0 = 32 * (front ? b : b - a.nbf), n = front ? a.n_front : a.n_window; // rows i0 .. i0 + 31 of those that exist
     const int ks = shared ? a.ks_shared : a.ks_own, nk = ks * 128, nv = shared ? 0 : a.nj * 64; // sixteen-byte pieces per plane
     char *out = shared ? a.img_shared + (size_t)b * a.ks_shared * 6144 : a.img + ((size_t)g * a.nb + b) * (a.ks_own * 6144 + a.nj * 3072);
+    int odd = 0;
     for (int x = tid; x < nk + nv; x += 256) {
         float v[8];
         sa_u4 p[3];
@@ -123,12 +133,17 @@ __global__ __launch_bounds__(256) void split_keys_kernel(sa_keys a) {
 #pragma unroll
             for (int q = 0; q < 3; q++) *(sa_u4 *)(out + ks * 6144 + (ct * 3 + q) * 1024 + lane * 16) = p[q];
         }
+#pragma unroll
+        for (int e = 0; e < 8; e++) odd |= !sa_finite(v[e]);
     }
+    odd = __syncthreads_or(odd);
+    if (tid == 0) a.odd[g * a.nb + b] = odd;
 }
 
 // ---------------------------------------------------------------------------------------------------- attention
 struct sa_attn {
     const char *img, *img_shared;
+    const int *odd, *odd_shared;
     int nbf, nb, ks_own, hpg;      // (heads per image)
     int pos0, first, T, window, pool, keep; // position of row 0, of window row 0
     const float *q;
@@ -166,8 +181,14 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     const int nfb = (nf + 31) / 32, wlo = max(pfirst - a.window + 1, 0) - a.first, wb0 = wlo / 32, nwb = (plast - a.first) / 32 - wb0 + 1, blocks = nfb + nwb;
     const int own = a.ks_own * 6, image = own + NJ * 3; // pieces of a head's own key part, of its image
     const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)sa_smem;
+    auto block_of = [&](const int it) { return it < nfb ? it : a.nbf + wb0 + it - nfb; };
+    // An infinite number's lower lines are zeros that the other operand's leading line meets, and it meets the other's lower lines, whose signs are their own: no number, where fp32 arithmetic has an
+    // infinite score or result.  Where a query of the wave or a key or value of its blocks is not finite, the wave joins the lines again and multiplies on the fp32 instruction.
+    auto odd_block = [&](const int *o, const int it) { return it < blocks ? o[block_of(it)] : 0; };
+    const int *odd_own = a.odd + (size_t)g * a.nb, *odd_shared = own < KS * 6 ? a.odd_shared : odd_own;
+    const int odd1 = odd_block(odd_own, lane), odd2 = odd_block(odd_shared, lane);
     auto request = [&](const int it) {
-        const int b = it < nfb ? it : a.nbf + wb0 + it - nfb;
+        const int b = block_of(it);
         const char *im = a.img + ((size_t)g * a.nb + b) * (image * 1024), *sh = a.img_shared + (size_t)b * ((KS * 6 - own) * 1024);
 #pragma unroll
         for (int x = 0; x < (PIECES + 7) / 8; x++) {
@@ -198,13 +219,18 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     }
     __syncthreads();
     sa_u4 q[KS][3];
+    int odd = odd1 | odd2;
+    for (int it = lane + 64; it < blocks; it += 64) odd |= odd_block(odd_own, it) | odd_block(odd_shared, it);
 #pragma unroll
     for (int s = 0; s < KS; s++) {
         float v[8];
         *(sa_f4 *)v = *(const sa_f4 *)(qs + lr * QLD + 32 * s + 8 * lq);
         *(sa_f4 *)(v + 4) = *(const sa_f4 *)(qs + lr * QLD + 32 * s + 8 * lq + 4);
         sa_split8<true>(v, q[s]);
+#pragma unroll
+        for (int e = 0; e < 8; e++) odd |= !sa_finite(v[e]);
     }
+    const bool plain = __any(odd); // (uniform)
     const float sc = a.scale * (a.temp ? a.temp[h] : 1.f), slope = DIST ? a.slope[h] : 0.f;
     float m = -INFINITY, l = 0.f; // (l: of this lane's own keys)
     sa_f4 acc[NJ];
@@ -212,25 +238,71 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     for (int j = 0; j < NJ; j++) acc[j] = sa_f4{0.f, 0.f, 0.f, 0.f};
     const int w0 = pfirst + 16 * wave, w1 = w0 + 15; // positions of the wave's rows
     const bool alive = 16 * wave < rows;
+    struct place { bool front, none, all; int j0, kp0; }; // of a block: nothing of it visible to the wave, or all of it to every row of it (uniform)
+    auto place_of = [&](const int it) {
+        place b;
+        b.front = it < nfb;
+        b.j0 = b.front ? 32 * it : 32 * (wb0 + it - nfb); // first row of the block, in the front store or behind `first`
+        b.kp0 = b.front ? b.j0 : a.first + b.j0;          // (kept first tokens: their positions)
+        if (b.front) {
+            const int o0 = w0 - a.window + 1, o1 = w1 - a.window + 1; // positions in front of the first and the last row's window
+            b.none = a.pool > 0 ? (b.j0 + 1) * a.pool > o1 : b.j0 >= o1;
+            b.all = a.pool > 0 ? (b.j0 + 32) * a.pool <= o0 : b.j0 + 31 < o0 && b.j0 + 31 < a.keep;
+        } else {
+            b.none = b.kp0 > w1 || b.kp0 + 31 <= w0 - a.window;
+            b.all = b.kp0 + 31 <= w0 && b.kp0 > w1 - a.window;
+        }
+        return b;
+    };
+    auto sees = [&](const place &b, const int i) { // this lane's row the block's key i
+        const int out = p - a.window + 1;
+        return b.front ? (a.pool > 0 ? (b.j0 + i + 1) * a.pool <= out : b.j0 + i < out && b.j0 + i < a.keep) : b.kp0 + i <= p && b.kp0 + i >= out;
+    };
+    // a block's products -> its weights; what was gathered in front of it is rescaled to the new maximum
+    auto soften = [&](const place &b, float (&e)[8]) {
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+            float v = e[x] * sc;
+            if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
+            const int kp = b.kp0 + 16 * (x >> 2) + 4 * lq + (x & 3);
+            if constexpr (DIST) v -= slope * (float)(p - kp);
+            e[x] = v;
+        }
+        if (!b.all) {
+#pragma unroll
+            for (int x = 0; x < 8; x++)
+                if (!sees(b, 16 * (x >> 2) + 4 * lq + (x & 3))) e[x] = -INFINITY;
+        }
+        float mx = e[0];
+#pragma unroll
+        for (int x = 1; x < 8; x++) mx = fmaxf(mx, e[x]);
+        {
+            auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+            auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = fmaxf(__uint_as_float(r2[0]), __uint_as_float(r2[1]));
+        }
+        const float mn = fmaxf(m, mx);
+        if (__any(mn > m)) { // (uniform)
+            const float corr = mn == -INFINITY ? 1.f : sa_exp(m - mn);
+            l *= corr;
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[j][i] *= corr;
+            m = mn;
+        }
+        const float off = m == -INFINITY ? 0.f : m; // (a row that has seen nothing yet: its weights are e^-inf)
+#pragma unroll
+        for (int x = 0; x < 8; x++) { e[x] = sa_exp(e[x] - off); l += e[x]; }
+    };
     for (int it = 0; it < blocks; it++) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); // the block has landed (this wave's share); the reads of the one before are back
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (it + 1 < blocks) request(it + 1);
-        const bool front = it < nfb;
-        const int j0 = front ? 32 * it : 32 * (wb0 + it - nfb); // first row of the block, in the front store or behind `first`
-        const int kp0 = front ? j0 : a.first + j0;              // (kept first tokens: their positions)
-        // nothing of the block visible to the wave, or all of it to every row of it (uniform)
-        bool none, all;
-        if (front) {
-            const int o0 = w0 - a.window + 1, o1 = w1 - a.window + 1; // positions in front of the first and the last row's window
-            none = a.pool > 0 ? (j0 + 1) * a.pool > o1 : j0 >= o1;
-            all = a.pool > 0 ? (j0 + 32) * a.pool <= o0 : j0 + 31 < o0 && j0 + 31 < a.keep;
-        } else {
-            none = kp0 > w1 || kp0 + 31 <= w0 - a.window;
-            all = kp0 + 31 <= w0 && kp0 > w1 - a.window;
-        }
-        if (!alive || none) continue;
+        const place b = place_of(it);
+        if (!alive || b.none || plain) continue;
         const char *st = sa_smem + (it & 1) * STAGE + lane * 16;
         sa_f4 s1[2], s2[2], s3[2]; // (chains of their own)
 #pragma unroll
@@ -265,43 +337,8 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
         }
         float e[8];
 #pragma unroll
-        for (int x = 0; x < 8; x++) {
-            float v = (s1[x >> 2][x & 3] + (s2[x >> 2][x & 3] + s3[x >> 2][x & 3])) * sc;
-            if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
-            const int kp = kp0 + 16 * (x >> 2) + 4 * lq + (x & 3);
-            if constexpr (DIST) v -= slope * (float)(p - kp);
-            e[x] = v;
-        }
-        if (!all) {
-#pragma unroll
-            for (int x = 0; x < 8; x++) {
-                const int i = 16 * (x >> 2) + 4 * lq + (x & 3), out = p - a.window + 1;
-                const bool sees = front ? (a.pool > 0 ? (j0 + i + 1) * a.pool <= out : j0 + i < out && j0 + i < a.keep) : kp0 + i <= p && kp0 + i >= out;
-                if (!sees) e[x] = -INFINITY;
-            }
-        }
-        float mx = e[0];
-#pragma unroll
-        for (int x = 1; x < 8; x++) mx = fmaxf(mx, e[x]);
-        {
-            auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-            mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-            auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-            mx = fmaxf(__uint_as_float(r2[0]), __uint_as_float(r2[1]));
-        }
-        const float mn = fmaxf(m, mx);
-        if (__any(mn > m)) { // (uniform)
-            const float corr = mn == -INFINITY ? 1.f : sa_exp(m - mn);
-            l *= corr;
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) acc[j][i] *= corr;
-            m = mn;
-        }
-        const float off = m == -INFINITY ? 0.f : m; // (a row that has seen nothing yet: its weights are e^-inf)
-#pragma unroll
-        for (int x = 0; x < 8; x++) { e[x] = sa_exp(e[x] - off); l += e[x]; }
+        for (int x = 0; x < 8; x++) e[x] = s1[x >> 2][x & 3] + (s2[x >> 2][x & 3] + s3[x >> 2][x & 3]);
+        soften(b, e);
         sa_u4 w[3], vf[2][2][3]; // (two column tiles side by side, the next two's pieces read in front of their products)
         sa_split8<false>(e, w);
         auto read_v = [&](const int j) {
@@ -327,6 +364,52 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
         }
     }
     if (!alive) return;
+    if (plain) { // the images straight from memory
+        for (int it = 0; it < blocks; it++) {
+            const place b = place_of(it);
+            if (b.none) continue;
+            const char *im = a.img + ((size_t)g * a.nb + block_of(it)) * (image * 1024) + lane * 16, *sh = a.img_shared + (size_t)block_of(it) * ((KS * 6 - own) * 1024) + lane * 16;
+            sa_u4 lines[3];
+            float v[8], y[8], e[8];
+            sa_f4 s1[2] = {sa_f4{0.f, 0.f, 0.f, 0.f}, sa_f4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const char *ks = 6 * s < own ? im + s * 6144 : sh + (6 * s - own) * 1024;
+                sa_join8(q[s], y);
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+#pragma unroll
+                    for (int x = 0; x < 3; x++) lines[x] = *(const sa_u4 *)(ks + (2 * x + u) * 1024);
+                    sa_join8(lines, v);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) s1[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], y[i], s1[u], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < 8; x++) e[x] = s1[x >> 2][x & 3];
+            soften(b, e);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+#pragma unroll
+                for (int x = 0; x < 3; x++) lines[x] = *(const sa_u4 *)(im + (own + j * 3 + x) * 1024);
+                sa_join8(lines, v);
+#pragma unroll
+                for (int x = 0; x < 8; x++) {
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa_finite(v[x]) ? v[x] : 0.f, e[x], acc[j], 0, 0, 0);
+                    if (__all(sa_finite(v[x]))) continue; // (uniform)
+                    for (int z = 0; z < 4; z++) { // a value that is not finite: for the rows that see its key, and no others
+                        const float wz = __shfl(e[x], lr + 16 * z, 64);
+                        const bool seen = sees(b, 16 * (x >> 2) + 4 * z + (x & 3));
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const float vz = __shfl(v[x], 4 * lq + i + 16 * z, 64);
+                            if (seen && !sa_finite(vz)) acc[j][i] += vz * wz;
+                        }
+                    }
+                }
+            }
+        }
+    }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     const int t = t0 + n;
@@ -359,7 +442,7 @@ bool psk_split_attn_ok(int own, int shared, int dv) { return dv == 128 && own % 
 // 166 | 137; 256 (2047 of 16, 1000 of 32) 318 | 142; 302 | 128, 319 | 160; keys of 128 with slopes: 1500 of 16 198 | 110.
 bool psk_split_attn_takes(int T, int H) { return (int64_t)((T + SA_ROWS - 1) / SA_ROWS) * H >= 80; }
 static size_t sa_images(int G, int own, int shared, int dv, int64_t blocks) { return (size_t)blocks * ((size_t)G * (own / 32 * 6144 + dv / 16 * 3072) + (size_t)shared / 32 * 6144); }
-size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window) { return sa_images(G, own, shared, dv, (n_front + 31) / 32 + (n_window + 31) / 32); }
+size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window) { return sa_images(G, own, shared, dv, (n_front + 31) / 32 + (n_window + 31) / 32) + (size_t)(G + 1) * ((n_front + 31) / 32 + (n_window + 31) / 32) * 4; }
 
 template <int KS, int NJ, bool DIST>
 static void sa_launch(hipStream_t st, const sa_attn &a, int H) {
@@ -378,8 +461,9 @@ void psk_split_attn(hipStream_t st, const psk_split_attn_args &x) {
     k.ks_own = x.own / 32; k.ks_shared = x.n_shared / 32; k.nj = 8; k.G = x.G;
     k.img = (char *)x.scratch;
     k.img_shared = k.img + (size_t)x.G * k.nb * (k.ks_own * 6144 + k.nj * 3072);
+    k.odd = (int *)(k.img + sa_images(x.G, x.own, x.n_shared, 128, k.nb));
     hipLaunchKernelGGL(split_keys_kernel, dim3(k.nb, x.G + (x.n_shared > 0)), dim3(256), 0, st, k);
-    sa_attn a{k.img, k.img_shared, k.nbf, k.nb, k.ks_own, x.H / x.G, (int)x.pos0, (int)x.first, x.T, x.window, x.pool, x.keep, x.q, x.ldq, x.own + x.n_shared, x.own, x.rot_dims, x.pairing, x.freq,
+    sa_attn a{k.img, k.img_shared, k.odd, k.odd + (size_t)x.G * k.nb, k.nbf, k.nb, k.ks_own, x.H / x.G, (int)x.pos0, (int)x.first, x.T, x.window, x.pool, x.keep, x.q, x.ldq, x.own + x.n_shared, x.own, x.rot_dims, x.pairing, x.freq,
               x.rot_mag, x.scale, x.softcap, x.temp, x.slope, x.sink, x.gate, x.ldg, x.gate_elem, x.o, x.ldo};
     if (x.own + x.n_shared == 192) x.slope ? sa_launch<6, 8, true>(st, a, x.H) : sa_launch<6, 8, false>(st, a, x.H);
     else x.slope ? sa_launch<4, 8, true>(st, a, x.H) : sa_launch<4, 8, false>(st, a, x.H);

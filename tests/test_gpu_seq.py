@@ -408,6 +408,43 @@ def test_attention_of_many_rows(ctx, tmp_path, which):
     assert err(got, want) < min(TOL["float32"], 2 * err(plain, want) + 2e-6)
 
 
+# the same attention with an infinite key, value or query of one token (64 heads of 150 and 140 rows: k_splitattn.hip): a score of -inf is a weight of nothing, an infinite value makes the rows that see
+# it infinite (not NaN), and rows that do not see the token -- those in front of it in the same 16 rows and 32 keys too -- are what they are without it
+@pytest.mark.parametrize("what", ["k", "v", "q"])
+def test_attention_of_many_rows_with_infinite_numbers(ctx, tmp_path, what):
+    cfg = synth.zusolix_config(64, 40, [synth.zusolix_layer("attention", synth.zusolix_attention(64, 8, 128, 128, 0.1))])
+    t = {n: a.copy() for n, a in synth.seq_tensors(cfg, 0).items()}
+    t["embed"][:, 3] = 0
+    t["embed"][7, 3] = 30  # token 7 alone has channel 3; of the norm's 8 = sqrt(64) it gets most
+    t["l0.norm1"][3] = 1
+    heads, row = range(24, 32), (25 if what == "q" else 3) * 128 + 5  # channel 5 of key / value head 3, which these heads read, or of head 25's query
+    for h in heads:
+        t["l0.mix.q"][h * 128 + 5], t["l0.mix.q.b"][h * 128 + 5] = 0, -5  # (a negative score with an infinite key)
+        t["l0.mix.o"][:, h * 128 + 5] = np.abs(t["l0.mix.o"][:, h * 128 + 5]) + 0.01
+    t["l0.mix." + what][row], t["l0.mix." + what + ".b"][row] = 0, 0
+    t["l0.mix." + what][row, 3] = 3e38
+    t = {n: (f32_to_bf16_bits(a).astype(np.uint32) << 16).view(np.float32).reshape(np.shape(a)) for n, a in t.items()}
+    synth.write_seq_model_dir(str(tmp_path), cfg, 0, t)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=200, n_slots=1, max_context=500)
+    toks = tokens_for(cfg, 290)
+    toks[toks == 7] = 8
+    toks[[20, 187]] = 7
+    per = []
+    seq_oracle.run_zusolix(cfg, t, toks, per)
+    m.capture_layers()
+    s, got = m.acquire(), []
+    for part in (toks[:150], toks[150:]):
+        m.forward(s, part)
+        got.append(m.layers(part.size)[-1].copy())
+    m.close()
+    got, want, at = np.concatenate(got), per[-1], np.arange(290)
+    fine = {"k": at >= 0, "v": at < 20, "q": toks != 7}[what]
+    assert np.all(np.isfinite(got[fine]))
+    assert np.abs(got[fine] - want[fine]).max() < TOL["float32"] * np.sqrt(np.mean(want[fine] ** 2))
+    if what == "v":
+        assert np.all(np.isinf(got[~fine])) and np.array_equal(np.sign(got[~fine]), np.sign(want[~fine]))
+
+
 # results without an epilogue (k_dense.hip dense_mm_ring_kernel): columns in fours, stored from the registers, the last four of a tile, one four and three fours into the next one; no fours
 # (through LDS); split along K, where the sums are stored in fours or one by one
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
