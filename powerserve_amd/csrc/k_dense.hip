@@ -1054,31 +1054,54 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
         }
     }
 }
+static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR && !g.em_table && (g.N % 4 || g.ldo % 4 || ((uintptr_t)g.out & 15)); }
 // Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
 // of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more; rounds of 256 work-groups (one per CU);
-// a split product pays a second launch and its parts' way through memory.  The 256 x 256 tiles' block is what they measured beside the 128 x 128 ones: 1.7 times their time where both fill the chip
-// once (512 tokens x 8192 x 2048: 28 us there, 48 here), half of it where the smaller ones need four rounds; they are not split (2047 x 2048 x 8192 in two: 98 us, 84 as 128 x 128 tiles).
+// a split product pays a second launch and its parts' way through memory.
+//   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, in us, fitted to 510 bf16 products of both forms
+// (K of 512 to 14336, 130 to 2047 tokens, 0.2 to 5 rounds): a round of the others 0.63 per block and 5, of these 1.03 and 16, and what the epilogue adds behind a tile (dn_epilogue); in three lines
+// 0.5 and 1.22 per line of a block (210 products).  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  They are taken where that says a tenth less, a fifth for
+// experts, whose last tiles are a guess.  6 of the 510 are then slower than the others by 2 % or more (7 % at most) and none of the 210; with 1700 clocks for a block of these it was 61 and 51:
+// 512 tokens x 16384 x 2048 of gate / up pairs take 64 us as 128 x 128 tiles and 80 as 256 x 256 (900: 119 and 89), 512 x 14336 x 4096 in three lines 206 and 251 (900: 391 and 257).
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
-static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines, int groups, bool bf, bool may_split, bool big) {
-    static const int shapes[4][2] = {{128, 128}, {64, 128}, {64, 64}, {DN_BIG, DN_BIG}};
+enum { DN_EPI_DIRECT, DN_EPI_FOURS, DN_EPI_ONES }; // results from the registers; through LDS, four at a time; an activation or bias each
+static int dn_epilogue(const dn_args &g) {
+    if (g.act == PSD_ACT_SILU_PAIR || g.act == PSD_ACT_RELU_PAIR || g.em_table || g.bias) return DN_EPI_ONES;
+    if (g.act == PSD_ACT_XIELU) return DN_EPI_FOURS;
+    if (g.act != PSD_ACT_NONE && (g.act != PSD_ACT_RELU2 || g.accum)) return DN_EPI_ONES;
+    return g.accum || dn_odd(g) ? DN_EPI_FOURS : DN_EPI_DIRECT;
+}
+static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines, int groups, bool bf, bool may_split, bool big, int epilogue) {
+    static const int shapes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
     const int64_t blocks = kbytes / 128;
     dn_ring_shape best{};
     double least = 0;
+    auto row_tiles = [&](int BM) { // (grouped: about half of the last tiles start a new one)
+        const int full = (rows + BM - 1) / BM;
+        return groups > 0 ? std::max(full, std::min(groups, rows)) + (rows > groups * BM ? groups / 2 : 0) : full;
+    };
     for (auto &q : shapes) {
-        if (q[0] == DN_BIG && !(bf && big)) continue;
-        const int BM = q[0], BN = q[1], full = (rows + BM - 1) / BM, n_tm = rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0), tn = (int)((N + BN - 1) / BN);
-        const int64_t tiles = (int64_t)(groups > 0 ? std::max(full, std::min(groups, rows)) + (rows > groups * BM ? groups / 2 : 0) : n_tm) * tn; // (grouped: about half of the last tiles start a new one)
-        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = BM == DN_BIG ? 1700 : std::max(lds, mfma) + 100;
-        for (int64_t S = 1; S <= (may_split && BM != DN_BIG ? 16 : 1); S++) {
+        const int BM = q[0], BN = q[1], n_tm = rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0), tn = (int)((N + BN - 1) / BN);
+        const int64_t tiles = (int64_t)row_tiles(BM) * tn;
+        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = std::max(lds, mfma) + 100;
+        for (int64_t S = 1; S <= (may_split ? 16 : 1); S++) {
             if (S > 1 && (blocks / S < 4 || tiles * S > 512 || (size_t)n_tm * tn * S * BM * BN * 4 > psk_dense_split_bytes())) break;
             const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * lines * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
             if (!best.BM || t < least) { least = t; best = dn_ring_shape{BM, BN, n_tm, tn, (int)S}; }
         }
     }
+    if (bf && big) {
+        static const double behind[3] = {0, 1, 4}, behind_big[3] = {0, 6, 27};
+        const int tn = (int)((N + DN_BIG - 1) / DN_BIG), n_tm = rows / DN_BIG + (groups > 0 ? std::min(groups, rows) : rows % DN_BIG ? 1 : 0);
+        auto rounds = [&](int BM, int64_t columns) { return (double)(((columns + 7) / 8 * row_tiles(BM) + 31) / 32); };
+        const double area = best.BM * best.BN / 16384.0, block = (lines == 3 ? 0.5 : 0.63) * (std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100) / 868;
+        const double other = rounds(best.BM, (int64_t)best.tn * best.S) * ((double)((blocks + best.S - 1) / best.S) * lines * block + (5 + behind[epilogue]) * area) + 4 + (best.S > 1 ? 9 : 0);
+        const double here = rounds(DN_BIG, tn) * ((double)blocks * lines * (lines == 3 ? 1.22 : 1.03) + 16 + behind_big[epilogue]) + 4;
+        if (here < (groups > 0 ? 0.8 : 0.9) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
+    }
     return best;
 }
 
-static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR && !g.em_table && (g.N % 4 || g.ldo % 4 || ((uintptr_t)g.out & 15)); }
 template <typename WT, int BM, int BN, bool ODD, int PL>
 static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if constexpr (!ODD)
@@ -1121,7 +1144,7 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     }
     const int64_t each = g.N;
     g.N *= copies;
-    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, PL, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes(), (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 22)); // (rows of a tile by 32-bit offsets)
+    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, PL, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes(), (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 22), dn_epilogue(g)); // (rows of a tile by 32-bit offsets)
     dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes * PL, r.n_tm, r.tn, r.S, a.split};
     p.each = copies > 1 ? each : 0;
     p.copy = a.T * kbytes * PL;
