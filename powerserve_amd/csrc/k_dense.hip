@@ -1060,8 +1060,8 @@ static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.ac
 // a split product pays a second launch and its parts' way through memory.
 //   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, in us, fitted to 510 bf16 products of both forms
 // (K of 512 to 14336, 130 to 2047 tokens, 0.2 to 5 rounds): a round of the others 0.63 per block and 5, of these 1.03 and 16, and what the epilogue adds behind a tile (dn_epilogue); in three lines
-// 0.5 and 1.22 per line of a block (210 products).  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  They are taken where that says a tenth less, a fifth for
-// experts, whose last tiles are a guess.  6 of the 510 are then slower than the others by 2 % or more (7 % at most) and none of the 210; with 1700 clocks for a block of these it was 61 and 51:
+// 0.5 and 1.22 per line of a block (210 products).  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  They are taken where that says a tenth less, for
+// experts, whose last tiles are a guess, a fifth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  6 of the 510 are then slower than the others by 2 % or more (7 % at most) and none of the 210; with 1700 clocks for a block of these it was 61 and 51:
 // 512 tokens x 16384 x 2048 of gate / up pairs take 64 us as 128 x 128 tiles and 80 as 256 x 256 (900: 119 and 89), 512 x 14336 x 4096 in three lines 206 and 251 (900: 391 and 257).
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
 enum { DN_EPI_DIRECT, DN_EPI_FOURS, DN_EPI_ONES }; // results from the registers; through LDS, four at a time; an activation or bias each
@@ -1097,7 +1097,7 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines
         const double area = best.BM * best.BN / 16384.0, block = (lines == 3 ? 0.5 : 0.63) * (std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100) / 868;
         const double other = rounds(best.BM, (int64_t)best.tn * best.S) * ((double)((blocks + best.S - 1) / best.S) * lines * block + (5 + behind[epilogue]) * area) + 4 + (best.S > 1 ? 9 : 0);
         const double here = rounds(DN_BIG, tn) * ((double)blocks * lines * (lines == 3 ? 1.22 : 1.03) + 16 + behind_big[epilogue]) + 4;
-        if (here < (groups > 0 ? 0.8 : 0.9) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
+        if (here < (groups == 0 ? 0.9 : rows > 1.4 * DN_BIG * groups ? 0.95 : 0.8) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
     }
     return best;
 }
@@ -1163,7 +1163,10 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
 }
 static bool dn_wide(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
     if (a.w->dtype == PS_BF16) return dn_ring_take<unsigned short, 1>(st, a, g);
-    return (a.w->half && dn_ring_take<unsigned short, 3>(st, a, g)) || dn_ring_take<float, 1>(st, a, g);
+    // (a small matrix and few rows: three lines are a launch more.  us on the fp32 instruction and in three lines, 64 tokens: 768 x 768 9.3 and 11.9, 1024 x 1024 10.0 and 12.0, 256 x 2048 9.8 and 12.0; 256
+    // tokens: 13.3 and 15.7, 12.6 and 15.5 for the latter two)
+    const bool small = a.small_f32 && !g.groups && !a.n_more && g.N * g.K <= (1 << 20) && a.T * g.N * g.K <= (1 << 28);
+    return (a.w->half && !small && dn_ring_take<unsigned short, 3>(st, a, g)) || dn_ring_take<float, 1>(st, a, g);
 }
 
 // Products with an inner size of a few numbers (the second matrix of a low-rank decay): a thread has an output column, its KP weights in registers, and runs over sixteen tokens whose
@@ -1792,7 +1795,8 @@ bool psk_dense_takes_pre(const psk_dense_args &a) {
     const int64_t K = a.w->K, unit = a.w->dtype == PS_BF16 ? 512 : 256; // (whole units of the stream; four runs a thread)
     const psk_dense_pre &r = a.pre;
     if (K % unit || K > 8192 || !aligned(a.a) || !aligned(r.w)) return false;
-    // (heads: 4096 numbers and as many of the gate read by 512 work-groups take what the launch in front did: a token of Ranutar 2048 x 6 367 -> 360 us with it, of 4096 x 3 335 -> 336)
+    // (heads: a token of six Ranutar layers in us, a launch in front | in the product: 1024 channels 259 | 249, 1536 285 | 277, 2048 343 | 335, 2560 396 | 392, 3072 424 | 421, three of 4096 314 | 312 in one
+    // measurement, 335 | 336 in another: 4096 numbers and as many of the gate read by 512 work-groups take what the launch did)
     if (r.kind == psk_dense_pre::HEADS) return K <= 2048 && aligned(r.gate) && r.part >= 4 && r.part <= 256 && (r.part & (r.part - 1)) == 0 && K % r.part == 0 && r.w_stride % 4 == 0;
     return r.kind == psk_dense_pre::BOUNDARY && aligned(r.y) && aligned(r.xout) && r.xout != a.a;
 }
@@ -1802,6 +1806,16 @@ bool psk_dense_wide16(const psk_dense_args &a) {
 }
 bool psk_dense_listed16(const psk_dense_args &a) { // (as dn_ring_take)
     return a.w && a.w->dtype == PS_BF16 && a.groups > 0 && a.g_list && !a.force_tiled && a.pack && a.w->K % 64 == 0 && (size_t)a.T * a.w->K * 2 <= a.pack_bytes;
+}
+// fp32 products of two to four tokens that the mat-vec takes first, though the wide mat-mul takes them: its launches (packing, product, sum) against a second column of the streamed rows.  us there and
+// here, weights from memory (bf16 ones stay there: 4096 x 2048 14.9 and 13.1 alone, but a layer's rows come rounded, and whole requests of two tokens are 1 to 4 % faster with the wide one):
+//   two tokens, 2048 x 768 11.0 and 7.9, 4096 x 2048 18.2 and 13.8, 4096 x 4096 30.3 and 24.9, but 512 x 4096 12.7 and 14.5; in three lines 11.8 and 7.9, 18.3 and 13.8, 2048 x 3072 15.7 and 14.6, but
+//   4096 x 4096 21.6 and 24.9;  three and four, without the lines, 8192 x 2048 30.7 and 23.7, 30.7 and 24.9, but 2048 x 2048 14.2 and 15.6, 14.2 and 16.7
+static bool dn_few_first(const psk_dense_args &a, const dn_args &g) {
+    if (a.T < 2 || a.T > 4 || a.a16 || a.out16) return false; // (rounded rows are the wide one's to read and to write)
+    if (a.w->dtype == PS_BF16) return false;
+    if (a.w->half) return a.T == 2 && g.K <= 3072;
+    return a.T == 2 ? g.K <= 2048 || 4 * g.N >= g.K : g.N >= 4 * g.K;
 }
 int psk_dense(hipStream_t st, const psk_dense_args &a) {
     if (!a.w || a.T <= 0) return 0;
@@ -1843,6 +1857,32 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);
         return 0;
     }
+    auto few = [&]() { // the mat-vecs, where they take the product
+        if (a.force_tiled || a.T > 8) return false;
+        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 0>(st, g, nullptr, 0, &a))) return true;
+        const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
+        if (kp4 * C <= 64 * 1024) {
+            // (a token's rows that the stream does not take: four per wave would leave at most 64 blocks.  1004 x 4102 14.2 us, with one per wave 11.9; 512 x 1026 6.7 and 5.3)
+            const bool one_row = C == 1 && g.N <= 1024 && g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR;
+            if (one_row) {
+                if (bf) dn_launch_mv<unsigned short, 1, 1>(st, g);
+                else dn_launch_mv<float, 1, 1>(st, g);
+            } else if (bf) {
+                if (C == 1) dn_launch_mv<unsigned short, 1>(st, g);
+                else if (C == 2) dn_launch_mv<unsigned short, 2>(st, g);
+                else if (C == 4) dn_launch_mv<unsigned short, 4>(st, g);
+                else dn_launch_mv<unsigned short, 8>(st, g);
+            } else {
+                if (C == 1) dn_launch_mv<float, 1>(st, g);
+                else if (C == 2) dn_launch_mv<float, 2>(st, g);
+                else if (C == 4) dn_launch_mv<float, 4>(st, g);
+                else dn_launch_mv<float, 8>(st, g);
+            }
+            return true;
+        }
+        return false;
+    };
+    if (dn_few_first(a, g) && few()) return 0;
     if (!a.force_tiled && a.T > 8 && g.K <= 32 && !g.mu && !g.a_mod && !g.a_step && !g.a_row0) {
         const dim3 grid((unsigned)((g.N + 255) / 256), (unsigned)((a.T + 15) / 16));
         auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g); };
@@ -1870,29 +1910,7 @@ int psk_dense(hipStream_t st, const psk_dense_args &a) {
         return 0;
     }
     if (a.T > PSD_FEW && dn_wide(st, a, g)) return 0;
-    if (!a.force_tiled && a.T <= 8) {
-        if (a.T == 1 && (bf ? dn_launch_mv1<unsigned short, 0>(st, g, nullptr, 0, &a) : dn_launch_mv1<float, 0>(st, g, nullptr, 0, &a))) return 0;
-        const int C = a.T <= 1 ? 1 : a.T <= 2 ? 2 : a.T <= 4 ? 4 : 8;
-        if (kp4 * C <= 64 * 1024) {
-            // (a token's rows that the stream does not take: four per wave would leave at most 64 blocks.  1004 x 4102 14.2 us, with one per wave 11.9; 512 x 1026 6.7 and 5.3)
-            const bool one_row = C == 1 && g.N <= 1024 && g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR;
-            if (one_row) {
-                if (bf) dn_launch_mv<unsigned short, 1, 1>(st, g);
-                else dn_launch_mv<float, 1, 1>(st, g);
-            } else if (bf) {
-                if (C == 1) dn_launch_mv<unsigned short, 1>(st, g);
-                else if (C == 2) dn_launch_mv<unsigned short, 2>(st, g);
-                else if (C == 4) dn_launch_mv<unsigned short, 4>(st, g);
-                else dn_launch_mv<unsigned short, 8>(st, g);
-            } else {
-                if (C == 1) dn_launch_mv<float, 1>(st, g);
-                else if (C == 2) dn_launch_mv<float, 2>(st, g);
-                else if (C == 4) dn_launch_mv<float, 4>(st, g);
-                else dn_launch_mv<float, 8>(st, g);
-            }
-            return 0;
-        }
-    }
+    if (few()) return 0;
     dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((a.T + 63) / 64));
     if (bf) hipLaunchKernelGGL(dense_mm_kernel<unsigned short>, grid, dim3(256), 0, st, g);
     else hipLaunchKernelGGL(dense_mm_kernel<float>, grid, dim3(256), 0, st, g);

@@ -182,11 +182,8 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     const int own = a.ks_own * 6, image = own + NJ * 3; // pieces of a head's own key part, of its image
     const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)sa_smem;
     auto block_of = [&](const int it) { return it < nfb ? it : a.nbf + wb0 + it - nfb; };
-    // An infinite number's lower lines are zeros that the other operand's leading line meets, and it meets the other's lower lines, whose signs are their own: no number, where fp32 arithmetic has an
-    // infinite score or result.  Where a query of the wave or a key or value of its blocks is not finite, the wave joins the lines again and multiplies on the fp32 instruction.
-    auto odd_block = [&](const int *o, const int it) { return it < blocks ? o[block_of(it)] : 0; };
-    const int *odd_own = a.odd + (size_t)g * a.nb, *odd_shared = own < KS * 6 ? a.odd_shared : odd_own;
-    const int odd1 = odd_block(odd_own, lane), odd2 = odd_block(odd_shared, lane);
+    const int *odd_own = a.odd + (size_t)g * a.nb;
+    const int odd1 = lane < blocks ? odd_own[block_of(lane)] : 0, odd2 = lane < blocks && own < KS * 6 ? a.odd_shared[block_of(lane)] : 0; // (asked for here, looked at behind the loop)
     auto request = [&](const int it) {
         const int b = block_of(it);
         const char *im = a.img + ((size_t)g * a.nb + b) * (image * 1024), *sh = a.img_shared + (size_t)b * ((KS * 6 - own) * 1024);
@@ -219,18 +216,13 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     }
     __syncthreads();
     sa_u4 q[KS][3];
-    int odd = odd1 | odd2;
-    for (int it = lane + 64; it < blocks; it += 64) odd |= odd_block(odd_own, it) | odd_block(odd_shared, it);
 #pragma unroll
     for (int s = 0; s < KS; s++) {
         float v[8];
         *(sa_f4 *)v = *(const sa_f4 *)(qs + lr * QLD + 32 * s + 8 * lq);
         *(sa_f4 *)(v + 4) = *(const sa_f4 *)(qs + lr * QLD + 32 * s + 8 * lq + 4);
         sa_split8<true>(v, q[s]);
-#pragma unroll
-        for (int e = 0; e < 8; e++) odd |= !sa_finite(v[e]);
     }
-    const bool plain = __any(odd); // (uniform)
     const float sc = a.scale * (a.temp ? a.temp[h] : 1.f), slope = DIST ? a.slope[h] : 0.f;
     float m = -INFINITY, l = 0.f; // (l: of this lane's own keys)
     sa_f4 acc[NJ];
@@ -302,7 +294,7 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
         asm volatile("" ::: "memory");
         if (it + 1 < blocks) request(it + 1);
         const place b = place_of(it);
-        if (!alive || b.none || plain) continue;
+        if (!alive || b.none) continue;
         const char *st = sa_smem + (it & 1) * STAGE + lane * 16;
         sa_f4 s1[2], s2[2], s3[2]; // (chains of their own)
 #pragma unroll
@@ -364,7 +356,20 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
         }
     }
     if (!alive) return;
-    if (plain) { // the images straight from memory
+    // An infinite number's lower lines are zeros that the other operand's leading line meets, and it meets the other's lower lines, whose signs are their own: no number, where fp32 arithmetic has an
+    // infinite score or result.  Where a query of the wave or a key or value of its blocks is not finite, the wave does it all again with the lines joined, on the fp32 instruction, the images straight
+    // from memory.
+    int odd = odd1 | odd2;
+    for (int it = lane + 64; it < blocks; it += 64) odd |= odd_own[block_of(it)] | (own < KS * 6 ? a.odd_shared[block_of(it)] : 0);
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) odd |= !sa_finite(__uint_as_float(q[s][0][e] << 16)) | !sa_finite(__uint_as_float(q[s][0][e] & 0xffff0000u));
+    if (__builtin_expect(__any(odd), 0)) { // (uniform)
+        m = -INFINITY;
+        l = 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[j] = sa_f4{0.f, 0.f, 0.f, 0.f};
         for (int it = 0; it < blocks; it++) {
             const place b = place_of(it);
             if (b.none) continue;
@@ -388,14 +393,15 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
 #pragma unroll
             for (int x = 0; x < 8; x++) e[x] = s1[x >> 2][x & 3];
             soften(b, e);
-#pragma unroll
+#pragma unroll 1
             for (int j = 0; j < NJ; j++) {
 #pragma unroll
                 for (int x = 0; x < 3; x++) lines[x] = *(const sa_u4 *)(im + (own + j * 3 + x) * 1024);
                 sa_join8(lines, v);
+                sa_f4 t = sa_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int x = 0; x < 8; x++) {
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa_finite(v[x]) ? v[x] : 0.f, e[x], acc[j], 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_16x16x4f32(sa_finite(v[x]) ? v[x] : 0.f, e[x], t, 0, 0, 0);
                     if (__all(sa_finite(v[x]))) continue; // (uniform)
                     for (int z = 0; z < 4; z++) { // a value that is not finite: for the rows that see its key, and no others
                         const float wz = __shfl(e[x], lr + 16 * z, 64);
@@ -403,10 +409,13 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
                             const float vz = __shfl(v[x], 4 * lq + i + 16 * z, 64);
-                            if (seen && !sa_finite(vz)) acc[j][i] += vz * wz;
+                            if (seen && !sa_finite(vz)) t[i] += vz * wz;
                         }
                     }
                 }
+#pragma unroll
+                for (int y = 0; y < NJ; y++) // (registers)
+                    if (y == j) acc[y] += t;
             }
         }
     }

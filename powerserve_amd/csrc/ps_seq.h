@@ -57,6 +57,7 @@ struct psk_dense_args {
     float act_p = 0.f, act_q = 0.f, alpha = 1.f; // xIELU: act_p = softplus(p), act_q = 1/2 + softplus(q)
     int accum = 0; // 1: out += the result (the residual stream takes a sublayer's output projection directly)
     const float *mu = nullptr, *shift0 = nullptr;
+    int small_f32 = 0; // 1: a small product of an fp32 matrix runs on the fp32 instruction though it has a bf16 form (dn_wide); 0: a product of several tokens on the bf16 one whatever its size
     int force_tiled = 0; // 1: the plain tiled mat-mul whatever the shape (A/B against the mat-vec and the wide mat-mul)
     void *pack = nullptr; // scratch for the wide mat-mul's copy of A (T rows of K in bf16, or for fp32 matrices three times that); without it the plain tiled kernel runs
     size_t pack_bytes = 0;
@@ -99,9 +100,12 @@ struct psk_dense_args {
 bool psk_dense_takes_pre(const psk_dense_args &a);
 // Tokens up to which a product of its own runs as a mat-vec where the wide mat-mul takes it too.  That one fills a tile with a few rows and streams the weights all the same; the mat-vec of a few
 // tokens stages their activations in every work-group.  Whole requests in us, mat-vecs | wide: Ranutar 2048 x 6 2 tokens 910 | 655, 3 3672 | 667, 8 4392 | 710; 4096 x 3 2 3268 | 512, 8 7037 | 545.
+// (fp32 products of two to four tokens: k_dense.hip dn_few_first.  Whole requests of 2, 4, 8 tokens in float32, mat-vecs | wide and they: Ranutar 2048 x 6 937, 4826, 5284 | 797, 875, 869; Sogavik 2048 x 6
+// 1160, 1654, 3429 | 1144, 1392, 1603, without the lines 1148, 1439, 2246.)
 static const int PSD_FEW = 1;
 // The same for a mixture's own products, whose mat-vecs read a matrix per slot and the wide mat-mul a tile per matrix: up to two tokens, and up to a quarter more slots than there are experts.  Top 2 of
 // 8, mat-vecs | wide, Pupidra 2048 x 6: 2 tokens 696 | 874, 4 788 | 904, 5 827 | 917, 6 905 | 928; 4096 x 3: 4 772 | 840, 5 819 | 873, 6 931 | 920; float32 4 1094 | 1237, 5 1164 | 1243, 6 1316 | 1257.
+// Top 6 of 64 experts of 512 at 2048 x 6, where 8 tokens touch about 35 of the matrices: mat-vecs 877 us for 8 tokens, wide 1328 for 12 (Pupidra); 879, 1328 (Zusolix).
 static inline bool psk_few_slots(int T, int top, int experts, bool wide) { return T <= 8 && (!wide || T <= 2 || 4 * T * top <= 5 * experts); } // (wide: the wide mat-mul takes both products)
 bool psk_dense_listed16(const psk_dense_args &a); // it will run this grouped product so: out16's and a16's rows are slots in g_list's order
 bool psk_dense_wide16(const psk_dense_args &a); // psk_dense will run this as the wide bf16 mat-mul over plain rows

@@ -639,7 +639,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         psk_dense_args g;
         if (copy16 && a == rounded && w && lda == w->K) g.a16 = copy16;
         if (out == rounded) rounded = nullptr;
-        g.w = w; g.a = a; g.lda = lda; g.T = T; g.out = out; g.ldo = ldo; g.force_tiled = tiled; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
+        g.w = w; g.a = a; g.lda = lda; g.T = T; g.out = out; g.ldo = ldo; g.small_f32 = 1; g.force_tiled = tiled; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
         return g;
     };
     // a sublayer boundary: x += norm_b(y) (after a sublayer), then hn = norm(x), h = conv(hn) (in front of the next one); one launch for a single token
@@ -1073,7 +1073,7 @@ static void seq_head(ps_hip_seq *m, const int32_t *idx, int rows, bool normed, b
         psk_rmsnorm(st, m->x, D.width, idx, D.final_norm, D.norm_offset, D.norm_eps, D.width, rows, m->xn, D.width, m->groups);
     }
     psk_dense_args g;
-    g.w = D.head; g.a = m->xn; g.lda = D.width; g.T = rows; g.out = m->logits; g.ldo = D.vocab; g.alpha = D.logit_scale; g.force_tiled = (m->mode & 2) != 0; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
+    g.w = D.head; g.a = m->xn; g.lda = D.width; g.T = rows; g.out = m->logits; g.ldo = D.vocab; g.alpha = D.logit_scale; g.small_f32 = 1; g.force_tiled = (m->mode & 2) != 0; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
     if (D.logit_softcap > 0.f) { g.act = PSD_ACT_SOFTCAP; g.act_p = D.logit_softcap; }
     psk_dense(st, g);
     if (argmax) psk_argmax_rows(st, m->logits, D.vocab, rows, m->amax);

@@ -320,25 +320,37 @@ def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights, dtype):
     dx.free(); do.free()
 
 
-# a float32 model in either form of its matrices: four mixes, several mixers' projections, the latent's window, experts; a joint projection of two mixers; portions and single tokens
+# a float32 model in either form of its matrices: four mixes, a feed-forward and a latent's window of more than 2^20 numbers (fewer run on the fp32 instruction in both: psk_dense_args small_f32),
+# experts; a joint projection of two mixers; portions and single tokens
 @pytest.mark.parametrize("dtype", ["float32", "float32 lines"])
 @pytest.mark.parametrize("which", ["mixes", "experts", "joint"])
 def test_float32_models_in_either_form(ctx, tmp_path, which, dtype):
     V = 40
     if which == "mixes":
-        run, cfg = seq_oracle.run, synth.seq_config(128, V, [L("wkv", 192, heads=4, dim=32), L("latent_attention", 64, heads=4, dim=32, vdim=32, q_rank=64, kv_rank=64, mask={"size": 33}, scale=0.2,
+        run, cfg = seq_oracle.run, synth.seq_config(128, V, [L("wkv", 192, heads=4, dim=32), L("latent_attention", 8256, heads=16, dim=128, vdim=128, q_rank=64, kv_rank=320, mask={"size": 33}, scale=0.1,
                                                                                              rot={"base": 100.0, "dims": 8}, rot_dim=16), L("delta", 64, heads=4, kv_heads=2, dim=32, vdim=32, conv=3)], taps=2)
     elif which == "experts":
         run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(128, V, [synth.pupidra_layer("attention", synth.pupidra_attention(2, 1, 64, 64, 0.3, 9, 2), moe=(5, 2, 128, 1.7), shared=64)])
     else:
-        run, cfg = seq_oracle.run_parallel, synth.parallel_config(128, V, [synth.parallel_layer(128, {"heads": 4, "kv_heads": 2, "dim": 32, "vdim": 32, "mask": {"size": 33, "pool": 3},
-                                                                  "rot": {"base": 100.0, "dims": 16}, "scale": 0.2}, {"heads": 4, "dim": 32, "vdim": 32, "tau": 4.0}, 1.0, 0.5)], taps=2)
+        run, cfg = seq_oracle.run_parallel, synth.parallel_config(512, V, [synth.parallel_layer(128, {"heads": 8, "kv_heads": 2, "dim": 64, "vdim": 64, "mask": {"size": 33, "pool": 3},
+                                                                  "rot": {"base": 100.0, "dims": 16}, "scale": 0.2}, {"heads": 8, "dim": 64, "vdim": 64, "tau": 4.0}, 1.0, 0.5)], taps=2)
     t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
     m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=300, n_slots=1, max_context=700, f32_form=FORMS[dtype])
     assert {ctx.L.ps_hip_dense_form(w) for w in m._up.mats} == {FORMS[dtype]}
     toks = tokens_for(cfg, 350)
     assert err(run_portions(m, toks, (300, 1, 5, 44)), run(cfg, t, toks)) < TOL["float32"]
     m.close()
+
+
+# a small matrix and few rows of a float32 model: on either side of the line between the fp32 instruction and three lines (k_dense.hip dn_wide), by rows (1024 x 1024: 256) and by the matrix (1024 x 1088)
+@pytest.mark.parametrize("ff", [1024, 1088])
+@pytest.mark.parametrize("sizes", [(256, 5), (257, 4)])
+def test_small_float32_products(made, ff, sizes):
+    cfg = synth.seq_config(1024, 40, [L("delta", ff, heads=2, kv_heads=1, dim=16, vdim=16, conv=2)], taps=2)
+    m, c, t = made(f"small-f32.{ff}", max_batch=260, cfg=cfg)
+    toks = tokens_for(c, 261)
+    assert {m.ctx.L.ps_hip_dense_form(w) for w in m._up.mats} == {hip.DENSE_F32_LINES}
+    assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
 # 256 x 256 tiles behind an epilogue (k_dense.hip dense_mm_big_kernel): an activation whose rounded rows the second product reads, pairs, the four mixes of a token shift, the slots of experts (tiles
@@ -482,6 +494,13 @@ def test_dense_matmul_of_few_tiles(ctx, dtype, T, N, K):
 @pytest.mark.parametrize("dtype", list(FORMS))
 @pytest.mark.parametrize("T,N,K", [(2, 1, 64), (3, 33, 128), (4, 129, 1024), (5, 70, 4160), (8, 2100, 192), (7, 65, 2048), (2, 300, 72), (8, 40, 1056)])
 def test_dense_matmul_of_a_few_tokens(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
+# both sides of the lines between the mat-vec and the wide mat-mul for two to four tokens (k_dense.hip dn_few_first)
+@pytest.mark.parametrize("dtype", list(FORMS))
+@pytest.mark.parametrize("T,N,K", [(2, 70, 2048), (2, 70, 2112), (2, 33, 3072), (2, 33, 3136), (2, 600, 2432), (2, 607, 2432), (3, 256, 64), (4, 255, 64), (5, 300, 64)])
+def test_dense_matmul_on_either_side_of_its_lines(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
 
 
