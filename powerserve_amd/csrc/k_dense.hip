@@ -1058,11 +1058,12 @@ static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.ac
 // Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
 // of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more; rounds of 256 work-groups (one per CU);
 // a split product pays a second launch and its parts' way through memory.
-//   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, in us, fitted to 510 bf16 products of both forms
-// (K of 512 to 14336, 130 to 2047 tokens, 0.2 to 5 rounds): a round of the others 0.63 per block and 5, of these 1.03 and 16, and what the epilogue adds behind a tile (dn_epilogue); in three lines
-// 0.5 and 1.22 per line of a block (210 products).  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  They are taken where that says a tenth less, for
-// experts, whose last tiles are a guess, a fifth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  6 of the 510 are then slower than the others by 2 % or more (7 % at most) and none of the 210; with 1700 clocks for a block of these it was 61 and 51:
-// 512 tokens x 16384 x 2048 of gate / up pairs take 64 us as 128 x 128 tiles and 80 as 256 x 256 (900: 119 and 89), 512 x 14336 x 4096 in three lines 206 and 251 (900: 391 and 257).
+//   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, fitted to 615 bf16 products of either form (K of
+// 512 to 14336, 130 to 2047 tokens, 0.1 to 8 rounds; 4 % off on average, 3 % for these) and 335 in three lines.  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  In us:
+// a round's blocks, its start and what the epilogue adds behind a tile (dn_epilogue), the results and the weights by their megabytes.  They are taken where that says 3 % less; for experts, whose last tiles are a
+// guess, a tenth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  4 of the 615 are then slower than
+// the others by 2 % or more (4 % at most) and none of the 335.  With 1700 clocks for a block of these in the estimate above it was one in nine and one in five: 512 tokens x 16384 x 2048 of gate / up pairs
+// take 64 us as 128 x 128 tiles and 80 as 256 x 256 (900: 119 and 89), 512 x 14336 x 4096 in three lines 206 and 251 (900: 391 and 257).
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
 enum { DN_EPI_DIRECT, DN_EPI_FOURS, DN_EPI_ONES }; // results from the registers; through LDS, four at a time; an activation or bias each
 static int dn_epilogue(const dn_args &g) {
@@ -1091,13 +1092,17 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines
         }
     }
     if (bf && big) {
-        static const double behind[3] = {0, 1, 4}, behind_big[3] = {0, 6, 27};
+        struct cost { double all, block, round, results, weights, behind[3]; };
+        static const cost small[2] = {{2.4, 0.527, 0.55, 0.377, 0.058, {0, 0.9, 5.1}}, {4.3, 0.495, -2.4, 0.576, 0.056, {0, 0.9, 5.1}}}, large[2] = {{-2.5, 1.023, 12.8, 0.145, 0.079, {0, 7.4, 27.4}}, {-8.4, 1.177, 20, 0.153, 0.105, {0, 7.4, 27.4}}};
+        const double results = rows * (double)N * 4e-6, weights = (double)N * kbytes * 1e-6 * std::max(groups, 1), per_block = std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100; // (clocks; 868 for 128 x 128)
+        auto time = [&](const cost &c, int BM, int64_t columns, double blocks, double area) {
+            const double rounds = (double)(((columns + 7) / 8 * row_tiles(BM) + 31) / 32);
+            return c.all + rounds * (blocks * lines * c.block + (c.round + c.behind[epilogue]) * area) + c.results * results + c.weights * weights;
+        };
         const int tn = (int)((N + DN_BIG - 1) / DN_BIG), n_tm = rows / DN_BIG + (groups > 0 ? std::min(groups, rows) : rows % DN_BIG ? 1 : 0);
-        auto rounds = [&](int BM, int64_t columns) { return (double)(((columns + 7) / 8 * row_tiles(BM) + 31) / 32); };
-        const double area = best.BM * best.BN / 16384.0, block = (lines == 3 ? 0.5 : 0.63) * (std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100) / 868;
-        const double other = rounds(best.BM, (int64_t)best.tn * best.S) * ((double)((blocks + best.S - 1) / best.S) * lines * block + (5 + behind[epilogue]) * area) + 4 + (best.S > 1 ? 9 : 0);
-        const double here = rounds(DN_BIG, tn) * ((double)blocks * lines * (lines == 3 ? 1.22 : 1.03) + 16 + behind_big[epilogue]) + 4;
-        if (here < (groups == 0 ? 0.9 : rows > 1.4 * DN_BIG * groups ? 0.95 : 0.8) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
+        const double other = time(small[lines == 3], best.BM, (int64_t)best.tn * best.S, (double)((blocks + best.S - 1) / best.S) * per_block / 868, best.BM * best.BN / 16384.0) + (best.S > 1 ? 9 : 0);
+        const double here = time(large[lines == 3], DN_BIG, tn, (double)blocks, 1);
+        if (here < (groups == 0 ? 0.97 : rows > 1.4 * DN_BIG * groups ? 0.95 : 0.9) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
     }
     return best;
 }
