@@ -2,14 +2,14 @@
 // fp32 throughout on v_mfma_f32_16x16x4_f32 (one rounding per product, fp32 adds: a true fp32 product, no reduced-precision mode), or on the bf16 instruction with the operand as three bf16 lines
 // and the weights as they came (dn_ring_take, PL 3: no product is rounded at all).
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
-//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than one token: 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
+//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than one token (fp32: two to four by dn_few_first): 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
-//   dense_mm_big_kernel   the same operands, bf16, 256 x 256 tiles where they fill the chip in fewer rounds
+//   dense_mm_big_kernel   the same operands, bf16, 256 x 256 tiles where they are the faster ones (dn_ring_plan)
 //   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
 //   dense_mm_narrow_kernel bf16, K a multiple of 128 up to 1024, more than one token, few tiles: 32 x 32 tiles, the waves share K
 //   dense_mv1_kernel<WT,FORM,RAGGED> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
 //   dense_mv2_kernel<WT,U,RAGGED> the second product of a few tokens' experts: the waves of a work-group share a row, the activations in registers
-//   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns) of a K the ring does not take: the activation rows live in LDS, a wave streams RW weight rows at a time
+//   dense_mv_kernel<WT,C,RW> a few tokens (C <= 8 columns) of a K the ring does not take, and of fp32 where it is the faster one (dn_few_first): the activation rows live in LDS, a wave streams RW weight rows at a time
 // All take the same operand description (ps_seq.h psk_dense_args): ring rows, the token-shift mix and the epilogue
 // (bias, activation, scale, a factor from a second table) are part of the launch, so no mixer needs a kernel of its own around its projections.
 #include "ps_seq.h"
@@ -1060,8 +1060,8 @@ static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.ac
 // a split product pays a second launch and its parts' way through memory.
 //   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, fitted to 615 bf16 products of either form (K of
 // 512 to 14336, 130 to 2047 tokens, 0.1 to 8 rounds; 4 % off on average, 3 % for these) and 335 in three lines.  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  In us:
-// a round's blocks, its start and what the epilogue adds behind a tile (dn_epilogue), the results and the weights by their megabytes.  They are taken where that says 3 % less; for experts, whose last tiles are a
-// guess, a tenth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  4 of the 615 are then slower than
+// a round's blocks, its start and what the epilogue adds behind a tile (dn_epilogue), the results and the weights by their megabytes.  They are taken where that says 2 % less; for experts, whose last tiles are a
+// guess, a tenth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  3 of the 615 are then slower than
 // the others by 2 % or more (4 % at most) and none of the 335.  With 1700 clocks for a block of these in the estimate above it was one in nine and one in five: 512 tokens x 16384 x 2048 of gate / up pairs
 // take 64 us as 128 x 128 tiles and 80 as 256 x 256 (900: 119 and 89), 512 x 14336 x 4096 in three lines 206 and 251 (900: 391 and 257).
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
@@ -1077,13 +1077,13 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines
     const int64_t blocks = kbytes / 128;
     dn_ring_shape best{};
     double least = 0;
-    auto row_tiles = [&](int BM) { // (grouped: about half of the last tiles start a new one)
+    auto row_tiles = [&](int BM, bool over) { // (grouped: about half of the last tiles start a new one; over: an expert has more than a tile)
         const int full = (rows + BM - 1) / BM;
-        return groups > 0 ? std::max(full, std::min(groups, rows)) + (rows > groups * BM ? groups / 2 : 0) : full;
+        return groups > 0 ? std::max(full, std::min(groups, rows)) + (over ? groups / 2 : 0) : full;
     };
     for (auto &q : shapes) {
         const int BM = q[0], BN = q[1], n_tm = rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0), tn = (int)((N + BN - 1) / BN);
-        const int64_t tiles = (int64_t)row_tiles(BM) * tn;
+        const int64_t tiles = (int64_t)row_tiles(BM, rows > groups * BM) * tn;
         const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = std::max(lds, mfma) + 100;
         for (int64_t S = 1; S <= (may_split ? 16 : 1); S++) {
             if (S > 1 && (blocks / S < 4 || tiles * S > 512 || (size_t)n_tm * tn * S * BM * BN * 4 > psk_dense_split_bytes())) break;
@@ -1096,13 +1096,13 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines
         static const cost small[2] = {{2.4, 0.527, 0.55, 0.377, 0.058, {0, 0.9, 5.1}}, {4.3, 0.495, -2.4, 0.576, 0.056, {0, 0.9, 5.1}}}, large[2] = {{-2.5, 1.023, 12.8, 0.145, 0.079, {0, 7.4, 27.4}}, {-8.4, 1.177, 20, 0.153, 0.105, {0, 7.4, 27.4}}};
         const double results = rows * (double)N * 4e-6, weights = (double)N * kbytes * 1e-6 * std::max(groups, 1), per_block = std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100; // (clocks; 868 for 128 x 128)
         auto time = [&](const cost &c, int BM, int64_t columns, double blocks, double area) {
-            const double rounds = (double)(((columns + 7) / 8 * row_tiles(BM) + 31) / 32);
+            const double rounds = (double)(((columns + 7) / 8 * row_tiles(BM, rows >= groups * BM) + 31) / 32);
             return c.all + rounds * (blocks * lines * c.block + (c.round + c.behind[epilogue]) * area) + c.results * results + c.weights * weights;
         };
         const int tn = (int)((N + DN_BIG - 1) / DN_BIG), n_tm = rows / DN_BIG + (groups > 0 ? std::min(groups, rows) : rows % DN_BIG ? 1 : 0);
         const double other = time(small[lines == 3], best.BM, (int64_t)best.tn * best.S, (double)((blocks + best.S - 1) / best.S) * per_block / 868, best.BM * best.BN / 16384.0) + (best.S > 1 ? 9 : 0);
         const double here = time(large[lines == 3], DN_BIG, tn, (double)blocks, 1);
-        if (here < (groups == 0 ? 0.97 : rows > 1.4 * DN_BIG * groups ? 0.95 : 0.9) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
+        if (here < (groups == 0 ? 0.98 : rows > 1.4 * DN_BIG * groups ? 0.95 : 0.9) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
     }
     return best;
 }
