@@ -449,7 +449,11 @@ bool psk_split_attn_ok(int own, int shared, int dv) { return dv == 128 && own % 
 // From 80 work-groups on: below, the fp32 form's eight waves per 32 rows hide more than the faster instruction saves.  Attention of a layer in us, fp32 form | this one with its images (keys of
 // 192; behind nothing and behind 1024 tokens): 64 work-groups (512 tokens of 16 heads) 50 | 68, 84 | 132; 96 (768 of 16; 384 of 32) 110 | 95, 162 | 135; 70 | 57, 160 | 141; 128 156 | 120,
 // 166 | 137; 256 (2047 of 16, 1000 of 32) 318 | 142; 302 | 128, 319 | 160; keys of 128 with slopes: 1500 of 16 198 | 110.
-bool psk_split_attn_takes(int T, int H) { return (int64_t)((T + SA_ROWS - 1) / SA_ROWS) * H >= 80; }
+// And from where 16 rows and a head make more than 512: as many the fp32 form has at once on the chip, so fewer take it one pass however many heads there are, while this form splits the window's
+// numbers first for rows that fill little of a work-group.  A request of one layer in us, fp32 form | this one, behind 64 and behind 1000 tokens (windows, keys of 128): 80 heads, 1 row 59 | 67,
+// 64 | 117; 96 rows 107 | 109, 160 | 176; 112 rows 131 | 110, 224 | 181; 40 heads, 192 rows 99 | 103, 149 | 168; 224 rows 123 | 109, 219 | 173; 64 heads, 128 rows 102 | 108, 152 | 176;
+// 129 rows 126 | 113, 221 | 182; 128 heads, 64 rows 117 | 119, 173 | 188; 80 rows 139 | 127, 231 | 210.
+bool psk_split_attn_takes(int T, int H) { return (int64_t)((T + SA_ROWS - 1) / SA_ROWS) * H >= 80 && (int64_t)((T + 15) / 16) * H > 512; }
 static size_t sa_images(int G, int own, int shared, int dv, int64_t blocks) { return (size_t)blocks * ((size_t)G * (own / 32 * 6144 + dv / 16 * 3072) + (size_t)shared / 32 * 6144); }
 size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window) { return sa_images(G, own, shared, dv, (n_front + 31) / 32 + (n_window + 31) / 32) + (size_t)(G + 1) * ((n_front + 31) / 32 + (n_window + 31) / 32) * 4; }
 

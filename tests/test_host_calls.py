@@ -230,6 +230,26 @@ for spare, want in ((with_ - without, took), (with_ - without - 1 - 256, plain))
 """.replace(".dir", str(child.tmp / "dir")))
 
 
+def test_portions_whose_attention_is_split(child):
+    """k_splitattn.hip takes 80 work-groups of 128 rows and more, and more than 512 of 16: 129 rows of 64 heads and 193 of 40, not 128, 192 or 256 of 39, nor a single row of many heads; keys of 128
+    and 192 numbers, values of 128"""
+    child("""
+ctx = hip.Ctx(0)
+def took(tokens, heads, dim=128, vdim=128):
+    cfg = synth.zusolix_config(64, 30, [synth.zusolix_layer("attention", synth.zusolix_attention(heads, 1, dim, vdim, 0.1))])
+    synth.write_seq_model_dir(".dir", cfg, 1)
+    m = seqmodel.SeqModel(ctx, ".dir", max_batch=300, n_slots=1, max_context=400)
+    s = m.acquire()
+    fake.fake_reset()
+    m.forward(s, [1] * tokens)
+    n = count("split_keys_kernel"), count("split_attn_kernel"), count("winattn_mfma_kernel")
+    m.close()
+    return n
+for sizes in ((129, 64), (193, 40), (97, 80), (65, 128), (257, 32), (129, 64, 192)): assert took(*sizes) == (1, 1, 0), sizes
+for sizes in ((128, 64), (192, 40), (96, 80), (64, 128), (256, 39), (256, 32), (1, 80), (2, 128), (1, 200), (129, 64, 160), (129, 64, 128, 96)): assert took(*sizes)[:2] == (0, 0), sizes
+""".replace(".dir", str(child.tmp / "dir")))
+
+
 def test_the_measured_products_of_experts_are_the_ones_that_run(child):
     """ps_hip_seq_bench_kernel: a portion's second product of the experts reads the rounded rows of the first one, in a step and where it is measured"""
     child("""
