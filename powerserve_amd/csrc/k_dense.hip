@@ -1168,9 +1168,10 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
 }
 static bool dn_wide(hipStream_t st, const psk_dense_args &a, const dn_args &g) {
     if (a.w->dtype == PS_BF16) return dn_ring_take<unsigned short, 1>(st, a, g);
-    // (a small matrix and few rows: three lines are a launch more.  us on the fp32 instruction and in three lines, 64 tokens: 768 x 768 9.3 and 11.9, 1024 x 1024 10.0 and 12.0, 256 x 2048 9.8 and 12.0; 256
-    // tokens: 13.3 and 15.7, 12.6 and 15.5 for the latter two)
-    const bool small = a.small_f32 && !g.groups && !a.n_more && g.N * g.K <= (1 << 20) && a.T * g.N * g.K <= (1 << 28);
+    // (a small matrix and few rows: three lines are a launch more.  us on the fp32 instruction and in three lines, weights from memory: 16 tokens 768 x 2048 11.7 and 13.8, 2048 x 1024 12.0 and 13.9,
+    // 2048 x 2048 14.3 and 15.3, 1024 x 4096 14.7 and 16.1, 4096 x 2048 18.5 and 18.5; 64 tokens 768 x 768 9.3 and 11.9, 2048 x 1024 11.9 and 14.1, 2048 x 2048 14.2 and 15.5, 2048 x 4096 18.6 and 19.6;
+    // 128 tokens 2048 x 1024 13.4 and 14.8, 2048 x 2048 17.7 and 18.0, 4096 x 2048 29.2 and 22.3; 256 tokens 1024 x 1024 12.6 and 15.5, 2048 x 1024 17.8 and 18.7, 2048 x 2048 27.8 and 22.7)
+    const bool small = a.small_f32 && !g.groups && !a.n_more && g.N * g.K <= (1 << 22) && a.T * g.N * g.K <= (1 << 28);
     return (a.w->half && !small && dn_ring_take<unsigned short, 3>(st, a, g)) || dn_ring_take<float, 1>(st, a, g);
 }
 

@@ -320,7 +320,7 @@ def test_float32_products_of_odd_numbers(ctx, T, N, K, odd_weights, dtype):
     dx.free(); do.free()
 
 
-# a float32 model in either form of its matrices: four mixes, a feed-forward and a latent's window of more than 2^20 numbers (fewer run on the fp32 instruction in both: psk_dense_args small_f32),
+# a float32 model in either form of its matrices: four mixes, a feed-forward and a latent's window large enough (what is small runs on the fp32 instruction in both: psk_dense_args small_f32),
 # experts; a joint projection of two mixers; portions and single tokens
 @pytest.mark.parametrize("dtype", ["float32", "float32 lines"])
 @pytest.mark.parametrize("which", ["mixes", "experts", "joint"])
@@ -342,9 +342,8 @@ def test_float32_models_in_either_form(ctx, tmp_path, which, dtype):
     m.close()
 
 
-# a small matrix and few rows of a float32 model: on either side of the line between the fp32 instruction and three lines (k_dense.hip dn_wide), by rows (1024 x 1024: 256) and by the matrix (1024 x 1088)
-@pytest.mark.parametrize("ff", [1024, 1088])
-@pytest.mark.parametrize("sizes", [(256, 5), (257, 4)])
+# a small matrix and few rows of a float32 model: on either side of the line between the fp32 instruction and three lines (k_dense.hip dn_wide), by rows (1024 x 1024: 256; 1024 x 4096: 64) and by the matrix (1024 x 4160)
+@pytest.mark.parametrize("ff,sizes", [(1024, (256, 5)), (1024, (257, 4)), (4096, (64, 65)), (4160, (64, 9))])
 def test_small_float32_products(made, ff, sizes):
     cfg = synth.seq_config(1024, 40, [L("delta", ff, heads=2, kv_heads=1, dim=16, vdim=16, conv=2)], taps=2)
     m, c, t = made(f"small-f32.{ff}", max_batch=260, cfg=cfg)
@@ -669,6 +668,7 @@ def test_a_long_input_in_launch_sequences_wider_than_max_batch(ctx, tmp_path, dt
     cfg = CONFIGS["mixed"]
     t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
     m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype, max_batch=max_batch, n_slots=1, max_context=max_context)
+    assert m.launch_rows == {64: 256, 150: 500, 63: 63}[max_batch]
     toks = tokens_for(cfg, n, seed=6)
     # (bfloat16: against calls of max_batch tokens.  Rounding alone moves row 151 by 0.1175, in portions of any size and token by token; another cut may round it the other way: a tenth of that)
     rows, tol = (seq_oracle.run(cfg, t, toks), TOL[dtype]) if dtype == "float32" else (run_portions(m, toks, (max_batch,)), 0.012)
