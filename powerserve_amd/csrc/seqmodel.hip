@@ -106,9 +106,10 @@ static int seq_fail(ps_hip_ctx *c, const std::string &msg) { c->err = msg; retur
 static uint64_t dense_bytes(const ps_dense *w) { return w ? (uint64_t)w->N * w->K * (w->dtype == PS_BF16 ? 2 : 4) : 0; }
 
 // Tokens of a launch sequence for an input longer than max_batch.  The wider it is, the fewer launches (5 us of a small one is its start), the larger the tiles that still fill the chip,
-// the fewer partly empty ones of an expert, and the fewer expansions of one window's keys: Ranutar 2048 x 6, 2047 tokens behind max_batch 512 in portions of 512, 1024, 2048: 5552, 4527,
-// 3947 us; Pupidra 2048 x 6, 1500 tokens: 6118, 5060, 4280.  Not below 64, where the caller has asked for little memory; no more than four times what was asked for, and no more than
-// 2048, behind which the tiles fill the chip anyway.
+// the fewer partly empty ones of an expert, and the fewer expansions of one window's keys.  Requests behind max_batch 512 in sequences of 512 | 2048, in us, 600 and 2047 tokens: Ranutar 2048 x 6
+// 2072 | 1580, 5200 | 2904; Pupidra 3127 | 2029, 8139 | 4186; Vobisun 3323 | 2383, 8640 | 4749; Sogavik 4503 | 3219, 11269 | 5908; Pokatar 3242 | 2085, 8731 | 4177; Zusolix 3082 | 2223,
+// 8223 | 4720; 1024 x 6: 1350 | 935, 3308 | 1981.  Not below 64, where the caller has asked for little memory; no more than four times what was asked for, and no more than 2048, behind which the
+// tiles fill the chip anyway.
 static int64_t seq_rows(const ps_seq_desc *d, int times) {
     const int64_t B = d->max_batch, most = d->max_context > 0 ? d->max_context : 65536;
     return B < 64 ? B : std::max(B, std::min<int64_t>({times * B, 2048, most}));
