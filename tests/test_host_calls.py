@@ -121,13 +121,13 @@ for dtype, form, want in (("bfloat16", None, hip.DENSE_BF16), ("float32", None, 
 
 
 def test_a_joint_projection_without_room_for_its_second_form(child):
-    """ps_hip_seq_create: of all the memory a float32 model asks for, the bfloat16 form of two mixers' joint projection is the one piece that it can do without; its products then run as fp32 ones"""
+    """ps_hip_seq_create: of all the memory a float32 model asks for, the bfloat16 form of two mixers' joint projection is the one piece that it can do without; a portion's products then run as fp32 ones"""
     child("""
 ctx = hip.Ctx(0)
 att = {"heads": 8, "kv_heads": 1, "dim": 64, "vdim": 64, "mask": {"size": 9, "pool": 3}, "rot": {"base": 100.0, "dims": 8}, "scale": 0.2}
 cfg = synth.parallel_config(1024, 30, [synth.parallel_layer(None, att, {"heads": 8, "dim": 64, "vdim": 64, "tau": 4.0}, 1.0, 0.5)], taps=2)
 synth.write_seq_model_dir(".dir", cfg, 1)
-def load(): return seqmodel.SeqModel(ctx, ".dir", dtype="float32", max_batch=8)
+def load(): return seqmodel.SeqModel(ctx, ".dir", dtype="float32", max_batch=200, launch_rows=200)
 fake.fake_reset()
 load().close()
 took = []
@@ -138,14 +138,14 @@ for n in range(1, count("hipMalloc") + 1):
     except hip.PSHipError: continue
     s = m.acquire()
     fake.fake_reset()
-    m.forward(s, [1] * 8, want=[7])
+    m.forward(s, [1] * 200, want=[199])
     took.append((count("dense_mm_ring_kernelIf"), count("dense_mm_ring_kernelIt"), fake.fake_stray()))
     m.close()
 fake.fake_reset()
 m = load()
 s = m.acquire()
 fake.fake_reset()
-m.forward(s, [1] * 8, want=[7])
+m.forward(s, [1] * 200, want=[199])
 f32, lines = count("dense_mm_ring_kernelIf"), count("dense_mm_ring_kernelIt")
 assert lines > 0 and took == [(f32 + 1, lines - 1, 0)], (took, f32, lines)
 """.replace(".dir", str(child.tmp / "dir")))
