@@ -91,7 +91,6 @@ struct sa_keys {
     int ks_own, ks_shared, nj;      // k steps of 32 numbers of a head's own key part and of the shared one, value tiles of 16 columns
     int G;
     char *img, *img_shared;
-    int *odd; // [G + 1][nb]: does an image hold a number that is not finite (the shared ones last)
 };
 static __device__ __forceinline__ const float *sa_row(const sa_rows &r, long long step, int j) {
     int n = j + r.off;
@@ -104,7 +103,6 @@ __global__ __launch_bounds__(256) void split_keys_kernel(sa_keys a) {
     const int i0 = 32 * (front ? b : b - a.nbf), n = front ? a.n_front : a.n_window; // rows i0 .. i0 + 31 of those that exist
     const int ks = shared ? a.ks_shared : a.ks_own, nk = ks * 128, nv = shared ? 0 : a.nj * 64; // sixteen-byte pieces per plane
     char *out = shared ? a.img_shared + (size_t)b * a.ks_shared * 6144 : a.img + ((size_t)g * a.nb + b) * (a.ks_own * 6144 + a.nj * 3072);
-    int odd = 0;
     for (int x = tid; x < nk + nv; x += 256) {
         float v[8];
         sa_u4 p[3];
@@ -133,17 +131,12 @@ __global__ __launch_bounds__(256) void split_keys_kernel(sa_keys a) {
 #pragma unroll
             for (int q = 0; q < 3; q++) *(sa_u4 *)(out + ks * 6144 + (ct * 3 + q) * 1024 + lane * 16) = p[q];
         }
-#pragma unroll
-        for (int e = 0; e < 8; e++) odd |= !sa_finite(v[e]);
     }
-    odd = __syncthreads_or(odd);
-    if (tid == 0) a.odd[g * a.nb + b] = odd;
 }
 
 // ---------------------------------------------------------------------------------------------------- attention
 struct sa_attn {
     const char *img, *img_shared;
-    const int *odd, *odd_shared;
     int nbf, nb, ks_own, hpg;      // (heads per image)
     int pos0, first, T, window, pool, keep; // position of row 0, of window row 0
     const float *q;
@@ -182,8 +175,6 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     const int own = a.ks_own * 6, image = own + NJ * 3; // pieces of a head's own key part, of its image
     const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)sa_smem;
     auto block_of = [&](const int it) { return it < nfb ? it : a.nbf + wb0 + it - nfb; };
-    const int *odd_own = a.odd + (size_t)g * a.nb;
-    const int odd1 = lane < blocks ? odd_own[block_of(lane)] : 0, odd2 = lane < blocks && own < KS * 6 ? a.odd_shared[block_of(lane)] : 0; // (asked for here, looked at behind the loop)
     auto request = [&](const int it) {
         const int b = block_of(it);
         const char *im = a.img + ((size_t)g * a.nb + b) * (image * 1024), *sh = a.img_shared + (size_t)b * ((KS * 6 - own) * 1024);
@@ -356,16 +347,15 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
         }
     }
     if (!alive) return;
-    // An infinite number's lower lines are zeros that the other operand's leading line meets, and it meets the other's lower lines, whose signs are their own: no number, where fp32 arithmetic has an
-    // infinite score or result.  Where a query of the wave or a key or value of its blocks is not finite, the wave does it all again with the lines joined, on the fp32 instruction, the images straight
-    // from memory.
-    int odd = odd1 | odd2;
-    for (int it = lane + 64; it < blocks; it += 64) odd |= odd_own[block_of(it)] | (own < KS * 6 ? a.odd_shared[block_of(it)] : 0);
+    // An infinite number's lower lines are zeros that the other operand's leading line meets, and it meets the other's lower lines, whose signs are their own: the infinite number that fp32 arithmetic
+    // has, or no number; and one of a key that a row does not see meets its weight's zeros.  No number among the scores ends in the sum of the weights, among the products in the results: where a row
+    // of the wave has one there, or an infinite one, the wave does it all again with the lines joined, on the fp32 instruction, the images straight from memory.
+    float odd = l * 0.f;
 #pragma unroll
-    for (int s = 0; s < KS; s++)
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) odd |= !sa_finite(__uint_as_float(q[s][0][e] << 16)) | !sa_finite(__uint_as_float(q[s][0][e] & 0xffff0000u));
-    if (__builtin_expect(__any(odd), 0)) { // (uniform)
+        for (int i = 0; i < 4; i++) odd = fmaf(acc[j][i], 0.f, odd);
+    if (__builtin_expect(__any(!sa_finite(odd)), 0)) { // (uniform)
         m = -INFINITY;
         l = 0.f;
 #pragma unroll
@@ -455,7 +445,7 @@ bool psk_split_attn_ok(int own, int shared, int dv) { return dv == 128 && own % 
 // 129 rows 126 | 113, 221 | 182; 128 heads, 64 rows 117 | 119, 173 | 188; 80 rows 139 | 127, 231 | 210.
 bool psk_split_attn_takes(int T, int H) { return (int64_t)((T + SA_ROWS - 1) / SA_ROWS) * H >= 80 && (int64_t)((T + 15) / 16) * H > 512; }
 static size_t sa_images(int G, int own, int shared, int dv, int64_t blocks) { return (size_t)blocks * ((size_t)G * (own / 32 * 6144 + dv / 16 * 3072) + (size_t)shared / 32 * 6144); }
-size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window) { return sa_images(G, own, shared, dv, (n_front + 31) / 32 + (n_window + 31) / 32) + (size_t)(G + 1) * ((n_front + 31) / 32 + (n_window + 31) / 32) * 4; }
+size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window) { return sa_images(G, own, shared, dv, (n_front + 31) / 32 + (n_window + 31) / 32); }
 
 template <int KS, int NJ, bool DIST>
 static void sa_launch(hipStream_t st, const sa_attn &a, int H) {
@@ -474,9 +464,8 @@ void psk_split_attn(hipStream_t st, const psk_split_attn_args &x) {
     k.ks_own = x.own / 32; k.ks_shared = x.n_shared / 32; k.nj = 8; k.G = x.G;
     k.img = (char *)x.scratch;
     k.img_shared = k.img + (size_t)x.G * k.nb * (k.ks_own * 6144 + k.nj * 3072);
-    k.odd = (int *)(k.img + sa_images(x.G, x.own, x.n_shared, 128, k.nb));
     hipLaunchKernelGGL(split_keys_kernel, dim3(k.nb, x.G + (x.n_shared > 0)), dim3(256), 0, st, k);
-    sa_attn a{k.img, k.img_shared, k.odd, k.odd + (size_t)x.G * k.nb, k.nbf, k.nb, k.ks_own, x.H / x.G, (int)x.pos0, (int)x.first, x.T, x.window, x.pool, x.keep, x.q, x.ldq, x.own + x.n_shared, x.own, x.rot_dims, x.pairing, x.freq,
+    sa_attn a{k.img, k.img_shared, k.nbf, k.nb, k.ks_own, x.H / x.G, (int)x.pos0, (int)x.first, x.T, x.window, x.pool, x.keep, x.q, x.ldq, x.own + x.n_shared, x.own, x.rot_dims, x.pairing, x.freq,
               x.rot_mag, x.scale, x.softcap, x.temp, x.slope, x.sink, x.gate, x.ldg, x.gate_elem, x.o, x.ldo};
     if (x.own + x.n_shared == 192) x.slope ? sa_launch<6, 8, true>(st, a, x.H) : sa_launch<6, 8, false>(st, a, x.H);
     else x.slope ? sa_launch<4, 8, true>(st, a, x.H) : sa_launch<4, 8, false>(st, a, x.H);
