@@ -455,7 +455,7 @@ static void dn_launch_mv_grouped(hipStream_t st, const dn_args &g, int rows, siz
 //     behind it block k may be read and the stage of block k - 1 refilled.
 //   * Operand fragments: 16 bytes per lane.  bf16: the eight k of v_mfma_f32_32x32x16_bf16.  fp32: four k, one per v_mfma_f32_32x32x2_f32 (lanes 0-31 and 32-63 hold different k;
 //     both operands use the same assignment, so every k meets itself).
-//   * Work-group order: the token tiles of one weight piece sit 8 apart -- same XCD, same time -- so a weight is fetched into one L2 once.
+//   * Work-group order: dn_ring_place.
 // Rows beyond T and outputs beyond N repeat the last one and are not stored.
 // Measured (kernel trace, before -> now, bf16, 512 tokens): 2048 x 2048 45 -> 14 us, 8192 x 2048 72 -> 32 us (7 of them the xIELU of its epilogue), 2048 x 8192 190 -> 25 + 13 us (the
 // sum); fp32, 300 tokens: 2048 x 2048 180 -> 30 + 11 us, 2048 x 8192 700 -> 103 + 11 us.  Loading alone takes 1030 cycles a block of 32 KiB, multiplying alone 530.  Tried and not
@@ -629,6 +629,32 @@ static __device__ __forceinline__ bool dn_ring_rows(const dn_args &g, int tm, in
     return t0 < T;
 }
 
+// The tile and split of a work-group.  Work-group b runs on XCD b % 8: an XCD has an eighth of the items there are, neighbours in the order of panels of four output tiles, so its L2 sees few token
+// rows and few weights at a time, and no XCD has a column more than another.  With whole columns of tiles per XCD 1500 x 10304 of K = 2048 (41 columns of six tiles: 36 for one XCD, 30 for others) took
+// two rounds, 97 us; 67 so.  Whole requests: pupidra-prompt 3 406 -> 3 245 us, ranutar-f32-prompt 963 -> 919, ranutar-prompt 2 875 -> 2 812, ranutar-prompt-ragged 859 -> 847.
+#define DN_PANEL 4
+template <int BM>
+static __device__ __forceinline__ bool dn_ring_place(const dn_args &g, const dn_ring &p, int &tm, int &tn, int &s) {
+    int n_tm = p.n_tm;
+    if (g.g_seg) { // (the host's number is a bound)
+        n_tm = 0;
+        for (int e = 0, at = g.g_seg[0]; e < g.groups; e++) {
+            const int next = g.g_seg[e + 1];
+            n_tm += (next - at + BM - 1) / BM;
+            at = next;
+        }
+    }
+    const int tiles = n_tm * p.tn, items = tiles * p.S, each = (items + 7) >> 3, j = (int)blockIdx.x >> 3;
+    int i = ((int)blockIdx.x & 7) * each + j;
+    if (j >= each || i >= items) return false;
+    s = p.S > 1 ? i / tiles : 0;
+    i -= s * tiles;
+    const int panel = i / (n_tm * DN_PANEL), width = min(DN_PANEL, p.tn - panel * DN_PANEL), r = i - panel * n_tm * DN_PANEL;
+    tm = r / width;
+    tn = panel * DN_PANEL + r % width;
+    return true;
+}
+
 template <typename WT, int BM, int BN, bool ODD, int PL>
 __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p) {
     extern __shared__ __attribute__((aligned(16))) char dn_lds[];
@@ -636,10 +662,8 @@ __global__ __launch_bounds__(512) void dense_mm_ring_kernel(dn_args g, dn_ring p
     constexpr int NA = BM / 32, NW = BN / 32, WL = NS * BM * 128; // PL 3: of them of the operand and of the weights; where the weights' two stages begin
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = (wave >> 1) & 1, wn = wave & 1;
     const bool loads = wave >= 4;
-    const int per = 8 * p.n_tm, b_in = (int)blockIdx.x % per, wp = ((int)blockIdx.x / per) * 8 + (b_in & 7), tm = b_in >> 3;
-    if (wp >= p.tn * p.S) return;
-    const int s = wp % p.S, tn = wp / p.S;
-    int e, T, t0;
+    int tm, tn, s, e, T, t0;
+    if (!dn_ring_place<BM>(g, p, tm, tn, s)) return; // (uniform per work-group)
     long long row0;
     if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return; // (uniform per work-group)
     const long long n0 = (long long)tn * BN, ldw = g.K * (long long)sizeof(WT);
@@ -879,9 +903,8 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
     extern __shared__ __attribute__((aligned(16))) char dn_lds[];
     constexpr int BM = DN_BIG, BN = DN_BIG, HALF = 128 * 128;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3;
-    const int per = 8 * p.n_tm, b_in = (int)blockIdx.x % per, tn = ((int)blockIdx.x / per) * 8 + (b_in & 7), tm = b_in >> 3;
-    if (tn >= p.tn) return;
-    int e, T, t0;
+    int tm, tn, s, e, T, t0;
+    if (!dn_ring_place<BM>(g, p, tm, tn, s)) return; // (uniform per work-group)
     long long row0;
     if (!dn_ring_rows<BM>(g, tm, e, row0, T, t0)) return; // (uniform per work-group)
     const long long n0 = (long long)tn * BN, ldw = g.K * 2;
@@ -1059,7 +1082,7 @@ static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.ac
 // of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more; rounds of 256 work-groups (one per CU);
 // a split product pays a second launch and its parts' way through memory.
 //   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, fitted to 615 bf16 products of either form (K of
-// 512 to 14336, 130 to 2047 tokens, 0.1 to 8 rounds; 4 % off on average, 3 % for these) and 335 in three lines.  A round is 32 work-groups of an XCD, whose columns are whole (the kernels' order).  In us:
+// 512 to 14336, 130 to 2047 tokens, 0.1 to 8 rounds; 4 % off on average, 3 % for these) and 335 in three lines.  In us:
 // a round's blocks, its start and what the epilogue adds behind a tile (dn_epilogue), the results and the weights by their megabytes.  They are taken where that says 2 % less; for experts, whose last tiles are a
 // guess, a tenth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  3 of the 615 are then slower than
 // the others by 2 % or more (4 % at most) and none of the 335.  With 1700 clocks for a block of these in the estimate above it was one in nine and one in five: 512 tokens x 16384 x 2048 of gate / up pairs
@@ -1096,7 +1119,7 @@ static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines
         static const cost small[2] = {{2.4, 0.527, 0.55, 0.377, 0.058, {0, 0.9, 5.1}}, {4.3, 0.495, -2.4, 0.576, 0.056, {0, 0.9, 5.1}}}, large[2] = {{-2.5, 1.023, 12.8, 0.145, 0.079, {0, 7.4, 27.4}}, {-8.4, 1.177, 20, 0.153, 0.105, {0, 7.4, 27.4}}};
         const double results = rows * (double)N * 4e-6, weights = (double)N * kbytes * 1e-6 * std::max(groups, 1), per_block = std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100; // (clocks; 868 for 128 x 128)
         auto time = [&](const cost &c, int BM, int64_t columns, double blocks, double area) {
-            const double rounds = (double)(((columns + 7) / 8 * row_tiles(BM, rows >= groups * BM) + 31) / 32);
+            const double rounds = (double)((columns * row_tiles(BM, rows >= groups * BM) + 255) / 256);
             return c.all + rounds * (blocks * lines * c.block + (c.round + c.behind[epilogue]) * area) + c.results * results + c.weights * weights;
         };
         const int tn = (int)((N + DN_BIG - 1) / DN_BIG), n_tm = rows / DN_BIG + (groups > 0 ? std::min(groups, rows) : rows % DN_BIG ? 1 : 0);
@@ -1114,7 +1137,7 @@ static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
     constexpr int LDS = DN_STAGES * (BM + BN) * 128;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_ring_kernel<WT, BM, BN, ODD, PL>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-    const unsigned grid = (unsigned)((p.tn * p.S + 7) / 8 * 8) * p.n_tm;
+    const unsigned grid = (unsigned)(((long long)p.tn * p.S * p.n_tm + 7) / 8 * 8);
     hipLaunchKernelGGL((dense_mm_ring_kernel<WT, BM, BN, ODD, PL>), dim3(grid), dim3(512), LDS, st, g, p);
     if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN, ODD>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
 }
@@ -1125,7 +1148,7 @@ static void dn_launch_big(hipStream_t st, const dn_args &g, const dn_ring &p) {
         if (dn_odd(g)) return dn_launch_big<true, PL>(st, g, p);
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_big_kernel<ODD, PL>, hipFuncAttributeMaxDynamicSharedMemorySize, DN_BIG_LDS);
-    hipLaunchKernelGGL((dense_mm_big_kernel<ODD, PL>), dim3((unsigned)((p.tn + 7) / 8 * 8) * p.n_tm), dim3(512), DN_BIG_LDS, st, g, p);
+    hipLaunchKernelGGL((dense_mm_big_kernel<ODD, PL>), dim3((unsigned)(((long long)p.tn * p.n_tm + 7) / 8 * 8)), dim3(512), DN_BIG_LDS, st, g, p);
 }
 
 // The wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed.  PL 3 (WT: bf16): an fp32 product on the bf16 instruction -- the weights as they came, which is in
