@@ -2,9 +2,9 @@
 // fp32 throughout on v_mfma_f32_16x16x4_f32 (one rounding per product, fp32 adds: a true fp32 product, no reduced-precision mode), or on the bf16 instruction with the operand as three bf16 lines
 // and the weights as they came (dn_ring_take, PL 3: no product is rounded at all).
 //   dense_mm_kernel<WT>   tiled mat-mul, 64 tokens x 64 outputs per work-group of four waves, any T / N / K (edges zero-filled)
-//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than one token (fp32: two to four by dn_few_first): 128 x 128 or 64 x 128 tiles over an operand packed by dense_pack_kernel (fp32: in place where its rows
+//   dense_mm_ring_kernel  rows of K in whole 128-byte blocks, more than one token (fp32: two to four by dn_few_first): tiles of 64 x 64 to 192 x 128 over an operand packed by dense_pack_kernel (fp32: in place where its rows
 //                         are plain), split along K where the tiles do not fill the chip (dense_mm_sum_kernel adds the parts)
-//   dense_mm_big_kernel   the same operands, bf16, 256 x 256 tiles where they are the faster ones (dn_ring_plan)
+//   dense_mm_big_kernel   the same operands, bf16, tiles of 128, 192 or 256 rows x 256 columns where they are the faster ones (dn_ring_plan)
 //   dense_mm_few_kernel   K up to 32, more than 8 tokens: a thread per output column
 //   dense_mm_narrow_kernel bf16, K a multiple of 128 up to 1024, more than one token, few tiles: 32 x 32 tiles, the waves share K
 //   dense_mv1_kernel<WT,FORM,RAGGED> a single token, or a few tokens' experts' first product: every wave streams its rows, the requests run ahead of everything else
@@ -443,7 +443,7 @@ static void dn_launch_mv_grouped(hipStream_t st, const dn_args &g, int rows, siz
 }
 
 // ---------------------------------------------------------------------------------------------------- wide mat-mul (bf16: K % 64 == 0, fp32: K % 32 == 0)
-// BM x BN (128 x 128, 64 x 128 or 64 x 64) tokens x outputs per work-group: four waves multiply, four load.  Both operands in blocks of 128 bytes of K per row (64 bf16 or 32 fp32)
+// BM x BN (192 x 128, 128 x 128, 64 x 128 or 64 x 64) tokens x outputs per work-group: four waves multiply, four load.  Both operands in blocks of 128 bytes of K per row (64 bf16 or 32 fp32)
 // through a ring of four LDS stages that the memory system fills by itself (global_load_lds_dwordx4: no registers, three blocks in flight).  What bounded the form before this one --
 // 128 x 128 tiles, one block in flight through registers, two barriers per block -- was the latency of a block: 512 x 2048 x 2048 has 64 such tiles, one wave per SIMD on a quarter
 // of the chip.  Hence the ring, smaller tiles or SPLITS of K where the tiles are fewer than the CUs (dn_ring_plan): a split product's partial tiles go to a scratch in register
@@ -884,24 +884,24 @@ __global__ __launch_bounds__(256) void dense_mm_sum_kernel(dn_args g, dn_ring p)
     if (t < T) dn_put4<ODD>(g, dn_orow(g, row0, t, T), (long long)tn * BN + wn * NJ * 32 + (ij % NJ) * 32 + c, *(const dn_f4 *)&turn[r * 36 + c]);
 }
 
-// 256 x 256 tiles, for products that fill the chip with them (bf16).  Eight waves, a wave 64 x 32 of each quarter of the tile; K in blocks of 64, two LDS stages in four pieces of 128 rows (half
-// of the tokens' rows or of the weights').  A block is four phases, one per quarter, a phase two slots: in one a wave reads fragments and requests a piece, in the other it multiplies (sixteen
-// instructions), and the waves 4 - 7 are one slot behind the waves 0 - 3 of the same SIMDs, so that the matrix cores have one wave of a SIMD in every slot while the other's requests and reads hold
-// only that one.  A piece is requested over the one that all waves have just read (both groups' reads are back at the barrier in front), six phases before it is read itself; a wait per
-// phase is for all but the six youngest pieces.
-// What bounded the 128 x 128 tiles here were the bytes from L2 (64 a clock and CU for the matrix instructions' rate, half of that comes) and the reads in front of them; these take half of both per
-// product.  Without requests and reads a block takes 1.03 us, the matrix instructions at the 2 GHz they hold; 1.15 as it is.  2047 tokens, bf16, in the 128 x 128 form and here: 8192 x 2048
-// 122 -> 59 us (16 of them the 67 MB of results, behind the last product of a CU's only tile), 6208 x 2048 96 -> 57; 1000 tokens 14336 x 4096 177 -> 117.
+// Tiles of 64 MI rows (MI 2, 3 or 4) x 256 columns, bf16.  Eight waves, a wave 16 MI x 32 of each quarter of the tile; K in blocks of 64, two LDS stages in four pieces (half of the tokens' rows or of
+// the weights').  A block is two phases, one per half of the tokens' rows, a phase two slots: in one a wave reads fragments and requests pieces, in the other it multiplies (8 MI instructions), and the
+// waves 4 - 7 are one slot behind the waves 0 - 3 of the same SIMDs, so that the matrix cores have one wave of a SIMD in every slot while the other's requests and reads hold only that one.  Pieces are
+// requested over what all waves have just read (both groups' reads are back at the barrier in front), three phases before they are read themselves; a wait per phase is for all but the requests of the
+// youngest two phases.  (Four phases, one per quarter, held a block of any height to 1.1 us, the time of eight slots of reads and requests: 1 090 x 6 208 of K = 4 096 in tiles of 128 rows 80 -> 72 us.)
+// What bounded the 128 x 128 tiles here were the bytes from L2 (dn_ring_plan); these take half to three quarters of them per product.  A block takes 1.05 us with 256 rows (the matrix instructions
+// alone 1.03, at the 2 GHz they hold), 0.88 with 192, 0.72 with 128.  2047 tokens, bf16, in the 128 x 128 form and here: 8192 x 2048 122 -> 59 us (16 of them the 67 MB of results, behind the last
+// product of a CU's only tile); 1000 tokens 14336 x 4096 177 -> 117.  The heights against 256 rows only: 900 x 8192 x 4096 88 -> 74, 1532 x 8192 x 14336 332 -> 292.
 #define DN_BIG 256
-#define DN_BIG_LDS ((DN_BIG / 2) * (DN_BIG + 4) * 4)
+static constexpr int dn_big_lds(int MI) { return std::max(4 * (32 * MI + 128) * 128, 32 * MI * (DN_BIG + 4) * 4); } // the stages, then half of the tile
 static __device__ __forceinline__ void dn_dma_at(const char *base, unsigned off, unsigned lds_dst) { // (as dn_dma, from a uniform base)
     unsigned keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst) : "memory");
 }
-template <bool ODD, int PL>
+template <bool ODD, int PL, int MI>
 __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p) {
     extern __shared__ __attribute__((aligned(16))) char dn_lds[];
-    constexpr int BM = DN_BIG, BN = DN_BIG, HALF = 128 * 128;
+    constexpr int BM = 64 * MI, BN = DN_BIG, HR = 32 * MI, HALF_A = HR * 128, HALF = 128 * 128; // (HR: rows of a half of the tokens)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3;
     int tm, tn, s, e, T, t0;
     if (!dn_ring_place<BM>(g, p, tm, tn, s)) return; // (uniform per work-group)
@@ -921,41 +921,51 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
     }
     A += (g.g_seg ? row0 + t0 : t0) * p.lda;
     W += nw * ldw;
-    unsigned oa[2][2], ob[2][2];
+    // A piece of HR rows is 4 MI requests: where they are not a multiple of the waves, the waves 0 - 3 have one more of the first half and 4 - 7 of the second
+    constexpr int NA = (MI + 1) / 2;
+    unsigned oa[2][NA], ob[2][2];
+    auto piece = [&](const int h, const int j) { return MI == 3 ? (j ? 8 + (wave & 3) : wave) : NA * wave + j; };
+    auto has = [&](const int h, const int j) { return MI != 3 || j == 0 || (wm != 0) == (h != 0); }; // (uniform)
 #pragma unroll
-    for (int h = 0; h < 2; h++)
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int j = 0; j < NA; j++) {
+            const int r = 8 * piece(h, j) + (lane >> 3), kq = (lane & 7) ^ ((r >> 1) & 7);
+            oa[h][j] = (unsigned)min(h * HR + r, T - 1 - t0) * (unsigned)p.lda + kq * 16;
+        }
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int r = 16 * wave + 8 * j + (lane >> 3), kq = (lane & 7) ^ ((r >> 1) & 7);
-            oa[h][j] = (unsigned)min(h * 128 + r, T - 1 - t0) * (unsigned)p.lda + kq * 16;
             ob[h][j] = (unsigned)min((long long)(h * 128 + r), n_rows - 1 - nw) * (unsigned)ldw + kq * 16;
         }
-    const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)dn_lds + (unsigned)(wave * 2048);
+    }
+    const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)dn_lds;
     auto request_a = [&](const int kb, const int h) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) dn_dma_at(A + (PL == 3 ? kb % 3 * ldw + (long long)(kb / 3) * 128 : (long long)kb * 128), oa[h][j], lds0 + (unsigned)((2 * (kb & 1) + h) * HALF + j * 1024));
+        for (int j = 0; j < NA; j++)
+            if (has(h, j)) dn_dma_at(A + (PL == 3 ? kb % 3 * ldw + (long long)(kb / 3) * 128 : (long long)kb * 128), oa[h][j], lds0 + (unsigned)((2 * (kb & 1) + h) * HALF_A + piece(h, j) * 1024));
     };
     auto request_w = [&](const int kb, const int h) { // (PL 3: kb counts blocks of K)
 #pragma unroll
-        for (int j = 0; j < 2; j++) dn_dma_at(W + (long long)kb * 128, ob[h][j], lds0 + (unsigned)((4 + 2 * (kb & 1) + h) * HALF + j * 1024));
+        for (int j = 0; j < 2; j++) dn_dma_at(W + (long long)kb * 128, ob[h][j], lds0 + (unsigned)(4 * HALF_A + (2 * (kb & 1) + h) * HALF + wave * 2048 + j * 1024));
     };
-    dn_f4 acc[2][2][4][2], xa[2][4], xb[2][2][2]; // (tokens' half, weights' half)
+    dn_f4 acc[2][2][MI][2], xa[2][MI], xb[2][2][2]; // (tokens' half, weights' half)
 #pragma unroll
     for (int mh = 0; mh < 2; mh++)
 #pragma unroll
         for (int nh = 0; nh < 2; nh++)
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
                 for (int j = 0; j < 2; j++) acc[mh][nh][i][j] = dn_f4{0.f, 0.f, 0.f, 0.f};
     const int fr = lane & 15, po = (((lane >> 4) ^ (fr >> 1)) << 4); // (row bases are multiples of sixteen; the second half of a block: the piece's number with its third bit turned)
-    const char *fa[2] = {dn_lds + (wm * 64 + fr) * 128 + po, dn_lds + (wm * 64 + fr) * 128 + (po ^ 64)};
-    const char *fb[2] = {dn_lds + 4 * HALF + (wn * 32 + fr) * 128 + po, dn_lds + 4 * HALF + (wn * 32 + fr) * 128 + (po ^ 64)};
+    const char *fa[2] = {dn_lds + (wm * 16 * MI + fr) * 128 + po, dn_lds + (wm * 16 * MI + fr) * 128 + (po ^ 64)};
+    const char *fb[2] = {dn_lds + 4 * HALF_A + (wn * 32 + fr) * 128 + po, dn_lds + 4 * HALF_A + (wn * 32 + fr) * 128 + (po ^ 64)};
     auto read_a = [&](const int kb, const int h) {
 #pragma unroll
         for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) xa[u][i] = *(const dn_f4 *)(fa[u] + (2 * (kb & 1) + h) * HALF + i * 2048);
+            for (int i = 0; i < MI; i++) xa[u][i] = *(const dn_f4 *)(fa[u] + (2 * (kb & 1) + h) * HALF_A + i * 2048);
     };
     auto read_w = [&](const int kb, const int h) {
 #pragma unroll
@@ -963,7 +973,7 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #pragma unroll
             for (int j = 0; j < 2; j++) xb[h][u][j] = *(const dn_f4 *)(fb[u] + (2 * ((PL == 3 ? kb / 3 : kb) & 1) + h) * HALF + j * 2048);
     };
-    auto multiply = [&](const int mh, const int nh) { // between two barriers: the other group's slot of reads and requests
+    auto multiply = [&](const int mh) { // between two barriers: the other group's slot of reads and requests
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
@@ -971,59 +981,51 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #pragma unroll
         for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    dn_bf8 za, zb;
-                    __builtin_memcpy(&za, &xa[u][i], 16);
-                    __builtin_memcpy(&zb, &xb[nh][u][j], 16);
-                    acc[mh][nh][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(zb, za, acc[mh][nh][i][j], 0, 0, 0);
-                }
+                for (int nh = 0; nh < 2; nh++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        dn_bf8 za, zb;
+                        __builtin_memcpy(&za, &xa[u][i], 16);
+                        __builtin_memcpy(&zb, &xb[nh][u][j], 16);
+                        acc[mh][nh][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(zb, za, acc[mh][nh][i][j], 0, 0, 0);
+                    }
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    if constexpr (PL == 3) {
-        request_w(0, 0); request_a(0, 0); request_w(0, 1); request_a(0, 1); request_a(1, 0); request_a(1, 1);
-    } else {
-        for (int kb = 0; kb < min(nk, 2); kb++) { request_w(kb, 0); request_a(kb, 0); request_w(kb, 1); request_a(kb, 1); }
-    }
-    if (PL == 3) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (nk > 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    read_w(0, 0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    // requests behind the piece that is waited for: those of two phases (PL 3: of them the operand's)
+    constexpr int LATER = MI + (PL == 3 ? 0 : 4);
+    request_w(0, 0); request_w(0, 1); request_a(0, 0); request_a(0, 1);
+    if (nk > 1) {
+        if (PL == 1) { request_w(1, 0); request_w(1, 1); }
+        request_a(1, 0);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(MI / 2 + (PL == 3 ? 0 : 4)) : "memory");
+    } else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (wm) __builtin_amdgcn_s_barrier();
     for (int kb = 0; kb < nk; kb++) {
-        const bool more = kb + 2 < nk;
-#define DN_BIG_LANDED                                                     \
-    if (PL == 3 && more) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); \
-    else if (more) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");      \
+#define DN_BIG_LANDED(more)                                                    \
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(LATER) : "memory");     \
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        // (PL 3: the next block of K's weights with its first line; behind the piece that is waited for are three of the operand's)
-        const bool more_w = PL == 3 ? kb % 3 == 0 && kb + 3 < nk : more;
-        const int kw = PL == 3 ? kb / 3 + 1 : kb + 2;
-        read_a(kb, 0);
-        if (more_w) request_w(kw, 0);
-        DN_BIG_LANDED
-        multiply(0, 0);
+        const bool more = kb + 2 < nk;
+        read_w(kb, 0);
         read_w(kb, 1);
-        if (more) request_a(kb + 2, 0);
-        DN_BIG_LANDED
-        multiply(0, 1);
+        read_a(kb, 0);
+        if (kb + 1 < nk) request_a(kb + 1, 1);
+        DN_BIG_LANDED(more)
+        multiply(0);
         read_a(kb, 1);
-        if (more_w) request_w(kw, 1);
-        DN_BIG_LANDED
-        multiply(1, 0);
-        if (kb + 1 < nk) read_w(kb + 1, 0);
-        if (more) request_a(kb + 2, 1);
-        DN_BIG_LANDED
-        multiply(1, 1);
+        if (more) {
+            if (PL == 1) { request_w(kb + 2, 0); request_w(kb + 2, 1); }
+            else if ((kb + 2) % 3 == 0) { request_w((kb + 2) / 3, 0); request_w((kb + 2) / 3, 1); }
+            request_a(kb + 2, 0);
+        }
+        DN_BIG_LANDED(more)
+        multiply(1);
 #undef DN_BIG_LANDED
     }
     if (!wm) __builtin_amdgcn_s_barrier();
@@ -1031,8 +1033,8 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #pragma unroll
         for (int mh = 0; mh < 2; mh++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int t = t0 + mh * 128 + wm * 64 + i * 16 + fr;
+            for (int i = 0; i < MI; i++) {
+                const int t = t0 + mh * HR + wm * 16 * MI + i * 16 + fr;
                 if (t >= T) continue;
                 const long long to = dn_orow(g, row0, t, T), at = to * g.ldo + n0;
                 const float f = g.out_scale ? g.alpha * dn_row_scale(g, to) : g.alpha;
@@ -1066,27 +1068,27 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
 #pragma unroll
         for (int nh = 0; nh < 2; nh++)
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) *(dn_f4 *)&tile[(wm * 64 + i * 16 + fr) * LD + nh * 128 + wn * 32 + j * 16 + 4 * (lane >> 4)] = acc[mh][nh][i][j];
+                for (int j = 0; j < 2; j++) *(dn_f4 *)&tile[(wm * 16 * MI + i * 16 + fr) * LD + nh * 128 + wn * 32 + j * 16 + 4 * (lane >> 4)] = acc[mh][nh][i][j];
         __syncthreads();
-        for (int r = wave; r < 128; r += 8) {
-            const int t = t0 + mh * 128 + r;
+        for (int r = wave; r < HR; r += 8) {
+            const int t = t0 + mh * HR + r;
             if (t >= T) break;
             dn_put4<ODD>(g, dn_orow(g, row0, t, T), n0 + 4 * lane, *(const dn_f4 *)&tile[r * LD + 4 * lane]);
         }
     }
 }
 static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR && !g.em_table && (g.N % 4 || g.ldo % 4 || ((uintptr_t)g.out & 15)); }
-// Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices, each with a last tile of its own).  The estimate behind the choice, in shader clocks: a block
-// of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more; rounds of 256 work-groups (one per CU);
-// a split product pays a second launch and its parts' way through memory.
-//   The 256 x 256 tiles (not split: 2047 x 2048 x 8192 in two 98 us, 84 as 128 x 128 tiles) stand beside the best of those in an estimate of their own, fitted to 615 bf16 products of either form (K of
-// 512 to 14336, 130 to 2047 tokens, 0.1 to 8 rounds; 4 % off on average, 3 % for these) and 335 in three lines.  In us:
-// a round's blocks, its start and what the epilogue adds behind a tile (dn_epilogue), the results and the weights by their megabytes.  They are taken where that says 2 % less; for experts, whose last tiles are a
-// guess, a tenth, or a twentieth where an expert has more than one of these on average (3072 slots of 8 x 2048 x 3072 84 us there and 78 here, 2000 slots 75 and 83).  3 of the 615 are then slower than
-// the others by 2 % or more (4 % at most) and none of the 335.  With 1700 clocks for a block of these in the estimate above it was one in nine and one in five: 512 tokens x 16384 x 2048 of gate / up pairs
-// take 64 us as 128 x 128 tiles and 80 as 256 x 256 (900: 119 and 89), 512 x 14336 x 4096 in three lines 206 and 251 (900: 391 and 257).
+// Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices).  bf16 and three lines: the least of an estimate in us, rounds of 256 work-groups times (blocks of K times what a block
+// of the shape costs, its start, what the epilogue adds behind a tile: dn_epilogue), and for a split product its second launch and its parts' way through memory.  Fitted to 2 600 products (9 to 2 047
+// tokens, N 1 024 .. 24 576, K 1 536 .. 14 336, every shape, up to twelve splits; plain results): what it picks takes 0.9 % longer than the best of all on average (three lines 0.7 %), 15 % at most; the rule
+// before, without the 192 rows and the 128 and 192 x 256 tiles, 5.3 % and 6.3 % on average, up to 33 %.  Us there and here: 1 090 x 6 208 x 4 096 93 and 72, 954 x 8 192 x 6 144 136 and 102,
+// 389 x 16 384 x 2 048 54 and 44, 1 477 x 6 144 x 8 192 179 and 151, in three lines 273 x 10 304 x 4 096 125 and 108, 617 x 14 336 x 4 096 300 and 267.
+//   A block costs the bytes it fetches: a CU has about 16 KB of requests outstanding, which the mean way to L2 and beyond (a fifth to a third of the rows are not there yet) makes 60 bytes a ns, whatever
+// the shape -- 32 KB in 0.5 us of 128 x 128, 64 KB in 1.05 of 256 x 256.  So larger tiles do more per byte, and a height that leaves no round nearly empty counts as much.
+//   Experts' rows: an expert has rows / groups on average, spread as a random routing and some more; the expected number of its tiles.
+// The fp32 instruction (dn_ring_plan_f32): a block of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more.
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
 enum { DN_EPI_DIRECT, DN_EPI_FOURS, DN_EPI_ONES }; // results from the registers; through LDS, four at a time; an activation or bias each
 static int dn_epilogue(const dn_args &g) {
@@ -1095,37 +1097,57 @@ static int dn_epilogue(const dn_args &g) {
     if (g.act != PSD_ACT_NONE && (g.act != PSD_ACT_RELU2 || g.accum)) return DN_EPI_ONES;
     return g.accum || dn_odd(g) ? DN_EPI_FOURS : DN_EPI_DIRECT;
 }
-static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines, int groups, bool bf, bool may_split, bool big, int epilogue) {
+static int dn_row_tiles(int rows, int BM, int groups) { // at most
+    return rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0);
+}
+static double dn_mean_row_tiles(int rows, int BM, int groups) {
+    if (!groups) return (rows + BM - 1) / BM;
+    const double mean = (double)rows / groups, sd = std::sqrt(mean) + mean / 16;
+    double tiles = 0;
+    for (int k = 0; k <= rows / BM; k++) { // an expert has its tile k where it has more than k BM rows
+        const double p = 0.5 * std::erfc((k * BM + 0.5 - mean) / (sd * 1.41421356));
+        tiles += p;
+        if (p < 1e-3) break;
+    }
+    return std::max(1.0, groups * tiles);
+}
+static dn_ring_shape dn_ring_plan_f32(int rows, int64_t N, int64_t kbytes, int groups, bool may_split) {
     static const int shapes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
     const int64_t blocks = kbytes / 128;
     dn_ring_shape best{};
     double least = 0;
-    auto row_tiles = [&](int BM, bool over) { // (grouped: about half of the last tiles start a new one; over: an expert has more than a tile)
-        const int full = (rows + BM - 1) / BM;
-        return groups > 0 ? std::max(full, std::min(groups, rows)) + (over ? groups / 2 : 0) : full;
-    };
     for (auto &q : shapes) {
-        const int BM = q[0], BN = q[1], n_tm = rows / BM + (groups > 0 ? std::min(groups, rows) : rows % BM ? 1 : 0), tn = (int)((N + BN - 1) / BN);
-        const int64_t tiles = (int64_t)row_tiles(BM, rows > groups * BM) * tn;
-        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * (bf ? 2 : 16), block = std::max(lds, mfma) + 100;
+        const int BM = q[0], BN = q[1], n_tm = dn_row_tiles(rows, BM, groups), tn = (int)((N + BN - 1) / BN), full = (rows + BM - 1) / BM;
+        const int64_t tiles = (int64_t)(groups > 0 ? std::max(full, std::min(groups, rows)) + (rows > groups * BM ? groups / 2 : 0) : full) * tn; // (grouped: about half of the last tiles start a new one)
+        const double lds = 3.0 * (BM + BN), mfma = BM * BN / 64.0 * 16, block = std::max(lds, mfma) + 100;
         for (int64_t S = 1; S <= (may_split ? 16 : 1); S++) {
             if (S > 1 && (blocks / S < 4 || tiles * S > 512 || (size_t)n_tm * tn * S * BM * BN * 4 > psk_dense_split_bytes())) break;
-            const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * lines * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
+            const double rounds = (double)((tiles * S + 255) / 256), t = rounds * (double)((blocks + S - 1) / S) * block + 4000 + (S > 1 ? 9000 + (double)tiles * S * BM * BN * 4 / 3000 : 0);
             if (!best.BM || t < least) { least = t; best = dn_ring_shape{BM, BN, n_tm, tn, (int)S}; }
         }
     }
-    if (bf && big) {
-        struct cost { double all, block, round, results, weights, behind[3]; };
-        static const cost small[2] = {{2.4, 0.527, 0.55, 0.377, 0.058, {0, 0.9, 5.1}}, {4.3, 0.495, -2.4, 0.576, 0.056, {0, 0.9, 5.1}}}, large[2] = {{-2.5, 1.023, 12.8, 0.145, 0.079, {0, 7.4, 27.4}}, {-8.4, 1.177, 20, 0.153, 0.105, {0, 7.4, 27.4}}};
-        const double results = rows * (double)N * 4e-6, weights = (double)N * kbytes * 1e-6 * std::max(groups, 1), per_block = std::max(3.0 * (best.BM + best.BN), best.BM * best.BN / 32.0) + 100; // (clocks; 868 for 128 x 128)
-        auto time = [&](const cost &c, int BM, int64_t columns, double blocks, double area) {
-            const double rounds = (double)((columns * row_tiles(BM, rows >= groups * BM) + 255) / 256);
-            return c.all + rounds * (blocks * lines * c.block + (c.round + c.behind[epilogue]) * area) + c.results * results + c.weights * weights;
-        };
-        const int tn = (int)((N + DN_BIG - 1) / DN_BIG), n_tm = rows / DN_BIG + (groups > 0 ? std::min(groups, rows) : rows % DN_BIG ? 1 : 0);
-        const double other = time(small[lines == 3], best.BM, (int64_t)best.tn * best.S, (double)((blocks + best.S - 1) / best.S) * per_block / 868, best.BM * best.BN / 16384.0) + (best.S > 1 ? 9 : 0);
-        const double here = time(large[lines == 3], DN_BIG, tn, (double)blocks, 1);
-        if (here < (groups == 0 ? 0.98 : rows > 1.4 * DN_BIG * groups ? 0.95 : 0.9) * other) best = dn_ring_shape{DN_BIG, DN_BIG, n_tm, tn, 1};
+    return best;
+}
+static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines, int groups, bool may_split, bool big, int epilogue) {
+    struct shape { int BM, BN; double block[2], round[2]; }; // (bf16, three lines; us)
+    static const shape shapes[7] = {{256, 256, {1.046, 3.651}, {0.05, 2.05}}, {192, 256, {0.882, 3.514}, {0.07, 0.05}}, {128, 256, {0.719, 2.875}, {0.05, 0.05}}, {192, 128, {0.512, 1.842}, {2.96, 0.05}},
+                                    {128, 128, {0.388, 1.368}, {2.25, 0.12}}, {64, 128, {0.275, 0.83}, {1.76, 0.34}}, {64, 64, {0.167, 0.508}, {0.91, 0.05}}};
+    static const double behind[2][3] = {{0, 0.9, 5.1}, {0, 1.85, 6.85}}; // by 128 x 128 numbers; of tiles of 128 columns and less, of 256
+    static const double sums[2] = {2.8, 1.1}, parts[2] = {0.21, 0.30}; // a split product: once, by MB
+    const int64_t blocks = kbytes / 128;
+    const int l = lines == 3;
+    dn_ring_shape best{};
+    double least = 0;
+    for (auto &q : shapes) {
+        if (q.BN == DN_BIG && !big) continue;
+        const int n_tm = dn_row_tiles(rows, q.BM, groups), tn = (int)((N + q.BN - 1) / q.BN);
+        const double area = q.BM * q.BN / 16384.0, tiles = dn_mean_row_tiles(rows, q.BM, groups) * tn;
+        for (int64_t S = 1; S <= (may_split && q.BN < DN_BIG ? 16 : 1); S++) {
+            if (S > 1 && (blocks / S < 4 || tiles * S > 700 || (size_t)n_tm * tn * S * q.BM * q.BN * 4 > psk_dense_split_bytes())) break;
+            const double t = std::ceil(tiles * S / 256) * ((double)((blocks + S - 1) / S) * q.block[l] + q.round[l] + (S == 1 ? behind[q.BN == DN_BIG][epilogue] * area : 0)) +
+                             (S > 1 ? sums[l] + parts[l] * tiles * S * area * 0.0655 : 0);
+            if (!best.BM || t < least) { least = t; best = dn_ring_shape{q.BM, q.BN, n_tm, tn, (int)S}; }
+        }
     }
     return best;
 }
@@ -1142,13 +1164,14 @@ static void dn_launch_ring(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if (p.S > 1) hipLaunchKernelGGL((dense_mm_sum_kernel<BM, BN, ODD>), dim3((unsigned)(p.n_tm * p.tn * (BM / 64) * (BN / 64) * 4)), dim3(256), 0, st, g, p);
 }
 
-template <bool ODD, int PL>
+template <bool ODD, int PL, int MI>
 static void dn_launch_big(hipStream_t st, const dn_args &g, const dn_ring &p) {
     if constexpr (!ODD)
-        if (dn_odd(g)) return dn_launch_big<true, PL>(st, g, p);
+        if (dn_odd(g)) return dn_launch_big<true, PL, MI>(st, g, p);
+    constexpr int LDS = dn_big_lds(MI);
     static unsigned long long mask = 0;
-    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_big_kernel<ODD, PL>, hipFuncAttributeMaxDynamicSharedMemorySize, DN_BIG_LDS);
-    hipLaunchKernelGGL((dense_mm_big_kernel<ODD, PL>), dim3((unsigned)(((long long)p.tn * p.n_tm + 7) / 8 * 8)), dim3(512), DN_BIG_LDS, st, g, p);
+    if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)dense_mm_big_kernel<ODD, PL, MI>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    hipLaunchKernelGGL((dense_mm_big_kernel<ODD, PL, MI>), dim3((unsigned)(((long long)p.tn * p.n_tm + 7) / 8 * 8)), dim3(512), LDS, st, g, p);
 }
 
 // The wide mat-mul, where it takes the product: whole blocks of K, room for what has to be packed.  PL 3 (WT: bf16): an fp32 product on the bf16 instruction -- the weights as they came, which is in
@@ -1172,7 +1195,9 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     }
     const int64_t each = g.N;
     g.N *= copies;
-    const dn_ring_shape r = dn_ring_plan(a.T, g.N, kbytes, PL, g.groups, sizeof(WT) == 2, a.split && a.split_bytes >= psk_dense_split_bytes(), (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 22), dn_epilogue(g)); // (rows of a tile by 32-bit offsets)
+    const bool may_split = a.split && a.split_bytes >= psk_dense_split_bytes();
+    const dn_ring_shape r = sizeof(WT) == 4 ? dn_ring_plan_f32(a.T, g.N, kbytes, g.groups, may_split)
+                                            : dn_ring_plan(a.T, g.N, kbytes, PL, g.groups, may_split, (each % DN_BIG == 0 || copies == 1) && kbytes < (1 << 22), dn_epilogue(g)); // (rows of a tile by 32-bit offsets)
     dn_ring p{handed ? (const char *)a.a16 : plain ? nullptr : (const char *)a.pack, kbytes * PL, r.n_tm, r.tn, r.S, a.split};
     p.each = copies > 1 ? each : 0;
     p.copy = a.T * kbytes * PL;
@@ -1182,8 +1207,14 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
         const int mixes = pb >= 256 ? copies : 1; // (few tokens: as many work-groups as there are mixes)
         hipLaunchKernelGGL((dense_pack_kernel<WT, PL>), dim3((unsigned)std::min<int64_t>(pb, 8192), (unsigned)(copies / mixes)), dim3(256), 0, st, g, (WT *)a.pack, mixes);
     }
-    if (r.BM == DN_BIG) {
-        if constexpr (sizeof(WT) == 2) dn_launch_big<false, PL>(st, g, p);
+    if (r.BN == DN_BIG) {
+        if constexpr (sizeof(WT) == 2) {
+            if (r.BM == 128) dn_launch_big<false, PL, 2>(st, g, p);
+            else if (r.BM == 192) dn_launch_big<false, PL, 3>(st, g, p);
+            else dn_launch_big<false, PL, 4>(st, g, p);
+        }
+    } else if (r.BM == 192) {
+        if constexpr (sizeof(WT) == 2) dn_launch_ring<WT, 192, 128, false, PL>(st, g, p);
     } else if (r.BM == 128) dn_launch_ring<WT, 128, 128, false, PL>(st, g, p);
     else if (r.BN == 128) dn_launch_ring<WT, 64, 128, false, PL>(st, g, p);
     else dn_launch_ring<WT, 64, 64, false, PL>(st, g, p);

@@ -474,6 +474,15 @@ def test_odd_rows_behind_an_epilogue(made, dtype, width, ff):
     assert err(run_portions(m, toks, [64, 11]), seq_oracle.run(cfg, t, toks)) < TOL[dtype]
 
 
+# tiles of 128 and 192 rows x 256 columns and of 192 x 128 (k_dense.hip dense_mm_big_kernel, dense_mm_ring_kernel; dn_ring_plan takes them here, in bfloat16 or in three lines): one block of K, two, an odd
+# and an even number; a row, a column and four columns more and less than a tile, no fours; split along K; columns of tiles that are no multiple of a panel or of the XCDs
+@pytest.mark.parametrize("dtype", list(FORMS))
+@pytest.mark.parametrize("T,N,K", [(1153, 6148, 64), (641, 8196, 64), (1345, 3076, 64), (640, 8192, 128), (385, 14340, 320), (1345, 6145, 192), (2047, 4100, 192), (1025, 8200, 192), (1537, 2049, 192),
+                                   (1345, 3077, 256), (193, 14340, 64), (577, 2052, 2112), (1345, 3076, 1088), (961, 4101, 1088)])
+def test_dense_matmul_of_other_tile_heights(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
 # K up to 32 (k_dense.hip dense_mm_few_kernel): one below, at and above its two widths (33: the tiled kernel), one token and one column more and less than a work-group's
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,N,K", [(9, 1, 1), (15, 255, 7), (16, 256, 8), (17, 257, 9), (33, 70, 31), (31, 513, 32), (40, 65, 33)])
