@@ -3,16 +3,20 @@
 // apart).  Each of those is exact, and a sum of 192 passes 36 roundings where v_mfma_f32_16x16x4_f32 has one for each of its 48 steps; six of the fast instructions cost 96 clocks where the
 // fp32 one's eight steps cost 256.  The serving layers' forms (k_latent.hip, k_winattn.hip: portions of any size, and what this does not take) run on the fp32 instruction.
 //   split_keys_kernel   the keys and values a portion sees, in blocks of 32 and split, as the images the attention's stages are filled with: 1 KB per instruction operand in lane order
-//   split_attn_kernel   128 rows (consecutive tokens) of one head per work-group, a wave 16 of them against all keys; blocks of 32 keys through two LDS stages
+//   split_attn_kernel   128 rows (consecutive tokens) of one head per work-group, a wave 16 of them against all keys, or a part of them; blocks of 32 keys through two LDS stages
+//   split_join_kernel   the parts of such rows together (sa_plan_of)
 // S^T = K Q^T, so that a lane has one row: maximum and sum run over its own registers, two lane moves join the four lanes of a row.  D's rows are the keys 4 (l / 16) + i of two tiles, and the
 // second product, O^T = V^T P^T, takes its 32 keys in any order that both operands share: a lane's eight weights are its piece of the operand as they are, and the value images are laid out so.
 // What bounded the fp32 form: 2560 clocks of matrix instructions per 16 x 16 scores beside as much again of soft-max in its accumulator layout (four moves per row reduction, weights turned
 // in LDS), keys straight from the L2s for 32 rows at a time.  2047 tokens of 16 heads, keys of 192, a window of 1024: 318 -> 141 us, 17 of them the images; 3 us a block of 32 keys and
-// work-group, 1.9 of it matrix instructions; without its reads, its requests or its soft-max it is 0.7, 0.3 and 0.5 less.  (The second wave of every SIMD a block behind with its second product, so
+// work-group, 1.9 of it matrix instructions; without its reads, its requests or its soft-max it is 0.7, 0.3 and 0.5 less.  (The queries are turned by split_keys_kernel and come straight into the operand registers: through LDS, turned by every head's work-groups,
+// a work-group's first product stood 9 us behind its start.)  (The second wave of every SIMD a block behind with its second product, so
 // that its soft-max runs beside the others' products: 137 us without the images against 126.)  Error against 64 bits over four seeds: keys of 192 5.6e-7 -> 5.4e-7, 128 with slopes 6.4e-7 -> 4.1e-7.
 #include "ps_seq.h"
 
+#include <algorithm>
 #include <cmath>
+#include <vector>
 
 typedef float sa_f4 __attribute__((ext_vector_type(4)));
 typedef float sa_f2 __attribute__((ext_vector_type(2)));
@@ -76,7 +80,9 @@ static __device__ __forceinline__ float sa_sigmoid(float x) { return 1.f / (1.f 
 
 // ---------------------------------------------------------------------------------------------------- images
 // Block b of head (or key / value group) g: rows 32 b .. of the front store for b < nbf, else window rows 32 (b - nbf) ..; rows beyond the last are zeros.  The image: [k step][plane][16 keys][lane]
-// 16 bytes, then [16 value columns][plane][lane].  blockIdx.y == G: the key parts that all heads share, an image of their own.
+// 16 bytes, then [16 value columns][plane][lane].  The last of blockIdx.y: the key parts that all heads share, an image of their own; the first
+// `turners`: the turned part of the queries of rows 32 b .. (behind the images they were the launch's tail: 28 us for 2047 tokens of 16 heads, 21 without them)
+#define SA_TURNERS 8 // work-groups that share the heads of 32 rows
 struct sa_rows { // window row j (counted from the portion's first visible position) = row j + off of base, wrapped once at mod (0: no wrap)
     const float *base;
     long long ld;
@@ -91,6 +97,10 @@ struct sa_keys {
     int ks_own, ks_shared, nj;      // k steps of 32 numbers of a head's own key part and of the shared one, value tiles of 16 columns
     int G;
     char *img, *img_shared;
+    const float *q, *freq; // the queries, whose part of the shared numbers is turned (rot_dims > 0; a group is a head): q_turned [T][G][32 ks_shared]
+    long long ldq;
+    float rot_mag, *q_turned;
+    int rot_dims, pairing, pos0, T, turners;
 };
 static __device__ __forceinline__ const float *sa_row(const sa_rows &r, long long step, int j) {
     int n = j + r.off;
@@ -98,7 +108,27 @@ static __device__ __forceinline__ const float *sa_row(const sa_rows &r, long lon
     return r.base + step + n * r.ld;
 }
 __global__ __launch_bounds__(256) void split_keys_kernel(sa_keys a) {
-    const int b = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
+    const int b = blockIdx.x, g = (int)blockIdx.y - a.turners, tid = threadIdx.x;
+    if (g < 0) {
+        const int dr = 32 * a.ks_shared, half = a.rot_dims / 2;
+        for (int x = tid; x < 32 * (dr - half); x += 256) {
+            const int t = 32 * b + x / (dr - half), i = x % (dr - half); // pair i, or a number that is not turned
+            if (t >= a.T) break;
+            const bool pair = i < half, near = a.pairing == PS_ROT_NEIGHBOURS;
+            const int c = !pair ? half + i : near ? 2 * i : i, d = near ? 1 : half;
+            const float ang = pair ? (float)(a.pos0 + t) * a.freq[i] : 0.f, cs = cosf(ang) * a.rot_mag, sn = sinf(ang) * a.rot_mag;
+            const long long own = 32 * a.ks_own + dr;
+            const float *q = a.q + t * a.ldq + 32 * a.ks_own + c;
+            float *o = a.q_turned + (long long)t * a.G * dr + c;
+#pragma unroll 4
+            for (int h = g + a.turners; h < a.G; h += a.turners) {
+                const float u = q[h * own], v = q[h * own + (pair ? d : 0)];
+                o[h * dr] = pair ? u * cs - v * sn : u;
+                if (pair) o[h * dr + d] = v * cs + u * sn;
+            }
+        }
+        return;
+    }
     const bool shared = g == a.G, front = b < a.nbf;
     const int i0 = 32 * (front ? b : b - a.nbf), n = front ? a.n_front : a.n_window; // rows i0 .. i0 + 31 of those that exist
     const int ks = shared ? a.ks_shared : a.ks_own, nk = ks * 128, nv = shared ? 0 : a.nj * 64; // sixteen-byte pieces per plane
@@ -141,39 +171,78 @@ struct sa_attn {
     int pos0, first, T, window, pool, keep; // position of row 0, of window row 0
     const float *q;
     long long ldq;
-    int d, rot_at, rot_dims, pairing; // numbers of a head's query; its rotated part begins at rot_at (rot_dims 0: it comes rotated)
-    const float *freq;
-    float rot_mag, scale, softcap;
+    const float *q_turned; // [T][H][numbers of the shared key part], or NULL: those of q as they are
+    float scale, softcap;
     const float *temp, *slope, *sink, *gate;
     long long ldg;
     int gate_elem;
     float *o;
     long long ldo;
+    int q16;               // rows of q by sixteen bytes
+    int H, most;           // blocks of a part at most: a tile with more of them is worked on by several work-groups, whose results split_join_kernel adds
+    float *part, *part_ml; // [work-groups] results of 128 rows not yet divided, their maxima and sums
 };
+// the blocks of keys of the 128 rows from t0 on: those of the front store that the last row sees, then the window's from the first row's first key to the last row's own
+struct sa_span { int nfb, wb0, blocks; };
+static __host__ __device__ __forceinline__ int sa_parts(int blocks, int most) { return (blocks + most - 1) / most; }
+static __host__ __device__ __forceinline__ sa_span sa_span_of(int t0, int pos0, int first, int T, int window, int pool, int keep) {
+    const int plast = pos0 + (t0 + 128 < T ? t0 + 128 : T) - 1, pfirst = pos0 + t0, lo = pfirst - window + 1;
+    int nf = plast - window + 1;
+    nf = nf <= 0 ? 0 : pool > 0 ? nf / pool : nf < keep ? nf : keep;
+    const int nfb = (nf + 31) / 32, wb0 = ((lo > 0 ? lo : 0) - first) / 32;
+    return sa_span{nfb, wb0, nfb + (plast - first) / 32 - wb0 + 1};
+}
 static __device__ __forceinline__ void sa_dma(const char *base, unsigned off, unsigned lds_dst) { // one wave-instruction: lane l's 16 bytes at base + off go to lds_dst + 16 l
     unsigned keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst) : "memory");
 }
-#define SA_ROWS 128
-template <int KS, int NJ>
-static constexpr int sa_lds() { // two stages; before the second one is filled the queries lie there
-    const int q = SA_ROWS * (KS * 32 + 4) * 4, s = KS * 6144 + NJ * 3072;
-    return s + (q > s ? q : s);
+// a row's results from its maximum, the sum of its weights and their products (a lane: columns 16 j + 4 lq ..)
+template <int NJ>
+static __device__ __forceinline__ void sa_finish(const sa_attn &a, int h, int t, int lq, float m, float l, const sa_f4 (&acc)[NJ]) {
+    float f;
+    if (a.sink) { // (k_winattn.hip wa_finish)
+        const float sk = a.sink[h], M = fmaxf(m, sk), c = expf(m - M);
+        f = c / (l * c + expf(sk - M));
+    } else {
+        f = 1.f / l;
+    }
+    if (a.gate && !a.gate_elem) f *= sa_sigmoid(a.gate[(long long)t * a.ldg + h]);
+    float *o = a.o + (long long)t * a.ldo + (long long)h * (16 * NJ) + 4 * lq;
+    const float *ge = a.gate && a.gate_elem ? a.gate + (long long)t * a.ldg + (long long)h * (16 * NJ) + 4 * lq : nullptr;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        sa_f4 v = sa_f4{acc[j][0] * f, acc[j][1] * f, acc[j][2] * f, acc[j][3] * f};
+        if (ge) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] *= sa_sigmoid(ge[16 * j + i]);
+        }
+        *(sa_f4 *)(o + 16 * j) = v;
+    }
 }
+#define SA_ROWS 128
+#define SA_CUS 256
+#define SA_PART (SA_ROWS * (128 + 2) * 4) // bytes of a part of a tile
+template <int KS, int NJ>
+static constexpr int sa_lds() { return 2 * (KS * 6144 + NJ * 3072); } // two stages
 template <int KS, int NJ, bool DIST>
 __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     extern __shared__ __attribute__((aligned(16))) char sa_smem[];
-    constexpr int STAGE = KS * 6144 + NJ * 3072, PIECES = KS * 6 + NJ * 3, QLD = KS * 32 + 4;
+    constexpr int STAGE = KS * 6144 + NJ * 3072, PIECES = KS * 6 + NJ * 3;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lq = lane >> 4;
-    const int h = blockIdx.x, t0 = SA_ROWS * ((int)gridDim.y - 1 - (int)blockIdx.y), g = h / a.hpg; // (the rows with the most keys first)
-    const int rows = min(SA_ROWS, a.T - t0), n = 16 * wave + lr, p = a.pos0 + t0 + n;               // this lane's row and its position
-    // blocks of this work-group: those of the front store that its last row sees, then the window's from the first row's first key to the last row's own
-    const int plast = a.pos0 + t0 + rows - 1, pfirst = a.pos0 + t0;
-    int nf = plast - a.window + 1;
-    nf = nf <= 0 ? 0 : a.pool > 0 ? nf / a.pool : min(nf, a.keep);
-    const int nfb = (nf + 31) / 32, wlo = max(pfirst - a.window + 1, 0) - a.first, wb0 = wlo / 32, nwb = (plast - a.first) / 32 - wb0 + 1, blocks = nfb + nwb;
-    const int own = a.ks_own * 6, image = own + NJ * 3; // pieces of a head's own key part, of its image
     const unsigned lds0 = (unsigned)(size_t)(const __attribute__((address_space(3))) char *)sa_smem;
+    // a part of a tile's blocks (the rows with the most keys first)
+    const int h = (int)blockIdx.x % a.H, slot = (int)blockIdx.x;
+    int t0 = (a.T - 1) / SA_ROWS * SA_ROWS, part = slot / a.H, parts;
+    sa_span span;
+    for (;; t0 -= SA_ROWS) { // (uniform; there are as many work-groups as parts)
+        span = sa_span_of(t0, a.pos0, a.first, a.T, a.window, a.pool, a.keep);
+        parts = sa_parts(span.blocks, a.most);
+        if (part < parts || t0 == 0) break;
+        part -= parts;
+    }
+    const int nfb = span.nfb, wb0 = span.wb0, it0 = span.blocks * part / parts, it1 = span.blocks * (part + 1) / parts, g = h / a.hpg;
+    const int rows = min(SA_ROWS, a.T - t0), n = 16 * wave + lr, p = a.pos0 + t0 + n, pfirst = a.pos0 + t0; // this lane's row and its position
+    const int own = a.ks_own * 6, image = own + NJ * 3; // pieces of a head's own key part, of its image
     auto block_of = [&](const int it) { return it < nfb ? it : a.nbf + wb0 + it - nfb; };
     auto request = [&](const int it) {
         const int b = block_of(it);
@@ -181,38 +250,29 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
 #pragma unroll
         for (int x = 0; x < (PIECES + 7) / 8; x++) {
             const int pc = x * 8 + wave;
-            if (pc < PIECES) sa_dma(pc < own ? im + pc * 1024 : pc < KS * 6 ? sh + (pc - own) * 1024 : im + (pc - KS * 6 + own) * 1024, lane * 16, lds0 + (unsigned)((it & 1) * STAGE + pc * 1024));
+            if (pc < PIECES) sa_dma(pc < own ? im + pc * 1024 : pc < KS * 6 ? sh + (pc - own) * 1024 : im + (pc - KS * 6 + own) * 1024, lane * 16, lds0 + (unsigned)(((it - it0) & 1) * STAGE + pc * 1024));
         }
     };
-    request(0);
-    // this wave's query rows, rotated, through LDS (behind the first stage) into its operand registers
-    float *qs = (float *)(sa_smem + STAGE) + 16 * wave * QLD;
-    const int half = a.rot_dims / 2;
-    // (sixteen rows' numbers requested at a time; rows that do not exist repeat the last one)
-    const float *qw = a.q + (long long)h * a.d;
-    auto row_at = [&](const int r) { return qw + (long long)min(t0 + 16 * wave + r, a.T - 1) * a.ldq; };
-    for (int c = lane; c < a.d; c += 64) {
-        float x[16];
-#pragma unroll
-        for (int r = 0; r < 16; r++) x[r] = row_at(r)[c];
-#pragma unroll
-        for (int r = 0; r < 16; r++) qs[r * QLD + c] = x[r];
-    }
-    for (int x = lane; x < 16 * half; x += 64) { // (a wave's rows are its own: no barrier)
-        const int r = x / half, i = x - r * half;
-        float *pa = qs + r * QLD + a.rot_at + (a.pairing == PS_ROT_NEIGHBOURS ? 2 * i : i), *pb = pa + (a.pairing == PS_ROT_NEIGHBOURS ? 1 : half);
-        const float ang = (float)(a.pos0 + t0 + 16 * wave + r) * a.freq[i], cs = cosf(ang) * a.rot_mag, sn = sinf(ang) * a.rot_mag, u = *pa, v = *pb;
-        *pa = u * cs - v * sn;
-        *pb = v * cs + u * sn;
-    }
-    __syncthreads();
+    request(it0);
+    // this lane's share of its query row (rows that do not exist repeat the last one)
     sa_u4 q[KS][3];
+    {
+        const int t = min(t0 + n, a.T - 1);
+        const float *qr = a.q + (long long)t * a.ldq + (long long)h * (32 * KS) + 8 * lq, *qt = a.q_turned ? a.q_turned + ((long long)t * a.H + h) * (32 * (KS - a.ks_own)) + 8 * lq - 32 * a.ks_own : qr;
+        float v[KS][8];
 #pragma unroll
-    for (int s = 0; s < KS; s++) {
-        float v[8];
-        *(sa_f4 *)v = *(const sa_f4 *)(qs + lr * QLD + 32 * s + 8 * lq);
-        *(sa_f4 *)(v + 4) = *(const sa_f4 *)(qs + lr * QLD + 32 * s + 8 * lq + 4);
-        sa_split8<true>(v, q[s]);
+        for (int s = 0; s < KS; s++) {
+            const float *x = (s < a.ks_own ? qr : qt) + 32 * s;
+            if (a.q16) { // (uniform)
+                *(sa_f4 *)v[s] = *(const sa_f4 *)x;
+                *(sa_f4 *)(v[s] + 4) = *(const sa_f4 *)(x + 4);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[s][e] = x[e];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < KS; s++) sa_split8<true>(v[s], q[s]);
     }
     const float sc = a.scale * (a.temp ? a.temp[h] : 1.f), slope = DIST ? a.slope[h] : 0.f;
     float m = -INFINITY, l = 0.f; // (l: of this lane's own keys)
@@ -279,14 +339,14 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
 #pragma unroll
         for (int x = 0; x < 8; x++) { e[x] = sa_exp(e[x] - off); l += e[x]; }
     };
-    for (int it = 0; it < blocks; it++) {
+    for (int it = it0; it < it1; it++) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); // the block has landed (this wave's share); the reads of the one before are back
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (it + 1 < blocks) request(it + 1);
+        if (it + 1 < it1) request(it + 1);
         const place b = place_of(it);
         if (!alive || b.none) continue;
-        const char *st = sa_smem + (it & 1) * STAGE + lane * 16;
+        const char *st = sa_smem + ((it - it0) & 1) * STAGE + lane * 16;
         sa_f4 s1[2], s2[2], s3[2]; // (chains of their own)
 #pragma unroll
         for (int u = 0; u < 2; u++) s1[u] = s2[u] = s3[u] = sa_f4{0.f, 0.f, 0.f, 0.f};
@@ -360,7 +420,7 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
         l = 0.f;
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[j] = sa_f4{0.f, 0.f, 0.f, 0.f};
-        for (int it = 0; it < blocks; it++) {
+        for (int it = it0; it < it1; it++) {
             const place b = place_of(it);
             if (b.none) continue;
             const char *im = a.img + ((size_t)g * a.nb + block_of(it)) * (image * 1024) + lane * 16, *sh = a.img_shared + (size_t)block_of(it) * ((KS * 6 - own) * 1024) + lane * 16;
@@ -411,27 +471,44 @@ __global__ __launch_bounds__(512) void split_attn_kernel(sa_attn a) {
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    const int t = t0 + n;
-    if (n >= rows) return;
-    float f;
-    if (a.sink) { // (k_winattn.hip wa_finish)
-        const float sk = a.sink[h], M = fmaxf(m, sk), c = expf(m - M);
-        f = c / (l * c + expf(sk - M));
-    } else {
-        f = 1.f / l;
+    if (parts == 1) {
+        if (n < rows) sa_finish<NJ>(a, h, t0 + n, lq, m, l, acc);
+        return;
     }
-    if (a.gate && !a.gate_elem) f *= sa_sigmoid(a.gate[(long long)t * a.ldg + h]);
-    float *o = a.o + (long long)t * a.ldo + (long long)h * (16 * NJ) + 4 * lq;
-    const float *ge = a.gate && a.gate_elem ? a.gate + (long long)t * a.ldg + (long long)h * (16 * NJ) + 4 * lq : nullptr;
+    // as they are, for split_join_kernel
+    float *o = a.part + (size_t)slot * (SA_ROWS * 16 * NJ) + (wave * NJ * 64 + lane) * 4;
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        sa_f4 v = sa_f4{acc[j][0] * f, acc[j][1] * f, acc[j][2] * f, acc[j][3] * f};
-        if (ge) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] *= sa_sigmoid(ge[16 * j + i]);
-        }
-        *(sa_f4 *)(o + 16 * j) = v;
+    for (int j = 0; j < NJ; j++) *(sa_f4 *)(o + j * 256) = acc[j];
+    if (lq == 0) *(sa_f2 *)(a.part_ml + (size_t)slot * (2 * SA_ROWS) + 2 * n) = sa_f2{m, l};
+}
+// The parts of a tile, brought to their common maximum, added in order and finished: a wave has sixteen rows of it.
+template <int NJ>
+__global__ __launch_bounds__(256) void split_join_kernel(sa_attn a) {
+    const int lane = threadIdx.x & 63, wave = 4 * (int)blockIdx.y + (int)(threadIdx.x >> 6), lr = lane & 15, lq = lane >> 4, h = (int)blockIdx.x % a.H, n = 16 * wave + lr;
+    int t0 = (a.T - 1) / SA_ROWS * SA_ROWS, tile = (int)blockIdx.x / a.H, first = 0, parts; // (tiles in the same order)
+    for (;; t0 -= SA_ROWS, tile--) {
+        parts = sa_parts(sa_span_of(t0, a.pos0, a.first, a.T, a.window, a.pool, a.keep).blocks, a.most);
+        if (tile == 0 || t0 == 0) break;
+        first += parts;
     }
+    if (parts == 1 || t0 + 16 * wave >= a.T) return;
+    auto slot = [&](const int x) { return (size_t)((first + x) * a.H + h); };
+    float m = -INFINITY;
+    for (int x = 0; x < parts; x++) m = fmaxf(m, a.part_ml[slot(x) * (2 * SA_ROWS) + 2 * n]);
+    float l = 0.f;
+    sa_f4 acc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[j] = sa_f4{0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < parts; x++) {
+        const sa_f2 ml = *(const sa_f2 *)(a.part_ml + slot(x) * (2 * SA_ROWS) + 2 * n);
+        const float *o = a.part + slot(x) * (SA_ROWS * 16 * NJ) + (wave * NJ * 64 + lane) * 4;
+        if (ml[0] == -INFINITY && ml[1] == 0.f) continue; // (the row sees no key of this part)
+        const float f = ml[0] == m ? 1.f : sa_exp(ml[0] - m);
+        l += ml[1] * f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[j] += *(const sa_f4 *)(o + j * 256) * f;
+    }
+    if (t0 + n < a.T) sa_finish<NJ>(a, h, t0 + n, lq, m, l, acc);
 }
 
 // ---------------------------------------------------------------------------------------------------- host
@@ -444,14 +521,61 @@ bool psk_split_attn_ok(int own, int shared, int dv) { return dv == 128 && own % 
 // 64 | 117; 96 rows 107 | 109, 160 | 176; 112 rows 131 | 110, 224 | 181; 40 heads, 192 rows 99 | 103, 149 | 168; 224 rows 123 | 109, 219 | 173; 64 heads, 128 rows 102 | 108, 152 | 176;
 // 129 rows 126 | 113, 221 | 182; 128 heads, 64 rows 117 | 119, 173 | 188; 80 rows 139 | 127, 231 | 210.
 bool psk_split_attn_takes(int T, int H) { return (int64_t)((T + SA_ROWS - 1) / SA_ROWS) * H >= 80 && (int64_t)((T + 15) / 16) * H > 512; }
-static size_t sa_images(int G, int own, int shared, int dv, int64_t blocks) { return (size_t)blocks * ((size_t)G * (own / 32 * 6144 + dv / 16 * 3072) + (size_t)shared / 32 * 6144); }
+static size_t sa_images(int G, int own, int shared, int dv, int64_t blocks) { return (size_t)blocks * ((size_t)G * (own / 32 * 6144 + dv / 16 * 3072) + (size_t)shared / 32 * 6144 + (size_t)G * shared * 128); }
 size_t psk_split_attn_scratch(int G, int own, int shared, int dv, int64_t n_front, int64_t n_window) { return sa_images(G, own, shared, dv, (n_front + 31) / 32 + (n_window + 31) / 32); }
 
+struct sa_plan { int most, wgs; bool join; };
+// How many blocks a work-group has at most.  The rows of a tile have up to a window of keys, and where the tiles are fewer than the CUs, or some have many more keys than others, the chip waits for the
+// longest: 1500 tokens of 16 heads behind a window of 1024 are 192 tiles of 4 to 36 blocks.  A tile in parts costs each of them a start (the queries, the first block: as much as four blocks) and a launch that
+// joins them.  So the host follows the CUs through the work-groups, in the order they are dispatched, for whole tiles and for parts of at most 15 / 16, 14 / 16, .. of the longest, and takes the shortest time; whole
+// tiles where that is within 6 % (a tile more of one to its time is what the model is off by).  us, whole and so, with the joining: those 1500 tokens, keys of 192 136 and 92, keys of 128 with slopes and means of
+// blocks in front (up to 47 blocks) 104 and 82.
+static sa_plan sa_plan_of(const sa_attn &a, size_t part_bytes) {
+    const int tiles = (a.T + SA_ROWS - 1) / SA_ROWS;
+    const sa_plan whole{1 << 30, tiles * a.H, false};
+    if (tiles > 64 || tiles * a.H > 4 * SA_CUS) return whole;
+    int blocks[64], longest = 0;
+    for (int i = 0; i < tiles; i++) longest = std::max(longest, blocks[i] = sa_span_of(SA_ROWS * (tiles - 1 - i), a.pos0, a.first, a.T, a.window, a.pool, a.keep).blocks);
+    constexpr int START = 4;
+    std::vector<int> idle;
+    auto end_of = [&](const sa_plan &p) { // in blocks
+        idle.assign((size_t)(p.wgs / SA_CUS + 2) * (std::min(longest, p.most) + START) + 1, 0); // CUs that become idle at a time
+        idle[0] = SA_CUS;
+        int now = 0, end = 0;
+        for (int i = 0; i < tiles; i++) {
+            const int parts = sa_parts(blocks[i], p.most);
+            for (int x = 0; x < parts; x++) {
+                const int time = blocks[i] * (x + 1) / parts - blocks[i] * x / parts + START;
+                for (int n = a.H; n > 0;) {
+                    while (!idle[now]) now++;
+                    const int k = std::min(n, idle[now]);
+                    idle[now] -= k;
+                    idle[now + time] += k;
+                    end = std::max(end, now + time);
+                    n -= k;
+                }
+            }
+        }
+        return end;
+    };
+    sa_plan best = whole;
+    double least = 0.94 * end_of(whole);
+    for (int s = 15; s >= 2; s--) {
+        sa_plan p{(longest * s + 15) / 16, 0, true};
+        if (p.most < 4) break;
+        for (int i = 0; i < tiles; i++) p.wgs += sa_parts(blocks[i], p.most) * a.H;
+        if ((size_t)p.wgs * SA_PART > part_bytes) break;
+        const double t = end_of(p) + 1.3 + 0.0044 * p.wgs;
+        if (t < least) { least = t; best = p; }
+    }
+    return best;
+}
 template <int KS, int NJ, bool DIST>
-static void sa_launch(hipStream_t st, const sa_attn &a, int H) {
+static void sa_launch(hipStream_t st, const sa_attn &a, const sa_plan &p, int H) {
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) (void)hipFuncSetAttribute((const void *)split_attn_kernel<KS, NJ, DIST>, hipFuncAttributeMaxDynamicSharedMemorySize, sa_lds<KS, NJ>());
-    hipLaunchKernelGGL((split_attn_kernel<KS, NJ, DIST>), dim3(H, (a.T + SA_ROWS - 1) / SA_ROWS), dim3(512), (sa_lds<KS, NJ>()), st, a);
+    hipLaunchKernelGGL((split_attn_kernel<KS, NJ, DIST>), dim3(p.wgs), dim3(512), (sa_lds<KS, NJ>()), st, a);
+    if (p.join) hipLaunchKernelGGL((split_join_kernel<NJ>), dim3(H * ((a.T + SA_ROWS - 1) / SA_ROWS), 2), dim3(256), 0, st, a);
 }
 void psk_split_attn(hipStream_t st, const psk_split_attn_args &x) {
     sa_keys k{};
@@ -464,9 +588,15 @@ void psk_split_attn(hipStream_t st, const psk_split_attn_args &x) {
     k.ks_own = x.own / 32; k.ks_shared = x.n_shared / 32; k.nj = 8; k.G = x.G;
     k.img = (char *)x.scratch;
     k.img_shared = k.img + (size_t)x.G * k.nb * (k.ks_own * 6144 + k.nj * 3072);
-    hipLaunchKernelGGL(split_keys_kernel, dim3(k.nb, x.G + (x.n_shared > 0)), dim3(256), 0, st, k);
-    sa_attn a{k.img, k.img_shared, k.nbf, k.nb, k.ks_own, x.H / x.G, (int)x.pos0, (int)x.first, x.T, x.window, x.pool, x.keep, x.q, x.ldq, x.own + x.n_shared, x.own, x.rot_dims, x.pairing, x.freq,
-              x.rot_mag, x.scale, x.softcap, x.temp, x.slope, x.sink, x.gate, x.ldg, x.gate_elem, x.o, x.ldo};
-    if (x.own + x.n_shared == 192) x.slope ? sa_launch<6, 8, true>(st, a, x.H) : sa_launch<6, 8, false>(st, a, x.H);
-    else x.slope ? sa_launch<4, 8, true>(st, a, x.H) : sa_launch<4, 8, false>(st, a, x.H);
+    k.q = x.q; k.ldq = x.ldq; k.freq = x.freq; k.rot_mag = x.rot_mag; k.rot_dims = x.rot_dims; k.pairing = x.pairing; k.pos0 = (int)x.pos0; k.T = x.T; k.turners = x.rot_dims > 0 ? SA_TURNERS : 0;
+    k.q_turned = x.rot_dims > 0 ? (float *)(k.img_shared + (size_t)k.nb * k.ks_shared * 6144) : nullptr;
+    hipLaunchKernelGGL(split_keys_kernel, dim3(k.nb, k.turners + x.G + (x.n_shared > 0)), dim3(256), 0, st, k);
+    sa_attn a{k.img, k.img_shared, k.nbf, k.nb, k.ks_own, x.H / x.G, (int)x.pos0, (int)x.first, x.T, x.window, x.pool, x.keep, x.q, x.ldq, k.q_turned, x.scale, x.softcap,
+               x.temp, x.slope, x.sink, x.gate, x.ldg, x.gate_elem, x.o, x.ldo, x.ldq % 4 == 0 && ((uintptr_t)x.q & 15) == 0, x.H};
+    const sa_plan p = sa_plan_of(a, x.part_bytes);
+    a.most = p.most;
+    a.part = x.part;
+    a.part_ml = x.part + (size_t)p.wgs * (SA_ROWS * 128);
+    if (x.own + x.n_shared == 192) x.slope ? sa_launch<6, 8, true>(st, a, p, x.H) : sa_launch<6, 8, false>(st, a, p, x.H);
+    else x.slope ? sa_launch<4, 8, true>(st, a, p, x.H) : sa_launch<4, 8, false>(st, a, p, x.H);
 }

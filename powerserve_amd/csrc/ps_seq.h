@@ -273,7 +273,7 @@ struct psk_split_attn_args {
     const float *k = nullptr, *v = nullptr, *shared = nullptr, *front_k = nullptr, *front_v = nullptr;
     int64_t ldk = 0, ld_shared = 0;
     int mod = 0, off = 0, shared_mod = 0, shared_off = 0;
-    const float *q = nullptr; // head h of row t: q + t ldq + h (own + n_shared); its part behind `own` is rotated here where rot_dims > 0
+    const float *q = nullptr; // head h of row t: q + t ldq + h (own + n_shared); its part behind `own` is rotated here where rot_dims > 0 (G == H then)
     int64_t ldq = 0;
     const float *freq = nullptr;
     int rot_dims = 0, pairing = 0;
@@ -284,6 +284,8 @@ struct psk_split_attn_args {
     float *o = nullptr; // [T][ldo], head h at 128 h
     int64_t ldo = 0;
     void *scratch = nullptr; // psk_split_attn_scratch bytes
+    float *part = nullptr;   // for the parts of rows that several work-groups share (too small or none: they don't)
+    size_t part_bytes = 0;
 };
 bool psk_split_attn_ok(int own, int shared, int dv);
 bool psk_split_attn_takes(int T, int H); // enough rows to fill the chip

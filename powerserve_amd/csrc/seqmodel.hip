@@ -665,6 +665,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
     };
     auto split_attn_run = [&](const ps_seq_layer &l, psk_split_attn_args &g) {
         g.H = l.heads; g.own = l.dim; g.pos0 = pos0; g.T = T; g.window = l.window; g.scale = l.scale; g.o = m->t3; g.ldo = (int64_t)l.heads * l.vdim; g.scratch = m->sa_scratch;
+        g.part = m->split; g.part_bytes = m->split_bytes; // (between a layer's products)
         psk_split_attn(st, g);
     };
     // what the next layer's first product, which reads x, does to it in front of that (post-norm layers, a single token): x is then where that launch leaves it

@@ -419,6 +419,34 @@ def test_attention_of_many_rows(ctx, tmp_path, which):
     assert err(got, want) < min(TOL["float32"], 2 * err(plain, want) + 2e-6)
 
 
+# the same with rows whose keys several work-groups share (k_splitattn.hip split_join_kernel): parts in which some rows, or all, see no key; kept first tokens and means of blocks in parts of their own;
+# queries turned beforehand, in rows that no 16-byte load fits (81 gates behind them); the last rows of a tile missing; sinks, gates, a soft cap and slopes behind the sum
+@pytest.mark.parametrize("which", ["latent", "latent odd", "keep", "pool", "softcap"])
+def test_attention_of_many_rows_in_parts(ctx, tmp_path, which):
+    V, sizes = 40, (260, 140)
+    if which == "latent":
+        run, cfg = seq_oracle.run, synth.seq_config(64, V, [L("latent_attention", None, heads=64, dim=128, vdim=128, q_rank=40, kv_rank=64, mask={"size": 390}, scale=0.09,
+                                                              rot={"base": 500.0, "dims": 48}, rot_dim=64)], taps=2)
+    elif which == "latent odd":
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("latent_attention", synth.pupidra_latent(81, 96, 32, 128, 32, 0.1, 1e4))])
+    elif which == "keep":
+        at = lambda size, keep, own=None: synth.pupidra_attention(64, 2, 128, 128, 1.0, size, keep, own)
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("attention", at(150, 200)), synth.pupidra_layer("attention", at(310, 5, 0))])
+    elif which == "pool":
+        at = {"heads": 64, "kv_heads": 4, "dim": 128, "vdim": 128, "mask": {"size": 33, "pool": 2}, "rot": {"base": 100.0, "dims": 64}, "scale": 0.1}
+        run, cfg = seq_oracle.run_parallel, synth.parallel_config(64, V, [synth.parallel_layer(None, at, {"heads": 1, "dim": 16, "vdim": 16, "tau": 4.0}, 1.0, 0.5)], taps=2)
+    else:
+        run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(64, 8, 128, 128, 0.1, 5.0, (0.4, 7)), ff=64)])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=100, n_slots=1, max_context=500)
+    toks = tokens_for(cfg, sum(sizes))
+    want, got = run(cfg, t, toks), run_portions(m, toks, sizes)
+    m.set_mode(2)  # the plain kernels
+    plain = run_portions(m, toks, sizes)
+    m.close()
+    assert err(got, want) < min(TOL["float32"], 2 * err(plain, want) + 2e-6)
+
+
 # the same attention with an infinite key, value or query of one token (64 heads of 150 and 140 rows: k_splitattn.hip): a score of -inf is a weight of nothing, an infinite value makes the rows that see
 # it infinite (not NaN), and rows that do not see the token -- those in front of it in the same 16 rows and 32 keys too -- are what they are without it
 @pytest.mark.parametrize("what", ["k", "v", "q"])

@@ -250,6 +250,27 @@ for sizes in ((128, 64), (192, 40), (96, 80), (64, 128), (256, 39), (256, 32), (
 """.replace(".dir", str(child.tmp / "dir")))
 
 
+def test_portions_whose_rows_several_work_groups_share(child):
+    """k_splitattn.hip sa_plan_of: where whole tiles of 128 rows leave CUs waiting -- fewer tiles than CUs behind many keys -- their parts are joined; tiles of a few blocks and many tiles stay whole"""
+    child("""
+ctx = hip.Ctx(0)
+def joined(tokens, heads, behind=0):
+    cfg = synth.zusolix_config(64, 30, [synth.zusolix_layer("attention", synth.zusolix_attention(heads, 1, 128, 128, 0.1))])
+    synth.write_seq_model_dir(".dir", cfg, 1)
+    m = seqmodel.SeqModel(ctx, ".dir", max_batch=1500, n_slots=1, max_context=3000)
+    s = m.acquire()
+    if behind: m.forward(s, [1] * behind)
+    fake.fake_reset()
+    m.forward(s, [1] * tokens)
+    assert count("split_attn_kernel") == 1
+    n = count("split_join_kernel")
+    m.close()
+    return n
+for sizes in ((1400, 16), (129, 64, 1000), (700, 32)): assert joined(*sizes) == 1, sizes
+for sizes in ((129, 64), (400, 64), (1024, 128)): assert joined(*sizes) == 0, sizes
+""".replace(".dir", str(child.tmp / "dir")))
+
+
 def test_the_measured_products_of_experts_are_the_ones_that_run(child):
     """ps_hip_seq_bench_kernel: a portion's second product of the experts reads the rounded rows of the first one, in a step and where it is measured"""
     child("""
