@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void sq_norm_residual_kernel(float *x, const f
 // The same and the norm in front of the next sublayer (wn NULL: without it), a block per row with C runs of four numbers per thread in registers: hn = x / rms(x) * (offset + wn).  One launch
 // and one reading of x instead of two: 512 rows of 2048, 7.7 + 5.0 us before, 5.5 now.
 template <int C>
-__global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, const float *y, const float *w, const float *wn, float offset, float eps, int n, float *hn,
+__global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(const float *x, float *xo, const float *y, const float *w, const float *wn, float offset, float eps, int n, float *hn,
                                                                      unsigned short *copy16) {
     __shared__ float red[2][16];
     const int tid = threadIdx.x, nw = blockDim.x >> 6;
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, c
             xv[c][e] += yv[c][e] * inv * (offset + g[c][e]);
             s += xv[c][e] * xv[c][e];
         }
-        if (i < n) *(sq_f4 *)(x + at + i) = xv[c];
+        if (i < n) *(sq_f4 *)(xo + at + i) = xv[c];
         if (i < n && copy16) *(sq_us4 *)(copy16 + at + i) = sq_bf16x4(xv[c]);
     }
     if (!wn) return;
@@ -216,17 +216,20 @@ __global__ __launch_bounds__(1024) void sq_norm_residual_fast_kernel(float *x, c
         if (i < n) *(sq_f4 *)(hn + at + i) = o;
     }
 }
-bool psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups, const float *wn, float *hn, uint16_t *copy16) {
+bool psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups, const float *wn, float *hn, uint16_t *copy16,
+                       float *xo) {
     if (rows <= 0) return false;
-    if (groups == 1 && n % 4 == 0 && n <= 8192 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w | (uintptr_t)wn | (uintptr_t)hn) & 15) == 0) {
+    if (!xo) xo = x;
+    if (groups == 1 && n % 4 == 0 && n <= 8192 && (((uintptr_t)x | (uintptr_t)xo | (uintptr_t)y | (uintptr_t)w | (uintptr_t)wn | (uintptr_t)hn) & 15) == 0) {
         const int c = n <= 1024 ? 1 : n <= 2048 ? 2 : 4;
         const int threads = (int)((n / 4 + c - 1) / c + 63) / 64 * 64;
-        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, st, x, y, w, wn, offset, eps, (int)n, hn, copy16); };
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, st, x, xo, y, w, wn, offset, eps, (int)n, hn, copy16); };
         c == 1 ? go(sq_norm_residual_fast_kernel<1>) : c == 2 ? go(sq_norm_residual_fast_kernel<2>) : go(sq_norm_residual_fast_kernel<4>);
         return copy16 != nullptr;
     }
-    hipLaunchKernelGGL(sq_norm_residual_kernel, dim3(rows, groups), dim3(256), 0, st, x, y, w, offset, eps, (long long)(n / groups));
-    if (wn) psk_rmsnorm(st, x, n, nullptr, wn, offset, eps, n, rows, hn, n, groups);
+    if (xo != x) psk_copy(st, x, xo, (int64_t)rows * n);
+    hipLaunchKernelGGL(sq_norm_residual_kernel, dim3(rows, groups), dim3(256), 0, st, xo, y, w, offset, eps, (long long)(n / groups));
+    if (wn) psk_rmsnorm(st, xo, n, nullptr, wn, offset, eps, n, rows, hn, n, groups);
     return false;
 }
 
@@ -358,6 +361,113 @@ bool psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, 
     hipLaunchKernelGGL(sq_conv_kernel, dim3(gx, gy), dim3(256), 0, st, step, (long long)tail_off, in, (long long)ldi, w, taps, mode, (long long)C, T, out, (long long)ldo, bias);
     if (gy > 1 && taps > 1) hipLaunchKernelGGL(sq_conv_tail_kernel, dim3(gx), dim3(256), 0, st, step, (long long)tail_off, in, (long long)ldi, taps, (long long)C, T);
     return false;
+}
+
+// A portion's sublayer boundary in one launch: x + norm_b(y) -> xo, hn = norm(that), h = hn + its four-tap filter (y NULL: x as it is, nothing written to xo).  R rows per work-group, four channels per thread, and
+// the three rows in front of them again, whose norms the filter needs: everything is requested at once, the R + 3 rows' sums run side by side, and hn never leaves the registers.  xo is not x: the rows in
+// front are another work-group's.  The first work-group reads the tail instead of rows in front, and brings it up to date: the portion's last three rows are its own three.
+// What bounds it: the way of a row through memory, two sums and back where the work-groups stand on the chip at once, five passes over the rows beyond.  Four rows a work-group share the three in front better
+// than three, and three leave more work-groups, so three while they all stand on the chip (T <= 512).  Rows of more than 2048 numbers are sixteen waves, one work-group per CU: up to 256 of them their sums take
+// as long as the launch saves.  us, norms and filter in a launch each | R = 3 | 4: 2047 x 2048 23.3 | - | 18.5, 1100 16.7 | - | 13.7, 600 12.6 | - | 9.8, 300 (fp32) 9.9 | 6.8 | 7.6, 40 8.8 | 7.2 | 7.8;
+// 900 x 4096 23.5 | - | 16.7, 400 15.4 | 13.6 | 14.7, 203 11.8 | 12.1 | 13.1.  (Six and eight rows: 20 and 22 us of 2047 x 2048.)
+template <int R>
+__global__ __launch_bounds__(1024) void sq_boundary_rows_kernel(const ps_seq_step *step, long long tail_off, const float *x, float *xo, const float *y, const float *wb, const float *wn, const float *cw,
+                                                                float offset, float eps, int n, int T, float *h, unsigned short *copy16) {
+    static_assert(R >= 3, "only the first work-group reads the tail");
+    constexpr int S = R + 3;
+    __shared__ __attribute__((aligned(16))) float red[2][S][64]; // a sum of every sixteen lanes
+    const int tid = threadIdx.x, nw = blockDim.x >> 6, c = tid * 4, per = (int)gridDim.x >> 3, chunk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3), t0 = chunk * R; // (neighbours on one XCD)
+    if (t0 >= T) return; // (uniform)
+    const bool in = c < n, first = chunk == 0;
+    float *tail = step->state + tail_off;
+    // (rows that do not exist repeat others, threads behind the row its last four numbers: no load stands behind a branch)
+    auto row = [&](const int s) { return min(max(first && s < 3 ? T - 3 + s : t0 - 3 + s, 0), T - 1); };
+    const int ci = min(c, n - 4);
+    sq_f4 xv[S], yv[S], old[3], f[4], g = {}, gn = *(const sq_f4 *)(wn + ci);
+#pragma unroll
+    for (int s = 0; s < S; s++) xv[s] = *(const sq_f4 *)(x + (long long)row(s) * n + ci);
+    if (y) { // (uniform)
+        g = *(const sq_f4 *)(wb + ci);
+#pragma unroll
+        for (int s = 0; s < S; s++) yv[s] = *(const sq_f4 *)(y + (long long)row(s) * n + ci);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) f[j] = *(const sq_f4 *)(cw + (long long)ci * 4 + 4 * j); // channel ci + j's taps
+    if (first) { // (uniform)
+#pragma unroll
+        for (int i = 0; i < 3; i++) old[i] = *(const sq_f4 *)(tail + (long long)i * n + ci);
+    }
+    auto scales = [&](const sq_f4 (&v)[S], float (&r)[S][64], float (&inv)[S]) { // of every row
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            float q = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) q += v[s][e] * v[s][e];
+            q = sq_row_sum(in ? q : 0.f);
+            if ((tid & 15) == 0) r[s][tid >> 4] = q;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < S; s += 4) { // sixteen lanes a row, a wave's four sums each (a thread that adds them for itself, one behind the other, and for every row: 31 us of 2047 x 2048, R = 8)
+            const int mine = s + ((tid & 63) >> 4), u = tid & 15;
+            const sq_f4 w = mine < S && u < nw ? *(const sq_f4 *)&r[mine][4 * u] : sq_f4{0.f, 0.f, 0.f, 0.f};
+            const float v = 1.f / sqrtf(sq_row_sum((w[0] + w[1]) + (w[2] + w[3])) / (float)n + eps);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (s + q < S) inv[s + q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16 * q));
+        }
+    };
+    float inv[S];
+    if (y) { // (uniform)
+        scales(yv, red[0], inv);
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) xv[s][e] += yv[s][e] * inv[s] * (offset + g[e]);
+            if (s >= 3 && in && t0 - 3 + s < T) *(sq_f4 *)(xo + (long long)(t0 - 3 + s) * n + c) = xv[s];
+        }
+    }
+    scales(xv, red[1], inv);
+    if (!in) return;
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) xv[s][e] = xv[s][e] * inv[s] * (offset + gn[e]);
+    if (first) { // (uniform)
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const sq_f4 last = T - 3 + i >= 0 ? xv[i] : old[2]; // (two tokens: the old tail moves by as many)
+            xv[i] = old[i];
+            *(sq_f4 *)(tail + (long long)i * n + c) = last;
+        }
+    }
+#pragma unroll
+    for (int s = 3; s < S; s++) {
+        const long long t = t0 - 3 + s;
+        if (t >= T) break;
+        sq_f4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float q = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) q = fmaf(f[e][j], xv[s - 3 + j][e], q);
+            o[e] = xv[s][e] + q;
+        }
+        *(sq_f4 *)(h + t * n + c) = o;
+        if (copy16) *(sq_us4 *)(copy16 + t * n + c) = sq_bf16x4(o);
+    }
+}
+bool psk_boundary_rows(hipStream_t st, const ps_seq_step *step, const float *x, float *xo, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off, float offset, float eps,
+                       int64_t n, int T, float *h, uint16_t *copy16) {
+    if (T < 2 || taps != 4 || n % 4 || n > (T > 256 ? 4096 : 2048) || tail_off % 4 || x == xo ||
+        (((uintptr_t)x | (uintptr_t)xo | (uintptr_t)y | (uintptr_t)wb | (uintptr_t)wn | (uintptr_t)cw | (uintptr_t)h) & 15) || ((uintptr_t)copy16 & 7))
+        return false;
+    const int threads = (int)(n / 4 + 63) / 64 * 64;
+    auto go = [&](auto kernel, const int R) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(((T + R - 1) / R + 7) / 8 * 8)), dim3(threads), 0, st, step, (long long)tail_off, x, xo, y, wb, wn, cw, offset, eps, (int)n, T, h, copy16);
+    };
+    T > 512 ? go(sq_boundary_rows_kernel<4>, 4) : go(sq_boundary_rows_kernel<3>, 3);
+    return true;
 }
 
 __global__ void sq_state_store_kernel(const ps_seq_step *step, long long off, const float *src, long long n) {

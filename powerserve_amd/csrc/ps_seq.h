@@ -132,7 +132,7 @@ void psk_rmsnorm(hipStream_t st, const float *x, int64_t ldx, const int32_t *idx
 // (wn given: hn = norm(x) (offset + wn) behind it)
 // (copy16 of these and of psk_causal_conv, psk_headnorm_gate, psk_gate_partnorm: also the result -- x here -- rounded to bf16, rows side by side; returns whether that was done)
 bool psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups = 1, const float *wn = nullptr,
-                       float *hn = nullptr, uint16_t *copy16 = nullptr);
+                       float *hn = nullptr, uint16_t *copy16 = nullptr, float *xo = nullptr);
 // The front of a parallel layer that has no input filter, in one launch: x[r] = sum_j mix[j] X_j[row(r)] over the nmix streams X_j = src + j stride (mix NULL:
 // the last stream alone), row(r) = idx ? idx[r] : r, stored to xout[r] (NULL: not kept); then h[r] = norm(x) (offset + w1) and h2[r] = norm(x) (offset + w2) with
 // the norm taken over `groups` parts -- two norms of one vector share their statistics.  w1 / w2 NULL: that output is not made.
@@ -152,11 +152,17 @@ void psk_mingru_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off,
 // (a residual around the convolution), mode 1: f = silu(sum + bias[c]) (bias NULL: none).  The tail is brought up to date behind it.
 bool psk_causal_conv(hipStream_t st, const ps_seq_step *step, int64_t tail_off, const float *in, int64_t ldi, const float *w, int taps, int mode,
                      int64_t C, int T, float *out, int64_t ldo, const float *bias = nullptr, uint16_t *copy16 = nullptr);
-static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane gets it: rotations inside a row of sixteen, then the four rows' sums (no trip through LDS)
+// a sequential layer's boundary of several rows: xo = x + norm_b(y) (xo is not x; y NULL: x as it is), h = conv(norm(that)); false: not done (other taps, wide or unaligned rows)
+bool psk_boundary_rows(hipStream_t st, const ps_seq_step *step, const float *x, float *xo, const float *y, const float *wb, const float *wn, const float *cw, int taps, int64_t tail_off, float offset, float eps,
+                       int64_t n, int T, float *h, uint16_t *copy16);
+static __device__ __forceinline__ float sq_row_sum(float v) { // of sixteen neighbouring lanes, by rotations; every lane gets it
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));
+}
+static __device__ __forceinline__ float sq_wave_sum(float v) { // every lane gets it: rotations inside a row of sixteen, then the four rows' sums (no trip through LDS)
+    v = sq_row_sum(v);
     auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
     return (row(0) + row(16)) + (row(32) + row(48));
 }

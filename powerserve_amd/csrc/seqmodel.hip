@@ -644,7 +644,8 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         return g;
     };
     // a sublayer boundary: x += norm_b(y) (after a sublayer), then hn = norm(x), h = conv(hn) (in front of the next one); one launch for a single token
-    bool final_made = false;
+    bool final_made = false, sequential = m->groups == 1 && !m->hist; // (of nothing but sequential layers, m->hn has no other reader: the residual stream of several rows stands there for some layers)
+    for (auto &P : m->L) sequential = sequential && P.d.form == PS_LAYER_SEQUENTIAL;
     const bool plain_final = T == 1 && rows == 1 && !tiled && m->groups == 1 && !m->hist && !D.norm_center && !D.final_norm_bias;
     auto boundary = [&](const float *y, const float *wb, const float *wn, const float *cw, int64_t tail_off, const bool last = false) {
         if (T == 1 && !tiled && m->groups == 1) {
@@ -653,7 +654,17 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             else if (psk_boundary1(st, m->step, x, y, wb, wn, cw, D.canon_taps, tail_off, D.norm_offset, D.norm_eps, W, m->h, m->hn, x == m->x ? m->x2 : m->x)) x = x == m->x ? m->x2 : m->x;
             return;
         }
-        if (y) rounded = psk_norm_residual(st, x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn, wn ? nullptr : copy16) ? x : nullptr;
+        float *const other = x == m->x ? m->hn : m->x;
+        if (wn && sequential && !tiled && psk_boundary_rows(st, m->step, x, other, y, wb, wn, cw, D.canon_taps, tail_off, D.norm_offset, D.norm_eps, W, T, m->h, copy16)) {
+            if (y) x = other;
+            rounded = copy16 ? m->h : nullptr;
+            return;
+        }
+        if (y) {
+            const bool made = psk_norm_residual(st, x, y, wb, D.norm_offset, D.norm_eps, W, T, m->groups, wn, m->hn, wn ? nullptr : copy16, m->x);
+            x = m->x;
+            rounded = made ? x : nullptr;
+        }
         if (wn) {
             if (!y) psk_rmsnorm(st, x, W, nullptr, wn, D.norm_offset, D.norm_eps, W, T, m->hn, W, m->groups);
             rounded = psk_causal_conv(st, m->step, tail_off, m->hn, W, cw, D.canon_taps, 0, W, T, m->h, W, nullptr, copy16) ? m->h : nullptr;

@@ -78,6 +78,25 @@ def run_portions(m, toks, sizes):
     return np.concatenate(out)
 
 
+# a portion's boundaries in one launch each (k_seqmix.hip sq_boundary_rows_kernel): portions of fewer tokens than the filter reaches back, whole and begun work-groups of three rows and of four (from 513
+# on), single tokens in between (a launch of their own, over the same tail), long rows of few tokens (as before: a launch each); rows that end inside a wave, in one of sixteen waves; a layer without feed-forward; the layers' results as well
+@pytest.mark.parametrize("width,sizes", [(64, (2, 3, 1, 4, 5, 2, 2)), (260, (9, 1, 64)), (1028, (33, 2, 2)), (4096, (257, 5)), (260, (513, 3)), (64, (518, 2))])
+def test_boundaries_of_a_portion(ctx, tmp_path, width, sizes):
+    cfg = synth.seq_config(width, 30, [L("wkv", 24, heads=1, dim=8), L("delta", None, heads=2, kv_heads=1, dim=8, vdim=4, conv=2), L("wkv", 40, heads=1, dim=8)], taps=4)
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=600, n_slots=1, max_context=700)
+    toks, per = tokens_for(cfg, 2 * sum(sizes) if sum(sizes) < 99 else sum(sizes)), []
+    want = seq_oracle.run(cfg, t, toks, per)
+    assert err(run_portions(m, toks, sizes), want) < TOL["float32"]
+    m.capture_layers()
+    s, first = m.acquire(), sizes[0]
+    m.forward(s, toks[:first])
+    got = m.layers(first)
+    m.close()
+    for g, w in zip(got, per):
+        assert err(g, w[:first]) < TOL["float32"]
+
+
 # wkv and delta rule in chunks of 16 tokens (k_chunk.hip): portions that end inside, on and one behind a chunk's edge, fewer than 32 tokens between them (the scan), state row tiles that
 # do not fill the four waves and more than they are, value columns that are no multiple of 16; decays from e^-20 a token to none at all
 @pytest.mark.parametrize("sizes", [(31, 33), (32,), (47, 5, 49), (64, 17), (100,)])
