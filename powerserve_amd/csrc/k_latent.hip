@@ -27,12 +27,23 @@ static __device__ __forceinline__ void la_pair(int i, int half, int pairing, int
     else { a = i; b = i + half; }
 }
 
-__global__ __launch_bounds__(256) void latent_prep_kernel(const ps_seq_step *step, long long ring_off, int cap, const float *y, long long ldy, const float *qnorm,
-                                                          const float *kvnorm, float eps, int q_rank, int kv_rank, int rot_dim, int rot_dims, const float *freq, float *cq,
-                                                          long long ldcq, float rot_mag, int pairing) {
+struct la_token { // psk_latent_row and what else the row's preparation takes
+    const float *y, *qnorm, *kvnorm;
+    long long ldy, ldcq;
+    float eps;
+    int q_rank, kv_rank, rot_dim, rot_dims, pairing;
+    float *cq;
+    const float *freq;
+    float rot_mag;
+};
+static __device__ __forceinline__ void la_prepare(const ps_seq_step *step, long long ring_off, int cap, const la_token &w, int t) { // by 256 threads
+    const float *y = w.y, *qnorm = w.qnorm, *kvnorm = w.kvnorm, *freq = w.freq;
+    float *cq = w.cq;
+    const long long ldy = w.ldy, ldcq = w.ldcq;
+    const float eps = w.eps, rot_mag = w.rot_mag;
+    const int q_rank = w.q_rank, kv_rank = w.kv_rank, rot_dim = w.rot_dim, rot_dims = w.rot_dims, pairing = w.pairing, tid = threadIdx.x;
     // (a thread's numbers and weights are requested together and held: 8 + 4 of them, what is beyond 2048 and 1024 is read again)
     __shared__ float red[8];
-    const int t = blockIdx.x, tid = threadIdx.x;
     const float *yt = y + (long long)t * ldy, *ckv = yt + q_rank, *kr = ckv + kv_rank;
     float qv[8], qw[8], kv[4], kw[4], a = 0.f, b = 0.f;
 #pragma unroll
@@ -80,10 +91,13 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const ps_seq_step *ste
     }
     for (int i = 2 * half + tid; i < rot_dim; i += 256) ring[kv_rank + i] = kr[i];
 }
-void psk_latent_prep(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *y, int64_t ldy, const float *qnorm, const float *kvnorm,
-                     float eps, int q_rank, int kv_rank, int rot_dim, int rot_dims, const float *freq, int T, float *cq, int64_t ldcq, float rot_mag, int pairing) {
-    hipLaunchKernelGGL(latent_prep_kernel, dim3(T), dim3(256), 0, st, step, (long long)ring_off, cap, y, (long long)ldy, qnorm, kvnorm, eps, q_rank, kv_rank, rot_dim,
-                       rot_dims, freq, cq, (long long)ldcq, rot_mag, pairing);
+__global__ __launch_bounds__(256) void latent_prep_kernel(const ps_seq_step *step, long long ring_off, int cap, la_token w) { la_prepare(step, ring_off, cap, w, blockIdx.x); }
+static la_token la_token_of(const psk_latent_row &r, int kv_rank, int rot_dim, int rot_dims, const float *freq, float rot_mag, int pairing) {
+    return la_token{r.y, r.qnorm, r.kvnorm, (long long)r.ldy, (long long)r.ldcq, r.eps, r.q_rank, kv_rank, rot_dim, rot_dims, pairing, r.cq, freq, rot_mag};
+}
+void psk_latent_prep(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const psk_latent_row &row, int kv_rank, int rot_dim, int rot_dims, const float *freq, int T, float rot_mag,
+                     int pairing) {
+    hipLaunchKernelGGL(latent_prep_kernel, dim3(T), dim3(256), 0, st, step, (long long)ring_off, cap, la_token_of(row, kv_rank, rot_dim, rot_dims, freq, rot_mag, pairing));
 }
 
 // dynamic LDS: qs [d + dr], ps [64]
@@ -251,12 +265,21 @@ void psk_latent_attn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_
 }
 
 // ---------------------------------------------------------------------------------------------------- single token, absorbed
-// qa[h][r] = sum_i q[h][i] Wuk[h * d + i][r]: a head's query folded into latent space, and behind it (the last block of a head) its rotated part: qa [H][R + dr].
+// qa[h][r] = sum_i q[h][i] Wuk[h * d + i][r]: a head's query folded into latent space, and behind it (a block of its own) its rotated part: qa [H][R + dr].  Where the queries come straight
+// from the joint projection (row.y given), one more block prepares the token's ring row, which stood a launch in front: a token of
+// Pupidra 2048 x 6 377 -> 371 us (two such layers).
 template <typename WT>
 __global__ __launch_bounds__(256) void latent_fold_q_kernel(const ps_seq_step *step, const float *q, int qstride, const WT *wuk, int d, int R, int dr, int rot_dims, const float *freq,
-                                                            float rot_mag, int pairing, float *qa) {
+                                                            float rot_mag, int pairing, float *qa, long long ring_off, int cap, la_token row) {
+    if (row.y) { // (uniform)
+        if (blockIdx.y == 0) {
+            if (blockIdx.x == 0) la_prepare(step, ring_off, cap, row, 0);
+            return;
+        }
+    }
+    const int by = (int)blockIdx.y - (row.y ? 1 : 0);
     __shared__ float part[4][64];
-    const int h = blockIdx.x, r = blockIdx.y * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6; // block: 64 latent indices x 4 slices of the head's rows
+    const int h = blockIdx.x, r = by * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6; // block: 64 latent indices x 4 slices of the head's rows
     const float *qh = q + (long long)h * qstride;
     qa += (long long)h * (R + dr);
     if (blockIdx.y + 1 == gridDim.y) {
@@ -431,13 +454,15 @@ bool psk_latent_absorbed_ok(int d, int dr, int dv, int R) { return R % 16 == 0 &
 size_t psk_latent_absorbed_scratch(int H, int R, int dr, int window) { return ((size_t)((window + 15) / 16 + 1) * H * (R + 4) + (size_t)H * (2 * R + dr)) * 4; }
 // q [H][d + dr] (row stride qstride) -> o [H * dv]; ukv: rows uk | uv of the expansion matrix [H d + H dv][R]; scratch from psk_latent_absorbed_scratch
 void psk_latent_absorbed(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int qstride, const ps_dense *ukv, const float *freq,
-                         int H, int d, int dr, int rot_dims, int dv, int R, int window, float scale, float *scratch, float *o, float rot_mag, const float *gate, int pairing) {
+                         int H, int d, int dr, int rot_dims, int dv, int R, int window, float scale, float *scratch, float *o, float rot_mag, const float *gate, int pairing,
+                         const psk_latent_row *row) {
     const int max_tiles = (window + 15) / 16 + 1; // (a window that does not start on a tile's edge touches one tile more)
     float *qa = scratch, *ol = qa + (size_t)H * (R + dr), *part = ol + (size_t)H * R;
     const bool bf = ukv->dtype == PS_BF16;
-    const dim3 fold(H, (R + 63) / 64 + 1), grid(max_tiles, (H + 15) / 16);
-    if (bf) hipLaunchKernelGGL(latent_fold_q_kernel<unsigned short>, fold, dim3(256), 0, st, step, q, qstride, (const unsigned short *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa);
-    else hipLaunchKernelGGL(latent_fold_q_kernel<float>, fold, dim3(256), 0, st, step, q, qstride, (const float *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa);
+    const la_token prep = row ? la_token_of(*row, R, dr, rot_dims, freq, rot_mag, pairing) : la_token{};
+    const dim3 fold(H, (R + 63) / 64 + 1 + (row ? 1 : 0)), grid(max_tiles, (H + 15) / 16);
+    if (bf) hipLaunchKernelGGL(latent_fold_q_kernel<unsigned short>, fold, dim3(256), 0, st, step, q, qstride, (const unsigned short *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa, (long long)ring_off, cap, prep);
+    else hipLaunchKernelGGL(latent_fold_q_kernel<float>, fold, dim3(256), 0, st, step, q, qstride, (const float *)ukv->data, d, R, dr, rot_dims, freq, rot_mag, pairing, qa, (long long)ring_off, cap, prep);
     const auto attend = R <= 256 ? latent_absorbed_kernel<1> : latent_absorbed_kernel<2>;
     hipLaunchKernelGGL(attend, grid, dim3(256), 0, st, step, (long long)ring_off, cap, qa, dr, H, R, window, scale, part);
     hipLaunchKernelGGL(latent_combine_kernel, dim3(H, (R + 63) / 64), dim3(256), max_tiles <= LA_HELD ? (size_t)max_tiles * 4 : 0, st, step, part, H, R, window, max_tiles, ol);

@@ -671,10 +671,19 @@ static __device__ __forceinline__ float sq_col_sum(float v, int R) {
 //   GLA = 0 (wkv)  o_j = sum_i r_i (S_ij + bonus_i k_i v_j), then S_ij <- w_i S_ij + k_i v_j,  w = exp(-exp(z))
 //   GLA = 1        S_ij <- w_i S_ij + k_i v_j, then o_j = sum_i (qscale r_i) S_ij,              w = sigmoid(z)^inv_tau = exp(-softplus(-z) inv_tau)
 // LDS: rs, ks, ws [TC][dp] (dp = NR * R, rows >= d zero), sc [TC] (sum_i r_i bonus_i k_i)
-template <int GLA, int TC>
+// FOLD (a single token): z is not there yet -- z = bias + w a, a of a few numbers, which every work-group makes of its head's rows where it would read them -- and the token's input is left behind as the
+// next one's neighbour.  A launch for the product and one for the copy, 4.4 us each behind 4096 channels, took more than the scan (5.1 us,
+// 6.0 with them): a token of Ranutar 4096 x 3 322 -> 317 us, 2048 x 6 346 -> 338.
+struct sq_fold {
+    const void *w; // [H d][rank]
+    const float *bias, *a, *src;
+    int bf16, eights, rank; // eights: rows of bf16 in whole eights
+    long long dst_off, n; // src [n] -> state + dst_off
+};
+template <int GLA, int TC, bool FOLD = false>
 __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *step, long long state_off, const float *r, const float *k, const float *v, const float *z,
                                                             long long ld, long long ldz, const float *bonus, int d, int dv, float qscale, float inv_tau, int R, int T,
-                                                            float *o, long long ldo) {
+                                                            float *o, long long ldo, sq_fold fold) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int dp = SQ_NR * R, cpb = 256 / R;
     float *rs = lds, *ks = rs + TC * dp, *ws = ks + TC * dp, *sc = ws + TC * dp;
@@ -688,6 +697,9 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
         S[m] = (col && i < d) ? S0[(long long)i * dv + j] : 0.f;
     }
     const long long hb = (long long)h * d, vb = (long long)h * dv;
+    if constexpr (FOLD) {
+        for (long long i = ((long long)h * gridDim.x + blockIdx.x) * 256 + tid; i < fold.n; i += (long long)gridDim.x * gridDim.y * 256) step->state[fold.dst_off + i] = fold.src[i];
+    }
     // the next round's inputs are requested before the current round's steps run, and land in LDS after them
     float pa[TC], pb[TC], pc[TC], pv[TC];
     auto fetch = [&](int t0) {
@@ -699,7 +711,23 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
             const long long at = (long long)(t0 + (in ? t : 0)) * ld + hb + (in ? i : 0);
             pa[e] = in ? r[at] : 0.f;
             pb[e] = in ? k[at] : 0.f;
-            pc[e] = in ? z[(long long)(t0 + t) * ldz + hb + i] : (GLA ? INFINITY : -INFINITY); // w = 1: with k = 0 a token that is not there leaves the state alone
+            if constexpr (FOLD) {
+                pc[e] = -INFINITY;
+                if (in) {
+                    const long long wi = (hb + i) * fold.rank;
+                    float c = 0.f;
+                    if (fold.eights) { // (uniform)
+                        for (int u = 0; u < fold.rank; u += 8) {
+                            const sq_us4 w0 = *(const sq_us4 *)((const unsigned short *)fold.w + wi + u), w1 = *(const sq_us4 *)((const unsigned short *)fold.w + wi + u + 4);
+#pragma unroll
+                            for (int x = 0; x < 8; x++) c = fmaf(__uint_as_float((unsigned)(x < 4 ? w0[x] : w1[x - 4]) << 16), fold.a[u + x], c);
+                        }
+                    } else {
+                        for (int u = 0; u < fold.rank; u++) c = fmaf(fold.bf16 ? __uint_as_float((unsigned)((const unsigned short *)fold.w)[wi + u] << 16) : ((const float *)fold.w)[wi + u], fold.a[u], c);
+                    }
+                    pc[e] = c + fold.bias[hb + i];
+                }
+            } else pc[e] = in ? z[(long long)(t0 + t) * ldz + hb + i] : (GLA ? INFINITY : -INFINITY); // w = 1: with k = 0 a token that is not there leaves the state alone
         }
 #pragma unroll
         for (int t = 0; t < TC; t++) pv[t] = (col && t < nt) ? v[(long long)(t0 + t) * ld + vb + j] : 0.f;
@@ -762,13 +790,14 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
     }
 }
 void psk_wkv_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *r, const float *k, const float *v, const float *z, int64_t ld,
-                  const float *bonus, int H, int d, int T, float *o, int64_t ldo) {
+                  const float *bonus, int H, int d, int T, float *o, int64_t ldo, const psk_wkv_fold *f) {
     const int R = sq_lanes_per_col(d), cpb = 256 / R;
     const int tc = T == 1 ? 1 : SQ_TC;
     const size_t lds = (size_t)(3 * tc * SQ_NR * R + tc) * 4;
-    const auto kernel = T == 1 ? sq_decay_scan_kernel<0, 1> : sq_decay_scan_kernel<0, SQ_TC>;
+    const auto kernel = f ? sq_decay_scan_kernel<0, 1, true> : T == 1 ? sq_decay_scan_kernel<0, 1> : sq_decay_scan_kernel<0, SQ_TC>; // (f: T == 1)
+    const sq_fold fold = f ? sq_fold{f->w->data, f->bias, f->a, f->src, f->w->dtype == PS_BF16, f->w->dtype == PS_BF16 && f->w->K % 8 == 0, (int)f->w->K, (long long)f->dst_off, (long long)f->n} : sq_fold{};
     hipLaunchKernelGGL(kernel, dim3((d + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, r, k, v, z, (long long)ld, (long long)ld, bonus, d, d, 1.f, 1.f,
-                       R, T, o, (long long)ldo);
+                       R, T, o, (long long)ldo, fold);
 }
 void psk_gla_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *q, const float *k, const float *v, int64_t ld, const float *z, int64_t ldz,
                   float tau, int H, int d, int dv, int T, float *o, int64_t ldo) {
@@ -777,7 +806,7 @@ void psk_gla_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, co
     const size_t lds = (size_t)(3 * tc * SQ_NR * R + tc) * 4;
     const auto kernel = T == 1 ? sq_decay_scan_kernel<1, 1> : sq_decay_scan_kernel<1, SQ_TC>;
     hipLaunchKernelGGL(kernel, dim3((dv + cpb - 1) / cpb, H), dim3(256), lds, st, step, (long long)state_off, q, k, v, z, (long long)ld, (long long)ldz, nullptr, d, dv,
-                       1.f / sqrtf((float)d), 1.f / tau, R, T, o, (long long)ldo);
+                       1.f / sqrtf((float)d), 1.f / tau, R, T, o, (long long)ldo, sq_fold{});
 }
 
 // LDS: qs, ks [TC][dp]; per token: g, beta, kq

@@ -178,8 +178,14 @@ void psk_copy(hipStream_t st, const float *src, float *dst, int64_t n);
 
 // wkv scan.  r, k, v, z: [T][H*d] (row stride ld), z = the decay's pre-activation (w = exp(-exp(z))); bonus [H*d]; state [H][d][d] fp32 at
 // step->state + state_off.  o[t][h][j] = sum_i r_i (S_ij + bonus_i k_i v_j), then S_ij = w_i S_ij + k_i v_j.
+// f (a single token): z = f.bias + f.w f.a instead (f.w [H d][a few]), and src [n] -> step->state + dst_off.
+struct psk_wkv_fold {
+    const ps_dense *w = nullptr;
+    const float *bias = nullptr, *a = nullptr, *src = nullptr;
+    int64_t dst_off = 0, n = 0;
+};
 void psk_wkv_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *r, const float *k, const float *v, const float *z, int64_t ld,
-                  const float *bonus, int H, int d, int T, float *o, int64_t ldo);
+                  const float *bonus, int H, int d, int T, float *o, int64_t ldo, const psk_wkv_fold *f = nullptr);
 // gated linear attention scan.  q, k [T][H*d], v [T][H*dv] (row stride ld), z [T][H*d] (row stride ldz) the decay's pre-activation; state [H][d][dv] fp32.
 // Per head: S <- diag(sigmoid(z)^(1/tau)) S + k v^T, then o = S^T (q d^-1/2).
 void psk_gla_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *q, const float *k, const float *v, int64_t ld, const float *z, int64_t ldz,
@@ -249,8 +255,16 @@ void psk_moe_combine(hipStream_t st, float *x, const float *y, int top, float al
 // ---- k_latent.hip
 // One token per block.  y[t] = [ dq (q_rank) | ckv (kv_rank) | kr (rot_dim) ]:  cq[t] = rmsnorm(dq) * qnorm;  ring row (pos mod cap):
 // c = rmsnorm(ckv) * kvnorm, kr with its first rot_dims numbers rotated at pos (angle of pair i: pos * freq[i]; pairs after `pairing`, a ps_rot_pairing, the same in all launches of a mixer).  Ring at step->state + ring_off: [cap][kv_rank + rot_dim].
-void psk_latent_prep(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *y, int64_t ldy, const float *qnorm, const float *kvnorm,
-                     float eps, int q_rank, int kv_rank, int rot_dim, int rot_dims, const float *freq, int T, float *cq, int64_t ldcq,
+struct psk_latent_row {
+    const float *y = nullptr;
+    int64_t ldy = 0;
+    const float *qnorm = nullptr, *kvnorm = nullptr;
+    float eps = 0.f;
+    int q_rank = 0;
+    float *cq = nullptr;
+    int64_t ldcq = 0;
+};
+void psk_latent_prep(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const psk_latent_row &row, int kv_rank, int rot_dim, int rot_dims, const float *freq, int T,
                      float rot_mag = 1.f, int pairing = PS_ROT_HALVES); // cos and sin of every rotation of this mixer are multiplied by rot_mag (the same value in all its launches); q_rank 0: no query latent
 // Windowed soft-max attention over expanded keys / values.  q [T][H*(d+dr)] (rotated part not yet rotated), kv [Nw][H*d + H*dv] for the positions
 // first .. first + Nw - 1 where first = max(0, pos0 - window + 1) (the caller expands exactly these ring rows), rotated key parts from the ring.
@@ -268,7 +282,7 @@ bool psk_latent_absorbed_ok(int d, int dr, int dv, int R);
 size_t psk_latent_absorbed_scratch(int H, int R, int dr, int window);
 void psk_latent_absorbed(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, const float *q, int qstride, const ps_dense *ukv, const float *freq,
                          int H, int d, int dr, int rot_dims, int dv, int R, int window, float scale, float *scratch, float *o, float rot_mag = 1.f,
-                         const float *gate = nullptr, int pairing = PS_ROT_HALVES);
+                         const float *gate = nullptr, int pairing = PS_ROT_HALVES, const psk_latent_row *row = nullptr);
 
 // ---- k_splitattn.hip: the attention of a portion of many rows (position pos0 and on, H heads over G key / value groups) whose window is known on the host
 struct psk_split_attn_args {

@@ -727,13 +727,19 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 auto g = mm(l.decay1, in, W, m->t2, l.decay_rank);
                 g.mu = l.mu + 4 * W; g.shift0 = state + P.off_shift; g.act = PSD_ACT_TANH;
                 psk_dense(st, g);
+            }
+            psk_wkv_fold f;
+            const bool folds = T == 1 && !tiled && l.decay_rank <= 64; // (a longer rank: rows that want a launch of their own)
+            if (folds) {
+                f.w = l.decay2; f.bias = l.decay0; f.a = m->t2; f.src = in; f.dst_off = P.off_shift; f.n = W;
+            } else {
                 auto g2 = mm(l.decay2, m->t2, l.decay_rank, m->t1 + 4 * Hd, NW);
                 g2.bias = l.decay0;
                 psk_dense(st, g2);
+                psk_state_store(st, m->step, P.off_shift, in + (int64_t)(T - 1) * W, W);
             }
-            psk_state_store(st, m->step, P.off_shift, in + (int64_t)(T - 1) * W, W);
             if (chunked && psk_chunked_ok((int)d)) psk_wkv_chunked(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->ssd_scratch, m->t3, Hd);
-            else psk_wkv_scan(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->t3, Hd);
+            else psk_wkv_scan(st, m->step, P.off_S, m->t1, m->t1 + Hd, m->t1 + 2 * Hd, m->t1 + 4 * Hd, NW, l.bonus, (int)H, (int)d, T, m->t3, Hd, folds ? &f : nullptr);
             normed_out(m->t3, d, m->t1 + 3 * Hd, NW, l.onorm, (int)d);
         } else if (l.kind == PS_MIX_DELTA) {
             const int64_t KHd = (int64_t)l.kv_heads * d, Hv = H * dv;
@@ -837,13 +843,14 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             const int64_t ldq = direct ? P.ncat : nq;
             const float *gate = l.gated ? m->t1 + P.ncat - H : nullptr;
             first_product(mm(l.in_cat, in, W, m->t1, P.ncat));
-            psk_latent_prep(st, m->step, P.off_ring, P.cap, direct ? m->t1 + nq : m->t1, P.ncat, l.qnorm, l.kvnorm, D.norm_eps, l.q_rank, l.kv_rank, (int)dr, l.rot_dims, P.freq, T,
-                            cq, l.q_rank, P.rot_mag, l.rot_pairing);
-            if (!direct) psk_dense(st, mm(l.uq, cq, l.q_rank, q, nq));
             const bool plain = (m->mode & 2) != 0, rows4 = (l.kv_rank + dr) % 4 == 0 && l.kv_rank % 4 == 0;
-            if (T == 1 && !plain && m->abs_scratch && psk_latent_absorbed_ok((int)d, (int)dr, (int)dv, l.kv_rank)) {
+            const bool absorbed = T == 1 && !plain && m->abs_scratch && psk_latent_absorbed_ok((int)d, (int)dr, (int)dv, l.kv_rank);
+            const psk_latent_row row{direct ? m->t1 + nq : m->t1, P.ncat, l.qnorm, l.kvnorm, D.norm_eps, l.q_rank, cq, l.q_rank};
+            if (!absorbed || !direct) psk_latent_prep(st, m->step, P.off_ring, P.cap, row, l.kv_rank, (int)dr, l.rot_dims, P.freq, T, P.rot_mag, l.rot_pairing);
+            if (!direct) psk_dense(st, mm(l.uq, cq, l.q_rank, q, nq));
+            if (absorbed) {
                 psk_latent_absorbed(st, m->step, P.off_ring, P.cap, q, (int)(d + dr), l.ukv, P.freq, (int)H, (int)d, (int)dr, l.rot_dims, (int)dv, l.kv_rank, l.window,
-                                    l.scale, m->abs_scratch, m->t3, P.rot_mag, gate, l.rot_pairing);
+                                    l.scale, m->abs_scratch, m->t3, P.rot_mag, gate, l.rot_pairing, direct ? &row : nullptr);
             } else {
                 // the window's keys and values, expanded from the ring rows  max(0, pos0 - window + 1) .. pos0 + T - 1
                 auto g = mm(l.ukv, state + P.off_ring, rs, m->kvx, H * d + Hv);

@@ -97,6 +97,19 @@ def test_boundaries_of_a_portion(ctx, tmp_path, width, sizes):
         assert err(g, w[:first]) < TOL["float32"]
 
 
+# a single token's decay, its second product inside the scan (k_seqmix.hip sq_fold): ranks in whole eights and not, the longest there and the first with a launch of its own, in both formats; heads of few
+# rows and of many; the next token's neighbour, behind a portion and behind single tokens
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rank", [1, 8, 13, 64, 65])
+def test_decay_of_a_single_token(ctx, tmp_path, rank, dtype):
+    cfg = synth.seq_config(160, 40, [L("wkv", None, heads=2, dim=24), L("wkv", 24, heads=1, dim=250)], taps=2)
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 3, synth.seq_tensors(cfg, 3, rank))
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype, max_batch=16, n_slots=1)
+    toks = tokens_for(cfg, 12)
+    assert err(run_portions(m, toks, (1, 1, 5, 1, 1, 1)), seq_oracle.run(cfg, t, toks)) < TOL[dtype]
+    m.close()
+
+
 # wkv and delta rule in chunks of 16 tokens (k_chunk.hip): portions that end inside, on and one behind a chunk's edge, fewer than 32 tokens between them (the scan), state row tiles that
 # do not fill the four waves and more than they are, value columns that are no multiple of 16; decays from e^-20 a token to none at all
 @pytest.mark.parametrize("sizes", [(31, 33), (32,), (47, 5, 49), (64, 17), (100,)])
