@@ -39,6 +39,22 @@ static __device__ __forceinline__ long long wa_front(long long p, int window, in
 // and one of the first `keep` tokens' rows into the front store too (store_off).
 // A step of ONE token also brings its block's sum up to date here (the thread that wrote a channel adds it: the same sum, in the same order, as
 // winattn_pool_kernel makes for a portion).  dynamic LDS: rot_dims floats (cos | sin of the token's angles, shared by all heads).
+// element i of a projection (c = its index in its head of d): normed, and where c < 2 half turned together with its partner (cs: half cosines, half sines); wc: 1 = one weight vector of d
+// numbers for every head (indexed by c), 0 = a weight per element of the projection
+static __device__ __forceinline__ float wa_turned(const float *src, const float *w, float inv, int i, int wc, int d, int half, int pairing, const float *cs) {
+    const int c = i % d;
+    if (w && wc) w += c - i;
+    const float self = src[i] * inv * (w ? w[i] : 1.f);
+    if (c >= 2 * half) return self;
+    int partner, pair;
+    bool first;
+    if (pairing == PS_ROT_NEIGHBOURS) { partner = i - c + (c ^ 1); pair = c >> 1; first = !(c & 1); }
+    else { first = c < half; partner = first ? i + half : i - half; pair = first ? c : c - half; }
+    const float other = src[partner] * inv * (w ? w[partner] : 1.f);
+    return first ? self * cs[pair] - other * cs[half + pair] : self * cs[pair] + other * cs[half + pair];
+}
+// a query temperature that grows with the position in steps of `every` tokens: 1 + coef ln(floor((pos + 1) / every) + 1)
+static __device__ __forceinline__ float wa_qtemp(long long pos, float coef, int every) { return every > 0 ? 1.f + coef * logf((float)((pos + 1) / every) + 1.f) : 1.f; }
 __global__ __launch_bounds__(256) void winattn_prep_kernel(const ps_seq_step *step, long long ring_off, int cap, long long store_off, int pool, int keep, const float *y,
                                                            long long ldy, const float *qnorm, const float *knorm, float eps, int H, int G, int d, int dv, int rot_dims,
                                                            int pairing, const float *freq, float *qo, long long ldq, float qt_coef, int qt_every, int head_norm,
@@ -50,8 +66,7 @@ __global__ __launch_bounds__(256) void winattn_prep_kernel(const ps_seq_step *st
     const int nq = H * d, nk = G * d, nv = G * dv, half = rot_dims / 2;
     const float *qt = y + (long long)t * ldy, *kt = qt + nq, *vt = kt + nk;
     float *ring = step->state + ring_off + (pos % cap) * (long long)(nk + nv);
-    // a query temperature that grows with the position in steps of qt_every tokens: 1 + coef ln(floor((pos + 1) / every) + 1)
-    const float qtemp = qt_every > 0 ? 1.f + qt_coef * logf((float)((pos + 1) / qt_every) + 1.f) : 1.f;
+    const float qtemp = wa_qtemp(pos, qt_coef, qt_every);
     for (int i = tid; i < half; i += 256) {
         const float ang = (float)pos * freq[i];
         cs[i] = cosf(ang) * rot_mag;
@@ -66,20 +81,7 @@ __global__ __launch_bounds__(256) void winattn_prep_kernel(const ps_seq_step *st
     __syncthreads();
     const float ia = qnorm && !head_norm ? 1.f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)nq + eps) : 1.f;
     const float ib = knorm && !head_norm ? 1.f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)nk + eps) : 1.f;
-    // element i of a projection (c = its index in its head): normed, and where c < rot_dims turned together with its partner; wc: 1 = one weight vector of d
-    // numbers for every head (indexed by c), 0 = a weight per element of the projection
-    auto turned = [&](const float *src, const float *w, float inv, int i, int wc) {
-        const int c = i % d;
-        if (w && wc) w += c - i;
-        const float self = src[i] * inv * (w ? w[i] : 1.f);
-        if (c >= 2 * half) return self;
-        int partner, pair;
-        bool first;
-        if (pairing == PS_ROT_NEIGHBOURS) { partner = i - c + (c ^ 1); pair = c >> 1; first = !(c & 1); }
-        else { first = c < half; partner = first ? i + half : i - half; pair = first ? c : c - half; }
-        const float other = src[partner] * inv * (w ? w[partner] : 1.f);
-        return first ? self * cs[pair] - other * cs[half + pair] : self * cs[pair] + other * cs[half + pair];
-    };
+    auto turned = [&](const float *src, const float *w, float inv, int i, int wc) { return wa_turned(src, w, inv, i, wc, d, half, pairing, cs); };
     // the block of a single token: its sum so far (nothing before the block's first position), the mean once the block is complete
     const bool own_pool = pool > 0 && gridDim.x == 1;
     const long long pb = own_pool ? pos / pool : 0;
@@ -326,22 +328,67 @@ void psk_winattn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off,
 // A single token.  Rows = the heads that share key / value group g (16 per block); the keys are cut into tiles of 16 in one index space -- tiles
 // 0 .. nbt - 1 the visible front rows, then the window from its first position -- and wave w of block (x, head tile, g) takes tile 4 x + w.
 // Partials per (tile, head): [o[dv] unnormalised, m, l, -, -], merged by winattn_merge_kernel, where the sink and the gate come in.
-// dynamic LDS: 16 x (d + 4) + 4 x 16 x 17
-template <int NJ, bool DIST>
+// ROW (psk_winattn_row: no sum over a whole projection is wanted): the block makes its sixteen queries of the projections itself, and the block that has the token's own tile its key and value, which it appends
+// and reads back, with the block mean and the kept row: winattn_prep_kernel's launch, one of three, is not needed.  A token of Pupidra 2048 x 6 (two such layers)
+// 366 -> 362 us.
+// dynamic LDS: 16 x (d + 4) + 4 x 16 x 17, ROW: + rot_dims
+template <int NJ, bool DIST, bool ROW>
 __global__ __launch_bounds__(256) void winattn_step_kernel(const ps_seq_step *step, long long ring_off, int cap, long long store_off, int pool, int keep, const float *q,
                                                            const float *temp, int H, int G, int d, int dv, int window, float scale, float *part, float softcap,
-                                                           const float *slope) {
+                                                           const float *slope, psk_winattn_row row) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4, g = blockIdx.z, hpg = H / G, r0 = blockIdx.y * 16;
     const int qld = d + 4;
     float *qs = lds, *pt = lds + 16 * qld + wave * 16 * 17;
     const long long p = step->pos0, lo = p - window + 1 > 0 ? p - window + 1 : 0, nb = wa_front(p, window, pool, keep), nbt = (nb + 15) / 16;
     const long long tile = (long long)blockIdx.x * 4 + wave, ntiles = nbt + (p - lo) / 16 + 1;
-    // the group's 16 queries into LDS, each already times its head's temperature (the scores of a tile then share one scale)
-    for (int r = wave; r < 16; r += 4) {
-        const int hh = r0 + r, h = g * hpg + hh;
-        const float tp = hh < hpg && temp ? temp[h] : 1.f;
-        for (int c = lane; c < d; c += 64) qs[r * qld + c] = hh < hpg ? q[(long long)h * d + c] * tp : 0.f;
+    if constexpr (ROW) {
+        if ((long long)blockIdx.x * 4 >= ntiles) return; // (uniform)
+        float *cs = lds + 16 * qld + 4 * 16 * 17;
+        const int half = row.rot_dims / 2, nk = G * d;
+        for (int i = threadIdx.x; i < half; i += 256) {
+            const float ang = (float)p * row.freq[i];
+            cs[i] = cosf(ang) * row.rot_mag;
+            cs[half + i] = sinf(ang) * row.rot_mag;
+        }
+        __syncthreads();
+        const float qtemp = wa_qtemp(p, row.qt_coef, row.qt_every);
+        auto scale_of = [&](const float *x, int n, bool own) { // a head's own norm
+            float ss = 0.f;
+            if (own) for (int c = lane; c < n; c += 64) ss += x[c] * x[c];
+            return own ? 1.f / sqrtf(wa_wave_sum(ss) / (float)n + row.eps) : 1.f;
+        };
+        for (int r = wave; r < 16; r += 4) {
+            const int hh = r0 + r, h = g * hpg + hh;
+            const float tp = hh < hpg && temp ? temp[h] : 1.f, inv = hh < hpg ? scale_of(row.y + (long long)h * d, d, row.qnorm != nullptr) : 0.f;
+            for (int c = lane; c < d; c += 64) qs[r * qld + c] = hh < hpg ? wa_turned(row.y, row.qnorm, inv, h * d + c, 1, d, half, row.pairing, cs) * qtemp * tp : 0.f;
+        }
+        if (row.appends && (ntiles - 1) / 4 == blockIdx.x && wave < 2) { // (every block.y writes the same row, as it reads it; the first one the front store's)
+            const bool isk = wave == 0;
+            const int n = isk ? d : dv, e0 = g * n, at = isk ? 0 : nk;
+            const float *src = row.y + (long long)H * d + at, *w = isk ? row.knorm : nullptr;
+            const float inv = scale_of(src + e0, n, isk ? w != nullptr : row.v_unit != 0);
+            const long long rs = (long long)nk + (long long)G * dv, pb = pool > 0 ? p / pool : 0;
+            float *ring = step->state + ring_off + (p % cap) * rs + at, *mean = step->state + store_off + pb * rs + at, *kept = p < row.keep ? step->state + store_off + p * rs + at : nullptr;
+            for (int c = lane; c < n; c += 64) {
+                const int i = e0 + c;
+                const float v = isk ? wa_turned(src, w, inv, i, 1, d, half, row.pairing, cs) : src[i] * inv;
+                ring[i] = v;
+                if (blockIdx.y) continue;
+                if (kept) kept[i] = v;
+                if (pool > 0) {
+                    const float sum = (p == pb * pool ? 0.f : mean[i]) + v;
+                    mean[i] = p == pb * pool + pool - 1 ? sum / (float)pool : sum;
+                }
+            }
+        }
+    } else {
+        // the group's 16 queries into LDS, each already times its head's temperature (the scores of a tile then share one scale)
+        for (int r = wave; r < 16; r += 4) {
+            const int hh = r0 + r, h = g * hpg + hh;
+            const float tp = hh < hpg && temp ? temp[h] : 1.f;
+            for (int c = lane; c < d; c += 64) qs[r * qld + c] = hh < hpg ? q[(long long)h * d + c] * tp : 0.f;
+        }
     }
     __syncthreads();
     if (tile >= ntiles) return;
@@ -439,18 +486,18 @@ size_t psk_winattn_step_scratch(int H, int dv, int window, psk_front_store fs, i
 // q [H * d] -> o [H * dv]; gate [H] raw or NULL; scratch from psk_winattn_step_scratch
 void psk_winattn_step(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, psk_front_store fs, const float *q, const float *gate, const float *temp,
                       const float *sink, int H, int G, int d, int dv, int window, float scale, int64_t max_context, float *scratch, float *o, float softcap, int gate_elem,
-                      const float *slope) {
+                      const float *slope, const psk_winattn_row *row) {
     const int max_tiles = wa_max_tiles(window, fs, max_context);
-    const size_t lds = (size_t)(16 * (d + 4) + 4 * 16 * 17) * 4;
+    const size_t lds = (size_t)(16 * (d + 4) + 4 * 16 * 17 + (row ? row->rot_dims : 0)) * 4;
     static unsigned long long mask = 0;
     if (ps_first_on_device(&mask)) {
-        (void)hipFuncSetAttribute((const void *)winattn_step_kernel<8, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void *)winattn_step_kernel<8, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (auto k : {winattn_step_kernel<8, false, false>, winattn_step_kernel<8, true, false>, winattn_step_kernel<8, false, true>, winattn_step_kernel<8, true, true>})
+            (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     }
     const dim3 grid((max_tiles + 3) / 4, (H / G + 15) / 16, G);
-    const auto kernel = slope ? winattn_step_kernel<8, true> : winattn_step_kernel<8, false>;
+    const auto kernel = row ? (slope ? winattn_step_kernel<8, true, true> : winattn_step_kernel<8, false, true>) : slope ? winattn_step_kernel<8, true, false> : winattn_step_kernel<8, false, false>;
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, step, (long long)ring_off, cap, (long long)fs.off, fs.pool, fs.keep, q, temp, H, G, d, dv, window, scale, scratch,
-                       softcap, slope);
+                       softcap, slope, row ? *row : psk_winattn_row());
     hipLaunchKernelGGL(winattn_merge_kernel, dim3(H), dim3(256), grid.x * 4 <= WA_HELD ? (size_t)grid.x * 4 * 4 : 0, st, step, scratch, gate, sink, fs.pool, fs.keep, H, dv, window, (int)grid.x * 4, o,
                        gate_elem);
 }

@@ -771,14 +771,19 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 first_product(g);
             }
             const bool reads = P.owner >= 0; // (another layer's keys and values: queries only)
-            psk_winattn_prep(st, m->step, P.off_ring, P.cap, psk_front_store{P.off_pool, l.pool, reads ? 0 : P.keep_rows}, t1, ld1, l.qnorm, l.knorm, D.norm_eps, (int)H,
-                             reads ? 0 : (int)G, (int)d, (int)dv, l.rot_dims, l.rot_pairing, P.freq, T, m->t2, Hd, l.qtemp_coef, l.qtemp_every, l.head_norm, l.v_unit,
-                             P.rot_mag);
             const psk_front_store fs{P.off_pool, l.pool, l.keep_first};
             const float *gate = l.gated ? t1 + Hd + (reads ? 0 : G * d + G * dv) : nullptr;
             const int ge = l.gated == 2; // a gate per output element
             const bool mfma = (m->mode & 2) == 0 && (G * (d + dv)) % 4 == 0 && psk_winattn_mfma_ok((int)d, (int)dv);
-            if (mfma && split_attn(l, 0)) {
+            const bool splits = mfma && split_attn(l, 0), steps = !splits && mfma && T == 1 && m->win_scratch, itself = steps && (l.head_norm || (!l.qnorm && !l.knorm));
+            psk_winattn_row row;
+            row.y = t1; row.qnorm = l.qnorm; row.knorm = l.knorm; row.freq = P.freq; row.eps = D.norm_eps; row.qt_coef = l.qtemp_coef; row.rot_mag = P.rot_mag;
+            row.rot_dims = l.rot_dims; row.pairing = l.rot_pairing; row.qt_every = l.qtemp_every; row.v_unit = l.v_unit; row.appends = !reads; row.keep = reads ? 0 : P.keep_rows;
+            if (!itself)
+                psk_winattn_prep(st, m->step, P.off_ring, P.cap, psk_front_store{P.off_pool, l.pool, reads ? 0 : P.keep_rows}, t1, ld1, l.qnorm, l.knorm, D.norm_eps, (int)H,
+                                 reads ? 0 : (int)G, (int)d, (int)dv, l.rot_dims, l.rot_pairing, P.freq, T, m->t2, Hd, l.qtemp_coef, l.qtemp_every, l.head_norm, l.v_unit,
+                                 P.rot_mag);
+            if (splits) {
                 const int64_t past = std::min<int64_t>(pos0, l.window - 1), out = pos0 + T - l.window; // (positions in front of the last token's window)
                 psk_split_attn_args g;
                 g.G = (int)G; g.first = pos0 - past;
@@ -788,9 +793,9 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 g.q = m->t2; g.ldq = Hd;
                 g.softcap = l.softcap; g.temp = l.temp; g.slope = l.dist_slope; g.sink = l.sink; g.gate = gate; g.ldg = ld1; g.gate_elem = ge;
                 split_attn_run(l, g);
-            } else if (mfma && T == 1 && m->win_scratch)
+            } else if (steps)
                 psk_winattn_step(st, m->step, P.off_ring, P.cap, fs, m->t2, gate, l.temp, l.sink, (int)H, (int)G, (int)d, (int)dv, l.window, l.scale,
-                                 m->max_context, m->win_scratch, m->t3, l.softcap, ge, l.dist_slope);
+                                 m->max_context, m->win_scratch, m->t3, l.softcap, ge, l.dist_slope, itself ? &row : nullptr);
             else if (mfma)
                 psk_winattn_mfma(st, m->step, P.off_ring, P.cap, fs, m->t2, Hd, gate, ld1, l.temp, l.sink, (int)H, (int)G, (int)d, (int)dv, l.window, l.scale,
                                  T, m->t3, Hv, l.softcap, ge, l.dist_slope);

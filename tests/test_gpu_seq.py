@@ -97,6 +97,27 @@ def test_boundaries_of_a_portion(ctx, tmp_path, width, sizes):
         assert err(g, w[:first]) < TOL["float32"]
 
 
+# a single token's queries, key and value made inside its attention (k_winattn.hip winattn_step_kernel, ROW): groups of more than sixteen heads, whose blocks all append the row and of which one updates
+# the block means and the kept rows; a ring that wraps; a reader of another layer's keys and values; norms per head with queries that turn; means begun by a portion and finished by single tokens
+@pytest.mark.parametrize("which", ["pool", "keep", "head norms"])
+@pytest.mark.parametrize("sizes", [(1,), (1, 1, 7, 1, 1, 1, 1)])
+def test_a_token_that_appends_itself(ctx, tmp_path, which, sizes):
+    V = 40
+    if which == "pool":
+        at = {"heads": 36, "kv_heads": 2, "dim": 32, "vdim": 32, "mask": {"size": 5, "pool": 3}, "rot": {"base": 100.0, "dims": 16}, "scale": 0.2}
+        run, cfg = seq_oracle.run_parallel, synth.parallel_config(64, V, [synth.parallel_layer(None, at, {"heads": 1, "dim": 16, "vdim": 16, "tau": 4.0}, 1.0, 0.5)], taps=2)
+    elif which == "keep":
+        at = lambda size, keep, own=None: synth.pupidra_attention(34, 2, 32, 32, 1.0, size, keep, own)
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("attention", at(9, 20)), synth.pupidra_layer("attention", at(4, 7, 0))])
+    else:
+        run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(6, 2, 48, 32, 0.1, 5.0, (0.4, 7)), ff=64)])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=16, n_slots=1, max_context=100)
+    toks = tokens_for(cfg, 50)
+    assert err(run_portions(m, toks, sizes), run(cfg, t, toks)) < TOL["float32"]
+    m.close()
+
+
 # a single token's decay, its second product inside the scan (k_seqmix.hip sq_fold): ranks in whole eights and not, the longest there and the first with a launch of its own, in both formats; heads of few
 # rows and of many; the next token's neighbour, behind a portion and behind single tokens
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
