@@ -1513,7 +1513,6 @@ __global__ __launch_bounds__(FL_NT) void attn_flash16_kernel(psl_attn_args a) {
 }
 
 // ---------------------------------------------------------------- arg-max, first maximum (prob_array.cpp:65-67)
-constexpr int AM_PARTS = 64;
 __global__ __launch_bounds__(256) void argmax_partial_kernel(const float *src, int64_t n, float *pv, int *pi) {
     __shared__ float bv[4];
     __shared__ int bi[4];
@@ -1537,21 +1536,10 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const float *src, i
         pv[blockIdx.y * AM_PARTS + blockIdx.x] = best; pi[blockIdx.y * AM_PARTS + blockIdx.x] = idx;
     }
 }
-// one wave per row; optionally also performs the greedy-decode bookkeeping (feeds the id back as the next token)
-__global__ __launch_bounds__(64) void argmax_final_kernel(const float *pv, const int *pi, int32_t *out, ps_step_state *st,
-                                                          int32_t *token, int32_t *ids) {
-    const int lane = threadIdx.x;
-    float best = pv[blockIdx.x * AM_PARTS + lane]; int idx = pi[blockIdx.x * AM_PARTS + lane];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(idx, o, 64);
-        if (ov > best || (ov == best && oi < idx)) { best = ov; idx = oi; }
-    }
-    if (lane == 0) {
-        if (idx == 0x7fffffff) idx = 0; // a row of NaNs: std::max_element (prob_array.cpp:65-67) returns the first element
-        out[blockIdx.x] = idx;
-        if (st) { token[0] = idx; ids[st->n_out] = idx; st->n_out += 1; st->pos0 += 1; }
-    }
+// one wave per row
+__global__ __launch_bounds__(64) void argmax_final_kernel(const float *pv, const int *pi, int32_t *out) {
+    const int idx = ps_argmax_join(pv + blockIdx.x * AM_PARTS, pi + blockIdx.x * AM_PARTS);
+    if (threadIdx.x == 0) out[blockIdx.x] = idx;
 }
 
 } // namespace
@@ -1751,8 +1739,10 @@ void psl_attn_decode1(hipStream_t st, int n_cu, const psl_attn_args &a, bool rop
     else hipLaunchKernelGGL(attn_decode1_kernel<1>, g, b, lds, st, a, ch, (int)rope);
 }
 
-void psl_argmax2(hipStream_t st, const float *src, int64_t n, int64_t rows, int32_t *out, float *part_v, int *part_i,
-                 ps_step_state *state, int32_t *token, int32_t *ids) {
+void psl_argmax_parts(hipStream_t st, const float *src, int64_t n, int64_t rows, float *part_v, int *part_i) {
     hipLaunchKernelGGL(argmax_partial_kernel, dim3(AM_PARTS, (unsigned)rows), dim3(256), 0, st, src, n, part_v, part_i);
-    hipLaunchKernelGGL(argmax_final_kernel, dim3((unsigned)rows), dim3(64), 0, st, part_v, part_i, out, state, token, ids);
+}
+void psl_argmax2(hipStream_t st, const float *src, int64_t n, int64_t rows, int32_t *out, float *part_v, int *part_i) {
+    psl_argmax_parts(st, src, n, rows, part_v, part_i);
+    hipLaunchKernelGGL(argmax_final_kernel, dim3((unsigned)rows), dim3(64), 0, st, part_v, part_i, out);
 }

@@ -47,7 +47,7 @@ struct ps_hip_model {
     std::vector<const float *> attn_norm, ffn_norm, bq, bk, bv;
     std::vector<const ps_weight *> wq, wk, wv, wo, wg, wu, wd;
     // arena
-    float *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *att = nullptr, *hb = nullptr, *g1 = nullptr, *u1 = nullptr;
+    float *x = nullptr, *x_next = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *att = nullptr, *hb = nullptr, *g1 = nullptr, *u1 = nullptr;
     unsigned *attn_sync = nullptr; // [2048] words: [31] the one-launch attention's rendezvous-timeout flag
     unsigned *attn_flag_host = nullptr; // pinned: [31] travels here behind every single-token forward (async copy on the stream)
     bool attn_unchecked = false;        // such a forward was enqueued and its flag has not been looked at yet
@@ -265,7 +265,8 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
     auto act_for = [&](int64_t K) { return ps_act_carve(m->act_mem, K, m->max_batch); };
     (void)act;
 
-    psl_get_rows(st, m->token_embd, m->tokens_dev, bs, m->x);
+    // (a greedy run's step: its token's row is in x_next already, the last step's next_token_kernel has put it there)
+    if (!advance) psl_get_rows(st, m->token_embd, m->tokens_dev, bs, m->x);
     psl_attn_args aa{};
     aa.n_heads = (int)f.n_heads; aa.n_kv_heads = (int)f.n_kv_heads; aa.head_size = (int)f.head_size; aa.n_ctx = (int)f.seq_len;
     aa.neox = (f.rope.mode & 2) ? 1 : 0; aa.n_dims = f.rope.n_dims; aa.state = m->state; aa.rope_table = m->rope_table;
@@ -298,6 +299,7 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
     aa.n_kv_hi = m->n_kv_host > 0 ? m->n_kv_host : m->n_kv_bound > 0 ? m->n_kv_bound : (int)f.seq_len;
 
     for (uint32_t L = 0; L < f.n_layers; L++) {
+        const float *const xin = advance && L == 0 ? m->x_next : m->x;
         ps_act a1 = act_for(dim);
         psk_gemv_args g{};
         g.n_w = 3;
@@ -305,7 +307,7 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         g.out[0] = m->q; g.out[1] = m->k; g.out[2] = m->v;
         g.ldo[0] = dim; g.ldo[1] = kvd; g.ldo[2] = kvd;
         if (m->qwen2) { g.bias[0] = m->bq[L]; g.bias[1] = m->bk[L]; g.bias[2] = m->bv[L]; }
-        g.pro = 1; g.pro_x = m->x; g.pro_norm_w = m->attn_norm[L]; g.pro_eps = f.norm_eps; // RMSNorm + quantize in the prologue
+        g.pro = 1; g.pro_x = xin; g.pro_norm_w = m->attn_norm[L]; g.pro_eps = f.norm_eps; // RMSNorm + quantize in the prologue
         aa.k_cache = m->k_cache[L]; aa.v_cache = m->v_cache[L];
         const bool kv16 = (m->mode & 8) && !m->k16.empty();
         aa.k16 = kv16 ? m->k16[L] : nullptr; aa.v16 = kv16 ? m->v16[L] : nullptr; aa.part = m->attn_part;
@@ -402,7 +404,7 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         }
 
         psk_gemv_args go{};
-        go.n_w = 1; go.w[0] = m->wo[L]; go.out[0] = m->x; go.ldo[0] = dim; go.residual = m->x;
+        go.n_w = 1; go.w[0] = m->wo[L]; go.out[0] = m->x; go.ldo[0] = dim; go.residual = xin;
         go.pro = 2; go.pro_x = m->att;
         if (att_quantized) { go.pro = 0; go.pro_x = nullptr; } // (the V.p kernel left `att` quantized in a1)
         ps_act a2 = act_for(hid);
@@ -445,7 +447,10 @@ static int enqueue_forward(ps_hip_model *m, int bs, bool lm_head, bool use_tree,
         gl.n_w = 1; gl.w[0] = ow; gl.out[0] = m->logits; gl.ldo[0] = f.vocab_size;
         gl.pro = 1; gl.pro_x = m->x; gl.pro_norm_w = m->output_norm; gl.pro_eps = f.norm_eps;
         if (mm(m, gl, a1, dim, bs)) return 2;
-        psl_argmax2(st, m->logits, f.vocab_size, bs, m->argmax_dev, m->am_v, m->am_i, advance ? m->state : nullptr, m->tokens_dev, m->ids_dev);
+        if (advance) {
+            psl_argmax_parts(st, m->logits, f.vocab_size, 1, m->am_v, m->am_i);
+            psl_next_token(st, m->am_v, m->am_i, m->argmax_dev, m->state, m->tokens_dev, m->ids_dev, m->token_embd, m->x_next);
+        } else psl_argmax2(st, m->logits, f.vocab_size, bs, m->argmax_dev, m->am_v, m->am_i);
     }
     PS_CHECK(c, hipGetLastError());
     return 0;
@@ -502,7 +507,7 @@ int ps_hip_model_create(ps_hip_ctx *c, const ps_model_desc *d, ps_hip_model **ou
 
     const size_t mb = (size_t)m->max_batch, dim = f.dim, kvd = f.kv_dim, hid = f.hidden_dim, nctx = f.seq_len;
     auto fail = [&]() { ps_hip_model_destroy(m); return 1; };
-    if (dmalloc(m, (void **)&m->x, mb * dim * 4) || dmalloc(m, (void **)&m->q, mb * dim * 4) ||
+    if (dmalloc(m, (void **)&m->x, mb * dim * 4) || dmalloc(m, (void **)&m->x_next, dim * 4) || dmalloc(m, (void **)&m->q, mb * dim * 4) ||
         dmalloc(m, (void **)&m->k, mb * kvd * 4) || dmalloc(m, (void **)&m->v, mb * kvd * 4) ||
         dmalloc(m, (void **)&m->att, mb * dim * 4) || dmalloc(m, (void **)&m->hb, mb * hid * 4) ||
         dmalloc(m, (void **)&m->g1, mb * hid * 4) || dmalloc(m, (void **)&m->u1, mb * hid * 4) ||
@@ -865,6 +870,7 @@ static int decode_greedy_impl(ps_hip_model *m, int32_t token, int steps, int32_t
     const ps_piece in = {m->tokens_dev, &token, 4};
     PS_CHECK(c, ps_put(c->stream, &in, 1));
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, c->stream, m->state, (int)m->position, 1, 0);
+    psl_get_rows(c->stream, m->token_embd, m->tokens_dev, 1, m->x_next); // (the steps behind the first find theirs there)
     int s = 0;
     // the captured step carries the position it was captured at as a prefetch hint (n_kv_lo): keep it a LOWER bound that
     // is not far behind (plan_outlived: a stale hint costs time, never results)

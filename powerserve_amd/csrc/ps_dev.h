@@ -274,3 +274,16 @@ __device__ __forceinline__ void ps_scale_min_k4(int is, uint32_t s0, uint32_t s1
         m  = (c >> 4) | ((b >> 6) << 4);
     }
 }
+// the best of a row's 64 partial maxima (the first one of equals), by one wave, to every lane; a row of NaNs: std::max_element (prob_array.cpp:65-67) returns the first element
+constexpr int AM_PARTS = 64;
+static __device__ __forceinline__ int ps_argmax_join(const float *pv, const int *pi) {
+    float best = pv[threadIdx.x & 63];
+    int idx = pi[threadIdx.x & 63];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const float ov = __shfl_xor(best, o, 64);
+        const int oi = __shfl_xor(idx, o, 64);
+        if (ov > best || (ov == best && oi < idx)) { best = ov; idx = oi; }
+    }
+    return idx == 0x7fffffff ? 0 : idx;
+}

@@ -68,10 +68,11 @@ void psl_attn_decode1(hipStream_t st, int n_cu, const psl_attn_args &a, bool rop
 // layer instead of five; false: not covered, the caller issues psk_gemv4 + psl_attn_decode2
 bool psk_qkv_attn(hipStream_t st, int n_cu, const psk_gemv_args &g, int64_t K, const psl_attn_args &a);
 size_t psl_attn_softmax_pv_lds(const psl_attn_args &a); // dynamic LDS bytes (grows with n_ctx)
-// two-stage arg-max (64 partials per row).  With state != NULL the final stage also does the greedy-decode
-// bookkeeping: token[0] = id, ids[state->n_out++] = id, state->pos0++.
-void psl_argmax2(hipStream_t st, const float *src, int64_t n, int64_t rows, int32_t *out, float *part_v, int *part_i,
-                 ps_step_state *state, int32_t *token, int32_t *ids);
+// two-stage arg-max (64 partials per row)
+void psl_argmax2(hipStream_t st, const float *src, int64_t n, int64_t rows, int32_t *out, float *part_v, int *part_i);
+// the first stage, and a greedy step's second one with what follows from it: out = token[0] = ids[state->n_out++] = the id, state->pos0++, and the id's row of the embedding -> x [w->K]
+void psl_argmax_parts(hipStream_t st, const float *src, int64_t n, int64_t rows, float *part_v, int *part_i);
+void psl_next_token(hipStream_t st, const float *part_v, const int *part_i, int32_t *out, ps_step_state *state, int32_t *token, int32_t *ids, const ps_weight *w, float *x);
 
 // host restatement of ggml_rope_cache_init for positions [0, n_pos) -> table[n_pos][ne0]
 void ps_rope_table_host(const ps_rope_params *rp, int64_t ne0, const int32_t *pos, int n_pos, float *table);
