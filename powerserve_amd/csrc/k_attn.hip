@@ -1345,23 +1345,29 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_pv_mfma_lds_kernel(psl_attn_a
     ps_f32x4 res = (t3[0] + t3[1]) + (t3[2] + t3[3]);
     const float *pr = a.scores + ((int64_t)i * a.n_heads + (int64_t)kvh * r2 + g) * a.n_ctx;
     const float *vl = a.v_cache + ((int64_t)kvh * hs + d0 + 4 * m) * a.n_ctx;
-    // leftovers: sumf += x[j] * y[j], in order.  Eight positions' operands are requested before the first one is used (clamped addresses): one at
-    // a time every leftover was a memory round trip of its own, up to 31 in a row at the end of every launch
-    for (int j0 = np; j0 < n_kv; j0 += 8) {
-        float pj[8], vv[8][4];
+    // leftovers: sumf += x[j] * y[j], in order, up to 31 of them behind the blocks of 32.  The accumulators are through, so there are registers for all their operands: one trip to memory (rows are
+    // whole 16-byte pieces; what lies past the row's end repeats its last piece and is not used).  Eight positions at a time, a trip each, were 3 of the 17.7 us of 12 columns behind 700 positions.
+    if (np < n_kv) { // (uniform)
+        float4 pj[8], vv[8][4];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            const int jj = j0 + k < n_kv ? j0 + k : n_kv - 1;
-            pj[k] = pr[jj];
+            const int jj = min(np + 4 * k, a.n_ctx - 4);
+            pj[k] = *(const float4 *)(pr + jj);
 #pragma unroll
-            for (int r = 0; r < 4; r++) vv[k][r] = vl[(int64_t)r * a.n_ctx + jj];
+            for (int r = 0; r < 4; r++) vv[k][r] = *(const float4 *)(vl + (int64_t)r * a.n_ctx + jj);
         }
 #pragma unroll
-        for (int k = 0; k < 8; k++)
-            if (j0 + k < n_kv) {
+        for (int k = 0; k < 8; k++) {
+            if (np + 4 * k >= n_kv) break; // (uniform)
+            const float pe[4] = {pj[k].x, pj[k].y, pj[k].z, pj[k].w};
 #pragma unroll
-                for (int r = 0; r < 4; r++) res[r] = ps_dot_left(res[r], vv[k][r], pj[k], j0 + k - np, n_kv - np);
+            for (int r = 0; r < 4; r++) {
+                const float ve[4] = {vv[k][r].x, vv[k][r].y, vv[k][r].z, vv[k][r].w};
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (np + 4 * k + e < n_kv) res[r] = ps_dot_left(res[r], ve[e], pe[e], 4 * k + e, n_kv - np);
             }
+        }
     }
     if (bx * 16 + rl < N)
         *(float4 *)(a.att + (int64_t)i * dim + ((int64_t)kvh * r2 + g) * hs + d0 + 4 * m) = make_float4(res[0], res[1], res[2], res[3]);

@@ -632,6 +632,28 @@ def test_batches_with_a_large_context_window(ctx, oracle, tmp_path, preset, n_ct
     om.close()
 
 
+@pytest.mark.parametrize("preset,wt,n_ctx", [("small-llama-hs128", 8, 128), ("small-llama-hs128", 12, 124), ("small-llama", 2, 116), ("tiny-qwen2", 8, 100)])
+def test_batches_whose_positions_are_no_whole_blocks(ctx, oracle, tmp_path, preset, wt, n_ctx):
+    """the positions behind the blocks of 32 of a batch (attn_pv_mfma_lds_kernel): 9, 17, 25, 1, 10, 18, 31 and 4 of them, none, and the last slots of the
+    window; logits on bits"""
+    from oracle import binding as B
+    from powerserve_amd import hip, synth
+    d = str(tmp_path / "m")
+    mj = synth.write_model_dir(d, preset, wt, n_ctx=n_ctx, seed=5)
+    cfg = B.make_config(mj["llm_config"])
+    om = oracle.model(cfg, mj["model_arch"], load_tensors(os.path.join(d, "ggml/weights.gguf")), n_threads=4)
+    gm = hip.Model(ctx, d, max_batch=32)
+    toks = np.random.default_rng(n_ctx).integers(0, cfg.vocab_size, n_ctx)
+    at = (0, 9, 17, 25, 33, 42, 50, 63, 72, 100, n_ctx - 8 if n_ctx > 109 else n_ctx, n_ctx)
+    for lo, hi in zip(at, at[1:]):
+        if lo == hi: continue
+        want = om.forward(toks[lo:hi], np.arange(lo, hi), True)
+        got, _ = gm.forward(toks[lo:hi], np.arange(lo, hi), True)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (lo, rel_err(got, want))
+    gm.close()
+    om.close()
+
+
 @pytest.mark.parametrize("preset,wt,n_ctx", [("small-llama-hs128", 8, 96), ("small-llama-hs128", 12, 64), ("small-llama", 2, 96), ("tiny-qwen2", 8, 68)])
 def test_context_windows_shorter_than_one_attention_step(ctx, oracle, tmp_path, preset, wt, n_ctx):
     """n_ctx below 128 slots (not a multiple of 32 either): the batch V.p kernel stages 128 positions per step, and a lane whose segment lies past the
