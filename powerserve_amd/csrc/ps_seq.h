@@ -130,7 +130,8 @@ void psk_rmsnorm(hipStream_t st, const float *x, int64_t ldx, const int32_t *idx
                  int groups = 1);
 // x[r] += y[r] / sqrt(mean(y^2) + eps) * (offset + w)
 // (wn given: hn = norm(x) (offset + wn) behind it)
-// (copy16 of these and of psk_causal_conv, psk_headnorm_gate, psk_gate_partnorm: also the result -- x here -- rounded to bf16, rows side by side; returns whether that was done)
+// (copy16 of these and of psk_causal_conv, psk_headnorm_gate, psk_gate_partnorm: also the result -- x here -- rounded to bf16, rows side by side; returns whether that was done.  only16 with it: the fp32 result need not be
+// written, its one reader takes the rounded rows)
 bool psk_norm_residual(hipStream_t st, float *x, const float *y, const float *w, float offset, float eps, int64_t n, int rows, int groups = 1, const float *wn = nullptr,
                        float *hn = nullptr, uint16_t *copy16 = nullptr, float *xo = nullptr);
 // The front of a parallel layer that has no input filter, in one launch: x[r] = sum_j mix[j] X_j[row(r)] over the nmix streams X_j = src + j stride (mix NULL:
@@ -199,9 +200,9 @@ void psk_delta_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, 
 void psk_ssd_scan(hipStream_t st, const ps_seq_step *step, int64_t state_off, const float *x, const float *B, const float *C, int64_t ld, const float *dtraw, int64_t ldb,
                   const float *a_log, const float *dt_bias, const float *skip, int H, int G, int N, int P, int T, float *o, int64_t ldo);
 // o[t] = part_norm(o[t] * silu(z[t])) * w: the gate first, then each of `parts` equal stretches of n / parts divided by its own root mean square
-bool psk_gate_partnorm(hipStream_t st, float *o, int64_t ldo, const float *z, int64_t ldz, const float *w, int parts, float eps, int64_t n, int T, uint16_t *copy16 = nullptr);
+bool psk_gate_partnorm(hipStream_t st, float *o, int64_t ldo, const float *z, int64_t ldz, const float *w, int parts, float eps, int64_t n, int T, uint16_t *copy16 = nullptr, bool only16 = false);
 // o[t][h][:] = o / sqrt(mean_j o^2 + eps) * w(h, :) * silu(g[t][h][:]);  w_stride = dv (a weight per head) or 0 (one shared by the heads)
-bool psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, int64_t ldg, const float *w, int w_stride, float eps, int H, int dv, int T, uint16_t *copy16 = nullptr);
+bool psk_headnorm_gate(hipStream_t st, float *o, int64_t ldo, const float *g, int64_t ldg, const float *w, int w_stride, float eps, int H, int dv, int T, uint16_t *copy16 = nullptr, bool only16 = false);
 // Matrix memory with exponential gates.  q, k [T][H*d], v [T][H*dv] (row stride ld), iraw / fraw [T][H] (row stride ldb) the gates' pre-activations; state per head [dv + 1][d] fp32 at
 // step->state + state_off (a column's d numbers together; the last column is n, the memory of k alone), the running maximum [H] at step->state + m_off.
 //   i = c(iraw), f = ln sigmoid(c(fraw)), c(z) = cap tanh(z / cap);  m' = max(f + m, i);  S <- exp(f + m - m') S + exp(i - m') k v^T, n alike

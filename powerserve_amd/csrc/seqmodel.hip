@@ -643,6 +643,8 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
         g.w = w; g.a = a; g.lda = lda; g.T = T; g.out = out; g.ldo = ldo; g.small_f32 = 1; g.force_tiled = tiled; g.pack = m->pack; g.pack_bytes = m->pack_bytes; g.split = m->split; g.split_bytes = m->split_bytes;
         return g;
     };
+    // a product that takes the rounded rows of its input [T][lda] and does not read the others
+    auto takes16 = [&](const ps_dense *w, int64_t lda) { return copy16 && w && w->K == lda && psk_dense_wide16(mm(w, nullptr, lda, nullptr, w->N)); };
     // a sublayer boundary: x += norm_b(y) (after a sublayer), then hn = norm(x), h = conv(hn) (in front of the next one); one launch for a single token
     bool final_made = false, sequential = m->groups == 1 && !m->hist; // (of nothing but sequential layers, m->hn has no other reader: the residual stream of several rows stands there for some layers)
     for (auto &P : m->L) sequential = sequential && P.d.form == PS_LAYER_SEQUENTIAL;
@@ -711,7 +713,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             psk_dense_pre r;
             r.kind = psk_dense_pre::HEADS; r.gate = gate; r.w = w; r.w_stride = w_stride; r.part = (int)n; r.eps = D.norm_eps;
             if (T == 1 && out_proj(o, H * n, &r)) return;
-            rounded = psk_headnorm_gate(st, o, H * n, gate, ldg, w, w_stride, D.norm_eps, (int)H, (int)n, T, copy16) ? o : nullptr;
+            rounded = psk_headnorm_gate(st, o, H * n, gate, ldg, w, w_stride, D.norm_eps, (int)H, (int)n, T, copy16, takes16(l.out, H * n)) ? o : nullptr;
             out_proj(o, H * n);
         };
         if (l.kind == PS_MIX_WKV) {
@@ -813,7 +815,7 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 psk_ssd_chunked(st, m->step, P.off_S, x, Bv, Cv, P.cqkv, dt, ld1, l.a_log, l.dt_bias, l.skip, (int)H, l.kv_heads, (int)d, (int)dv, T, m->ssd_scratch, m->t3, inner);
             else
                 psk_ssd_scan(st, m->step, P.off_S, x, Bv, Cv, P.cqkv, dt, ld1, l.a_log, l.dt_bias, l.skip, (int)H, l.kv_heads, (int)d, (int)dv, T, m->t3, inner);
-            rounded = psk_gate_partnorm(st, m->t3, inner, t1, ld1, l.onorm, l.norm_parts, D.norm_eps, inner, T, copy16) ? m->t3 : nullptr;
+            rounded = psk_gate_partnorm(st, m->t3, inner, t1, ld1, l.onorm, l.norm_parts, D.norm_eps, inner, T, copy16, takes16(l.out, inner)) ? m->t3 : nullptr;
             out_proj(m->t3, inner);
         } else if (l.kind == PS_MIX_MLSTM) {
             // t1 = [ q | k | v | g | i | f ] (+ bias); the memory -> t3, its products with n and running maxima -> lstm_aux; denominator, head norm and gate; out

@@ -97,6 +97,19 @@ def test_boundaries_of_a_portion(ctx, tmp_path, width, sizes):
         assert err(g, w[:first]) < TOL["float32"]
 
 
+# the gated part norms of several rows (k_seqmix.hip sq_gate_partnorm_rows_kernel): parts of one run of four numbers, that end inside a wave's first, second and third run, of its last ones; of more and of
+# no whole fours (the other form), as are 8 rows and fewer; in bfloat16 with an inner size whose rounded rows alone are written and one whose product reads the others
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,dim,parts", [(8, 4, 8), (4, 64, 1), (5, 52, 1), (16, 32, 1), (33, 16, 1), (16, 64, 1), (17, 64, 1), (18, 9, 3), (16, 64, 8)])
+def test_part_norms_of_several_rows(ctx, tmp_path, heads, dim, parts, dtype):
+    cfg = synth.pupidra_config(64, 40, [synth.pupidra_layer("mamba2", synth.pupidra_mamba2(heads, dim, 16, 1, 4, parts))])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype, max_batch=40, n_slots=1)
+    toks = tokens_for(cfg, 60)
+    assert err(run_portions(m, toks, (9, 8, 33, 10)), seq_oracle.run_pupidra(cfg, t, toks)) < TOL[dtype]
+    m.close()
+
+
 # a single token's queries, key and value made inside its attention (k_winattn.hip winattn_step_kernel, ROW): groups of more than sixteen heads, whose blocks all append the row and of which one updates
 # the block means and the kept rows; a ring that wraps; a reader of another layer's keys and values; norms per head with queries that turn; means begun by a portion and finished by single tokens
 @pytest.mark.parametrize("which", ["pool", "keep", "head norms"])
