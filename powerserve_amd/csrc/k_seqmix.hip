@@ -716,14 +716,15 @@ __global__ __launch_bounds__(256) void sq_decay_scan_kernel(const ps_seq_step *s
                 if (in) {
                     const long long wi = (hb + i) * fold.rank;
                     float c = 0.f;
+                    auto a_of = [&](const int u) { return fold.bf16 ? __uint_as_float((unsigned)sq_bf16(fold.a[u]) << 16) : fold.a[u]; }; // (rounded as the product of a portion rounds it)
                     if (fold.eights) { // (uniform)
                         for (int u = 0; u < fold.rank; u += 8) {
                             const sq_us4 w0 = *(const sq_us4 *)((const unsigned short *)fold.w + wi + u), w1 = *(const sq_us4 *)((const unsigned short *)fold.w + wi + u + 4);
 #pragma unroll
-                            for (int x = 0; x < 8; x++) c = fmaf(__uint_as_float((unsigned)(x < 4 ? w0[x] : w1[x - 4]) << 16), fold.a[u + x], c);
+                            for (int x = 0; x < 8; x++) c = fmaf(__uint_as_float((unsigned)(x < 4 ? w0[x] : w1[x - 4]) << 16), a_of(u + x), c);
                         }
                     } else {
-                        for (int u = 0; u < fold.rank; u++) c = fmaf(fold.bf16 ? __uint_as_float((unsigned)((const unsigned short *)fold.w)[wi + u] << 16) : ((const float *)fold.w)[wi + u], fold.a[u], c);
+                        for (int u = 0; u < fold.rank; u++) c = fmaf(fold.bf16 ? __uint_as_float((unsigned)((const unsigned short *)fold.w)[wi + u] << 16) : ((const float *)fold.w)[wi + u], a_of(u), c);
                     }
                     pc[e] = c + fold.bias[hb + i];
                 }

@@ -144,6 +144,26 @@ def test_decay_of_a_single_token(ctx, tmp_path, rank, dtype):
     m.close()
 
 
+# the same decay in bfloat16 is a portion's: the vector in front of its second product is rounded in both.  w = exp(-exp(1024 a - 1020)) of an a that rounds from 0.995 to 255 / 256 for every token: 0.37, and 0.7 of one
+# that is not rounded
+@pytest.mark.parametrize("rank", [1, 8])
+def test_decay_of_a_single_token_is_that_of_a_portion(ctx, tmp_path, rank):
+    cfg = synth.seq_config(64, 40, [L("wkv", None, heads=2, dim=24)], taps=2)
+    t = synth.seq_tensors(cfg, 3, rank)
+    m = "l0.mix."
+    t["embed"][:, 0] = 50.0  # a channel that is the same for every token, which the decay alone reads
+    t["l0.norm1"][0] = t[m + "mu.w"][0] = 0.0
+    t["l0.canon1"][0] = t["head"][:, 0] = 0.0
+    for n in "rkvg": t[m + n][:, 0] = 0.0
+    t[m + "w1"][:], t[m + "w2"][:], t[m + "w0"][:] = 0.0, 0.0, -1020.0
+    t[m + "w1"][0, 0], t[m + "w2"][:, 0] = 0.38, 1024.0
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 3, t)
+    model = seqmodel.load_model(ctx, str(tmp_path), dtype="bfloat16", max_batch=16, n_slots=1)
+    toks = tokens_for(cfg, 12)
+    assert err(run_portions(model, toks, (1,)), run_portions(model, toks, (12,))) < 0.02
+    model.close()
+
+
 # wkv and delta rule in chunks of 16 tokens (k_chunk.hip): portions that end inside, on and one behind a chunk's edge, fewer than 32 tokens between them (the scan), state row tiles that
 # do not fill the four waves and more than they are, value columns that are no multiple of 16; decays from e^-20 a token to none at all
 @pytest.mark.parametrize("sizes", [(31, 33), (32,), (47, 5, 49), (64, 17), (100,)])
