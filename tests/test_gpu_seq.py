@@ -505,8 +505,9 @@ def test_attention_of_many_rows(ctx, tmp_path, which):
     assert err(got, want) < min(TOL["float32"], 2 * err(plain, want) + 2e-6)
 
 
-# the same with rows whose keys several work-groups share (k_splitattn.hip split_join_kernel): parts in which some rows, or all, see no key; kept first tokens and means of blocks in parts of their own;
-# queries turned beforehand, in rows that no 16-byte load fits (81 gates behind them); the last rows of a tile missing; sinks, gates, a soft cap and slopes behind the sum
+# the same with rows whose keys several work-groups share (k_splitattn.hip split_join_kernel; two parts, in the second portion): parts in which some rows, or all, see no key; kept first tokens and means of
+# blocks in parts of their own; the last rows of a tile missing; sinks, gates, a soft cap and slopes behind the sum.  "latent odd": whole tiles, queries turned beforehand, in rows that no 16-byte load
+# fits (81 gates behind them)
 @pytest.mark.parametrize("which", ["latent", "latent odd", "keep", "pool", "softcap"])
 def test_attention_of_many_rows_in_parts(ctx, tmp_path, which):
     V, sizes = 40, (260, 140)
@@ -525,6 +526,25 @@ def test_attention_of_many_rows_in_parts(ctx, tmp_path, which):
         run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(64, 8, 128, 128, 0.1, 5.0, (0.4, 7)), ff=64)])
     t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
     m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=100, n_slots=1, max_context=500)
+    toks = tokens_for(cfg, sum(sizes))
+    want, got = run(cfg, t, toks), run_portions(m, toks, sizes)
+    m.set_mode(2)  # the plain kernels
+    plain = run_portions(m, toks, sizes)
+    m.close()
+    assert err(got, want) < min(TOL["float32"], 2 * err(plain, want) + 2e-6)
+
+
+# tiles of one, two and three parts in one launch (260 tokens of 41 heads: 4, 8 and 9 blocks), then two of three parts each (the launches: test_host_calls.py); queries turned beforehand in rows that no
+# 16-byte load fits (41 gates behind them), a soft cap and gates
+@pytest.mark.parametrize("which", ["latent odd", "softcap"])
+def test_attention_of_tiles_in_one_to_three_parts(ctx, tmp_path, which):
+    V, sizes = 40, (260, 200)
+    if which == "latent odd":
+        run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("latent_attention", synth.pupidra_latent(41, 96, 32, 128, 32, 0.1, 1e4))])
+    else:
+        run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(41, 1, 128, 128, 0.1, 5.0, (0.4, 7)), ff=64)])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=260, n_slots=1, max_context=500)
     toks = tokens_for(cfg, sum(sizes))
     want, got = run(cfg, t, toks), run_portions(m, toks, sizes)
     m.set_mode(2)  # the plain kernels

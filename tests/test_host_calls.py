@@ -271,6 +271,27 @@ for sizes in ((129, 64), (400, 64), (1024, 128)): assert joined(*sizes) == 0, si
 """.replace(".dir", str(child.tmp / "dir")))
 
 
+def test_tiles_of_several_parts_are_joined(child):
+    """k_splitattn.hip sa_plan_of: the portions whose results tests/test_gpu_seq.py compares -- 41 heads in parts in both portions, 81 in whole tiles"""
+    child("""
+ctx = hip.Ctx(0)
+def joined(cfg):
+    synth.write_seq_model_dir(".dir", cfg, 1)
+    m = seqmodel.SeqModel(ctx, ".dir", dtype="float32", max_batch=260, n_slots=1, max_context=500)
+    s, n = m.acquire(), []
+    for T in (260, 200):
+        fake.fake_reset()
+        m.forward(s, [1] * T)
+        n.append((count("split_attn_kernel"), count("split_join_kernel")))
+    m.close()
+    return n
+latent = lambda heads: synth.pupidra_config(64, 30, [synth.pupidra_layer("latent_attention", synth.pupidra_latent(heads, 96, 32, 128, 32, 0.1, 1e4))])
+assert joined(latent(41)) == [(1, 1), (1, 1)]
+assert joined(latent(81)) == [(1, 0), (1, 0)]
+assert joined(synth.zusolix_config(64, 30, [synth.zusolix_layer("attention", synth.zusolix_attention(41, 1, 128, 128, 0.1, 5.0, (0.4, 7)), ff=64)])) == [(1, 1), (1, 1)]
+""".replace(".dir", str(child.tmp / "dir")))
+
+
 def test_the_measured_products_of_experts_are_the_ones_that_run(child):
     """ps_hip_seq_bench_kernel: a portion's second product of the experts reads the rounded rows of the first one, in a step and where it is measured"""
     child("""
