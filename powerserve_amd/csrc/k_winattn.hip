@@ -35,10 +35,6 @@ static __device__ __forceinline__ long long wa_front(long long p, int window, in
     return pool > 0 ? n / pool : (n < keep ? n : keep);
 }
 
-// y[t] = [ q (H d) | k (G d) | v (G dv) | ... ].  q -> qo[t] normed and rotated; k (normed, rotated) and v -> ring row pos mod cap: [G d | G dv],
-// and one of the first `keep` tokens' rows into the front store too (store_off).
-// A step of ONE token also brings its block's sum up to date here (the thread that wrote a channel adds it: the same sum, in the same order, as
-// winattn_pool_kernel makes for a portion).  dynamic LDS: rot_dims floats (cos | sin of the token's angles, shared by all heads).
 // element i of a projection (c = its index in its head of d): normed, and where c < 2 half turned together with its partner (cs: half cosines, half sines); wc: 1 = one weight vector of d
 // numbers for every head (indexed by c), 0 = a weight per element of the projection
 static __device__ __forceinline__ float wa_turned(const float *src, const float *w, float inv, int i, int wc, int d, int half, int pairing, const float *cs) {
@@ -55,6 +51,10 @@ static __device__ __forceinline__ float wa_turned(const float *src, const float 
 }
 // a query temperature that grows with the position in steps of `every` tokens: 1 + coef ln(floor((pos + 1) / every) + 1)
 static __device__ __forceinline__ float wa_qtemp(long long pos, float coef, int every) { return every > 0 ? 1.f + coef * logf((float)((pos + 1) / every) + 1.f) : 1.f; }
+// y[t] = [ q (H d) | k (G d) | v (G dv) | ... ].  q -> qo[t] normed and rotated; k (normed, rotated) and v -> ring row pos mod cap: [G d | G dv],
+// and one of the first `keep` tokens' rows into the front store too (store_off).
+// A step of ONE token also brings its block's sum up to date here (the thread that wrote a channel adds it: the same sum, in the same order, as
+// winattn_pool_kernel makes for a portion).  dynamic LDS: rot_dims floats (cos | sin of the token's angles, shared by all heads).
 __global__ __launch_bounds__(256) void winattn_prep_kernel(const ps_seq_step *step, long long ring_off, int cap, long long store_off, int pool, int keep, const float *y,
                                                            long long ldy, const float *qnorm, const float *knorm, float eps, int H, int G, int d, int dv, int rot_dims,
                                                            int pairing, const float *freq, float *qo, long long ldq, float qt_coef, int qt_every, int head_norm,

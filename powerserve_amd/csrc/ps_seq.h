@@ -342,14 +342,14 @@ bool psk_winattn_mfma_ok(int d, int dv);
 void psk_winattn_mfma(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, psk_front_store fs, const float *q, int64_t ldq, const float *gate,
                       int64_t ldg, const float *temp, const float *sink, int H, int G, int d, int dv, int window, float scale, int T, float *o, int64_t ldo,
                       float softcap = 0.f, int gate_elem = 0, const float *slope = nullptr);
-// A single token on the matrix cores: rows = the heads of a key / value group, the keys spread over waves, partials merged in a second launch (same sizes).
-size_t psk_winattn_step_scratch(int H, int dv, int window, psk_front_store fs, int64_t max_context);
-// row (psk_winattn_prep's token, without norms over whole projections: none, or those of every head): the step makes the queries and appends the token itself, q is not read
+// (psk_winattn_step) psk_winattn_prep's token, without norms over whole projections -- none, or those of every head: the step makes the queries and appends the token itself, q is not read
 struct psk_winattn_row {
     const float *y = nullptr, *qnorm = nullptr, *knorm = nullptr, *freq = nullptr;
     float eps = 0.f, qt_coef = 0.f, rot_mag = 1.f;
     int rot_dims = 0, pairing = 0, qt_every = 0, v_unit = 0, appends = 0, keep = 0; // appends 0: another layer's keys and values; keep: kept rows of the store
 };
+// A single token on the matrix cores: rows = the heads of a key / value group, the keys spread over waves, partials merged in a second launch (same sizes).
+size_t psk_winattn_step_scratch(int H, int dv, int window, psk_front_store fs, int64_t max_context);
 void psk_winattn_step(hipStream_t st, const ps_seq_step *step, int64_t ring_off, int cap, psk_front_store fs, const float *q, const float *gate, const float *temp,
                       const float *sink, int H, int G, int d, int dv, int window, float scale, int64_t max_context, float *scratch, float *o, float softcap = 0.f,
                       int gate_elem = 0, const float *slope = nullptr, const psk_winattn_row *row = nullptr);
