@@ -631,7 +631,7 @@ static __device__ __forceinline__ bool dn_ring_rows(const dn_args &g, int tm, in
 
 // The tile and split of a work-group.  Work-group b runs on XCD b % 8: an XCD has an eighth of the items there are, neighbours in the order of panels of four output tiles, so its L2 sees few token
 // rows and few weights at a time, and no XCD has a column more than another.  With whole columns of tiles per XCD 1500 x 10304 of K = 2048 (41 columns of six tiles: 36 for one XCD, 30 for others) took
-// two rounds, 97 us; 67 so.  Whole requests: pupidra-prompt 3 406 -> 3 245 us, ranutar-f32-prompt 963 -> 919, ranutar-prompt 2 875 -> 2 812, ranutar-prompt-ragged 859 -> 847.
+// two rounds, 97 us; 67 so.
 #define DN_PANEL 4
 template <int BM>
 static __device__ __forceinline__ bool dn_ring_place(const dn_args &g, const dn_ring &p, int &tm, int &tn, int &s) {
@@ -1080,13 +1080,16 @@ __global__ __launch_bounds__(512) void dense_mm_big_kernel(dn_args g, dn_ring p)
     }
 }
 static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.act != PSD_ACT_RELU_PAIR && !g.em_table && (g.N % 4 || g.ldo % 4 || ((uintptr_t)g.out & 15)); }
-// Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices).  bf16 and three lines: the least of an estimate in us, rounds of 256 work-groups times (blocks of K times what a block
-// of the shape costs, its start, what the epilogue adds behind a tile: dn_epilogue), and for a split product its second launch and its parts' way through memory.  Fitted to 2 600 products (9 to 2 047
-// tokens, N 1 024 .. 24 576, K 1 536 .. 14 336, every shape, up to twelve splits; plain results): what it picks takes 0.9 % longer than the best of all on average (three lines 0.7 %), 15 % at most; the rule
-// before, without the 192 rows and the 128 and 192 x 256 tiles, 5.3 % and 6.3 % on average, up to 33 %.  Us there and here: 1 090 x 6 208 x 4 096 93 and 72, 954 x 8 192 x 6 144 136 and 102,
-// 389 x 16 384 x 2 048 54 and 44, 1 477 x 6 144 x 8 192 179 and 151, in three lines 273 x 10 304 x 4 096 125 and 108, 617 x 14 336 x 4 096 300 and 267.
-//   A block costs the bytes it fetches: a CU has about 16 KB of requests outstanding, which the mean way to L2 and beyond (a fifth to a third of the rows are not there yet) makes 60 bytes a ns, whatever
-// the shape -- 32 KB in 0.5 us of 128 x 128, 64 KB in 1.05 of 256 x 256.  So larger tiles do more per byte, and a height that leaves no round nearly empty counts as much.
+// Tile and splits of a product of `rows` tokens (grouped: slots of `groups` matrices).  bf16 and three lines: the least of an estimate in us of what a shape makes of a product -- not of its time, which has more
+// in it that all shapes have in common (the launch, packing, the results and what of the weights is not there yet: 2.6 us and up in bf16, 6 in three lines): rounds of 256 work-groups times (blocks of K times what a
+// block of the shape costs, its start, what the epilogue adds behind a tile: dn_epilogue), and for a split product its second launch and its parts' way through memory.  64 x 64 stands twice on a CU: two of them
+// hide each other's waits, one alone does not.  Fitted to 1 200 products of models (six families at widths 2 048 and 4 096, 2 to 2 047 tokens, K 512 .. 14 336, experts, epilogues; ten shapes and splits each,
+// timed where they stand in a portion), to 1 240 alone (N 1 024 .. 24 576, K from 512, weights from memory) and to 260 of K 64 .. 384.  What it picks, against the best of all, on average, and the rule before (one
+// cost of 64 x 64, no more for few blocks; fitted from 9 tokens and K of 1 536 on): in models bf16 1.0 % and 1.2 % of their time, three lines 0.4 % and 1.8 % (2 to 64 tokens 0.8 % and 4.4 %); on 480 that it was not
+// fitted to bf16 0.7 % and 0.7 %, three lines 0.4 % and 0.8 %; K 64 .. 384 in bf16 0.6 % and 11 %.  Us there and here, alone: 300 x 2 048 x 4 096 20.9 and 18.0, 620 x 1 024 x 4 096 20.7 and 17.8, 300 x 512 x 64 7.4
+// and 4.3; in three lines 2 x 4 096 x 4 096 22.7 and 20.1, 8 x 8 192 x 2 048 22.7 and 20.0, 190 x 5 120 x 2 560 38.8 and 32.8.
+//   A block costs the bytes it fetches: a CU has about 16 KB of requests outstanding, which the mean way to L2 and beyond makes some 60 bytes a ns, whatever the shape -- 32 KB in 0.5 us of 128 x 128, start
+// included, 64 KB in 1.0 of 256 x 256.  So larger tiles do more per byte, and a height that leaves no round nearly empty counts as much.
 //   Experts' rows: an expert has rows / groups on average, spread as a random routing and some more; the expected number of its tiles.
 // The fp32 instruction (dn_ring_plan_f32): a block of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more.
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
@@ -1129,22 +1132,25 @@ static dn_ring_shape dn_ring_plan_f32(int rows, int64_t N, int64_t kbytes, int g
     return best;
 }
 static dn_ring_shape dn_ring_plan(int rows, int64_t N, int64_t kbytes, int lines, int groups, bool may_split, bool big, int epilogue) {
-    struct shape { int BM, BN; double block[2], round[2]; }; // (bf16, three lines; us)
-    static const shape shapes[7] = {{256, 256, {1.046, 3.651}, {0.05, 2.05}}, {192, 256, {0.882, 3.514}, {0.07, 0.05}}, {128, 256, {0.719, 2.875}, {0.05, 0.05}}, {192, 128, {0.512, 1.842}, {2.96, 0.05}},
-                                    {128, 128, {0.388, 1.368}, {2.25, 0.12}}, {64, 128, {0.275, 0.83}, {1.76, 0.34}}, {64, 64, {0.167, 0.508}, {0.91, 0.05}}};
-    static const double behind[2][3] = {{0, 0.9, 5.1}, {0, 1.85, 6.85}}; // by 128 x 128 numbers; of tiles of 128 columns and less, of 256
-    static const double sums[2] = {2.8, 1.1}, parts[2] = {0.21, 0.30}; // a split product: once, by MB
+    struct shape { int BM, BN; double block[2], round[2]; }; // (bf16, three lines: a block of 128 x 256 there is 3.2, two of 128 x 128 are 2.9.  64 x 64: of two work-groups of a CU, each)
+    static const shape shapes[7] = {{256, 256, {1.010, 4.085}, {0.09, 1.65}}, {192, 256, {0.892, 3.571}, {0, 0.12}}, {128, 256, {0.774, 0}, {0.05, 0}}, {192, 128, {0.518, 1.960}, {2.72, 0}},
+                                    {128, 128, {0.383, 1.431}, {2.27, 0}}, {64, 128, {0.285, 0.843}, {1.54, 0.37}}, {64, 64, {0.169, 0.543}, {0.87, 0.11}}};
+    static const double alone[2] = {0.191, 0.596};                        // 64 x 64 without a second work-group on the CU
+    static const double behind[2][3] = {{0, 0.95, 5.2}, {0, 2.0, 6.25}};  // by 128 x 128 numbers; of tiles of 128 columns and less, of 256
+    static const double sums[2] = {2.48, 1.60}, parts[2] = {0.194, 0.289}; // a split product: once, by MB
+    static const double few = 4;                                          // what fewer than eight blocks of K don't hide of the start of 256 columns, at none; bf16
     const int64_t blocks = kbytes / 128;
     const int l = lines == 3;
     dn_ring_shape best{};
     double least = 0;
     for (auto &q : shapes) {
-        if (q.BN == DN_BIG && !big) continue;
+        if (q.BN == DN_BIG && (!big || q.block[l] == 0)) continue;
         const int n_tm = dn_row_tiles(rows, q.BM, groups), tn = (int)((N + q.BN - 1) / q.BN);
-        const double area = q.BM * q.BN / 16384.0, tiles = dn_mean_row_tiles(rows, q.BM, groups) * tn;
+        const double area = q.BM * q.BN / 16384.0, tiles = dn_mean_row_tiles(rows, q.BM, groups) * tn, start = q.round[l] + (l == 0 && q.BN == DN_BIG && blocks < 8 ? few * (8 - blocks) / 8 : 0);
         for (int64_t S = 1; S <= (may_split && q.BN < DN_BIG ? 16 : 1); S++) {
             if (S > 1 && (blocks / S < 4 || tiles * S > 700 || (size_t)n_tm * tn * S * q.BM * q.BN * 4 > psk_dense_split_bytes())) break;
-            const double t = std::ceil(tiles * S / 256) * ((double)((blocks + S - 1) / S) * q.block[l] + q.round[l] + (S == 1 ? behind[q.BN == DN_BIG][epilogue] * area : 0)) +
+            const double rounds = std::ceil(tiles * S / 256), single = q.BN == 64 ? std::fmod(rounds, 2) : 0, starts = q.BN == 64 ? (rounds + single) / 2 : rounds; // (two work-groups start together)
+            const double t = (double)((blocks + S - 1) / S) * ((rounds - single) * q.block[l] + single * alone[l]) + starts * start + (S == 1 ? rounds * behind[q.BN == DN_BIG][epilogue] * area : 0) +
                              (S > 1 ? sums[l] + parts[l] * tiles * S * area * 0.0655 : 0);
             if (!best.BM || t < least) { least = t; best = dn_ring_shape{q.BM, q.BN, n_tm, tn, (int)S}; }
         }
@@ -1209,8 +1215,9 @@ static bool dn_ring_take(hipStream_t st, const psk_dense_args &a, dn_args g) {
     }
     if (r.BN == DN_BIG) {
         if constexpr (sizeof(WT) == 2) {
-            if (r.BM == 128) dn_launch_big<false, PL, 2>(st, g, p);
-            else if (r.BM == 192) dn_launch_big<false, PL, 3>(st, g, p);
+            if (r.BM == 128) {
+                if constexpr (PL == 1) dn_launch_big<false, PL, 2>(st, g, p);
+            } else if (r.BM == 192) dn_launch_big<false, PL, 3>(st, g, p);
             else dn_launch_big<false, PL, 4>(st, g, p);
         }
     } else if (r.BM == 192) {

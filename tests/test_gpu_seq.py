@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import seq_oracle
+import wide_tiles
 from powerserve_amd import hip, host, seqmodel, synth
 from powerserve_amd.safetensors_io import f32_to_bf16_bits
 
@@ -285,7 +286,7 @@ def test_latent_attention_of_a_very_long_window(ctx, tmp_path, window):
 @pytest.mark.parametrize("dtype", list(FORMS))
 @pytest.mark.parametrize("T,N,K", [(9, 1, 64), (63, 127, 128), (64, 128, 192), (65, 129, 256), (127, 63, 320), (128, 65, 576), (129, 200, 64), (300, 130, 1088), (16, 8, 4096), (40, 100, 4160),
                                    (200, 256, 2240), (520, 2100, 128),
-                                   # dense_mm_big_kernel (bf16): one block of K, two, three and more than its stages; a row, a column and four columns more than a tile; no fours
+                                   # many tiles of few blocks of K (every form by its name: test_dense_matmul_of_every_tile)
                                    (2047, 2100, 64), (2049, 2305, 64), (1999, 3001, 192), (1030, 4100, 320), (1793, 2304, 128), (300, 20004, 64)])
 def test_dense_matmul_wide(ctx, dtype, T, N, K):
     import ctypes as C
@@ -438,8 +439,8 @@ def test_small_float32_products(made, ff, sizes):
     assert err(run_portions(m, toks, sizes), seq_oracle.run(c, t, toks)) < TOL["float32"]
 
 
-# 256 x 256 tiles behind an epilogue (k_dense.hip dense_mm_big_kernel): an activation whose rounded rows the second product reads, pairs, the four mixes of a token shift, the slots of experts (tiles
-# that end inside an expert, an expert without slots) with a factor per row
+# wide tiles behind an epilogue (by their names: test_every_tile_behind_an_epilogue): an activation whose rounded rows the second product reads, pairs, the four mixes of a token shift, the slots of
+# experts (tiles that end inside an expert, an expert without slots) with a factor per row
 @pytest.mark.parametrize("which", ["xielu", "pairs", "experts", "mixes"])
 def test_large_tiles_behind_an_epilogue(ctx, tmp_path, which):
     V = 30
@@ -460,6 +461,20 @@ def test_large_tiles_behind_an_epilogue(ctx, tmp_path, which):
     m.close()
     # both round the same numbers; their fp32 sums differ in order, so a rounding behind them may go the other way (2^-9 of a number, a few numbers of a row).  A row that is not its own: ~1
     assert err(got, plain) < 0.03
+
+
+# the same for the tiles of 256 columns at each of their heights, and for 192 x 128 whole and in parts (wide_tiles.py; which kernel runs: test_host_calls.py)
+@pytest.mark.parametrize("which,dtype,size,tokens,width", [(which, dtype, *case[:3]) for (which, dtype), cases in wide_tiles.EPILOGUES.items() for case in cases])
+def test_every_tile_behind_an_epilogue(ctx, tmp_path, which, dtype, size, tokens, width):
+    cfg = wide_tiles.layers(synth, which, size, width)
+    synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype, max_batch=tokens, n_slots=1, max_context=tokens + 100, f32_form=FORMS["float32 lines"] if dtype == "float32" else None)
+    toks = tokens_for(cfg, tokens)
+    got = run_portions(m, toks, (tokens,))
+    m.set_mode(2)  # the tiled mat-mul
+    plain = run_portions(m, toks, (tokens,))
+    m.close()
+    assert err(got, plain) < (0.03 if dtype == "bfloat16" else TOL["float32"])  # (bf16: as above)
 
 
 # xIELU behind a wide product (k_dense.hip dn_xielu): arguments from 2^-20 to beyond -64, where its exponent is held; rows of the first product scaled up and the second's columns down, so
@@ -608,12 +623,17 @@ def test_odd_rows_behind_an_epilogue(made, dtype, width, ff):
     assert err(run_portions(m, toks, [64, 11]), seq_oracle.run(cfg, t, toks)) < TOL[dtype]
 
 
-# tiles of 128 and 192 rows x 256 columns and of 192 x 128 (k_dense.hip dense_mm_big_kernel, dense_mm_ring_kernel; dn_ring_plan takes them here, in bfloat16 or in three lines): one block of K, two, an odd
-# and an even number; a row, a column and four columns more and less than a tile, no fours; split along K; columns of tiles that are no multiple of a panel or of the XCDs
+# few blocks of K: a row, a column and four columns more and less than a tile of 128 and 192 rows x 256 columns and of 192 x 128, no fours; columns of tiles that are no multiple of a panel or of the XCDs
 @pytest.mark.parametrize("dtype", list(FORMS))
 @pytest.mark.parametrize("T,N,K", [(1153, 6148, 64), (641, 8196, 64), (1345, 3076, 64), (640, 8192, 128), (385, 14340, 320), (1345, 6145, 192), (2047, 4100, 192), (1025, 8200, 192), (1537, 2049, 192),
                                    (1345, 3077, 256), (193, 14340, 64), (577, 2052, 2112), (1345, 3076, 1088), (961, 4101, 1088)])
 def test_dense_matmul_of_other_tile_heights(ctx, dtype, T, N, K):
+    test_dense_matmul_wide(ctx, dtype, T, N, K)
+
+
+# every tile of the wide mat-mul, whole and in parts of K (wide_tiles.py; which kernel runs: test_host_calls.py)
+@pytest.mark.parametrize("dtype,T,N,K", [(dtype, T, N, K) for (dtype, _, _), sizes in wide_tiles.PRODUCTS.items() for T, N, K, _ in sizes])
+def test_dense_matmul_of_every_tile(ctx, dtype, T, N, K):
     test_dense_matmul_wide(ctx, dtype, T, N, K)
 
 

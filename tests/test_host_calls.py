@@ -6,6 +6,7 @@ import sys
 
 import pytest
 
+import wide_tiles
 from powerserve_amd import hip
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -290,6 +291,47 @@ assert joined(latent(41)) == [(1, 1), (1, 1)]
 assert joined(latent(81)) == [(1, 0), (1, 0)]
 assert joined(synth.zusolix_config(64, 30, [synth.zusolix_layer("attention", synth.zusolix_attention(41, 1, 128, 128, 0.1, 5.0, (0.4, 7)), ff=64)])) == [(1, 1), (1, 1)]
 """.replace(".dir", str(child.tmp / "dir")))
+
+
+def test_the_tiles_of_wide_products(child):
+    """k_dense.hip dn_ring_plan: the tile and the parts of every product of wide_tiles.py, by the launch's name"""
+    products = [(fmt, T, N, K, wide_tiles.kernel(fmt, BM, BN, int(N % 4 != 0)), f"dense_mm_sum_kernelILi{BM}ELi{BN}E", S) for (fmt, BM, BN), sizes in wide_tiles.PRODUCTS.items() for T, N, K, S in sizes]
+    child("""
+ctx = hip.Ctx(0)
+bits = np.zeros(26 << 20, np.uint16)
+wrong = []
+for fmt, T, N, K, kernel, sums, S in PRODUCTS:
+    w = C.c_void_p()
+    form = hip.DENSE_BF16 if fmt == "bfloat16" else hip.DENSE_F32_LINES
+    x, o = hip.DevArray(ctx, (T, K), np.float32), hip.DevArray(ctx, (T, N), np.float32)
+    ctx.check(ctx.L.ps_hip_dense_upload(ctx.h, bits.ctypes.data_as(C.c_void_p), N, K, form, C.byref(w)))
+    fake.fake_reset()
+    ctx.check(ctx.L.ps_hip_dense_matmul(ctx.h, w, x.ptr, T, o.ptr, 1.0))
+    if (count(kernel), count(sums)) != (1, int(S > 1)): wrong.append((fmt, T, N, K, kernel, count(kernel), count(sums)))
+    ctx.L.ps_hip_dense_free(ctx.h, w)
+    x.free(); o.free()
+assert not wrong, "\\n".join(map(str, wrong))
+""".replace("PRODUCTS", repr(products)))
+
+
+def test_the_tiles_of_products_with_an_epilogue(child):
+    """the same of the models of wide_tiles.EPILOGUES: one launch of the named kernel in their portion"""
+    models = [(which, fmt, size, T, width, wide_tiles.kernel(fmt, BM, BN, 0), f"dense_mm_sum_kernelILi{BM}ELi{BN}E", S) for (which, fmt), cases in wide_tiles.EPILOGUES.items() for size, T, width, BM, BN, S in cases]
+    child("""
+sys.path.insert(0, TESTS)
+import wide_tiles
+ctx = hip.Ctx(0)
+wrong = []
+for which, fmt, size, T, width, kernel, sums, S in MODELS:
+    synth.write_seq_model_dir(".dir", wide_tiles.layers(synth, which, size, width), 1)
+    m = seqmodel.SeqModel(ctx, ".dir", dtype=fmt, max_batch=T, n_slots=1, max_context=T + 100, f32_form=hip.DENSE_F32_LINES if fmt == "float32" else None)
+    s = m.acquire()
+    fake.fake_reset()
+    m.forward(s, [1] * T)
+    if (count(kernel), count(sums)) != (1, S): wrong.append((which, fmt, size, T, width, kernel, count(kernel), count(sums)))
+    m.close()
+assert not wrong, "\\n".join(map(str, wrong))
+""".replace("TESTS", repr(HERE)).replace("MODELS", repr(models)).replace(".dir", str(child.tmp / "dir")))
 
 
 def test_the_measured_products_of_experts_are_the_ones_that_run(child):
