@@ -609,20 +609,43 @@ static __device__ __forceinline__ void dn_dma(const char *src, unsigned lds_dst)
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds_dst) : "memory");
 }
 
+static __device__ __forceinline__ int dn_wave_upto(int v) { // the sum of the lanes up to this one
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true); // one, two, four and eight lanes on in a row of sixteen, then a row's last lane to the next row and the second row's to the upper half
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+}
+// 64 matrices' slots at a time, a lane each (lanes behind the last matrix: none).  A loop over them one by one was a chain of loads in front of a work-group's first request, and two of them -- their number in
+// dn_ring_place, this tile's here -- were half of the time of many experts: four layers of 2 048 with 256 of them, two a token, 150 tokens 2 726 -> 1 528 us, 1 500 4 831 -> 3 309; 64 of them, 1 500 tokens
+// 1 935 -> 1 833.
+template <int BM>
+static __device__ __forceinline__ int dn_ring_slots(const dn_args &g, int base, int &at, int &next) { // tiles of this lane's matrix
+    const int e = base + (int)(threadIdx.x & 63);
+    at = g.g_seg[min(e, g.groups)];
+    next = g.g_seg[min(e + 1, g.groups)];
+    return (next - at + BM - 1) / BM;
+}
 // which tokens a tile holds: matrix e (grouped), its rows row0 .. row0 + T - 1, first local row t0; false: nothing
 template <int BM>
 static __device__ __forceinline__ bool dn_ring_rows(const dn_args &g, int tm, int &e, long long &row0, int &T, int &t0) {
     e = 0;
-    if (g.g_seg) {
-        for (; e < g.groups; e++) { // (tiles are counted matrix by matrix)
-            row0 = g.g_seg[e];
-            T = g.g_seg[e + 1] - (int)row0;
-            const int c = (T + BM - 1) / BM;
-            if (tm < c) break;
-            tm -= c;
+    if (g.g_seg) { // (uniform; tiles are counted matrix by matrix)
+        for (int base = 0; base < g.groups; base += 64) {
+            int at, next;
+            const int c = dn_ring_slots<BM>(g, base, at, next), upto = dn_wave_upto(c), all = __builtin_amdgcn_readlane(upto, 63);
+            if (tm < all) { // (uniform)
+                const int l = __popcll(__ballot(upto <= tm));
+                e = base + l;
+                row0 = __builtin_amdgcn_readlane(at, l);
+                T = __builtin_amdgcn_readlane(next, l) - (int)row0;
+                t0 = (tm - __builtin_amdgcn_readlane(upto - c, l)) * BM;
+                return true;
+            }
+            tm -= all;
         }
-        t0 = tm * BM;
-        return e < g.groups;
+        return false;
     }
     dn_rows(g, row0, T);
     t0 = tm * BM;
@@ -638,11 +661,12 @@ static __device__ __forceinline__ bool dn_ring_place(const dn_args &g, const dn_
     int n_tm = p.n_tm;
     if (g.g_seg) { // (the host's number is a bound)
         n_tm = 0;
-        for (int e = 0, at = g.g_seg[0]; e < g.groups; e++) {
-            const int next = g.g_seg[e + 1];
-            n_tm += (next - at + BM - 1) / BM;
-            at = next;
+#pragma unroll 4
+        for (int base = 0; base < g.groups; base += 64) {
+            int at, next;
+            n_tm += dn_ring_slots<BM>(g, base, at, next);
         }
+        n_tm = __builtin_amdgcn_readlane(dn_wave_upto(n_tm), 63);
     }
     const int tiles = n_tm * p.tn, items = tiles * p.S, each = (items + 7) >> 3, j = (int)blockIdx.x >> 3;
     int i = ((int)blockIdx.x & 7) * each + j;

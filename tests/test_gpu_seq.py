@@ -463,6 +463,25 @@ def test_large_tiles_behind_an_epilogue(ctx, tmp_path, which):
     assert err(got, plain) < 0.03
 
 
+# matrices counted by the lanes of a wave (k_dense.hip dn_ring_rows): as many experts as lanes, one and two more, three waves full; few tokens, most of whose experts have no slot, and portions in which
+# they have from none to many; products whole and, behind a short inner size, in parts of K
+@pytest.mark.parametrize("dtype", ["float32", "float32 lines", "bfloat16"])
+@pytest.mark.parametrize("experts,ff", [(64, 128), (65, 64), (66, 192), (192, 64), (70, 1152)])
+def test_more_experts_than_lanes(ctx, tmp_path, experts, ff, dtype):
+    cfg = synth.pupidra_config(128, 40, [synth.pupidra_layer("attention", synth.pupidra_attention(2, 1, 16, 16, 0.3, 9, 2), moe=(experts, 3, ff, 1.7), shared=8)])
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+    m = seqmodel.load_model(ctx, str(tmp_path), dtype=dtype.split()[0], max_batch=300, n_slots=1, max_context=400, f32_form=None if dtype == "bfloat16" else FORMS[dtype])
+    toks = tokens_for(cfg, 320)
+    got = run_portions(m, toks, (9, 300, 11))
+    if dtype == "bfloat16":  # (a near tie may be routed the other way behind 16 bits: against the tiled mat-mul)
+        m.set_mode(2)
+        want = run_portions(m, toks, (9, 300, 11))
+    else:
+        want = seq_oracle.run_pupidra(cfg, t, toks)
+    m.close()
+    assert err(got, want) < (0.03 if dtype == "bfloat16" else TOL["float32"])
+
+
 # the same for the tiles of 256 columns at each of their heights, and for 192 x 128 whole and in parts (wide_tiles.py; which kernel runs: test_host_calls.py)
 @pytest.mark.parametrize("which,dtype,size,tokens,width", [(which, dtype, *case[:3]) for (which, dtype), cases in wide_tiles.EPILOGUES.items() for case in cases])
 def test_every_tile_behind_an_epilogue(ctx, tmp_path, which, dtype, size, tokens, width):
