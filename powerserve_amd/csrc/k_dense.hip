@@ -1114,7 +1114,8 @@ static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.ac
 // and 4.3; in three lines 2 x 4 096 x 4 096 22.7 and 20.1, 8 x 8 192 x 2 048 22.7 and 20.0, 190 x 5 120 x 2 560 38.8 and 32.8.
 //   A block costs the bytes it fetches: a CU has about 16 KB of requests outstanding, which the mean way to L2 and beyond makes some 60 bytes a ns, whatever the shape -- 32 KB in 0.5 us of 128 x 128, start
 // included, 64 KB in 1.0 of 256 x 256.  So larger tiles do more per byte, and a height that leaves no round nearly empty counts as much.
-//   Experts' rows: an expert has rows / groups on average, spread as a random routing and some more; the expected number of its tiles.
+//   Experts' rows: an expert has rows / groups on average, spread as a random routing and some more; the expected number of its tiles (few slots of many experts: of experts that have one.  Nine
+// tokens, two of 64 experts, counted as 22 tiles instead of 16 took shapes of two rounds: 584 us of four layers, 553 so).
 // The fp32 instruction (dn_ring_plan_f32): a block of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more.
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
 enum { DN_EPI_DIRECT, DN_EPI_FOURS, DN_EPI_ONES }; // results from the registers; through LDS, four at a time; an activation or bias each
@@ -1132,7 +1133,7 @@ static double dn_mean_row_tiles(int rows, int BM, int groups) {
     const double mean = (double)rows / groups, sd = std::sqrt(mean) + mean / 16;
     double tiles = 0;
     for (int k = 0; k <= rows / BM; k++) { // an expert has its tile k where it has more than k BM rows
-        const double p = 0.5 * std::erfc((k * BM + 0.5 - mean) / (sd * 1.41421356));
+        const double p = k ? 0.5 * std::erfc((k * BM + 0.5 - mean) / (sd * 1.41421356)) : 1 - std::exp(-mean); // (one tile at least: a slot at all, few of them too)
         tiles += p;
         if (p < 1e-3) break;
     }
