@@ -731,7 +731,9 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
                 psk_dense(st, g);
             }
             psk_wkv_fold f;
-            const bool folds = T == 1 && !tiled && l.decay_rank <= 64; // (a longer rank: rows that want a launch of their own)
+            // (a thread reads a row of the second matrix by itself, one piece behind the other, so a longer one wants a launch of its own.  A token of four layers of 2048 in us, so | in the scan: rank 4 203 | 186, 8 200 | 189,
+            // 16 200 | 191, 24 201 | 195, 32 202 | 200, 48 200 | 206, 64 200 | 213; no whole eights 20 206 | 201, 28 203 | 206, 31 205 | 209; float32 8 249 | 235, 24 247 | 246, 28 248 | 246, 32 252 | 252, 64 251 | 273)
+            const bool folds = T == 1 && !tiled && l.decay_rank <= (l.decay2->dtype == PS_BF16 && l.decay_rank % 8 == 0 ? 32 : 24);
             if (folds) {
                 f.w = l.decay2; f.bias = l.decay0; f.a = m->t2; f.src = in; f.dst_off = P.off_shift; f.n = W;
             } else {

@@ -132,10 +132,10 @@ def test_a_token_that_appends_itself(ctx, tmp_path, which, sizes):
     m.close()
 
 
-# a single token's decay, its second product inside the scan (k_seqmix.hip sq_fold): ranks in whole eights and not, the longest there and the first with a launch of its own, in both formats; heads of few
-# rows and of many; the next token's neighbour, behind a portion and behind single tokens
+# a single token's decay, its second product inside the scan (k_seqmix.hip sq_fold): ranks in whole eights and not, the longest there (32 in eights of bfloat16, else 24) and longer ones with a launch of its own
+# (test_host_calls.py), in both formats; heads of few rows and of many; the next token's neighbour, behind a portion and behind single tokens
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("rank", [1, 8, 13, 64, 65])
+@pytest.mark.parametrize("rank", [1, 8, 13, 23, 24, 25, 32, 33, 64, 65])
 def test_decay_of_a_single_token(ctx, tmp_path, rank, dtype):
     cfg = synth.seq_config(160, 40, [L("wkv", None, heads=2, dim=24), L("wkv", 24, heads=1, dim=250)], taps=2)
     t = synth.write_seq_model_dir(str(tmp_path), cfg, 3, synth.seq_tensors(cfg, 3, rank))

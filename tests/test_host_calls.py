@@ -272,6 +272,21 @@ for sizes in ((129, 64), (400, 64), (1024, 128)): assert joined(*sizes) == 0, si
 """.replace(".dir", str(child.tmp / "dir")))
 
 
+@pytest.mark.parametrize("dtype,rank,folds", [("bfloat16", 1, 1), ("bfloat16", 24, 1), ("bfloat16", 25, 0), ("bfloat16", 32, 1), ("bfloat16", 40, 0), ("bfloat16", 64, 0), ("float32", 24, 1), ("float32", 25, 0), ("float32", 32, 0)])
+def test_a_tokens_decay_inside_its_scan(child, dtype, rank, folds):
+    """seqmodel.hip: the decay's second product and the copy of the token's input are launches of their own for the ranks where those are the faster ones"""
+    child("""
+ctx = hip.Ctx(0)
+cfg = synth.seq_config(64, 30, [L("wkv", None, heads=2, dim=32)], taps=2)
+synth.write_seq_model_dir(".dir", cfg, 1, synth.seq_tensors(cfg, 1, RANK))
+m = seqmodel.SeqModel(ctx, ".dir", dtype="DTYPE", max_batch=8)
+s = m.acquire()
+fake.fake_reset()
+m.forward(s, [1])
+assert (count("sq_decay_scan_kernelILi0ELi1ELb1E"), count("sq_decay_scan_kernelILi0ELi1ELb0E")) == (FOLDS, 1 - FOLDS)
+""".replace(".dir", str(child.tmp / "dir")).replace("RANK", str(rank)).replace("DTYPE", dtype).replace("FOLDS", str(folds)))
+
+
 def test_tiles_of_several_parts_are_joined(child):
     """k_splitattn.hip sa_plan_of: the portions whose results tests/test_gpu_seq.py compares -- 41 heads in parts in both portions, 81 in whole tiles"""
     child("""
