@@ -779,7 +779,10 @@ static bool seq_layers(ps_hip_seq *m, float *state, int T, int64_t pos0, bool an
             const float *gate = l.gated ? t1 + Hd + (reads ? 0 : G * d + G * dv) : nullptr;
             const int ge = l.gated == 2; // a gate per output element
             const bool mfma = (m->mode & 2) == 0 && (G * (d + dv)) % 4 == 0 && psk_winattn_mfma_ok((int)d, (int)dv);
-            const bool splits = mfma && split_attn(l, 0), steps = !splits && mfma && T == 1 && m->win_scratch, itself = steps && (l.head_norm || (!l.qnorm && !l.knorm));
+            // itself: the step makes its queries, key and value (psk_winattn_row), where that is the faster one.  A wave makes its heads one behind the other, each with a sum of its own where they are normed: a token of four
+            // layers behind 20 and 300, us with a launch in front | itself: norms, 4 heads a group 160 164 | 155 159, 8 155 161 | 154 156, 12 159 163 | 158 164, 24 168 172 | 170 176, 32 174 178 | 175 182; none, 8 157 160 |
+            // 152 154, 16 166 169 | 158 163, 32 177 182 | 169 171
+            const bool splits = mfma && split_attn(l, 0), steps = !splits && mfma && T == 1 && m->win_scratch, itself = steps && ((!l.qnorm && !l.knorm) || (l.head_norm && H <= 12 * G));
             psk_winattn_row row;
             row.y = t1; row.qnorm = l.qnorm; row.knorm = l.knorm; row.freq = P.freq; row.eps = D.norm_eps; row.qt_coef = l.qtemp_coef; row.rot_mag = P.rot_mag;
             row.rot_dims = l.rot_dims; row.pairing = l.rot_pairing; row.qt_every = l.qtemp_every; row.v_unit = l.v_unit; row.appends = !reads; row.keep = reads ? 0 : P.keep_rows;

@@ -111,21 +111,23 @@ def test_part_norms_of_several_rows(ctx, tmp_path, heads, dim, parts, dtype):
     m.close()
 
 
-# a single token's queries, key and value made inside its attention (k_winattn.hip winattn_step_kernel, ROW): groups of more than sixteen heads, whose blocks all append the row and of which one updates
-# the block means and the kept rows; a ring that wraps; a reader of another layer's keys and values; norms per head with queries that turn; means begun by a portion and finished by single tokens
-@pytest.mark.parametrize("which", ["pool", "keep", "head norms"])
+# a single token's queries, key and value made inside its attention (k_winattn.hip winattn_step_kernel, ROW): groups of more than sixteen heads without norms, whose blocks all append the row and of which one updates
+# the block means; of twelve with norms of their own and kept rows (more of those, and norms over whole projections, have a launch in front: test_host_calls.py); a ring that wraps; a reader of another layer's keys and values; norms per head with queries that turn; means begun by a portion and finished by single tokens
+@pytest.mark.parametrize("which", ["pool", "pool without norms", "keep", "keep 12", "head norms", "18 heads"])
 @pytest.mark.parametrize("sizes", [(1,), (1, 1, 7, 1, 1, 1, 1)])
 def test_a_token_that_appends_itself(ctx, tmp_path, which, sizes):
     V = 40
-    if which == "pool":
+    if which.startswith("pool"):
         at = {"heads": 36, "kv_heads": 2, "dim": 32, "vdim": 32, "mask": {"size": 5, "pool": 3}, "rot": {"base": 100.0, "dims": 16}, "scale": 0.2}
         run, cfg = seq_oracle.run_parallel, synth.parallel_config(64, V, [synth.parallel_layer(None, at, {"heads": 1, "dim": 16, "vdim": 16, "tau": 4.0}, 1.0, 0.5)], taps=2)
-    elif which == "keep":
-        at = lambda size, keep, own=None: synth.pupidra_attention(34, 2, 32, 32, 1.0, size, keep, own)
+    elif which.startswith("keep"):
+        at = lambda size, keep, own=None: synth.pupidra_attention(24 if which == "keep 12" else 34, 2, 32, 32, 1.0, size, keep, own)
         run, cfg = seq_oracle.run_pupidra, synth.pupidra_config(64, V, [synth.pupidra_layer("attention", at(9, 20)), synth.pupidra_layer("attention", at(4, 7, 0))])
     else:
-        run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(6, 2, 48, 32, 0.1, 5.0, (0.4, 7)), ff=64)])
-    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, None)
+        run, cfg = seq_oracle.run_zusolix, synth.zusolix_config(64, V, [synth.zusolix_layer("attention", synth.zusolix_attention(36 if which == "18 heads" else 6, 2, 48, 32, 0.1, 5.0, (0.4, 7)), ff=64)])
+    t = synth.seq_tensors(cfg)
+    if which == "pool without norms": t = {n: v for n, v in t.items() if not n.endswith(("q.norm", "k.norm"))}  # (those over whole projections: a launch in front)
+    t = synth.write_seq_model_dir(str(tmp_path), cfg, 0, t)
     m = seqmodel.load_model(ctx, str(tmp_path), dtype="float32", max_batch=16, n_slots=1, max_context=100)
     toks = tokens_for(cfg, 50)
     assert err(run_portions(m, toks, sizes), run(cfg, t, toks)) < TOL["float32"]

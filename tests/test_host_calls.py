@@ -287,6 +287,26 @@ assert (count("sq_decay_scan_kernelILi0ELi1ELb1E"), count("sq_decay_scan_kernelI
 """.replace(".dir", str(child.tmp / "dir")).replace("RANK", str(rank)).replace("DTYPE", dtype).replace("FOLDS", str(folds)))
 
 
+@pytest.mark.parametrize("heads,norms,itself", [(8, "heads", 1), (24, "heads", 1), (26, "heads", 0), (36, "none", 1), (36, "whole", 0)])
+def test_a_token_whose_attention_makes_its_own_row(child, heads, norms, itself):
+    """seqmodel.hip: without norms, or with those of every head and up to twelve heads a group; more, and norms over whole projections, have the preparation's launch in front"""
+    child("""
+ctx = hip.Ctx(0)
+if NORMS == "heads":
+    cfg = synth.pupidra_config(64, 30, [synth.pupidra_layer("attention", synth.pupidra_attention(HEADS, 2, 32, 32, 1.0, 9, 20))])
+else:
+    at = {"heads": HEADS, "kv_heads": 2, "dim": 32, "vdim": 32, "mask": {"size": 5, "pool": 3}, "rot": {"base": 100.0, "dims": 16}, "scale": 0.2}
+    cfg = synth.parallel_config(64, 30, [synth.parallel_layer(None, at, {"heads": 1, "dim": 16, "vdim": 16, "tau": 4.0}, 1.0, 0.5)], taps=2)
+t = {n: v for n, v in synth.seq_tensors(cfg).items() if NORMS != "none" or not n.endswith(("q.norm", "k.norm"))}
+synth.write_seq_model_dir(".dir", cfg, 1, t)
+m = seqmodel.SeqModel(ctx, ".dir", max_batch=8, n_slots=1, max_context=100)
+s = m.acquire()
+fake.fake_reset()
+m.forward(s, [1])
+assert (count("winattn_step_kernel"), count("winattn_prep_kernel")) == (1, 1 - ITSELF)
+""".replace(".dir", str(child.tmp / "dir")).replace("HEADS", str(heads)).replace("NORMS", repr(norms)).replace("ITSELF", str(itself)))
+
+
 def test_tiles_of_several_parts_are_joined(child):
     """k_splitattn.hip sa_plan_of: the portions whose results tests/test_gpu_seq.py compares -- 41 heads in parts in both portions, 81 in whole tiles"""
     child("""
