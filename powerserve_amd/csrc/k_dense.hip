@@ -1115,7 +1115,8 @@ static bool dn_odd(const dn_args &g) { return g.act != PSD_ACT_SILU_PAIR && g.ac
 //   A block costs the bytes it fetches: a CU has about 16 KB of requests outstanding, which the mean way to L2 and beyond makes some 60 bytes a ns, whatever the shape -- 32 KB in 0.5 us of 128 x 128, start
 // included, 64 KB in 1.0 of 256 x 256.  So larger tiles do more per byte, and a height that leaves no round nearly empty counts as much.
 //   Experts' rows: an expert has rows / groups on average, spread as a random routing and some more; the expected number of its tiles (few slots of many experts: of experts that have one.  Nine
-// tokens, two of 64 experts, counted as 22 tiles instead of 16 took shapes of two rounds: 584 us of four layers, 553 so).
+// tokens, two of 64 experts, counted as 22 tiles instead of 16 took shapes of two rounds: 584 us of four layers, 553 so; 300 slots of eight matrices of 2 048 x 2 048, 8.01 tiles of 64
+// rows, 34 us in 64 x 128 and 28 in 64 x 64).
 // The fp32 instruction (dn_ring_plan_f32): a block of K costs its tile's matrix instructions, or its LDS traffic (fragments read by four waves, the block written), whichever is more.
 struct dn_ring_shape { int BM, BN, n_tm, tn, S; };
 enum { DN_EPI_DIRECT, DN_EPI_FOURS, DN_EPI_ONES }; // results from the registers; through LDS, four at a time; an activation or bias each
@@ -1137,7 +1138,7 @@ static double dn_mean_row_tiles(int rows, int BM, int groups) {
         tiles += p;
         if (p < 1e-3) break;
     }
-    return std::max(1.0, groups * tiles);
+    return std::max(1.0, std::ceil(groups * tiles - 0.3)); // (what most routings have: a second tile that one in a hundred experts needs made two rounds of 256 tiles)
 }
 static dn_ring_shape dn_ring_plan_f32(int rows, int64_t N, int64_t kbytes, int groups, bool may_split) {
     static const int shapes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
