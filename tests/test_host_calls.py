@@ -369,6 +369,21 @@ assert not wrong, "\\n".join(map(str, wrong))
 """.replace("TESTS", repr(HERE)).replace("MODELS", repr(models)).replace(".dir", str(child.tmp / "dir")))
 
 
+@pytest.mark.parametrize("width,experts,ff,tokens", [(1024, 64, 768, 9), (2048, 8, 1536, 150)])
+def test_the_tiles_of_experts(child, width, experts, ff, tokens):
+    """k_dense.hip dn_mean_row_tiles: 18 slots of 64 matrices are 16 tiles of 64 rows, 300 slots of eight are eight -- one round of 64 x 64 tiles, not the start of a second one"""
+    child("""
+ctx = hip.Ctx(0)
+cfg = synth.pupidra_config(WIDTH, 30, [synth.pupidra_layer("attention", synth.pupidra_attention(2, 1, 16, 16, 0.3, 9, 2), moe=(EXPERTS, 2, FF, 1.7), shared=8)])
+synth.write_seq_model_dir(".dir", cfg, 1)
+m = seqmodel.SeqModel(ctx, ".dir", max_batch=TOKENS, n_slots=1, max_context=400)
+s = m.acquire()
+fake.fake_reset()
+m.forward(s, [1] * TOKENS)
+assert count("dense_mm_ring_kernelItLi64ELi64E") >= 2 and count("dense_mm_ring_kernelItLi64ELi128E") == 0
+""".replace(".dir", str(child.tmp / "dir")).replace("WIDTH", str(width)).replace("EXPERTS", str(experts)).replace("FF", str(ff)).replace("TOKENS", str(tokens)))
+
+
 def test_the_measured_products_of_experts_are_the_ones_that_run(child):
     """ps_hip_seq_bench_kernel: a portion's second product of the experts reads the rounded rows of the first one, in a step and where it is measured"""
     child("""
